@@ -18,9 +18,12 @@
 //    fetched into registers while a stage is multiplied and go into the other half of the LDS buffer behind it.  The state is read when the rows
 //    of the launch do not start the sequence and written back after the last row, so a prompt cut into portions, single
 //    decode tokens and a slot that another request held all take one path.
-//  * ssm_post_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
+//  * Prompt batches: ssm_chunk_operands_kernel and ssm_chunk_walk_kernel in place of the three, 32 tokens at a time on the matrix
+//    cores, every operand and sum fp32.
+//  * ssm_post_kernel / ssm_post_vec_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
 #include "common.h"
+#include "mfma_frag.h"
 
 namespace semipd {
 
@@ -38,6 +41,7 @@ struct SsmArgs {
   int64_t batch, num_tokens;
   int H, G, N, E, taps;
   void* out; int64_t out_ld;                       // [T, H E] of the activation type
+  float* frags;                                    // operands of the chunks (matrix-core form), see ssm_chunk_operands_kernel
 };
 
 __device__ __forceinline__ float ssm_silu(float x) { return x / (1.0f + expf(-x)); }
@@ -302,6 +306,507 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------- prompt batches: 32 tokens at a time
+// With la_t = log of the decay, b_t its running sum inside a chunk of 32 tokens and S the state in front of the chunk:
+//     y_t = e^(b_t) S^T C_t + sum_(s <= t) (C_t . B_s) e^(b_t - b_s) dt_s x_s + D x_t
+//     S  <- e^(b_last) S + sum_s B_s (e^(b_last - b_s) dt_s x_s)^T
+// Every exponent is at most 0.  All products are fp32 on v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 sums: nothing is split or
+// rounded to 16 bits); b is summed, and its differences are taken, in 64 bits, so a weight near 1 behind a strong decay is as
+// good as the product of the decays themselves.
+// Bound: token by token a step is a chain of LDS reads, 64 multiply-adds and lane sums (1.0 us of a wave's time; 7262 tokens of 4
+// requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (36 GFLOP at
+// 154 TFLOP/s = 235 us) and the vector work between its products: 560 us, operands 73.  Chunks of 32 and not 64: the same products
+// with S, half the ones inside a chunk, and three workgroups' LDS on a CU in place of one (64 tokens, two heads a workgroup: 952 us).
+constexpr int kSsmChunk = 32;
+constexpr int kSsmChunkTaps = 4;        // taps at most
+
+// fp32 elements of the operands of one (chunk, group): C [32][NP] | B^T [NP][32] | C B^T [32][32] | a flag in a piece of 4,
+// and behind those of all chunks, of one (chunk, head): b in log2 units, 64 bits [32] | dt | e^(b_t) | e^(b_last - b_t) dt_t | decay
+__host__ __device__ constexpr int64_t ssm_frag_elems(int np) { return 2 * (int64_t)kSsmChunk * np + kSsmChunk * kSsmChunk + 4; }
+constexpr int kSsmSteps = 6 * kSsmChunk;
+
+// Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
+__device__ __forceinline__ bool ssm_find_chunk(const SsmArgs& a, int64_t idx, int& b, int64_t& c) {
+  const int lane = threadIdx.x & 63;
+  int64_t before = 0;
+  for (int r0 = 0; r0 < (int)a.batch; r0 += 64) {
+    const int n = r0 + lane < (int)a.batch ? max(0, (a.q_len[r0 + lane] + kSsmChunk - 1) / kSsmChunk) : 0;
+    int s = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(s, o, 64);
+      if (lane >= o) s += t;
+    }
+    const int total = __shfl(s, 63, 64);
+    if (idx < before + total) {
+      const uint64_t past = __ballot(before + s > idx);
+      const int first = __ffsll((unsigned long long)past) - 1;
+      b = r0 + first;
+      c = idx - before - (__shfl(s, first, 64) - __shfl(n, first, 64));
+      return true;
+    }
+    before += total;
+  }
+  return false;
+}
+// how many chunks the requests in front of b have
+__device__ __forceinline__ int64_t ssm_chunks_before(const SsmArgs& a, int b) {
+  const int lane = threadIdx.x & 63;
+  int s = 0;
+  for (int r = lane; r < b; r += 64) s += max(0, (a.q_len[r] + kSsmChunk - 1) / kSsmChunk);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
+// silu of the chunked form: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal
+// and one correction of it and of the result: within an ulp of x / (1 + expf(-x)), 14 instructions in place of 30
+__device__ __forceinline__ float ssm_silu_fast(float x) {
+  const float c = fmaxf(x, -87.f);
+  const float hi = c * -1.44269502f, lo = fmaf(c, -1.44269502f, -hi) + c * -1.92596299e-8f;
+  float e = __builtin_amdgcn_exp2f(hi);
+  e = fmaf(e, lo * 0.693147182f, e);
+  const float d = 1.0f + e;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float q = x * r;
+  return fmaf(fmaf(-d, q, x), r, q);
+}
+
+__device__ __forceinline__ bool ssm_finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+
+// What the heads of a group share, a workgroup per (chunk, group): convolution + bias + silu of the group's B and C channels (a
+// channel per thread, its taps and the last inputs in registers), B also transposed so that the state's update reads four
+// tokens of a row at once, and the 32 x 32 products C B^T; the step sizes and running log decays of the group's heads.  NP: N up to a multiple of 64, zeros behind N and behind the portion.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
+  __shared__ __attribute__((aligned(16))) float c_l[kSsmChunk * (NP + 4)];
+  __shared__ __attribute__((aligned(16))) float b_l[kSsmChunk * (NP + 4)];
+  const int tid = threadIdx.x, g = blockIdx.y;
+  int b;
+  int64_t ck;
+  if (!ssm_find_chunk(a, blockIdx.x, b, ck)) return;
+  const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
+  if (first_pos < 0) return;
+  const int64_t l0 = ck * kSsmChunk, t0 = a.q_start[b] + l0;
+  const int cnt = (int)(n - l0 < kSsmChunk ? n - l0 : kSsmChunk);
+  const int N = a.N, taps = a.taps;
+  const int C = a.H * a.E + 2 * a.G * N;
+  float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * ssm_frag_elems(NP);
+  bool bad = false;
+  for (int ch = tid; ch < 2 * NP; ch += 256) {
+    const bool is_c = ch >= NP;
+    const int r = is_c ? ch - NP : ch;
+    float* dst = (is_c ? c_l : b_l) + r;
+    if (r < N) {
+      const int col = a.H * a.E + (is_c ? a.G * N : 0) + g * N + r;               // among the convolution's channels
+      const T* p = (const T*)a.p + t0 * a.ld + a.x_off + col;
+      const T* cw = (const T*)a.conv_w + (int64_t)col * taps;
+      const float bias = a.conv_b ? Elem<T>::to_f(((const T*)a.conv_b)[col]) : 0.f;
+      float wt[kSsmChunkTaps], in[kSsmChunkTaps];                                     // weight and input i tokens back
+#pragma unroll
+      for (int i = 0; i < kSsmChunkTaps; ++i) {
+        wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
+        in[i] = 0.f;
+        if (i > 0 && i < taps) {
+          if (l0 - i >= 0) in[i] = Elem<T>::to_f(p[-(int64_t)i * a.ld]);
+          else if (first_pos > 0) in[i] = a.conv_state[a.state_indices[b] * a.conv_ld + (int64_t)(taps - 1 + l0 - i) * C + col];
+        }
+      }
+      float x[kSsmChunk];
+#pragma unroll
+      for (int i = 0; i < kSsmChunk; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
+#pragma unroll
+      for (int t = 0; t < kSsmChunk; ++t) {
+        in[0] = x[t];
+        float y = bias;
+#pragma unroll
+        for (int i = 0; i < kSsmChunkTaps; ++i)
+          if (i < taps) y += wt[i] * in[i];
+#pragma unroll
+        for (int i = kSsmChunkTaps - 1; i > 0; --i) in[i] = in[i - 1];
+        x[t] = t < cnt ? ssm_silu(y) : 0.f;
+        bad |= !ssm_finite(x[t]);
+      }
+#pragma unroll
+      for (int t = 0; t < kSsmChunk; ++t) dst[t * (NP + 4)] = x[t];
+      if (!is_c) {
+        float* bt = frag + (int64_t)kSsmChunk * NP + (int64_t)r * kSsmChunk;
+#pragma unroll
+        for (int t = 0; t < kSsmChunk; t += 4) *reinterpret_cast<float4*>(bt + t) = float4{x[t], x[t + 1], x[t + 2], x[t + 3]};
+      }
+    } else {
+      for (int t = 0; t < kSsmChunk; ++t) dst[t * (NP + 4)] = 0.f;
+      if (!is_c) {
+        float* bt = frag + (int64_t)kSsmChunk * NP + (int64_t)r * kSsmChunk;
+        for (int t = 0; t < kSsmChunk; t += 4) *reinterpret_cast<float4*>(bt + t) = float4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  // half a wave per head (lane = token): step sizes, running sums of the log decays
+  for (int hh = tid >> 5; hh < a.H / a.G; hh += 8) {
+    const int h = g * (a.H / a.G) + hh, t = tid & 31;
+    const float dt = t < cnt ? ssm_softplus(Elem<T>::to_f(((const T*)a.p)[(t0 + t) * a.ld + a.dt_off + h]) + a.dt_bias[h]) : 0.f;
+    const float la = t < cnt ? -expf(a.a_log[h]) * dt : 0.f;
+    double cum = (double)la * 1.4426950408889634;
+#pragma unroll
+    for (int o = 1; o < kSsmChunk; o <<= 1) {
+      const double v = __shfl_up(cum, o, kSsmChunk);
+      if (t >= o) cum += v;
+    }
+    const double last = __shfl(cum, kSsmChunk - 1, kSsmChunk);
+    float* sp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmSteps;
+    reinterpret_cast<double*>(sp)[t] = cum;
+    sp[2 * kSsmChunk + t] = dt;
+    sp[3 * kSsmChunk + t] = __builtin_amdgcn_exp2f((float)cum);
+    sp[4 * kSsmChunk + t] = __builtin_amdgcn_exp2f((float)(last - cum)) * dt;
+    sp[5 * kSsmChunk + t] = expf(la);
+  }
+  const int any_bad = __syncthreads_or(bad);
+  if (tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
+  for (int i = tid; i < kSsmChunk * NP / 4; i += 256) {
+    const int t = i / (NP / 4), c = 4 * (i % (NP / 4));
+    *reinterpret_cast<float4*>(frag + (int64_t)t * NP + c) = *reinterpret_cast<const float4*>(c_l + t * (NP + 4) + c);
+  }
+  // C B^T, a 16 x 16 tile a wave; k runs 16 at a time, lane group kq takes k = 4 kq .. 4 kq + 3 in four steps (both operands alike)
+  const int lane = tid & 63, r16 = lane & 15, kq = lane >> 4, i0 = (tid >> 7) * 16, j0 = ((tid >> 6) & 1) * 16;
+  f32x4 acc = {};
+#pragma unroll 4
+  for (int k = 0; k < NP; k += 16) {
+    const f32x4 av = *reinterpret_cast<const f32x4*>(c_l + (i0 + r16) * (NP + 4) + k + 4 * kq);
+    const f32x4 bv = *reinterpret_cast<const f32x4*>(b_l + (j0 + r16) * (NP + 4) + k + 4 * kq);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
+  }
+  float* cb = frag + 2 * (int64_t)kSsmChunk * NP;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) cb[(i0 + 4 * kq + r) * kSsmChunk + j0 + r16] = acc[r];
+}
+
+// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S); a wave has 16 columns of S, its NP rows in
+// accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16.  That is also how a wave holds the right-hand operand of
+// a product over the rows, so S goes from one chunk's sum into the next one's product without leaving its registers, and so do
+// the chunk's x (lane: tokens 16 j + 4 kq + s of its column), which each lane computes itself from the projection's rows: x
+// never touches memory.  C, B^T (shared by the group's heads) and the head's weighted C B^T are read from LDS, 16 bytes for four
+// steps; the next chunk's loads are in flight during the products.  52 KB of LDS: three workgroups a CU, the weights and
+// convolutions of one beside the products of the others.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
+  constexpr int L = kSsmChunk, LT = L / 16, NT = NP / 16;
+  constexpr int CS = NP + 4, TS = L + 4, XS = 68;            // row strides in LDS: rows that are read together start in different banks
+  constexpr int V = 16 / sizeof(T);                           // elements of a 16-byte piece
+  constexpr int HALO = kSsmChunkTaps - 1;
+  constexpr int PF = L * NP / 4 / 256;                        // 16-byte pieces per thread: of C, of B^T
+  constexpr int PX = ((L + HALO) * 64 / V + 255) / 256;       // ... of the projection's rows
+  __shared__ __attribute__((aligned(16))) float c_l[L * CS];
+  __shared__ __attribute__((aligned(16))) float bt_l[NP * TS];
+  __shared__ __attribute__((aligned(16))) float m_l[L * TS];              // weighted C B^T
+  __shared__ __attribute__((aligned(16))) float x_l[(L + HALO) * XS];     // inputs of the convolution
+  __shared__ __attribute__((aligned(16))) float steps_l[kSsmSteps];
+  const double* cum_l = reinterpret_cast<const double*>(steps_l);         // b in log2 units | dt | e^(b_t) | e^(b_last - b_t) dt_t | decay
+  const float *dt_l = steps_l + 2 * L, *eb_l = dt_l + L, *wt_l = eb_l + L, *dec_l = wt_l + L;
+  __shared__ int flag_l[2];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+  // workgroups of one (request, group) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
+  const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, per = H / G;
+  const int eblocks = (E + 63) / 64, members = per * eblocks;
+  const int turn = blockIdx.x / 8, unit = turn / members * 8 + blockIdx.x % 8;
+  if (unit >= (int)a.batch * G) return;
+  const int member = turn % members, b = unit / G, g = unit % G;
+  const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
+  const int n = a.q_len[b];
+  if (n <= 0 || first_pos < 0) return;
+  const int64_t chunk0 = ssm_chunks_before(a, b);
+  if (chunk0 + (n + L - 1) / L > max_chunks) return;          // (requests that share rows: more rows than the launch has)
+  const int h = g * per + member / eblocks;
+  const int e0 = member % eblocks * 64, e = e0 + 16 * w + r16;
+  const bool e_ok = e < E;
+  const int C = H * E + 2 * G * N;
+  const int64_t slot = a.state_indices[b];
+  float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
+  f32x4 S[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * t + 4 * kq + r;
+      S[t][r] = (first_pos > 0 && e_ok && row < N) ? st[row * E] : 0.f;
+    }
+  float wt[kSsmChunkTaps];
+#pragma unroll
+  for (int i = 0; i < kSsmChunkTaps; ++i) wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_w)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
+  const float bias = (a.conv_b && e_ok) ? Elem<T>::to_f(((const T*)a.conv_b)[h * E + e]) : 0.f;
+  const float dskip = a.d_skip ? a.d_skip[h] : 0.f;
+  const int64_t frag_ld = (int64_t)G * ssm_frag_elems(NP);
+  const float* f = a.frags + chunk0 * frag_ld + g * ssm_frag_elems(NP);      // the operands of the chunk that is fetched next
+  const T* p = (const T*)a.p + t0 * a.ld + a.x_off + h * E + e0;
+  const float* fs = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kSsmSteps;
+  const uint32_t xo = (uint32_t)(tid / (64 / V)) * (uint32_t)a.ld + tid % (64 / V) * V;      // this thread's first piece of the rows
+
+  f32x4 pc[PF], pb[PF], pcb, ps;
+  Vec16<T> px[PX];
+  float pflag = 0.f;
+  const int mi = tid >> 3, mj = (tid & 7) * 4;                // this thread's four elements of the weighted C B^T
+  const bool wide = e0 + 64 <= E;
+  auto fetch = [&](int l0) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      pc[u] = *reinterpret_cast<const f32x4*>(f + 4 * (u * 256 + tid));
+      pb[u] = *reinterpret_cast<const f32x4*>(f + L * NP + 4 * (u * 256 + tid));
+    }
+    pcb = *reinterpret_cast<const f32x4*>(f + 2 * L * NP + 4 * tid);
+    pflag = f[ssm_frag_elems(NP) - 4];
+    f += frag_ld;
+    if (tid < kSsmSteps / 4) ps = *reinterpret_cast<const f32x4*>(fs + 4 * tid);
+    fs += (int64_t)H * kSsmSteps;
+    const T* rows = p + (int64_t)(l0 - HALO) * a.ld;
+    if (wide && l0 >= HALO && l0 + L <= n) {                  // every row and column of the tile is there
+#pragma unroll
+      for (int u = 0; u < PX; ++u)
+        if ((u + 1) * 256 <= (L + HALO) * 64 / V || u * 256 + tid < (L + HALO) * 64 / V)
+          px[u] = load16(rows + (int64_t)u * 256 / (64 / V) * a.ld + xo);
+    } else {
+#pragma unroll
+      for (int u = 0; u < PX; ++u) {
+        const int it = u * 256 + tid, row = it / (64 / V), c = it % (64 / V) * V, l = l0 - HALO + row;
+        if (row < L + HALO && l >= 0 && l < n && e0 + c < E) px[u] = load16(rows + (int64_t)row * a.ld + c);
+        else
+#pragma unroll
+          for (int v = 0; v < V; ++v) px[u].e[v] = Elem<T>::from_f(0.f);
+      }
+    }
+  };
+  fetch(0);
+  if (tid < 2) flag_l[tid] = 0;
+  __syncthreads();
+  for (int l0 = 0; l0 < n; l0 += L) {
+    const int cnt = n - l0 < L ? n - l0 : L;
+    const int par = (l0 / L) & 1;
+    bool bad = pflag != 0.f;
+    // ---- what came in: C, B^T, inputs of the convolution; running sums of the log decays (lane = token)
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int it = u * 256 + tid;
+      *reinterpret_cast<f32x4*>(c_l + it / (NP / 4) * CS + 4 * (it % (NP / 4))) = pc[u];
+      *reinterpret_cast<f32x4*>(bt_l + it / (L / 4) * TS + 4 * (it % (L / 4))) = pb[u];
+    }
+#pragma unroll
+    for (int u = 0; u < PX; ++u) {
+      const int it = u * 256 + tid, row = it / (64 / V), c = it % (64 / V) * V;
+      if (row < L + HALO)
+#pragma unroll
+        for (int v = 0; v < V; v += 4)
+          *reinterpret_cast<f32x4*>(x_l + row * XS + c + v) = f32x4{Elem<T>::to_f(px[u].e[v]), Elem<T>::to_f(px[u].e[v + 1]),
+                                                                     Elem<T>::to_f(px[u].e[v + 2]), Elem<T>::to_f(px[u].e[v + 3])};
+    }
+    if (l0 == 0 && first_pos > 0 && taps > 1) {               // the inputs in front of the portion: from the state row, fp32
+      __syncthreads();
+      for (int i = tid; i < (taps - 1) * 64; i += 256) {
+        const int back = i / 64 + 1, c = i % 64;
+        if (e0 + c < E) x_l[(HALO - back) * XS + c] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 - back) * C + h * E + e0 + c];
+      }
+    }
+    if (tid < kSsmSteps / 4) {
+      *reinterpret_cast<f32x4*>(steps_l + 4 * tid) = ps;
+      if (4 * tid >= 2 * L) bad |= !ssm_finite(ps[0]) || !ssm_finite(ps[1]) || !ssm_finite(ps[2]) || !ssm_finite(ps[3]);
+    }
+    __syncthreads();
+    // ---- this lane's x of the chunk; the head's weighted C B^T
+    float xr[4 * LT];
+#pragma unroll
+    for (int j = 0; j < LT; ++j) {
+      float in[HALO + 4];
+#pragma unroll
+      for (int i = 0; i < HALO + 4; ++i) in[i] = i >= kSsmChunkTaps - taps ? x_l[(16 * j + 4 * kq + i) * XS + 16 * w + r16] : 0.f;
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float y = bias;
+#pragma unroll
+        for (int i = 0; i < kSsmChunkTaps; ++i)
+          if (i < taps) y += wt[i] * in[s + HALO - i];
+        const bool ok = ssm_finite(y);                          // (silu of infinity: itself; of minus infinity: inf / inf)
+        xr[4 * j + s] = ok ? ssm_silu_fast(y) : (y > 0.f ? y : __builtin_nanf(""));
+        bad |= !ok;
+      }
+    }
+    if (cnt < L)
+#pragma unroll
+      for (int j = 0; j < LT; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xr[4 * j + s] = 16 * j + 4 * kq + s < cnt ? xr[4 * j + s] : 0.f;
+    {
+      const double bi = cum_l[mi];
+      f32x4 m;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) m[v] = mj + v <= mi ? pcb[v] * (__builtin_amdgcn_exp2f((float)(bi - cum_l[mj + v])) * dt_l[mj + v]) : 0.f;
+      *reinterpret_cast<f32x4*>(m_l + mi * TS + mj) = m;
+    }
+    if (__any(bad) && lane == 0) flag_l[par] = 1;
+    if (tid == 0) flag_l[par ^ 1] = 0;
+    __syncthreads();
+    const bool serial = flag_l[par] != 0;
+    if (l0 + L < n) fetch(l0 + L);
+    float* yo = a.work + (t0 + l0) * a.wld;
+    const uint32_t yc = (uint32_t)(h * E + e), yk = (uint32_t)(4 * kq) * (uint32_t)a.wld + yc;
+    if (!serial) {
+      f32x4 acc[LT] = {};
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        f32x4 av[LT];
+#pragma unroll
+        for (int i = 0; i < LT; ++i) av[i] = *reinterpret_cast<const f32x4*>(c_l + (16 * i + r16) * CS + 16 * t + 4 * kq);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < LT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], S[t][s], acc[i], 0, 0, 0);
+        if (t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 0; i < LT; ++i) acc[i] *= *reinterpret_cast<const f32x4*>(eb_l + 16 * i + 4 * kq);
+#pragma unroll
+      for (int k = 0; k < LT; ++k) {
+        f32x4 av[LT];
+#pragma unroll
+        for (int i = k; i < LT; ++i) av[i] = *reinterpret_cast<const f32x4*>(m_l + (16 * i + r16) * TS + 16 * k + 4 * kq);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = k; i < LT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], xr[4 * k + s], acc[i], 0, 0, 0);
+      }
+      if (cnt == L && wide) {
+#pragma unroll
+        for (int i = 0; i < LT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) (yo + (int64_t)(16 * i + r) * a.wld)[yk] = acc[i][r] + dskip * xr[4 * i + r];
+      } else {
+#pragma unroll
+        for (int i = 0; i < LT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * i + 4 * kq + r < cnt && e_ok) (yo + (int64_t)(16 * i + r) * a.wld)[yk] = acc[i][r] + dskip * xr[4 * i + r];
+      }
+      const float keep = eb_l[L - 1];
+#pragma unroll
+      for (int k = 0; k < LT; ++k) {
+        const f32x4 wv = *reinterpret_cast<const f32x4*>(wt_l + 16 * k + 4 * kq);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) xr[4 * k + s] *= wv[s];
+      }
+#pragma unroll
+      for (int t = 0; t < NT; t += 2) {
+        S[t] *= keep;
+        S[t + 1] *= keep;
+#pragma unroll
+        for (int k = 0; k < LT; ++k) {
+          f32x4 av[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) av[i] = *reinterpret_cast<const f32x4*>(bt_l + (16 * (t + i) + r16) * TS + 16 * k + 4 * kq);
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) S[t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], xr[4 * k + s], S[t + i], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      // an infinity or a NaN in the chunk would reach the tokens in front of it through a product with a weight of zero: such a
+      // chunk goes token by token, S in the state row meanwhile (a rare path: it must not set the kernel's registers); x through
+      // LDS, a wave writes and reads its own columns
+#pragma unroll
+      for (int j = 0; j < LT; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) x_l[(16 * j + 4 * kq + s) * XS + 16 * w + r16] = xr[4 * j + s];
+      __syncthreads();
+      int rows = N, step = E;
+      asm volatile("" : "+s"(rows), "+s"(step));
+      if (e_ok) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll 1
+      for (int t = 0; t < cnt; ++t) {
+        const float xv = x_l[t * XS + 16 * w + r16], dec = dec_l[t], dx = dt_l[t] * xv;
+        float y = 0.f;
+#pragma unroll 1
+        for (int u = 0; u < 4 * NT; ++u) {
+          const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
+          if (row < rows && e_ok) {
+            const float v = dec * st[row * step] + bt_l[row * TS + t] * dx;
+            st[row * step] = v;
+            y += v * c_l[t * CS + row];
+          }
+        }
+        y += __shfl_xor(y, 16, 64);
+        y += __shfl_xor(y, 32, 64);
+        if (kq == 0 && e_ok) yo[t * a.wld + yc] = y + dskip * xv;
+      }
+      if (e_ok) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * t + 4 * kq + r < rows) S[t][r] = st[(16 * t + 4 * kq + r) * step];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    __syncthreads();
+  }
+  int rows = N, step = E;
+  asm volatile("" : "+s"(rows), "+s"(step));                   // (nor their addresses)
+  if (e_ok)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 16 * t + 4 * kq + r;
+        if (row < rows) st[row * step] = S[t][r];
+      }
+}
+
+// gate, grouped norm, weight, one pass: a workgroup per (token, norm group), the group's elements in registers, 16-byte accesses
+// (8 elements a piece, at most kPostPieces pieces a thread).  Bound by HBM: 7262 x 8192 169 us (two passes, 2- and 4-byte accesses) ->
+// 89 = 5.4 TB/s; 32 rows 28 -> 7 us.
+constexpr int kPostPieces = 4;
+template <typename T>
+__global__ void __launch_bounds__(256) ssm_post_vec_kernel(SsmArgs a) {
+  __shared__ float red[16];
+  const int gs = a.H * a.E / a.norm_groups;
+  const int64_t t = blockIdx.x, c0 = (int64_t)blockIdx.y * gs;
+  const float* yr = a.work + t * a.wld + c0;
+  const T* z = (const T*)a.p + t * a.ld + a.z_off + c0;
+  float v[kPostPieces][8], sq = 0.f;
+#pragma unroll
+  for (int u = 0; u < kPostPieces; ++u) {
+    const int c = 8 * (u * 256 + (int)threadIdx.x);
+    if (c >= gs) break;
+    const float4 y0 = *reinterpret_cast<const float4*>(yr + c), y1 = *reinterpret_cast<const float4*>(yr + c + 4);
+    const float yy[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+    const Vec16<T> zv = load16(z + c);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[u][i] = yy[i] * ssm_silu(Elem<T>::to_f(zv.e[i]));
+      sq += v[u][i] * v[u][i];
+    }
+  }
+  const float rs = 1.0f / sqrtf(block_sum(sq, red) / (float)gs + a.eps);
+  T* o = (T*)a.out + t * a.out_ld + c0;
+  const T* nw = (const T*)a.norm_w + c0;
+#pragma unroll
+  for (int u = 0; u < kPostPieces; ++u) {
+    const int c = 8 * (u * 256 + (int)threadIdx.x);
+    if (c >= gs) break;
+    const Vec16<T> wv = load16(nw + c);
+    Vec16<T> r;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) r.e[i] = Elem<T>::from_f(v[u][i] * rs * Elem<T>::to_f(wv.e[i]));
+    store16(o + c, r);
+  }
+}
+
 // ---------------------------------------------------------------------------------- gate, grouped norm, weight
 template <typename T>
 __device__ __forceinline__ void ssm_gate_norm_store(const SsmArgs& a, const float* y, const T* z, T* o, float* red) {
@@ -396,13 +901,34 @@ extern "C" int64_t semipd_state_space_work_width(int num_heads, int groups, int 
   return (w + 3) / 4 * 4;
 }
 
-extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
+// The rows per request (on average) from which a prompt batch goes in chunks, and how many chunks a launch can have.  Token by
+// token against chunks, whole call, 128 heads of 128 x 64: 1 request of 8 rows 34.0 / 36.1 us, 12 rows 37.3 / 36.4, 32 rows 56 / 40,
+// 256 rows 327 / 79; 32 requests of 8 rows 185 / 148, 32 rows 548 / 191, 256 rows 3058 / 782; 64 heads: 1 request of 12 rows 34.3 / 33.8,
+// 32 requests of 8 rows 110 / 88.
+constexpr int64_t kSsmChunkMinRows = 12;
+static int64_t ssm_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kSsmChunk + batch; }
+static int ssm_padded_state(int state_size) { return state_size <= 64 ? 64 : 128; }
+
+extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state_size, int v_dim, int taps) {
+  if (batch <= 0 || groups <= 0 || num_tokens < kSsmChunkMinRows * batch || state_size > 128 || v_dim % 8 != 0 || taps > kSsmChunkTaps) return 0;
+  return ssm_max_chunks(num_tokens, batch) * (groups * ssm_frag_elems(ssm_padded_state(state_size)) + (int64_t)num_heads * kSsmSteps);
+}
+
+template <typename T, int NP>
+static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
+  const int64_t chunks = ssm_max_chunks(a.num_tokens, a.batch);
+  hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
+  const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
+  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);
+}
+
+static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
                                   const void* conv_b, const float* dt_bias, const float* a_log, const float* d_skip,
                                   const void* norm_w, int norm_groups, float eps, float* work, int64_t work_ld, float* state,
                                   int64_t state_ld, float* conv_state, int64_t conv_ld, const int64_t* state_indices,
                                   const int64_t* seq_lens, const int32_t* q_start, const int32_t* q_len, int64_t batch,
                                   int64_t num_tokens, int num_heads, int groups, int state_size, int v_dim, int taps, void* out,
-                                  int64_t out_ld, int fused_decode, int dtype, void* stream) {
+                                  int64_t out_ld, int fused_decode, float* chunk_work, int64_t chunk_elems, int dtype, void* stream) {
   SEMIPD_CHECK_ARG(batch >= 0 && num_tokens >= 0, SEMIPD_EINVAL, "state_space: bad sizes");
   if (batch == 0 || num_tokens == 0) return 0;
   SEMIPD_CHECK_ARG(num_heads > 0 && groups > 0 && num_heads % groups == 0 && state_size > 0 && v_dim > 0 && taps >= 1 && taps <= 64,
@@ -423,7 +949,7 @@ extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, i
                    SEMIPD_EINVAL, "state_space: a column range leaves the row");
   SsmArgs a{proj, ld, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_w, norm_groups, eps, work, work_ld, state,
             state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, groups, state_size,
-            v_dim, taps, out, out_ld};
+            v_dim, taps, out, out_ld, chunk_work};
   hipStream_t s = as_stream(stream);
   const size_t dec_lds = (size_t)(C + 2 * num_heads + inner) * sizeof(float);
   if (q_start == nullptr && fused_decode && dec_lds <= 160 * 1024 - 256) {
@@ -440,6 +966,26 @@ extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, i
   }
   SEMIPD_CHECK_ARG(work && work_ld >= semipd_state_space_work_width(num_heads, groups, state_size, v_dim), SEMIPD_EINVAL,
                    "state_space: the work rows are missing or too short");
+  // gate and norm with 16-byte accesses and the row in registers
+  const int64_t gs = inner / norm_groups;
+  const bool post8 = dtype != SEMIPD_F32 && gs % 8 == 0 && gs <= 8 * 256 * kPostPieces && z_off % 8 == 0 && ld % 8 == 0 && out_ld % 8 == 0 &&
+                     work_ld % 4 == 0 && aligned16(proj) && aligned16(out) && aligned16(norm_w) && aligned16(work);
+  auto post = [&]() -> int {
+    const dim3 vgrid((unsigned)num_tokens, (unsigned)norm_groups);
+    if (post8) SEMIPD_DISPATCH_HALF(dtype, T, hipLaunchKernelGGL((ssm_post_vec_kernel<T>), vgrid, dim3(256), 0, s, a))
+    else SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a))
+    return 0;
+  };
+  const int64_t want = q_start ? semipd_state_space_chunk_elems(num_tokens, batch, num_heads, groups, state_size, v_dim, taps) : 0;
+  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work) && x_off % 8 == 0 && ld % 8 == 0 && aligned16(proj)) {
+    SEMIPD_DISPATCH_DTYPE(dtype, T, if (state_size <= 64) launch_ssm_chunks<T, 64>(a, s); else launch_ssm_chunks<T, 128>(a, s));
+    if (taps > 1) {
+      const dim3 grid((unsigned)((C + 255) / 256), (unsigned)batch);
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), grid, dim3(256), 0, s, a));
+    }
+    if (post()) return SEMIPD_EDTYPE;
+    return launch_status("state_space(chunks)");
+  }
   const unsigned cblocks = (unsigned)((C + kPrepChannels - 1) / kPrepChannels);
   // four channels per thread: every row and column range starts on a multiple of four elements
   const bool prep4 = C % 4 == 0 && x_off % 4 == 0 && ld % 4 == 0 && work_ld % 4 == 0 && (taps == 1 || conv_ld % 4 == 0) &&
@@ -472,6 +1018,30 @@ extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, i
   else if (state_size <= 128) SEMIPD_SSM_SCAN(32, 4);
   else SEMIPD_SSM_SCAN(32, 8);
 #undef SEMIPD_SSM_SCAN
-  SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a));
+  if (post()) return SEMIPD_EDTYPE;
   return launch_status("state_space");
+}
+
+extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
+                                  const void* conv_b, const float* dt_bias, const float* a_log, const float* d_skip,
+                                  const void* norm_w, int norm_groups, float eps, float* work, int64_t work_ld, float* state,
+                                  int64_t state_ld, float* conv_state, int64_t conv_ld, const int64_t* state_indices,
+                                  const int64_t* seq_lens, const int32_t* q_start, const int32_t* q_len, int64_t batch,
+                                  int64_t num_tokens, int num_heads, int groups, int state_size, int v_dim, int taps, void* out,
+                                  int64_t out_ld, int fused_decode, int dtype, void* stream) {
+  return state_space(proj, ld, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_w, norm_groups, eps, work, work_ld, state,
+                     state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, groups,
+                     state_size, v_dim, taps, out, out_ld, fused_decode, nullptr, 0, dtype, stream);
+}
+
+extern "C" int semipd_state_space_prompt(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
+                                         const void* conv_b, const float* dt_bias, const float* a_log, const float* d_skip,
+                                         const void* norm_w, int norm_groups, float eps, float* work, int64_t work_ld, float* state,
+                                         int64_t state_ld, float* conv_state, int64_t conv_ld, const int64_t* state_indices,
+                                         const int64_t* seq_lens, const int32_t* q_start, const int32_t* q_len, int64_t batch,
+                                         int64_t num_tokens, int num_heads, int groups, int state_size, int v_dim, int taps, void* out,
+                                         int64_t out_ld, float* chunk_work, int64_t chunk_elems, int dtype, void* stream) {
+  return state_space(proj, ld, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_w, norm_groups, eps, work, work_ld, state,
+                     state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, groups,
+                     state_size, v_dim, taps, out, out_ld, 0, chunk_work, chunk_elems, dtype, stream);
 }

@@ -1,0 +1,117 @@
+"""Recurrences over prompt batches in chunks of 32 tokens, against the recurrence itself, token by token in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+F64 = torch.float64
+
+
+def _conv_silu(x, weight, bias, before):
+    xs = torch.cat([before, x])
+    y = sum(xs[i: i + x.shape[0]] * weight[:, i] for i in range(weight.shape[1]))
+    return torch.nn.functional.silu(y if bias is None else y + bias), xs[x.shape[0]:]
+
+
+def _ssm_inputs(H, G, N, E, taps, lens, dtype, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    inner, C = H * E, H * E + 2 * G * N
+    w = dict(conv=(0.5 * torch.randn(C, taps, generator=g)).to(dtype), bias=(0.1 * torch.randn(C, generator=g)).to(dtype),
+             dt_bias=0.5 * torch.randn(H, generator=g) - 1, a_log=0.5 * torch.randn(H, generator=g) - 1 + (scale > 1) * 2.0,
+             skip=torch.randn(H, generator=g), norm=(1 + 0.1 * torch.randn(inner, generator=g)).to(dtype))
+    cols = -(-(2 * inner + 2 * G * N + H) // 8) * 8
+    rows = [(scale * torch.randn(n, cols, generator=g)).to(dtype) for n in lens]
+    state = 0.3 * torch.randn(len(lens), H, N, E, generator=g)
+    before = torch.randn(len(lens), taps - 1, C, generator=g)
+    return w, rows, state, before
+
+
+def _ssm_truth(w, row, state, before, H, G, N, E, parts, eps=1e-5):
+    """[n, H E], the state behind it and the last inputs of the convolution."""
+    inner, C = H * E, H * E + 2 * G * N
+    x = row.to(F64)
+    y, last = _conv_silu(x[:, inner: inner + C], w["conv"].to(F64), w["bias"].to(F64), before.to(F64))
+    xs, B, Cm = y.split([inner, G * N, G * N], 1)
+    of = torch.arange(H) // (H // G)
+    dt = torch.nn.functional.softplus(x[:, inner + C: inner + C + H] + w["dt_bias"].to(F64))
+    dec = torch.exp(-torch.exp(w["a_log"].to(F64)) * dt)
+    S, o = state.to(F64).clone(), []
+    for t in range(x.shape[0]):
+        xt = xs[t].view(H, E)
+        S = dec[t][:, None, None] * S + B[t].view(G, N)[of][:, :, None] * (dt[t][:, None] * xt)[:, None]
+        o.append((S * Cm[t].view(G, N)[of][:, :, None]).sum(1) + w["skip"].to(F64)[:, None] * xt)
+    o = torch.stack(o).view(-1, inner) * torch.nn.functional.silu(x[:, :inner])
+    v = o.view(-1, parts, inner // parts)
+    return (v / (v.square().mean(-1, keepdim=True) + eps).sqrt()).view(-1, inner) * w["norm"].to(F64), S, last
+
+
+def _ssm_run(w, rows, state, before, first, H, G, N, E, parts, eps=1e-5):
+    from semi_pd_amd import ops
+    inner, C, taps = H * E, H * E + 2 * G * N, w["conv"].shape[1]
+    B = len(rows)
+    lens = [r.shape[0] for r in rows]
+    sw, cw = inner * N, (taps - 1) * C
+    slab = torch.full((B + 1, 3 + sw + cw + 2), 7.0, device=DEV)                   # (column ranges that start on odd elements)
+    slab[1:, 3: 3 + sw] = state.reshape(B, -1).to(DEV)
+    slab[1:, 3 + sw: 3 + sw + cw] = before.reshape(B, -1).to(DEV)
+    start, at = [], 0
+    for n in lens:
+        start.append(at)
+        at += n
+    d = {k: v.to(DEV) for k, v in w.items()}
+    out = ops.state_space(torch.cat(rows).to(DEV), 0, inner, inner + C, d["conv"], d["bias"], d["dt_bias"], d["a_log"], d["skip"], d["norm"],
+                          parts, eps, slab[:, 3: 3 + sw], slab[:, 3 + sw: 3 + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
+                          torch.tensor([n + f for n, f in zip(lens, first)], device=DEV), torch.tensor(start, dtype=torch.int32, device=DEV),
+                          torch.tensor(lens, dtype=torch.int32, device=DEV), H, G, N, E)
+    slab = slab.cpu()
+    assert bool((slab[0] == 7).all() and (slab[:, :3] == 7).all() and (slab[:, -2:] == 7).all())
+    return out.cpu().split(lens), slab[1:, 3: 3 + sw].view(B, H, N, E), slab[1:, 3 + sw: 3 + sw + cw].view(B, taps - 1, C)
+
+
+# (sizes: rows of S in and below a padded block, columns over one and two workgroups, a group of three heads; two heads a
+# workgroup in the last two.  rows: one, around multiples of 32, a single token beside a long prompt)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,N,E,taps,parts,lens", [
+    (4, 2, 128, 64, 4, 1, [64, 1, 130]), (6, 2, 40, 40, 2, 2, [63, 65]), (3, 1, 7, 72, 1, 1, [128, 127]), (2, 2, 65, 8, 3, 2, [16, 200]),
+    (260, 4, 16, 8, 4, 4, [33, 65]), (66, 22, 24, 24, 3, 1, [17] * 7 + [70])])
+def test_state_space_in_chunks(dtype, H, G, N, E, taps, parts, lens):
+    """Fresh sequences and portions (every second request) in one launch.  fp32: products and sums of 32 bits over at most 200 tokens;
+    16-bit types: the rounding of the result, half a unit in the last place, on top."""
+    first = [0 if i % 2 == 0 else 37 for i in range(len(lens))]
+    w, rows, state, before = _ssm_inputs(H, G, N, E, taps, lens, dtype, H * 131 + E)
+    outs, after, last = _ssm_run(w, rows, state, before, first, H, G, N, E, parts)
+    ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for b, n in enumerate(lens):
+        want, S, tail = _ssm_truth(w, rows[b], state[b] if first[b] else torch.zeros_like(state[b]),
+                                   before[b] if first[b] else torch.zeros_like(before[b]), H, G, N, E, parts)
+        torch.testing.assert_close(outs[b].to(F64), want, rtol=ulp + 2e-5, atol=2e-5)
+        torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+
+
+def test_state_space_in_chunks_strong_decays():
+    """Steps that leave nothing of the state beside steps that keep nearly all of it: a weight near 1 behind a lost state is as exact as
+    its own decays are (the differences of the running sums are taken in 64 bits)."""
+    H, G, N, E, lens = 4, 2, 32, 16, [150]
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 4, lens, torch.float32, 5, scale=12.0)
+    outs, after, _ = _ssm_run(w, rows, state, before, [9], H, G, N, E, 1)
+    want, S, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
+    assert float((outs[0].to(F64) - want).norm() / want.norm()) < 2e-6
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 2e-6
+
+
+@pytest.mark.parametrize("col", ["x", "B", "dt"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_state_space_in_chunks_not_finite(col, value):
+    """A NaN or an infinity at a token leaves the tokens in front of it, and the other request, as they were."""
+    H, G, N, E, lens, at = 4, 2, 32, 16, [100, 100], 90
+    inner = H * E
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 1, lens, torch.float32, 6)
+    clean, _, _ = _ssm_run(w, rows, state, before, [0, 9], H, G, N, E, 1)
+    c = {"x": inner, "B": 2 * inner + 3, "dt": 2 * inner + 2 * G * N}[col]
+    rows[0][at, c] = value
+    got, _, _ = _ssm_run(w, rows, state, before, [0, 9], H, G, N, E, 1)
+    torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
+    if col != "dt" or value != value:
+        assert not bool(torch.isfinite(got[0][at:]).all())
