@@ -924,6 +924,17 @@ int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
                       const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
                       const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
                       int k_dim, int v_dim, int taps, void* out, int64_t out_ld, int dtype, void* stream);
+/* fp32 elements that semipd_delta_rule_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
+int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps);
+/* semipd_delta_rule of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a
+ * time on the matrix cores in fp32.  Without room, or where sizes do not allow it: as semipd_delta_rule. */
+int semipd_delta_rule_prompt(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
+                      int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
+                      const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
+                      int64_t work_ld, float* state, int64_t state_ld, float* conv_state, int64_t conv_ld,
+                      const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
+                      const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
+                      int k_dim, int v_dim, int taps, void* out, int64_t out_ld, float* chunk_work, int64_t chunk_elems, int dtype, void* stream);
 int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, int k_dim, int v_dim);
 /* Rows of `groups` x [gate ff | up ff] -> rows of `groups` x ff: a = min(gate, limit), b = clamp(up, -limit, limit),
  * y = a * sigmoid(alpha a) * (b + 1); with routing (topk_weights fp32 / topk_ids int32 [rows, topk]) times the weight of

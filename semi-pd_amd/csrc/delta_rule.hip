@@ -17,9 +17,12 @@
 //    as 16-byte pieces that are in flight a stage ahead and sit in LDS (k . q, g, beta beside them); o leaves the same way.
 //    The state is read when the rows of the launch do not start the sequence and written back after the last row, so a
 //    prompt cut into portions, single decode tokens and a slot that another request held all take one path.
-//  * delta_post_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
+//  * Prompt batches: delta_chunk_operands_kernel and delta_chunk_walk_kernel in place of the three, 32 tokens at a time on the
+//    matrix cores, every operand and sum fp32.
+//  * delta_post_kernel / delta_post_vec_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
 //  * delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, head).
 #include "common.h"
+#include "mfma_frag.h"
 
 namespace semipd {
 
@@ -38,6 +41,7 @@ struct DeltaArgs {
   int H, G, D, E, taps;
   float eps;
   void* out; int64_t out_ld;                       // [T, H E] of the activation type
+  float* frags;                                    // operands of the chunks (matrix-core form), see delta_chunk_operands_kernel
 };
 
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
@@ -466,6 +470,574 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
   }
 }
 
+// ---------------------------------------------------------------------------------- prompt batches: 32 tokens at a time
+// With b_t the running sum of the log decays inside a chunk of 32 tokens and S the state in front of it:
+//     u_t = beta_t (v_t - e^(b_t) S^T k_t - sum_(s < t) e^(b_t - b_s) (k_t . k_s) u_s)
+//     o_t = e^(b_t) S^T q_t + sum_(s <= t) e^(b_t - b_s) (q_t . k_s) u_s
+//     S  <- e^(b_last) S + sum_s k_s (e^(b_last - b_s) u_s)^T
+// The sums over s < t are a unit lower triangular matrix A, so U = (I + A)^-1 diag(beta) (V - diag(e^b) K S); everything in
+// front of V and S is independent of the chunks before it and is computed for all chunks at once.  All operands and sums are
+// fp32 (v_mfma_f32_16x16x4_f32; nothing is split or rounded to 16 bits), every exponent is at most 0, b is summed, and its
+// differences are taken, in 64 bits.
+// Bound: token by token a step is a chain of two dot products, a lane sum and an update (0.8 us; 7262 tokens of 4 requests, 32 heads of
+// 128 x 128: 1861 us + 317 of preparation); in chunks a wave's chain of 216 products of 32 cycles a chunk (72 chunks: 207 us, one
+// wave a SIMD at 4 requests): 390 us, operands 91.  With the raw inputs of v fetched at the end of a chunk and convolved in
+// front of the products 483 (the loads of 35 rows 24 KB apart were waited for): they are fetched a whole chunk ahead.
+constexpr int kDeltaChunk = 32;
+constexpr int kDeltaChunkTaps = 4;        // taps at most
+
+// fp32 elements of the operands of one (chunk, key head): K, Q and K^T as left-hand operands of 16 x 16 x 16 products, the
+// order in which they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a
+// piece of 4.  Of one (chunk, head): tiles 00, 10, 11 of (I + A)^-1 diag(beta) and of the weighted Q K^T, then
+// e^(b_t) | e^(b_last - b_t) | decay | beta.
+__host__ __device__ constexpr int64_t delta_frag_elems(int np) { return 3 * (int64_t)kDeltaChunk * np + 4; }
+constexpr int kDeltaHead = 6 * 256 + 4 * kDeltaChunk;
+
+// Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
+__device__ __forceinline__ bool delta_find_chunk(const DeltaArgs& a, int64_t idx, int& b, int64_t& c) {
+  const int lane = threadIdx.x & 63;
+  int64_t before = 0;
+  for (int r0 = 0; r0 < (int)a.batch; r0 += 64) {
+    const int n = r0 + lane < (int)a.batch ? max(0, (a.q_len[r0 + lane] + kDeltaChunk - 1) / kDeltaChunk) : 0;
+    int s = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(s, o, 64);
+      if (lane >= o) s += t;
+    }
+    const int total = __shfl(s, 63, 64);
+    if (idx < before + total) {
+      const uint64_t past = __ballot(before + s > idx);
+      const int first = __ffsll((unsigned long long)past) - 1;
+      b = r0 + first;
+      c = idx - before - (__shfl(s, first, 64) - __shfl(n, first, 64));
+      return true;
+    }
+    before += total;
+  }
+  return false;
+}
+// how many chunks the requests in front of b have
+__device__ __forceinline__ int64_t delta_chunks_before(const DeltaArgs& a, int b) {
+  const int lane = threadIdx.x & 63;
+  int s = 0;
+  for (int r = lane; r < b; r += 64) s += max(0, (a.q_len[r] + kDeltaChunk - 1) / kDeltaChunk);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
+__device__ __forceinline__ bool delta_finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+
+// silu: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal and one correction
+// of it and of the result: within an ulp of x / (1 + expf(-x)), 14 instructions in place of 30
+__device__ __forceinline__ float delta_silu_fast(float x) {
+  const float c = fmaxf(x, -87.f);
+  const float hi = c * -1.44269502f, lo = fmaf(c, -1.44269502f, -hi) + c * -1.92596299e-8f;
+  float e = __builtin_amdgcn_exp2f(hi);
+  e = fmaf(e, lo * 0.693147182f, e);
+  const float d = 1.0f + e;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float q = x * r;
+  return fmaf(fmaf(-d, q, x), r, q);
+}
+
+// A workgroup per (chunk, key head): convolution, silu and unit norm of its q and k (a channel per thread), K K^T and Q K^T, then
+// half a wave per head of the group: gates, A, its inverse column by column (lane = column, forward substitution), weights.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) {
+  constexpr int L = kDeltaChunk, CS = NP + 4, PS = L + 4;
+  __shared__ __attribute__((aligned(16))) float kq_l[2 * L * CS > 8 * L * L ? 2 * L * CS : 8 * L * L];     // K [32][CS] | Q; later A, one per half wave
+  __shared__ __attribute__((aligned(16))) float kk_l[L * PS], qk_l[L * PS];
+  __shared__ double cum_l[8 * L];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4, g = blockIdx.y;
+  int b;
+  int64_t ck;
+  if (!delta_find_chunk(a, blockIdx.x, b, ck)) return;
+  const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
+  if (first_pos < 0) return;
+  const int64_t l0 = ck * L, t0 = a.q_start[b] + l0;
+  const int cnt = (int)(n - l0 < L ? n - l0 : L);
+  const int D = a.D, taps = a.taps, C = 2 * a.G * D + a.H * a.E, per = a.H / a.G;
+  float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * delta_frag_elems(NP);
+  bool bad = false;
+  for (int ch = tid; ch < 2 * NP; ch += 256) {
+    const bool is_q = ch >= NP;
+    const int d = is_q ? ch - NP : ch;
+    float* dst = kq_l + (is_q ? L * CS : 0) + d;
+    if (d < D) {
+      const int cc = (is_q ? 0 : a.G * D) + g * D + d;                                      // channel in the state's order (q | k | v)
+      const T* p = (const T*)a.p + t0 * a.ld + (is_q ? a.q_off : a.k_off) + g * D + d;
+      const T* cw = (const T*)(is_q ? a.conv_q : a.conv_k) + (int64_t)(g * D + d) * taps;
+      float wt[kDeltaChunkTaps], in[kDeltaChunkTaps];
+#pragma unroll
+      for (int i = 0; i < kDeltaChunkTaps; ++i) {
+        wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
+        in[i] = 0.f;
+        if (i > 0 && i < taps) {
+          if (l0 - i >= 0) in[i] = Elem<T>::to_f(p[-(int64_t)i * a.ld]);
+          else if (first_pos > 0) in[i] = a.conv_state[a.state_indices[b] * a.conv_ld + (int64_t)(taps - 1 + l0 - i) * C + cc];
+        }
+      }
+      float x[L];
+      if (cnt == L) {
+#pragma unroll
+        for (int i = 0; i < L; ++i) x[i] = Elem<T>::to_f(p[(int64_t)i * a.ld]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < L; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < L; ++t) {
+        in[0] = x[t];
+        float y = 0.f;
+#pragma unroll
+        for (int i = 0; i < kDeltaChunkTaps; ++i)
+          if (i < taps) y += wt[i] * in[i];
+#pragma unroll
+        for (int i = kDeltaChunkTaps - 1; i > 0; --i) in[i] = in[i - 1];
+        const float z = delta_finite(y) ? delta_silu_fast(y) : (y > 0.f ? y : __builtin_nanf(""));
+        dst[t * CS] = t < cnt ? z : 0.f;
+      }
+    } else {
+      for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
+    }
+  }
+  __syncthreads();
+  // unit norms: four lanes a row
+  {
+    const int row = tid >> 2, part = tid & 3;                    // rows 0 .. 31: k, 32 .. 63: q
+    float* x = kq_l + (row >= L ? L * CS : 0) + (row % L) * CS;
+    float sq = 0.f;
+    for (int d = 4 * part; d < NP; d += 16) {
+      const float4 v = *reinterpret_cast<const float4*>(x + d);
+      sq += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
+    }
+    sq = quad_sum<4>(sq);
+    const float inv = (row >= L ? rsqrtf((float)D) : 1.0f) / sqrtf(sq + 1e-6f);
+    for (int d = 4 * part; d < NP; d += 16) {
+      float4 v = *reinterpret_cast<const float4*>(x + d);
+      v = float4{v.x * inv, v.y * inv, v.z * inv, v.w * inv};
+      *reinterpret_cast<float4*>(x + d) = v;
+      bad |= !delta_finite(v.x) || !delta_finite(v.y) || !delta_finite(v.z) || !delta_finite(v.w);
+    }
+  }
+  __syncthreads();
+  // the operands in the order in which they are held
+  for (int i = tid; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
+    const int half = i / (L * NP / 4), it = i % (L * NP / 4), tile = it >> 6, ln = it & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
+    *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(kq_l + half * L * CS + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
+  }
+  for (int i = tid; i < L * NP / 4; i += 256) {                  // K^T: tile (row of S, tokens)
+    const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
+    const float* s = kq_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
+    *reinterpret_cast<float4*>(frag + 2 * L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+  }
+  {
+    const int i0 = (w >> 1) * 16, j0 = (w & 1) * 16;
+    f32x4 kk = {}, qk = {};
+#pragma unroll 4
+    for (int k = 0; k < NP; k += 16) {
+      const f32x4 ak = *reinterpret_cast<const f32x4*>(kq_l + (i0 + r16) * CS + k + 4 * kq);
+      const f32x4 aq = *reinterpret_cast<const f32x4*>(kq_l + L * CS + (i0 + r16) * CS + k + 4 * kq);
+      const f32x4 bv = *reinterpret_cast<const f32x4*>(kq_l + (j0 + r16) * CS + k + 4 * kq);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        kk = __builtin_amdgcn_mfma_f32_16x16x4f32(ak[s], bv[s], kk, 0, 0, 0);
+        qk = __builtin_amdgcn_mfma_f32_16x16x4f32(aq[s], bv[s], qk, 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      kk_l[(i0 + 4 * kq + r) * PS + j0 + r16] = kk[r];
+      qk_l[(i0 + 4 * kq + r) * PS + j0 + r16] = qk[r];
+    }
+  }
+  __syncthreads();                                                // (kq_l is free from here on)
+  const int hw = tid >> 5, ln = tid & 31;
+  float* a_l = kq_l + hw * L * L;
+  double* cum = cum_l + hw * L;
+  for (int hh = hw; hh < per; hh += 8) {
+    const int h = g * per + hh;
+    const T* pr = (const T*)a.p + (t0 + ln) * a.ld;
+    const bool on = ln < cnt;
+    const float la = on ? -expf(a.a_log[h]) * softplus_f(Elem<T>::to_f(pr[a.a_off + h]) + a.dt_bias[h]) : 0.f;
+    const float beta = on ? sigmoid_f(Elem<T>::to_f(pr[a.b_off + h])) : 0.f;
+    double c = (double)la * 1.4426950408889634;
+#pragma unroll
+    for (int o = 1; o < L; o <<= 1) {
+      const double v = __shfl_up(c, o, L);
+      if (ln >= o) c += v;
+    }
+    const double last = __shfl(c, L - 1, L);
+    cum[ln] = c;
+    float* hp = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kDeltaHead;
+    const float eb = __builtin_amdgcn_exp2f((float)c), wt = __builtin_amdgcn_exp2f((float)(last - c)), dec = expf(la);
+    hp[1536 + ln] = eb;
+    hp[1536 + L + ln] = wt;
+    hp[1536 + 2 * L + ln] = dec;
+    hp[1536 + 3 * L + ln] = beta;
+    bad |= !delta_finite(eb) || !delta_finite(wt) || !delta_finite(dec) || !delta_finite(beta) || !delta_finite(la);
+    __builtin_amdgcn_wave_barrier();
+    // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s)
+    const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);
+    int lv = ln;
+    asm volatile("" : "+v"(lv));                                  // (rows of K K^T and Q K^T are read per head, not held for all of them)
+#pragma unroll 4
+    for (int t = 0; t < L; ++t) {
+      const float bt = __shfl(beta, t, L);
+      const float e = ln <= t ? __builtin_amdgcn_exp2f((float)(cum[t] - c)) : 0.f;
+      a_l[t * L + ln] = ln < t ? bt * (e * kk_l[t * PS + lv]) : 0.f;
+      if (t >= 16 || st == 0) hp[768 + ((t >> 4) + st) * 256 + sl + (t & 15) * 4] = ln <= t ? e * qk_l[t * PS + lv] : 0.f;
+    }
+    __builtin_amdgcn_wave_barrier();
+    // column ln of (I + A)^-1, four terms of a row at a time
+    float x[L];
+#pragma unroll
+    for (int t = 0; t < L; ++t) {
+      float acc = t == ln ? 1.f : 0.f;
+#pragma unroll
+      for (int s = 0; s < t; s += 4) {
+        const float4 av = *reinterpret_cast<const float4*>(a_l + t * L + s);
+        acc -= av.x * x[s];
+        if (s + 1 < t) acc -= av.y * x[s + 1];
+        if (s + 2 < t) acc -= av.z * x[s + 2];
+        if (s + 3 < t) acc -= av.w * x[s + 3];
+      }
+      x[t] = acc;
+      asm volatile("" : "+v"(x[t]));                             // (row by row: not all rows of A first and the sums behind them)
+    }
+#pragma unroll
+    for (int t = 0; t < L; ++t)
+      if (t >= 16 || st == 0) hp[((t >> 4) + st) * 256 + sl + (t & 15) * 4] = x[t] * beta;
+    __builtin_amdgcn_wave_barrier();
+  }
+  const int any_bad = __syncthreads_or(bad);
+  if (tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
+}
+
+// The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
+// sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, which is
+// also how the right-hand operand of a product over the rows is held, so S, R = V - e^b K S and U go from sums into products
+// without moving; v is convolved in its place by the lane that needs it.  Left-hand operands come straight into registers in the
+// order they are used, the next chunk's into the registers that this chunk has just read: no LDS, no barriers.
+template <typename T, int NP>
+__global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
+  constexpr int L = kDeltaChunk, NT = NP / 16, HALO = kDeltaChunkTaps - 1;
+  __shared__ float v_l[4][L * 16];                              // (token by token only: a wave's v)
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+  // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
+  const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
+  const int eblocks = (E + 63) / 64, members = per * eblocks;
+  const int turn = blockIdx.x / 8, unit = turn / members * 8 + blockIdx.x % 8;
+  if (unit >= (int)a.batch * G) return;
+  const int member = turn % members, b = unit / G, g = unit % G;
+  const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
+  const int n = a.q_len[b];
+  if (n <= 0 || first_pos < 0) return;
+  const int64_t chunk0 = delta_chunks_before(a, b);
+  if (chunk0 + (n + L - 1) / L > max_chunks) return;            // (requests that share rows: more rows than the launch has)
+  const int h = g * per + member / eblocks;
+  const int e0 = member % eblocks * 64 + 16 * w, e = e0 + r16;
+  if (e0 >= E) return;
+  const bool e_ok = e < E, wide = e0 + 16 <= E;
+  const int C = 2 * G * D + H * E;
+  const int64_t slot = a.state_indices[b];
+  float* st = a.state + slot * a.state_ld + (int64_t)h * D * E + e;
+  f32x4 S[NT];
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = 16 * t + 4 * kq + r;
+      S[t][r] = (first_pos > 0 && e_ok && row < D) ? st[row * E] : 0.f;
+    }
+  float wt[kDeltaChunkTaps];
+#pragma unroll
+  for (int i = 0; i < kDeltaChunkTaps; ++i)
+    wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_v)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
+  const int64_t frag_ld = (int64_t)G * delta_frag_elems(NP), head_ld = (int64_t)H * kDeltaHead;
+  const float* f = a.frags + chunk0 * frag_ld + g * delta_frag_elems(NP) + 4 * lane;
+  const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kDeltaHead;
+  const T* p = (const T*)a.p + t0 * a.ld + a.v_off + h * E + e0;
+  const uint32_t vo = (uint32_t)(4 * kq) * (uint32_t)a.ld + (e_ok ? r16 : 0);
+  float* yo = a.work + t0 * a.wld + 2 * G * D + h * E + e0;
+  const uint32_t yk = (uint32_t)(4 * kq) * (uint32_t)a.wld + r16;
+
+  // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
+  T vin[2][HALO + 4];
+  auto fetch_v = [&](int l0) {
+    const T* pr = p + (int64_t)(l0 - HALO) * a.ld;
+    if (wide && l0 + L <= n) {
+#pragma unroll
+      for (int r = 0; r < 16 + HALO + 4; ++r) {
+        if (r < HALO + 4) vin[0][r] = pr[vo];
+        if (r >= 16) vin[1][r - 16] = pr[vo];
+        pr += a.ld;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < HALO + 4; ++i) {
+          const int l = l0 + 16 * j + 4 * kq + i - HALO;
+          vin[j][i] = e_ok && l < n ? p[(int64_t)l * a.ld + r16] : Elem<T>::from_f(0.f);
+        }
+    }
+  };
+  // v of this lane's tokens, zero behind the portion; taps that the layer does not have see zeros
+  auto convolve = [&](const float (&x)[2][HALO + 4], int cnt, f32x4 (&v)[2], bool& bad) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        float y = wt[0] * x[j][s + HALO];
+#pragma unroll
+        for (int i = 1; i < kDeltaChunkTaps; ++i) y += wt[i] * __int_as_float(__float_as_int(x[j][s + HALO - i]) & (i < taps ? -1 : 0));
+        const bool ok = delta_finite(y), in = 16 * j + 4 * kq + s < cnt;     // (silu of infinity: itself; of minus infinity: inf / inf)
+        float z = delta_silu_fast(y);
+        asm volatile("" : "+v"(z));                              // (straight-line code: it goes between the products)
+        z = ok ? z : (y > 0.f ? y : __builtin_nanf(""));
+        v[j][s] = in ? z : 0.f;
+        bad |= in && !ok;
+      }
+  };
+  f32x4 v[2];
+  bool bad = false;
+  {
+    float x[2][HALO + 4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < HALO + 4; ++i) {
+        const int l = 16 * j + 4 * kq + i - HALO;
+        x[j][i] = 0.f;
+        if (e_ok && l < n) {
+          if (l >= 0) x[j][i] = Elem<T>::to_f(p[(int64_t)l * a.ld + r16]);
+          else if (first_pos > 0 && taps - 1 + l >= 0) x[j][i] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 + l) * C + 2 * G * D + h * E + e];
+        }
+      }
+    convolve(x, n, v, bad);
+  }
+  f32x4 K[2 * NT], Q[2 * NT], KT[2 * NT], Ti[3], M[3], eb[2], wv[2];
+  float flag;
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) K[i] = *reinterpret_cast<const f32x4*>(f + 256 * i);
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) Q[i] = *reinterpret_cast<const f32x4*>(f + L * NP + 256 * i);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    Ti[i] = *reinterpret_cast<const f32x4*>(fh + 256 * i + 4 * lane);
+    M[i] = *reinterpret_cast<const f32x4*>(fh + 768 + 256 * i + 4 * lane);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    eb[i] = *reinterpret_cast<const f32x4*>(fh + 1536 + 16 * i + 4 * kq);
+    wv[i] = *reinterpret_cast<const f32x4*>(fh + 1536 + L + 16 * i + 4 * kq);
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * NT; ++i) KT[i] = *reinterpret_cast<const f32x4*>(f + 2 * L * NP + 256 * i);
+  flag = f[3 * L * NP - 4 * lane];
+  if (L < n) fetch_v(L);
+
+  for (int l0 = 0; l0 < n; l0 += L) {
+    const int cnt = n - l0 < L ? n - l0 : L;
+    const bool more = l0 + L < n;
+    const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
+    const float* fhn = fh + (more ? head_ld : 0);
+    float* yr = yo + (int64_t)l0 * a.wld;
+    // An infinity or a NaN in the chunk would reach the tokens in front of it through a product with a weight of zero: the wave takes
+    // such a chunk token by token behind the products, which then count for nothing, from S in the state row and v in LDS (a rare
+    // path: it must not set the kernel's registers)
+    const bool serial = __any(bad || flag != 0.f);
+    int rows = D, step = E;
+    asm volatile("" : "+s"(rows), "+s"(step));
+    if (serial) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) v_l[w][(16 * j + 4 * kq + s) * 16 + r16] = v[j][s];
+      if (e_ok)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    {
+      const float keep = __shfl(eb[1][3], 63, 64);
+      f32x4 P[2] = {}, O[2] = {};
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) P[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(K[i * NT + t][s], S[t][s], P[i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2 * NT; ++i) K[i] = *reinterpret_cast<const f32x4*>(fn + 256 * i);
+      flag = fn[3 * L * NP - 4 * lane];
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Q[i * NT + t][s], S[t][s], O[i], 0, 0, 0);
+      // the next chunk's v between the products: a product keeps the matrix pipe for 32 cycles, in which a few of these fit
+      f32x4 vn[2];
+      bad = false;
+      {
+        float x[2][HALO + 4];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < HALO + 4; ++i) x[j][i] = Elem<T>::to_f(vin[j][i]);
+        convolve(x, n - l0 - L, vn, bad);
+      }
+#pragma unroll
+      for (int i = 0; i < 8 * NT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < 2 * NT; ++i) Q[i] = *reinterpret_cast<const f32x4*>(fn + L * NP + 256 * i);
+      if (l0 + 2 * L < n) fetch_v(l0 + 2 * L);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        v[i] -= eb[i] * P[i];
+        O[i] *= eb[i];
+      }
+      f32x4 U[2] = {};
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) U[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ti[i][s], v[0][s], U[i], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) U[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ti[2][s], v[1][s], U[1], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[i][s], U[0][s], O[i], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) O[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[2][s], U[1][s], O[1], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) U[i] *= wv[i];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        Ti[i] = *reinterpret_cast<const f32x4*>(fhn + 256 * i + 4 * lane);
+        M[i] = *reinterpret_cast<const f32x4*>(fhn + 768 + 256 * i + 4 * lane);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        eb[i] = *reinterpret_cast<const f32x4*>(fhn + 1536 + 16 * i + 4 * kq);
+        wv[i] = *reinterpret_cast<const f32x4*>(fhn + 1536 + L + 16 * i + 4 * kq);
+      }
+      if (serial) {
+      } else if (cnt == L && wide) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) (yr + (int64_t)(16 * i + r) * a.wld)[yk] = O[i][r];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * i + 4 * kq + r < cnt && e_ok) (yr + (int64_t)(16 * i + r) * a.wld)[yk] = O[i][r];
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] *= keep;
+#pragma unroll
+      for (int t = 0; t < NT; t += 2)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) S[t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[2 * (t + i) + k][s], U[k][s], S[t + i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2 * NT; ++i) KT[i] = *reinterpret_cast<const f32x4*>(fn + 2 * L * NP + 256 * i);
+      v[0] = vn[0];
+      v[1] = vn[1];
+    }
+    if (serial) {
+#pragma unroll 1
+      for (int t = 0; t < cnt; ++t) {
+        // row t of K (tile row t / 16, lane r16 = t % 16): this lane group's four of every 16
+        const float* kr = f - 4 * lane + (t >> 4) * NT * 256 + 4 * (16 * kq + (t & 15));
+        float dk = 0.f, dq = 0.f, kd = 0.f;
+#pragma unroll 1
+        for (int u = 0; u < 4 * NT; ++u) {
+          const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
+          if (row < rows) {
+            const float kv = kr[(u >> 2) * 256 + (u & 3)], qv = kr[L * NP + (u >> 2) * 256 + (u & 3)], sv = e_ok ? st[row * step] : 0.f;
+            dk += sv * kv;
+            dq += sv * qv;
+            kd += kv * qv;
+          }
+        }
+        dk += __shfl_xor(dk, 16, 64);
+        dk += __shfl_xor(dk, 32, 64);
+        dq += __shfl_xor(dq, 16, 64);
+        dq += __shfl_xor(dq, 32, 64);
+        kd += __shfl_xor(kd, 16, 64);
+        kd += __shfl_xor(kd, 32, 64);
+        const float gt = fh[1536 + 2 * L + t], bt = fh[1536 + 3 * L + t];
+        const float u1 = bt * (v_l[w][t * 16 + r16] - gt * dk);
+#pragma unroll 1
+        for (int u = 0; u < 4 * NT; ++u) {
+          const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
+          if (row < rows && e_ok) st[row * step] = gt * st[row * step] + kr[(u >> 2) * 256 + (u & 3)] * u1;
+        }
+        if (kq == 0 && e_ok) yr[(int64_t)t * a.wld + r16] = gt * dq + u1 * kd;
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          S[t][r] = e_ok && 16 * t + 4 * kq + r < rows ? st[(16 * t + 4 * kq + r) * step] : 0.f;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    f = fn;
+    fh = fhn;
+  }
+  int rows = D, step = E;
+  asm volatile("" : "+s"(rows), "+s"(step));                     // (no addresses of 32 rows held over the loop)
+  if (e_ok)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
+}
+
+// The same with 16-byte accesses: a head is taken by LP = E / 8 lanes (a power of two), 64 / LP heads per wave.  Bound by HBM: 7262
+// tokens of 32 heads of 128, 238 MB: 84 us -> 44.
+template <typename T, int LP>
+__global__ void __launch_bounds__(256) delta_post_vec_kernel(DeltaArgs a) {
+  const int lane = threadIdx.x & 63, sl = lane % LP, E = a.E;
+  const int64_t item = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LP) + lane / LP;
+  const bool on = item < a.num_tokens * a.H;
+  const int64_t t = on ? item / a.H : 0;
+  const int h = on ? (int)(item % a.H) : 0;
+  const float* o = a.work + t * a.wld + 2 * a.G * a.D + (int64_t)h * E + sl * 8;
+  const float4 o0 = *reinterpret_cast<const float4*>(o), o1 = *reinterpret_cast<const float4*>(o + 4);
+  const Vec16<T> gate = load16((const T*)a.p + t * a.ld + a.gate_off + (int64_t)h * E + sl * 8), nw = load16((const T*)a.norm_w + sl * 8);
+  const float x[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+  float sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sq += x[i] * x[i];
+#pragma unroll
+  for (int m = LP / 2; m > 0; m >>= 1) sq += __shfl_xor(sq, m, 64);
+  if (!on) return;
+  const float inv = 1.0f / sqrtf(sq / (float)E + a.eps);
+  Vec16<T> r;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) r.e[i] = Elem<T>::from_f(x[i] * inv * Elem<T>::to_f(nw.e[i]) * silu_f(Elem<T>::to_f(gate.e[i])));
+  store16((T*)a.out + t * a.out_ld + (int64_t)h * E + sl * 8, r);
+}
+
 }  // namespace semipd
 
 using namespace semipd;
@@ -475,13 +1047,60 @@ extern "C" int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, 
   return (w + 3) / 4 * 4;
 }
 
-extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
+// The rows per request (on average) from which a prompt batch goes in chunks.  Token by token against chunks, whole call, 32 heads of
+// 128 x 128: 1 request of 2 rows 51 / 43 us, 64 rows 96 / 54, 256 rows 251 / 92; 4 requests of 2 rows 53 / 44; 32 requests of 8 rows
+// 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; heads of 64 x 64: 4 requests of 2 rows 49 / 37, 32 requests of 8 rows 60 / 78, 16 rows
+// 82 / 83, 64 rows 200 / 134.  A few requests take chunks whatever their length.
+constexpr int64_t kDeltaChunkMinRows = 16, kDeltaChunkFewRequests = 4;
+static int64_t delta_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kDeltaChunk + batch; }
+
+extern "C" int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps) {
+  if (batch <= 0 || num_heads <= 0 || num_k_heads <= 0 || (batch > kDeltaChunkFewRequests && num_tokens < kDeltaChunkMinRows * batch) || k_dim > 128 || taps > kDeltaChunkTaps) return 0;
+  return delta_max_chunks(num_tokens, batch) * (num_k_heads * delta_frag_elems(k_dim <= 64 ? 64 : 128) + (int64_t)num_heads * kDeltaHead);
+}
+
+template <typename T, int NP>
+static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
+  const int64_t chunks = delta_max_chunks(a.num_tokens, a.batch);
+  hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
+  const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
+  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);
+}
+
+// gate and norm; 16-byte accesses where a head is a power of two of pieces and everything starts on one
+static int launch_delta_post(const DeltaArgs& a, int dtype, hipStream_t s) {
+  const int lp = a.E / 8;
+  const bool vec = dtype != SEMIPD_F32 && a.E % 8 == 0 && lp <= 64 && (lp & (lp - 1)) == 0 && a.gate_off % 8 == 0 && a.ld % 8 == 0 &&
+                   a.out_ld % 8 == 0 && a.wld % 4 == 0 && (2 * a.G * a.D) % 4 == 0 && aligned16(a.p) && aligned16(a.out) && aligned16(a.work) &&
+                   aligned16(a.norm_w);
+  if (!vec) {
+    SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_post_kernel<T>), dim3((unsigned)a.num_tokens), dim3(256), 0, s, a));
+    return 0;
+  }
+  const int64_t items = a.num_tokens * a.H, per = 4 * (64 / lp);
+  const dim3 grid((unsigned)((items + per - 1) / per));
+  SEMIPD_DISPATCH_HALF(dtype, T, {
+    switch (lp) {
+      case 1: hipLaunchKernelGGL((delta_post_vec_kernel<T, 1>), grid, dim3(256), 0, s, a); break;
+      case 2: hipLaunchKernelGGL((delta_post_vec_kernel<T, 2>), grid, dim3(256), 0, s, a); break;
+      case 4: hipLaunchKernelGGL((delta_post_vec_kernel<T, 4>), grid, dim3(256), 0, s, a); break;
+      case 8: hipLaunchKernelGGL((delta_post_vec_kernel<T, 8>), grid, dim3(256), 0, s, a); break;
+      case 16: hipLaunchKernelGGL((delta_post_vec_kernel<T, 16>), grid, dim3(256), 0, s, a); break;
+      case 32: hipLaunchKernelGGL((delta_post_vec_kernel<T, 32>), grid, dim3(256), 0, s, a); break;
+      default: hipLaunchKernelGGL((delta_post_vec_kernel<T, 64>), grid, dim3(256), 0, s, a); break;
+    }
+  });
+  return 0;
+}
+
+static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
                                  int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
                                  const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
                                  int64_t work_ld, float* state, int64_t state_ld, float* conv_state, int64_t conv_ld,
                                  const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
                                  const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
-                                 int k_dim, int v_dim, int taps, void* out, int64_t out_ld, int dtype, void* stream) {
+                                 int k_dim, int v_dim, int taps, void* out, int64_t out_ld, float* chunk_work, int64_t chunk_elems,
+                      int dtype, void* stream) {
   SEMIPD_CHECK_ARG(batch >= 0 && num_tokens >= 0, SEMIPD_EINVAL, "delta_rule: bad sizes");
   if (batch == 0 || num_tokens == 0) return 0;
   SEMIPD_CHECK_ARG(num_heads > 0 && num_k_heads > 0 && num_heads % num_k_heads == 0, SEMIPD_ESHAPE,
@@ -499,7 +1118,7 @@ extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, in
                    SEMIPD_EINVAL, "delta_rule: a row of the work buffer, the state or the output is too short");
   DeltaArgs a{proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight,
               work, work_ld, state, state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens,
-              num_heads, num_k_heads, k_dim, v_dim, taps, eps, out, out_ld};
+              num_heads, num_k_heads, k_dim, v_dim, taps, eps, out, out_ld, chunk_work};
   hipStream_t st = as_stream(stream);
   // lanes per column and rows of S per lane: four lanes share a column from 32 rows up
   const int ds = k_dim >= 32 ? 4 : 1;
@@ -533,6 +1152,15 @@ extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, in
                                                          dim3(256), 0, st, a));
     return launch_status("delta_rule(decode)");
   }
+  const int64_t want = q_start ? semipd_delta_rule_chunk_elems(num_tokens, batch, num_heads, num_k_heads, k_dim, taps) : 0;
+  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work)) {
+    SEMIPD_DISPATCH_DTYPE(dtype, T, if (k_dim <= 64) launch_delta_chunks<T, 64>(a, st); else launch_delta_chunks<T, 128>(a, st));
+    if (taps > 1)
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch),
+                                                         dim3(256), 0, st, a));
+    if (launch_delta_post(a, dtype, st)) return SEMIPD_EDTYPE;
+    return launch_status("delta_rule(chunks)");
+  }
   SEMIPD_DISPATCH_DTYPE(dtype, T, {
     hipLaunchKernelGGL((delta_prep_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, st, a);
     if (taps > 1)
@@ -561,7 +1189,30 @@ extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, in
     }
   }
 #undef SEMIPD_DELTA_SCAN
-  SEMIPD_DISPATCH_DTYPE(dtype, T,
-                        hipLaunchKernelGGL((delta_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, st, a));
+  if (launch_delta_post(a, dtype, st)) return SEMIPD_EDTYPE;
   return launch_status("delta_rule");
+}
+
+extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
+                                 int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
+                                 const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
+                                 int64_t work_ld, float* state, int64_t state_ld, float* conv_state, int64_t conv_ld,
+                                 const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
+                                 const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
+                                 int k_dim, int v_dim, int taps, void* out, int64_t out_ld, int dtype, void* stream) {
+  return delta_rule(proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, eps, work, work_ld,
+                    state, state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, num_k_heads, k_dim,
+                    v_dim, taps, out, out_ld, nullptr, 0, dtype, stream);
+}
+
+extern "C" int semipd_delta_rule_prompt(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
+                                 int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
+                                 const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
+                                 int64_t work_ld, float* state, int64_t state_ld, float* conv_state, int64_t conv_ld,
+                                 const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
+                                 const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
+                                 int k_dim, int v_dim, int taps, void* out, int64_t out_ld, float* chunk_work, int64_t chunk_elems, int dtype, void* stream) {
+  return delta_rule(proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, eps, work, work_ld,
+                    state, state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, num_k_heads, k_dim,
+                    v_dim, taps, out, out_ld, chunk_work, chunk_elems, dtype, stream);
 }

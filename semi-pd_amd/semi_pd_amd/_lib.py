@@ -171,6 +171,9 @@ _SIGNATURES = {
                                 _i32, _f32, _vp, _i32, _vp, _i32, _i32, _vp],
     "semipd_delta_rule": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _i64,
                           _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
+    "semipd_delta_rule_chunk_elems": [_i64, _i64, _i32, _i32, _i32, _i32],
+    "semipd_delta_rule_prompt": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _i64,
+                          _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64, _i32, _vp],
     "semipd_delta_rule_work_width": [_i32, _i32, _i32, _i32],
     "semipd_clamped_glu": [_vp, _i64, _vp, _i64, _i64, _i64, _i32, _vp, _vp, _i32, _f32, _f32, _i32, _vp],
     "semipd_topk_sigmoid": [_vp, _vp, _vp, _i64, _i32, _i32, _i32, _f32, _i32, _vp],
@@ -213,7 +216,7 @@ _SIGNATURES = {
 _RESTYPES = {"semipd_last_error": C.c_char_p, "semipd_lm_head_argmax_workspace": _sz,
              "semipd_linear_workspace": _sz, "semipd_stream_linear_workspace": _sz, "semipd_dense_gemm_report": _sz, "semipd_ar_meta_size": _sz, "semipd_ar_region_size": _sz,
              "semipd_matrix_memory_workspace": _i64, "semipd_linear_attention_workspace": _i64, "semipd_matrix_memory_state_width": _i64,
-             "semipd_min_gru_workspace": _i64, "semipd_delta_rule_work_width": _i64, "semipd_state_space_work_width": _i64,
+             "semipd_min_gru_workspace": _i64, "semipd_delta_rule_work_width": _i64, "semipd_delta_rule_chunk_elems": _i64, "semipd_state_space_work_width": _i64,
              "semipd_state_space_chunk_elems": _i64}
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)

@@ -1747,11 +1747,16 @@ def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.
     lib = _lib.load()
     wld = int(lib.semipd_delta_rule_work_width(num_heads, num_k_heads, k_dim, v_dim))
     work = torch.empty((T, wld), dtype=torch.float32, device=proj.device)
-    check(lib.semipd_delta_rule(ptr(proj), proj.stride(0), *[int(o) for o in offsets], ptr(conv_q), ptr(conv_k), ptr(conv_v),
-                                ptr(a_log), ptr(dt_bias), ptr(norm_weight), float(eps), ptr(work), wld, ptr(state), state.stride(0),
-                                ptr(conv_state), conv_state.stride(0) if conv_state is not None else 0, ptr(state_indices),
-                                ptr(seq_lens), ptr(q_start), ptr(q_len), B, T, num_heads, num_k_heads, k_dim, v_dim, taps, ptr(out),
-                                out.stride(0), dtype_code(proj.dtype), current_stream(proj.device)), "delta_rule")
+    args = (ptr(proj), proj.stride(0), *[int(o) for o in offsets], ptr(conv_q), ptr(conv_k), ptr(conv_v), ptr(a_log), ptr(dt_bias),
+            ptr(norm_weight), float(eps), ptr(work), wld, ptr(state), state.stride(0), ptr(conv_state),
+            conv_state.stride(0) if conv_state is not None else 0, ptr(state_indices), ptr(seq_lens), ptr(q_start), ptr(q_len), B, T,
+            num_heads, num_k_heads, k_dim, v_dim, taps, ptr(out), out.stride(0))
+    elems = int(lib.semipd_delta_rule_chunk_elems(T, B, num_heads, num_k_heads, k_dim, taps)) if q_start is not None else 0
+    if elems:         # a prompt batch: room for the operands of its chunks of 32 tokens
+        chunk_work = torch.empty(elems, dtype=torch.float32, device=proj.device)
+        check(lib.semipd_delta_rule_prompt(*args, ptr(chunk_work), elems, dtype_code(proj.dtype), current_stream(proj.device)), "delta_rule")
+    else:
+        check(lib.semipd_delta_rule(*args, dtype_code(proj.dtype), current_stream(proj.device)), "delta_rule")
     return out
 
 

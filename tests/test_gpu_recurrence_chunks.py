@@ -115,3 +115,106 @@ def test_state_space_in_chunks_not_finite(col, value):
     torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
     if col != "dt" or value != value:
         assert not bool(torch.isfinite(got[0][at:]).all())
+
+
+# ----------------------------------------------------------------------------------------------- gated delta rule
+def _delta_inputs(H, G, D, E, taps, lens, dtype, seed, scale=1.0):
+    g = torch.Generator().manual_seed(seed)
+    gd, hv = G * D, H * E
+    w = dict(cq=(0.5 * torch.randn(gd, taps, generator=g)).to(dtype), ck=(0.5 * torch.randn(gd, taps, generator=g)).to(dtype),
+             cv=(0.5 * torch.randn(hv, taps, generator=g)).to(dtype), a_log=0.5 * torch.randn(H, generator=g) - 1 + (scale > 1) * 2.0,
+             dt_bias=0.5 * torch.randn(H, generator=g), norm=(1 + 0.1 * torch.randn(E, generator=g)).to(dtype))
+    rows = [(scale * torch.randn(n, 2 * gd + 2 * hv + 2 * H, generator=g)).to(dtype) for n in lens]
+    return w, rows, 0.3 * torch.randn(len(lens), H, D, E, generator=g), torch.randn(len(lens), taps - 1, 2 * gd + hv, generator=g)
+
+
+def _delta_truth(w, row, state, before, H, G, D, E, eps=1e-5):
+    gd, hv = G * D, H * E
+    x = row.to(F64)
+    y, last = _conv_silu(x[:, : 2 * gd + hv], torch.cat([w["cq"], w["ck"], w["cv"]]).to(F64), None, before.to(F64))
+    q, k, v = y.split([gd, gd, hv], 1)
+    n = x.shape[0]
+    q, k = (z.view(n, G, D) / (z.view(n, G, D).square().sum(-1, keepdim=True) + 1e-6).sqrt() for z in (q, k))
+    q, k, v = (q * D ** -0.5).repeat_interleave(H // G, 1), k.repeat_interleave(H // G, 1), v.view(n, H, E)
+    a, b = x[:, 2 * gd + 2 * hv: 2 * gd + 2 * hv + H], x[:, 2 * gd + 2 * hv + H:]
+    dec = torch.exp(-torch.exp(w["a_log"].to(F64)) * torch.nn.functional.softplus(a + w["dt_bias"].to(F64)))
+    S, o = state.to(F64).clone(), []
+    for t in range(n):
+        S = dec[t][:, None, None] * S
+        u = torch.sigmoid(b[t])[:, None] * (v[t] - (k[t][:, None] @ S).squeeze(1))
+        S = S + k[t][:, :, None] * u[:, None]
+        o.append((q[t][:, None] @ S).squeeze(1))
+    o = torch.stack(o)
+    o = o / (o.square().mean(-1, keepdim=True) + eps).sqrt() * w["norm"].to(F64)
+    return o.reshape(n, hv) * torch.nn.functional.silu(x[:, 2 * gd + hv: 2 * gd + 2 * hv]), S, last
+
+
+def _delta_run(w, rows, state, before, first, H, G, D, E, eps=1e-5):
+    from semi_pd_amd import ops
+    gd, hv, taps, B = G * D, H * E, w["cq"].shape[1], len(rows)
+    lens = [r.shape[0] for r in rows]
+    sw, cw = H * D * E, (taps - 1) * (2 * gd + hv)
+    slab = torch.full((B + 1, 3 + sw + cw + 2), 7.0, device=DEV)
+    slab[1:, 3: 3 + sw] = state.reshape(B, -1).to(DEV)
+    slab[1:, 3 + sw: 3 + sw + cw] = before.reshape(B, -1).to(DEV)
+    start, at = [], 0
+    for n in lens:
+        start.append(at)
+        at += n
+    d = {k: v.to(DEV) for k, v in w.items()}
+    offs = [0, gd, 2 * gd, 2 * gd + hv, 2 * gd + 2 * hv, 2 * gd + 2 * hv + H]
+    out = ops.delta_rule(torch.cat(rows).to(DEV), offs, d["cq"], d["ck"], d["cv"], d["a_log"], d["dt_bias"], d["norm"], eps, slab[:, 3: 3 + sw],
+                         slab[:, 3 + sw: 3 + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
+                         torch.tensor([n + f for n, f in zip(lens, first)], device=DEV), torch.tensor(start, dtype=torch.int32, device=DEV),
+                         torch.tensor(lens, dtype=torch.int32, device=DEV), H, G, D, E)
+    slab = slab.cpu()
+    assert bool((slab[0] == 7).all() and (slab[:, :3] == 7).all() and (slab[:, -2:] == 7).all())
+    return out.cpu().split(lens), slab[1:, 3: 3 + sw].view(B, H, D, E), slab[1:, 3 + sw: 3 + sw + cw].view(B, taps - 1, 2 * gd + hv)
+
+
+# (rows of S in, at and below a padded block; columns over part of a wave, one and two workgroups, odd; more heads than half waves)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,D,E,taps,lens", [(4, 2, 128, 128, 4, [64, 1, 130]), (6, 2, 40, 40, 2, [63, 65]), (3, 1, 7, 72, 1, [31, 33]),
+                                               (2, 2, 65, 7, 3, [16, 200]), (9, 1, 64, 16, 4, [32, 70])])
+def test_delta_rule_in_chunks(dtype, H, G, D, E, taps, lens):
+    """Fresh sequences and portions (every second request) in one launch; tolerances as above."""
+    first = [0 if i % 2 == 0 else 37 for i in range(len(lens))]
+    w, rows, state, before = _delta_inputs(H, G, D, E, taps, lens, dtype, H * 131 + E)
+    outs, after, last = _delta_run(w, rows, state, before, first, H, G, D, E)
+    ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for b, n in enumerate(lens):
+        want, S, tail = _delta_truth(w, rows[b], state[b] if first[b] else torch.zeros_like(state[b]),
+                                     before[b] if first[b] else torch.zeros_like(before[b]), H, G, D, E)
+        torch.testing.assert_close(outs[b].to(F64), want, rtol=ulp + 2e-5, atol=2e-5)
+        torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+
+
+def test_delta_rule_in_chunks_repeated_keys():
+    """One key for all tokens, written in full (beta near 1) and kept (decay near 1): the system to invert is as far from the identity as
+    it gets, and every token must replace what the one in front of it wrote."""
+    H, G, D, E, lens = 4, 2, 64, 32, [100]
+    w, rows, state, before = _delta_inputs(H, G, D, E, 1, lens, torch.float32, 8)
+    gd, hv = G * D, H * E
+    rows[0][:, gd: 2 * gd] = rows[0][0, gd: 2 * gd]
+    rows[0][:, 2 * gd + 2 * hv:] = torch.cat([torch.full((H,), -12.0), torch.full((H,), 12.0)])
+    outs, after, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    want, S, _ = _delta_truth(w, rows[0], state[0], before[0], H, G, D, E)
+    assert float((outs[0].to(F64) - want).norm() / want.norm()) < 3e-6
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 3e-6
+
+
+@pytest.mark.parametrize("col", ["k", "v", "a"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_delta_rule_in_chunks_not_finite(col, value):
+    H, G, D, E, lens, at = 4, 2, 32, 24, [100, 100], 90
+    gd, hv = G * D, H * E
+    w, rows, state, before = _delta_inputs(H, G, D, E, 1, lens, torch.float32, 6)
+    clean, _, _ = _delta_run(w, rows, state, before, [0, 9], H, G, D, E)
+    c = {"k": gd + 3, "v": 2 * gd + 1, "a": 2 * gd + 2 * hv}[col]
+    rows[0][at, c] = value
+    got, _, _ = _delta_run(w, rows, state, before, [0, 9], H, G, D, E)
+    torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
+    torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
+    if col != "a" or value != value:
+        assert not bool(torch.isfinite(got[0][at:]).all())
