@@ -1004,7 +1004,7 @@ int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
                        const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int groups, int state_size, int v_dim,
                        int taps, void* out, int64_t out_ld, int fused_decode, int dtype, void* stream);
 /* fp32 elements that semipd_state_space_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
-int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state, int v_dim, int taps);
+int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state, int taps);
 /* semipd_state_space of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a
  * time on the matrix cores in fp32.  Without room, or where sizes or alignment do not allow it: as semipd_state_space. */
 int semipd_state_space_prompt(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,

@@ -22,7 +22,7 @@
 //  * delta_post_kernel / delta_post_vec_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
 //  * delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, head).
 #include "common.h"
-#include "mfma_frag.h"
+#include "recurrent_chunks.h"
 
 namespace semipd {
 
@@ -481,80 +481,29 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
 // differences are taken, in 64 bits.
 // Bound: token by token a step is a chain of two dot products, a lane sum and an update (0.8 us; 7262 tokens of 4 requests, 32 heads of
 // 128 x 128: 1861 us + 317 of preparation); in chunks a wave's chain of 216 products of 32 cycles a chunk (72 chunks: 207 us, one
-// wave a SIMD at 4 requests): 390 us, operands 91.  With the raw inputs of v fetched at the end of a chunk and convolved in
-// front of the products 483 (the loads of 35 rows 24 KB apart were waited for): they are fetched a whole chunk ahead.
-constexpr int kDeltaChunk = 32;
-constexpr int kDeltaChunkTaps = 4;        // taps at most
+// wave a SIMD at 4 requests): 370 us, operands 91.  With the raw inputs of v fetched at the end of a chunk and convolved in
+// front of the products 483 (the loads of 35 rows 24 KB apart were waited for), fetched a whole chunk ahead 390, by 16 bytes a lane
+// through the wave's LDS 370.
 
 // fp32 elements of the operands of one (chunk, key head): K, Q and K^T as left-hand operands of 16 x 16 x 16 products, the
 // order in which they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a
 // piece of 4.  Of one (chunk, head): tiles 00, 10, 11 of (I + A)^-1 diag(beta) and of the weighted Q K^T, then
 // e^(b_t) | e^(b_last - b_t) | decay | beta.
-__host__ __device__ constexpr int64_t delta_frag_elems(int np) { return 3 * (int64_t)kDeltaChunk * np + 4; }
-constexpr int kDeltaHead = 6 * 256 + 4 * kDeltaChunk;
-
-// Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
-__device__ __forceinline__ bool delta_find_chunk(const DeltaArgs& a, int64_t idx, int& b, int64_t& c) {
-  const int lane = threadIdx.x & 63;
-  int64_t before = 0;
-  for (int r0 = 0; r0 < (int)a.batch; r0 += 64) {
-    const int n = r0 + lane < (int)a.batch ? max(0, (a.q_len[r0 + lane] + kDeltaChunk - 1) / kDeltaChunk) : 0;
-    int s = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(s, o, 64);
-      if (lane >= o) s += t;
-    }
-    const int total = __shfl(s, 63, 64);
-    if (idx < before + total) {
-      const uint64_t past = __ballot(before + s > idx);
-      const int first = __ffsll((unsigned long long)past) - 1;
-      b = r0 + first;
-      c = idx - before - (__shfl(s, first, 64) - __shfl(n, first, 64));
-      return true;
-    }
-    before += total;
-  }
-  return false;
-}
-// how many chunks the requests in front of b have
-__device__ __forceinline__ int64_t delta_chunks_before(const DeltaArgs& a, int b) {
-  const int lane = threadIdx.x & 63;
-  int s = 0;
-  for (int r = lane; r < b; r += 64) s += max(0, (a.q_len[r] + kDeltaChunk - 1) / kDeltaChunk);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  return s;
-}
-
-__device__ __forceinline__ bool delta_finite(float x) { return fabsf(x) <= 3.402823466e38f; }
-
-// silu: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal and one correction
-// of it and of the result: within an ulp of x / (1 + expf(-x)), 14 instructions in place of 30
-__device__ __forceinline__ float delta_silu_fast(float x) {
-  const float c = fmaxf(x, -87.f);
-  const float hi = c * -1.44269502f, lo = fmaf(c, -1.44269502f, -hi) + c * -1.92596299e-8f;
-  float e = __builtin_amdgcn_exp2f(hi);
-  e = fmaf(e, lo * 0.693147182f, e);
-  const float d = 1.0f + e;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.0f), r, r);
-  const float q = x * r;
-  return fmaf(fmaf(-d, q, x), r, q);
-}
+__host__ __device__ constexpr int64_t delta_frag_elems(int np) { return 3 * (int64_t)kRecChunk * np + 4; }
+constexpr int kDeltaHead = 6 * 256 + 4 * kRecChunk;
 
 // A workgroup per (chunk, key head): convolution, silu and unit norm of its q and k (a channel per thread), K K^T and Q K^T, then
 // half a wave per head of the group: gates, A, its inverse column by column (lane = column, forward substitution), weights.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) {
-  constexpr int L = kDeltaChunk, CS = NP + 4, PS = L + 4;
+  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4;
   __shared__ __attribute__((aligned(16))) float kq_l[2 * L * CS > 8 * L * L ? 2 * L * CS : 8 * L * L];     // K [32][CS] | Q; later A, one per half wave
   __shared__ __attribute__((aligned(16))) float kk_l[L * PS], qk_l[L * PS];
   __shared__ double cum_l[8 * L];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4, g = blockIdx.y;
   int b;
   int64_t ck;
-  if (!delta_find_chunk(a, blockIdx.x, b, ck)) return;
+  if (!rec_find_chunk(a.q_len, (int)a.batch, blockIdx.x, b, ck)) return;
   const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
   if (first_pos < 0) return;
   const int64_t l0 = ck * L, t0 = a.q_start[b] + l0;
@@ -570,9 +519,9 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
       const int cc = (is_q ? 0 : a.G * D) + g * D + d;                                      // channel in the state's order (q | k | v)
       const T* p = (const T*)a.p + t0 * a.ld + (is_q ? a.q_off : a.k_off) + g * D + d;
       const T* cw = (const T*)(is_q ? a.conv_q : a.conv_k) + (int64_t)(g * D + d) * taps;
-      float wt[kDeltaChunkTaps], in[kDeltaChunkTaps];
+      float wt[kRecTaps], in[kRecTaps];
 #pragma unroll
-      for (int i = 0; i < kDeltaChunkTaps; ++i) {
+      for (int i = 0; i < kRecTaps; ++i) {
         wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
         in[i] = 0.f;
         if (i > 0 && i < taps) {
@@ -593,12 +542,11 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
         in[0] = x[t];
         float y = 0.f;
 #pragma unroll
-        for (int i = 0; i < kDeltaChunkTaps; ++i)
+        for (int i = 0; i < kRecTaps; ++i)
           if (i < taps) y += wt[i] * in[i];
 #pragma unroll
-        for (int i = kDeltaChunkTaps - 1; i > 0; --i) in[i] = in[i - 1];
-        const float z = delta_finite(y) ? delta_silu_fast(y) : (y > 0.f ? y : __builtin_nanf(""));
-        dst[t * CS] = t < cnt ? z : 0.f;
+        for (int i = kRecTaps - 1; i > 0; --i) in[i] = in[i - 1];
+        dst[t * CS] = t < cnt ? rec_silu_or_not_finite(y, rec_silu(y)) : 0.f;
       }
     } else {
       for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
@@ -620,7 +568,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
       float4 v = *reinterpret_cast<const float4*>(x + d);
       v = float4{v.x * inv, v.y * inv, v.z * inv, v.w * inv};
       *reinterpret_cast<float4*>(x + d) = v;
-      bad |= !delta_finite(v.x) || !delta_finite(v.y) || !delta_finite(v.z) || !delta_finite(v.w);
+      bad |= !rec_finite(v.x) || !rec_finite(v.y) || !rec_finite(v.z) || !rec_finite(v.w);
     }
   }
   __syncthreads();
@@ -673,12 +621,12 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
     const double last = __shfl(c, L - 1, L);
     cum[ln] = c;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kDeltaHead;
-    const float eb = __builtin_amdgcn_exp2f((float)c), wt = __builtin_amdgcn_exp2f((float)(last - c)), dec = expf(la);
+    const float eb = rec_exp2(c), wt = rec_exp2(last - c), dec = expf(la);
     hp[1536 + ln] = eb;
     hp[1536 + L + ln] = wt;
     hp[1536 + 2 * L + ln] = dec;
     hp[1536 + 3 * L + ln] = beta;
-    bad |= !delta_finite(eb) || !delta_finite(wt) || !delta_finite(dec) || !delta_finite(beta) || !delta_finite(la);
+    bad |= !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_finite(la);
     __builtin_amdgcn_wave_barrier();
     // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s)
     const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);
@@ -687,7 +635,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
 #pragma unroll 4
     for (int t = 0; t < L; ++t) {
       const float bt = __shfl(beta, t, L);
-      const float e = ln <= t ? __builtin_amdgcn_exp2f((float)(cum[t] - c)) : 0.f;
+      const float e = ln <= t ? rec_exp2(cum[t] - c) : 0.f;
       a_l[t * L + ln] = ln < t ? bt * (e * kk_l[t * PS + lv]) : 0.f;
       if (t >= 16 || st == 0) hp[768 + ((t >> 4) + st) * 256 + sl + (t & 15) * 4] = ln <= t ? e * qk_l[t * PS + lv] : 0.f;
     }
@@ -724,8 +672,9 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
 // order they are used, the next chunk's into the registers that this chunk has just read: no LDS, no barriers.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
-  constexpr int L = kDeltaChunk, NT = NP / 16, HALO = kDeltaChunkTaps - 1;
-  __shared__ float v_l[4][L * 16];                              // (token by token only: a wave's v)
+  constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
+  __shared__ __attribute__((aligned(16))) T in_l[4][RowTile<T>::kElems];       // a wave's own: raw inputs of its convolution
+  __shared__ __attribute__((aligned(16))) float o_l[4][L * kOutStride];         // ... results on their way out (token by token: its v)
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
   // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
@@ -736,7 +685,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
-  const int64_t chunk0 = delta_chunks_before(a, b);
+  const int64_t chunk0 = rec_chunks_before(a.q_len, b);
   if (chunk0 + (n + L - 1) / L > max_chunks) return;            // (requests that share rows: more rows than the launch has)
   const int h = g * per + member / eblocks;
   const int e0 = member % eblocks * 64 + 16 * w, e = e0 + r16;
@@ -753,39 +702,22 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
       const int row = 16 * t + 4 * kq + r;
       S[t][r] = (first_pos > 0 && e_ok && row < D) ? st[row * E] : 0.f;
     }
-  float wt[kDeltaChunkTaps];
+  float wt[kRecTaps];
 #pragma unroll
-  for (int i = 0; i < kDeltaChunkTaps; ++i)
+  for (int i = 0; i < kRecTaps; ++i)
     wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_v)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
   const int64_t frag_ld = (int64_t)G * delta_frag_elems(NP), head_ld = (int64_t)H * kDeltaHead;
   const float* f = a.frags + chunk0 * frag_ld + g * delta_frag_elems(NP) + 4 * lane;
   const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kDeltaHead;
   const T* p = (const T*)a.p + t0 * a.ld + a.v_off + h * E + e0;
-  const uint32_t vo = (uint32_t)(4 * kq) * (uint32_t)a.ld + (e_ok ? r16 : 0);
   float* yo = a.work + t0 * a.wld + 2 * G * D + h * E + e0;
-  const uint32_t yk = (uint32_t)(4 * kq) * (uint32_t)a.wld + r16;
+  // 16-byte pieces of the projection's and of the result's rows: everything starts on one
+  const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
 
   // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
-  T vin[2][HALO + 4];
-  auto fetch_v = [&](int l0) {
-    const T* pr = p + (int64_t)(l0 - HALO) * a.ld;
-    if (wide && l0 + L <= n) {
-#pragma unroll
-      for (int r = 0; r < 16 + HALO + 4; ++r) {
-        if (r < HALO + 4) vin[0][r] = pr[vo];
-        if (r >= 16) vin[1][r - 16] = pr[vo];
-        pr += a.ld;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < HALO + 4; ++i) {
-          const int l = l0 + 16 * j + 4 * kq + i - HALO;
-          vin[j][i] = e_ok && l < n ? p[(int64_t)l * a.ld + r16] : Elem<T>::from_f(0.f);
-        }
-    }
-  };
+  RowTile<T> tile;
+  auto fetch_v = [&](int l0) { if (vec) tile.fetch(p, a.ld, l0, n, lane); };
   // v of this lane's tokens, zero behind the portion; taps that the layer does not have see zeros
   auto convolve = [&](const float (&x)[2][HALO + 4], int cnt, f32x4 (&v)[2], bool& bad) {
 #pragma unroll
@@ -794,13 +726,12 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
       for (int s = 0; s < 4; ++s) {
         float y = wt[0] * x[j][s + HALO];
 #pragma unroll
-        for (int i = 1; i < kDeltaChunkTaps; ++i) y += wt[i] * __int_as_float(__float_as_int(x[j][s + HALO - i]) & (i < taps ? -1 : 0));
-        const bool ok = delta_finite(y), in = 16 * j + 4 * kq + s < cnt;     // (silu of infinity: itself; of minus infinity: inf / inf)
-        float z = delta_silu_fast(y);
+        for (int i = 1; i < kRecTaps; ++i) y += wt[i] * __int_as_float(__float_as_int(x[j][s + HALO - i]) & (i < taps ? -1 : 0));
+        float z = rec_silu(y);
         asm volatile("" : "+v"(z));                              // (straight-line code: it goes between the products)
-        z = ok ? z : (y > 0.f ? y : __builtin_nanf(""));
-        v[j][s] = in ? z : 0.f;
-        bad |= in && !ok;
+        const bool in = 16 * j + 4 * kq + s < cnt;
+        v[j][s] = in ? rec_silu_or_not_finite(y, z) : 0.f;
+        bad |= in && !rec_finite(y);
       }
   };
   f32x4 v[2];
@@ -857,7 +788,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) v_l[w][(16 * j + 4 * kq + s) * 16 + r16] = v[j][s];
+        for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = v[j][s];
       if (e_ok)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
@@ -889,10 +820,17 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
       bad = false;
       {
         float x[2][HALO + 4];
+        if (vec) {
+          tile.place(in_l[w], lane);
+        } else {                                                 // (rows or columns that start off a 16-byte boundary: not fetched ahead)
+          for (int r = kq; r < L + HALO; r += 4)
+            in_l[w][r * RowTile<T>::kStride + r16] = e_ok && l0 + L - HALO + r < n ? p[(int64_t)(l0 + L - HALO + r) * a.ld + r16] : Elem<T>::from_f(0.f);
+        }
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int i = 0; i < HALO + 4; ++i) x[j][i] = Elem<T>::to_f(vin[j][i]);
+          for (int i = 0; i < HALO + 4; ++i) x[j][i] = Elem<T>::to_f(in_l[w][(16 * j + 4 * kq + i) * RowTile<T>::kStride + r16]);
         convolve(x, n - l0 - L, vn, bad);
       }
 #pragma unroll
@@ -934,17 +872,14 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
         wv[i] = *reinterpret_cast<const f32x4*>(fhn + 1536 + L + 16 * i + 4 * kq);
       }
       if (serial) {
-      } else if (cnt == L && wide) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) (yr + (int64_t)(16 * i + r) * a.wld)[yk] = O[i][r];
+      } else if (cnt == L && vec) {
+        rec_store_tile(O, o_l[w], yr, a.wld, lane);
       } else {
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            if (16 * i + 4 * kq + r < cnt && e_ok) (yr + (int64_t)(16 * i + r) * a.wld)[yk] = O[i][r];
+            if (16 * i + 4 * kq + r < cnt && e_ok) yr[(int64_t)(16 * i + 4 * kq + r) * a.wld + r16] = O[i][r];
       }
 #pragma unroll
       for (int t = 0; t < NT; ++t) S[t] *= keep;
@@ -984,7 +919,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
         kd += __shfl_xor(kd, 16, 64);
         kd += __shfl_xor(kd, 32, 64);
         const float gt = fh[1536 + 2 * L + t], bt = fh[1536 + 3 * L + t];
-        const float u1 = bt * (v_l[w][t * 16 + r16] - gt * dk);
+        const float u1 = bt * (o_l[w][t * kOutStride + r16] - gt * dk);
 #pragma unroll 1
         for (int u = 0; u < 4 * NT; ++u) {
           const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
@@ -1052,16 +987,15 @@ extern "C" int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, 
 // 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; heads of 64 x 64: 4 requests of 2 rows 49 / 37, 32 requests of 8 rows 60 / 78, 16 rows
 // 82 / 83, 64 rows 200 / 134.  A few requests take chunks whatever their length.
 constexpr int64_t kDeltaChunkMinRows = 16, kDeltaChunkFewRequests = 4;
-static int64_t delta_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kDeltaChunk + batch; }
 
 extern "C" int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps) {
-  if (batch <= 0 || num_heads <= 0 || num_k_heads <= 0 || (batch > kDeltaChunkFewRequests && num_tokens < kDeltaChunkMinRows * batch) || k_dim > 128 || taps > kDeltaChunkTaps) return 0;
-  return delta_max_chunks(num_tokens, batch) * (num_k_heads * delta_frag_elems(k_dim <= 64 ? 64 : 128) + (int64_t)num_heads * kDeltaHead);
+  if (batch <= 0 || num_heads <= 0 || num_k_heads <= 0 || (batch > kDeltaChunkFewRequests && num_tokens < kDeltaChunkMinRows * batch) || k_dim > 128 || taps > kRecTaps) return 0;
+  return rec_max_chunks(num_tokens, batch) * (num_k_heads * delta_frag_elems(k_dim <= 64 ? 64 : 128) + (int64_t)num_heads * kDeltaHead);
 }
 
 template <typename T, int NP>
 static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
-  const int64_t chunks = delta_max_chunks(a.num_tokens, a.batch);
+  const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
   hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
   hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);

@@ -1,0 +1,118 @@
+// What the chunked forms of the recurrences with a matrix state share (state_space.hip, delta_rule.hip): where a chunk of a
+// launch lies, accurate exponentials, and the tiles that a wave moves between rows in memory and its accumulators' places.
+#pragma once
+#include "common.h"
+#include "mfma_frag.h"
+
+namespace semipd {
+
+constexpr int kRecChunk = 32;            // tokens of a chunk
+constexpr int kRecTaps = 4;              // taps of the convolution at most
+constexpr int kRecHalo = kRecTaps - 1;   // rows in front of a chunk that its convolution looks at
+
+inline int64_t rec_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kRecChunk + batch; }
+
+// Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
+__device__ __forceinline__ bool rec_find_chunk(const int32_t* q_len, int batch, int64_t idx, int& b, int64_t& c) {
+  const int lane = threadIdx.x & 63;
+  int64_t before = 0;
+  for (int r0 = 0; r0 < batch; r0 += 64) {
+    const int n = r0 + lane < batch ? max(0, (q_len[r0 + lane] + kRecChunk - 1) / kRecChunk) : 0;
+    int s = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(s, o, 64);
+      if (lane >= o) s += t;
+    }
+    const int total = __shfl(s, 63, 64);
+    if (idx < before + total) {
+      const uint64_t past = __ballot(before + s > idx);
+      const int first = __ffsll((unsigned long long)past) - 1;
+      b = r0 + first;
+      c = idx - before - (__shfl(s, first, 64) - __shfl(n, first, 64));
+      return true;
+    }
+    before += total;
+  }
+  return false;
+}
+// how many chunks the requests in front of b have
+__device__ __forceinline__ int64_t rec_chunks_before(const int32_t* q_len, int b) {
+  const int lane = threadIdx.x & 63;
+  int s = 0;
+  for (int r = lane; r < b; r += 64) s += max(0, (q_len[r] + kRecChunk - 1) / kRecChunk);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  return s;
+}
+
+__device__ __forceinline__ bool rec_finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+
+// silu of a finite x: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal and one
+// correction of it and of the result: within an ulp of x / (1 + expf(-x)), 14 instructions in place of 30
+__device__ __forceinline__ float rec_silu(float x) {
+  const float c = fmaxf(x, -87.f);
+  const float hi = c * -1.44269502f, lo = fmaf(c, -1.44269502f, -hi) + c * -1.92596299e-8f;
+  float e = __builtin_amdgcn_exp2f(hi);
+  e = fmaf(e, lo * 0.693147182f, e);
+  const float d = 1.0f + e;
+  float r = __builtin_amdgcn_rcpf(d);
+  r = fmaf(fmaf(-d, r, 1.0f), r, r);
+  const float q = x * r;
+  return fmaf(fmaf(-d, q, x), r, q);
+}
+// ... and of one that is not: infinity itself, of minus infinity inf / inf
+__device__ __forceinline__ float rec_silu_or_not_finite(float y, float silu) { return rec_finite(y) ? silu : (y > 0.f ? y : __builtin_nanf("")); }
+
+// 2^x of a 64-bit exponent: what rounding it to 32 bits takes away is multiplied in
+__device__ __forceinline__ float rec_exp2(double x) {
+  const float hi = (float)x, lo = (float)(x - (double)hi);
+  const float e = __builtin_amdgcn_exp2f(hi);
+  return hi < -126.f ? e : fmaf(e, lo * 0.693147182f, e);
+}
+
+// Rows of 16 columns that one wave needs (its convolution's inputs: a chunk and the rows in front of it), 16 bytes a lane: a load
+// per token, element and lane would be 14 requests of 2 bytes for the two or three here.  `fetch` leaves them in registers,
+// `place` puts them into the wave's own LDS (48 / 80 bytes a row: rows that are read together start in different banks).
+template <typename T> struct RowTile {
+  static constexpr int kPerRow = 16 * (int)sizeof(T) / 16;          // 16-byte pieces a row
+  static constexpr int kRows = kRecChunk + kRecHalo;
+  static constexpr int kLoads = (kRows * kPerRow + 63) / 64;
+  static constexpr int kStride = sizeof(T) == 2 ? 24 : 20;          // elements of T between rows in LDS
+  static constexpr int kElems = kRows * kStride;
+  uint4 v[kLoads];
+  // rows l0 - halo .. l0 + 31 of `p` (row 0 = the portion's first), zeros behind row n - 1; l0 > 0
+  __device__ __forceinline__ void fetch(const T* p, int64_t ld, int l0, int n, int lane) {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int it = u * 64 + lane, row = it / kPerRow, l = l0 - kRecHalo + row;
+      v[u] = uint4{0u, 0u, 0u, 0u};
+      if (row < kRows && l < n) v[u] = *reinterpret_cast<const uint4*>(p + (int64_t)l * ld + it % kPerRow * (16 / (int)sizeof(T)));
+    }
+  }
+  __device__ __forceinline__ void place(T* lds, int lane) const {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int it = u * 64 + lane, row = it / kPerRow;
+      if (row < kRows) *reinterpret_cast<uint4*>(lds + row * kStride + it % kPerRow * (16 / (int)sizeof(T))) = v[u];
+    }
+  }
+};
+
+// A wave's 32 x 16 results (lane (r16, kq): rows 16 i + 4 kq + r of column r16) to rows in memory, 16 bytes a lane by way of its LDS
+constexpr int kOutStride = 20;            // floats between rows in LDS
+__device__ __forceinline__ void rec_store_tile(const f32x4 (&o)[2], float* lds, float* y, int64_t ld, int lane) {
+  const int r16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lds[(16 * i + 4 * kq + r) * kOutStride + r16] = o[i][r];
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int row = 16 * i + (lane >> 2);
+    *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + 4 * (lane & 3)) = *reinterpret_cast<const f32x4*>(lds + row * kOutStride + 4 * (lane & 3));
+  }
+}
+
+}  // namespace semipd

@@ -23,7 +23,7 @@
 //  * ssm_post_kernel / ssm_post_vec_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
 #include "common.h"
-#include "mfma_frag.h"
+#include "recurrent_chunks.h"
 
 namespace semipd {
 
@@ -317,80 +317,33 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
 // requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (36 GFLOP at
 // 154 TFLOP/s = 235 us) and the vector work between its products: 560 us, operands 73.  Chunks of 32 and not 64: the same products
 // with S, half the ones inside a chunk, and three workgroups' LDS on a CU in place of one (64 tokens, two heads a workgroup: 952 us).
-constexpr int kSsmChunk = 32;
-constexpr int kSsmChunkTaps = 4;        // taps at most
 
-// fp32 elements of the operands of one (chunk, group): C [32][NP] | B^T [NP][32] | C B^T [32][32] | a flag in a piece of 4,
-// and behind those of all chunks, of one (chunk, head): b in log2 units, 64 bits [32] | dt | e^(b_t) | e^(b_last - b_t) dt_t | decay
-__host__ __device__ constexpr int64_t ssm_frag_elems(int np) { return 2 * (int64_t)kSsmChunk * np + kSsmChunk * kSsmChunk + 4; }
-constexpr int kSsmSteps = 6 * kSsmChunk;
-
-// Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
-__device__ __forceinline__ bool ssm_find_chunk(const SsmArgs& a, int64_t idx, int& b, int64_t& c) {
-  const int lane = threadIdx.x & 63;
-  int64_t before = 0;
-  for (int r0 = 0; r0 < (int)a.batch; r0 += 64) {
-    const int n = r0 + lane < (int)a.batch ? max(0, (a.q_len[r0 + lane] + kSsmChunk - 1) / kSsmChunk) : 0;
-    int s = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int t = __shfl_up(s, o, 64);
-      if (lane >= o) s += t;
-    }
-    const int total = __shfl(s, 63, 64);
-    if (idx < before + total) {
-      const uint64_t past = __ballot(before + s > idx);
-      const int first = __ffsll((unsigned long long)past) - 1;
-      b = r0 + first;
-      c = idx - before - (__shfl(s, first, 64) - __shfl(n, first, 64));
-      return true;
-    }
-    before += total;
-  }
-  return false;
-}
-// how many chunks the requests in front of b have
-__device__ __forceinline__ int64_t ssm_chunks_before(const SsmArgs& a, int b) {
-  const int lane = threadIdx.x & 63;
-  int s = 0;
-  for (int r = lane; r < b; r += 64) s += max(0, (a.q_len[r] + kSsmChunk - 1) / kSsmChunk);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  return s;
-}
-
-// silu of the chunked form: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal
-// and one correction of it and of the result: within an ulp of x / (1 + expf(-x)), 14 instructions in place of 30
-__device__ __forceinline__ float ssm_silu_fast(float x) {
-  const float c = fmaxf(x, -87.f);
-  const float hi = c * -1.44269502f, lo = fmaf(c, -1.44269502f, -hi) + c * -1.92596299e-8f;
-  float e = __builtin_amdgcn_exp2f(hi);
-  e = fmaf(e, lo * 0.693147182f, e);
-  const float d = 1.0f + e;
-  float r = __builtin_amdgcn_rcpf(d);
-  r = fmaf(fmaf(-d, r, 1.0f), r, r);
-  const float q = x * r;
-  return fmaf(fmaf(-d, q, x), r, q);
-}
-
-__device__ __forceinline__ bool ssm_finite(float x) { return fabsf(x) <= 3.402823466e38f; }
+// fp32 elements of the operands of one (chunk, group): C and B^T as left-hand operands of 16 x 16 x 16 products, in the order in which
+// they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a piece of 4.  Of one
+// (chunk, head): tiles 00, 10, 11 of the weighted C B^T, then e^(b_t) | e^(b_last - b_t) dt_t | dt | decay.
+__host__ __device__ constexpr int64_t ssm_frag_elems(int np) { return 2 * (int64_t)kRecChunk * np + 4; }
+constexpr int kSsmHead = 3 * 256 + 4 * kRecChunk;
 
 // What the heads of a group share, a workgroup per (chunk, group): convolution + bias + silu of the group's B and C channels (a
-// channel per thread, its taps and the last inputs in registers), B also transposed so that the state's update reads four
-// tokens of a row at once, and the 32 x 32 products C B^T; the step sizes and running log decays of the group's heads.  NP: N up to a multiple of 64, zeros behind N and behind the portion.
+// channel per thread, its taps and the last inputs in registers), laid down as operands; the 32 x 32 products C B^T and, half a wave
+// per head in turn (lane = token), step sizes, running log decays and the weighted C B^T.  NP: N up to a multiple of 64, zeros behind
+// N and behind the portion.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
-  __shared__ __attribute__((aligned(16))) float c_l[kSsmChunk * (NP + 4)];
-  __shared__ __attribute__((aligned(16))) float b_l[kSsmChunk * (NP + 4)];
+  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 1;
+  __shared__ __attribute__((aligned(16))) float c_l[L * CS];
+  __shared__ __attribute__((aligned(16))) float b_l[L * CS];
+  __shared__ float cb_l[L * PS];
+  __shared__ double cum_l[8 * L];
   const int tid = threadIdx.x, g = blockIdx.y;
   int b;
   int64_t ck;
-  if (!ssm_find_chunk(a, blockIdx.x, b, ck)) return;
+  if (!rec_find_chunk(a.q_len, (int)a.batch, blockIdx.x, b, ck)) return;
   const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
   if (first_pos < 0) return;
-  const int64_t l0 = ck * kSsmChunk, t0 = a.q_start[b] + l0;
-  const int cnt = (int)(n - l0 < kSsmChunk ? n - l0 : kSsmChunk);
-  const int N = a.N, taps = a.taps;
+  const int64_t l0 = ck * L, t0 = a.q_start[b] + l0;
+  const int cnt = (int)(n - l0 < L ? n - l0 : L);
+  const int N = a.N, taps = a.taps, per = a.H / a.G;
   const int C = a.H * a.E + 2 * a.G * N;
   float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * ssm_frag_elems(NP);
   bool bad = false;
@@ -403,9 +356,9 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
       const T* p = (const T*)a.p + t0 * a.ld + a.x_off + col;
       const T* cw = (const T*)a.conv_w + (int64_t)col * taps;
       const float bias = a.conv_b ? Elem<T>::to_f(((const T*)a.conv_b)[col]) : 0.f;
-      float wt[kSsmChunkTaps], in[kSsmChunkTaps];                                     // weight and input i tokens back
+      float wt[kRecTaps], in[kRecTaps];                                   // weight and input i tokens back
 #pragma unroll
-      for (int i = 0; i < kSsmChunkTaps; ++i) {
+      for (int i = 0; i < kRecTaps; ++i) {
         wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
         in[i] = 0.f;
         if (i > 0 && i < taps) {
@@ -413,99 +366,107 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
           else if (first_pos > 0) in[i] = a.conv_state[a.state_indices[b] * a.conv_ld + (int64_t)(taps - 1 + l0 - i) * C + col];
         }
       }
-      float x[kSsmChunk];
+      float x[L];
+      if (cnt == L) {
 #pragma unroll
-      for (int i = 0; i < kSsmChunk; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
+        for (int i = 0; i < L; ++i) x[i] = Elem<T>::to_f(p[(int64_t)i * a.ld]);
+      } else {
 #pragma unroll
-      for (int t = 0; t < kSsmChunk; ++t) {
+        for (int i = 0; i < L; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
+      }
+#pragma unroll
+      for (int t = 0; t < L; ++t) {
         in[0] = x[t];
         float y = bias;
 #pragma unroll
-        for (int i = 0; i < kSsmChunkTaps; ++i)
+        for (int i = 0; i < kRecTaps; ++i)
           if (i < taps) y += wt[i] * in[i];
 #pragma unroll
-        for (int i = kSsmChunkTaps - 1; i > 0; --i) in[i] = in[i - 1];
-        x[t] = t < cnt ? ssm_silu(y) : 0.f;
-        bad |= !ssm_finite(x[t]);
-      }
-#pragma unroll
-      for (int t = 0; t < kSsmChunk; ++t) dst[t * (NP + 4)] = x[t];
-      if (!is_c) {
-        float* bt = frag + (int64_t)kSsmChunk * NP + (int64_t)r * kSsmChunk;
-#pragma unroll
-        for (int t = 0; t < kSsmChunk; t += 4) *reinterpret_cast<float4*>(bt + t) = float4{x[t], x[t + 1], x[t + 2], x[t + 3]};
+        for (int i = kRecTaps - 1; i > 0; --i) in[i] = in[i - 1];
+        dst[t * CS] = t < cnt ? rec_silu_or_not_finite(y, rec_silu(y)) : 0.f;
+        bad |= t < cnt && !rec_finite(y);
       }
     } else {
-      for (int t = 0; t < kSsmChunk; ++t) dst[t * (NP + 4)] = 0.f;
-      if (!is_c) {
-        float* bt = frag + (int64_t)kSsmChunk * NP + (int64_t)r * kSsmChunk;
-        for (int t = 0; t < kSsmChunk; t += 4) *reinterpret_cast<float4*>(bt + t) = float4{0.f, 0.f, 0.f, 0.f};
-      }
+      for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
     }
   }
-  // half a wave per head (lane = token): step sizes, running sums of the log decays
-  for (int hh = tid >> 5; hh < a.H / a.G; hh += 8) {
-    const int h = g * (a.H / a.G) + hh, t = tid & 31;
+  __syncthreads();
+  for (int i = tid; i < L * NP / 4; i += 256) {                  // C: tile (tokens, rows of S)
+    const int tile = i >> 6, ln = i & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
+    *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(c_l + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
+  }
+  for (int i = tid; i < L * NP / 4; i += 256) {                  // B^T: tile (rows of S, tokens)
+    const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
+    const float* s = b_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
+    *reinterpret_cast<float4*>(frag + L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+  }
+  // C B^T, a 16 x 16 tile a wave; k runs 16 at a time, lane group kq takes k = 4 kq .. 4 kq + 3 in four steps (both operands alike)
+  {
+    const int lane = tid & 63, r16 = lane & 15, kq = lane >> 4, i0 = (tid >> 7) * 16, j0 = ((tid >> 6) & 1) * 16;
+    f32x4 acc = {};
+#pragma unroll 4
+    for (int k = 0; k < NP; k += 16) {
+      const f32x4 av = *reinterpret_cast<const f32x4*>(c_l + (i0 + r16) * CS + k + 4 * kq);
+      const f32x4 bv = *reinterpret_cast<const f32x4*>(b_l + (j0 + r16) * CS + k + 4 * kq);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) cb_l[(i0 + 4 * kq + r) * PS + j0 + r16] = acc[r];
+  }
+  __syncthreads();
+  const int hw = tid >> 5, t = tid & 31;
+  double* cum = cum_l + hw * L;
+  for (int hh = hw; hh < per; hh += 8) {
+    const int h = g * per + hh;
     const float dt = t < cnt ? ssm_softplus(Elem<T>::to_f(((const T*)a.p)[(t0 + t) * a.ld + a.dt_off + h]) + a.dt_bias[h]) : 0.f;
     const float la = t < cnt ? -expf(a.a_log[h]) * dt : 0.f;
-    double cum = (double)la * 1.4426950408889634;
+    double c = (double)la * 1.4426950408889634;
 #pragma unroll
-    for (int o = 1; o < kSsmChunk; o <<= 1) {
-      const double v = __shfl_up(cum, o, kSsmChunk);
-      if (t >= o) cum += v;
+    for (int o = 1; o < L; o <<= 1) {
+      const double v = __shfl_up(c, o, L);
+      if (t >= o) c += v;
     }
-    const double last = __shfl(cum, kSsmChunk - 1, kSsmChunk);
-    float* sp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmSteps;
-    reinterpret_cast<double*>(sp)[t] = cum;
-    sp[2 * kSsmChunk + t] = dt;
-    sp[3 * kSsmChunk + t] = __builtin_amdgcn_exp2f((float)cum);
-    sp[4 * kSsmChunk + t] = __builtin_amdgcn_exp2f((float)(last - cum)) * dt;
-    sp[5 * kSsmChunk + t] = expf(la);
+    const double last = __shfl(c, L - 1, L);
+    cum[t] = c;
+    float* hp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmHead;
+    const float eb = rec_exp2(c), wt = rec_exp2(last - c) * dt, dec = expf(la);
+    hp[768 + t] = eb;
+    hp[768 + L + t] = wt;
+    hp[768 + 2 * L + t] = dt;
+    hp[768 + 3 * L + t] = dec;
+    bad |= !rec_finite(dt) || !rec_finite(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
+    __builtin_amdgcn_wave_barrier();
+    // the weighted C B^T, 16 bytes a lane: piece i of 192 is lane i % 64 of tile i / 64; the step size of column s from lane s
+#pragma unroll
+    for (int u = 0; u < 6; ++u) {
+      const int i = u * 32 + t, tile = i >> 6, ln = i & 63, row = (tile ? 16 : 0) + (ln & 15), col = (tile == 2 ? 16 : 0) + 4 * (ln >> 4);
+      const double bt = cum[row];
+      f32x4 m;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const float ds = __shfl(dt, col + v, L);
+        m[v] = col + v <= row ? cb_l[row * PS + col + v] * (rec_exp2(bt - cum[col + v]) * ds) : 0.f;
+      }
+      *reinterpret_cast<f32x4*>(hp + 4 * i) = m;
+    }
+    __builtin_amdgcn_wave_barrier();
   }
   const int any_bad = __syncthreads_or(bad);
   if (tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
-  for (int i = tid; i < kSsmChunk * NP / 4; i += 256) {
-    const int t = i / (NP / 4), c = 4 * (i % (NP / 4));
-    *reinterpret_cast<float4*>(frag + (int64_t)t * NP + c) = *reinterpret_cast<const float4*>(c_l + t * (NP + 4) + c);
-  }
-  // C B^T, a 16 x 16 tile a wave; k runs 16 at a time, lane group kq takes k = 4 kq .. 4 kq + 3 in four steps (both operands alike)
-  const int lane = tid & 63, r16 = lane & 15, kq = lane >> 4, i0 = (tid >> 7) * 16, j0 = ((tid >> 6) & 1) * 16;
-  f32x4 acc = {};
-#pragma unroll 4
-  for (int k = 0; k < NP; k += 16) {
-    const f32x4 av = *reinterpret_cast<const f32x4*>(c_l + (i0 + r16) * (NP + 4) + k + 4 * kq);
-    const f32x4 bv = *reinterpret_cast<const f32x4*>(b_l + (j0 + r16) * (NP + 4) + k + 4 * kq);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
-  }
-  float* cb = frag + 2 * (int64_t)kSsmChunk * NP;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) cb[(i0 + 4 * kq + r) * kSsmChunk + j0 + r16] = acc[r];
 }
 
-// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S); a wave has 16 columns of S, its NP rows in
-// accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16.  That is also how a wave holds the right-hand operand of
-// a product over the rows, so S goes from one chunk's sum into the next one's product without leaving its registers, and so do
-// the chunk's x (lane: tokens 16 j + 4 kq + s of its column), which each lane computes itself from the projection's rows: x
-// never touches memory.  C, B^T (shared by the group's heads) and the head's weighted C B^T are read from LDS, 16 bytes for four
-// steps; the next chunk's loads are in flight during the products.  52 KB of LDS: three workgroups a CU, the weights and
-// convolutions of one beside the products of the others.
+// The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
+// sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16.  That is
+// also how a wave holds the right-hand operand of a product over the rows, so S goes from one chunk's sum into the next one's product
+// without leaving its registers, and so do the chunk's x (lane: tokens 16 j + 4 kq + s of its column), which each lane convolves in
+// their place: x never touches memory.  Left-hand operands come straight into registers in the order they are used: B^T of a chunk
+// into the registers its C was read from, the next chunk's C into those of B^T.  No LDS, no barriers.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
-  constexpr int L = kSsmChunk, LT = L / 16, NT = NP / 16;
-  constexpr int CS = NP + 4, TS = L + 4, XS = 68;            // row strides in LDS: rows that are read together start in different banks
-  constexpr int V = 16 / sizeof(T);                           // elements of a 16-byte piece
-  constexpr int HALO = kSsmChunkTaps - 1;
-  constexpr int PF = L * NP / 4 / 256;                        // 16-byte pieces per thread: of C, of B^T
-  constexpr int PX = ((L + HALO) * 64 / V + 255) / 256;       // ... of the projection's rows
-  __shared__ __attribute__((aligned(16))) float c_l[L * CS];
-  __shared__ __attribute__((aligned(16))) float bt_l[NP * TS];
-  __shared__ __attribute__((aligned(16))) float m_l[L * TS];              // weighted C B^T
-  __shared__ __attribute__((aligned(16))) float x_l[(L + HALO) * XS];     // inputs of the convolution
-  __shared__ __attribute__((aligned(16))) float steps_l[kSsmSteps];
-  const double* cum_l = reinterpret_cast<const double*>(steps_l);         // b in log2 units | dt | e^(b_t) | e^(b_last - b_t) dt_t | decay
-  const float *dt_l = steps_l + 2 * L, *eb_l = dt_l + L, *wt_l = eb_l + L, *dec_l = wt_l + L;
-  __shared__ int flag_l[2];
+  constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
+  __shared__ __attribute__((aligned(16))) T in_l[4][RowTile<T>::kElems];       // a wave's own: raw inputs of its convolution
+  __shared__ __attribute__((aligned(16))) float o_l[4][L * kOutStride];         // ... results on their way out (token by token: its x)
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
   // workgroups of one (request, group) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, per = H / G;
@@ -516,11 +477,12 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
-  const int64_t chunk0 = ssm_chunks_before(a, b);
+  const int64_t chunk0 = rec_chunks_before(a.q_len, b);
   if (chunk0 + (n + L - 1) / L > max_chunks) return;          // (requests that share rows: more rows than the launch has)
   const int h = g * per + member / eblocks;
-  const int e0 = member % eblocks * 64, e = e0 + 16 * w + r16;
-  const bool e_ok = e < E;
+  const int e0 = member % eblocks * 64 + 16 * w, e = e0 + r16;
+  if (e0 >= E) return;
+  const bool e_ok = e < E, wide = e0 + 16 <= E;
   const int C = H * E + 2 * G * N;
   const int64_t slot = a.state_indices[b];
   float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
@@ -532,239 +494,215 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
       const int row = 16 * t + 4 * kq + r;
       S[t][r] = (first_pos > 0 && e_ok && row < N) ? st[row * E] : 0.f;
     }
-  float wt[kSsmChunkTaps];
+  float wt[kRecTaps];
 #pragma unroll
-  for (int i = 0; i < kSsmChunkTaps; ++i) wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_w)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
+  for (int i = 0; i < kRecTaps; ++i) wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_w)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
   const float bias = (a.conv_b && e_ok) ? Elem<T>::to_f(((const T*)a.conv_b)[h * E + e]) : 0.f;
   const float dskip = a.d_skip ? a.d_skip[h] : 0.f;
-  const int64_t frag_ld = (int64_t)G * ssm_frag_elems(NP);
-  const float* f = a.frags + chunk0 * frag_ld + g * ssm_frag_elems(NP);      // the operands of the chunk that is fetched next
+  const int64_t frag_ld = (int64_t)G * ssm_frag_elems(NP), head_ld = (int64_t)H * kSsmHead;
+  const float* f = a.frags + chunk0 * frag_ld + g * ssm_frag_elems(NP) + 4 * lane;
+  const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kSsmHead;
   const T* p = (const T*)a.p + t0 * a.ld + a.x_off + h * E + e0;
-  const float* fs = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kSsmSteps;
-  const uint32_t xo = (uint32_t)(tid / (64 / V)) * (uint32_t)a.ld + tid % (64 / V) * V;      // this thread's first piece of the rows
+  float* yo = a.work + t0 * a.wld + h * E + e0;
+  // 16-byte pieces of the projection's and of the result's rows: everything starts on one
+  const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
 
-  f32x4 pc[PF], pb[PF], pcb, ps;
-  Vec16<T> px[PX];
-  float pflag = 0.f;
-  const int mi = tid >> 3, mj = (tid & 7) * 4;                // this thread's four elements of the weighted C B^T
-  const bool wide = e0 + 64 <= E;
-  auto fetch = [&](int l0) {
+  // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
+  RowTile<T> tile;
+  auto fetch_x = [&](int l0) { if (vec) tile.fetch(p, a.ld, l0, n, lane); };
+  // x of this lane's tokens, zero behind the portion; taps that the layer does not have see zeros
+  auto convolve = [&](const float (&raw)[2][HALO + 4], int cnt, f32x4 (&x)[2], bool& bad) {
 #pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      pc[u] = *reinterpret_cast<const f32x4*>(f + 4 * (u * 256 + tid));
-      pb[u] = *reinterpret_cast<const f32x4*>(f + L * NP + 4 * (u * 256 + tid));
-    }
-    pcb = *reinterpret_cast<const f32x4*>(f + 2 * L * NP + 4 * tid);
-    pflag = f[ssm_frag_elems(NP) - 4];
-    f += frag_ld;
-    if (tid < kSsmSteps / 4) ps = *reinterpret_cast<const f32x4*>(fs + 4 * tid);
-    fs += (int64_t)H * kSsmSteps;
-    const T* rows = p + (int64_t)(l0 - HALO) * a.ld;
-    if (wide && l0 >= HALO && l0 + L <= n) {                  // every row and column of the tile is there
-#pragma unroll
-      for (int u = 0; u < PX; ++u)
-        if ((u + 1) * 256 <= (L + HALO) * 64 / V || u * 256 + tid < (L + HALO) * 64 / V)
-          px[u] = load16(rows + (int64_t)u * 256 / (64 / V) * a.ld + xo);
-    } else {
-#pragma unroll
-      for (int u = 0; u < PX; ++u) {
-        const int it = u * 256 + tid, row = it / (64 / V), c = it % (64 / V) * V, l = l0 - HALO + row;
-        if (row < L + HALO && l >= 0 && l < n && e0 + c < E) px[u] = load16(rows + (int64_t)row * a.ld + c);
-        else
-#pragma unroll
-          for (int v = 0; v < V; ++v) px[u].e[v] = Elem<T>::from_f(0.f);
-      }
-    }
-  };
-  fetch(0);
-  if (tid < 2) flag_l[tid] = 0;
-  __syncthreads();
-  for (int l0 = 0; l0 < n; l0 += L) {
-    const int cnt = n - l0 < L ? n - l0 : L;
-    const int par = (l0 / L) & 1;
-    bool bad = pflag != 0.f;
-    // ---- what came in: C, B^T, inputs of the convolution; running sums of the log decays (lane = token)
-#pragma unroll
-    for (int u = 0; u < PF; ++u) {
-      const int it = u * 256 + tid;
-      *reinterpret_cast<f32x4*>(c_l + it / (NP / 4) * CS + 4 * (it % (NP / 4))) = pc[u];
-      *reinterpret_cast<f32x4*>(bt_l + it / (L / 4) * TS + 4 * (it % (L / 4))) = pb[u];
-    }
-#pragma unroll
-    for (int u = 0; u < PX; ++u) {
-      const int it = u * 256 + tid, row = it / (64 / V), c = it % (64 / V) * V;
-      if (row < L + HALO)
-#pragma unroll
-        for (int v = 0; v < V; v += 4)
-          *reinterpret_cast<f32x4*>(x_l + row * XS + c + v) = f32x4{Elem<T>::to_f(px[u].e[v]), Elem<T>::to_f(px[u].e[v + 1]),
-                                                                     Elem<T>::to_f(px[u].e[v + 2]), Elem<T>::to_f(px[u].e[v + 3])};
-    }
-    if (l0 == 0 && first_pos > 0 && taps > 1) {               // the inputs in front of the portion: from the state row, fp32
-      __syncthreads();
-      for (int i = tid; i < (taps - 1) * 64; i += 256) {
-        const int back = i / 64 + 1, c = i % 64;
-        if (e0 + c < E) x_l[(HALO - back) * XS + c] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 - back) * C + h * E + e0 + c];
-      }
-    }
-    if (tid < kSsmSteps / 4) {
-      *reinterpret_cast<f32x4*>(steps_l + 4 * tid) = ps;
-      if (4 * tid >= 2 * L) bad |= !ssm_finite(ps[0]) || !ssm_finite(ps[1]) || !ssm_finite(ps[2]) || !ssm_finite(ps[3]);
-    }
-    __syncthreads();
-    // ---- this lane's x of the chunk; the head's weighted C B^T
-    float xr[4 * LT];
-#pragma unroll
-    for (int j = 0; j < LT; ++j) {
-      float in[HALO + 4];
-#pragma unroll
-      for (int i = 0; i < HALO + 4; ++i) in[i] = i >= kSsmChunkTaps - taps ? x_l[(16 * j + 4 * kq + i) * XS + 16 * w + r16] : 0.f;
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        float y = bias;
+        float y = bias + wt[0] * raw[j][s + HALO];
 #pragma unroll
-        for (int i = 0; i < kSsmChunkTaps; ++i)
-          if (i < taps) y += wt[i] * in[s + HALO - i];
-        const bool ok = ssm_finite(y);                          // (silu of infinity: itself; of minus infinity: inf / inf)
-        xr[4 * j + s] = ok ? ssm_silu_fast(y) : (y > 0.f ? y : __builtin_nanf(""));
-        bad |= !ok;
+        for (int i = 1; i < kRecTaps; ++i) y += wt[i] * __int_as_float(__float_as_int(raw[j][s + HALO - i]) & (i < taps ? -1 : 0));
+        float z = rec_silu(y);
+        asm volatile("" : "+v"(z));                              // (straight-line code: it goes between the products)
+        const bool in = 16 * j + 4 * kq + s < cnt;
+        x[j][s] = in ? rec_silu_or_not_finite(y, z) : 0.f;
+        bad |= in && !rec_finite(y);
       }
-    }
-    if (cnt < L)
+  };
+  f32x4 x[2];
+  bool bad = false;
+  {
+    float in[2][HALO + 4];
 #pragma unroll
-      for (int j = 0; j < LT; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) xr[4 * j + s] = 16 * j + 4 * kq + s < cnt ? xr[4 * j + s] : 0.f;
-    {
-      const double bi = cum_l[mi];
-      f32x4 m;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) m[v] = mj + v <= mi ? pcb[v] * (__builtin_amdgcn_exp2f((float)(bi - cum_l[mj + v])) * dt_l[mj + v]) : 0.f;
-      *reinterpret_cast<f32x4*>(m_l + mi * TS + mj) = m;
-    }
-    if (__any(bad) && lane == 0) flag_l[par] = 1;
-    if (tid == 0) flag_l[par ^ 1] = 0;
-    __syncthreads();
-    const bool serial = flag_l[par] != 0;
-    if (l0 + L < n) fetch(l0 + L);
-    float* yo = a.work + (t0 + l0) * a.wld;
-    const uint32_t yc = (uint32_t)(h * E + e), yk = (uint32_t)(4 * kq) * (uint32_t)a.wld + yc;
-    if (!serial) {
-      f32x4 acc[LT] = {};
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        f32x4 av[LT];
-#pragma unroll
-        for (int i = 0; i < LT; ++i) av[i] = *reinterpret_cast<const f32x4*>(c_l + (16 * i + r16) * CS + 16 * t + 4 * kq);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = 0; i < LT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], S[t][s], acc[i], 0, 0, 0);
-        if (t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int i = 0; i < LT; ++i) acc[i] *= *reinterpret_cast<const f32x4*>(eb_l + 16 * i + 4 * kq);
-#pragma unroll
-      for (int k = 0; k < LT; ++k) {
-        f32x4 av[LT];
-#pragma unroll
-        for (int i = k; i < LT; ++i) av[i] = *reinterpret_cast<const f32x4*>(m_l + (16 * i + r16) * TS + 16 * k + 4 * kq);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = k; i < LT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], xr[4 * k + s], acc[i], 0, 0, 0);
-      }
-      if (cnt == L && wide) {
-#pragma unroll
-        for (int i = 0; i < LT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) (yo + (int64_t)(16 * i + r) * a.wld)[yk] = acc[i][r] + dskip * xr[4 * i + r];
-      } else {
-#pragma unroll
-        for (int i = 0; i < LT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (16 * i + 4 * kq + r < cnt && e_ok) (yo + (int64_t)(16 * i + r) * a.wld)[yk] = acc[i][r] + dskip * xr[4 * i + r];
-      }
-      const float keep = eb_l[L - 1];
-#pragma unroll
-      for (int k = 0; k < LT; ++k) {
-        const f32x4 wv = *reinterpret_cast<const f32x4*>(wt_l + 16 * k + 4 * kq);
-#pragma unroll
-        for (int s = 0; s < 4; ++s) xr[4 * k + s] *= wv[s];
-      }
-#pragma unroll
-      for (int t = 0; t < NT; t += 2) {
-        S[t] *= keep;
-        S[t + 1] *= keep;
-#pragma unroll
-        for (int k = 0; k < LT; ++k) {
-          f32x4 av[2];
-#pragma unroll
-          for (int i = 0; i < 2; ++i) av[i] = *reinterpret_cast<const f32x4*>(bt_l + (16 * (t + i) + r16) * TS + 16 * k + 4 * kq);
-#pragma unroll
-          for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) S[t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[i][s], xr[4 * k + s], S[t + i], 0, 0, 0);
+      for (int i = 0; i < HALO + 4; ++i) {
+        const int l = 16 * j + 4 * kq + i - HALO;
+        in[j][i] = 0.f;
+        if (e_ok && l < n) {
+          if (l >= 0) in[j][i] = Elem<T>::to_f(p[(int64_t)l * a.ld + r16]);
+          else if (first_pos > 0 && taps - 1 + l >= 0) in[j][i] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 + l) * C + h * E + e];
         }
-        __builtin_amdgcn_sched_barrier(0);
       }
-    } else {
-      // an infinity or a NaN in the chunk would reach the tokens in front of it through a product with a weight of zero: such a
-      // chunk goes token by token, S in the state row meanwhile (a rare path: it must not set the kernel's registers); x through
-      // LDS, a wave writes and reads its own columns
+    convolve(in, n, x, bad);
+  }
+  f32x4 A[2 * NT], M[3], eb[2], wv[2];
+  float flag;
 #pragma unroll
-      for (int j = 0; j < LT; ++j)
+  for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(f + 256 * i);
+  flag = f[2 * L * NP - 4 * lane];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) x_l[(16 * j + 4 * kq + s) * XS + 16 * w + r16] = xr[4 * j + s];
-      __syncthreads();
-      int rows = N, step = E;
-      asm volatile("" : "+s"(rows), "+s"(step));
-      if (e_ok) {
+  for (int i = 0; i < 3; ++i) M[i] = *reinterpret_cast<const f32x4*>(fh + 256 * i + 4 * lane);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    eb[i] = *reinterpret_cast<const f32x4*>(fh + 768 + 16 * i + 4 * kq);
+    wv[i] = *reinterpret_cast<const f32x4*>(fh + 768 + L + 16 * i + 4 * kq);
+  }
+  if (L < n) fetch_x(L);
+
+  for (int l0 = 0; l0 < n; l0 += L) {
+    const int cnt = n - l0 < L ? n - l0 : L;
+    const bool more = l0 + L < n;
+    const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
+    const float* fhn = fh + (more ? head_ld : 0);
+    float* yr = yo + (int64_t)l0 * a.wld;
+    // An infinity or a NaN in the chunk would reach the tokens in front of it through a product with a weight of zero: the wave takes
+    // such a chunk token by token behind the products, which then count for nothing, from S in the state row and x in LDS (a rare
+    // path: it must not set the kernel's registers)
+    const bool serial = __any(bad || flag != 0.f);
+    int rows = N, step = E;
+    asm volatile("" : "+s"(rows), "+s"(step));
+    if (serial) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = x[j][s];
+      if (e_ok)
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
-        __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    f32x4 xn[2];
+    {
+      const float keep = __shfl(eb[1][3], 63, 64);
+      f32x4 O[2] = {};
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[i * NT + t][s], S[t][s], O[i], 0, 0, 0);
+      // the next chunk's x between the products: a product keeps the matrix pipe for 32 cycles, in which a few of these fit
+      bad = false;
+      {
+        float in[2][HALO + 4];
+        if (vec) {
+          tile.place(in_l[w], lane);
+        } else {                                                 // (rows or columns that start off a 16-byte boundary: not fetched ahead)
+          for (int r = kq; r < L + HALO; r += 4)
+            in_l[w][r * RowTile<T>::kStride + r16] = e_ok && l0 + L - HALO + r < n ? p[(int64_t)(l0 + L - HALO + r) * a.ld + r16] : Elem<T>::from_f(0.f);
+        }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < HALO + 4; ++i) in[j][i] = Elem<T>::to_f(in_l[w][(16 * j + 4 * kq + i) * RowTile<T>::kStride + r16]);
+        convolve(in, n - l0 - L, xn, bad);
       }
+#pragma unroll
+      for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(f + L * NP + 256 * i);
+      flag = fn[2 * L * NP - 4 * lane];
+#pragma unroll
+      for (int i = 0; i < 8 * NT; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+      }
+      if (l0 + 2 * L < n) fetch_x(l0 + 2 * L);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) O[i] *= eb[i];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[i][s], x[0][s], O[i], 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) O[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[2][s], x[1][s], O[1], 0, 0, 0);
+      f32x4 U[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        O[i] += dskip * x[i];
+        U[i] = x[i] * wv[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) M[i] = *reinterpret_cast<const f32x4*>(fhn + 256 * i + 4 * lane);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        eb[i] = *reinterpret_cast<const f32x4*>(fhn + 768 + 16 * i + 4 * kq);
+        wv[i] = *reinterpret_cast<const f32x4*>(fhn + 768 + L + 16 * i + 4 * kq);
+      }
+      if (serial) {
+      } else if (cnt == L && vec) {
+        rec_store_tile(O, o_l[w], yr, a.wld, lane);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (16 * i + 4 * kq + r < cnt && e_ok) yr[(int64_t)(16 * i + 4 * kq + r) * a.wld + r16] = O[i][r];
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) S[t] *= keep;
+#pragma unroll
+      for (int t = 0; t < NT; t += 2)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) S[t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[2 * (t + i) + k][s], U[k][s], S[t + i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(fn + 256 * i);
+    }
+    if (serial) {
 #pragma unroll 1
       for (int t = 0; t < cnt; ++t) {
-        const float xv = x_l[t * XS + 16 * w + r16], dec = dec_l[t], dx = dt_l[t] * xv;
+        const float xv = o_l[w][t * kOutStride + r16], dt = fh[768 + 2 * L + t], dec = fh[768 + 3 * L + t], dx = dt * xv;
+        const float* cr = f - 4 * lane + (t >> 4) * NT * 256 + 4 * (16 * kq + (t & 15));           // row t of C: this lane group's four of every 16
+        const float* br = f - 4 * lane + L * NP + (t >> 4) * 256 + 4 * (16 * ((t & 15) >> 2) + 4 * kq) + (t & 3);     // column t of B^T
         float y = 0.f;
 #pragma unroll 1
         for (int u = 0; u < 4 * NT; ++u) {
           const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
           if (row < rows && e_ok) {
-            const float v = dec * st[row * step] + bt_l[row * TS + t] * dx;
+            const float v = dec * st[row * step] + br[(u >> 2) * 512 + 4 * (u & 3)] * dx;
             st[row * step] = v;
-            y += v * c_l[t * CS + row];
+            y += v * cr[(u >> 2) * 256 + (u & 3)];
           }
         }
         y += __shfl_xor(y, 16, 64);
         y += __shfl_xor(y, 32, 64);
-        if (kq == 0 && e_ok) yo[t * a.wld + yc] = y + dskip * xv;
+        if (kq == 0 && e_ok) yr[(int64_t)t * a.wld + r16] = y + dskip * xv;
       }
-      if (e_ok) {
 #pragma unroll
-        for (int t = 0; t < NT; ++t)
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (16 * t + 4 * kq + r < rows) S[t][r] = st[(16 * t + 4 * kq + r) * step];
-        __builtin_amdgcn_sched_barrier(0);
-      }
+        for (int r = 0; r < 4; ++r)
+          S[t][r] = e_ok && 16 * t + 4 * kq + r < rows ? st[(16 * t + 4 * kq + r) * step] : 0.f;
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __syncthreads();
+    x[0] = xn[0];
+    x[1] = xn[1];
+    f = fn;
+    fh = fhn;
   }
   int rows = N, step = E;
-  asm volatile("" : "+s"(rows), "+s"(step));                   // (nor their addresses)
+  asm volatile("" : "+s"(rows), "+s"(step));                     // (no addresses of 32 rows held over the loop)
   if (e_ok)
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = 16 * t + 4 * kq + r;
-        if (row < rows) st[row * step] = S[t][r];
-      }
+      for (int r = 0; r < 4; ++r)
+        if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
 }
 
 // gate, grouped norm, weight, one pass: a workgroup per (token, norm group), the group's elements in registers, 16-byte accesses
@@ -906,17 +844,16 @@ extern "C" int64_t semipd_state_space_work_width(int num_heads, int groups, int 
 // 256 rows 327 / 79; 32 requests of 8 rows 185 / 148, 32 rows 548 / 191, 256 rows 3058 / 782; 64 heads: 1 request of 12 rows 34.3 / 33.8,
 // 32 requests of 8 rows 110 / 88.
 constexpr int64_t kSsmChunkMinRows = 12;
-static int64_t ssm_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kSsmChunk + batch; }
 static int ssm_padded_state(int state_size) { return state_size <= 64 ? 64 : 128; }
 
-extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state_size, int v_dim, int taps) {
-  if (batch <= 0 || groups <= 0 || num_tokens < kSsmChunkMinRows * batch || state_size > 128 || v_dim % 8 != 0 || taps > kSsmChunkTaps) return 0;
-  return ssm_max_chunks(num_tokens, batch) * (groups * ssm_frag_elems(ssm_padded_state(state_size)) + (int64_t)num_heads * kSsmSteps);
+extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state_size, int taps) {
+  if (batch <= 0 || groups <= 0 || num_tokens < kSsmChunkMinRows * batch || state_size > 128 || taps > kRecTaps) return 0;
+  return rec_max_chunks(num_tokens, batch) * (groups * ssm_frag_elems(ssm_padded_state(state_size)) + (int64_t)num_heads * kSsmHead);
 }
 
 template <typename T, int NP>
 static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
-  const int64_t chunks = ssm_max_chunks(a.num_tokens, a.batch);
+  const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
   hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
   hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);
@@ -976,8 +913,8 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     else SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a))
     return 0;
   };
-  const int64_t want = q_start ? semipd_state_space_chunk_elems(num_tokens, batch, num_heads, groups, state_size, v_dim, taps) : 0;
-  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work) && x_off % 8 == 0 && ld % 8 == 0 && aligned16(proj)) {
+  const int64_t want = q_start ? semipd_state_space_chunk_elems(num_tokens, batch, num_heads, groups, state_size, taps) : 0;
+  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work)) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, if (state_size <= 64) launch_ssm_chunks<T, 64>(a, s); else launch_ssm_chunks<T, 128>(a, s));
     if (taps > 1) {
       const dim3 grid((unsigned)((C + 255) / 256), (unsigned)batch);

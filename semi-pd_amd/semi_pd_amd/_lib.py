@@ -190,7 +190,7 @@ _SIGNATURES = {
     "semipd_state_space_work_width": [_i32, _i32, _i32, _i32],
     "semipd_state_space": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _i64, _vp, _i64, _vp, _i64,
                            _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _i32, _vp],
-    "semipd_state_space_chunk_elems": [_i64, _i64, _i32, _i32, _i32, _i32, _i32],
+    "semipd_state_space_chunk_elems": [_i64, _i64, _i32, _i32, _i32, _i32],
     "semipd_state_space_prompt": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _i64, _vp, _i64, _vp, _i64,
                                   _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64, _i32, _vp],
     "semipd_outnorm_stream": [_vp, _i64, _vp, _i64, _vp, _f32, _f32, _vp, _f32, _f32, _vp, _i64, _i64, _i64, _i32, _vp],

@@ -2023,7 +2023,7 @@ def state_space(proj: torch.Tensor, z_off: int, x_off: int, dt_off: int, conv_w:
             ptr(d_skip), ptr(norm_weight), int(norm_groups), float(eps), ptr(work), wld, ptr(state), state.stride(0), ptr(conv_state),
             conv_state.stride(0) if conv_state is not None else 0, ptr(state_indices), ptr(seq_lens), ptr(q_start), ptr(q_len), B, T,
             num_heads, groups, state_size, v_dim, taps, ptr(out), out.stride(0))
-    elems = int(lib.semipd_state_space_chunk_elems(T, B, num_heads, groups, state_size, v_dim, taps)) if q_start is not None else 0
+    elems = int(lib.semipd_state_space_chunk_elems(T, B, num_heads, groups, state_size, taps)) if q_start is not None else 0
     if elems:         # a prompt batch: room for the operands of its chunks of 32 tokens
         chunk_work = torch.empty(elems, dtype=torch.float32, device=proj.device)
         check(lib.semipd_state_space_prompt(*args, ptr(chunk_work), elems, dtype_code(proj.dtype), current_stream(proj.device)), "state_space")
