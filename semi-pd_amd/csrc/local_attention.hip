@@ -1429,6 +1429,8 @@ __global__ void __launch_bounds__(64) local_attention_merge_kernel(LocalAttnArgs
 
 }  // namespace semipd
 
+#include "local_attention_prompt.h"
+
 using namespace semipd;
 
 static inline bool local_mfma_shape_ok(int qk_dim, int v_dim) {
@@ -1583,6 +1585,11 @@ static int launch_attention(LocalAttnArgs a, int64_t max_q_len, int form, int dt
         }
       }
       return launch_status("local_attention_decode");
+    }
+    if constexpr (!POOL) {
+      int rc = 0;
+      if (dtype == SEMIPD_BF16 ? prompt_attention<bf16_t>(a, as_stream(stream), rc) : prompt_attention<f16_t>(a, as_stream(stream), rc))
+        return rc ? rc : launch_status("prompt_attention");
     }
     a.n_tiles = (num_tokens + 63) / 64 + batch;
     const dim3 grid((unsigned)((a.n_tiles * num_q_heads + 7) / 8 * 8));

@@ -1,0 +1,307 @@
+// Prompt attention over paged pools, 32 query rows a wave (gfx950): the form of local_attention_mfma_kernel for head sizes of 64 or
+// 128 (value rows up to 256).  Included by local_attention.hip behind what it needs (LocalAttnArgs, ScoreMap, range_lo).
+//
+//  * A workgroup: NW waves = HW query heads of ONE key/value head x NW / HW blocks of 32 rows, so the rows of K and V that it
+//    stages serve up to NW heads.  Heads share the visible range, and every wave of a workgroup has the same number of steps.
+//  * A step: KT keys (64, or 32).  Their K and V rows go through two pairs of LDS tiles (step i + 1 lands in registers while step i is
+//    multiplied; one barrier a step).  S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16: a lane holds one query's column
+//    throughout, P^T goes from the accumulators into the second product in place (its key order is matched by the rows that the
+//    transposing reads of V take).
+//  * 16-byte chunk c of row r lies at c ^ (r & 15) of a K tile (the 32 rows of an operand read start in different banks), the 64-byte
+//    group t at t ^ (r & 3) of a V tile (the four rows of a transposing read likewise).
+//  * The running maximum is the row's own at every step, so its largest weight is 1 and rounds to 16 bits without an error: letting
+//    it lag by up to 2^6 (fewer rescalings: 7262 tokens in blocks of 1024 118 -> 114 us, value rows of 256 380 -> 331) was 2 .. 5 %
+//    further from the 64-bit result.
+// Bound: at 64 keys a wave multiplies for 32 x 32 cycles (128 / 128), reads 32 KB of LDS and takes 32 exponentials a lane (16 cycles
+// each) with five instructions around each: matrix pipe, LDS and vector unit are close to each other, two waves a SIMD fill each
+// other's gaps.  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves
+// of one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 260 -> 110 us (500 TFLOP/s); value rows of 256: 2030 -> 380 (steps
+// of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000: 69 -> 48; 8 x 40: 10.6 -> 9.8.  A fresh prompt of at most 20
+// tokens is one step of either, 7.7 -> 8.4 us; behind 100 tokens the same rows are 12.7 -> 10.0.
+#pragma once
+
+namespace semipd {
+
+template <typename T, int D, int E, int NW, int KT, bool SIG>
+__global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnArgs a, int hw) {
+  constexpr int NT = 64 * NW, KU = KT / 32;                     // KT: keys a step
+  constexpr int KB = D * 2, VB = E * 2, CK = D / 8, CV = E / 8;  // bytes and 16-byte chunks of a row
+  constexpr int NK = KT * CK / NT, NV = KT * CV / NT;          // chunks a thread stages
+  constexpr int KSW = CK < 16 ? CK - 1 : 15, VSW = E >= 128 ? 3 : 1;
+  constexpr int ET = E / 32;
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+  uint8_t* const k_lds = lds;                                   // [2][KT][KB]
+  uint8_t* const v_lds = lds + 2 * KT * KB;                     // [2][KT][VB]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
+  // Workgroup -> (kv head, tile, heads of the group), the last fastest, an XCD walking a contiguous range of items: the workgroups
+  // that read the same K and V rows run next to each other on one L2.  Tiles from the last (most keys) to the first.
+  const int rows_wg = 32 * (NW / hw);
+  const int rep = a.H / a.G, sets = rep / hw;
+  const int64_t n_items = gridDim.x, item = (int64_t)(blockIdx.x & 7) * (n_items >> 3) + (blockIdx.x >> 3);
+  const int64_t n_tiles = a.n_tiles;
+  if (item >= n_tiles * a.G * sets) return;
+  const int gk = (int)(item / (n_tiles * sets)), set = (int)(item % sets);
+  const int64_t tile_id = n_tiles - 1 - (item / sets) % n_tiles;
+  int b = -1;
+  int q0 = 0;
+  {
+    int64_t left = tile_id;
+    for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 8) {     // eight lengths per round trip
+      int32_t n[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) n[u] = rq0 + u < (int)a.batch ? a.q_len[rq0 + u] : 0;
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const int64_t tiles = ((int64_t)n[u] + rows_wg - 1) / rows_wg;
+        if (b < 0 && left < tiles) {
+          b = rq0 + u;
+          q0 = (int)left * rows_wg;
+        }
+        if (b < 0) left -= tiles;
+      }
+    }
+  }
+  if (b < 0) return;
+  b = __builtin_amdgcn_readfirstlane(b);
+  q0 = __builtin_amdgcn_readfirstlane(q0);
+  const int h = gk * rep + set * hw + wave % hw;
+  const int qn = a.q_len[b], base_pos = (int)(a.seq_lens[b] - qn);
+  const int64_t t0 = a.q_start[b];
+  const int keep = a.window > 0 ? a.keep_first : 0;
+  const int wg_last = min(q0 + rows_wg, qn) - 1;
+  const int key_lo = (int)range_lo(a, base_pos + q0), key_hi = base_pos + wg_last;
+  // this wave's 32 rows
+  const int wq0 = q0 + 32 * (wave / hw);
+  const bool wave_on = wq0 < qn;
+  const int wq_last = min(wq0 + 31, qn - 1);
+  const int w_first = base_pos + wq0, w_hi = base_pos + wq_last;
+  const int w_lo = (int)range_lo(a, w_first), w_full = (int)range_lo(a, w_hi);     // first key that any / every row of the wave sees
+  const bool q_ok = wq0 + col < qn;
+  const int my_q = q_ok ? wq0 + col : (wave_on ? wq_last : 0);
+  const int my_pos = q_ok ? base_pos + my_q : -1, my_lo = (int)range_lo(a, base_pos + my_q);
+  Frag16 qf[D / 16];
+  {
+    const T* q = (const T*)a.q + (t0 + my_q) * a.q_ld + (int64_t)h * D + hi * 8;
+#pragma unroll
+    for (int ks = 0; ks < D / 16; ++ks) qf[ks].u = *reinterpret_cast<const uint4*>(q + ks * 16);
+  }
+  f32x16 o[ET];
+#pragma unroll
+  for (int t = 0; t < ET; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o[t][r] = 0.f;
+  float m = -INFINITY, l = 0.f;
+  const ScoreMap smap(a.scale, a.cap);
+  const bool capped_scores = smap.A != 0.f;
+  const float c = capped_scores ? 1.0f : smap.c;                // what multiplies a score in the exponent
+  const float hb = (SIG && a.head_bias) ? a.head_bias[h] * kLog2e : 0.f;
+
+  // the walk: the kept first positions in front of the tile's range, then the range; steps of 64 keys, each within one of the two
+  const int n_first = keep < key_lo ? keep : key_lo;
+  const int first_steps = (n_first + KT - 1) / KT, steps = first_steps + (key_hi - key_lo) / KT + 1;
+  const int32_t* row = a.req_to_token + a.req_pool_indices[b] * a.r2t_stride;
+  const T* kp = (const T*)a.k_pool + (int64_t)gk * D;
+  const T* vp = (const T*)a.v_pool + (a.v_shared ? 0 : (int64_t)gk * E);
+  const int kr0 = tid / CK, kc = tid % CK, vr0 = tid / CV, vc = tid % CV;      // this thread's chunks: rows kr0 + i NT / CK, chunk kc
+  int k_slot[NK] = {}, v_slot[NV] = {};
+  u32x4 kv[NK], vv[NV];
+  auto load_slots = [&](int it) {
+    const bool first = it < first_steps;
+    const int j0 = first ? it * KT : key_lo + (it - first_steps) * KT, last = first ? n_first - 1 : key_hi;
+#pragma unroll
+    for (int i = 0; i < NK; ++i) k_slot[i] = row[min(j0 + kr0 + i * (NT / CK), last)];       // (past the end: the last key, masked)
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v_slot[i] = CV == CK ? k_slot[i < NK ? i : 0] : row[min(j0 + vr0 + i * (NT / CV), last)];
+  };
+  auto load_rows = [&]() {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) kv[i] = *reinterpret_cast<const u32x4*>(kp + (int64_t)k_slot[i] * a.k_ld + kc * 8);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) vv[i] = *reinterpret_cast<const u32x4*>(vp + (int64_t)v_slot[i] * a.v_ld + vc * 8);
+  };
+  auto store_rows = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+      const int r = kr0 + i * (NT / CK);
+      *reinterpret_cast<u32x4*>(k_lds + buf * KT * KB + r * KB + ((kc ^ (r & KSW)) << 4)) = kv[i];
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int r = vr0 + i * (NT / CV);
+      *reinterpret_cast<u32x4*>(v_lds + buf * KT * VB + r * VB + ((vc ^ ((r & VSW) << 2)) << 4)) = vv[i];
+    }
+  };
+  // operand addresses: K row `col` (+ 32), chunk 2 ks + hi; V rows 4 hi + gi / 4 (+ 8, + 16 s), columns 32 t + 16 g1 + 4 (gi & 3)
+  const int gi = lane & 15, g1 = (lane >> 4) & 1, vrow = 4 * hi + (gi >> 2);
+  const uint8_t* ka = k_lds + col * KB;
+  const uint8_t* va = v_lds + vrow * VB + g1 * 32 + (gi & 3) * 8;
+  const int kx = col & KSW, vx = vrow & VSW;
+
+  load_slots(0);
+  load_rows();
+  if (steps > 1) load_slots(1);
+  store_rows(0);
+  __syncthreads();
+  for (int it = 0; it < steps; ++it) {
+    const int buf = it & 1;
+    if (it + 1 < steps) {
+      load_rows();
+      if (it + 2 < steps) load_slots(it + 2);
+    }
+    const bool first = it < first_steps;
+    const int j0 = first ? it * KT : key_lo + (it - first_steps) * KT;
+    // 0: no row of the wave sees a key of the step; 2: every row sees all of them
+    const bool some = wave_on && (first || (j0 <= w_hi && (j0 + KT - 1 >= w_lo || j0 < keep)));
+    if (some) {
+      const uint8_t* kb = ka + buf * KT * KB;
+      const uint8_t* vb = va + buf * KT * VB;
+      f32x16 s[KU] = {};
+#pragma unroll
+      for (int ks = 0; ks < D / 16; ++ks) {
+        Frag16 kf[KU];
+#pragma unroll
+        for (int u = 0; u < KU; ++u) kf[u].u = *reinterpret_cast<const uint4*>(kb + u * 32 * KB + (((2 * ks + hi) ^ kx) << 4));
+#pragma unroll
+        for (int u = 0; u < KU; ++u) s[u] = Mfma<T>::mma(as_frag<T>(kf[u]), as_frag<T>(qf[ks]), s[u]);
+      }
+      if (capped_scores)
+#pragma unroll
+        for (int u = 0; u < KU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) s[u][r] = smap(s[u][r]);
+      const bool whole = first ? j0 + KT <= n_first : (j0 + KT - 1 <= w_first && j0 >= w_full);
+      if (!whole) {
+        // (row (r & 3) + 8 (r >> 2) + 4 hi of a 32-key block)
+        const int top = (first ? (q_ok ? n_first - 1 : -1) : my_pos) - j0 - 4 * hi, from = first ? -KT : my_lo - j0 - 4 * hi, kept = first ? 0 : keep - j0 - 4 * hi;
+#pragma unroll
+        for (int u = 0; u < KU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int j = 32 * u + (r & 3) + 8 * (r >> 2);
+            s[u][r] = j <= top && (j >= from || j < kept) ? s[u][r] : -INFINITY;
+          }
+      }
+      Frag16 p[2 * KU];                                              // keys 16 s + {0 .. 3, 8 .. 11} + 4 hi of this lane's column
+      if constexpr (SIG) {
+        // independent weights sigmoid(score + hb), base 2: a masked key has score -inf: exp2(+inf) = inf, 1 / inf = 0
+#pragma unroll
+        for (int u = 0; u < KU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            const float p0 = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-fmaf(s[u][r], c, hb)));
+            const float p1 = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-fmaf(s[u][r + 1], c, hb)));
+            p[2 * u + (r >> 3)].w[(r & 7) >> 1] = pack2<T>(p0, p1);
+          }
+      } else {
+        float mx = s[0][0];
+#pragma unroll
+        for (int u = 0; u < KU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[u][r]);
+        {
+          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+          mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c;        // (c > 0; -inf stays -inf)
+        }
+        if (__any(mx > m)) {
+          const float m_new = fmaxf(m, mx), alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
+          l *= alpha;
+#pragma unroll
+          for (int t = 0; t < ET; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+          m = m_new;
+        }
+        const float m_use = m == -INFINITY ? 0.f : m;
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < KU; ++u)
+#pragma unroll
+          for (int r = 0; r < 16; r += 2) {
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[u][r], c, -m_use)), p1 = __builtin_amdgcn_exp2f(fmaf(s[u][r + 1], c, -m_use));
+            sum += p0 + p1;
+            p[2 * u + (r >> 3)].w[(r & 7) >> 1] = pack2<T>(p0, p1);
+          }
+        l += sum;
+      }
+#pragma unroll
+      for (int s4 = 0; s4 < 2 * KU; ++s4)
+#pragma unroll
+        for (int t = 0; t < ET; ++t) {
+          Frag16 vf;
+          const uint8_t* vq = vb + s4 * 16 * VB + ((t ^ vx) << 6);
+          vf.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vq));
+          vf.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vq + 8 * VB));
+          o[t] = Mfma<T>::mma(as_frag<T>(vf), as_frag<T>(p[s4]), o[t]);
+        }
+    }
+    if (it + 1 < steps) store_rows(buf ^ 1);
+    __syncthreads();                                            // the next step's rows are in place, everyone is done with this step's
+  }
+  if constexpr (!SIG) {
+    const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
+    l = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
+    if (a.sink != nullptr) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e - m);
+  }
+  if (!wave_on) return;
+  const float inv = q_ok ? (SIG ? a.out_scale : a.out_scale / l) : 0.f;
+  // out through the wave's part of the tiles (the walk ended on a barrier): a lane holds four neighbouring elements of one row at a
+  // time, rows leave in 16-byte pieces of consecutive lanes
+  constexpr int OS = E * 2 + 16;
+  uint8_t* ol = lds + wave * 32 * OS;
+#pragma unroll
+  for (int t = 0; t < ET; ++t)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+      uint2 w;
+      w.x = pack2<T>(o[t][r] * inv, o[t][r + 1] * inv);
+      w.y = pack2<T>(o[t][r + 2] * inv, o[t][r + 3] * inv);
+      *reinterpret_cast<uint2*>(ol + col * OS + (32 * t + 2 * r + 4 * hi) * 2) = w;
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 4
+  for (int i = lane; i < 32 * CV; i += 64) {
+    const int rr = i / CV, ec = i % CV;
+    if (wq0 + rr >= qn) break;
+    Vec16<T> v = *reinterpret_cast<const Vec16<T>*>(ol + rr * OS + ec * 16);
+    const int64_t t = t0 + wq0 + rr;
+    if (a.gate) {
+      const Vec16<T> gv = load16((const T*)a.gate + t * a.gate_ld + (int64_t)h * E + ec * 8);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        v.e[u] = Elem<T>::from_f(Elem<T>::to_f(v.e[u]) * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * Elem<T>::to_f(gv.e[u]))));
+    }
+    store16((T*)a.out + t * a.out_ld + (int64_t)h * E + ec * 8, v);
+  }
+}
+
+// true: launched.  Head sizes 64 / 64, 64 / 128, 128 / 128, 128 / 256 (sigmoid weights: 64 / 64, 128 / 128), a positive scale, 16-bit
+// types, everything aligned as local_attention_mfma_kernel wants it.
+template <typename T, int D, int E, int NW, int KT, bool SIG>
+static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
+  const int rep = a.H / a.G;
+  int hw = NW;
+  while (rep % hw) hw >>= 1;
+  const int rows = 32 * (NW / hw);
+  a.n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
+  constexpr size_t tiles = 2 * KT * (size_t)(D + E) * 2, epilogue = NW * 32 * (size_t)(E * 2 + 16), bytes = tiles > epilogue ? tiles : epilogue;
+  static std::atomic<uint64_t> done{0};
+  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
+  const int64_t items = a.n_tiles * a.G * (rep / hw);
+  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, SIG>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(64 * NW), bytes, s, a, hw);
+  return 0;
+}
+template <typename T>
+static bool prompt_attention(const LocalAttnArgs& a, hipStream_t s, int& rc) {
+  const bool sig = a.sigmoid != 0;
+  if (!(a.scale > 0.f)) return false;
+  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, false>(a, s);
+  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, false>(a, s);
+  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, false>(a, s);
+  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, false>(a, s);
+  else return false;
+  return true;
+}
+
+}  // namespace semipd

@@ -314,10 +314,10 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
 // rounded to 16 bits); b is summed, and its differences are taken, in 64 bits, so a weight near 1 behind a strong decay is as
 // good as the product of the decays themselves.
 // Bound: token by token a step is a chain of LDS reads, 64 multiply-adds and lane sums (1.0 us of a wave's time; 7262 tokens of 4
-// requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (36 GFLOP at
-// 154 TFLOP/s = 235 us) and the vector work between its products: 560 us, operands 73.  Chunks of 32 and not 64: the same products
-// with S, half the ones inside a chunk, and three workgroups' LDS on a CU in place of one (64 tokens, two heads a workgroup: 952 us).
-
+// requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (140 products
+// of 32 cycles a wave and chunk: 250 us here), the vector work between its products and their loads: 545 us, operands 72.  Chunks of
+// 32 and not 64: the same products with S, half the ones inside a chunk; operands straight into registers and not through LDS: no
+// barriers, 560 -> 545 (64 tokens, operands in LDS, two heads a workgroup: 952 us).
 // fp32 elements of the operands of one (chunk, group): C and B^T as left-hand operands of 16 x 16 x 16 products, in the order in which
 // they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a piece of 4.  Of one
 // (chunk, head): tiles 00, 10, 11 of the weighted C B^T, then e^(b_t) | e^(b_last - b_t) dt_t | dt | decay.

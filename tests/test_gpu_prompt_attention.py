@@ -1,0 +1,109 @@
+"""Prompt attention with 32 query rows a wave (csrc/local_attention_prompt.h) against a dense softmax / sigmoid in 64 bits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# heads over key/value heads: four heads a workgroup, two, one (three heads of a group), sixteen
+GROUPS = {"4": (8, 2), "2": (4, 2), "3": (6, 2), "16": (16, 1)}
+
+
+def _batch(lens, olds, H, G, D, E, dtype, seed, shared=False):
+    g = torch.Generator().manual_seed(seed)
+    totals = [n + m for n, m in zip(lens, olds)]
+    slots = torch.randperm(sum(totals), generator=g) + 1
+    table, at = torch.zeros(len(lens), max(totals), dtype=torch.int32), 0
+    for b, n in enumerate(totals):
+        table[b, :n] = slots[at: at + n]
+        at += n
+    t = dict(q=torch.randn(sum(lens), H * D, generator=g).to(dtype), k=torch.randn(sum(totals) + 1, G, D, generator=g).to(dtype),
+             v=torch.randn(sum(totals) + 1, G, E, generator=g).to(dtype), table=table, totals=totals)
+    return t, g
+
+
+def _dense(t, lens, olds, H, G, D, E, see, weights, shared=False):
+    out, at = [], 0
+    for b, (n, m) in enumerate(zip(lens, olds)):
+        rows = t["table"][b, : n + m].long()
+        p, j = torch.arange(m, m + n)[:, None], torch.arange(n + m)[None]
+        ok = see(p, j)
+        heads = []
+        for h in range(H):
+            gk = h // (H // G)
+            s = t["q"][at: at + n, h * D: (h + 1) * D].double() @ t["k"][rows, gk].double().t() * D ** -0.5
+            v = t["v"][rows].double().reshape(n + m, -1) if shared else t["v"][rows, gk].double()
+            heads.append(weights(s, ok, h) @ v)
+        out.append(torch.stack(heads, 1))
+        at += n
+    return torch.cat(out).reshape(sum(lens), -1)
+
+
+def _softmax(sink=None, cap=0.0):
+    def f(s, ok, h):
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        s = s.masked_fill(~ok, -float("inf"))
+        if sink is None:
+            return torch.softmax(s, -1)
+        return torch.softmax(torch.cat([s, sink[h].double().expand(s.shape[0], 1)], 1), -1)[:, :-1]
+    return f
+
+
+# rows: one tile of 32, its edges, several; keys: a step of 64 and its edges, behind cached tokens, a block / window edge inside a step
+CASES = [([1, 33, 64], [0, 0, 5]), ([31, 129], [100, 0]), ([70], [63])]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,olds", CASES)
+@pytest.mark.parametrize("group,D", [("4", 128), ("2", 64), ("3", 128), ("16", 64)])
+@pytest.mark.parametrize("form", ["block", "causal", "cap", "window", "keep", "sigmoid"])
+def test_prompt_attention(dtype, lens, olds, group, D, form):
+    """Weights are rounded to 16 bits once (half a unit in the last place each, independent) and so is the result: 1.5 units of the
+    largest partial sums, which are a few times the result's own size."""
+    from semi_pd_amd import ops
+    H, G = GROUPS[group]
+    t, g = _batch(lens, olds, H, G, D, D, dtype, H * D + len(lens))
+    per_head, gate = torch.randn(H, generator=g), torch.randn(sum(lens), H * D, generator=g).to(dtype)
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+    out = torch.empty_like(d["q"])
+    batch = (d["q"], out, d["k"], d["v"], d["table"], torch.arange(len(lens), device=DEV), torch.tensor(t["totals"], device=DEV), start.to(DEV),
+             n.to(DEV), max(lens), D ** -0.5)
+    head = per_head.to(DEV)
+    if form == "block":
+        ops.local_attention_fwd(*batch, 0.0, 48, head, gate.to(DEV))
+        want = _dense(t, lens, olds, H, G, D, D, lambda p, j: (j <= p) & (j // 48 == p // 48), _softmax(per_head)) * torch.sigmoid(gate.double())
+    elif form in ("causal", "cap"):
+        cap = 2.0 if form == "cap" else 0.0
+        ops.local_attention_fwd(*batch, cap, 0, None, None)
+        want = _dense(t, lens, olds, H, G, D, D, lambda p, j: j <= p, _softmax(cap=cap))
+    else:
+        keep = 0 if form == "window" else 70 if form == "keep" else 3
+        see = lambda p, j: (j <= p) & ((p - j < 40) | (j < keep))          # noqa: E731
+        if form == "sigmoid":
+            ops.window_attention_fwd(*batch, 40, keep, head, True, None, 1.2)
+            want = _dense(t, lens, olds, H, G, D, D, see, lambda s, ok, h: 1.2 * torch.sigmoid(s + per_head[h].double()).masked_fill(~ok, 0.0))
+        else:
+            ops.window_attention_fwd(*batch, 40, keep, None, False, head, 1.0)
+            want = _dense(t, lens, olds, H, G, D, D, see, _softmax(per_head))
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    err = (out.cpu().double() - want).norm() / want.norm()
+    assert float(err) < 1.5 * ulp, float(err)
+    torch.testing.assert_close(out.cpu().double(), want, rtol=6 * ulp, atol=12 * ulp)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("lens,olds", CASES)
+@pytest.mark.parametrize("H,G,D", [(16, 2, 128), (6, 2, 128), (8, 2, 64)])
+def test_prompt_attention_over_shared_values(dtype, lens, olds, H, G, D):
+    from semi_pd_amd import ops
+    t, g = _batch(lens, olds, H, G, D, D, dtype, H * D)
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+    out = torch.empty(sum(lens), H * G * D, dtype=dtype, device=DEV)
+    ops.shared_value_attention_fwd(d["q"], out, d["k"], d["v"], d["table"], torch.arange(len(lens), device=DEV),
+                                   torch.tensor(t["totals"], device=DEV), start.to(DEV), n.to(DEV), max(lens), D ** -0.5)
+    want = _dense(t, lens, olds, H, G, D, D, lambda p, j: j <= p, _softmax(), shared=True)
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert float((out.cpu().double() - want).norm() / want.norm()) < 1.5 * ulp
+    torch.testing.assert_close(out.cpu().double(), want, rtol=6 * ulp, atol=12 * ulp)
