@@ -460,6 +460,64 @@ __global__ void __launch_bounds__(256) talk_mix_kernel(const T* __restrict__ par
 }
 
 // ------------------------------------------------------------------------------------------------ shared pieces
+// The same for 16-bit types on the matrix cores, fp32 operands and sums (v_mfma_f32_16x16x4_f32): out^T = parts^T talk^T, 16 elements
+// by up to 16 heads of one key/value head a tile, the tiles of a token taken by the four waves in turn.  The token's row of `parts`
+// lies in LDS once (16 bytes of padding behind every head: the rows that the four lane groups read start in different banks), the
+// result leaves by way of LDS in 16-byte pieces.  Bound: an element of the row is multiplied for the H / G heads of its key/value
+// head; on the vector unit every product was an LDS read of its own (7262 tokens, 32 heads over 2 of 128: 158 us -> 64, 178 MB).
+template <typename T, int KT>           // heads up to 16 KT
+__global__ void __launch_bounds__(256) talk_mix_mfma_kernel(const T* __restrict__ parts, int64_t p_ld, const float* __restrict__ talk,
+                                                            T* __restrict__ out, int64_t out_ld, int H, int G, int E) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t mix_b[];     // H rows of G * E elements + 16 bytes | out [H * E]
+  const int64_t t = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+  const int row = G * E, rs = row * 2 + 16, per = H / G, pieces = row / 8;
+  const T* p = parts + t * p_ld;
+  {
+    const int dr = 256 / pieces, dc = 256 % pieces;
+    int r = tid / pieces, c = tid % pieces;
+#pragma unroll 4
+    for (int i = tid; i < H * pieces; i += 256) {
+      *reinterpret_cast<uint4*>(mix_b + r * rs + c * 16) = *reinterpret_cast<const uint4*>(p + (int64_t)i * 8);
+      r += dr;
+      c += dc;
+      if (c >= pieces) {
+        c -= pieces;
+        ++r;
+      }
+    }
+  }
+  T* o_l = reinterpret_cast<T*>(mix_b + (size_t)H * rs);
+  __syncthreads();
+  const int ht = (per + 15) / 16, et = E / 16;
+  const uint8_t* ap = mix_b + 4 * kq * rs + r16 * 2;
+  for (int ch = 0; ch < G * ht; ++ch) {
+    const int c = ch / ht, h0 = c * per + (ch - c * ht) * 16;
+    const bool h_ok = h0 + r16 < (c + 1) * per;
+    float bv[KT][4];                                            // talk[head r16][16 k + 4 kq + s]
+#pragma unroll
+    for (int k = 0; k < KT; ++k)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) bv[k][s] = h_ok && 16 * k + 4 * kq + s < H ? talk[(int64_t)(h0 + r16) * H + 16 * k + 4 * kq + s] : 0.f;
+    for (int e = wave; e < et; e += 4) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      const uint8_t* ae = ap + (c * E + e * 16) * 2;
+      float av[KT][4];
+#pragma unroll
+      for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) av[k][s] = 16 * k + 4 * kq + s < H ? Elem<T>::to_f(*reinterpret_cast<const T*>(ae + (16 * k + s) * rs)) : 0.f;
+#pragma unroll
+      for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[k][s], bv[k][s], acc, 0, 0, 0);
+      if (h_ok) *reinterpret_cast<uint2*>(o_l + (h0 + r16) * E + e * 16 + 4 * kq) = uint2{pack2<T>(acc[0], acc[1]), pack2<T>(acc[2], acc[3])};
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < H * E / 8; i += 256) *reinterpret_cast<uint4*>(out + t * out_ld + i * 8) = *reinterpret_cast<const uint4*>(o_l + i * 8);
+}
+
 struct LocalAttnArgs {
   const void* q; int64_t q_ld;
   const void* gate; int64_t gate_ld;
@@ -1811,6 +1869,19 @@ extern "C" int semipd_talk_mix(const void* parts, int64_t parts_ld, const float*
   SEMIPD_CHECK_ARG(parts && talk && out && parts_ld >= (int64_t)num_q_heads * num_kv_heads * v_dim &&
                        out_ld >= (int64_t)num_q_heads * v_dim,
                    SEMIPD_EINVAL, "talk_mix: null pointer or rows too short");
+  const size_t held = (size_t)num_q_heads * ((size_t)num_kv_heads * v_dim * 2 + 16) + (size_t)num_q_heads * v_dim * 2;
+  if ((dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
+      aligned16(out) && held <= 65536 && num_q_heads <= 64) {
+    SEMIPD_DISPATCH_HALF(dtype, T, {
+      if (num_q_heads <= 32)
+        hipLaunchKernelGGL((talk_mix_mfma_kernel<T, 2>), dim3((unsigned)num_tokens), dim3(256), held, as_stream(stream), (const T*)parts,
+                           parts_ld, talk, (T*)out, out_ld, num_q_heads, num_kv_heads, v_dim);
+      else
+        hipLaunchKernelGGL((talk_mix_mfma_kernel<T, 4>), dim3((unsigned)num_tokens), dim3(256), held, as_stream(stream), (const T*)parts,
+                           parts_ld, talk, (T*)out, out_ld, num_q_heads, num_kv_heads, v_dim);
+    });
+    return launch_status("talk_mix");
+  }
   const size_t staged = ((size_t)num_q_heads * num_q_heads + (size_t)num_q_heads * num_kv_heads * v_dim) * sizeof(float);
   SEMIPD_DISPATCH_DTYPE(dtype, T, {
     if (staged <= 65536)

@@ -107,3 +107,20 @@ def test_prompt_attention_over_shared_values(dtype, lens, olds, H, G, D):
     ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     assert float((out.cpu().double() - want).norm() / want.norm()) < 1.5 * ulp
     torch.testing.assert_close(out.cpu().double(), want, rtol=6 * ulp, atol=12 * ulp)
+
+
+# heads over one and two tiles of 16 a key/value head, sums over one to four steps of 16, neither whole
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,E", [(32, 2, 128), (24, 2, 64), (40, 4, 16), (33, 1, 32), (64, 2, 16), (6, 3, 48)])
+def test_talk_mix(dtype, H, G, E):
+    """fp32 products and sums of at most 64 terms, the result rounded once.  With p significant bits half a unit in the last place of x is
+    at most 2^-p |x| (just above a power of two): 2^-8 for bf16, 2^-11 for fp16; the sum: 64 roundings of 2^-24 of its terms."""
+    from semi_pd_amd import ops
+    g = torch.Generator().manual_seed(H + E)
+    parts, talk = torch.randn(5, H * G * E, generator=g).to(dtype), torch.randn(H, H, generator=g)
+    out = ops.talk_mix(parts.to(DEV), talk.to(DEV), G).cpu().double().view(5, H, E)
+    x = parts.double().view(5, H, G, E)[:, :, torch.arange(H) // (H // G)]                    # [t, g, c(h), e]
+    want = torch.einsum("hg,tghe->the", talk.double(), x)
+    terms = torch.einsum("hg,tghe->the", talk.double().abs(), x.abs())
+    half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert bool(((out - want).abs() <= half * want.abs() + 64 * 2.0 ** -24 * terms + 1e-7).all())
