@@ -21,6 +21,7 @@
 //  * Prompt batches: ssm_chunk_operands_kernel and ssm_chunk_walk_kernel in place of the three, 32 tokens at a time on the matrix
 //    cores, every operand and sum fp32.
 //  * ssm_post_kernel / ssm_post_vec_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
+//  * ssm_step_kernel: batches of one token per request in place of preparation and recurrence, a workgroup per (head, request).
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
 #include "common.h"
 #include "recurrent_chunks.h"
@@ -772,6 +773,68 @@ __global__ void __launch_bounds__(256) ssm_post_kernel(SsmArgs a) {
   ssm_gate_norm_store<T>(a, a.work + t * a.wld, (const T*)a.p + t * a.ld + a.z_off, (T*)a.out + t * a.out_ld, red);
 }
 
+// ---------------------------------------------------------------------------------- one token per request, a state of some size
+// A workgroup per (head, request): the head's x, B and C channels through the convolution into LDS, step size and decay, then S in
+// 16-byte pieces, all of a thread's pieces in flight from the start: thread = four columns and every 1024 / E-th row, a step
+// per piece, the read-out summed over lanes and waves.  B and C are convolved again for every head of a group (2 N channels of
+// 4 taps: nothing against N E of state).  Bound by HBM, the state read and written once: 32 requests, 128 heads of 128 x 64 (268 MB):
+// the recurrence's kernel for prompts, which waited for one row per lane and step of its chain, 110 us + 10 of preparation -> 50.
+template <typename T, int NIT>
+__global__ void __launch_bounds__(256) ssm_step_kernel(SsmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];       // x [E] | B [N] | C [N] | sums [4][E]
+  const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int64_t first_pos = a.seq_lens[b] - 1;
+  if (first_pos < 0) return;
+  const bool fresh = first_pos == 0;
+  const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, g = h / (H / G);
+  const int inner = H * E, C = inner + 2 * G * N, quads = E / 4, rows = 256 / quads;
+  const int64_t slot = a.state_indices[b];
+  float* st = a.state + slot * a.state_ld + (int64_t)h * N * E;
+  const int n0 = tid / quads, e = tid % quads * 4;
+  float4 S[NIT];
+#pragma unroll
+  for (int i = 0; i < NIT; ++i) {
+    const int n = n0 + i * rows;
+    S[i] = (!fresh && n < N) ? *reinterpret_cast<const float4*>(st + n * E + e) : float4{0.f, 0.f, 0.f, 0.f};
+  }
+  const T* p = (const T*)a.p + (int64_t)b * a.ld;
+  const float* cs = a.conv_state + slot * a.conv_ld;
+  for (int i = tid; i < E + 2 * N; i += 256) {
+    const int c = i < E ? h * E + i : inner + (i < E + N ? g * N + (i - E) : G * N + g * N + (i - E - N));
+    const T* cw = (const T*)a.conv_w + (int64_t)c * taps;
+    float y = (a.conv_b ? Elem<T>::to_f(((const T*)a.conv_b)[c]) : 0.f) + Elem<T>::to_f(cw[taps - 1]) * Elem<T>::to_f(p[a.x_off + c]);
+    if (!fresh)
+      for (int k = 1; k < taps; ++k) y += Elem<T>::to_f(cw[taps - 1 - k]) * cs[(int64_t)(taps - 1 - k) * C + c];
+    lds[i] = ssm_silu(y);
+  }
+  const float dt = ssm_softplus(Elem<T>::to_f(p[a.dt_off + h]) + a.dt_bias[h]), dec = expf(-expf(a.a_log[h]) * dt);
+  __syncthreads();
+  const float4 x = *reinterpret_cast<const float4*>(lds + e);
+  const float4 dx = {dt * x.x, dt * x.y, dt * x.z, dt * x.w};
+  float4 y = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < NIT; ++i) {
+    const int n = n0 + i * rows;
+    if (n < N) {
+      const float bv = lds[E + n], cv = lds[E + N + n];
+      S[i] = float4{dec * S[i].x + bv * dx.x, dec * S[i].y + bv * dx.y, dec * S[i].z + bv * dx.z, dec * S[i].w + bv * dx.w};
+      *reinterpret_cast<float4*>(st + n * E + e) = S[i];
+      y = float4{y.x + S[i].x * cv, y.y + S[i].y * cv, y.z + S[i].z * cv, y.w + S[i].w * cv};
+    }
+  }
+  for (int o = quads; o < 64; o <<= 1) {
+    y.x += __shfl_xor(y.x, o, 64);
+    y.y += __shfl_xor(y.y, o, 64);
+    y.z += __shfl_xor(y.z, o, 64);
+    y.w += __shfl_xor(y.w, o, 64);
+  }
+  float* sums = lds + E + 2 * N;
+  if (lane < quads) *reinterpret_cast<float4*>(sums + (tid >> 6) * E + e) = y;
+  __syncthreads();
+  if (tid < E)
+    a.work[(int64_t)b * a.wld + h * E + tid] = (sums[tid] + sums[E + tid]) + (sums[2 * E + tid] + sums[3 * E + tid]) + (a.d_skip ? a.d_skip[h] : 0.f) * lds[tid];
+}
+
 // ---------------------------------------------------------------------------------- one token per request: one launch
 // A workgroup per request: convolution of the token's channels into LDS (and the shifted inputs back into the state row),
 // step sizes and decays, then thread (h, e) walks column e of head h's S in the state row (N multiply-adds for the update,
@@ -922,6 +985,24 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     }
     if (post()) return SEMIPD_EDTYPE;
     return launch_status("state_space(chunks)");
+  }
+  // a decode batch whose state rows lie on 16-byte boundaries: up to 16 pieces of four columns a thread
+  const bool pow2 = v_dim >= 16 && v_dim <= 256 && (v_dim & (v_dim - 1)) == 0;
+  if (q_start == nullptr && batch <= 65535 && pow2 && (int64_t)state_size * v_dim <= 16 * 1024 && state_size % 4 == 0 && aligned16(state) && state_ld % 4 == 0) {
+    const int nit = (state_size * v_dim + 1023) / 1024;
+    const size_t bytes = (size_t)(v_dim + 2 * state_size + 4 * v_dim) * sizeof(float);
+    const dim3 grid((unsigned)num_heads, (unsigned)batch);
+    SEMIPD_DISPATCH_DTYPE(dtype, T, {
+      if (nit <= 4) hipLaunchKernelGGL((ssm_step_kernel<T, 4>), grid, dim3(256), bytes, s, a);
+      else if (nit <= 8) hipLaunchKernelGGL((ssm_step_kernel<T, 8>), grid, dim3(256), bytes, s, a);
+      else hipLaunchKernelGGL((ssm_step_kernel<T, 16>), grid, dim3(256), bytes, s, a);
+    });
+    if (taps > 1) {
+      const dim3 cgrid((unsigned)((C + 255) / 256), (unsigned)batch);
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), cgrid, dim3(256), 0, s, a));
+    }
+    if (post()) return SEMIPD_EDTYPE;
+    return launch_status("state_space(step)");
   }
   const unsigned cblocks = (unsigned)((C + kPrepChannels - 1) / kPrepChannels);
   // four channels per thread: every row and column range starts on a multiple of four elements

@@ -45,27 +45,28 @@ def _ssm_truth(w, row, state, before, H, G, N, E, parts, eps=1e-5):
     return (v / (v.square().mean(-1, keepdim=True) + eps).sqrt()).view(-1, inner) * w["norm"].to(F64), S, last
 
 
-def _ssm_run(w, rows, state, before, first, H, G, N, E, parts, eps=1e-5):
+def _ssm_run(w, rows, state, before, first, H, G, N, E, parts, eps=1e-5, decode=False):
     from semi_pd_amd import ops
     inner, C, taps = H * E, H * E + 2 * G * N, w["conv"].shape[1]
     B = len(rows)
     lens = [r.shape[0] for r in rows]
     sw, cw = inner * N, (taps - 1) * C
-    slab = torch.full((B + 1, 3 + sw + cw + 2), 7.0, device=DEV)                   # (column ranges that start on odd elements)
-    slab[1:, 3: 3 + sw] = state.reshape(B, -1).to(DEV)
-    slab[1:, 3 + sw: 3 + sw + cw] = before.reshape(B, -1).to(DEV)
+    lo = 4 if decode else 3                                                         # (column ranges that start on odd elements)
+    slab = torch.full((B + 1, -(-(lo + sw + cw + 2) // 4) * 4 + lo % 4), 7.0, device=DEV)
+    slab[1:, lo: lo + sw] = state.reshape(B, -1).to(DEV)
+    slab[1:, lo + sw: lo + sw + cw] = before.reshape(B, -1).to(DEV)
     start, at = [], 0
     for n in lens:
         start.append(at)
         at += n
     d = {k: v.to(DEV) for k, v in w.items()}
+    start, n = torch.tensor(start, dtype=torch.int32, device=DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
     out = ops.state_space(torch.cat(rows).to(DEV), 0, inner, inner + C, d["conv"], d["bias"], d["dt_bias"], d["a_log"], d["skip"], d["norm"],
-                          parts, eps, slab[:, 3: 3 + sw], slab[:, 3 + sw: 3 + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
-                          torch.tensor([n + f for n, f in zip(lens, first)], device=DEV), torch.tensor(start, dtype=torch.int32, device=DEV),
-                          torch.tensor(lens, dtype=torch.int32, device=DEV), H, G, N, E)
+                          parts, eps, slab[:, lo: lo + sw], slab[:, lo + sw: lo + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
+                          torch.tensor([x + f for x, f in zip(lens, first)], device=DEV), None if decode else start, None if decode else n, H, G, N, E)
     slab = slab.cpu()
-    assert bool((slab[0] == 7).all() and (slab[:, :3] == 7).all() and (slab[:, -2:] == 7).all())
-    return out.cpu().split(lens), slab[1:, 3: 3 + sw].view(B, H, N, E), slab[1:, 3 + sw: 3 + sw + cw].view(B, taps - 1, C)
+    assert bool((slab[0] == 7).all() and (slab[:, :lo] == 7).all() and (slab[:, lo + sw + cw:] == 7).all())
+    return out.cpu().split(lens), slab[1:, lo: lo + sw].view(B, H, N, E), slab[1:, lo + sw: lo + sw + cw].view(B, taps - 1, C)
 
 
 # (sizes: rows of S in and below a padded block, columns over one and two workgroups, a group of three heads; two heads a
@@ -98,6 +99,25 @@ def test_state_space_in_chunks_strong_decays():
     want, S, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
     assert float((outs[0].to(F64) - want).norm() / want.norm()) < 2e-6
     assert float((after[0].to(F64) - S).norm() / S.norm()) < 2e-6
+
+
+# (one, some and all rows of pieces; E over part of a wave and over all four; several steps of the same requests)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,N,E,taps,parts", [(16, 2, 128, 64, 4, 1), (96, 3, 20, 32, 2, 3), (8, 8, 64, 256, 1, 8), (40, 5, 100, 16, 4, 1)])
+def test_state_space_decode_step(dtype, H, G, N, E, taps, parts):
+    w, rows, state, before = _ssm_inputs(H, G, N, E, taps, [1, 1, 1], dtype, 3)
+    first = [5, 0, 900]
+    ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dtype]
+    for step in range(2):
+        outs, after, last = _ssm_run(w, rows, state, before, first, H, G, N, E, parts, decode=True)
+        for b in range(3):
+            zero = first[b] == 0
+            want, S, tail = _ssm_truth(w, rows[b], torch.zeros_like(state[b]) if zero else state[b],
+                                       torch.zeros_like(before[b]) if zero else before[b], H, G, N, E, parts)
+            torch.testing.assert_close(outs[b].to(F64), want, rtol=ulp + 2e-5, atol=2e-5)
+            torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+            torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+        state, before, first = after.clone(), last.clone(), [f + 1 for f in first]
 
 
 @pytest.mark.parametrize("col", ["x", "B", "dt"])
@@ -149,27 +169,28 @@ def _delta_truth(w, row, state, before, H, G, D, E, eps=1e-5):
     return o.reshape(n, hv) * torch.nn.functional.silu(x[:, 2 * gd + hv: 2 * gd + 2 * hv]), S, last
 
 
-def _delta_run(w, rows, state, before, first, H, G, D, E, eps=1e-5):
+def _delta_run(w, rows, state, before, first, H, G, D, E, eps=1e-5, decode=False):
     from semi_pd_amd import ops
     gd, hv, taps, B = G * D, H * E, w["cq"].shape[1], len(rows)
     lens = [r.shape[0] for r in rows]
     sw, cw = H * D * E, (taps - 1) * (2 * gd + hv)
-    slab = torch.full((B + 1, 3 + sw + cw + 2), 7.0, device=DEV)
-    slab[1:, 3: 3 + sw] = state.reshape(B, -1).to(DEV)
-    slab[1:, 3 + sw: 3 + sw + cw] = before.reshape(B, -1).to(DEV)
+    lo = 4 if decode else 3
+    slab = torch.full((B + 1, -(-(lo + sw + cw + 2) // 4) * 4 + lo % 4), 7.0, device=DEV)
+    slab[1:, lo: lo + sw] = state.reshape(B, -1).to(DEV)
+    slab[1:, lo + sw: lo + sw + cw] = before.reshape(B, -1).to(DEV)
     start, at = [], 0
     for n in lens:
         start.append(at)
         at += n
     d = {k: v.to(DEV) for k, v in w.items()}
     offs = [0, gd, 2 * gd, 2 * gd + hv, 2 * gd + 2 * hv, 2 * gd + 2 * hv + H]
-    out = ops.delta_rule(torch.cat(rows).to(DEV), offs, d["cq"], d["ck"], d["cv"], d["a_log"], d["dt_bias"], d["norm"], eps, slab[:, 3: 3 + sw],
-                         slab[:, 3 + sw: 3 + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
-                         torch.tensor([n + f for n, f in zip(lens, first)], device=DEV), torch.tensor(start, dtype=torch.int32, device=DEV),
-                         torch.tensor(lens, dtype=torch.int32, device=DEV), H, G, D, E)
+    start, n = torch.tensor(start, dtype=torch.int32, device=DEV), torch.tensor(lens, dtype=torch.int32, device=DEV)
+    out = ops.delta_rule(torch.cat(rows).to(DEV), offs, d["cq"], d["ck"], d["cv"], d["a_log"], d["dt_bias"], d["norm"], eps, slab[:, lo: lo + sw],
+                         slab[:, lo + sw: lo + sw + cw] if cw else None, torch.arange(1, B + 1, device=DEV),
+                         torch.tensor([x + f for x, f in zip(lens, first)], device=DEV), None if decode else start, None if decode else n, H, G, D, E)
     slab = slab.cpu()
-    assert bool((slab[0] == 7).all() and (slab[:, :3] == 7).all() and (slab[:, -2:] == 7).all())
-    return out.cpu().split(lens), slab[1:, 3: 3 + sw].view(B, H, D, E), slab[1:, 3 + sw: 3 + sw + cw].view(B, taps - 1, 2 * gd + hv)
+    assert bool((slab[0] == 7).all() and (slab[:, :lo] == 7).all() and (slab[:, lo + sw + cw:] == 7).all())
+    return out.cpu().split(lens), slab[1:, lo: lo + sw].view(B, H, D, E), slab[1:, lo + sw: lo + sw + cw].view(B, taps - 1, 2 * gd + hv)
 
 
 # (rows of S in, at and below a padded block; columns over part of a wave, one and two workgroups, odd; more heads than half waves)
