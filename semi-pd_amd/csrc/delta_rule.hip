@@ -20,7 +20,8 @@
 //  * Prompt batches: delta_chunk_operands_kernel and delta_chunk_walk_kernel in place of the three, 32 tokens at a time on the
 //    matrix cores, every operand and sum fp32.
 //  * delta_post_kernel / delta_post_vec_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
-//  * delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, head).
+//  * delta_step_kernel / delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, key
+//    head) where the state lies on 16-byte boundaries, else per (request, head).
 #include "common.h"
 #include "recurrent_chunks.h"
 
@@ -446,6 +447,130 @@ __global__ void __launch_bounds__(1024) delta_decode_kernel(DeltaArgs a) {
     const float inv = 1.0f / sqrtf(sq_o / (float)E + a.eps);
     const float gate = Elem<T>::to_f(p[a.gate_off + h * E + j]);
     ((T*)a.out)[(int64_t)b * a.out_ld + h * E + j] = Elem<T>::from_f(o * inv * Elem<T>::to_f(((const T*)a.norm_w)[j]) * silu_f(gate));
+  }
+}
+
+// The same with S in 16-byte pieces and in ONE launch: a workgroup per (key head, request) with a team of four waves per value head (in
+// turn, where there are more heads than teams: a piece of the next one is fetched as one of this is stored), so the convolution's
+// channels belong to one workgroup, which moves their inputs on itself.  A thread of a team has four columns and every 1024 / E-th row
+// of S, all of its pieces in flight from the start; the two dot products are summed over lanes and the team's waves.  Bound by HBM, the
+// state read and written once: 32 requests, 32 heads of 128 x 128 (134 MB): a column of S by four lanes of four bytes each 57.7 -> 32.3
+// us; 3 requests, 32 heads of 64 x 64: 10.6 (two launches) -> 9.8.
+template <typename T, int NIT>
+__global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];       // q [D] | k [D] | v, later o [per E] | sums of every team [4][2][E] | scalars
+  const int g = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, team = tid >> 8, tt = tid & 255, teams = blockDim.x >> 8;
+  const int64_t pos = a.seq_lens[b] - 1;
+  if (pos < 0) return;
+  const bool fresh = pos == 0;
+  const int D = a.D, E = a.E, G = a.G, H = a.H, taps = a.taps, per = H / G, C = 2 * G * D + H * E;
+  const int quads = E / 4, rows = 256 / quads, n0 = tt / quads, e = tt % quads * 4;
+  const int64_t slot = a.state_indices[b];
+  const T* p = (const T*)a.p + (int64_t)b * a.ld;
+  float* q_l = lds;
+  float* k_l = lds + D;
+  float* v_l = lds + 2 * D;
+  float* sums = v_l + per * E + team * 8 * E;
+  float* sc = v_l + per * E + teams * 8 * E;
+  float4 S[NIT];
+  auto piece = [&](int hh, int n) {
+    return !fresh && hh < per && n < D ? *reinterpret_cast<const float4*>(a.state + slot * a.state_ld + ((int64_t)(g * per + hh) * D + n) * E + e) : float4{0.f, 0.f, 0.f, 0.f};
+  };
+#pragma unroll
+  for (int i = 0; i < NIT; ++i) S[i] = piece(team, n0 + i * rows);
+  float* cs = a.conv_state + slot * a.conv_ld;
+  for (int i = tid; i < 2 * D + per * E; i += blockDim.x) {
+    const bool is_v = i >= 2 * D;
+    const int d = is_v ? g * per * E + i - 2 * D : g * D + (i < D ? i : i - D);                              // channel within q, k or v
+    const int ch = is_v ? 2 * G * D + d : (i < D ? d : G * D + d);                                           // its place in the state
+    const T* cw = (const T*)(is_v ? a.conv_v : (i < D ? a.conv_q : a.conv_k)) + (int64_t)d * taps;
+    const float cur = Elem<T>::to_f(p[(is_v ? a.v_off : (i < D ? a.q_off : a.k_off)) + d]);
+    float y = Elem<T>::to_f(cw[taps - 1]) * cur;
+    // state entry s is the input s - (taps - 1) tokens back; every entry moves one place down and the token comes in last
+    for (int k = 1; k < taps; ++k) {
+      const int s = taps - 1 - k;
+      const float x = fresh ? 0.f : cs[(int64_t)s * C + ch];
+      if (!fresh) y += Elem<T>::to_f(cw[s]) * x;
+    }
+    for (int s = 1; s < taps - 1; ++s) cs[(int64_t)(s - 1) * C + ch] = fresh ? 0.f : cs[(int64_t)s * C + ch];
+    if (taps > 1) cs[(int64_t)(taps - 2) * C + ch] = cur;
+    lds[i] = silu_f(y);
+  }
+  __syncthreads();
+  if (tid < 64) {
+    float sk = 0.f, sq = 0.f, kq = 0.f;
+    for (int d = lane; d < D; d += 64) {
+      sk += k_l[d] * k_l[d];
+      sq += q_l[d] * q_l[d];
+      kq += k_l[d] * q_l[d];
+    }
+    sk = wave_sum(sk);
+    sq = wave_sum(sq);
+    kq = wave_sum(kq);
+    if (lane == 0) {
+      const float ik = 1.0f / sqrtf(sk + 1e-6f), iq = rsqrtf((float)D) / sqrtf(sq + 1e-6f);
+      sc[0] = ik;
+      sc[1] = iq;
+      sc[2] = kq * ik * iq;
+    }
+  }
+  __syncthreads();
+  const float ik = sc[0], iq = sc[1], kq = sc[2];
+  for (int h0 = 0; h0 < per; h0 += teams) {                         // (every team goes round as often: there are barriers inside)
+    const int hh = h0 + team, h = g * per + (hh < per ? hh : per - 1);
+    const bool on = hh < per;
+    float4 dk = {0.f, 0.f, 0.f, 0.f}, dq = {0.f, 0.f, 0.f, 0.f};
+    if (on)
+#pragma unroll
+      for (int i = 0; i < NIT; ++i) {
+        const int n = n0 + i * rows;
+        if (n < D) {
+          const float kv = k_l[n] * ik, qv = q_l[n] * iq;
+          dk = float4{dk.x + S[i].x * kv, dk.y + S[i].y * kv, dk.z + S[i].z * kv, dk.w + S[i].w * kv};
+          dq = float4{dq.x + S[i].x * qv, dq.y + S[i].y * qv, dq.z + S[i].z * qv, dq.w + S[i].w * qv};
+        }
+      }
+    for (int o = quads; o < 64; o <<= 1) {
+      dk.x += __shfl_xor(dk.x, o, 64); dk.y += __shfl_xor(dk.y, o, 64); dk.z += __shfl_xor(dk.z, o, 64); dk.w += __shfl_xor(dk.w, o, 64);
+      dq.x += __shfl_xor(dq.x, o, 64); dq.y += __shfl_xor(dq.y, o, 64); dq.z += __shfl_xor(dq.z, o, 64); dq.w += __shfl_xor(dq.w, o, 64);
+    }
+    if (lane < quads) {
+      *reinterpret_cast<float4*>(sums + (tt >> 6) * 2 * E + e) = dk;
+      *reinterpret_cast<float4*>(sums + (tt >> 6) * 2 * E + E + e) = dq;
+    }
+    __syncthreads();
+    const float gt = expf(-expf(a.a_log[h]) * softplus_f(Elem<T>::to_f(p[a.a_off + h]) + a.dt_bias[h])), beta = sigmoid_f(Elem<T>::to_f(p[a.b_off + h]));
+    float u[4], o4[4], sq_o = 0.f;
+    const float* vh = v_l + (on ? hh : 0) * E + e;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float* sk = sums + e + c;
+      const float dkc = (sk[0] + sk[2 * E]) + (sk[4 * E] + sk[6 * E]), dqc = (sk[E] + sk[3 * E]) + (sk[5 * E] + sk[7 * E]);
+      u[c] = beta * (vh[c] - gt * dkc);
+      o4[c] = gt * dqc + u[c] * kq;
+      sq_o += o4[c] * o4[c];
+    }
+    if (on) {
+      float* st = a.state + slot * a.state_ld + (int64_t)h * D * E;
+#pragma unroll
+      for (int i = 0; i < NIT; ++i) {
+        const int n = n0 + i * rows;
+        if (n < D) {
+          const float kv = k_l[n] * ik;
+          *reinterpret_cast<float4*>(st + n * E + e) = float4{gt * S[i].x + kv * u[0], gt * S[i].y + kv * u[1], gt * S[i].z + kv * u[2], gt * S[i].w + kv * u[3]};
+        }
+        S[i] = piece(hh + teams, n);                                 // (the team's next head)
+      }
+    }
+    for (int o = 1; o < quads; o <<= 1) sq_o += __shfl_xor(sq_o, o, 64);       // (a row of S is `quads` neighbouring lanes, all columns)
+    if (on && n0 == 0) {
+      const float inv = 1.0f / sqrtf(sq_o / (float)E + a.eps);
+      T* out = (T*)a.out + (int64_t)b * a.out_ld + h * E + e;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        out[c] = Elem<T>::from_f(o4[c] * inv * Elem<T>::to_f(((const T*)a.norm_w)[e + c]) * silu_f(Elem<T>::to_f(p[a.gate_off + h * E + e + c])));
+    }
+    __syncthreads();
   }
 }
 
@@ -1058,6 +1183,22 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
   const int ds = k_dim >= 32 ? 4 : 1;
   const int per = (k_dim + ds - 1) / ds;
   const int dpt = per <= 4 ? 4 : (per <= 8 ? 8 : (per <= 16 ? 16 : (per <= 32 ? 32 : 64)));
+  // a decode batch whose state rows lie on 16-byte boundaries: up to 16 pieces of four columns a thread.  Four teams a workgroup while
+  // the chip takes all workgroups at once, two where a CU goes through several, so that one loads while another computes (32 heads
+  // of 64 x 64, 8 key heads, four teams / two, us: 3 requests 9.8 / 12.1, 32 13.2 / 15.3, 48 22.9 / 18.3, 128 47.7 / 37.7)
+  const int per_group = num_heads / num_k_heads, most = k_dim * v_dim > 4 * 1024 || batch * num_k_heads > 256 ? 2 : 4, teams = per_group < most ? per_group : most;
+  const size_t step_lds = ((size_t)2 * k_dim + (size_t)per_group * v_dim + (size_t)teams * 8 * v_dim + 4) * sizeof(float);
+  if (q_start == nullptr && batch <= 65535 && v_dim >= 16 && v_dim <= 256 && (v_dim & (v_dim - 1)) == 0 && k_dim % 2 == 0 && k_dim * v_dim <= 16 * 1024 &&
+      aligned16(state) && state_ld % 4 == 0 && step_lds <= 65536) {
+    const int nit = (k_dim * v_dim + 1023) / 1024;
+    const dim3 sgrid((unsigned)num_k_heads, (unsigned)batch);
+    SEMIPD_DISPATCH_DTYPE(dtype, T, {
+      if (nit <= 4) hipLaunchKernelGGL((delta_step_kernel<T, 4>), sgrid, dim3(256 * teams), step_lds, st, a);
+      else if (nit <= 8) hipLaunchKernelGGL((delta_step_kernel<T, 8>), sgrid, dim3(256 * teams), step_lds, st, a);
+      else hipLaunchKernelGGL((delta_step_kernel<T, 16>), sgrid, dim3(256 * teams), step_lds, st, a);
+    });
+    return launch_status("delta_rule(step)");
+  }
   if (q_start == nullptr && (int64_t)ds * v_dim <= 1024) {
     // a decode batch: one launch, then the convolutions' inputs move on (the launch above has read the old ones)
     const int threads = (ds * v_dim + 63) / 64 * 64;

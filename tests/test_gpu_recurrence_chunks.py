@@ -239,3 +239,22 @@ def test_delta_rule_in_chunks_not_finite(col, value):
     torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
     if col != "a" or value != value:
         assert not bool(torch.isfinite(got[0][at:]).all())
+
+
+# (a team per head: one, several in one workgroup, more heads than teams; one, some and all rows of pieces)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,E,taps", [(8, 2, 128, 128, 4), (3, 3, 64, 64, 2), (12, 2, 20, 16, 3), (7, 1, 64, 256, 1), (4, 2, 100, 32, 5)])
+def test_delta_rule_decode_step(dtype, H, G, D, E, taps):
+    w, rows, state, before = _delta_inputs(H, G, D, E, taps, [1, 1, 1], dtype, 3)
+    first = [5, 0, 900]
+    ulp = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8}[dtype]
+    for step in range(2):
+        outs, after, last = _delta_run(w, rows, state, before, first, H, G, D, E, decode=True)
+        for b in range(3):
+            zero = first[b] == 0
+            want, S, tail = _delta_truth(w, rows[b], torch.zeros_like(state[b]) if zero else state[b],
+                                         torch.zeros_like(before[b]) if zero else before[b], H, G, D, E)
+            torch.testing.assert_close(outs[b].to(F64), want, rtol=ulp + 2e-5, atol=2e-5)
+            torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+            torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+        state, before, first = after.clone(), last.clone(), [f + 1 for f in first]
