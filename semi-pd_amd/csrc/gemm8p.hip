@@ -29,6 +29,8 @@
 // layers/activation.py:41-53) for 65 .. 256-row decode batches, and _get_logits (layers/logits_processor.py:394-445).
 #include "common.h"
 
+#include <type_traits>
+
 namespace semipd {
 
 typedef float g8_f32x4 __attribute__((ext_vector_type(4)));
@@ -117,6 +119,16 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
   int tile_m, tile_n;
   if (GR || ORDER == 0) {
     tile_m = blockIdx.x / tiles_n, tile_n = blockIdx.x - tile_m * tiles_n;   // neighbours share the x tile
+    const int first = tile_m & ~1, t = (int)blockIdx.x - first * tiles_n;
+    if (GR && (first + 1) * tiles_n < (int)gridDim.x && (first + 1) * G::BM < grp.num_post_pad[0] &&
+        grp.expert_ids[first] == grp.expert_ids[first + 1]) {
+      // two row tiles of one expert: the two workgroups of a W tile are 8 ids apart, on one XCD (id % 8) at one time, and the
+      // second finds the tile in that L2 (384 rows an expert 572 -> 557 us, 768: 1000 -> 962; in plain order where a pair of
+      // tiles has two experts: there the eight neighbours sharing an x tile are worth 1 %)
+      const int whole = tiles_n / 8 * 16, rem = tiles_n & 7;
+      if (t < whole) tile_m = first + (t >> 3 & 1), tile_n = (t >> 4) * 8 + (t & 7);
+      else tile_m = first + (t - whole) / rem, tile_n = tiles_n - rem + (t - whole) % rem;
+    }
   } else {
     // several row tiles (prefill-sized calls): workgroup id runs on XCD id % 8; give every XCD a contiguous range of
     // logical tiles and walk the row tiles fastest, so that the row tiles of one W tile sit on ONE XCD next to each
@@ -151,6 +163,7 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
     for (int h = 0; h < 2; ++h) {
       int xrow = m0 + XH * (rp / (XH / 2)) + (XH / 2) * h + (rp % (XH / 2));
       if (GR) {
+        xrow = m0 + XH * h + rp;                                  // (the wave bands in turn: see `live`)
         const int id = grp.sorted_ids[xrow];
         xrow = id < grp.num_valid ? id / grp.top_k_div : 0;      // padding entries read row 0 (discarded)
       } else {
@@ -212,6 +225,19 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
     for (int j = 0; j < 2 * NT2; ++j) acc[i][j] = g8_f32x4{0.f, 0.f, 0.f, 0.f};
   G8Frag fx[MT2][2], fw[2 * NT2][2];     // x fragments of the current half; W fragments: [0 .. NT2) lo, [NT2 .. 2 NT2) hi
 
+  // Grouped: an expert's last tile is filled up with padding entries, and a quadrant of a wave whose rows are all padding reads no
+  // fragments and multiplies nothing (the DMA, the waits and the barriers stay: all waves pass them).  For that the two wave bands
+  // take the entries of a tile by turns, XH / 2 at a time: up to XH routed rows are the first half of BOTH groups, which go on covering
+  // each other's reads.  64 experts, K = 2048, N = 2816 and 1408, whole layer, this and the order of the tiles together: 281 rows an
+  // expert 548 -> 501 us, 328 rows 572 -> 530, 562 rows 854 -> 790.  A tile with 25 rows still takes 0.4 of a full one, the flight
+  // time of its loads: not staging the padding rows changed nothing (513).
+  bool live[2] = {true, true};
+  if (GR) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      live[h] = __ballot(grp.sorted_ids[m0 + XH * h + (XH / 2) * wr + lane % (XH / 2)] < grp.num_valid) != 0;
+  }
+
   // ---- prologue: K steps 0 and 1 up to the point the steady state expects (issue order = order of first use) ----
   stage_x(0, 0), stage_w(0, 0), stage_w(1, 0), stage_x(1, 0), stage_x(0, 1), stage_w(0, 1);
   g8_wait_vm<G::kInFlight>();         // x0(0), W0(0) landed (this wave's share)
@@ -230,51 +256,62 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
     __builtin_amdgcn_s_setprio(0);
   };
 
+  // (three loops instead of a branch per phase: what a fragment read is still to write passes no join of control flow)
+  auto walk = [&](auto lo_c, auto hi_c) __attribute__((always_inline)) {
+  constexpr bool LO = decltype(lo_c)::value, HI = decltype(hi_c)::value;
   for (int kt = 0; kt < nkt; ++kt) {
     const uint32_t par = (kt & 1) * G::kParity;
     // phase 1: x half 0 + W half 0 of this step; DMA W1(kt + 1)
+    if constexpr (LO || HI)
 #pragma unroll
-    for (int j = 0; j < NT2; ++j)
+      for (int j = 0; j < NT2; ++j)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) fw[j][s].u = g8_lds_read16(wa + par + off_s[s], j * 2048);
+        for (int s = 0; s < 2; ++s) fw[j][s].u = g8_lds_read16(wa + par + off_s[s], j * 2048);
+    if constexpr (LO)
 #pragma unroll
-    for (int i = 0; i < MT2; ++i)
+      for (int i = 0; i < MT2; ++i)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) fx[i][s].u = g8_lds_read16(xa + par + off_s[s], i * 2048);
+        for (int s = 0; s < 2; ++s) fx[i][s].u = g8_lds_read16(xa + par + off_s[s], i * 2048);
     stage_w(1, kt + 1);
     g8_wait_vm<G::kInFlight>();       // W1(kt) landed; x1(kt), x0(kt+1), W0(kt+1), W1(kt+1) may be in flight
     g8_barrier();
     g8_wait_lgkm0();
-    mfma_quadrant(0, 0);
+    if constexpr (LO) mfma_quadrant(0, 0);
     g8_barrier();
     // phase 2: W half 1; DMA x1(kt + 1)
+    if constexpr (LO || HI)
 #pragma unroll
-    for (int j = 0; j < NT2; ++j)
+      for (int j = 0; j < NT2; ++j)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) fw[NT2 + j][s].u = g8_lds_read16(wa + par + G::kWHalf + off_s[s], j * 2048);
+        for (int s = 0; s < 2; ++s) fw[NT2 + j][s].u = g8_lds_read16(wa + par + G::kWHalf + off_s[s], j * 2048);
     stage_x(1, kt + 1);
     g8_wait_vm<G::kInFlight>();       // x1(kt) landed
     g8_barrier();
     g8_wait_lgkm0();
-    mfma_quadrant(0, NT2);
+    if constexpr (LO) mfma_quadrant(0, NT2);
     g8_barrier();
     // phase 3: x half 1 (into the x registers); DMA x0(kt + 2)
+    if constexpr (HI)
 #pragma unroll
-    for (int i = 0; i < MT2; ++i)
+      for (int i = 0; i < MT2; ++i)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) fx[i][s].u = g8_lds_read16(xa + par + G::kXHalf + off_s[s], i * 2048);
+        for (int s = 0; s < 2; ++s) fx[i][s].u = g8_lds_read16(xa + par + G::kXHalf + off_s[s], i * 2048);
     stage_x(0, kt + 2);
     g8_barrier();
     g8_wait_lgkm0();
-    mfma_quadrant(MT2, NT2);
+    if constexpr (HI) mfma_quadrant(MT2, NT2);
     g8_barrier();
     // phase 4: nothing to read (W lo is still in registers); DMA W0(kt + 2)
     stage_w(0, kt + 2);
     g8_wait_vm<G::kInFlight>();       // x0(kt+1), W0(kt+1) landed
     g8_barrier();
-    mfma_quadrant(MT2, 0);
+    if constexpr (HI) mfma_quadrant(MT2, 0);
     g8_barrier();
   }
+  };
+  if (!GR || live[1]) walk(std::true_type{}, std::true_type{});
+  else if (live[0]) walk(std::true_type{}, std::false_type{});
+  else walk(std::false_type{}, std::false_type{});
   g8_wait_vm<0>();                    // no DMA may land in LDS that the next workgroup owns
   if (wr == 0) g8_barrier();          // the barrier group 1 spent up front
 
@@ -305,7 +342,7 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
       int m = mb + 16 * i;
       float scale = 1.f;
       if (GR) {
-        m = grp.sorted_ids[m];                                   // output row = the routed entry itself
+        m = grp.sorted_ids[m0 + XH * (i / MT2) + (XH / 2) * wr + 16 * (i % MT2) + c16];                                   // output row = the routed entry itself
         if (m < grp.num_valid && grp.mul_routed_weight) scale = grp.topk_weights[m];
       }
 #pragma unroll
@@ -325,7 +362,7 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
 #pragma unroll
     for (int i = 0; i < 2 * MT2; ++i) {
       int m = mb + 16 * i;
-      if (GR) m = grp.sorted_ids[m];
+      if (GR) m = grp.sorted_ids[m0 + XH * (i / MT2) + (XH / 2) * wr + 16 * (i % MT2) + c16];
 #pragma unroll
       for (int j = 0; j < NT2; ++j) {
         const int n = n0 + (WH / 4) * wc + 16 * j + 4 * q4;
