@@ -5,7 +5,10 @@ hipGraphLaunch.  Padded slots use seq_len = 1 and write their KV to the dummy sl
 from __future__ import annotations
 
 import bisect
+import contextlib
+import gc
 import os
+import threading
 from typing import Dict, List, Tuple
 
 import torch
@@ -22,6 +25,28 @@ def get_batch_sizes_to_capture(max_bs: int) -> List[int]:
 
 
 _PARKED: list = []   # see _capture_one
+
+_capturing = threading.Lock()
+_captures, _gc_was_on = 0, False
+
+
+@contextlib.contextmanager
+def without_cycle_collection():
+    """No cyclic garbage collection inside: a dead engine is a cycle that holds graphs, and a graph that dies synchronises the
+    device, which a stream capture of this process does not allow -- the error leaves a destructor and ends the process."""
+    global _captures, _gc_was_on
+    with _capturing:
+        if _captures == 0:
+            _gc_was_on = gc.isenabled()
+            gc.disable()
+        _captures += 1
+    try:
+        yield
+    finally:
+        with _capturing:
+            _captures -= 1
+            if _captures == 0 and _gc_was_on:
+                gc.enable()
 
 # fault injection for tests: a callable (bs, outputs) run inside the capture.  Installed only by a test plugin that the
 # scheduler process loads at start-up (entrypoints/engine.py: ServerArgs.test_plugin); never set in production.
@@ -139,7 +164,7 @@ class HipGraphRunner:
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         try:
-            with torch.cuda.graph(g, pool=self.pool, stream=self.stream):
+            with without_cycle_collection(), torch.cuda.graph(g, pool=self.pool, stream=self.stream):
                 out = run_once()
                 if capture_fault_hook is not None:
                     capture_fault_hook(bs, out)
