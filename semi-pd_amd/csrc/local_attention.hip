@@ -8,7 +8,9 @@
 //    a decode step are the same walk: query at position p sees keys lo(p) .. p, lo(p) = floor(p / chunk) * chunk
 //    (chunk 0: lo = 0).  score = cap * tanh(scale * q.k / cap) (cap 0: none); the softmax denominator holds one more
 //    term exp(sink[head]) that has no value row.  Optional epilogue: out *= sigmoid(gate).
-//  * local_attention_mfma_kernel (bf16 / f16, head sizes in steps of 32 / 16): 64 query rows of one request and head
+//  * prompt_attention_kernel (local_attention_prompt.h; bf16 / f16, the head sizes listed there): 32 query rows per wave on
+//    v_mfma_f32_32x32x16, the query heads of a key head sharing staged rows.
+//  * local_attention_mfma_kernel (bf16 / f16, other head sizes in steps of 32 / 16, pooled blocks): 64 query rows of one request and head
 //    per workgroup, S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_16x16x32, P^T taken from the accumulators in place, V^T
 //    through transposing reads of a row-major LDS tile, the next step's loads in flight during the current one.
 //  * local_attention_decode_kernel (bf16 / f16): one workgroup per (request, kv head); the waves split the visible keys,
