@@ -629,7 +629,7 @@ int semipd_ipc_get_handle(const void* dev_ptr, uint8_t handle[64], uint64_t* off
  * of semipd_ipc_get_handle, which was measured on one runtime.  library plumbing (no reference counterpart). */
 int semipd_runtime_version(int* runtime, int* driver);
 /* A stream the caller owns (hipStreamCreateWithFlags, non-blocking) for graph capture, and the way out of a capture
- * that failed half way.  Measured on ROCm 7.0 (tools/probe_capture_abort.py): an invalidated capture cannot be ended --
+ * that failed half way.  On ROCm 7.0 an invalidated capture cannot be ended --
  * hipStreamEndCapture returns hipErrorStreamCaptureInvalidated and the stream stays invalidated -- and while it exists
  * every synchronising call of the process, on any stream, fails with that error; destroying the stream clears it.
  * semipd_stream_abort_capture = end the capture, drop the graph, DESTROY the stream (the handle is dead afterwards),

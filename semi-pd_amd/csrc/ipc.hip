@@ -66,7 +66,7 @@ int semipd_ipc_get_handle(const void* dev_ptr, uint8_t handle[64], uint64_t* off
   SEMIPD_HIP(hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)dev_ptr));
   // ROCm 7.2 / dmabuf IPC: hipIpcOpenMemHandle in the importing process never returns when the
   // allocation size modulo 4 GiB is 2 GiB or more (measured: 2.5 GiB and 6.1 GiB hang; 1.9, 5.0, 9.5, 20,
-  // 40 GiB map in < 1 ms; tools/ipc_big_probe.py).  Refuse to export such an allocation instead of
+  // 40 GiB map in < 1 ms).  Refuse to export such an allocation instead of
   // hanging the importer; large buffers meant for sharing are sized around it (memory_pool.py).
   // The rule was measured on ONE runtime (HIP 7.2): it is applied on every runtime (padding is harmless where the
   // importer would not have hung), can be switched off with SEMIPD_IPC_SIZE_RULE=off once a runtime is known to be

@@ -63,8 +63,7 @@ def _destroy_stream(raw: int) -> None:
 
 def recover_after_failed_capture(device) -> None:
     """After HipGraphRunner raised out of a capture (its stream is destroyed, what lived on it parked): the sequence that
-    brings the process back on ROCm 7.0 (tools/probe_capture_abort.py, tests/test_gpu_ops.py::
-    test_abort_of_a_failed_stream_capture) -- one throw-away call takes the hipErrorInvalidValue the framework's
+    brings the process back on ROCm 7.0 (tests/test_gpu_ops.py::test_abort_of_a_failed_stream_capture) -- one throw-away call takes the hipErrorInvalidValue the framework's
     bookkeeping left behind, one small clean capture on a fresh stream settles its capture state."""
     import ctypes
     from semi_pd_amd import _lib

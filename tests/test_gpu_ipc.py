@@ -140,7 +140,7 @@ def test_cu_masked_stream_confines_workgroups(device):
 
 def test_export_refuses_allocation_sizes_the_importer_cannot_map(device):
     """ROCm 7.2 dmabuf IPC: hipIpcOpenMemHandle never returns when the allocation size modulo 4 GiB is
-    >= 2 GiB (tools/ipc_big_probe.py).  The exporter must fail loudly instead of hanging the prefill
+    >= 2 GiB.  The exporter must fail loudly instead of hanging the prefill
     instance at start-up, and the pools must size their slabs around it."""
     import semi_pd_ipc
     from semi_pd_amd.mem_cache.memory_pool import ipc_safe_zeros
