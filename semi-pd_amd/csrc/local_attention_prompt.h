@@ -9,9 +9,9 @@
 //    transposing reads of V take).
 //  * 16-byte chunk c of row r lies at c ^ (r & 15) of a K tile (the 32 rows of an operand read start in different banks), the 64-byte
 //    group t at t ^ (r & 3) of a V tile (the four rows of a transposing read likewise).
-//  * The running maximum is the row's own at every step, so its largest weight is 1 and rounds to 16 bits without an error: letting
-//    it lag by up to 2^6 (fewer rescalings: 7262 tokens in blocks of 1024 118 -> 114 us, value rows of 256 380 -> 331) was 2 .. 5 %
-//    further from the 64-bit result.
+//  * The running maximum is the row's own and is taken every 32 keys, also in steps of 64: the largest weight of every 32 is 1 and
+//    rounds to 16 bits without an error (a maximum per 64 keys: the result of the window batch below was 0.5 % further from the 64-bit
+//    one).  Letting it lag by up to 2^6 was 2 .. 5 % further.
 // Bound: at 64 keys a wave multiplies for 32 x 32 cycles (128 / 128), reads 32 KB of LDS and takes 32 exponentials a lane (16 cycles
 // each) with five instructions around each: matrix pipe, LDS and vector unit are close to each other, two waves a SIMD fill each
 // other's gaps.  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves
@@ -182,6 +182,14 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
           }
       }
       Frag16 p[2 * KU];                                              // keys 16 s + {0 .. 3, 8 .. 11} + 4 hi of this lane's column
+      float m_of[KU], l_next = 0.f;                                  // running maximum behind every 32 keys, the second 32's share of l
+      auto rescale = [&](float by) {
+        l *= by;
+#pragma unroll
+        for (int t = 0; t < ET; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) o[t][r] *= by;
+      };
       if constexpr (SIG) {
         // independent weights sigmoid(score + hb), base 2: a masked key has score -inf: exp2(+inf) = inf, 1 / inf = 0
 #pragma unroll
@@ -193,38 +201,43 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
             p[2 * u + (r >> 3)].w[(r & 7) >> 1] = pack2<T>(p0, p1);
           }
       } else {
-        float mx = s[0][0];
+        float mx[KU];
 #pragma unroll
-        for (int u = 0; u < KU; ++u)
+        for (int u = 0; u < KU; ++u) {
+          mx[u] = s[u][0];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[u][r]);
-        {
-          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-          mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c;        // (c > 0; -inf stays -inf)
+          for (int r = 1; r < 16; ++r) mx[u] = fmaxf(mx[u], s[u][r]);
+          const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx[u]), __float_as_uint(mx[u]), false, false);
+          mx[u] = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])) * c;        // (c > 0; -inf stays -inf)
         }
-        if (__any(mx > m)) {
-          const float m_new = fmaxf(m, mx), alpha = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new);
-          l *= alpha;
-#pragma unroll
-          for (int t = 0; t < ET; ++t)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+        if (__any(mx[0] > m)) {
+          const float m_new = fmaxf(m, mx[0]);
+          rescale(m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - m_new));
           m = m_new;
         }
-        const float m_use = m == -INFINITY ? 0.f : m;
-        float sum = 0.f;
+        m_of[0] = m;
+        if constexpr (KU == 2) m = m_of[1] = fmaxf(m, mx[1]);
+        float sum[KU] = {};
 #pragma unroll
-        for (int u = 0; u < KU; ++u)
+        for (int u = 0; u < KU; ++u) {
+          const float m_use = m_of[u] == -INFINITY ? 0.f : m_of[u];
 #pragma unroll
           for (int r = 0; r < 16; r += 2) {
             const float p0 = __builtin_amdgcn_exp2f(fmaf(s[u][r], c, -m_use)), p1 = __builtin_amdgcn_exp2f(fmaf(s[u][r + 1], c, -m_use));
-            sum += p0 + p1;
+            sum[u] += p0 + p1;
             p[2 * u + (r >> 3)].w[(r & 7) >> 1] = pack2<T>(p0, p1);
           }
-        l += sum;
+        }
+        l += sum[0];
+        if constexpr (KU == 2) l_next = sum[1];
       }
 #pragma unroll
-      for (int s4 = 0; s4 < 2 * KU; ++s4)
+      for (int s4 = 0; s4 < 2 * KU; ++s4) {
+        if constexpr (!SIG && KU == 2)
+          if (s4 == 2) {
+            if (__any(m_of[1] > m_of[0])) rescale(m_of[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_of[0] - m_of[1]));
+            l += l_next;
+          }
 #pragma unroll
         for (int t = 0; t < ET; ++t) {
           Frag16 vf;
@@ -233,6 +246,7 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
           vf.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vq + 8 * VB));
           o[t] = Mfma<T>::mma(as_frag<T>(vf), as_frag<T>(p[s4]), o[t]);
         }
+      }
     }
     if (it + 1 < steps) store_rows(buf ^ 1);
     __syncthreads();                                            // the next step's rows are in place, everyone is done with this step's

@@ -93,6 +93,33 @@ def test_prompt_attention(dtype, lens, olds, group, D, form):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+def test_largest_weight_of_every_32_keys_is_not_rounded(dtype, D):
+    """Two keys carry the weight, one in the first 32 and a larger one in the next 32, and their values cancel all but the rounding of
+    the smaller one's weight to 16 bits.  Weight 1 at the time it is rounded, a factor in fp32 (four roundings of 2^-23, values of
+    256) behind it; the result is rounded once."""
+    from semi_pd_amd import ops
+    H, G, n, small, large = 4, 1, 64, 5, 40
+    scores = torch.linspace(0.1, 2.0, n - large).to(dtype)                        # of the larger key, row by row
+    weight = torch.exp(-scores.double())
+    q, k, v = torch.zeros(n, H, D), torch.zeros(n + 1, G, D), torch.zeros(n + 1, G, D)
+    q[:, :, 1] = 1.0
+    q[large:, :, 0] = scores.float()[:, None]
+    k[1:, 0, 1] = -200.0
+    k[1 + small, 0, 1], k[1 + large, 0, :2] = 0.0, torch.tensor([1.0, 0.0])
+    v[1 + small, 0] = 256.0
+    v[1 + large, 0, : n - large] = -256.0 * weight.to(dtype).float()
+    q, k, v = (x.to(dtype).to(DEV) for x in (q.view(n, H * D), k, v))
+    one = lambda x, t=torch.int32: torch.tensor([x], dtype=t, device=DEV)          # noqa: E731
+    out = torch.empty_like(q)
+    ops.local_attention_fwd(q, out, k, v, torch.arange(1, n + 1, dtype=torch.int32, device=DEV)[None], one(0, torch.int64), one(n, torch.int64),
+                            one(0), one(n), n, 1.0, 0.0, 0, None, None)
+    want = ((v[1 + small, 0].double().cpu() * weight[:, None] + v[1 + large, 0].double().cpu()) / (1 + weight[:, None]))[:, None]
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    torch.testing.assert_close(out[large:].view(-1, H, D).double().cpu(), want.expand(-1, H, D), rtol=ulp, atol=256 * 2.0 ** -21)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("lens,olds", CASES)
 @pytest.mark.parametrize("H,G,D", [(16, 2, 128), (6, 2, 128), (8, 2, 64)])
 def test_prompt_attention_over_shared_values(dtype, lens, olds, H, G, D):
