@@ -12,6 +12,8 @@
 //  * The running maximum is the row's own and is taken every 32 keys, also in steps of 64: the largest weight of every 32 is 1 and
 //    rounds to 16 bits without an error (a maximum per 64 keys: the result of the window batch below was 0.5 % further from the 64-bit
 //    one).  Letting it lag by up to 2^6 was 2 .. 5 % further.
+//  * A weight of zero does not hide an infinity or a NaN from a product, and a wave multiplies keys that some of its rows do not see: a
+//    wave that ends with sums that are not finite takes its rows again, one by one.
 // Bound: at 64 keys a wave multiplies for 32 x 32 cycles (128 / 128), reads 32 KB of LDS and takes 32 exponentials a lane (16 cycles
 // each) with five instructions around each: matrix pipe, LDS and vector unit are close to each other, two waves a SIMD fill each
 // other's gaps.  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves
@@ -21,6 +23,67 @@
 #pragma once
 
 namespace semipd {
+
+// Rows wq0 .. wq0 + 31 of request b and head h by one wave, a row at a time from its own keys alone, fp32 throughout (rare: it must not
+// set the kernel's registers)
+template <typename T, int D, int E, bool SIG>
+__device__ __forceinline__ void prompt_rows_one_by_one(const LocalAttnArgs& a, int b, int h, int wq0, int lane) {
+  const int qn = a.q_len[b], gk = h / (a.H / a.G);
+  const int base_pos = (int)(a.seq_lens[b] - qn);
+  const int32_t* row = a.req_to_token + a.req_pool_indices[b] * a.r2t_stride;
+  const T* kp = (const T*)a.k_pool + (int64_t)gk * D;
+  const T* vp = (const T*)a.v_pool + (a.v_shared ? 0 : (int64_t)gk * E) + lane;
+  const ScoreMap smap(a.scale, a.cap);
+  const float hb = (SIG && a.head_bias) ? a.head_bias[h] * kLog2e : 0.f;
+#pragma unroll 1
+  for (int r = wq0; r < qn && r < wq0 + 32; ++r) {
+    const int pos = base_pos + r, lo = (int)range_lo(a, pos), n_first = (int)kept_before(a, lo), n = n_first + pos - lo + 1;
+    const int64_t t = a.q_start[b] + r;
+    const T* q = (const T*)a.q + t * a.q_ld + (int64_t)h * D;
+    float m = -INFINITY, l = 0.f, acc[E / 64] = {};
+#pragma unroll 1
+    for (int i0 = 0; i0 < n; i0 += 64) {
+      const bool there = i0 + lane < n;
+      const int i = there ? i0 + lane : n - 1, slot = row[i < n_first ? i : lo + i - n_first];
+      float dot = 0.f;
+#pragma unroll 1
+      for (int d = 0; d < D; d += 8) {
+        const Vec16<T> qv = load16(q + d), kv = load16(kp + (int64_t)slot * a.k_ld + d);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) dot += Elem<T>::to_f(qv.e[u]) * Elem<T>::to_f(kv.e[u]);
+      }
+      const float s = smap(dot);
+      float p;
+      if constexpr (SIG) {
+        p = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-(s + hb)));
+      } else {
+        const float m_new = fmaxf(m, wave_max(there ? s : -INFINITY)), m_use = m_new == -INFINITY ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m - m_use);
+        p = __builtin_amdgcn_exp2f(s - m_use);
+        l = l * alpha + wave_sum(there ? p : 0.f);
+#pragma unroll
+        for (int u = 0; u < E / 64; ++u) acc[u] *= alpha;
+        m = m_new;
+      }
+#pragma unroll 1
+      for (int k = 0; k < 64 && i0 + k < n; ++k) {
+        const float pk = __shfl(p, k, 64);
+        const T* v = vp + (int64_t)__shfl(slot, k, 64) * a.v_ld;
+#pragma unroll
+        for (int u = 0; u < E / 64; ++u) acc[u] += pk * Elem<T>::to_f(v[64 * u]);
+      }
+    }
+    if (!SIG && a.sink != nullptr) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e - m);
+    const float inv = SIG ? a.out_scale : a.out_scale / l;
+    T* out = (T*)a.out + t * a.out_ld + (int64_t)h * E + lane;
+#pragma unroll
+    for (int u = 0; u < E / 64; ++u) {
+      float y = acc[u] * inv;
+      if (a.gate) y *= __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-kLog2e * Elem<T>::to_f(((const T*)a.gate)[t * a.gate_ld + (int64_t)h * E + lane + 64 * u])));
+      out[64 * u] = Elem<T>::from_f(y);
+    }
+  }
+}
 
 template <typename T, int D, int E, int NW, int KT, bool SIG>
 __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnArgs a, int hw) {
@@ -257,6 +320,22 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
     if (a.sink != nullptr) l += __builtin_amdgcn_exp2f(a.sink[h] * kLog2e - m);
   }
   if (!wave_on) return;
+  {
+    float z[4] = {};
+#pragma unroll
+    for (int t = 0; t < ET; ++t)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) z[r & 3] = fmaf(o[t][r], 0.f, z[r & 3]);
+    if (__any(!((z[0] + z[1]) + (z[2] + z[3]) == 0.f))) {
+      auto args = (const __attribute__((address_space(4))) void*)__builtin_amdgcn_kernarg_segment_ptr();
+      int b1 = b, h1 = h, row1 = wq0, lane1 = lane;
+      asm volatile("" : "+s"(args), "+s"(b1), "+s"(h1), "+s"(row1), "+v"(lane1));      // (read and computed again, not held over the walk)
+      LocalAttnArgs again;
+      __builtin_memcpy(&again, (const void*)args, sizeof(again));
+      prompt_rows_one_by_one<T, D, E, SIG>(again, b1, h1, row1, lane1);
+      return;
+    }
+  }
   const float inv = q_ok ? (SIG ? a.out_scale : a.out_scale / l) : 0.f;
   // out through the wave's part of the tiles (the walk ended on a barrier): a lane holds four neighbouring elements of one row at a
   // time, rows leave in 16-byte pieces of consecutive lanes

@@ -93,6 +93,51 @@ def test_prompt_attention(dtype, lens, olds, group, D, form):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("form,D,E", [("causal", 128, 128), ("block", 64, 64), ("window", 64, 64), ("keep", 128, 128), ("sigmoid", 64, 64),
+                                      ("shared", 128, 256), ("shared", 64, 128)])
+def test_values_that_are_not_finite_stay_with_the_rows_that_see_them(dtype, value, form, D, E):
+    """One element of the value rows of a few keys: rows that do not see them are as without them (to the rounding of their weights, as
+    above), the others hold what the sum holds."""
+    from semi_pd_amd import ops
+    H, G, lens, olds = (4, 2, [150], [40]) if form != "shared" else (4, 2, [90, 70], [0, 33])
+    t, g = _batch(lens, olds, H, G, D, E // 2 if form == "shared" else E, dtype, D + E)
+    head = torch.randn(H, generator=g).to(DEV)
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    bad = [3, 77, 101]                                                              # positions, of every request
+
+    def run(v):
+        d = {k: x.to(DEV) for k, x in t.items() if k != "totals"}
+        d["v"] = v.to(DEV)
+        out = torch.empty(sum(lens), H * E, dtype=dtype, device=DEV)
+        batch = (d["q"], out, d["k"], d["v"], d["table"], torch.arange(len(lens), device=DEV), torch.tensor(t["totals"], device=DEV), start.to(DEV),
+                 n.to(DEV), max(lens), D ** -0.5)
+        if form == "shared":
+            ops.shared_value_attention_fwd(*batch)
+        elif form in ("causal", "block"):
+            ops.local_attention_fwd(*batch, 0.0, 48 if form == "block" else 0, None, None)
+        else:
+            ops.window_attention_fwd(*batch, 40, 0 if form == "window" else 2 if form == "sigmoid" else 70, head, form == "sigmoid", None, 1.0)
+        return out.cpu().float().view(-1, H, E)
+
+    clean, v = run(t["v"]), t["v"].clone()
+    for b in range(len(lens)):
+        v[t["table"][b, bad].long(), 0, 5] = value
+    got, at = run(v), 0
+    heads = slice(0, H) if form == "shared" else slice(0, H // G)                    # (the first key/value head's, or the row that all share)
+    hit = torch.zeros_like(got, dtype=torch.bool)
+    for b, (new, old) in enumerate(zip(lens, olds)):
+        p, j = torch.arange(old, old + new)[:, None], torch.tensor(bad)[None]
+        see = {"causal": j <= p, "shared": j <= p, "block": (j <= p) & (j // 48 == p // 48)}.get(
+            form, (j <= p) & ((p - j < 40) | (j < (0 if form == "window" else 2 if form == "sigmoid" else 70))))
+        hit[at: at + new, heads, 5] = see.any(1)[:, None]
+        at += new
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    torch.testing.assert_close(got[~hit], clean[~hit], rtol=6 * ulp, atol=12 * ulp)
+    assert bool(torch.isnan(got[hit]).all() if value != value else (got[hit] == value).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("D", [64, 128])
 def test_largest_weight_of_every_32_keys_is_not_rounded(dtype, D):
     """Two keys carry the weight, one in the first 32 and a larger one in the next 32, and their values cancel all but the rounding of
