@@ -671,7 +671,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
           if (i < taps) y += wt[i] * in[i];
 #pragma unroll
         for (int i = kRecTaps - 1; i > 0; --i) in[i] = in[i - 1];
-        dst[t * CS] = t < cnt ? rec_silu_or_not_finite(y, rec_silu(y)) : 0.f;
+        dst[t * CS] = t < cnt ? (rec_moderate(y) ? rec_silu(y) : rec_silu_if_large(y)) : 0.f;
       }
     } else {
       for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
@@ -855,8 +855,8 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
         float z = rec_silu(y);
         asm volatile("" : "+v"(z));                              // (straight-line code: it goes between the products)
         const bool in = 16 * j + 4 * kq + s < cnt;
-        v[j][s] = in ? rec_silu_or_not_finite(y, z) : 0.f;
-        bad |= in && !rec_finite(y);
+        v[j][s] = in ? (rec_moderate(y) ? z : y) : 0.f;       // (one that is not: see `serial`)
+        bad |= in && !rec_moderate(y);
       }
   };
   f32x4 v[2];
@@ -903,9 +903,9 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
     const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
     const float* fhn = fh + (more ? head_ld : 0);
     float* yr = yo + (int64_t)l0 * a.wld;
-    // An infinity or a NaN in the chunk would reach the tokens in front of it through a product with a weight of zero: the wave takes
-    // such a chunk token by token behind the products, which then count for nothing, from S in the state row and v in LDS (a rare
-    // path: it must not set the kernel's registers)
+    // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
+    // with a weight of zero: the wave takes such a chunk token by token behind the products, which then count for nothing, from S in the
+    // state row and v in LDS (a rare path: it must not set the kernel's registers)
     const bool serial = __any(bad || flag != 0.f);
     int rows = D, step = E;
     asm volatile("" : "+s"(rows), "+s"(step));
@@ -913,7 +913,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = v[j][s];
+        for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = rec_silu_if_large(v[j][s]);
       if (e_ok)
 #pragma unroll
         for (int t = 0; t < NT; ++t)

@@ -137,6 +137,38 @@ def test_state_space_in_chunks_not_finite(col, value):
         assert not bool(torch.isfinite(got[0][at:]).all())
 
 
+@pytest.mark.parametrize("large", [False, True])
+def test_state_space_in_chunks_activation_over_its_whole_range(large):
+    """The state behind a token that nothing else is left in: B dt silu(x), a dozen roundings; a silu(x) where exp(-x) leaves 32 bits,
+    2.7e-37 at most, may be lost (B dt below 1).  Values up to 2^59 in the products, larger ones token by token; the tokens in front
+    are as they would be without it."""
+    H, G, N, E, lens = 2, 1, 8, 64, [45]
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 1, lens, torch.float32, 11)
+    w["conv"], w["bias"], w["a_log"] = torch.ones_like(w["conv"]), torch.zeros_like(w["bias"]), torch.full((H,), 6.0)
+    ends = [1e20, 1e34, 2.3e38, 2.5e38, 3.3e38] if large else [1e3, 1e10, 5e17]
+    x = torch.cat([torch.tensor(ends + [-e for e in ends]), torch.linspace(-104, -80, 60), torch.linspace(-80, 100, H * E - 60 - 2 * len(ends))])
+    rows[0][-1, H * E: 2 * H * E] = x
+    rows[0][-1, 2 * H * E: 2 * H * E + N] = torch.linspace(0.2, 1.0, N)
+    rows[0][-1, 2 * H * E + 2 * G * N:], w["dt_bias"] = 0.0, torch.zeros(H)
+    outs, after, _ = _ssm_run(w, rows, state, before, [9], H, G, N, E, 1)
+    want, S, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
+    torch.testing.assert_close(outs[0][:-1].to(F64), want[:-1], rtol=2e-5, atol=2e-5)
+    torch.testing.assert_close(after[0].to(F64), S, rtol=2e-6, atol=2.0 ** -120)
+
+
+def test_state_space_in_chunks_large_operands():
+    """B of one token and C of a later one whose product leaves 32 bits, nothing of the state being left in between."""
+    H, G, N, E, lens, n = 4, 2, 32, 16, [100], 3
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 1, lens, torch.float32, 6)
+    inner = H * E
+    w["conv"], w["bias"], w["a_log"] = torch.ones_like(w["conv"]), torch.zeros_like(w["bias"]), torch.full((H,), 6.0)
+    rows[0][:, 2 * inner + n], rows[0][:, 2 * inner + G * N + n] = 0.0, 0.0
+    rows[0][70, 2 * inner + n], rows[0][80, 2 * inner + G * N + n] = 1e30, 1e30
+    outs, _, _ = _ssm_run(w, rows, state, before, [9], H, G, N, E, 1)
+    want, _, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
+    torch.testing.assert_close(outs[0].to(F64), want, rtol=2e-5, atol=2e-5)
+
+
 # ----------------------------------------------------------------------------------------------- gated delta rule
 def _delta_inputs(H, G, D, E, taps, lens, dtype, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
@@ -239,6 +271,20 @@ def test_delta_rule_in_chunks_not_finite(col, value):
     torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
     if col != "a" or value != value:
         assert not bool(torch.isfinite(got[0][at:]).all())
+
+
+def test_delta_rule_in_chunks_large_values():
+    """Two large values under opposite keys, their sum beyond 32 bits: the tokens in front of them are as they were."""
+    H, G, D, E, lens, at = 4, 2, 32, 24, [100], 90
+    gd, hv = G * D, H * E
+    w, rows, state, before = _delta_inputs(H, G, D, E, 1, lens, torch.float32, 6)
+    w["ck"], w["cv"] = torch.ones_like(w["ck"]), torch.ones_like(w["cv"])
+    rows[0][:, 2 * gd + 2 * hv:] = torch.cat([torch.full((H,), -12.0), torch.full((H,), 12.0)])
+    clean, _, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    rows[0][at: at + 2, gd: 2 * gd] = torch.tensor([[-1.28], [1.28]])
+    rows[0][at: at + 2, 2 * gd + 1] = 2.3e38
+    got, _, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
 
 
 # (a team per head: one, several in one workgroup, more heads than teams; one, some and all rows of pieces)
