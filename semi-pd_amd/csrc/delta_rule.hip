@@ -751,7 +751,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
     hp[1536 + L + ln] = wt;
     hp[1536 + 2 * L + ln] = dec;
     hp[1536 + 3 * L + ln] = beta;
-    bad |= !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_finite(la);
+    bad |= !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_moderate_decay(la);
     __builtin_amdgcn_wave_barrier();
     // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s)
     const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);

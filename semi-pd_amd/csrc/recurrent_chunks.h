@@ -51,6 +51,11 @@ __device__ __forceinline__ bool rec_finite(float x) { return fabsf(x) <= 3.40282
 // up to here a sum of 128 products of two values stays within 32 bits: a chunk with a larger one is taken token by token
 __device__ __forceinline__ bool rec_moderate(float x) { return fabsf(x) <= 0x1p59f; }
 
+// Log decays whose running sums, and the differences of these, are good to 64 bits less 26: a chunk of 32 sums to less than 2^26 (base 2),
+// so a difference is off by 2^-27 at most, which costs a weight less than its own rounding.  One of -1e14 among them costs the weights
+// behind it 6e-3, one of -1e16 sets them to 1: a chunk with such a step is taken token by token.
+__device__ __forceinline__ bool rec_moderate_decay(float la) { return fabsf(la) <= 0x1p20f; }
+
 // silu of a moderate x: e^(-x) as 2^(hi + lo) with lo = what the product with log2 e rounds away, the quotient by a reciprocal and one
 // correction of it and of the result: at most 2.8 units in the last place from the 64-bit value (x / (1 + expf(-x)): 3.4).  The
 // quotient is 2^32 times as large until the end, so that it stays in the normal range as far as e^(-x) does, to -88.722; x below has

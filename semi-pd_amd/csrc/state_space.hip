@@ -436,7 +436,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     hp[768 + L + t] = wt;
     hp[768 + 2 * L + t] = dt;
     hp[768 + 3 * L + t] = dec;
-    bad |= !rec_finite(dt) || !rec_finite(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
+    bad |= !rec_finite(dt) || !rec_moderate_decay(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
     __builtin_amdgcn_wave_barrier();
     // the weighted C B^T, 16 bytes a lane: piece i of 192 is lane i % 64 of tile i / 64; the step size of column s from lane s
 #pragma unroll

@@ -156,6 +156,21 @@ def test_state_space_in_chunks_activation_over_its_whole_range(large):
     torch.testing.assert_close(after[0].to(F64), S, rtol=2e-6, atol=2.0 ** -120)
 
 
+@pytest.mark.parametrize("largest", [6.0, 13.8, 30.0, 80.0])
+def test_state_space_in_chunks_reset(largest):
+    """A step that leaves nothing of the state, its log decay from -e^largest in front of 2^20 to behind 2^60: the tokens behind it decay
+    among themselves as without it.  The state is a sum of 19 terms of a dozen roundings each."""
+    H, G, N, E, lens, at = 4, 2, 32, 16, [60], 40
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 1, lens, torch.float32, 6)
+    w["a_log"], w["dt_bias"] = torch.full((H,), largest + 0.37), torch.zeros(H)
+    dt = rows[0][:, 2 * H * E + 2 * G * N: 2 * H * E + 2 * G * N + H]
+    dt.copy_(0.5 * dt - largest)                                                    # log decays around -1
+    dt[at] = 0.0
+    _, after, _ = _ssm_run(w, rows, state, before, [9], H, G, N, E, 1)
+    _, S, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 2e-6
+
+
 def test_state_space_in_chunks_large_operands():
     """B of one token and C of a later one whose product leaves 32 bits, nothing of the state being left in between."""
     H, G, N, E, lens, n = 4, 2, 32, 16, [100], 3
@@ -271,6 +286,21 @@ def test_delta_rule_in_chunks_not_finite(col, value):
     torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
     if col != "a" or value != value:
         assert not bool(torch.isfinite(got[0][at:]).all())
+
+
+@pytest.mark.parametrize("largest", [6.0, 13.8, 30.0, 80.0])
+def test_delta_rule_in_chunks_reset(largest):
+    """As for the state-space recurrence."""
+    H, G, D, E, lens, at = 4, 2, 32, 24, [60], 40
+    w, rows, state, before = _delta_inputs(H, G, D, E, 1, lens, torch.float32, 6)
+    w["a_log"], w["dt_bias"] = torch.full((H,), largest + 0.37), torch.zeros(H)
+    a = rows[0][:, 2 * G * D + 2 * H * E: 2 * G * D + 2 * H * E + H]
+    a.copy_(0.5 * a - largest)
+    a[at] = 0.0
+    outs, after, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    want, S, _ = _delta_truth(w, rows[0], state[0], before[0], H, G, D, E)
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 2e-6
+    assert float((outs[0].to(F64) - want).norm() / want.norm()) < 2e-6
 
 
 def test_delta_rule_in_chunks_large_values():
