@@ -84,7 +84,7 @@ def recover_after_failed_capture(device) -> None:
     if x is None:
         x = torch.ones(8, device=device)
     g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=st):
+    with without_cycle_collection(), torch.cuda.graph(g, stream=st):
         y = x * 2
     _PARKED.append((x, y, g, st))
     torch.cuda.synchronize()
@@ -162,22 +162,23 @@ class HipGraphRunner:
         torch.cuda.current_stream().wait_stream(self.stream)
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
-        try:
-            with without_cycle_collection(), torch.cuda.graph(g, pool=self.pool, stream=self.stream):
-                out = run_once()
-                if capture_fault_hook is not None:
-                    capture_fault_hook(bs, out)
-        except BaseException:
-            # something in the step refused capture (a collective of this TP backend, say): the invalidated capture
-            # poisons every later synchronising call of the process until its stream is destroyed
-            from semi_pd_amd import _lib
-            _lib.load().semipd_stream_abort_capture(self._raw_stream)
-            self._raw_stream = None
-            self._stream_finalizer.detach()   # the abort destroyed the stream
-            # nothing that lives on the dead stream may be freed (the allocator would touch the stream again): the graphs,
-            # their outputs and the runner itself are parked for the life of the process
-            _PARKED.append((self, g, self.graphs, self.outputs, self.pool, self.stream))
-            raise
+        with without_cycle_collection():           # (until a broken capture is gone as well)
+            try:
+                with torch.cuda.graph(g, pool=self.pool, stream=self.stream):
+                    out = run_once()
+                    if capture_fault_hook is not None:
+                        capture_fault_hook(bs, out)
+            except BaseException:
+                # something in the step refused capture (a collective of this TP backend, say): the invalidated capture
+                # poisons every later synchronising call of the process until its stream is destroyed
+                from semi_pd_amd import _lib
+                _lib.load().semipd_stream_abort_capture(self._raw_stream)
+                self._raw_stream = None
+                self._stream_finalizer.detach()   # the abort destroyed the stream
+                # nothing that lives on the dead stream may be freed (the allocator would touch the stream again): the graphs,
+                # their outputs and the runner itself are parked for the life of the process
+                _PARKED.append((self, g, self.graphs, self.outputs, self.pool, self.stream))
+                raise
         self.pool = self.pool or g.pool()
         self.graphs[(self._cus, bs)] = g
         self.outputs[(self._cus, bs)] = out
