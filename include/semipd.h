@@ -927,7 +927,8 @@ int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
 /* fp32 elements that semipd_delta_rule_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
 int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps);
 /* semipd_delta_rule of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a
- * time on the matrix cores in fp32.  Without room, or where sizes do not allow it: as semipd_delta_rule. */
+ * time on the matrix cores in fp32; the work rows then hold the result alone (work_ld >= num_heads * v_dim).  Without room, or where
+ * sizes do not allow it: as semipd_delta_rule. */
 int semipd_delta_rule_prompt(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
                       int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
                       const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
@@ -1006,7 +1007,8 @@ int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
 /* fp32 elements that semipd_state_space_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
 int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state, int taps);
 /* semipd_state_space of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a
- * time on the matrix cores in fp32.  Without room, or where sizes or alignment do not allow it: as semipd_state_space. */
+ * time on the matrix cores in fp32; the work rows then hold the result alone (work_ld >= num_heads * v_dim).  Without room, or where
+ * sizes or alignment do not allow it: as semipd_state_space. */
 int semipd_state_space_prompt(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
                        const void* conv_b, const float* dt_bias, const float* a_log, const float* d_skip, const void* norm_w,
                        int norm_groups, float eps, float* work, int64_t work_ld, float* state, int64_t state_ld, float* conv_state,

@@ -42,6 +42,7 @@ struct DeltaArgs {
   int H, G, D, E, taps;
   float eps;
   void* out; int64_t out_ld;                       // [T, H E] of the activation type
+  int o_off;                                       // column of o in a work row: 2 G D, in the matrix-core form (rows of o alone) 0
   float* frags;                                    // operands of the chunks (matrix-core form), see delta_chunk_operands_kernel
 };
 
@@ -582,7 +583,7 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
   const int64_t t = blockIdx.x;
   const int E = a.E;
   for (int h = threadIdx.x >> 6; h < a.H; h += 4) {
-  const float* o = a.work + t * a.wld + 2 * a.G * a.D + h * E;
+  const float* o = a.work + t * a.wld + a.o_off + h * E;
   float sq = 0.f;
   for (int e = lane; e < E; e += 64) sq += o[e] * o[e];
   sq = wave_sum(sq);
@@ -835,7 +836,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
   const float* f = a.frags + chunk0 * frag_ld + g * delta_frag_elems(NP) + 4 * lane;
   const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kDeltaHead;
   const T* p = (const T*)a.p + t0 * a.ld + a.v_off + h * E + e0;
-  float* yo = a.work + t0 * a.wld + 2 * G * D + h * E + e0;
+  float* yo = a.work + t0 * a.wld + h * E + e0;
   // 16-byte pieces of the projection's and of the result's rows: everything starts on one
   const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
                    ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
@@ -1081,7 +1082,7 @@ __global__ void __launch_bounds__(256) delta_post_vec_kernel(DeltaArgs a) {
   const bool on = item < a.num_tokens * a.H;
   const int64_t t = on ? item / a.H : 0;
   const int h = on ? (int)(item % a.H) : 0;
-  const float* o = a.work + t * a.wld + 2 * a.G * a.D + (int64_t)h * E + sl * 8;
+  const float* o = a.work + t * a.wld + a.o_off + (int64_t)h * E + sl * 8;
   const float4 o0 = *reinterpret_cast<const float4*>(o), o1 = *reinterpret_cast<const float4*>(o + 4);
   const Vec16<T> gate = load16((const T*)a.p + t * a.ld + a.gate_off + (int64_t)h * E + sl * 8), nw = load16((const T*)a.norm_w + sl * 8);
   const float x[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
@@ -1130,7 +1131,7 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
 static int launch_delta_post(const DeltaArgs& a, int dtype, hipStream_t s) {
   const int lp = a.E / 8;
   const bool vec = dtype != SEMIPD_F32 && a.E % 8 == 0 && lp <= 64 && (lp & (lp - 1)) == 0 && a.gate_off % 8 == 0 && a.ld % 8 == 0 &&
-                   a.out_ld % 8 == 0 && a.wld % 4 == 0 && (2 * a.G * a.D) % 4 == 0 && aligned16(a.p) && aligned16(a.out) && aligned16(a.work) &&
+                   a.out_ld % 8 == 0 && a.wld % 4 == 0 && a.o_off % 4 == 0 && aligned16(a.p) && aligned16(a.out) && aligned16(a.work) &&
                    aligned16(a.norm_w);
   if (!vec) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_post_kernel<T>), dim3((unsigned)a.num_tokens), dim3(256), 0, s, a));
@@ -1172,12 +1173,14 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
   SEMIPD_CHECK_ARG((q_start == nullptr) == (q_len == nullptr), SEMIPD_EINVAL, "delta_rule: q_start and q_len come together");
   SEMIPD_CHECK_ARG(q_start != nullptr || num_tokens == batch, SEMIPD_EINVAL, "delta_rule: one row per request without q_start");
   const int64_t C = 2 * (int64_t)num_k_heads * k_dim + (int64_t)num_heads * v_dim;
-  SEMIPD_CHECK_ARG(work_ld >= C + 2 * num_heads && state_ld >= (int64_t)num_heads * k_dim * v_dim &&
+  const int64_t want = q_start ? semipd_delta_rule_chunk_elems(num_tokens, batch, num_heads, num_k_heads, k_dim, taps) : 0;
+  const bool chunks = want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work);
+  SEMIPD_CHECK_ARG(work_ld >= (chunks ? (int64_t)num_heads * v_dim : C + 2 * num_heads) && state_ld >= (int64_t)num_heads * k_dim * v_dim &&
                        (taps == 1 || conv_ld >= (taps - 1) * C) && out_ld >= (int64_t)num_heads * v_dim,
                    SEMIPD_EINVAL, "delta_rule: a row of the work buffer, the state or the output is too short");
   DeltaArgs a{proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight,
               work, work_ld, state, state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens,
-              num_heads, num_k_heads, k_dim, v_dim, taps, eps, out, out_ld, chunk_work};
+              num_heads, num_k_heads, k_dim, v_dim, taps, eps, out, out_ld, chunks ? 0 : 2 * num_k_heads * k_dim, chunk_work};
   hipStream_t st = as_stream(stream);
   // lanes per column and rows of S per lane: four lanes share a column from 32 rows up
   const int ds = k_dim >= 32 ? 4 : 1;
@@ -1227,8 +1230,7 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
                                                          dim3(256), 0, st, a));
     return launch_status("delta_rule(decode)");
   }
-  const int64_t want = q_start ? semipd_delta_rule_chunk_elems(num_tokens, batch, num_heads, num_k_heads, k_dim, taps) : 0;
-  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work)) {
+  if (chunks) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, if (k_dim <= 64) launch_delta_chunks<T, 64>(a, st); else launch_delta_chunks<T, 128>(a, st));
     if (taps > 1)
       SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch),

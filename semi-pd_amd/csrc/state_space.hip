@@ -964,7 +964,9 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     if (rc) return SEMIPD_EINVAL;
     return launch_status("state_space_decode");
   }
-  SEMIPD_CHECK_ARG(work && work_ld >= semipd_state_space_work_width(num_heads, groups, state_size, v_dim), SEMIPD_EINVAL,
+  const int64_t want = q_start ? semipd_state_space_chunk_elems(num_tokens, batch, num_heads, groups, state_size, taps) : 0;
+  const bool chunks = want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work);
+  SEMIPD_CHECK_ARG(work && work_ld >= (chunks ? inner : semipd_state_space_work_width(num_heads, groups, state_size, v_dim)), SEMIPD_EINVAL,
                    "state_space: the work rows are missing or too short");
   // gate and norm with 16-byte accesses and the row in registers
   const int64_t gs = inner / norm_groups;
@@ -976,8 +978,7 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     else SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a))
     return 0;
   };
-  const int64_t want = q_start ? semipd_state_space_chunk_elems(num_tokens, batch, num_heads, groups, state_size, taps) : 0;
-  if (want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work)) {
+  if (chunks) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, if (state_size <= 64) launch_ssm_chunks<T, 64>(a, s); else launch_ssm_chunks<T, 128>(a, s));
     if (taps > 1) {
       const dim3 grid((unsigned)((C + 255) / 256), (unsigned)batch);

@@ -1709,6 +1709,19 @@ def latent_attention_fwd(q: torch.Tensor, out: torch.Tensor, pool: torch.Tensor,
                                               current_stream(q.device)), "latent_attention")
 
 
+def _chunk_room(tokens: int, width: int, elems: int, device):
+    """What a recurrence over a prompt batch wants to take it in chunks of 32 tokens: work rows of the result alone, `width` fp32
+    columns, and room for the operands of the chunks, `elems` fp32 elements (0: it does not go in chunks).  (None, None) where the device
+    has not that much memory left: the form that goes token by token needs less in all."""
+    if elems == 0:
+        return None, None
+    try:
+        room = torch.empty(elems, dtype=torch.float32, device=device)
+        return torch.empty((tokens, -(-width // 4) * 4), dtype=torch.float32, device=device), room
+    except torch.OutOfMemoryError:
+        return None, None
+
+
 def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.Tensor, conv_v: torch.Tensor, a_log: torch.Tensor,
                dt_bias: torch.Tensor, norm_weight: torch.Tensor, eps: float, state: torch.Tensor, conv_state: Optional[torch.Tensor],
                state_indices: torch.Tensor, seq_lens: torch.Tensor, q_start: Optional[torch.Tensor], q_len: Optional[torch.Tensor],
@@ -1745,15 +1758,15 @@ def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.
     elif out.shape != (T, hv) or out.dtype != proj.dtype or out.stride(1) != 1:
         raise RuntimeError("delta_rule: out is [T, H * v_dim] of the activation type")
     lib = _lib.load()
-    wld = int(lib.semipd_delta_rule_work_width(num_heads, num_k_heads, k_dim, v_dim))
-    work = torch.empty((T, wld), dtype=torch.float32, device=proj.device)
+    elems = int(lib.semipd_delta_rule_chunk_elems(T, B, num_heads, num_k_heads, k_dim, taps)) if q_start is not None else 0
+    work, chunk_work = _chunk_room(T, hv, elems, proj.device)
+    if work is None:
+        work = torch.empty((T, int(lib.semipd_delta_rule_work_width(num_heads, num_k_heads, k_dim, v_dim))), dtype=torch.float32, device=proj.device)
     args = (ptr(proj), proj.stride(0), *[int(o) for o in offsets], ptr(conv_q), ptr(conv_k), ptr(conv_v), ptr(a_log), ptr(dt_bias),
-            ptr(norm_weight), float(eps), ptr(work), wld, ptr(state), state.stride(0), ptr(conv_state),
+            ptr(norm_weight), float(eps), ptr(work), work.stride(0), ptr(state), state.stride(0), ptr(conv_state),
             conv_state.stride(0) if conv_state is not None else 0, ptr(state_indices), ptr(seq_lens), ptr(q_start), ptr(q_len), B, T,
             num_heads, num_k_heads, k_dim, v_dim, taps, ptr(out), out.stride(0))
-    elems = int(lib.semipd_delta_rule_chunk_elems(T, B, num_heads, num_k_heads, k_dim, taps)) if q_start is not None else 0
-    if elems:         # a prompt batch: room for the operands of its chunks of 32 tokens
-        chunk_work = torch.empty(elems, dtype=torch.float32, device=proj.device)
+    if chunk_work is not None:
         check(lib.semipd_delta_rule_prompt(*args, ptr(chunk_work), elems, dtype_code(proj.dtype), current_stream(proj.device)), "delta_rule")
     else:
         check(lib.semipd_delta_rule(*args, dtype_code(proj.dtype), current_stream(proj.device)), "delta_rule")
@@ -2015,17 +2028,17 @@ def state_space(proj: torch.Tensor, z_off: int, x_off: int, dt_off: int, conv_w:
         raise RuntimeError("state_space: out is [T, H * E] of the activation type")
     lib = _lib.load()
     fused = q_start is None and inner * state_size * 4 <= STATE_SPACE_FUSED_DECODE_BYTES
-    wld, work = 0, None
-    if not fused:
-        wld = int(lib.semipd_state_space_work_width(num_heads, groups, state_size, v_dim))
-        work = torch.empty((T, wld), dtype=torch.float32, device=proj.device)
+    elems = int(lib.semipd_state_space_chunk_elems(T, B, num_heads, groups, state_size, taps)) if q_start is not None else 0
+    work, chunk_work = _chunk_room(T, inner, elems, proj.device)
+    if work is None and not fused:
+        work = torch.empty((T, int(lib.semipd_state_space_work_width(num_heads, groups, state_size, v_dim))), dtype=torch.float32,
+                           device=proj.device)
     args = (ptr(proj), proj.stride(0), int(z_off), int(x_off), int(dt_off), ptr(conv_w), ptr(conv_b), ptr(dt_bias), ptr(a_log),
-            ptr(d_skip), ptr(norm_weight), int(norm_groups), float(eps), ptr(work), wld, ptr(state), state.stride(0), ptr(conv_state),
+            ptr(d_skip), ptr(norm_weight), int(norm_groups), float(eps), ptr(work), work.stride(0) if work is not None else 0, ptr(state),
+            state.stride(0), ptr(conv_state),
             conv_state.stride(0) if conv_state is not None else 0, ptr(state_indices), ptr(seq_lens), ptr(q_start), ptr(q_len), B, T,
             num_heads, groups, state_size, v_dim, taps, ptr(out), out.stride(0))
-    elems = int(lib.semipd_state_space_chunk_elems(T, B, num_heads, groups, state_size, taps)) if q_start is not None else 0
-    if elems:         # a prompt batch: room for the operands of its chunks of 32 tokens
-        chunk_work = torch.empty(elems, dtype=torch.float32, device=proj.device)
+    if chunk_work is not None:
         check(lib.semipd_state_space_prompt(*args, ptr(chunk_work), elems, dtype_code(proj.dtype), current_stream(proj.device)), "state_space")
     else:
         check(lib.semipd_state_space(*args, 1 if fused else 0, dtype_code(proj.dtype), current_stream(proj.device)), "state_space")

@@ -334,3 +334,40 @@ def test_delta_rule_decode_step(dtype, H, G, D, E, taps):
             torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
             torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
         state, before, first = after.clone(), last.clone(), [f + 1 for f in first]
+
+
+@pytest.mark.parametrize("scarce", [False, True])
+@pytest.mark.parametrize("kind", ["state_space", "delta_rule"])
+def test_room_for_the_chunks(kind, scarce, monkeypatch):
+    """Beside the operands of the chunks a prompt batch takes one fp32 row of the result per token; where the device has no room for the
+    operands, the call runs in what it took without them."""
+    from semi_pd_amd import _lib
+    lib, empty, sizes = _lib.load(), torch.empty, []
+    if kind == "state_space":
+        H, G, N, E, lens = 4, 2, 128, 64, [64, 130]
+        w, rows, state, before = _ssm_inputs(H, G, N, E, 4, lens, torch.float32, 2)
+        run, truth, extra = _ssm_run, _ssm_truth, (1,)
+        elems = lib.semipd_state_space_chunk_elems(sum(lens), 2, H, G, N, 4)
+        wide = lib.semipd_state_space_work_width(H, G, N, E)
+    else:
+        H, G, N, E, lens = 4, 2, 128, 128, [64, 130]
+        w, rows, state, before = _delta_inputs(H, G, N, E, 4, lens, torch.float32, 2)
+        run, truth, extra = _delta_run, _delta_truth, ()
+        elems = lib.semipd_delta_rule_chunk_elems(sum(lens), 2, H, G, N, 4)
+        wide = lib.semipd_delta_rule_work_width(H, G, N, E)
+
+    def limited(*size, **kw):
+        n = size[0] if isinstance(size[0], int) else size[0][0] * size[0][1]
+        if n == elems and scarce:
+            raise torch.OutOfMemoryError("no room")
+        sizes.append(n)
+        return empty(*size, **kw)
+
+    monkeypatch.setattr(torch, "empty", limited)
+    outs, after, _ = run(w, rows, state, before, [9, 9], H, G, N, E, *extra)
+    monkeypatch.undo()
+    assert sum(sizes) <= sum(lens) * (H * E + wide) if scarce else sum(sizes) <= elems + 2 * sum(lens) * H * E
+    for b in range(2):
+        want, S, _ = truth(w, rows[b], state[b], before[b], H, G, N, E, *extra)
+        torch.testing.assert_close(outs[b].to(F64), want, rtol=2e-5, atol=2e-5)
+        torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
