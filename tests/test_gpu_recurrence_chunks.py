@@ -371,3 +371,25 @@ def test_room_for_the_chunks(kind, scarce, monkeypatch):
         want, S, _ = truth(w, rows[b], state[b], before[b], H, G, N, E, *extra)
         torch.testing.assert_close(outs[b].to(F64), want, rtol=2e-5, atol=2e-5)
         torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["state_space", "delta_rule"])
+def test_many_requests_in_chunks(kind):
+    """More than one wave's lanes of requests (131, then a part of another 64), uneven, some without a row in the launch: a request's
+    chunks are found by counting the ones in front of it, 64 requests at a time."""
+    lens = [(40, 1, 0, 33, 17)[i % 5] for i in range(131)]
+    first = [37 if n == 0 or i % 2 else 0 for i, n in enumerate(lens)]
+    H, G, N, E = 2, 1, 8, 16
+    inputs, run, truth, extra = ((_ssm_inputs, _ssm_run, _ssm_truth, (1,)) if kind == "state_space" else
+                                 (_delta_inputs, _delta_run, _delta_truth, ()))
+    w, rows, state, before = inputs(H, G, N, E, 4, lens, torch.float32, 17)
+    outs, after, last = run(w, rows, state, before, first, H, G, N, E, *extra)
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert torch.equal(after[b], state[b]) and torch.equal(last[b], before[b])
+            continue
+        s, c = (state[b], before[b]) if first[b] else (torch.zeros_like(state[b]), torch.zeros_like(before[b]))
+        want, S, tail = truth(w, rows[b], s, c, H, G, N, E, *extra)
+        torch.testing.assert_close(outs[b].to(F64), want, rtol=2e-5, atol=2e-5)
+        torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
