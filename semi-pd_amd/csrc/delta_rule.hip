@@ -607,9 +607,9 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
 // differences are taken, in 64 bits.
 // Bound: token by token a step is a chain of two dot products, a lane sum and an update (0.8 us; 7262 tokens of 4 requests, 32 heads of
 // 128 x 128: 1861 us + 317 of preparation); in chunks a wave's chain of 216 products of 32 cycles a chunk (72 chunks: 207 us, one
-// wave a SIMD at 4 requests): 370 us, operands 91.  With the raw inputs of v fetched at the end of a chunk and convolved in
+// wave a SIMD at 4 requests; busy for 45 % of the SIMD cycles, the vector unit for 18 %): 385 us, operands 95.  With the raw inputs of v fetched at the end of a chunk and convolved in
 // front of the products 483 (the loads of 35 rows 24 KB apart were waited for), fetched a whole chunk ahead 390, by 16 bytes a lane
-// through the wave's LDS 370.
+// through the wave's LDS 370 (then; 385 with the larger range of silu).
 
 // fp32 elements of the operands of one (chunk, key head): K, Q and K^T as left-hand operands of 16 x 16 x 16 products, the
 // order in which they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a
@@ -794,8 +794,9 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
 // The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
 // sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, which is
 // also how the right-hand operand of a product over the rows is held, so S, R = V - e^b K S and U go from sums into products
-// without moving; v is convolved in its place by the lane that needs it.  Left-hand operands come straight into registers in the
-// order they are used, the next chunk's into the registers that this chunk has just read: no LDS, no barriers.
+// without moving; v is convolved in its place by the lane that needs it, from raw inputs in the wave's own LDS.  Left-hand operands
+// come straight into registers in the order they are used, not through LDS, the next chunk's into the registers that this chunk has
+// just read.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
   constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
@@ -1074,7 +1075,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
 }
 
 // The same with 16-byte accesses: a head is taken by LP = E / 8 lanes (a power of two), 64 / LP heads per wave.  Bound by HBM: 7262
-// tokens of 32 heads of 128, 238 MB: 84 us -> 44.
+// tokens of 32 heads of 128, 238 MB: 84 us -> 46.
 template <typename T, int LP>
 __global__ void __launch_bounds__(256) delta_post_vec_kernel(DeltaArgs a) {
   const int lane = threadIdx.x & 63, sl = lane % LP, E = a.E;
@@ -1108,7 +1109,8 @@ extern "C" int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, 
   return (w + 3) / 4 * 4;
 }
 
-// The rows per request (on average) from which a prompt batch goes in chunks.  Token by token against chunks, whole call, 32 heads of
+// The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
+// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call, 32 heads of
 // 128 x 128: 1 request of 2 rows 51 / 43 us, 64 rows 96 / 54, 256 rows 251 / 92; 4 requests of 2 rows 53 / 44; 32 requests of 8 rows
 // 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; heads of 64 x 64: 4 requests of 2 rows 49 / 37, 32 requests of 8 rows 60 / 78, 16 rows
 // 82 / 83, 64 rows 200 / 134.  A few requests take chunks whatever their length.

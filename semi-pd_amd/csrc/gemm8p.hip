@@ -23,6 +23,8 @@
 //     the other reads LDS and issues DMA.  The two groups share the SIMDs pairwise (wave w and w + 4).
 //   * ordering of LDS-DMA data: a wave waits (counted vmcnt) for ITS share of a half-tile before a barrier that every
 //     reader passes before its ds_read; a slot is re-filled at least two phases after its last read.
+// Grouped (experts): the two wave bands take the entries of a tile by turns, so half h of x is entries XH h .. XH h + XH - 1 of the tile
+// in their order, band wr of it the XH / 2 from XH / 2 wr on, and a lane's output rows are found through the same order (`live` below).
 // Epilogues: plain store, SiLU(gate) * up for a merged [gate; up] weight (W half 0 = gate rows, half 1 = the up rows of
 // the same columns), fp32 K-slice planes for split-K.
 // replaces UnquantizedLinearMethod.apply -> F.linear (+ SiluAndMul) (layers/linear.py:165-172, models/llama.py:88-92,
@@ -150,7 +152,7 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
 
   // ---- DMA sources.  A half-tile of R rows is R / 8 wave instructions (8 rows x 128 B each); a wave issues instructions
   //      wave * L + e; instruction j fills LDS rows r' = 8 j + (lane >> 3) with chunk position lane & 7, i.e. source chunk
-  //      (lane & 7) ^ ((r' >> 1) & 7).  x half h holds rows h XH/2 .. + XH/2 - 1 of both wave bands; W half h rows
+  //      (lane & 7) ^ ((r' >> 1) & 7).  x half h holds rows h XH/2 .. + XH/2 - 1 of both wave bands (grouped: entries h XH .. + XH - 1); W half h rows
   //      h WH/4 .. + WH/4 - 1 of the four wave columns (SiLU form: half 0 = gate rows, half 1 = the up rows of the same
   //      output columns). ----
   const T* srcx[2][LX];
@@ -315,7 +317,8 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
   g8_wait_vm<0>();                    // no DMA may land in LDS that the next workgroup owns
   if (wr == 0) g8_barrier();          // the barrier group 1 spent up front
 
-  // ---- epilogue: lane holds out[m = m0 + XH wr + 16 i + c16][n = n0 + (WH / 2) wc + 16 j + 4 q4 + r] ----
+  // ---- epilogue: lane holds out[m = m0 + XH wr + 16 i + c16][n = n0 + (WH / 2) wc + 16 j + 4 q4 + r] (grouped: of entry
+  //      m0 + XH (i / MT2) + XH / 2 wr + 16 (i % MT2) + c16) ----
   const int mb = m0 + XH * wr + c16;
   if (planes != nullptr) {
     float* pl = planes + (int64_t)ks * M * N;

@@ -3,8 +3,8 @@
 //
 //  * A workgroup: NW waves = HW query heads of ONE key/value head x NW / HW blocks of 32 rows, so the rows of K and V that it
 //    stages serve up to NW heads.  Heads share the visible range, and every wave of a workgroup has the same number of steps.
-//  * A step: KT keys (64, or 32).  Their K and V rows go through two pairs of LDS tiles (step i + 1 lands in registers while step i is
-//    multiplied; one barrier a step).  S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16: a lane holds one query's column
+//  * A step: KT keys (64; 32 for value rows of 256).  Their K and V rows go through two pairs of LDS tiles (step i + 1 lands in
+//    registers while step i is multiplied; one barrier a step).  S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16: a lane holds one query's column
 //    throughout, P^T goes from the accumulators into the second product in place (its key order is matched by the rows that the
 //    transposing reads of V take).
 //  * 16-byte chunk c of row r lies at c ^ (r & 15) of a K tile (the 32 rows of an operand read start in different banks), the 64-byte
@@ -14,12 +14,15 @@
 //    one).  Letting it lag by up to 2^6 was 2 .. 5 % further.
 //  * A weight of zero does not hide an infinity or a NaN from a product, and a wave multiplies keys that some of its rows do not see: a
 //    wave that ends with sums that are not finite takes its rows again, one by one.
-// Bound: at 64 keys a wave multiplies for 32 x 32 cycles (128 / 128), reads 32 KB of LDS and takes 32 exponentials a lane (16 cycles
-// each) with five instructions around each: matrix pipe, LDS and vector unit are close to each other, two waves a SIMD fill each
-// other's gaps.  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves
-// of one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 260 -> 110 us (500 TFLOP/s); value rows of 256: 2030 -> 380 (steps
-// of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000: 69 -> 48; 8 x 40: 10.6 -> 9.8.  A fresh prompt of at most 20
-// tokens is one step of either, 7.7 -> 8.4 us; behind 100 tokens the same rows are 12.7 -> 10.0.
+// Bound: a wave multiplies for 32 x 32 cycles a step of 64 keys (128 / 128), reads 32 KB of LDS and takes 32 exponentials a lane (16
+// cycles each) with five instructions around each.  Of the SIMD cycles of the batch below the vector unit is busy for 42 %, the matrix
+// pipe for 20 %, the LDS for about a third of its own; two waves a SIMD fill only part of each other's gaps (value rows of 256: 30, 19
+// and a third).  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves of
+// one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 110 us (500 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
+// 341 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.  A fresh
+// prompt of at most 32 tokens is one step of either, and its 32 x 64 products are four times those of the wave of 16 rows: 20 tokens 6.5
+// -> 7.8 us, 8 x 20 7.0 -> 8.1; behind 100 tokens 11.7 -> 9.6 and 12.3 -> 9.9 (how far a request reaches back is on the device, so the host
+// cannot choose; leaving out a step's second 32 keys where there are none took 0.5 us off the short ones and put 10 on the large).
 #pragma once
 
 namespace semipd {

@@ -316,9 +316,9 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
 // good as the product of the decays themselves.
 // Bound: token by token a step is a chain of LDS reads, 64 multiply-adds and lane sums (1.0 us of a wave's time; 7262 tokens of 4
 // requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (140 products
-// of 32 cycles a wave and chunk: 250 us here), the vector work between its products and their loads: 545 us, operands 72.  Chunks of
-// 32 and not 64: the same products with S, half the ones inside a chunk; operands straight into registers and not through LDS: no
-// barriers, 560 -> 545 (64 tokens, operands in LDS, two heads a workgroup: 952 us).
+// of 32 cycles a wave and chunk: 250 us here, busy for 38 % of the SIMD cycles), the vector work between its products (17 %) and their
+// loads: 560 us, operands 72.  Chunks of 32 and not 64: the same products with S, half the ones inside a chunk; operands straight
+// into registers and not through LDS: no barriers, 15 us less (64 tokens, operands in LDS, two heads a workgroup: 952 us).
 // fp32 elements of the operands of one (chunk, group): C and B^T as left-hand operands of 16 x 16 x 16 products, in the order in which
 // they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a piece of 4.  Of one
 // (chunk, head): tiles 00, 10, 11 of the weighted C B^T, then e^(b_t) | e^(b_last - b_t) dt_t | dt | decay.
@@ -461,8 +461,9 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
 // sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16.  That is
 // also how a wave holds the right-hand operand of a product over the rows, so S goes from one chunk's sum into the next one's product
 // without leaving its registers, and so do the chunk's x (lane: tokens 16 j + 4 kq + s of its column), which each lane convolves in
-// their place: x never touches memory.  Left-hand operands come straight into registers in the order they are used: B^T of a chunk
-// into the registers its C was read from, the next chunk's C into those of B^T.  No LDS, no barriers.
+// their place from raw inputs in the wave's own LDS: x is not written to memory.  Left-hand operands come straight into registers in
+// the order they are used, not through LDS: B^T of a chunk into the registers its C was read from, the next chunk's C into those of
+// B^T.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
   constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
@@ -708,7 +709,7 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
 
 // gate, grouped norm, weight, one pass: a workgroup per (token, norm group), the group's elements in registers, 16-byte accesses
 // (8 elements a piece, at most kPostPieces pieces a thread).  Bound by HBM: 7262 x 8192 169 us (two passes, 2- and 4-byte accesses) ->
-// 89 = 5.4 TB/s; 32 rows 28 -> 7 us.
+// 86 = 5.5 TB/s; 32 rows 28 -> 7 us.
 constexpr int kPostPieces = 4;
 template <typename T>
 __global__ void __launch_bounds__(256) ssm_post_vec_kernel(SsmArgs a) {
@@ -902,8 +903,8 @@ extern "C" int64_t semipd_state_space_work_width(int num_heads, int groups, int 
   return (w + 3) / 4 * 4;
 }
 
-// The rows per request (on average) from which a prompt batch goes in chunks, and how many chunks a launch can have.  Token by
-// token against chunks, whole call, 128 heads of 128 x 64: 1 request of 8 rows 34.0 / 36.1 us, 12 rows 37.3 / 36.4, 32 rows 56 / 40,
+// The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
+// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call, 128 heads of 128 x 64: 1 request of 8 rows 34.0 / 36.1 us, 12 rows 37.3 / 36.4, 32 rows 56 / 40,
 // 256 rows 327 / 79; 32 requests of 8 rows 185 / 148, 32 rows 548 / 191, 256 rows 3058 / 782; 64 heads: 1 request of 12 rows 34.3 / 33.8,
 // 32 requests of 8 rows 110 / 88.
 constexpr int64_t kSsmChunkMinRows = 12;

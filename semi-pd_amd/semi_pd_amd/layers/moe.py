@@ -71,8 +71,9 @@ MOE_TALL_MIN_ROWS = int(os.environ.get("SEMIPD_MOE_TALL_MIN_ROWS", "4096"))
 MOE_TALL_MIN_ROWS_PER_EXPERT = int(os.environ.get("SEMIPD_MOE_TALL_MIN_ROWS_PER_EXPERT", "128"))
 # below those bounds, from this many rows per expert up: the 128-row x 512-column geometry of the same kernel (most experts
 # are one block; the 256-row geometry takes over where most would be two).  One prefill request of DeepSeek-V2-Lite on
-# the 128-CU share: T = 512 338 -> 306 us, 1024 381 -> 331, 1280 ~470 -> 417; from 1408 tokens the 256-row geometry
-# (632 -> 463 at 1536) (profiles/r03_kbench_moe_mid_geometry.txt)
+# the 128-CU share: T = 512 338 -> 306 us, 1024 381 -> 331, 1280 ~470 -> 417; the 256-row geometry from 128 rows per expert
+# (632 -> 463 at 1536 tokens) (profiles/r03_kbench_moe_mid_geometry.txt).  Since it leaves padding quadrants out the 256-row
+# geometry is ahead on the whole chip at 112 rows already (314 against 343 us): the bound is from before that.
 MOE_MID_MIN_ROWS_PER_EXPERT = int(os.environ.get("SEMIPD_MOE_MID_MIN_ROWS_PER_EXPERT", "40"))
 MOE_STREAM_DECODE = os.environ.get("SEMIPD_MOE_STREAM_DECODE", "1") != "0"   # A/B knob: 0 = the register-fragment kernel
 MOE_STREAM_MAX_TOKENS = int(os.environ.get("SEMIPD_MOE_STREAM_MAX_TOKENS", "320"))
