@@ -567,24 +567,13 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
     const float* fhn = fh + (more ? head_ld : 0);
     float* yr = yo + (int64_t)l0 * a.wld;
     // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
-    // with a weight of zero: the wave takes such a chunk token by token behind the products, which then count for nothing, from S in the
-    // state row and x in LDS (a rare path: it must not set the kernel's registers)
-    const bool serial = __any(bad || flag != 0.f);
+    // with a weight of zero, and so would a product of a large S with rows behind a step that resets it: the wave takes such a chunk
+    // token by token behind the products, which then count for nothing, from S in the state row and x in LDS (a rare path: it must
+    // not set the kernel's registers)
+    const bool flagged = bad || flag != 0.f;
     int rows = N, step = E;
     asm volatile("" : "+s"(rows), "+s"(step));
-    if (serial) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = rec_silu_if_large(x[j][s]);
-      if (e_ok)
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
-      __builtin_amdgcn_sched_barrier(0);
-    }
+    bool serial;
     f32x4 xn[2];
     {
       const float keep = __shfl(eb[1][3], 63, 64);
@@ -621,6 +610,33 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
         __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
       }
       if (l0 + 2 * L < n) fetch_x(l0 + 2 * L);
+      {
+        float z = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) z = fmaf(O[i / 4][i % 4], 0.f, z);
+        serial = __any(flagged);
+        if (__any(z != 0.f)) {                                   // (a column of S that is not finite stays so in either form)
+          float c = 0.f;
+#pragma unroll
+          for (int t = 0; t < NT; ++t) c = fmaf(S[t][0], 0.f, fmaf(S[t][1], 0.f, fmaf(S[t][2], 0.f, fmaf(S[t][3], 0.f, c))));
+          c += __shfl_xor(c, 16, 64);
+          c += __shfl_xor(c, 32, 64);
+          serial |= __any(z != 0.f && c == 0.f);
+        }
+      }
+      if (serial) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = rec_silu_if_large(x[j][s]);
+        if (e_ok)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int i = 0; i < 2; ++i) O[i] *= eb[i];
 #pragma unroll

@@ -184,6 +184,20 @@ def test_state_space_in_chunks_large_operands():
     torch.testing.assert_close(outs[0].to(F64), want, rtol=2e-5, atol=2e-5)
 
 
+def test_state_space_in_chunks_large_state():
+    """A state whose product with a later row of C leaves 32 bits, while all steps leave nothing of it: as token by token."""
+    H, G, N, E, lens = 4, 2, 32, 16, [45]
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 1, lens, torch.float32, 6)
+    inner = H * E
+    w["conv"], w["bias"], w["a_log"], w["dt_bias"] = torch.ones_like(w["conv"]), torch.zeros_like(w["bias"]), torch.full((H,), 6.0), torch.ones(H)
+    rows[0][:, 2 * inner + 2 * G * N: 2 * inner + 2 * G * N + H] = 0.0               # (log decays of -530)
+    rows[0][12, 2 * inner + G * N: 2 * inner + 2 * G * N] = 1e12
+    outs, after, _ = _ssm_run(w, rows, 1e30 * state, before, [9], H, G, N, E, 1)
+    want, S, _ = _ssm_truth(w, rows[0], 1e30 * state[0], before[0], H, G, N, E, 1)
+    torch.testing.assert_close(outs[0].to(F64), want, rtol=2e-5, atol=2e-5)
+    torch.testing.assert_close(after[0].to(F64), S, rtol=1e-5, atol=1e-5)
+
+
 # ----------------------------------------------------------------------------------------------- gated delta rule
 def _delta_inputs(H, G, D, E, taps, lens, dtype, seed, scale=1.0):
     g = torch.Generator().manual_seed(seed)
@@ -315,6 +329,22 @@ def test_delta_rule_in_chunks_large_values():
     rows[0][at: at + 2, 2 * gd + 1] = 2.3e38
     got, _, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
     torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
+
+
+def test_delta_rule_in_chunks_large_state():
+    """The same with the product of the state and a dense key; the first token's key has one element."""
+    H, G, D, E, lens = 4, 2, 128, 24, [45]
+    gd, hv = G * D, H * E
+    w, rows, state, before = _delta_inputs(H, G, D, E, 1, lens, torch.float32, 6)
+    w["ck"], w["a_log"], w["dt_bias"] = torch.ones_like(w["ck"]), torch.full((H,), 6.0), torch.zeros(H)
+    rows[0][:, 2 * gd + 2 * hv: 2 * gd + 2 * hv + H] = 2.0                           # (log decays of -850)
+    rows[0][:, gd: 2 * gd] = rows[0][:, gd: 2 * gd].abs() + 0.5
+    rows[0][0, gd: 2 * gd] = torch.tensor([4.0] + [0.0] * (D - 1)).repeat(G)
+    state = torch.full_like(state, 1.5e38)
+    outs, after, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    want, S, _ = _delta_truth(w, rows[0], state[0], before[0], H, G, D, E)
+    torch.testing.assert_close(outs[0].to(F64), want, rtol=2e-5, atol=2e-5)
+    torch.testing.assert_close(after[0].to(F64), S, rtol=1e-5, atol=1e-5)
 
 
 # (a team per head: one, several in one workgroup, more heads than teams; one, some and all rows of pieces)
