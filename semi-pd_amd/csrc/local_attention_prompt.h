@@ -19,10 +19,11 @@
 // pipe for 20 %, the LDS for about a third of its own; two waves a SIMD fill only part of each other's gaps (value rows of 256: 30, 19
 // and a third).  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves of
 // one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 110 us (500 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
-// 341 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.  A fresh
-// prompt of at most 32 tokens is one step of either, and its 32 x 64 products are four times those of the wave of 16 rows: 20 tokens 6.5
-// -> 7.8 us, 8 x 20 7.0 -> 8.1; behind 100 tokens 11.7 -> 9.6 and 12.3 -> 9.9 (how far a request reaches back is on the device, so the host
-// cannot choose; leaving out a step's second 32 keys where there are none took 0.5 us off the short ones and put 10 on the large).
+// 341 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.
+// A fresh prompt of at most 32 tokens is one step of either, and its 32 x 64 products are four times those of the wave of 16 rows: 20
+// tokens 7.3 -> 7.4 us, 32 tokens 7.4 -> 7.9, with sigmoid weights 6.5 -> 7.1 and 6.6 -> 7.6 (behind 100 tokens 20 tokens are 12.4 -> 9.6;
+// how far a request reaches back is on the device, so the host cannot choose; leaving out a step's second 32 keys where there
+// are none took 0.5 us off the short ones and put 10 on the large).
 #pragma once
 
 namespace semipd {
@@ -101,44 +102,65 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
   // Workgroup -> (kv head, tile, heads of the group), the last fastest, an XCD walking a contiguous range of items: the workgroups
   // that read the same K and V rows run next to each other on one L2.  Tiles from the last (most keys) to the first.
-  const int rows_wg = 32 * (NW / hw);
-  const int rep = a.H / a.G, sets = rep / hw;
-  const int64_t n_items = gridDim.x, item = (int64_t)(blockIdx.x & 7) * (n_items >> 3) + (blockIdx.x >> 3);
-  const int64_t n_tiles = a.n_tiles;
+  // (32 bits and shifts: with 64-bit quotients here and in the search for the request 20 tokens took 8.3 us for 7.4)
+  const int hw_shift = 31 - __builtin_clz(hw), shift = 31 - __builtin_clz(32 * NW) - hw_shift, rows_wg = 1 << shift;      // (hw: a power of two)
+  const uint32_t rep = a.H / a.G, sets = (rep + hw - 1) >> hw_shift, n_tiles = (uint32_t)a.n_tiles;
+  const uint32_t item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
   if (item >= n_tiles * a.G * sets) return;
-  const int gk = (int)(item / (n_tiles * sets)), set = (int)(item % sets);
-  const int64_t tile_id = n_tiles - 1 - (item / sets) % n_tiles;
+  const uint32_t of_set = item / sets;
+  const int set = (int)(item - of_set * sets), gk = (int)(of_set / n_tiles);
+  const uint32_t tile_id = n_tiles - 1 - (of_set - gk * n_tiles);
   int b = -1;
   int q0 = 0;
   {
-    int64_t left = tile_id;
-    for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 8) {     // eight lengths per round trip
+    int left = (int)tile_id;
+    if (a.batch <= 8) {                                          // eight lengths in a round trip
       int32_t n[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u) n[u] = rq0 + u < (int)a.batch ? a.q_len[rq0 + u] : 0;
+      for (int u = 0; u < 8; ++u) n[u] = u < (int)a.batch ? a.q_len[u] : 0;
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const int64_t tiles = ((int64_t)n[u] + rows_wg - 1) / rows_wg;
+        const int tiles = (n[u] + rows_wg - 1) >> shift;
         if (b < 0 && left < tiles) {
-          b = rq0 + u;
-          q0 = (int)left * rows_wg;
+          b = u;
+          q0 = left << shift;
         }
         if (b < 0) left -= tiles;
+      }
+    } else {                                                     // 64 of them, a lane each (eight at a time 96 requests of 300 tokens, 16 heads of 128: 229 us for 148)
+      for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 64) {
+        const int tiles = rq0 + lane < (int)a.batch ? (max(a.q_len[rq0 + lane], 0) + rows_wg - 1) >> shift : 0;
+        int upto = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+          const int below = __shfl_up(upto, d, 64);
+          if (lane >= d) upto += below;
+        }
+        const uint64_t past = __ballot(left < upto);
+        if (past != 0) {
+          const int first = __builtin_ctzll(past);
+          b = rq0 + first;
+          q0 = (left - (__shfl(upto, first, 64) - __shfl(tiles, first, 64))) << shift;
+        } else {
+          left -= __shfl(upto, 63, 64);
+        }
       }
     }
   }
   if (b < 0) return;
   b = __builtin_amdgcn_readfirstlane(b);
   q0 = __builtin_amdgcn_readfirstlane(q0);
-  const int h = gk * rep + set * hw + wave % hw;
+  const int hg = set * hw + (wave & (hw - 1));                  // head of the group (the last set may not be full)
+  const bool h_ok = hg < (int)rep;
+  const int h = gk * (int)rep + (h_ok ? hg : (int)rep - 1);
   const int qn = a.q_len[b], base_pos = (int)(a.seq_lens[b] - qn);
   const int64_t t0 = a.q_start[b];
   const int keep = a.window > 0 ? a.keep_first : 0;
   const int wg_last = min(q0 + rows_wg, qn) - 1;
   const int key_lo = (int)range_lo(a, base_pos + q0), key_hi = base_pos + wg_last;
   // this wave's 32 rows
-  const int wq0 = q0 + 32 * (wave / hw);
-  const bool wave_on = wq0 < qn;
+  const int wq0 = q0 + 32 * (wave >> hw_shift);
+  const bool wave_on = wq0 < qn && h_ok;
   const int wq_last = min(wq0 + 31, qn - 1);
   const int w_first = base_pos + wq0, w_hi = base_pos + wq_last;
   const int w_lo = (int)range_lo(a, w_first), w_full = (int)range_lo(a, w_hi);     // first key that any / every row of the wave sees
@@ -377,14 +399,21 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
 template <typename T, int D, int E, int NW, int KT, bool SIG>
 static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   const int rep = a.H / a.G;
-  int hw = NW;
+  // heads of a group in a workgroup: the largest power of two that divides them, or the next one above them (the last set's waves are not all
+  // busy) where that makes fewer workgroups of requests of the average length.  24 / 8 heads, 32 requests of 20 tokens: one head and room
+  // for 128 rows a workgroup 14.2 us, the three heads of a group 8.5; the same with 1900 tokens keeps the 128 rows.
+  int hw = NW, wide = 1;
   while (rep % hw) hw >>= 1;
+  while (wide < rep && wide < NW) wide <<= 1;
+  const int64_t avg = (a.num_tokens + a.batch - 1) / a.batch;
+  const auto count = [&](int w) { return (avg + 32 * (NW / w) - 1) / (32 * (NW / w)) * ((rep + w - 1) / w); };
+  if (count(wide) < count(hw)) hw = wide;
   const int rows = 32 * (NW / hw);
   a.n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
   constexpr size_t tiles = 2 * KT * (size_t)(D + E) * 2, epilogue = NW * 32 * (size_t)(E * 2 + 16), bytes = tiles > epilogue ? tiles : epilogue;
   static std::atomic<uint64_t> done{0};
   if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
-  const int64_t items = a.n_tiles * a.G * (rep / hw);
+  const int64_t items = a.n_tiles * a.G * ((rep + hw - 1) / hw);
   hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, SIG>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(64 * NW), bytes, s, a, hw);
   return 0;
 }

@@ -164,6 +164,30 @@ def test_largest_weight_of_every_32_keys_is_not_rounded(dtype, D):
     torch.testing.assert_close(out[large:].view(-1, H, D).double().cpu(), want.expand(-1, H, D), rtol=ulp, atol=256 * 2.0 ** -21)
 
 
+# (requests: the scalar search and the one by lanes, whole and part waves of them; heads: one, two or four of a group in a workgroup)
+@pytest.mark.parametrize("requests", [8, 9, 64, 65, 131])
+@pytest.mark.parametrize("H,G,D,E", [(7, 1, 64, 64), (6, 2, 128, 128), (3, 3, 64, 64), (14, 2, 64, 128), (11, 1, 128, 256)])
+def test_prompt_attention_of_many_requests(requests, H, G, D, E):
+    """Short uneven prompts, some without a row in the launch, some behind cached tokens."""
+    from semi_pd_amd import ops
+    lens = [(20, 1, 0, 33, 9)[i % 5] for i in range(requests)]
+    olds = [(0, 40, 3)[i % 3] if n else 5 for i, n in enumerate(lens)]
+    shared = E != D
+    t, g = _batch(lens, olds, H, G, D, E // G if shared else E, torch.bfloat16, requests + H)
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+    out = torch.full((sum(lens), H * E), 7.0, dtype=torch.bfloat16, device=DEV)
+    batch = (d["q"], out, d["k"], d["v"], d["table"], torch.arange(requests, device=DEV), torch.tensor(t["totals"], device=DEV), start.to(DEV),
+             n.to(DEV), max(lens), D ** -0.5)
+    if shared:
+        ops.shared_value_attention_fwd(*batch)
+    else:
+        ops.local_attention_fwd(*batch, 0.0, 0, None, None)
+    want = _dense(t, lens, olds, H, G, D, E, lambda p, j: j <= p, _softmax(), shared=shared)
+    assert float((out.cpu().double() - want).norm() / want.norm()) < 1.5 * 2.0 ** -8
+    torch.testing.assert_close(out.cpu().double(), want, rtol=6 * 2.0 ** -8, atol=12 * 2.0 ** -8)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("lens,olds", CASES)
 @pytest.mark.parametrize("H,G,D", [(16, 2, 128), (6, 2, 128), (8, 2, 64)])
