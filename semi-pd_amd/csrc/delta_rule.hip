@@ -699,11 +699,12 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
   }
   __syncthreads();
   // the operands in the order in which they are held
-  for (int i = tid; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
+  const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
+  for (int i = lays ? tid : 2 * L * NP; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
     const int half = i / (L * NP / 4), it = i % (L * NP / 4), tile = it >> 6, ln = it & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
     *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(kq_l + half * L * CS + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
   }
-  for (int i = tid; i < L * NP / 4; i += 256) {                  // K^T: tile (row of S, tokens)
+  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {                  // K^T: tile (row of S, tokens)
     const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
     const float* s = kq_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
     *reinterpret_cast<float4*>(frag + 2 * L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
@@ -732,7 +733,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
   const int hw = tid >> 5, ln = tid & 31;
   float* a_l = kq_l + hw * L * L;
   double* cum = cum_l + hw * L;
-  for (int hh = hw; hh < per; hh += 8) {
+  for (int hh = blockIdx.z * 8 + hw; hh < per; hh += 8 * gridDim.z) {
     const int h = g * per + hh;
     const T* pr = (const T*)a.p + (t0 + ln) * a.ld;
     const bool on = ln < cnt;
@@ -748,11 +749,11 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
     cum[ln] = c;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kDeltaHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c), dec = expf(la);
-    hp[1536 + ln] = eb;
+    const bool no = !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_moderate_decay(la);
+    hp[1536 + ln] = rec_flagged(eb, no);
     hp[1536 + L + ln] = wt;
     hp[1536 + 2 * L + ln] = dec;
     hp[1536 + 3 * L + ln] = beta;
-    bad |= !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_moderate_decay(la);
     __builtin_amdgcn_wave_barrier();
     // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s)
     const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);
@@ -788,7 +789,7 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
     __builtin_amdgcn_wave_barrier();
   }
   const int any_bad = __syncthreads_or(bad);
-  if (tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
+  if (lays && tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
 // The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
@@ -806,9 +807,9 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
   // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
   const int eblocks = (E + 63) / 64, members = per * eblocks;
-  const int turn = blockIdx.x / 8, unit = turn / members * 8 + blockIdx.x % 8;
-  if (unit >= (int)a.batch * G) return;
-  const int member = turn % members, b = unit / G, g = unit % G;
+  const RecPlace at = rec_place((int)a.batch * G, members);
+  if (at.unit < 0) return;
+  const int member = at.member, b = at.unit / G, g = at.unit % G;
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
@@ -961,7 +962,7 @@ __global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, i
         float z = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) z = fmaf(P[i / 4][i % 4], 0.f, z);      // (|q| = D^-1/2: its products stay below the largest of S)
-        serial = __any(flagged);
+        serial = __any(flagged || keep != keep);                 // (keep: see rec_flagged)
         if (__any(z != 0.f)) {                                   // (a column of S that is not finite stays so in either form)
           float c = 0.f;
 #pragma unroll
@@ -1140,9 +1141,9 @@ extern "C" int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t bat
 template <typename T, int NP>
 static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
-  hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G, rec_head_splits(chunks * a.G, a.H / a.G)), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
-  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);
+  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), dim3(rec_walk_blocks(a.batch * a.G, members)), dim3(256), 0, s, a, chunks);
 }
 
 // gate and norm; 16-byte accesses where a head is a power of two of pieces and everything starts on one

@@ -10,6 +10,31 @@ constexpr int kRecChunk = 32;            // tokens of a chunk
 constexpr int kRecTaps = 4;              // taps of the convolution at most
 constexpr int kRecHalo = kRecTaps - 1;   // rows in front of a chunk that its convolution looks at
 
+// The walks' workgroups: `units` of (request, group) with `members` each, which read the same operands.  A unit stays on one XCD (workgroup
+// ids go round the 8); fewer than 8 units have several each, or most of the chip would have none (128 heads of 128 x 64 in one group, 1
+// request of 12 rows, whole call: 66 -> 36 us; of 96 rows 99 -> 46).
+__host__ __device__ inline int rec_unit_xcds(int64_t units) { return units < 8 ? 8 / (int)units : 1; }
+inline unsigned rec_walk_blocks(int64_t units, int64_t members) {
+  const int x = rec_unit_xcds(units), at_once = 8 / x;
+  return (unsigned)((units + at_once - 1) / at_once * ((members + x - 1) / x) * 8);
+}
+struct RecPlace {
+  int unit, member;                      // (unit -1: none)
+};
+__device__ __forceinline__ RecPlace rec_place(int units, int members) {
+  const int x = rec_unit_xcds(units), turns = (members + x - 1) / x, turn = blockIdx.x / 8, xcd = blockIdx.x % 8;
+  const int unit = turn / turns * (8 / x) + xcd / x, member = turn % turns * x + xcd % x;
+  return unit < units && xcd / x < 8 / x && member < members ? RecPlace{unit, member} : RecPlace{-1, 0};
+}
+
+// Workgroups that share out the heads of a (chunk, group), eight each, as long as the chip is not full of them: `items` (chunk, group)s.
+// 128 heads of 128 x 64 in one group, 1 request of 12 rows, whole call: one workgroup for all heads 106 us, 16 of them 66 (token by
+// token 48).
+inline unsigned rec_head_splits(int64_t items, int heads) {
+  const int64_t most = (heads + 7) / 8, room = items < 512 ? 512 / items : 1;
+  return (unsigned)(most < room ? most : room);
+}
+
 inline int64_t rec_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kRecChunk + batch; }
 
 // Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.
@@ -73,6 +98,14 @@ __device__ __forceinline__ float rec_silu(float x) {
 }
 // ... where x stands for its silu because it is not moderate: x itself or 0, of minus infinity not a number
 __device__ __forceinline__ float rec_silu_if_large(float x) { return rec_moderate(x) ? x : (x > 0.f ? x : x * 0.f); }
+
+// The weight e^(b_t) of a head's chunk, by the half wave that has its 32 tokens: the last one is not a number where `no` holds for any
+// of them, and the chunk is taken token by token by that.
+__device__ __forceinline__ float rec_flagged(float eb, bool no) {
+  const uint64_t all = __ballot(no);
+  const bool any = (threadIdx.x & 32 ? all >> 32 : all & 0xffffffffull) != 0;
+  return any && (threadIdx.x & 31) == 31 ? __builtin_nanf("") : eb;
+}
 
 // 2^x of a 64-bit exponent: what rounding it to 32 bits takes away is multiplied in
 __device__ __forceinline__ float rec_exp2(double x) {

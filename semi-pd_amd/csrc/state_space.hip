@@ -392,11 +392,12 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     }
   }
   __syncthreads();
-  for (int i = tid; i < L * NP / 4; i += 256) {                  // C: tile (tokens, rows of S)
+  const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
+  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {  // C: tile (tokens, rows of S)
     const int tile = i >> 6, ln = i & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
     *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(c_l + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
   }
-  for (int i = tid; i < L * NP / 4; i += 256) {                  // B^T: tile (rows of S, tokens)
+  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {  // B^T: tile (rows of S, tokens)
     const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
     const float* s = b_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
     *reinterpret_cast<float4*>(frag + L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
@@ -418,7 +419,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
   __syncthreads();
   const int hw = tid >> 5, t = tid & 31;
   double* cum = cum_l + hw * L;
-  for (int hh = hw; hh < per; hh += 8) {
+  for (int hh = blockIdx.z * 8 + hw; hh < per; hh += 8 * gridDim.z) {
     const int h = g * per + hh;
     const float dt = t < cnt ? ssm_softplus(Elem<T>::to_f(((const T*)a.p)[(t0 + t) * a.ld + a.dt_off + h]) + a.dt_bias[h]) : 0.f;
     const float la = t < cnt ? -expf(a.a_log[h]) * dt : 0.f;
@@ -432,11 +433,11 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     cum[t] = c;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c) * dt, dec = expf(la);
-    hp[768 + t] = eb;
+    const bool no = !rec_finite(dt) || !rec_moderate_decay(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
+    hp[768 + t] = rec_flagged(eb, no);
     hp[768 + L + t] = wt;
     hp[768 + 2 * L + t] = dt;
     hp[768 + 3 * L + t] = dec;
-    bad |= !rec_finite(dt) || !rec_moderate_decay(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
     __builtin_amdgcn_wave_barrier();
     // the weighted C B^T, 16 bytes a lane: piece i of 192 is lane i % 64 of tile i / 64; the step size of column s from lane s
 #pragma unroll
@@ -454,7 +455,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     __builtin_amdgcn_wave_barrier();
   }
   const int any_bad = __syncthreads_or(bad);
-  if (tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
+  if (lays && tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
 // The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
@@ -473,9 +474,9 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
   // workgroups of one (request, group) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, per = H / G;
   const int eblocks = (E + 63) / 64, members = per * eblocks;
-  const int turn = blockIdx.x / 8, unit = turn / members * 8 + blockIdx.x % 8;
-  if (unit >= (int)a.batch * G) return;
-  const int member = turn % members, b = unit / G, g = unit % G;
+  const RecPlace at = rec_place((int)a.batch * G, members);
+  if (at.unit < 0) return;
+  const int member = at.member, b = at.unit / G, g = at.unit % G;
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
@@ -614,7 +615,7 @@ __global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64
         float z = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; ++i) z = fmaf(O[i / 4][i % 4], 0.f, z);
-        serial = __any(flagged);
+        serial = __any(flagged || keep != keep);                 // (keep: see rec_flagged)
         if (__any(z != 0.f)) {                                   // (a column of S that is not finite stays so in either form)
           float c = 0.f;
 #pragma unroll
@@ -934,9 +935,9 @@ extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t ba
 template <typename T, int NP>
 static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
   const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
-  hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G), dim3(256), 0, s, a);
+  hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G, rec_head_splits(chunks * a.G, a.H / a.G)), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
-  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3((unsigned)((a.batch * a.G + 7) / 8 * 8 * members)), dim3(256), 0, s, a, chunks);
+  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3(rec_walk_blocks(a.batch * a.G, members)), dim3(256), 0, s, a, chunks);
 }
 
 static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,

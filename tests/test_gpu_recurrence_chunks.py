@@ -423,3 +423,24 @@ def test_many_requests_in_chunks(kind):
         torch.testing.assert_close(outs[b].to(F64), want, rtol=2e-5, atol=2e-5)
         torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
         torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("kind", ["state_space", "delta_rule"])
+def test_many_heads_of_a_group_in_chunks(kind):
+    """Three workgroups with eight heads of a group each, one of them for four; an infinite gate of the thirteenth head stays its own."""
+    H, G, N, E, lens, at = 20, 1, 32, 16, [100, 100], 90
+    state_space = kind == "state_space"
+    inputs, run, truth, extra = ((_ssm_inputs, _ssm_run, _ssm_truth, (H,)) if state_space else (_delta_inputs, _delta_run, _delta_truth, ()))
+    w, rows, state, before = inputs(H, G, N, E, 1, lens, torch.float32, 6)
+    clean, after, _ = run(w, rows, state, before, [9, 9], H, G, N, E, *extra)
+    for b in range(2):
+        want, S, _ = truth(w, rows[b], state[b], before[b], H, G, N, E, *extra)
+        torch.testing.assert_close(clean[b].to(F64), want, rtol=2e-5, atol=2e-5)
+        torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
+    rows[0][at, (2 * H * E + 2 * G * N if state_space else 2 * G * N + 2 * H * E) + 12] = float("nan")
+    got, _, _ = run(w, rows, state, before, [9, 9], H, G, N, E, *extra)
+    others = [h for h in range(H) if h != 12]
+    torch.testing.assert_close(got[1], clean[1], rtol=0, atol=0)
+    torch.testing.assert_close(got[0].view(-1, H, E)[:, others], clean[0].view(-1, H, E)[:, others], rtol=0, atol=0)
+    torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
+    assert not bool(torch.isfinite(got[0].view(-1, H, E)[at:, 12]).any())
