@@ -798,8 +798,8 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
 // without moving; v is convolved in its place by the lane that needs it, from raw inputs in the wave's own LDS.  Left-hand operands
 // come straight into registers in the order they are used, not through LDS, the next chunk's into the registers that this chunk has
 // just read.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.
-template <typename T, int NP>
-__global__ void __launch_bounds__(256, 1) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
+template <typename T, int NP, int W>
+__global__ void __launch_bounds__(256, W) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
   constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
   __shared__ __attribute__((aligned(16))) T in_l[4][RowTile<T>::kElems];       // a wave's own: raw inputs of its convolution
   __shared__ __attribute__((aligned(16))) float o_l[4][L * kOutStride];         // ... results on their way out (token by token: its v)
@@ -1127,14 +1127,22 @@ extern "C" int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, 
 }
 
 // The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
-// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call, 32 heads of
-// 128 x 128: 1 request of 2 rows 51 / 43 us, 64 rows 96 / 54, 256 rows 251 / 92; 4 requests of 2 rows 53 / 44; 32 requests of 8 rows
-// 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; heads of 64 x 64: 4 requests of 2 rows 49 / 37, 32 requests of 8 rows 60 / 78, 16 rows
-// 82 / 83, 64 rows 200 / 134.  A few requests take chunks whatever their length.
-constexpr int64_t kDeltaChunkMinRows = 16, kDeltaChunkFewRequests = 4;
+// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  A chunk costs the same however few its
+// rows and heads; token by token a token's heads are prepared one behind another, so that form is ahead where there are few.
+// Token by token against chunks, whole call, 32 heads over 8 of 128 x 128: 1 request of 2 rows 51 / 43 us, 64 rows 96 / 54, 256 rows 251 / 92;
+// 4 requests of 2 rows 53 / 44; 32 requests of 8 rows 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; 32 heads of 64 x 64: 4 requests of
+// 2 rows 53 / 36, 32 requests of 20 rows 97 / 81.  8 heads over 1 of 128 x 128: 1 request of 2 rows 27 / 43, 24 rows 44 / 47, 32 rows 49 / 46;
+// 16 over 4 of 64 x 128: 16 requests of 20 rows 49 / 57, 32 rows 60 / 65, 48 rows 74 / 67; 8 over 1 of 64 x 64: 1 request of 32 rows 34 / 39,
+// 48 rows 41 / 42, 64 rows 47 / 43.
+static int64_t delta_chunk_min_rows(int64_t batch, int num_heads, int num_k_heads, int k_dim) {
+  const int heads = num_heads + 2 * num_k_heads;
+  if (heads >= 32) return batch <= 4 ? 0 : 16;
+  return k_dim > 64 ? 24 : heads >= 16 ? 32 : 48;
+}
 
 extern "C" int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps) {
-  if (batch <= 0 || num_heads <= 0 || num_k_heads <= 0 || (batch > kDeltaChunkFewRequests && num_tokens < kDeltaChunkMinRows * batch) || k_dim > 128 || taps > kRecTaps) return 0;
+  if (batch <= 0 || num_heads <= 0 || num_k_heads <= 0 || k_dim > 128 || taps > kRecTaps) return 0;
+  if (num_tokens < delta_chunk_min_rows(batch, num_heads, num_k_heads, k_dim) * batch) return 0;
   return rec_max_chunks(num_tokens, batch) * (num_k_heads * delta_frag_elems(k_dim <= 64 ? 64 : 128) + (int64_t)num_heads * kDeltaHead);
 }
 
@@ -1143,7 +1151,15 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
   hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G, rec_head_splits(chunks * a.G, a.H / a.G)), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
-  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), dim3(rec_walk_blocks(a.batch * a.G, members)), dim3(256), 0, s, a, chunks);
+  const dim3 grid(rec_walk_blocks(a.batch * a.G, members));
+  if constexpr (NP <= 64)                                        // (NP 128: twice the operands, no second workgroup a CU)
+    if (a.batch * a.G * members > 256) {
+      // more workgroups than CUs: two a CU, at the price of 40 spilled registers (32 heads of 64 x 64, one / two a CU, whole call: 64 requests
+      // of 64 rows 226 / 202 us; 4 requests of 96 rows, 128 workgroups: 52 / 58)
+      hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 2>), grid, dim3(256), 0, s, a, chunks);
+      return;
+    }
+  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 1>), grid, dim3(256), 0, s, a, chunks);
 }
 
 // gate and norm; 16-byte accesses where a head is a power of two of pieces and everything starts on one

@@ -923,12 +923,13 @@ extern "C" int64_t semipd_state_space_work_width(int num_heads, int groups, int 
 // The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
 // is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call, 128 heads of 128 x 64: 1 request of 8 rows 34.0 / 36.1 us, 12 rows 37.3 / 36.4, 32 rows 56 / 40,
 // 256 rows 327 / 79; 32 requests of 8 rows 185 / 148, 32 rows 548 / 191, 256 rows 3058 / 782; 64 heads: 1 request of 12 rows 34.3 / 33.8,
-// 32 requests of 8 rows 110 / 88.
+// 32 requests of 8 rows 110 / 88.  A state of 16 rows is padded to 64: 256 heads of 16 x 64, 1 request of 12 rows 54 / 59, 32 rows 65 / 62, 8
+// requests of 16 rows 90 / 107, 16 requests of 24 rows 204 / 175.
 constexpr int64_t kSsmChunkMinRows = 12;
 static int ssm_padded_state(int state_size) { return state_size <= 64 ? 64 : 128; }
 
 extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state_size, int taps) {
-  if (batch <= 0 || groups <= 0 || num_tokens < kSsmChunkMinRows * batch || state_size > 128 || taps > kRecTaps) return 0;
+  if (batch <= 0 || groups <= 0 || num_tokens < (state_size <= 16 ? 24 : kSsmChunkMinRows) * batch || state_size > 128 || taps > kRecTaps) return 0;
   return rec_max_chunks(num_tokens, batch) * (groups * ssm_frag_elems(ssm_padded_state(state_size)) + (int64_t)num_heads * kSsmHead);
 }
 

@@ -256,7 +256,7 @@ def _delta_run(w, rows, state, before, first, H, G, D, E, eps=1e-5, decode=False
 
 # (rows of S in, at and below a padded block; columns over part of a wave, one and two workgroups, odd; more heads than half waves)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H,G,D,E,taps,lens", [(4, 2, 128, 128, 4, [64, 1, 130]), (6, 2, 40, 40, 2, [63, 65]), (3, 1, 7, 72, 1, [31, 33]),
+@pytest.mark.parametrize("H,G,D,E,taps,lens", [(4, 2, 128, 128, 4, [64, 1, 130]), (6, 2, 40, 40, 2, [63, 65]), (3, 1, 7, 72, 1, [31, 33]), (3, 1, 7, 72, 1, [63, 97]),
                                                (2, 2, 65, 7, 3, [16, 200]), (9, 1, 64, 16, 4, [32, 70])])
 def test_delta_rule_in_chunks(dtype, H, G, D, E, taps, lens):
     """Fresh sequences and portions (every second request) in one launch; tolerances as above."""
@@ -407,7 +407,7 @@ def test_room_for_the_chunks(kind, scarce, monkeypatch):
 def test_many_requests_in_chunks(kind):
     """More than one wave's lanes of requests (131, then a part of another 64), uneven, some without a row in the launch: a request's
     chunks are found by counting the ones in front of it, 64 requests at a time."""
-    lens = [(40, 1, 0, 33, 17)[i % 5] for i in range(131)]
+    lens = [((40, 1, 0, 33, 17) if kind == "state_space" else (190, 1, 0, 65, 33))[i % 5] for i in range(131)]       # (enough rows for chunks)
     first = [37 if n == 0 or i % 2 else 0 for i, n in enumerate(lens)]
     H, G, N, E = 2, 1, 8, 16
     inputs, run, truth, extra = ((_ssm_inputs, _ssm_run, _ssm_truth, (1,)) if kind == "state_space" else
