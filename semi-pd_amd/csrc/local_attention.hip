@@ -1872,7 +1872,13 @@ extern "C" int semipd_talk_mix(const void* parts, int64_t parts_ld, const float*
                        out_ld >= (int64_t)num_q_heads * v_dim,
                    SEMIPD_EINVAL, "talk_mix: null pointer or rows too short");
   const size_t held = (size_t)num_q_heads * ((size_t)num_kv_heads * v_dim * 2 + 16) + (size_t)num_q_heads * v_dim * 2;
-  if ((dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
+  const size_t staged = ((size_t)num_q_heads * num_q_heads + (size_t)num_q_heads * num_kv_heads * v_dim) * sizeof(float);
+  // A tile is 16 heads of one key/value head by 16 elements: the matrix cores where enough of its rows are heads and every wave has a tile,
+  // and where the vector form could not stage its operands (32 rows, vector / matrix, us: heads over key/value heads of elements 12 / 2
+  // of 128 5.8 / 5.1, 16 / 2 of 64 4.6 / 4.3, 16 / 4 of 128 6.7 / 7.2, 8 / 2 of 128 4.1 / 5.0, 16 / 8 of 64 5.2 / 8.3, 8 / 1 of 32 3.2 / 3.6, 32 / 4
+  // of 32 5.8 / 5.9; not staged: 32 / 4 of 128 44 / 8.2, 48 / 8 of 64 57 / 14)
+  const bool tiles = (num_q_heads >= 6 * num_kv_heads && v_dim >= 64) || staged > 65536;
+  if (tiles && (dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
       aligned16(out) && held <= 65536 && num_q_heads <= 64) {
     SEMIPD_DISPATCH_HALF(dtype, T, {
       if (num_q_heads <= 32)
@@ -1884,7 +1890,6 @@ extern "C" int semipd_talk_mix(const void* parts, int64_t parts_ld, const float*
     });
     return launch_status("talk_mix");
   }
-  const size_t staged = ((size_t)num_q_heads * num_q_heads + (size_t)num_q_heads * num_kv_heads * v_dim) * sizeof(float);
   SEMIPD_DISPATCH_DTYPE(dtype, T, {
     if (staged <= 65536)
       hipLaunchKernelGGL((talk_mix_kernel<T, true>), dim3((unsigned)num_tokens), dim3(256), staged, as_stream(stream),

@@ -207,7 +207,8 @@ def test_prompt_attention_over_shared_values(dtype, lens, olds, H, G, D):
 
 # heads over one and two tiles of 16 a key/value head, sums over one to four steps of 16, neither whole
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("H,G,E", [(32, 2, 128), (24, 2, 64), (40, 4, 16), (33, 1, 32), (64, 2, 16), (6, 3, 48)])
+@pytest.mark.parametrize("H,G,E", [(32, 2, 128), (24, 2, 64), (40, 4, 16), (33, 1, 32), (64, 2, 16), (6, 3, 48), (40, 4, 64), (33, 1, 80), (64, 2, 64),
+                                   (48, 8, 64), (16, 4, 64), (15, 3, 64)])
 def test_talk_mix(dtype, H, G, E):
     """fp32 products and sums of at most 64 terms, the result rounded once.  With p significant bits half a unit in the last place of x is
     at most 2^-p |x| (just above a power of two): 2^-8 for bf16, 2^-11 for fp16; the sum: 64 roundings of 2^-24 of its terms."""
