@@ -451,9 +451,9 @@ __global__ void __launch_bounds__(1024) delta_decode_kernel(DeltaArgs a) {
   }
 }
 
-// The same with S in 16-byte pieces and in ONE launch: a workgroup per (key head, request) with a team of four waves per value head (in
-// turn, where there are more heads than teams: a piece of the next one is fetched as one of this is stored), so the convolution's
-// channels belong to one workgroup, which moves their inputs on itself.  A thread of a team has four columns and every 1024 / E-th row
+// The same with S in 16-byte pieces: a workgroup per (key head, request) with a team of four waves per value head (in turn, where there
+// are more heads than teams: a piece of the next one is fetched as one of this is stored), so the convolution's channels belong to
+// one workgroup, which moves their inputs on itself: ONE launch.  (gridDim.z > 1: the heads of a key head over several.)  A thread of a team has four columns and every 1024 / E-th row
 // of S, all of its pieces in flight from the start; the two dot products are summed over lanes and the team's waves.  Bound by HBM, the
 // state read and written once: 32 requests, 32 heads of 128 x 128 (134 MB): a column of S by four lanes of four bytes each 57.7 -> 32.3
 // us; 3 requests, 32 heads of 64 x 64: 10.6 (two launches) -> 9.8.
@@ -478,10 +478,11 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
     return !fresh && hh < per && n < D ? *reinterpret_cast<const float4*>(a.state + slot * a.state_ld + ((int64_t)(g * per + hh) * D + n) * E + e) : float4{0.f, 0.f, 0.f, 0.f};
   };
 #pragma unroll
-  for (int i = 0; i < NIT; ++i) S[i] = piece(team, n0 + i * rows);
+  for (int i = 0; i < NIT; ++i) S[i] = piece((int)blockIdx.z * teams + team, n0 + i * rows);
   float* cs = a.conv_state + slot * a.conv_ld;
   for (int i = tid; i < 2 * D + per * E; i += blockDim.x) {
     const bool is_v = i >= 2 * D;
+    if (is_v && gridDim.z > 1 && ((i - 2 * D) / E / teams) % gridDim.z != blockIdx.z) continue;                                  // (a head of another workgroup)
     const int d = is_v ? g * per * E + i - 2 * D : g * D + (i < D ? i : i - D);                              // channel within q, k or v
     const int ch = is_v ? 2 * G * D + d : (i < D ? d : G * D + d);                                           // its place in the state
     const T* cw = (const T*)(is_v ? a.conv_v : (i < D ? a.conv_q : a.conv_k)) + (int64_t)d * taps;
@@ -493,9 +494,10 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
       const float x = fresh ? 0.f : cs[(int64_t)s * C + ch];
       if (!fresh) y += Elem<T>::to_f(cw[s]) * x;
     }
+    lds[i] = silu_f(y);
+    if (gridDim.z > 1) continue;                                  // (several read the old inputs of q and k: they move on in a launch of their own)
     for (int s = 1; s < taps - 1; ++s) cs[(int64_t)(s - 1) * C + ch] = fresh ? 0.f : cs[(int64_t)s * C + ch];
     if (taps > 1) cs[(int64_t)(taps - 2) * C + ch] = cur;
-    lds[i] = silu_f(y);
   }
   __syncthreads();
   if (tid < 64) {
@@ -517,7 +519,7 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
   }
   __syncthreads();
   const float ik = sc[0], iq = sc[1], kq = sc[2];
-  for (int h0 = 0; h0 < per; h0 += teams) {                         // (every team goes round as often: there are barriers inside)
+  for (int h0 = blockIdx.z * teams; h0 < per; h0 += teams * gridDim.z) {       // (every team goes round as often: there are barriers inside)
     const int hh = h0 + team, h = g * per + (hh < per ? hh : per - 1);
     const bool on = hh < per;
     float4 dk = {0.f, 0.f, 0.f, 0.f}, dq = {0.f, 0.f, 0.f, 0.f};
@@ -560,7 +562,7 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
           const float kv = k_l[n] * ik;
           *reinterpret_cast<float4*>(st + n * E + e) = float4{gt * S[i].x + kv * u[0], gt * S[i].y + kv * u[1], gt * S[i].z + kv * u[2], gt * S[i].w + kv * u[3]};
         }
-        S[i] = piece(hh + teams, n);                                 // (the team's next head)
+        S[i] = piece(hh + teams * (int)gridDim.z, n);                // (the team's next head)
       }
     }
     for (int o = 1; o < quads; o <<= 1) sq_o += __shfl_xor(sq_o, o, 64);       // (a row of S is `quads` neighbouring lanes, all columns)
@@ -1225,16 +1227,27 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
   // the chip takes all workgroups at once, two where a CU goes through several, so that one loads while another computes (32 heads
   // of 64 x 64, 8 key heads, four teams / two, us: 3 requests 9.8 / 12.1, 32 13.2 / 15.3, 48 22.9 / 18.3, 128 47.7 / 37.7)
   const int per_group = num_heads / num_k_heads, most = k_dim * v_dim > 4 * 1024 || batch * num_k_heads > 256 ? 2 : 4, teams = per_group < most ? per_group : most;
+  // A key head with more value heads than teams goes round (shared out over several workgroups as long as the CUs have none, 256 in
+  // all; the convolutions' inputs then move on in a second launch).  The kernel below is ahead where these rounds are short (k_dim up to
+  // 64: from 128 workgroups on they are as long as its own; up to 1024 elements of state a head a team has idle threads).  Below / here,
+  // shared out / in turn, us: 32 heads over 1 of 128 x 128, 1 request 17.8 / 16.7 / 107, 32 requests 57 / 36 / 121; 8 over 1 of 64 x 64,
+  // 1 request 10.3 / 11.8 / 14.0, 128 requests 17.4 / 16.5 / 18.1; 64 over 2 of 32 x 32, 32 requests 12.8 / - / 43.
+  const int rounds = (per_group + teams - 1) / teams;
+  const bool step_pays = rounds == 1 || ((k_dim > 64 || batch * num_k_heads >= 128) && (k_dim * v_dim > 1024 || rounds <= 2));
   const size_t step_lds = ((size_t)2 * k_dim + (size_t)per_group * v_dim + (size_t)teams * 8 * v_dim + 4) * sizeof(float);
   if (q_start == nullptr && batch <= 65535 && v_dim >= 16 && v_dim <= 256 && (v_dim & (v_dim - 1)) == 0 && k_dim % 2 == 0 && k_dim * v_dim <= 16 * 1024 &&
-      aligned16(state) && state_ld % 4 == 0 && step_lds <= 65536) {
+      aligned16(state) && state_ld % 4 == 0 && step_lds <= 65536 && step_pays) {
     const int nit = (k_dim * v_dim + 1023) / 1024;
-    const dim3 sgrid((unsigned)num_k_heads, (unsigned)batch);
+    const int64_t room = 256 / (batch * num_k_heads), splits = rounds < room ? rounds : (room < 1 ? 1 : room);
+    const dim3 sgrid((unsigned)num_k_heads, (unsigned)batch, (unsigned)splits);
     SEMIPD_DISPATCH_DTYPE(dtype, T, {
       if (nit <= 4) hipLaunchKernelGGL((delta_step_kernel<T, 4>), sgrid, dim3(256 * teams), step_lds, st, a);
       else if (nit <= 8) hipLaunchKernelGGL((delta_step_kernel<T, 8>), sgrid, dim3(256 * teams), step_lds, st, a);
       else hipLaunchKernelGGL((delta_step_kernel<T, 16>), sgrid, dim3(256 * teams), step_lds, st, a);
     });
+    if (splits > 1 && taps > 1)
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch),
+                                                         dim3(256), 0, st, a));
     return launch_status("delta_rule(step)");
   }
   if (q_start == nullptr && (int64_t)ds * v_dim <= 1024) {

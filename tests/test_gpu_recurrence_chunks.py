@@ -347,9 +347,12 @@ def test_delta_rule_in_chunks_large_state():
     torch.testing.assert_close(after[0].to(F64), S, rtol=1e-5, atol=1e-5)
 
 
-# (a team per head: one, several in one workgroup, more heads than teams; one, some and all rows of pieces)
+# (a team per head: one, several in one workgroup, more heads than teams, shared out over workgroups wholly, in part and not at all; one, some
+# and all rows of pieces)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,G,D,E,taps", [(8, 2, 128, 128, 4), (3, 3, 64, 64, 2), (12, 2, 20, 16, 3), (7, 1, 64, 256, 1), (4, 2, 100, 32, 5)])
+@pytest.mark.parametrize("H,G,D,E,taps", [(8, 2, 128, 128, 4), (3, 3, 64, 64, 2), (12, 2, 20, 16, 3), (7, 1, 64, 256, 1), (4, 2, 100, 32, 5),
+                                            (384, 64, 20, 16, 2), (360, 30, 100, 32, 3), (33, 1, 32, 32, 4), (7, 7, 64, 256, 1),
+                                            (3, 1, 66, 128, 4)])
 def test_delta_rule_decode_step(dtype, H, G, D, E, taps):
     w, rows, state, before = _delta_inputs(H, G, D, E, taps, [1, 1, 1], dtype, 3)
     first = [5, 0, 900]
