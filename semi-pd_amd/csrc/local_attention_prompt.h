@@ -18,7 +18,7 @@
 // cycles each) with five instructions around each.  Of the SIMD cycles of the batch below the vector unit is busy for 42 %, the matrix
 // pipe for 20 %, the LDS for about a third of its own; two waves a SIMD fill only part of each other's gaps (value rows of 256: 30, 19
 // and a third).  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves of
-// one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 110 us (500 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
+// one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 109 us (505 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
 // 341 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.
 // A fresh prompt of at most 32 tokens is one step of either, and its 32 x 64 products are four times those of the wave of 16 rows: 20
 // tokens 7.3 -> 7.4 us, 32 tokens 7.4 -> 7.9, with sigmoid weights 6.5 -> 7.1 and 6.6 -> 7.6 (behind 100 tokens 20 tokens are 12.4 -> 9.6;
