@@ -843,7 +843,7 @@ __global__ void __launch_bounds__(256, W) delta_chunk_walk_kernel(DeltaArgs a, i
   float* yo = a.work + t0 * a.wld + h * E + e0;
   // 16-byte pieces of the projection's and of the result's rows: everything starts on one
   const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
-                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0 && a.ld < (1 << 24);
 
   // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
   RowTile<T> tile;

@@ -27,6 +27,21 @@ __device__ __forceinline__ RecPlace rec_place(int units, int members) {
   return unit < units && xcd / x < 8 / x && member < members ? RecPlace{unit, member} : RecPlace{-1, 0};
 }
 
+// Request at place `pos` of a launch: the longest first, so that none starts late; those behind the first `firsts` (which have a
+// CU each) from the shortest up, so that the ones that come to a long one's CU are short.  4 requests of 1330, 2034, 1599 and 2303 rows, two
+// workgroups a CU: in their order the second and the fourth share CUs (walk 412 us, so placed 345).  A whole wave asks.
+__device__ __forceinline__ int rec_by_length(const int32_t* q_len, int batch, int pos, int firsts) {
+  if (batch > 64) return pos;
+  const int lane = threadIdx.x & 63, n = lane < batch ? q_len[lane] : 0;
+  int rank = 0;
+  for (int j = 0; j < batch; ++j) {
+    const int m = __builtin_amdgcn_readlane(n, j);
+    rank += m > n || (m == n && j < lane) ? 1 : 0;
+  }
+  const int want = pos < firsts ? pos : batch - 1 - (pos - firsts);
+  return __builtin_ctzll(__ballot(lane < batch && rank == want));
+}
+
 // Workgroups that share out the heads of a (chunk, group), eight each, as long as the chip is not full of them: `items` (chunk, group)s.
 // 128 heads of 128 x 64 in one group, 1 request of 12 rows, whole call: one workgroup for all heads 106 us, 16 of them 66 (token by
 // token 48).
@@ -114,48 +129,121 @@ __device__ __forceinline__ float rec_exp2(double x) {
   return hi < -126.f ? e : fmaf(e, lo * 0.693147182f, e);
 }
 
+// ---- fp32 products on the bf16 matrix cores
+// x as the sum of three bf16 values, each the rounding of what those in front of it leave: 8 + 8 + 8 bits and the signs hold all 24 of x
+// (down to 2^-110, where the last piece leaves the format; what is off by 2^-134 there is below anything that is added up).
+// Eight of a lane's elements make an operand of v_mfma_f32_16x16x32_bf16: lane (r16, kq) has k = 4 kq .. + 3 and 16 + 4 kq .. + 3 of a step
+// of 32, both operands alike: two accumulator tiles of 16 rows are such an operand as they stand.
+struct Split3 {
+  Frag16 p[3];
+};
+__device__ __forceinline__ void rec_split2(float a, float b, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  hi = pack2<bf16_t>(a, b);
+  const float a1 = a - __uint_as_float(hi << 16), b1 = b - __uint_as_float(hi & 0xffff0000u);
+  mid = pack2<bf16_t>(a1, b1);
+  lo = pack2<bf16_t>(a1 - __uint_as_float(mid << 16), b1 - __uint_as_float(mid & 0xffff0000u));
+}
+__device__ __forceinline__ Split3 rec_split8(const f32x4& a, const f32x4& b) {
+  Split3 s;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    rec_split2(a[2 * i], a[2 * i + 1], s.p[0].w[i], s.p[1].w[i], s.p[2].w[i]);
+    rec_split2(b[2 * i], b[2 * i + 1], s.p[0].w[2 + i], s.p[1].w[2 + i], s.p[2].w[2 + i]);
+  }
+  return s;
+}
+// The same of values that may be anything: an infinity or a NaN stands in the first piece alone, and one that would round to an infinity
+// does not, so that the three add up to what they were made of.
+__device__ __forceinline__ Split3 rec_split8_any(const f32x4& a, const f32x4& b) {
+  Split3 s = rec_split8(a, b);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float x = i < 4 ? a[i] : b[i - 4];
+    if (fabsf(x) <= 0x1p126f) continue;
+    float x0 = x != x ? x : __uint_as_float(__float_as_uint(x) & 0xffff0000u), x1 = 0.f, x2 = 0.f;
+    if (rec_finite(x)) {
+      x1 = __uint_as_float(__float_as_uint(x - x0) & 0xffff0000u);
+      x2 = (x - x0) - x1;
+    }
+    s.p[0].e[i] = (uint16_t)(__float_as_uint(x0) >> 16 | (x != x ? 0x40 : 0));
+    s.p[1].e[i] = (uint16_t)(__float_as_uint(x1) >> 16);
+    s.p[2].e[i] = (uint16_t)(__float_as_uint(x2) >> 16);
+  }
+  return s;
+}
+// A B of the pieces without the three products below 2^-25 of the whole (mid lo, lo mid, lo lo): `big` takes the products of the first
+// pieces, `small` the other five.  On the 16 x 16 x 4 products of fp32 operands the same takes 8 x 32 cycles, here 6 x 16.
+// N row tiles side by side: a product that adds to what the one in front of it wrote waits for it.
+template <int N>
+__device__ __forceinline__ void rec_mma(const Frag16 (&a)[N][3], const Split3& b, f32x4* big, f32x4* small) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) small[i] = mma16<bf16_t>(a[i][2], b.p[0], small[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) big[i] = mma16<bf16_t>(a[i][0], b.p[0], big[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) small[i] = mma16<bf16_t>(a[i][0], b.p[2], small[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) small[i] = mma16<bf16_t>(a[i][1], b.p[1], small[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) small[i] = mma16<bf16_t>(a[i][1], b.p[0], small[i]);
+#pragma unroll
+  for (int i = 0; i < N; ++i) small[i] = mma16<bf16_t>(a[i][0], b.p[1], small[i]);
+}
+// ... the value that the pieces `plane` halves apart stand for
+__device__ __forceinline__ float rec_joined(const uint16_t* p, int plane) {
+  return (__uint_as_float((uint32_t)p[0] << 16) + __uint_as_float((uint32_t)p[plane] << 16)) + __uint_as_float((uint32_t)p[2 * plane] << 16);
+}
+
 // Rows of 16 columns that one wave needs (its convolution's inputs: a chunk and the rows in front of it), 16 bytes a lane: a load
 // per token, element and lane would be 14 requests of 2 bytes for the two or three here.  `fetch` leaves them in registers,
 // `place` puts them into the wave's own LDS (48 / 80 bytes a row: rows that are read together start in different banks).
-template <typename T> struct RowTile {
+template <typename T, int TOKENS = kRecChunk> struct RowTile {
   static constexpr int kPerRow = 16 * (int)sizeof(T) / 16;          // 16-byte pieces a row
-  static constexpr int kRows = kRecChunk + kRecHalo;
+  static constexpr int kRows = TOKENS + kRecHalo;
   static constexpr int kLoads = (kRows * kPerRow + 63) / 64;
   static constexpr int kStride = sizeof(T) == 2 ? 24 : 20;          // elements of T between rows in LDS
   static constexpr int kElems = kRows * kStride;
-  uint4 v[kLoads];
-  // rows l0 - halo .. l0 + 31 of `p` (row 0 = the portion's first), zeros behind row n - 1; l0 > 0
+  u32x4 v[kLoads];
+  // rows l0 - halo .. l0 + TOKENS - 1 of `p` (row 0 = the portion's first), row n - 1 in place of those behind it; l0 > 0, rows
+  // of less than 2^26 bytes
   __device__ __forceinline__ void fetch(const T* p, int64_t ld, int l0, int n, int lane) {
+    const int row0 = min(l0 - kRecHalo, n - 1), last = min(kRows, n - row0) - 1;       // (0 <= row0 <= row0 + last < n, also for l0 behind the portion)
+    const char* first = reinterpret_cast<const char*>(p + (int64_t)row0 * ld);
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
-      const int it = u * 64 + lane, row = it / kPerRow, l = l0 - kRecHalo + row;
-      v[u] = uint4{0u, 0u, 0u, 0u};
-      if (row < kRows && l < n) v[u] = *reinterpret_cast<const uint4*>(p + (int64_t)l * ld + it % kPerRow * (16 / (int)sizeof(T)));
+      const int it = u * 64 + lane;
+      v[u] = *reinterpret_cast<const u32x4*>(first + ((uint32_t)min(it / kPerRow, last) * (uint32_t)(ld * sizeof(T)) + (uint32_t)(it % kPerRow) * 16u));
     }
   }
   __device__ __forceinline__ void place(T* lds, int lane) const {
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
       const int it = u * 64 + lane, row = it / kPerRow;
-      if (row < kRows) *reinterpret_cast<uint4*>(lds + row * kStride + it % kPerRow * (16 / (int)sizeof(T))) = v[u];
+      if (row < kRows) *reinterpret_cast<u32x4*>(lds + row * kStride + it % kPerRow * (16 / (int)sizeof(T))) = v[u];
     }
   }
 };
 
 // A wave's 32 x 16 results (lane (r16, kq): rows 16 i + 4 kq + r of column r16) to rows in memory, 16 bytes a lane by way of its LDS
 constexpr int kOutStride = 20;            // floats between rows in LDS
-__device__ __forceinline__ void rec_store_tile(const f32x4 (&o)[2], float* lds, float* y, int64_t ld, int lane) {
+__device__ __forceinline__ void rec_place_tile(const f32x4 (&o)[2], float* lds, int lane) {
   const int r16 = lane & 15, kq = lane >> 4;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) lds[(16 * i + 4 * kq + r) * kOutStride + r16] = o[i][r];
+}
+__device__ __forceinline__ void rec_store_tile(const float* lds, float* y, int64_t ld, int lane) {
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 16 * i + (lane >> 2);
     *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + 4 * (lane & 3)) = *reinterpret_cast<const f32x4*>(lds + row * kOutStride + 4 * (lane & 3));
   }
+}
+__device__ __forceinline__ void rec_store_tile(const f32x4 (&o)[2], float* lds, float* y, int64_t ld, int lane) {
+  rec_place_tile(o, lds, lane);
+  rec_store_tile(lds, y, ld, lane);
 }
 
 }  // namespace semipd

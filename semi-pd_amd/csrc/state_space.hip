@@ -19,7 +19,7 @@
 //    of the launch do not start the sequence and written back after the last row, so a prompt cut into portions, single
 //    decode tokens and a slot that another request held all take one path.
 //  * Prompt batches: ssm_chunk_operands_kernel and ssm_chunk_walk_kernel in place of the three, 32 tokens at a time on the matrix
-//    cores, every operand and sum fp32.
+//    cores, operands of 24 bits and fp32 sums.
 //  * ssm_post_kernel / ssm_post_vec_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
 //  * ssm_step_kernel: batches of one token per request in place of preparation and recurrence, a workgroup per (head, request).
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
@@ -311,18 +311,23 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
 // With la_t = log of the decay, b_t its running sum inside a chunk of 32 tokens and S the state in front of the chunk:
 //     y_t = e^(b_t) S^T C_t + sum_(s <= t) (C_t . B_s) e^(b_t - b_s) dt_s x_s + D x_t
 //     S  <- e^(b_last) S + sum_s B_s (e^(b_last - b_s) dt_s x_s)^T
-// Every exponent is at most 0.  All products are fp32 on v_mfma_f32_16x16x4_f32 (fp32 operands, fp32 sums: nothing is split or
-// rounded to 16 bits); b is summed, and its differences are taken, in 64 bits, so a weight near 1 behind a strong decay is as
-// good as the product of the decays themselves.
+// Every exponent is at most 0.  The products with S are products of fp32 values on the bf16 matrix cores, three pieces a value (see
+// rec_mma), their sums fp32; the others are v_mfma_f32_16x16x4_f32.  The state behind 4 requests of 1900 tokens is 8.5e-8 from the 64-bit
+// one (2-norm; all products of fp32 operands: 9.6e-8; with the six products added to S one by one: 1.24e-7).  b is summed, and its
+// differences are taken, in 64 bits, so a weight near 1 behind a strong decay is as good as the product of the decays themselves.
 // Bound: token by token a step is a chain of LDS reads, 64 multiply-adds and lane sums (1.0 us of a wave's time; 7262 tokens of 4
-// requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows); in chunks the fp32 matrix pipe (140 products
-// of 32 cycles a wave and chunk: 250 us here, busy for 38 % of the SIMD cycles), the vector work between its products (17 %) and their
-// loads: 560 us, operands 72.  Chunks of 32 and not 64: the same products with S, half the ones inside a chunk; operands straight
-// into registers and not through LDS: no barriers, 15 us less (64 tokens, operands in LDS, two heads a workgroup: 952 us).
-// fp32 elements of the operands of one (chunk, group): C and B^T as left-hand operands of 16 x 16 x 16 products, in the order in which
-// they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a piece of 4.  Of one
-// (chunk, head): tiles 00, 10, 11 of the weighted C B^T, then e^(b_t) | e^(b_last - b_t) dt_t | dt | decay.
-__host__ __device__ constexpr int64_t ssm_frag_elems(int np) { return 2 * (int64_t)kRecChunk * np + 4; }
+// requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows).  In chunks on the fp32 matrix pipe, a wave all
+// rows of 16 columns: 560 us (140 products of 32 cycles a wave and chunk, 38 % of the SIMD cycles, waiting for its operands in between).
+// Here 335: per wave and chunk 48 products of 16 cycles, 6 of 32 and 340 vector instructions (pieces of S 88, convolution 110), of which
+// a SIMD takes one in 4 cycles from two waves or more but only one in 8 from one; LDS reads 22 % of its cycles.  What that took: C and B^T
+// once a workgroup through LDS (24 KB each; straight into registers every wave reads them again), two waves a column block with half the
+// rows each (four a SIMD instead of two: one request of 2303 rows 265 -> 235), requests placed by length (412 -> 345).  Operands 77.
+// Chunks of 32 and not 64: the same products with S, half the ones inside a chunk, half the LDS.
+// Elements of the operands of one (chunk, group), counted in fp32: C and B^T in three planes of bf16 each, left-hand operands of 16 x 16 x 32
+// products in the order in which they are held, [tile][lane][8] (see rec_split8; tiles of C: 16 tokens x 32 rows of S, of B^T: 16 rows x
+// the tokens), and a flag in a piece of 4.  Of one (chunk, head), fp32: tiles 00, 10, 11 of the weighted C B^T, left-hand operands of 16 x
+// 16 x 16 products, [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s, then e^(b_t) | e^(b_last - b_t) dt_t | dt | decay.
+__host__ __device__ constexpr int64_t ssm_frag_elems(int np) { return 3 * (int64_t)kRecChunk * np + 4; }
 constexpr int kSsmHead = 3 * 256 + 4 * kRecChunk;
 
 // What the heads of a group share, a workgroup per (chunk, group): convolution + bias + silu of the group's B and C channels (a
@@ -393,14 +398,24 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
   }
   __syncthreads();
   const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
-  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {  // C: tile (tokens, rows of S)
-    const int tile = i >> 6, ln = i & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
-    *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(c_l + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
-  }
-  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {  // B^T: tile (rows of S, tokens)
-    const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
-    const float* s = b_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
-    *reinterpret_cast<float4*>(frag + L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+  // pieces of three planes: C, tiles (16 tokens, 32 rows of S), and B^T, tiles (16 rows of S, the tokens)
+  for (int i = lays ? tid : L * NP; i < 2 * (L * NP / 8); i += 256) {
+    const bool is_c = i < L * NP / 8;
+    const int it = is_c ? i : i - L * NP / 8, tile = it >> 6, ln = it & 63, r = ln & 15, q4 = 4 * (ln >> 4);
+    f32x4 x0, x1;
+    if (is_c) {
+      const float* s = c_l + (16 * (tile / (NP / 32)) + r) * CS + 32 * (tile % (NP / 32)) + q4;
+      x0 = *reinterpret_cast<const f32x4*>(s);
+      x1 = *reinterpret_cast<const f32x4*>(s + 16);
+    } else {
+      const float* s = b_l + q4 * CS + 16 * tile + r;
+      x0 = f32x4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+      x1 = f32x4{s[16 * CS], s[17 * CS], s[18 * CS], s[19 * CS]};
+    }
+    const Split3 s3 = rec_split8_any(x0, x1);
+    uint4* dst = reinterpret_cast<uint4*>(frag + (is_c ? 0 : 3 * L * NP / 2)) + it;
+#pragma unroll
+    for (int p = 0; p < 3; ++p) dst[p * (L * NP / 8)] = s3.p[p].u;
   }
   // C B^T, a 16 x 16 tile a wave; k runs 16 at a time, lane group kq takes k = 4 kq .. 4 kq + 3 in four steps (both operands alike)
   {
@@ -433,8 +448,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     cum[t] = c;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c) * dt, dec = expf(la);
-    const bool no = !rec_finite(dt) || !rec_moderate_decay(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
-    hp[768 + t] = rec_flagged(eb, no);
+    bool no = !rec_finite(dt) || !rec_moderate_decay(la) || !rec_finite(wt) || !rec_finite(eb) || !rec_finite(dec);
     hp[768 + L + t] = wt;
     hp[768 + 2 * L + t] = dt;
     hp[768 + 3 * L + t] = dec;
@@ -449,279 +463,359 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
       for (int v = 0; v < 4; ++v) {
         const float ds = __shfl(dt, col + v, L);
         m[v] = col + v <= row ? cb_l[row * PS + col + v] * (rec_exp2(bt - cum[col + v]) * ds) : 0.f;
+        no |= !rec_finite(m[v]);
       }
       *reinterpret_cast<f32x4*>(hp + 4 * i) = m;
     }
+    hp[768 + t] = rec_flagged(eb, no);
     __builtin_amdgcn_wave_barrier();
   }
   const int any_bad = __syncthreads_or(bad);
   if (lays && tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
-// The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
-// sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16.  That is
-// also how a wave holds the right-hand operand of a product over the rows, so S goes from one chunk's sum into the next one's product
-// without leaving its registers, and so do the chunk's x (lane: tokens 16 j + 4 kq + s of its column), which each lane convolves in
-// their place from raw inputs in the wave's own LDS: x is not written to memory.  Left-hand operands come straight into registers in
-// the order they are used, not through LDS: B^T of a chunk into the registers its C was read from, the next chunk's C into those of
-// B^T.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.
+// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S), two waves per 16 columns.  A wave has half the rows
+// of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the right-hand operand of a product
+// over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving its registers.  The
+// halves of C S are added across the two waves in LDS, each finishing 16 of the tokens; it also convolves these tokens' x from raw inputs
+// in LDS of its own and hands x and the pieces of U = e^(b_last - b_t) dt_t x over: x is not written to memory.
 template <typename T, int NP>
-__global__ void __launch_bounds__(256, 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
-  constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
-  __shared__ __attribute__((aligned(16))) T in_l[4][RowTile<T>::kElems];       // a wave's own: raw inputs of its convolution
-  __shared__ __attribute__((aligned(16))) float o_l[4][L * kOutStride];         // ... results on their way out (token by token: its x)
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+__global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
+  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / 2, HALO = kRecHalo;      // HT: 16-row tiles of S a wave
+  constexpr int PB = L * NP * 2, ALL = 3 * PB / 16, PIECES = (ALL + 511) / 512;  // bytes of a plane; 16-byte pieces of three, a thread's
+  using Tile = RowTile<T, 16>;
+  constexpr int OWN = Tile::kElems * (int)sizeof(T) > 16 * kOutStride * 4 ? Tile::kElems * (int)sizeof(T) : 16 * kOutStride * 4;
+  __shared__ __attribute__((aligned(16))) uint8_t c_l[3 * PB], b_l[3 * PB];     // C and B^T of the chunk, as laid down
+  __shared__ __attribute__((aligned(16))) uint8_t u_l[4][3][1024];              // U of the chunk: [columns][piece][lane][16]; token by token x
+  __shared__ __attribute__((aligned(16))) uint8_t x_l[4][1024];                 // x of its tokens 0 .. 15, for the waves of 16 .. 31
+  __shared__ __attribute__((aligned(16))) uint8_t own_l[8][OWN];                // by turns a wave's half sum of C S, raw inputs, results on their way out
+  __shared__ int serial_l[2];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int cw = w & 3, half = w >> 2;
   // workgroups of one (request, group) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, per = H / G;
   const int eblocks = (E + 63) / 64, members = per * eblocks;
   const RecPlace at = rec_place((int)a.batch * G, members);
   if (at.unit < 0) return;
-  const int member = at.member, b = at.unit / G, g = at.unit % G;
+  const int per_request = G * members, firsts = 2 * 256 >= (int)a.batch * per_request ? (256 + per_request - 1) / per_request : (int)a.batch;
+  const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, min(firsts, (int)a.batch));
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
-  const int64_t chunk0 = rec_chunks_before(a.q_len, b);
+  const int64_t chunk0 = __builtin_amdgcn_readfirstlane((int)rec_chunks_before(a.q_len, b));
   if (chunk0 + (n + L - 1) / L > max_chunks) return;          // (requests that share rows: more rows than the launch has)
   const int h = g * per + member / eblocks;
-  const int e0 = member % eblocks * 64 + 16 * w, e = e0 + r16;
-  if (e0 >= E) return;
+  const int e0 = member % eblocks * 64 + 16 * cw, e = e0 + r16;
+  const bool on = e0 < E;                                        // (waves without columns take their part of the staging)
   const bool e_ok = e < E, wide = e0 + 16 <= E;
   const int C = H * E + 2 * G * N;
   const int64_t slot = a.state_indices[b];
   float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
-  f32x4 S[NT];
+  const int row0 = half * (NP / 2) + 4 * kq;                     // this lane's rows of S: row0 + 16 t + r
+  f32x4 S[HT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t)
+  for (int t = 0; t < HT; ++t)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = 16 * t + 4 * kq + r;
-      S[t][r] = (first_pos > 0 && e_ok && row < N) ? st[row * E] : 0.f;
-    }
+    for (int r = 0; r < 4; ++r) S[t][r] = (first_pos > 0 && e_ok && row0 + 16 * t + r < N) ? st[(row0 + 16 * t + r) * E] : 0.f;
   float wt[kRecTaps];
 #pragma unroll
   for (int i = 0; i < kRecTaps; ++i) wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_w)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
   const float bias = (a.conv_b && e_ok) ? Elem<T>::to_f(((const T*)a.conv_b)[h * E + e]) : 0.f;
   const float dskip = a.d_skip ? a.d_skip[h] : 0.f;
   const int64_t frag_ld = (int64_t)G * ssm_frag_elems(NP), head_ld = (int64_t)H * kSsmHead;
-  const float* f = a.frags + chunk0 * frag_ld + g * ssm_frag_elems(NP) + 4 * lane;
+  const float* f = a.frags + chunk0 * frag_ld + g * ssm_frag_elems(NP);
   const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kSsmHead;
   const T* p = (const T*)a.p + t0 * a.ld + a.x_off + h * E + e0;
   float* yo = a.work + t0 * a.wld + h * E + e0;
   // 16-byte pieces of the projection's and of the result's rows: everything starts on one
   const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
-                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0 && a.ld < (1 << 24) && a.wld < (1 << 24);
 
-  // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
-  RowTile<T> tile;
-  auto fetch_x = [&](int l0) { if (vec) tile.fetch(p, a.ld, l0, n, lane); };
-  // x of this lane's tokens, zero behind the portion; taps that the layer does not have see zeros
-  auto convolve = [&](const float (&raw)[2][HALO + 4], int cnt, f32x4 (&x)[2], bool& bad) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        float y = bias + wt[0] * raw[j][s + HALO];
-#pragma unroll
-        for (int i = 1; i < kRecTaps; ++i) y += wt[i] * __int_as_float(__float_as_int(raw[j][s + HALO - i]) & (i < taps ? -1 : 0));
-        float z = rec_silu(y);
-        asm volatile("" : "+v"(z));                              // (straight-line code: it goes between the products)
-        const bool in = 16 * j + 4 * kq + s < cnt;
-        x[j][s] = in ? (rec_moderate(y) ? z : y) : 0.f;       // (one that is not: see `serial`)
-        bad |= in && !rec_moderate(y);
-      }
+  // raw inputs of the convolution, tokens 16 half - HALO .. 16 half + 15 of the chunk at l0 > 0
+  Tile tile;
+  auto fetch_x = [&](int l0) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                                 // (addresses made where they are used, not held over the loop)
+    if (vec) tile.fetch(p, a.ld, l0 + 16 * half, n, ln);
   };
-  f32x4 x[2];
+  // x of this lane's tokens 16 half + 4 kq + s, zero behind the portion; taps that the layer does not have see zeros
+  auto convolve = [&](const float (&raw)[HALO + 4], int cnt, f32x4& x, bool& bad) {
+    f32x4 y;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) y[s] = bias + wt[0] * raw[s + HALO];
+    if (taps == kRecTaps) {
+#pragma unroll
+      for (int i = 1; i < kRecTaps; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) y[s] += wt[i] * raw[s + HALO - i];
+    } else {
+#pragma unroll
+      for (int i = 1; i < kRecTaps - 1; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) y[s] += wt[i] * __int_as_float(__float_as_int(raw[s + HALO - i]) & (i < taps ? -1 : 0));
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float z = rec_silu(y[s]);
+      const bool in = 16 * half + 4 * kq + s < cnt;
+      x[s] = in ? (rec_moderate(y[s]) ? z : y[s]) : 0.f;         // (one that is not: see `serial`)
+      bad |= in && !rec_moderate(y[s]);
+    }
+  };
+  // x and U = e^(b_last - b_t) dt_t x to where both waves of these columns find them
+  auto hand_over = [&](const f32x4& x, const f32x4& wv) {
+    if (half == 0) *reinterpret_cast<f32x4*>(&x_l[cw][16 * lane]) = x;
+    uint2 u[3];
+    rec_split2(x[0] * wv[0], x[1] * wv[1], u[0].x, u[1].x, u[2].x);
+    rec_split2(x[2] * wv[2], x[3] * wv[3], u[0].y, u[1].y, u[2].y);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(&u_l[cw][i][16 * lane + 8 * half]) = u[i];
+  };
+  u32x4 stage[PIECES];
+  auto fetch = [&](const float* src) {
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u)
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) stage[u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
+  };
+  auto place = [&](uint8_t* dst) {
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u)
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = stage[u];
+  };
+  f32x4 x;
   bool bad = false;
+  fetch(f);
   {
-    float in[2][HALO + 4];
+    float in[HALO + 4];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < HALO + 4; ++i) {
-        const int l = 16 * j + 4 * kq + i - HALO;
-        in[j][i] = 0.f;
-        if (e_ok && l < n) {
-          if (l >= 0) in[j][i] = Elem<T>::to_f(p[(int64_t)l * a.ld + r16]);
-          else if (first_pos > 0 && taps - 1 + l >= 0) in[j][i] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 + l) * C + h * E + e];
-        }
+    for (int i = 0; i < HALO + 4; ++i) {
+      const int l = 16 * half + 4 * kq + i - HALO;
+      in[i] = 0.f;
+      if (e_ok && l < n) {
+        if (l >= 0) in[i] = Elem<T>::to_f(p[(int64_t)l * a.ld + r16]);
+        else if (first_pos > 0 && taps - 1 + l >= 0) in[i] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 + l) * C + h * E + e];
       }
+    }
     convolve(in, n, x, bad);
   }
-  f32x4 A[2 * NT], M[3], eb[2], wv[2];
-  float flag;
-#pragma unroll
-  for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(f + 256 * i);
-  flag = f[2 * L * NP - 4 * lane];
-#pragma unroll
-  for (int i = 0; i < 3; ++i) M[i] = *reinterpret_cast<const f32x4*>(fh + 256 * i + 4 * lane);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    eb[i] = *reinterpret_cast<const f32x4*>(fh + 768 + 16 * i + 4 * kq);
-    wv[i] = *reinterpret_cast<const f32x4*>(fh + 768 + L + 16 * i + 4 * kq);
-  }
+  hand_over(x, *reinterpret_cast<const f32x4*>(fh + 768 + L + 16 * half + 4 * kq));
+  place(c_l);
+  if (tid < 2) serial_l[tid] = 0;
   if (L < n) fetch_x(L);
+  __syncthreads();
 
+  // Two steps a chunk, what the next one needs on its way into registers during each: C S while B^T comes, then the products inside the
+  // chunk and the new S while the next chunk's C comes.
   for (int l0 = 0; l0 < n; l0 += L) {
-    const int cnt = n - l0 < L ? n - l0 : L;
+    const int cnt = n - l0 < L ? n - l0 : L, turn = (l0 / L) & 1;
     const bool more = l0 + L < n;
     const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
     const float* fhn = fh + (more ? head_ld : 0);
-    float* yr = yo + (int64_t)l0 * a.wld;
-    // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
-    // with a weight of zero, and so would a product of a large S with rows behind a step that resets it: the wave takes such a chunk
-    // token by token behind the products, which then count for nothing, from S in the state row and x in LDS (a rare path: it must
-    // not set the kernel's registers)
-    const bool flagged = bad || flag != 0.f;
-    int rows = N, step = E;
-    asm volatile("" : "+s"(rows), "+s"(step));
-    bool serial;
-    f32x4 xn[2];
-    {
-      const float keep = __shfl(eb[1][3], 63, 64);
-      f32x4 O[2] = {};
+    float* yr = yo + (int64_t)(l0 + 16 * half) * a.wld;
+    fetch(f + 3 * L * NP / 2);
+    const float flag = f[3 * L * NP], keep = fh[768 + L - 1];
+    f32x4 M[2] = {}, eb = {}, wv = {};
+    auto fetch_head = [&]() {                                   // row tile `half` of the weighted C B^T, weights of this lane's tokens
+      M[0] = *reinterpret_cast<const f32x4*>(fh + 256 * half + 4 * lane);
+      M[1] = *reinterpret_cast<const f32x4*>(fh + 512 * half + 4 * lane);
+      eb = *reinterpret_cast<const f32x4*>(fh + 768 + 16 * half + 4 * kq);
+      wv = *reinterpret_cast<const f32x4*>(fhn + 768 + L + 16 * half + 4 * kq);
+    };
+    f32x4 O = {};
+    bool serial = false;
+    if (on) {
+      f32x4 P[2] = {}, Ps[2] = {};
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[i * NT + t][s], S[t][s], O[i], 0, 0, 0);
-      // the next chunk's x between the products: a product keeps the matrix pipe for 32 cycles, in which a few of these fit
-      bad = false;
-      {
-        float in[2][HALO + 4];
-        if (vec) {
-          tile.place(in_l[w], lane);
-        } else {                                                 // (rows or columns that start off a 16-byte boundary: not fetched ahead)
-          for (int r = kq; r < L + HALO; r += 4)
-            in_l[w][r * RowTile<T>::kStride + r16] = e_ok && l0 + L - HALO + r < n ? p[(int64_t)(l0 + L - HALO + r) * a.ld + r16] : Elem<T>::from_f(0.f);
-        }
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int i = 0; i < HALO + 4; ++i) in[j][i] = Elem<T>::to_f(in_l[w][(16 * j + 4 * kq + i) * RowTile<T>::kStride + r16]);
-        convolve(in, n - l0 - L, xn, bad);
-      }
-#pragma unroll
-      for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(f + L * NP + 256 * i);
-      flag = fn[2 * L * NP - 4 * lane];
-#pragma unroll
-      for (int i = 0; i < 8 * NT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-      }
-      if (l0 + 2 * L < n) fetch_x(l0 + 2 * L);
-      {
-        float z = 0.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) z = fmaf(O[i / 4][i % 4], 0.f, z);
-        serial = __any(flagged || keep != keep);                 // (keep: see rec_flagged)
-        if (__any(z != 0.f)) {                                   // (a column of S that is not finite stays so in either form)
-          float c = 0.f;
-#pragma unroll
-          for (int t = 0; t < NT; ++t) c = fmaf(S[t][0], 0.f, fmaf(S[t][1], 0.f, fmaf(S[t][2], 0.f, fmaf(S[t][3], 0.f, c))));
-          c += __shfl_xor(c, 16, 64);
-          c += __shfl_xor(c, 32, 64);
-          serial |= __any(z != 0.f && c == 0.f);
-        }
-      }
-      if (serial) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int s = 0; s < 4; ++s) o_l[w][(16 * j + 4 * kq + s) * kOutStride + r16] = rec_silu_if_large(x[j][s]);
-        if (e_ok)
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int i = 0; i < 2; ++i) O[i] *= eb[i];
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) O[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[i][s], x[0][s], O[i], 0, 0, 0);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) O[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(M[2][s], x[1][s], O[1], 0, 0, 0);
-      f32x4 U[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        O[i] += dskip * x[i];
-        U[i] = x[i] * wv[i];
-      }
-#pragma unroll
-      for (int i = 0; i < 3; ++i) M[i] = *reinterpret_cast<const f32x4*>(fhn + 256 * i + 4 * lane);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        eb[i] = *reinterpret_cast<const f32x4*>(fhn + 768 + 16 * i + 4 * kq);
-        wv[i] = *reinterpret_cast<const f32x4*>(fhn + 768 + L + 16 * i + 4 * kq);
-      }
-      if (serial) {
-      } else if (cnt == L && vec) {
-        rec_store_tile(O, o_l[w], yr, a.wld, lane);
-      } else {
+      for (int u = 0; u < HT / 2; ++u) {
+        const Split3 s = rec_split8(S[2 * u], S[2 * u + 1]);
+        Frag16 c[2][3];
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (16 * i + 4 * kq + r < cnt && e_ok) yr[(int64_t)(16 * i + 4 * kq + r) * a.wld + r16] = O[i][r];
+          for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(c_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+        rec_mma<2>(c, s, P, Ps);
       }
+      fetch_head();
+      float z = 0.f, top = 0.f;
 #pragma unroll
-      for (int t = 0; t < NT; ++t) S[t] *= keep;
+      for (int i = 0; i < 2; ++i) {
+        P[i] += Ps[i];
 #pragma unroll
-      for (int t = 0; t < NT; t += 2)
+        for (int r = 0; r < 4; ++r) {
+          z = fmaf(P[i][r], 0.f, z);
+          top = fmaxf(top, fabsf(P[i][r]));
+        }
+      }
+      O = half ? P[1] : P[0];
+      *reinterpret_cast<f32x4*>(&own_l[w ^ 4][16 * lane]) = half ? P[0] : P[1];
+      // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
+      // with a weight of zero, and so would a product of a large S with rows behind a step that resets it: the workgroup takes such a
+      // chunk token by token, from S in the state row and x in LDS (a rare path: it must not set the kernel's registers)
+      const bool off = z != 0.f || top > 0x1p126f;
+      if (__any(bad || flag != 0.f || keep != keep || off)) {    // (keep: see rec_flagged)
+        float c = 0.f, most = 0.f;                               // (a column of S that has a NaN and no infinity stays so in either form)
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
+        for (int t = 0; t < HT; ++t)
 #pragma unroll
-          for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) S[t + i] = __builtin_amdgcn_mfma_f32_16x16x4f32(A[2 * (t + i) + k][s], U[k][s], S[t + i], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 2 * NT; ++i) A[i] = *reinterpret_cast<const f32x4*>(fn + 256 * i);
+          for (int r = 0; r < 4; ++r) {
+            c = fmaf(S[t][r], 0.f, c);
+            most = fmaxf(most, fabsf(S[t][r]));
+          }
+        c += __shfl_xor(c, 16, 64);
+        c += __shfl_xor(c, 32, 64);
+        serial = __any(bad || flag != 0.f || keep != keep || (off && (c == 0.f || !rec_finite(most))));
+      }
+      if (serial && lane == 0) serial_l[turn] = 1;
     }
-    if (serial) {
-#pragma unroll 1
-      for (int t = 0; t < cnt; ++t) {
-        const float xv = o_l[w][t * kOutStride + r16], dt = fh[768 + 2 * L + t], dec = fh[768 + 3 * L + t], dx = dt * xv;
-        const float* cr = f - 4 * lane + (t >> 4) * NT * 256 + 4 * (16 * kq + (t & 15));           // row t of C: this lane group's four of every 16
-        const float* br = f - 4 * lane + L * NP + (t >> 4) * 256 + 4 * (16 * ((t & 15) >> 2) + 4 * kq) + (t & 3);     // column t of B^T
-        float y = 0.f;
-#pragma unroll 1
-        for (int u = 0; u < 4 * NT; ++u) {
-          const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
-          if (row < rows && e_ok) {
-            const float v = dec * st[row * step] + br[(u >> 2) * 512 + 4 * (u & 3)] * dx;
-            st[row * step] = v;
-            y += v * cr[(u >> 2) * 256 + (u & 3)];
+    place(b_l);
+    Split3 U;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) U.p[i].u = *reinterpret_cast<const uint4*>(&u_l[cw][i][16 * lane]);
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(&x_l[cw][16 * lane]);
+    __syncthreads();
+    fetch(fn);
+    serial = __builtin_amdgcn_readfirstlane(serial_l[turn]) != 0;
+    if (tid == 0) serial_l[turn ^ 1] = 0;
+    if (!serial) {
+      if (on) {
+        O = (O + *reinterpret_cast<const f32x4*>(&own_l[w][16 * lane])) * eb;
+        // (a row tile of the weights is at most two products of four columns for each of its rows: as they are, in fp32)
+        if (half == 0) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x[s], O, 0, 0, 0);
+        } else {
+          f32x4 O1 = {};
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x0[s], O, 0, 0, 0);
+            O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], x[s], O1, 0, 0, 0);
+          }
+          O += O1;
+        }
+#pragma unroll
+        for (int t = 0; t < HT; t += 2) {
+          Frag16 bt[2][3];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int q = 0; q < 3; ++q) bt[i][q].u = *reinterpret_cast<const uint4*>(b_l + q * PB + (half * HT + t + i) * 1024 + lane * 16);
+          }
+          f32x4 D[2] = {}, Ds[2] = {};
+          rec_mma<2>(bt, U, D, Ds);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            D[i] += Ds[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[t + i][r] = fmaf(S[t + i][r], keep, D[i][r]);
           }
         }
-        y += __shfl_xor(y, 16, 64);
-        y += __shfl_xor(y, 32, 64);
-        if (kq == 0 && e_ok) yr[(int64_t)t * a.wld + r16] = y + dskip * xv;
+        O += dskip * x;
       }
+    } else {
+      int rows = N, step = E;
+      asm volatile("" : "+s"(rows), "+s"(step));                 // (no addresses of 16 rows held over the loop)
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+      const int r16 = ln & 15, kq = ln >> 4, row0 = half * (NP / 2) + 4 * kq, e = e0 + r16;
+      const bool e_ok = e < E;
+      float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
+      float* xs = reinterpret_cast<float*>(u_l[0][0]) + 16 * cw + r16;           // x [32][64]
 #pragma unroll
-      for (int t = 0; t < NT; ++t)
+      for (int s = 0; s < 4; ++s) xs[(16 * half + 4 * kq + s) * 64] = rec_silu_if_large(x[s]);
+      if (e_ok)
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          S[t][r] = e_ok && 16 * t + 4 * kq + r < rows ? st[(16 * t + 4 * kq + r) * step] : 0.f;
+        for (int t = 0; t < HT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
+      __syncthreads();
+      if (half == 0 && on) {
+#pragma unroll 1
+        for (int t = 0; t < cnt; ++t) {
+          const float xv = xs[t * 64], dt = fh[768 + 2 * L + t], dec = fh[768 + 3 * L + t], dx = dt * xv;
+          // row t of C: this lane group's four of every 16; column t of B^T
+          const uint16_t* cr = reinterpret_cast<const uint16_t*>(f) + (t >> 4) * (NT / 2) * 512 + 8 * (16 * kq + (t & 15));
+          const uint16_t* br = reinterpret_cast<const uint16_t*>(f) + 3 * L * NP + 8 * (16 * ((t & 15) >> 2) + 4 * kq) + (t & 3) + 4 * (t >> 4);
+          float y = 0.f;
+#pragma unroll 1
+          for (int u = 0; u < 4 * NT; ++u) {
+            const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
+            if (row < rows && e_ok) {
+              const float v = dec * st[row * step] + rec_joined(br + (u >> 2) * 512 + 8 * (u & 3), L * NP) * dx;
+              st[row * step] = v;
+              y += v * rec_joined(cr + (u >> 3) * 512 + (u & 3) + (u & 4), L * NP);
+            }
+          }
+          y += __shfl_xor(y, 16, 64);
+          y += __shfl_xor(y, 32, 64);
+          if (kq == 0 && e_ok) yr[(int64_t)t * a.wld + r16] = y + dskip * xv;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < HT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][r] = e_ok && row0 + 16 * t + r < rows ? st[(row0 + 16 * t + r) * step] : 0.f;
       __builtin_amdgcn_sched_barrier(0);
     }
-    x[0] = xn[0];
-    x[1] = xn[1];
+    // the next chunk's x
+    f32x4 xn = {};
+    bad = false;
+    if (more) {
+      T* raw = reinterpret_cast<T*>(own_l[w]);
+      if (vec) {
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        tile.place(raw, ln);
+      } else {                                                   // (rows or columns that start off a 16-byte boundary: not fetched ahead)
+        const int first = l0 + L + 16 * half - HALO;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
+        const int r16 = ln & 15, kq = ln >> 4;
+        const bool e_ok = e0 + r16 < E;
+        for (int r = kq; r < 16 + HALO; r += 4) raw[r * Tile::kStride + r16] = e_ok && first + r < n ? p[(int64_t)(first + r) * a.ld + r16] : Elem<T>::from_f(0.f);
+      }
+      __builtin_amdgcn_wave_barrier();
+      float in[HALO + 4];
+#pragma unroll
+      for (int i = 0; i < HALO + 4; ++i) in[i] = Elem<T>::to_f(raw[(4 * kq + i) * Tile::kStride + r16]);
+      convolve(in, n - l0 - L, xn, bad);
+      hand_over(xn, wv);
+    }
+    place(c_l);
+    // behind the wait for the pieces (memory answers in order), so that it is the next one's: results out, raw inputs in
+    if (!serial) {
+      __builtin_amdgcn_wave_barrier();
+      float* ol = reinterpret_cast<float*>(own_l[w]);
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ol[(4 * kq + r) * kOutStride + r16] = O[r];
+      __builtin_amdgcn_wave_barrier();
+      if (vec) {
+        const int row = ln >> 2;
+        if (16 * half + row < cnt)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<char*>(yr) + ((uint32_t)row * (uint32_t)(a.wld * 4) + 16u * (ln & 3))) = *reinterpret_cast<const f32x4*>(ol + row * kOutStride + 4 * (ln & 3));
+      } else if (e_ok) {
+        const int r16 = ln & 15, kq = ln >> 4;
+#pragma unroll 1
+        for (int row = kq; row < 16 && 16 * half + row < cnt; row += 4) yr[(int64_t)row * a.wld + r16] = ol[row * kOutStride + r16];
+      }
+    }
+    if (l0 + 2 * L < n) fetch_x(l0 + 2 * L);
+    x = xn;
     f = fn;
     fh = fhn;
+    __syncthreads();
   }
   int rows = N, step = E;
-  asm volatile("" : "+s"(rows), "+s"(step));                     // (no addresses of 32 rows held over the loop)
+  asm volatile("" : "+s"(rows), "+s"(step));                     // (no addresses of 16 rows held over the loop)
   if (e_ok)
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+    for (int t = 0; t < HT; ++t)
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (16 * t + 4 * kq + r < rows) st[(16 * t + 4 * kq + r) * step] = S[t][r];
+        if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
 }
 
 // gate, grouped norm, weight, one pass: a workgroup per (token, norm group), the group's elements in registers, 16-byte accesses
@@ -938,7 +1032,7 @@ static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
   const int64_t chunks = rec_max_chunks(a.num_tokens, a.batch);
   hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G, rec_head_splits(chunks * a.G, a.H / a.G)), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
-  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3(rec_walk_blocks(a.batch * a.G, members)), dim3(256), 0, s, a, chunks);
+  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), dim3(rec_walk_blocks(a.batch * a.G, members)), dim3(512), 0, s, a, chunks);
 }
 
 static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,

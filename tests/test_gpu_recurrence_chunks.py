@@ -70,11 +70,12 @@ def _ssm_run(w, rows, state, before, first, H, G, N, E, parts, eps=1e-5, decode=
 
 
 # (sizes: rows of S in and below a padded block, columns over one and two workgroups, a group of three heads; two heads a
-# workgroup in the last two.  rows: one, around multiples of 32, a single token beside a long prompt)
+# workgroup in (260, ..) and (66, ..); more workgroups than CUs, fewer than two a CU, in the last.  rows: one, around multiples of 32, a single token beside a long prompt)
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,G,N,E,taps,parts,lens", [
     (4, 2, 128, 64, 4, 1, [64, 1, 130]), (6, 2, 40, 40, 2, 2, [63, 65]), (3, 1, 7, 72, 1, 1, [128, 127]), (2, 2, 65, 8, 3, 2, [16, 200]),
-    (260, 4, 16, 8, 4, 4, [33, 65]), (66, 22, 24, 24, 3, 1, [17] * 7 + [70])])
+    (260, 4, 16, 8, 4, 4, [33, 65]), (66, 22, 24, 24, 3, 1, [17] * 7 + [70]),
+    (100, 2, 16, 64, 4, 1, [33, 5, 90, 64, 1])])
 def test_state_space_in_chunks(dtype, H, G, N, E, taps, parts, lens):
     """Fresh sequences and portions (every second request) in one launch.  fp32: products and sums of 32 bits over at most 200 tokens;
     16-bit types: the rounding of the result, half a unit in the last place, on top."""
@@ -88,6 +89,18 @@ def test_state_space_in_chunks(dtype, H, G, N, E, taps, parts, lens):
         torch.testing.assert_close(outs[b].to(F64), want, rtol=ulp + 2e-5, atol=2e-5)
         torch.testing.assert_close(after[b].to(F64), S, rtol=1e-5, atol=1e-5)
         torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
+
+
+@pytest.mark.parametrize("N", [64, 128])
+def test_state_space_in_chunks_keeps_32_bits(N):
+    """Products of values in three pieces of 8 bits: a chunk rounds the state, and what it adds to it, three times by at most 2^-24, and
+    with decays of 0.7 on average about three of these roundings are left at the end; two pieces would be off by 2^-17."""
+    H, G, E, lens = 4, 2, 64, [512]
+    w, rows, state, before = _ssm_inputs(H, G, N, E, 4, lens, torch.float32, 7)
+    outs, after, _ = _ssm_run(w, rows, state, before, [9], H, G, N, E, 1)
+    want, S, _ = _ssm_truth(w, rows[0], state[0], before[0], H, G, N, E, 1)
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 2.0 ** -22
+    assert float((outs[0].to(F64) - want).norm() / want.norm()) < 2.0 ** -20
 
 
 def test_state_space_in_chunks_strong_decays():
