@@ -17,8 +17,8 @@
 //    as 16-byte pieces that are in flight a stage ahead and sit in LDS (k . q, g, beta beside them); o leaves the same way.
 //    The state is read when the rows of the launch do not start the sequence and written back after the last row, so a
 //    prompt cut into portions, single decode tokens and a slot that another request held all take one path.
-//  * Prompt batches: delta_chunk_operands_kernel and delta_chunk_walk_kernel in place of the three, 32 tokens at a time on the
-//    matrix cores, every operand and sum fp32.
+//  * Prompt batches: delta_chunk_operands_kernel and delta_chunk_walk_kernel (keys of up to 64: delta_chunk_walk_small_kernel) in place of
+//    the three, 32 tokens at a time on the matrix cores, operands of 24 bits and fp32 sums.
 //  * delta_post_kernel / delta_post_vec_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
 //  * delta_step_kernel / delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, key
 //    head) where the state lies on 16-byte boundaries, else per (request, head).
@@ -604,20 +604,22 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
 //     o_t = e^(b_t) S^T q_t + sum_(s <= t) e^(b_t - b_s) (q_t . k_s) u_s
 //     S  <- e^(b_last) S + sum_s k_s (e^(b_last - b_s) u_s)^T
 // The sums over s < t are a unit lower triangular matrix A, so U = (I + A)^-1 diag(beta) (V - diag(e^b) K S); everything in
-// front of V and S is independent of the chunks before it and is computed for all chunks at once.  All operands and sums are
-// fp32 (v_mfma_f32_16x16x4_f32; nothing is split or rounded to 16 bits), every exponent is at most 0, b is summed, and its
-// differences are taken, in 64 bits.
+// front of V and S is independent of the chunks before it and is computed for all chunks at once.  Every exponent is at most 0, b is
+// summed, and its differences are taken, in 64 bits.  All products are of fp32 operands (v_mfma_f32_16x16x4_f32), those with S of keys of
+// more than 64 on the bf16 matrix cores, three pieces a value (see rec_mma; state behind 4 requests of 1900 tokens 3.37e-8 from the 64-bit
+// one, in either form), sums fp32.
 // Bound: token by token a step is a chain of two dot products, a lane sum and an update (0.8 us; 7262 tokens of 4 requests, 32 heads of
-// 128 x 128: 1861 us + 317 of preparation); in chunks a wave's chain of 216 products of 32 cycles a chunk (72 chunks: 207 us, one
-// wave a SIMD at 4 requests; busy for 45 % of the SIMD cycles, the vector unit for 18 %): 385 us, operands 95.  With the raw inputs of v fetched at the end of a chunk and convolved in
-// front of the products 483 (the loads of 35 rows 24 KB apart were waited for), fetched a whole chunk ahead 390, by 16 bytes a lane
-// through the wave's LDS 370 (then; 385 with the larger range of silu).
-
-// fp32 elements of the operands of one (chunk, key head): K, Q and K^T as left-hand operands of 16 x 16 x 16 products, the
-// order in which they are held: [tile][lane][4], lane (r16, kq) element s = row r16, column 4 kq + s of the tile; a flag in a
-// piece of 4.  Of one (chunk, head): tiles 00, 10, 11 of (I + A)^-1 diag(beta) and of the weighted Q K^T, then
-// e^(b_t) | e^(b_last - b_t) | decay | beta.
-__host__ __device__ constexpr int64_t delta_frag_elems(int np) { return 3 * (int64_t)kRecChunk * np + 4; }
+// 128 x 128: 1861 us + 317 of preparation).  In chunks with all products in fp32, a wave all rows of 16 columns: a chain of 216 products of
+// 32 cycles a chunk, one wave a SIMD at 4 requests: 385 us.  In pieces, two waves a column block with half the rows each: 345, two waves a
+// SIMD, each with 72 products of 16 cycles, 16 or 20 of 32, 450 vector instructions and 50 LDS reads of 1 KB a chunk, which cover each other
+// in part (10 k cycles a chunk against 7 k one behind the other).  Operands 100.
+// Elements of the operands of one (chunk, key head), counted in fp32: keys of more than 64: K, Q and K^T in three planes of bf16 each,
+// left-hand operands of 16 x 16 x 32 products in the order in which they are held, [tile][lane][8] (see rec_split8; tiles of K and Q: 16
+// tokens x 32 rows of S, of K^T: 16 rows x the tokens); else in fp32, of 16 x 16 x 16 products, [tile][lane][4], lane (r16, kq) element s =
+// row r16, column 4 kq + s of the tile; a flag in a piece of 4.  Of one (chunk, head), fp32, [tile][lane][4]: tiles 00, 10, 11 of
+// (I + A)^-1 diag(beta) and of the weighted Q K^T, then e^(b_t) | e^(b_last - b_t) | decay | beta.
+constexpr int kDeltaSmall = 64;
+__host__ __device__ constexpr int64_t delta_frag_elems(int np) { return (np <= kDeltaSmall ? 3 : 4.5) * kRecChunk * np + 4; }
 constexpr int kDeltaHead = 6 * 256 + 4 * kRecChunk;
 
 // A workgroup per (chunk, key head): convolution, silu and unit norm of its q and k (a channel per thread), K K^T and Q K^T, then
@@ -702,14 +704,35 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
   __syncthreads();
   // the operands in the order in which they are held
   const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
-  for (int i = lays ? tid : 2 * L * NP; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
-    const int half = i / (L * NP / 4), it = i % (L * NP / 4), tile = it >> 6, ln = it & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
-    *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(kq_l + half * L * CS + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
-  }
-  for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {                  // K^T: tile (row of S, tokens)
-    const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
-    const float* s = kq_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
-    *reinterpret_cast<float4*>(frag + 2 * L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+  if constexpr (NP <= kDeltaSmall) {
+    for (int i = lays ? tid : 2 * L * NP; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
+      const int half = i / (L * NP / 4), it = i % (L * NP / 4), tile = it >> 6, ln = it & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
+      *reinterpret_cast<float4*>(frag + 4 * i) = *reinterpret_cast<const float4*>(kq_l + half * L * CS + (16 * rt + (ln & 15)) * CS + 16 * ct + 4 * (ln >> 4));
+    }
+    for (int i = lays ? tid : L * NP; i < L * NP / 4; i += 256) {                  // K^T: tile (row of S, tokens)
+      const int tile = i >> 6, ln = i & 63, rt = tile >> 1, ct = tile & 1;
+      const float* s = kq_l + (16 * ct + 4 * (ln >> 4)) * CS + 16 * rt + (ln & 15);
+      *reinterpret_cast<float4*>(frag + 2 * L * NP + 4 * i) = float4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+    }
+  } else {
+    // pieces of three planes: K and Q, tiles (16 tokens, 32 rows of S), and K^T, tiles (16 rows of S, the tokens)
+    for (int i = lays ? tid : L * NP; i < 3 * (L * NP / 8); i += 256) {
+      const int part = i / (L * NP / 8), it = i % (L * NP / 8), tile = it >> 6, ln = it & 63, r = ln & 15, q4 = 4 * (ln >> 4);
+      f32x4 x0, x1;
+      if (part < 2) {
+        const float* s = kq_l + part * L * CS + (16 * (tile / (NP / 32)) + r) * CS + 32 * (tile % (NP / 32)) + q4;
+        x0 = *reinterpret_cast<const f32x4*>(s);
+        x1 = *reinterpret_cast<const f32x4*>(s + 16);
+      } else {
+        const float* s = kq_l + q4 * CS + 16 * tile + r;
+        x0 = f32x4{s[0], s[CS], s[2 * CS], s[3 * CS]};
+        x1 = f32x4{s[16 * CS], s[17 * CS], s[18 * CS], s[19 * CS]};
+      }
+      const Split3 s3 = rec_split8_any(x0, x1);
+      uint4* dst = reinterpret_cast<uint4*>(frag + part * (3 * L * NP / 2)) + it;
+  #pragma unroll
+      for (int p = 0; p < 3; ++p) dst[p * (L * NP / 8)] = s3.p[p].u;
+    }
   }
   {
     const int i0 = (w >> 1) * 16, j0 = (w & 1) * 16;
@@ -794,15 +817,377 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
   if (lays && tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
-// The chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
+// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S), two waves per 16 columns.  A wave has half the rows
+// of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the right-hand operand of a product
+// over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving its registers.  The
+// halves of K S go to the other wave through LDS and both make U; of Q S, v and the results a wave finishes 16 of the tokens.
+template <typename T, int NP>
+__global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
+  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / 2, HALO = kRecHalo;      // HT: 16-row tiles of S a wave
+  constexpr int PB = L * NP * 2, ALL = 3 * PB / 16, PIECES = (ALL + 511) / 512;  // bytes of a plane; 16-byte pieces of three, a thread's
+  using Tile = RowTile<T, 16>;
+  static_assert(Tile::kElems * sizeof(T) <= 3072 && 16 * kOutStride * 4 <= 3072, "a wave's part of ex_l");
+  __shared__ __attribute__((aligned(16))) uint8_t k_l[3 * PB], q_l[3 * PB], kt_l[3 * PB];    // K, Q and K^T of the chunk, as laid down
+  __shared__ __attribute__((aligned(16))) float head_l[kDeltaHead];             // the head's weights
+  // by turns half sums for a wave from the other one of its columns, its raw inputs, its results on their way out (token by token: v)
+  __shared__ __attribute__((aligned(16))) uint8_t ex_l[8][3][1024];
+  __shared__ __attribute__((aligned(16))) uint8_t v_l[4][2][1024];              // v of the chunk: [columns][token tile][lane][16]
+  __shared__ int serial_l[2];
+  const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, kq = lane >> 4;
+  const int cw = w & 3, half = w >> 2;
+  // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
+  const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
+  const int eblocks = (E + 63) / 64, members = per * eblocks;
+  const RecPlace at = rec_place((int)a.batch * G, members);
+  if (at.unit < 0) return;
+  const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, rec_first_requests((int)a.batch, G * members));
+  const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
+  const int n = a.q_len[b];
+  if (n <= 0 || first_pos < 0) return;
+  const int64_t chunk0 = __builtin_amdgcn_readfirstlane((int)rec_chunks_before(a.q_len, b));
+  if (chunk0 + (n + L - 1) / L > max_chunks) return;            // (requests that share rows: more rows than the launch has)
+  const int h = g * per + member / eblocks;
+  const int e0 = member % eblocks * 64 + 16 * cw, e = e0 + r16;
+  const bool on = e0 < E;                                        // (waves without columns take their part of the staging)
+  const bool e_ok = e < E, wide = e0 + 16 <= E;
+  const int C = 2 * G * D + H * E;
+  const int64_t slot = a.state_indices[b];
+  float* st = a.state + slot * a.state_ld + (int64_t)h * D * E + e;
+  const int row0 = half * (NP / 2) + 4 * kq;                     // this lane's rows of S: row0 + 16 t + r
+  f32x4 S[HT];
+#pragma unroll
+  for (int t = 0; t < HT; ++t)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[t][r] = (first_pos > 0 && e_ok && row0 + 16 * t + r < D) ? st[(row0 + 16 * t + r) * E] : 0.f;
+  float wt[kRecTaps];
+#pragma unroll
+  for (int i = 0; i < kRecTaps; ++i) wt[i] = (i < taps && e_ok) ? Elem<T>::to_f(((const T*)a.conv_v)[(int64_t)(h * E + e) * taps + taps - 1 - i]) : 0.f;
+  const int64_t frag_ld = (int64_t)G * delta_frag_elems(NP), head_ld = (int64_t)H * kDeltaHead;
+  const float* f = a.frags + chunk0 * frag_ld + g * delta_frag_elems(NP);
+  const float* fh = a.frags + max_chunks * frag_ld + (chunk0 * H + h) * kDeltaHead;
+  const T* p = (const T*)a.p + t0 * a.ld + a.v_off + h * E + e0;
+  float* yo = a.work + t0 * a.wld + h * E + e0;
+  // 16-byte pieces of the projection's and of the result's rows: everything starts on one
+  const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0 && a.ld < (1 << 24) && a.wld < (1 << 24);
+
+  // raw inputs of the convolution, tokens 16 half - HALO .. 16 half + 15 of the chunk at l0 > 0
+  Tile tile;
+  auto fetch_v = [&](int l0) {
+    int ln = lane;
+    asm volatile("" : "+v"(ln));                                 // (addresses made where they are used, not held over the loop)
+    if (vec) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
+  };
+  // v of this lane's tokens 16 half + 4 kq + s, zero behind the portion; taps that the layer does not have see zeros
+  auto convolve = [&](const float (&raw)[HALO + 4], int cnt, f32x4& v, bool& bad) {
+    f32x4 y;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) y[s] = wt[0] * raw[s + HALO];
+#pragma unroll
+    for (int i = 1; i < kRecTaps; ++i)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) y[s] += wt[i] * __int_as_float(__float_as_int(raw[s + HALO - i]) & (i < taps ? -1 : 0));
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const float z = rec_silu(y[s]);
+      const bool in = 16 * half + 4 * kq + s < cnt;
+      v[s] = in ? (rec_moderate(y[s]) ? z : y[s]) : 0.f;         // (one that is not: see `serial`)
+      bad |= in && !rec_moderate(y[s]);
+    }
+  };
+  // ... of the chunk at l0 into this lane's place, by way of the wave's LDS
+  float in[HALO + 4];
+  auto place_v = [&](int l0) {
+    T* raw = reinterpret_cast<T*>(ex_l[w][0]);
+    int ln = lane;
+    asm volatile("" : "+v"(ln));
+    __builtin_amdgcn_wave_barrier();
+    if (vec) {
+      tile.place(raw, ln);
+    } else {                                                     // (rows or columns that start off a 16-byte boundary: not fetched ahead)
+      const int first = l0 + 16 * half - HALO, r16 = ln & 15;
+      const bool e_ok = e0 + r16 < E;
+      for (int r = ln >> 4; r < 16 + HALO; r += 4) raw[r * Tile::kStride + r16] = e_ok && first + r < n ? p[(int64_t)(first + r) * a.ld + r16] : Elem<T>::from_f(0.f);
+    }
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < HALO + 4; ++i) in[i] = Elem<T>::to_f(raw[(4 * (ln >> 4) + i) * Tile::kStride + (ln & 15)]);
+  };
+  u32x4 stage[2 * PIECES], head;
+  auto fetch_head = [&](const float* src) {
+    if (tid < kDeltaHead / 4) head = reinterpret_cast<const u32x4*>(src)[tid];
+  };
+  auto fetch = [&](const float* src, int at) {
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u)
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) stage[at + u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
+  };
+  auto place = [&](uint8_t* dst, int at) {
+#pragma unroll
+    for (int u = 0; u < PIECES; ++u)
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = stage[at + u];
+  };
+  bool bad = false;
+  fetch(f, 0);
+  fetch(f + 3 * L * NP / 2, PIECES);
+  if (L < n) fetch_v(L);
+  {
+#pragma unroll
+    for (int i = 0; i < HALO + 4; ++i) {
+      const int l = 16 * half + 4 * kq + i - HALO;
+      in[i] = 0.f;
+      if (e_ok && l < n) {
+        if (l >= 0) in[i] = Elem<T>::to_f(p[(int64_t)l * a.ld + r16]);
+        else if (first_pos > 0 && taps - 1 + l >= 0) in[i] = a.conv_state[slot * a.conv_ld + (int64_t)(taps - 1 + l) * C + 2 * G * D + h * E + e];
+      }
+    }
+    f32x4 v;
+    convolve(in, n, v, bad);
+    *reinterpret_cast<f32x4*>(&v_l[cw][half][16 * lane]) = v;
+  }
+  place(k_l, 0);
+  place(q_l, PIECES);
+  if (tid < 2) serial_l[tid] = 0;
+  if (L < n) place_v(L);
+  __syncthreads();
+
+  // Two steps a chunk, what the next one needs on its way into registers during each: K S and Q S while K^T comes, then U, the products
+  // inside the chunk and the new S while the next chunk's K and Q come.
+  for (int l0 = 0; l0 < n; l0 += L) {
+    const int cnt = n - l0 < L ? n - l0 : L, turn = (l0 / L) & 1;
+    const bool more = l0 + L < n;
+    const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
+    const float* fhn = fh + (more ? head_ld : 0);
+    float* yr = yo + (int64_t)(l0 + 16 * half) * a.wld;
+    fetch_head(fh);
+    fetch(f + 3 * L * NP, 0);
+    const float flag = f[9 * L * NP / 2], keep = fh[1536 + L - 1];
+    f32x4 O = {}, P[2] = {}, v[2] = {}, vn;
+    bool serial = false, bad_next = false;
+    if (on) {
+      f32x4 Q[2] = {};
+      {
+        f32x4 Ps[2] = {}, Qs[2] = {};
+#pragma unroll
+        for (int u = 0; u < HT / 2; ++u) {
+          const Split3 s = rec_split8(S[2 * u], S[2 * u + 1]);
+          Frag16 c[2][3];
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(k_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+          rec_mma<2>(c, s, P, Ps);
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(q_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+          rec_mma<2>(c, s, Q, Qs);
+        }
+        convolve(in, n - l0 - L, vn, bad_next);                  // (the next chunk's, between the products; there is none: zeros)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          P[i] += Ps[i];
+          Q[i] += Qs[i];
+        }
+      }
+      // the other wave of these columns gets all of K S and the tokens of Q S that it finishes
+      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][0][16 * lane]) = P[0];
+      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][1][16 * lane]) = P[1];
+      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][2][16 * lane]) = half ? Q[0] : Q[1];
+      O = half ? Q[1] : Q[0];
+      float z = 0.f, top = 0.f;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          z = fmaf(P[i][r], 0.f, z);
+          top = fmaxf(top, fabsf(P[i][r]));
+        }
+      // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
+      // with a weight of zero, and so would a product of a large S with rows behind a step that resets it: the workgroup takes such a
+      // chunk token by token, from S in the state row and v in LDS (a rare path: it must not set the kernel's registers).  Up to 2^90 what
+      // U grows to, 2^31 at most, and the sums of it stay within 32 bits; |q| = D^-1/2: its products stay below the largest of S.
+      const bool off = z != 0.f || top > 0x1p90f;
+      if (__any(bad || flag != 0.f || keep != keep || off)) {    // (keep: see rec_flagged)
+        float c = 0.f, most = 0.f;                               // (a column of S that has a NaN and no infinity stays so in either form)
+#pragma unroll
+        for (int t = 0; t < HT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            c = fmaf(S[t][r], 0.f, c);
+            most = fmaxf(most, fabsf(S[t][r]));
+          }
+        c += __shfl_xor(c, 16, 64);
+        c += __shfl_xor(c, 32, 64);
+        serial = __any(bad || flag != 0.f || keep != keep || (off && (c == 0.f || !rec_finite(most))));
+      }
+      if (serial && lane == 0) serial_l[turn] = 1;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) v[i] = *reinterpret_cast<const f32x4*>(&v_l[cw][i][16 * lane]);
+    }
+    place(kt_l, 0);
+    if (tid < kDeltaHead / 4) reinterpret_cast<u32x4*>(head_l)[tid] = head;
+    if (l0 + 2 * L < n) fetch_v(l0 + 2 * L);
+    __syncthreads();
+    fetch(fn, 0);
+    fetch(fn + 3 * L * NP / 2, PIECES);
+    serial = __builtin_amdgcn_readfirstlane(serial_l[turn]) != 0;
+    if (tid == 0) serial_l[turn ^ 1] = 0;
+    if (!serial) {
+      if (on) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const f32x4 eb = *reinterpret_cast<const f32x4*>(head_l + 1536 + 16 * i + 4 * kq);
+          P[i] += *reinterpret_cast<const f32x4*>(&ex_l[w][i][16 * lane]);
+          v[i] -= eb * P[i];
+        }
+        O = (O + *reinterpret_cast<const f32x4*>(&ex_l[w][2][16 * lane])) * *reinterpret_cast<const f32x4*>(head_l + 1536 + 16 * half + 4 * kq);
+        f32x4 Ti[3], M[2], wv[2];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) Ti[i] = *reinterpret_cast<const f32x4*>(head_l + 256 * i + 4 * lane);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) wv[i] = *reinterpret_cast<const f32x4*>(head_l + 1536 + L + 16 * i + 4 * kq);
+        M[0] = *reinterpret_cast<const f32x4*>(head_l + 768 + 256 * half + 4 * lane);       // row tile `half` of the weighted Q K^T
+        M[1] = *reinterpret_cast<const f32x4*>(head_l + 768 + 512 * half + 4 * lane);
+        // (products of 16 or 32 columns: as they are, in fp32; both waves of these columns make U)
+        f32x4 U[2] = {}, U1 = {};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          U[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ti[0][s], v[0][s], U[0], 0, 0, 0);
+          U[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(Ti[1][s], v[0][s], U[1], 0, 0, 0);
+          U1 = __builtin_amdgcn_mfma_f32_16x16x4f32(Ti[2][s], v[1][s], U1, 0, 0, 0);
+        }
+        U[1] += U1;
+        const Split3 us = rec_split8(U[0] * wv[0], U[1] * wv[1]);
+        f32x4 O1 = {};
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], U[0][s], O, 0, 0, 0);
+          if (half) O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], U[1][s], O1, 0, 0, 0);
+        }
+        O += O1;
+#pragma unroll
+        for (int t = 0; t < HT; t += 2) {
+          Frag16 kt[2][3];
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) kt[i][q].u = *reinterpret_cast<const uint4*>(kt_l + q * PB + (half * HT + t + i) * 1024 + lane * 16);
+          f32x4 A[2] = {}, As[2] = {};
+          rec_mma<2>(kt, us, A, As);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            A[i] += As[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[t + i][r] = fmaf(S[t + i][r], keep, A[i][r]);
+          }
+        }
+      }
+    } else {
+      int rows = D, step = E, ln = lane;
+      asm volatile("" : "+s"(rows), "+s"(step), "+v"(ln));       // (no addresses held over the loop)
+      const int r16 = ln & 15, kq = ln >> 4, row0 = half * (NP / 2) + 4 * kq, e = e0 + r16;
+      const bool e_ok = e < E;
+      float* st = a.state + slot * a.state_ld + (int64_t)h * D * E + e;
+      float* vs = reinterpret_cast<float*>(ex_l[0][0]) + 16 * cw + r16;          // v [32][64]
+#pragma unroll
+      for (int s = 0; s < 4; ++s) vs[(16 * half + 4 * kq + s) * 64] = rec_silu_if_large(half ? v[1][s] : v[0][s]);
+      if (e_ok)
+#pragma unroll
+        for (int t = 0; t < HT; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
+      __syncthreads();
+      if (half == 0 && on) {
+#pragma unroll 1
+        for (int t = 0; t < cnt; ++t) {
+          // row t of K: this lane group's four of every 16
+          const uint16_t* kr = reinterpret_cast<const uint16_t*>(f) + (t >> 4) * (NT / 2) * 512 + 8 * (16 * kq + (t & 15));
+          float dk = 0.f, dq = 0.f, kd = 0.f;
+#pragma unroll 1
+          for (int u = 0; u < 4 * NT; ++u) {
+            const int row = 16 * (u >> 2) + 4 * kq + (u & 3), at = (u >> 3) * 512 + (u & 3) + (u & 4);
+            if (row < rows) {
+              const float kv = rec_joined(kr + at, L * NP), qv = rec_joined(kr + 3 * L * NP + at, L * NP), sv = e_ok ? st[row * step] : 0.f;
+              dk += sv * kv;
+              dq += sv * qv;
+              kd += kv * qv;
+            }
+          }
+          dk += __shfl_xor(dk, 16, 64);
+          dk += __shfl_xor(dk, 32, 64);
+          dq += __shfl_xor(dq, 16, 64);
+          dq += __shfl_xor(dq, 32, 64);
+          kd += __shfl_xor(kd, 16, 64);
+          kd += __shfl_xor(kd, 32, 64);
+          const float gt = fh[1536 + 2 * L + t], bt = fh[1536 + 3 * L + t];
+          const float u1 = bt * (vs[t * 64] - gt * dk);
+#pragma unroll 1
+          for (int u = 0; u < 4 * NT; ++u) {
+            const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
+            if (row < rows && e_ok) st[row * step] = gt * st[row * step] + rec_joined(kr + (u >> 3) * 512 + (u & 3) + (u & 4), L * NP) * u1;
+          }
+          if (kq == 0 && e_ok) yr[(int64_t)t * a.wld + r16] = gt * dq + u1 * kd;
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < HT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) S[t][r] = e_ok && row0 + 16 * t + r < rows ? st[(row0 + 16 * t + r) * step] : 0.f;
+      __builtin_amdgcn_s_waitcnt(0x0f70);                        // (vmcnt(0) here, or the other path waits for what it has in flight where they join)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (more && on) *reinterpret_cast<f32x4*>(&v_l[cw][half][16 * lane]) = vn;
+    bad = bad_next;
+    place(k_l, 0);
+    place(q_l, PIECES);
+    // behind the wait for the pieces (memory answers in order), so that it is the next one's
+    if (!serial) {
+      __builtin_amdgcn_wave_barrier();
+      float* ol = reinterpret_cast<float*>(ex_l[w][0]);
+      int ln = lane;
+      asm volatile("" : "+v"(ln));
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ol[(4 * kq + r) * kOutStride + r16] = O[r];
+      __builtin_amdgcn_wave_barrier();
+      if (vec) {
+        const int row = ln >> 2;
+        if (16 * half + row < cnt)
+          *reinterpret_cast<f32x4*>(reinterpret_cast<char*>(yr) + ((uint32_t)row * (uint32_t)(a.wld * 4) + 16u * (ln & 3))) = *reinterpret_cast<const f32x4*>(ol + row * kOutStride + 4 * (ln & 3));
+      } else if (e_ok) {
+        const int r16 = ln & 15;
+#pragma unroll 1
+        for (int row = ln >> 4; row < 16 && 16 * half + row < cnt; row += 4) yr[(int64_t)row * a.wld + r16] = ol[row * kOutStride + r16];
+      }
+    }
+    if (l0 + 2 * L < n) place_v(l0 + 2 * L);
+    f = fn;
+    fh = fhn;
+    __syncthreads();
+  }
+  int rows = D, step = E;
+  asm volatile("" : "+s"(rows), "+s"(step));                     // (no addresses of 16 rows held over the loop)
+  if (e_ok)
+#pragma unroll
+    for (int t = 0; t < HT; ++t)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
+}
+
+// Keys of up to 64, operands of fp32: the chunks of a request in turn, a wave per (request, head, 16 columns of S) with nothing shared: four waves a workgroup for the
 // sake of their common loads.  S [NP x 16] stays in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, which is
 // also how the right-hand operand of a product over the rows is held, so S, R = V - e^b K S and U go from sums into products
 // without moving; v is convolved in its place by the lane that needs it, from raw inputs in the wave's own LDS.  Left-hand operands
 // come straight into registers in the order they are used, not through LDS, the next chunk's into the registers that this chunk has
-// just read.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.
-template <typename T, int NP, int W>
-__global__ void __launch_bounds__(256, W) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
-  constexpr int L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
+// just read.  Results leave by way of the wave's LDS; nothing is shared between waves, so there are no barriers.  Half the
+// products of keys of 128 leave the two barriers and the exchange of delta_chunk_walk_kernel nothing to cover them with: 32 heads of 64 x 64,
+// 1 request of 1000 rows 144 us, there 160; 1 of 4000 rows 456 / 531; 8 of 900 rows 212 / 236; 32 of 40 rows 95 / 97.
+template <typename T, int W>
+__global__ void __launch_bounds__(256, W) delta_chunk_walk_small_kernel(DeltaArgs a, int64_t max_chunks) {
+  constexpr int NP = kDeltaSmall, L = kRecChunk, NT = NP / 16, HALO = kRecHalo;
   __shared__ __attribute__((aligned(16))) T in_l[4][RowTile<T>::kElems];       // a wave's own: raw inputs of its convolution
   __shared__ __attribute__((aligned(16))) float o_l[4][L * kOutStride];         // ... results on their way out (token by token: its v)
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4;
@@ -843,7 +1228,7 @@ __global__ void __launch_bounds__(256, W) delta_chunk_walk_kernel(DeltaArgs a, i
   float* yo = a.work + t0 * a.wld + h * E + e0;
   // 16-byte pieces of the projection's and of the result's rows: everything starts on one
   const bool vec = wide && ((reinterpret_cast<uintptr_t>(p) | (uintptr_t)(a.ld * sizeof(T))) & 15) == 0 &&
-                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0 && a.ld < (1 << 24);
+                   ((reinterpret_cast<uintptr_t>(yo) | (uintptr_t)(a.wld * 4)) & 15) == 0;
 
   // raw inputs of the convolution, tokens 16 j + 4 kq - HALO + i of the chunk at l0 > 0
   RowTile<T> tile;
@@ -1154,14 +1539,15 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((delta_chunk_operands_kernel<T, NP>), dim3((unsigned)chunks, (unsigned)a.G, rec_head_splits(chunks * a.G, a.H / a.G)), dim3(256), 0, s, a);
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
   const dim3 grid(rec_walk_blocks(a.batch * a.G, members));
-  if constexpr (NP <= 64)                                        // (NP 128: twice the operands, no second workgroup a CU)
-    if (a.batch * a.G * members > 256) {
-      // more workgroups than CUs: two a CU, at the price of 40 spilled registers (32 heads of 64 x 64, one / two a CU, whole call: 64 requests
-      // of 64 rows 226 / 202 us; 4 requests of 96 rows, 128 workgroups: 52 / 58)
-      hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 2>), grid, dim3(256), 0, s, a, chunks);
-      return;
-    }
-  hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 1>), grid, dim3(256), 0, s, a, chunks);
+  if constexpr (NP > kDeltaSmall) {
+    hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), grid, dim3(512), 0, s, a, chunks);
+  } else if (a.batch * a.G * members > 256) {
+    // more workgroups than CUs: two a CU, at the price of 40 spilled registers (32 heads of 64 x 64, one / two a CU, whole call: 64 requests
+    // of 64 rows 226 / 202 us; 4 requests of 96 rows, 128 workgroups: 52 / 58)
+    hipLaunchKernelGGL((delta_chunk_walk_small_kernel<T, 2>), grid, dim3(256), 0, s, a, chunks);
+  } else {
+    hipLaunchKernelGGL((delta_chunk_walk_small_kernel<T, 1>), grid, dim3(256), 0, s, a, chunks);
+  }
 }
 
 // gate and norm; 16-byte accesses where a head is a power of two of pieces and everything starts on one

@@ -30,6 +30,9 @@ __device__ __forceinline__ RecPlace rec_place(int units, int members) {
 // Request at place `pos` of a launch: the longest first, so that none starts late; those behind the first `firsts` (which have a
 // CU each) from the shortest up, so that the ones that come to a long one's CU are short.  4 requests of 1330, 2034, 1599 and 2303 rows, two
 // workgroups a CU: in their order the second and the fourth share CUs (walk 412 us, so placed 345).  A whole wave asks.
+__device__ __forceinline__ int rec_first_requests(int batch, int per_request) {       // (workgroups of a request; more than two a CU: all from the longest down)
+  return batch * (int64_t)per_request > 512 ? batch : min(batch, (256 + per_request - 1) / per_request);
+}
 __device__ __forceinline__ int rec_by_length(const int32_t* q_len, int batch, int pos, int firsts) {
   if (batch > 64) return pos;
   const int lane = threadIdx.x & 63, n = lane < batch ? q_len[lane] : 0;
@@ -203,47 +206,51 @@ template <typename T, int TOKENS = kRecChunk> struct RowTile {
   static constexpr int kLoads = (kRows * kPerRow + 63) / 64;
   static constexpr int kStride = sizeof(T) == 2 ? 24 : 20;          // elements of T between rows in LDS
   static constexpr int kElems = kRows * kStride;
-  u32x4 v[kLoads];
-  // rows l0 - halo .. l0 + TOKENS - 1 of `p` (row 0 = the portion's first), row n - 1 in place of those behind it; l0 > 0, rows
-  // of less than 2^26 bytes
+  uint4 v[kLoads];
+  // rows l0 - halo .. l0 + TOKENS - 1 of `p` (row 0 = the portion's first), zeros behind row n - 1; l0 > 0
   __device__ __forceinline__ void fetch(const T* p, int64_t ld, int l0, int n, int lane) {
+#pragma unroll
+    for (int u = 0; u < kLoads; ++u) {
+      const int it = u * 64 + lane, row = it / kPerRow, l = l0 - kRecHalo + row;
+      v[u] = uint4{0u, 0u, 0u, 0u};
+      if (row < kRows && l < n) v[u] = *reinterpret_cast<const uint4*>(p + (int64_t)l * ld + it % kPerRow * (16 / (int)sizeof(T)));
+    }
+  }
+  // ... row n - 1 in place of those behind it, rows of less than 2^26 bytes: nothing is written to the registers but by the load, and the
+  // addresses are an offset of 32 bits a lane
+  __device__ __forceinline__ void fetch_clamped(const T* p, int64_t ld, int l0, int n, int lane) {
     const int row0 = min(l0 - kRecHalo, n - 1), last = min(kRows, n - row0) - 1;       // (0 <= row0 <= row0 + last < n, also for l0 behind the portion)
     const char* first = reinterpret_cast<const char*>(p + (int64_t)row0 * ld);
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
       const int it = u * 64 + lane;
-      v[u] = *reinterpret_cast<const u32x4*>(first + ((uint32_t)min(it / kPerRow, last) * (uint32_t)(ld * sizeof(T)) + (uint32_t)(it % kPerRow) * 16u));
+      if ((u + 1) * 64 <= kRows * kPerRow || it < kRows * kPerRow)
+        v[u] = *reinterpret_cast<const uint4*>(first + ((uint32_t)min(it / kPerRow, last) * (uint32_t)(ld * sizeof(T)) + (uint32_t)(it % kPerRow) * 16u));
     }
   }
   __device__ __forceinline__ void place(T* lds, int lane) const {
 #pragma unroll
     for (int u = 0; u < kLoads; ++u) {
       const int it = u * 64 + lane, row = it / kPerRow;
-      if (row < kRows) *reinterpret_cast<u32x4*>(lds + row * kStride + it % kPerRow * (16 / (int)sizeof(T))) = v[u];
+      if (row < kRows) *reinterpret_cast<uint4*>(lds + row * kStride + it % kPerRow * (16 / (int)sizeof(T))) = v[u];
     }
   }
 };
 
-// A wave's 32 x 16 results (lane (r16, kq): rows 16 i + 4 kq + r of column r16) to rows in memory, 16 bytes a lane by way of its LDS
-constexpr int kOutStride = 20;            // floats between rows in LDS
-__device__ __forceinline__ void rec_place_tile(const f32x4 (&o)[2], float* lds, int lane) {
+constexpr int kOutStride = 20;            // floats between rows of a wave's results in LDS, on their way to rows in memory 16 bytes a lane
+// ... of its 32 x 16 results (lane (r16, kq): rows 16 i + 4 kq + r of column r16)
+__device__ __forceinline__ void rec_store_tile(const f32x4 (&o)[2], float* lds, float* y, int64_t ld, int lane) {
   const int r16 = lane & 15, kq = lane >> 4;
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int r = 0; r < 4; ++r) lds[(16 * i + 4 * kq + r) * kOutStride + r16] = o[i][r];
-}
-__device__ __forceinline__ void rec_store_tile(const float* lds, float* y, int64_t ld, int lane) {
   __builtin_amdgcn_wave_barrier();
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 16 * i + (lane >> 2);
     *reinterpret_cast<f32x4*>(y + (int64_t)row * ld + 4 * (lane & 3)) = *reinterpret_cast<const f32x4*>(lds + row * kOutStride + 4 * (lane & 3));
   }
-}
-__device__ __forceinline__ void rec_store_tile(const f32x4 (&o)[2], float* lds, float* y, int64_t ld, int lane) {
-  rec_place_tile(o, lds, lane);
-  rec_store_tile(lds, y, ld, lane);
 }
 
 }  // namespace semipd

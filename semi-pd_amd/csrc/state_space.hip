@@ -318,10 +318,11 @@ __global__ void __launch_bounds__(64) ssm_scan_kernel(SsmArgs a) {
 // Bound: token by token a step is a chain of LDS reads, 64 multiply-adds and lane sums (1.0 us of a wave's time; 7262 tokens of 4
 // requests, 128 heads of 128 x 64: 2394 us + 322 of preparation through fp32 work rows).  In chunks on the fp32 matrix pipe, a wave all
 // rows of 16 columns: 560 us (140 products of 32 cycles a wave and chunk, 38 % of the SIMD cycles, waiting for its operands in between).
-// Here 335: per wave and chunk 48 products of 16 cycles, 6 of 32 and 340 vector instructions (pieces of S 88, convolution 110), of which
+// Here 325: per wave and chunk 48 products of 16 cycles, 6 of 32 and 340 vector instructions (pieces of S 88, convolution 110), of which
 // a SIMD takes one in 4 cycles from two waves or more but only one in 8 from one; LDS reads 22 % of its cycles.  What that took: C and B^T
 // once a workgroup through LDS (24 KB each; straight into registers every wave reads them again), two waves a column block with half the
-// rows each (four a SIMD instead of two: one request of 2303 rows 265 -> 235), requests placed by length (412 -> 345).  Operands 77.
+// rows each (four a SIMD instead of two: one request of 2303 rows 265 -> 235), requests placed by length (412 -> 345), and the waits of a rare path kept in
+// it (345 -> 325).  Operands 77.
 // Chunks of 32 and not 64: the same products with S, half the ones inside a chunk, half the LDS.
 // Elements of the operands of one (chunk, group), counted in fp32: C and B^T in three planes of bf16 each, left-hand operands of 16 x 16 x 32
 // products in the order in which they are held, [tile][lane][8] (see rec_split8; tiles of C: 16 tokens x 32 rows of S, of B^T: 16 rows x
@@ -497,8 +498,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
   const int eblocks = (E + 63) / 64, members = per * eblocks;
   const RecPlace at = rec_place((int)a.batch * G, members);
   if (at.unit < 0) return;
-  const int per_request = G * members, firsts = 2 * 256 >= (int)a.batch * per_request ? (256 + per_request - 1) / per_request : (int)a.batch;
-  const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, min(firsts, (int)a.batch));
+  const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, rec_first_requests((int)a.batch, G * members));
   const int64_t first_pos = a.seq_lens[b] - a.q_len[b], t0 = a.q_start[b];
   const int n = a.q_len[b];
   if (n <= 0 || first_pos < 0) return;
@@ -536,7 +536,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
   auto fetch_x = [&](int l0) {
     int ln = lane;
     asm volatile("" : "+v"(ln));                                 // (addresses made where they are used, not held over the loop)
-    if (vec) tile.fetch(p, a.ld, l0 + 16 * half, n, ln);
+    if (vec) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
   };
   // x of this lane's tokens 16 half + 4 kq + s, zero behind the portion; taps that the layer does not have see zeros
   auto convolve = [&](const float (&raw)[HALO + 4], int cnt, f32x4& x, bool& bad) {
@@ -756,6 +756,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
       for (int t = 0; t < HT; ++t)
 #pragma unroll
         for (int r = 0; r < 4; ++r) S[t][r] = e_ok && row0 + 16 * t + r < rows ? st[(row0 + 16 * t + r) * step] : 0.f;
+      __builtin_amdgcn_s_waitcnt(0x0f70);                        // (vmcnt(0) here, or the other path waits for what it has in flight where they join)
       __builtin_amdgcn_sched_barrier(0);
     }
     // the next chunk's x

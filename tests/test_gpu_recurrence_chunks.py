@@ -285,6 +285,17 @@ def test_delta_rule_in_chunks(dtype, H, G, D, E, taps, lens):
         torch.testing.assert_close(last[b].to(F64), tail, rtol=0, atol=0)
 
 
+@pytest.mark.parametrize("D", [72, 128])
+def test_delta_rule_in_chunks_keeps_32_bits(D):
+    """As for the state-space recurrence: a few roundings of 2^-24 against 2^-17 of two pieces of 8 bits."""
+    H, G, E, lens = 4, 2, 64, [512]
+    w, rows, state, before = _delta_inputs(H, G, D, E, 4, lens, torch.float32, 8)
+    outs, after, _ = _delta_run(w, rows, state, before, [9], H, G, D, E)
+    want, S, _ = _delta_truth(w, rows[0], state[0], before[0], H, G, D, E)
+    assert float((after[0].to(F64) - S).norm() / S.norm()) < 2.0 ** -21
+    assert float((outs[0].to(F64) - want).norm() / want.norm()) < 2.0 ** -20
+
+
 def test_delta_rule_in_chunks_repeated_keys():
     """One key for all tokens, written in full (beta near 1) and kept (decay near 1): the system to invert is as far from the identity as
     it gets, and every token must replace what the one in front of it wrote."""
