@@ -89,8 +89,18 @@ __device__ __forceinline__ void prompt_rows_one_by_one(const LocalAttnArgs& a, i
   }
 }
 
-template <typename T, int D, int E, int NW, int KT, bool SIG>
-__global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnArgs a, int hw) {
+// How the kv heads and tiles of a launch go to the 8 XCDs: 2^shift XCDs share `heads` heads, `tiles` tiles of a head each
+struct PromptShare {
+  uint32_t shift, heads, tiles;
+};
+__host__ __device__ inline PromptShare prompt_share(int G, uint32_t n_tiles) {
+  const int pow2 = G & -G, groups = pow2 < 8 ? pow2 : 8;          // (of XCDs)
+  const uint32_t shift = groups == 8 ? 0 : groups == 4 ? 1 : groups == 2 ? 2 : 3;
+  return PromptShare{shift, (uint32_t)(G / groups), (n_tiles + (1u << shift) - 1) >> shift};
+}
+
+template <typename T, int D, int E, int NW, int KT, int W, bool SIG>
+__global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnArgs a, int hw) {
   constexpr int NT = 64 * NW, KU = KT / 32;                     // KT: keys a step
   constexpr int KB = D * 2, VB = E * 2, CK = D / 8, CV = E / 8;  // bytes and 16-byte chunks of a row
   constexpr int NK = KT * CK / NT, NV = KT * CV / NT;          // chunks a thread stages
@@ -100,16 +110,19 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   uint8_t* const k_lds = lds;                                   // [2][KT][KB]
   uint8_t* const v_lds = lds + 2 * KT * KB;                     // [2][KT][VB]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
-  // Workgroup -> (kv head, tile, heads of the group), the last fastest, an XCD walking a contiguous range of items: the workgroups
-  // that read the same K and V rows run next to each other on one L2.  Tiles from the last (most keys) to the first.
+  // Workgroup -> (kv head, tile, heads of the group), the last fastest.  An XCD (workgroup ids go round the 8) has kv heads of its own, or
+  // shares them with the fewest others, every so many tiles its own: workgroups that read the same K and V rows run next to each other
+  // on one L2, and every XCD has as many long tiles.  Tiles from the last (most keys) to the first.  A contiguous range of all items an
+  // XCD gave the one with the ends of the longest prompts up to three times the work: 32 heads over 2 of 128, values of 256, 1 prompt
+  // of 7000 tokens 1352 -> 776 us (whole call), 4 of 1900 389 -> 310.
   // (32 bits and shifts: with 64-bit quotients here and in the search for the request 20 tokens took 8.3 us for 7.4)
   const int hw_shift = 31 - __builtin_clz(hw), shift = 31 - __builtin_clz(32 * NW) - hw_shift, rows_wg = 1 << shift;      // (hw: a power of two)
   const uint32_t rep = a.H / a.G, sets = (rep + hw - 1) >> hw_shift, n_tiles = (uint32_t)a.n_tiles;
-  const uint32_t item = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-  if (item >= n_tiles * a.G * sets) return;
-  const uint32_t of_set = item / sets;
-  const int set = (int)(item - of_set * sets), gk = (int)(of_set / n_tiles);
-  const uint32_t tile_id = n_tiles - 1 - (of_set - gk * n_tiles);
+  const PromptShare share = prompt_share(a.G, n_tiles);
+  const uint32_t of_set = (blockIdx.x >> 3) / sets, of_head = of_set / share.tiles, tile_at = (of_set - of_head * share.tiles) << share.shift | ((blockIdx.x & 7) & ((1 << share.shift) - 1));
+  const int set = (int)((blockIdx.x >> 3) - of_set * sets), gk = (int)(((blockIdx.x & 7) >> share.shift) * share.heads + of_head);
+  if (tile_at >= n_tiles || of_head >= share.heads) return;
+  const uint32_t tile_id = n_tiles - 1 - tile_at;
   int b = -1;
   int q0 = 0;
   {
@@ -188,10 +201,11 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   const int n_first = keep < key_lo ? keep : key_lo;
   const int first_steps = (n_first + KT - 1) / KT, steps = first_steps + (key_hi - key_lo) / KT + 1;
   const int32_t* row = a.req_to_token + a.req_pool_indices[b] * a.r2t_stride;
-  const T* kp = (const T*)a.k_pool + (int64_t)gk * D;
-  const T* vp = (const T*)a.v_pool + (a.v_shared ? 0 : (int64_t)gk * E);
   const int kr0 = tid / CK, kc = tid % CK, vr0 = tid / CV, vc = tid % CV;      // this thread's chunks: rows kr0 + i NT / CK, chunk kc
-  int k_slot[NK] = {}, v_slot[NV] = {};
+  const char* kp = (const char*)((const T*)a.k_pool + (int64_t)gk * D + kc * 8);
+  const char* vp = (const char*)((const T*)a.v_pool + (a.v_shared ? 0 : (int64_t)gk * E) + vc * 8);
+  const uint32_t k_row = (uint32_t)a.k_ld * 2u, v_row = (uint32_t)a.v_ld * 2u;       // (bytes between rows: 32 bits, see prompt_attention)
+  uint32_t k_slot[NK] = {}, v_slot[NV] = {};
   u32x4 kv[NK], vv[NV];
   auto load_slots = [&](int it) {
     const bool first = it < first_steps;
@@ -203,9 +217,9 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   };
   auto load_rows = [&]() {
 #pragma unroll
-    for (int i = 0; i < NK; ++i) kv[i] = *reinterpret_cast<const u32x4*>(kp + (int64_t)k_slot[i] * a.k_ld + kc * 8);
+    for (int i = 0; i < NK; ++i) kv[i] = *reinterpret_cast<const u32x4*>(kp + (uint64_t)k_slot[i] * k_row);
 #pragma unroll
-    for (int i = 0; i < NV; ++i) vv[i] = *reinterpret_cast<const u32x4*>(vp + (int64_t)v_slot[i] * a.v_ld + vc * 8);
+    for (int i = 0; i < NV; ++i) vv[i] = *reinterpret_cast<const u32x4*>(vp + (uint64_t)v_slot[i] * v_row);
   };
   auto store_rows = [&](int buf) {
 #pragma unroll
@@ -252,6 +266,15 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
 #pragma unroll
         for (int u = 0; u < KU; ++u) s[u] = Mfma<T>::mma(as_frag<T>(kf[u]), as_frag<T>(qf[ks]), s[u]);
       }
+      // rows of K three products ahead (left alone, they are read one at a time, the latency of LDS behind each: 1116 cycles a step of a
+      // wave for these, so 834)
+      __builtin_amdgcn_sched_group_barrier(0x100, 3 * KU, 0);
+#pragma unroll
+      for (int i = 0; i < D / 16 - 3; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, KU, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, KU, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, 3 * KU, 0);
       if (capped_scores)
 #pragma unroll
         for (int u = 0; u < KU; ++u)
@@ -396,7 +419,7 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
 
 // true: launched.  Head sizes 64 / 64, 64 / 128, 128 / 128, 128 / 256 (sigmoid weights: 64 / 64, 128 / 128), a positive scale, 16-bit
 // types, everything aligned as local_attention_mfma_kernel wants it.
-template <typename T, int D, int E, int NW, int KT, bool SIG>
+template <typename T, int D, int E, int NW, int KT, int W, bool SIG>
 static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   const int rep = a.H / a.G;
   // heads of a group in a workgroup: the largest power of two that divides them, or the next one above them (the last set's waves are not all
@@ -412,19 +435,20 @@ static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   a.n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
   constexpr size_t tiles = 2 * KT * (size_t)(D + E) * 2, epilogue = NW * 32 * (size_t)(E * 2 + 16), bytes = tiles > epilogue ? tiles : epilogue;
   static std::atomic<uint64_t> done{0};
-  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
-  const int64_t items = a.n_tiles * a.G * ((rep + hw - 1) / hw);
-  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, SIG>), dim3((unsigned)((items + 7) / 8 * 8)), dim3(64 * NW), bytes, s, a, hw);
+  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, W, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
+  const PromptShare share = prompt_share(a.G, (uint32_t)a.n_tiles);
+  const int64_t blocks = 8ll * share.heads * share.tiles * ((rep + hw - 1) / hw);
+  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, W, SIG>), dim3((unsigned)blocks), dim3(64 * NW), bytes, s, a, hw);
   return 0;
 }
 template <typename T>
 static bool prompt_attention(const LocalAttnArgs& a, hipStream_t s, int& rc) {
   const bool sig = a.sigmoid != 0;
-  if (!(a.scale > 0.f)) return false;
-  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, false>(a, s);
-  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, false>(a, s);
-  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, false>(a, s);
-  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, false>(a, s);
+  if (!(a.scale > 0.f) || a.k_ld <= 0 || a.v_ld <= 0 || a.k_ld >= (1ll << 31) || a.v_ld >= (1ll << 31)) return false;
+  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, 2, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, 2, false>(a, s);
+  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, 2, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, 2, false>(a, s);
+  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, 2, false>(a, s);
+  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, 2, false>(a, s);
   else return false;
   return true;
 }

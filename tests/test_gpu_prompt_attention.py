@@ -166,7 +166,8 @@ def test_largest_weight_of_every_32_keys_is_not_rounded(dtype, D):
 
 # (requests: the scalar search and the one by lanes, whole and part waves of them; heads: one, two or four of a group in a workgroup)
 @pytest.mark.parametrize("requests", [8, 9, 64, 65, 131])
-@pytest.mark.parametrize("H,G,D,E", [(7, 1, 64, 64), (6, 2, 128, 128), (3, 3, 64, 64), (14, 2, 64, 128), (11, 1, 128, 256)])
+@pytest.mark.parametrize("H,G,D,E", [(7, 1, 64, 64), (6, 2, 128, 128), (3, 3, 64, 64), (14, 2, 64, 128), (11, 1, 128, 256), (8, 4, 64, 64),
+                                     (8, 8, 128, 128), (24, 12, 64, 64)])
 def test_prompt_attention_of_many_requests(requests, H, G, D, E):
     """Short uneven prompts, some without a row in the launch, some behind cached tokens."""
     from semi_pd_amd import ops
