@@ -123,40 +123,33 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
   const int set = (int)((blockIdx.x >> 3) - of_set * sets), gk = (int)(((blockIdx.x & 7) >> share.shift) * share.heads + of_head);
   if (tile_at >= n_tiles || of_head >= share.heads) return;
   const uint32_t tile_id = n_tiles - 1 - tile_at;
-  int b = -1;
-  int q0 = 0;
+  // Its request: 64 at a time, a lane each, with all that is known of them in one round trip
+  int b = -1, q0 = 0, qn = 0, base_pos = 0;
+  int64_t t0 = 0, pool_row = 0;
   {
     int left = (int)tile_id;
-    if (a.batch <= 8) {                                          // eight lengths in a round trip
-      int32_t n[8];
+    for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 64) {
+      const int rq = min(rq0 + lane, (int)a.batch - 1);
+      const int n = a.q_len[rq], len = (int)a.seq_lens[rq], at = a.q_start[rq];
+      const int64_t in_pool = a.req_pool_indices[rq];
+      const int tiles = rq0 + lane < (int)a.batch ? (max(n, 0) + rows_wg - 1) >> shift : 0;
+      int upto = tiles;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) n[u] = u < (int)a.batch ? a.q_len[u] : 0;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int tiles = (n[u] + rows_wg - 1) >> shift;
-        if (b < 0 && left < tiles) {
-          b = u;
-          q0 = left << shift;
-        }
-        if (b < 0) left -= tiles;
+      for (int d = 1; d < 64; d <<= 1) {
+        const int below = __shfl_up(upto, d, 64);
+        if (lane >= d) upto += below;
       }
-    } else {                                                     // 64 of them, a lane each (eight at a time 96 requests of 300 tokens, 16 heads of 128: 229 us for 148)
-      for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 64) {
-        const int tiles = rq0 + lane < (int)a.batch ? (max(a.q_len[rq0 + lane], 0) + rows_wg - 1) >> shift : 0;
-        int upto = tiles;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-          const int below = __shfl_up(upto, d, 64);
-          if (lane >= d) upto += below;
-        }
-        const uint64_t past = __ballot(left < upto);
-        if (past != 0) {
-          const int first = __builtin_ctzll(past);
-          b = rq0 + first;
-          q0 = (left - (__shfl(upto, first, 64) - __shfl(tiles, first, 64))) << shift;
-        } else {
-          left -= __shfl(upto, 63, 64);
-        }
+      const uint64_t past = __ballot(left < upto);
+      if (past != 0) {
+        const int first = __builtin_ctzll(past);
+        b = rq0 + first;
+        q0 = (left - (__builtin_amdgcn_readlane(upto, first) - __builtin_amdgcn_readlane(tiles, first))) << shift;
+        qn = __builtin_amdgcn_readlane(n, first);
+        base_pos = __builtin_amdgcn_readlane(len, first) - qn;
+        t0 = __builtin_amdgcn_readlane(at, first);
+        pool_row = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)in_pool, first) | (int64_t)__builtin_amdgcn_readlane((int)(in_pool >> 32), first) << 32;
+      } else {
+        left -= __builtin_amdgcn_readlane(upto, 63);
       }
     }
   }
@@ -166,8 +159,6 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
   const int hg = set * hw + (wave & (hw - 1));                  // head of the group (the last set may not be full)
   const bool h_ok = hg < (int)rep;
   const int h = gk * (int)rep + (h_ok ? hg : (int)rep - 1);
-  const int qn = a.q_len[b], base_pos = (int)(a.seq_lens[b] - qn);
-  const int64_t t0 = a.q_start[b];
   const int keep = a.window > 0 ? a.keep_first : 0;
   const int wg_last = min(q0 + rows_wg, qn) - 1;
   const int key_lo = (int)range_lo(a, base_pos + q0), key_hi = base_pos + wg_last;
@@ -200,7 +191,7 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
   // the walk: the kept first positions in front of the tile's range, then the range; steps of 64 keys, each within one of the two
   const int n_first = keep < key_lo ? keep : key_lo;
   const int first_steps = (n_first + KT - 1) / KT, steps = first_steps + (key_hi - key_lo) / KT + 1;
-  const int32_t* row = a.req_to_token + a.req_pool_indices[b] * a.r2t_stride;
+  const int32_t* row = a.req_to_token + pool_row * a.r2t_stride;
   const int kr0 = tid / CK, kc = tid % CK, vr0 = tid / CV, vc = tid % CV;      // this thread's chunks: rows kr0 + i NT / CK, chunk kc
   const char* kp = (const char*)((const T*)a.k_pool + (int64_t)gk * D + kc * 8);
   const char* vp = (const char*)((const T*)a.v_pool + (a.v_shared ? 0 : (int64_t)gk * E) + vc * 8);
