@@ -405,7 +405,14 @@ def _takes_tiled_gemm(x: torch.Tensor, weight: torch.Tensor) -> bool:
     rows = x.shape[0]
     if ops.STREAM_LINEAR_DENSE_MAX_ROWS < rows <= GEMM_TALL_MAX_ROWS:
         return not ops.dense_gemm_is_tuned(weight) and ops.gemm_tall_is_supported(x, weight)
-    return rows > GEMM_TALL_MAX_ROWS and ops.tall_preferred(weight, rows) and ops.gemm_tall_is_supported(x, weight)
+    return rows > GEMM_TALL_MAX_ROWS and _prefers_tiled_gemm(weight, rows) and ops.gemm_tall_is_supported(x, weight)
+
+
+def _prefers_tiled_gemm(weight: torch.Tensor, rows: int, fuse_silu_mul: bool = False) -> bool:
+    """Prefill-sized batch: what was timed at start-up where it was, else by how full the chip is."""
+    if ops.dense_gemm_is_tuned(weight):
+        return ops.tall_preferred(weight, rows, fuse_silu_mul=fuse_silu_mul)
+    return ops.tiled_gemm_fills_chip(weight.shape[0], weight.shape[1], rows, fuse_silu_mul)
 
 
 def gate_up_silu(x: torch.Tensor, gate_up_proj: "MergedColumnParallelLinear", act_fn) -> torch.Tensor:
@@ -423,7 +430,7 @@ def gate_up_silu(x: torch.Tensor, gate_up_proj: "MergedColumnParallelLinear", ac
         return ops.gemm_tall(x, gate_up_proj.weight, fuse_silu_mul=True)   # SiLU * mul in the GEMM's epilogue
     if (_STREAM_LINEAR["enabled"] and gate_up_proj.quant_config is None and gate_up_proj.bias is None
             and isinstance(act_fn, SiluAndMul) and x.dim() == 2 and x.shape[0] > GEMM_TALL_MAX_ROWS
-            and ops.tall_preferred(gate_up_proj.weight, x.shape[0], fuse_silu_mul=True)
+            and _prefers_tiled_gemm(gate_up_proj.weight, x.shape[0], fuse_silu_mul=True)
             and ops.gemm_tall_is_supported(x, gate_up_proj.weight, fuse_silu_mul=True)):
         # prefill-sized batch: the tiled GEMM with the SiLU epilogue beat the library's winner + silu_and_mul on this share
         w = gate_up_proj.weight

@@ -528,6 +528,28 @@ def tall_preferred(weight: torch.Tensor, rows: int, fuse_silu_mul: bool = False)
     return best[1]
 
 
+def tiled_gemm_fills_chip(n: int, k: int, rows: int, fuse_silu_mul: bool = False) -> bool:
+    """Is gemm_tall the better choice for a prefill-sized batch of a layer that was not timed at start-up, on the whole chip?  Where its
+    256 x 256 tiles (256 x 128 columns of a merged gate and up) keep nearly all of the 256 CUs busy with rows that exist:
+      gate and up with SiLU in the epilogue (no [rows, 2 n] product to write and read again), from 0.8 of the chip's time: 28672 x 4096, 512
+        rows 104 -> 98 us, 1024 204 -> 187, 1400 (0.80) 281 -> 279, 2048 382 -> 370, 2600 573 -> 481; 0.68 (1560 rows) would be 339 -> 354;
+        16384 x 3072, 1024 rows 84 -> 77, 1833 155.5 -> 153, 2600 318 -> 216; 16384 x 2048, 850 rows 62 -> 54.
+      a long k (from 13824) cut into slices that fill one round, from 0.75 of its time: the library's own choice is a plain tiling for some
+        row counts, half the chip idle or less.  4096 x 14336, 512 rows 74 -> 63 us, 1024 109 -> 100, 1600 326 -> 162, 1833 175.5 -> 177;
+        3584 x 18944, 1024 rows 191 -> 143; 8192 x 28672, 512 rows 309 -> 192; 5120 x 13824, 1024 rows 125.5 -> 120, 1500 171 -> 175.  In two
+        rounds (4096 x 14336, 2300 rows) 214 -> 248; k of 8192 to 12288 (reduction and prologue weigh more) up to 10 % behind the library."""
+    if _DENSE_GEMM["cus"] not in (0, 256):
+        return False
+    row_tiles = -(-rows // 256)
+    if fuse_silu_mul:
+        tiles = row_tiles * -(-(n // 2) // 128)
+        return rows * (n // 2) >= 0.8 * -(-tiles // 256) * 256 * 256 * 128
+    if k < 13824:
+        return False
+    slices = min(256 // (row_tiles * -(-n // 256)), 8, _LINEAR_WS_BYTES // (4 * rows * n))
+    return rows * n * slices >= 0.75 * 256 * 256 * 256
+
+
 def dense_gemm_report() -> str:
     import ctypes as _C
     lib = _lib.load()
