@@ -4,12 +4,14 @@
 // whole row, values are its first 512 columns (absorbed formulation, models/deepseek_v2.py:633-706),
 // and all heads share it (MQA).  A workgroup owns (request, 16-head tile, kv split); its four waves
 // share one 32-token tile of latent rows in LDS, fetched from HBM exactly once per head tile:
-//   every wave:   S^T[token, head] = tile x Q^T          36 x v_mfma_f32_16x16x32 (A = ds_read_b128)
+//   wave (t, k half): S^T[16 t .. + 15, head] = tile x Q^T  9 x v_mfma_f32_16x16x32 (A = ds_read_b128), the halves added in LDS
 //   wave w:       O^T[128w..128w+127, head] += V^T P^T     8 x v_mfma_f32_16x16x32 (A = ds_read_b64_tr_b16)
-// The QK^T product is recomputed by each wave (4 x redundant) because the matrix pipes are idle
-// anyway: per tile a wave issues 44 MFMAs (~700 cycles) while the tile's 36.9 KB take ~3500 cycles of
-// the CU's share of HBM bandwidth.  Softmax bookkeeping is identical in the four waves, so no
-// cross-wave exchange is needed; the next tile is prefetched into registers during the MFMAs.
+// Softmax bookkeeping is identical in the four waves, so nothing else is exchanged.
+// Bound: the flight time of the rows (40 MB of 32 requests at 1.1 k tokens are 8.4 us of a copy's time): at one or two workgroups a CU
+// a tile in flight each does not cover it, so two are, in registers.  With all of S^T made by every wave (36 products and 36 KB
+// of LDS reads a wave and tile, Q in 72 registers) the second set of rows would spill.  16 heads, bf16 rows, whole call with the merge of
+// the splits: 32 requests at 1.1 k tokens 24.7 -> 21.8 us (kernel 21.5 -> 18), 1 at 300 19.4 -> 16.1, 160 at 3 k 138 -> 129; fp8 rows 26.6 -> 21.7,
+// 19.9 -> 16.2, 128 -> 102.
 //
 // Replaces _fwd_grouped_kernel_stage1 for Lk = 576 / Lv = 512
 // (layers/attention/triton_ops/decode_attention.py:234-390, BLOCK_DPE = 64 path).
@@ -57,7 +59,9 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
   constexpr int CPR = DK / 8;      // 72 16-byte chunks per row
   constexpr int NI = TOK * CPR / 256;  // 9 chunks per thread per tile
   constexpr int DTW = DV / 16 / 4;     // 8 d-tiles of 16 per wave
+  constexpr int KSW = KS / 2;          // k steps of S^T a wave
   __shared__ __attribute__((aligned(16))) uint8_t tile[TOK * RS];
+  __shared__ __attribute__((aligned(16))) f32x4 part[4][64];      // half sums of S^T: wave (token half, k half)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int c16 = lane & 15, q4 = lane >> 4;
@@ -82,14 +86,15 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
     return;
   }
 
-  // Q^T fragments (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
-  FragM qf[KS];
+  // Q^T fragments of this wave's k half (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
+  const int ks0 = (wave >> 1) * KSW;
+  FragM qf[KSW];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
+  for (int ks = 0; ks < KSW; ++ks) {
     qf[ks].u = make_uint4(0, 0, 0, 0);
     if (head_ok)
       qf[ks].u = *reinterpret_cast<const uint4*>(q + (int64_t)b * q_stride + (int64_t)(h0 + c16) * DK +
-                                                 ks * 32 + q4 * 8);
+                                                 (ks0 + ks) * 32 + q4 * 8);
   }
   f32x4 o_acc[DTW];
 #pragma unroll
@@ -99,55 +104,58 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
   const int32_t* idx_base = kv_indices + kv_start;
   const int n_tiles = (s_end - s_begin + TOK - 1) / TOK;
   using KVT = KVTraits<T, KV>;
-  int32_t idx[NI];
-  typename KVT::Raw reg[NI];
-  auto load_idx = [&](int ti) __attribute__((always_inline)) {
+  // Two tiles in flight, in two sets of registers; nothing of it is conditional (rows past the end: the last row, zeroed on its way into
+  // LDS), so that the wait for the older tile's rows leaves the younger one's in flight.
+  int32_t idx[2][NI];
+  typename KVT::Raw reg[2][NI];
+  auto load_idx = [&](int ti, int32_t (&idx)[NI]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int tok = s_begin + ti * TOK + (tid + i * 256) / CPR;
-      idx[i] = (ti < n_tiles && tok < s_end) ? idx_base[tok] : 0;
-    }
+    for (int i = 0; i < NI; ++i) idx[i] = idx_base[min(s_begin + ti * TOK + (tid + i * 256) / CPR, s_end - 1)];
   };
-  auto fetch = [&](int ti) __attribute__((always_inline)) {
+  auto fetch = [&](typename KVT::Raw (&to)[NI], const int32_t (&idx)[NI]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int item = tid + i * 256;
-      const int r = item / CPR, ch = item - r * CPR;
-      reg[i] = KVT::zero();  // rows past the end must be zero (0 * garbage could be NaN)
-      if (s_begin + ti * TOK + r < s_end) reg[i] = KVT::load8(kv_buf + (int64_t)idx[i] * kvbuf_stride + ch * 8);
-    }
+    for (int i = 0; i < NI; ++i) to[i] = KVT::load8(kv_buf + (int64_t)idx[i] * kvbuf_stride + (tid + i * 256) % CPR * 8);
   };
 
-  const uint8_t* krow = tile + c16 * RS + q4 * 16;                           // + t*16*RS + ks*64
+  const uint8_t* krow = tile + ((wave & 1) * 16 + c16) * RS + ks0 * 64 + q4 * 16;       // + ks*64
   const uint8_t* vrow = tile + (q4 * 4 + (c16 >> 2)) * RS + (c16 & 3) * 8 + wave * 256;  // + dt*32 (+16*RS)
 
-  load_idx(0);
-  fetch(0);
-  load_idx(1);
-  for (int ti = 0; ti < n_tiles; ++ti) {
+  // (memory answers in order: the slots of a tile are asked for in front of the rows of the tile before it)
+  load_idx(0, idx[0]);
+  load_idx(1, idx[1]);
+  fetch(reg[0], idx[0]);
+  load_idx(2, idx[0]);
+  fetch(reg[1], idx[1]);
+  auto step = [&](int ti, typename KVT::Raw (&rows)[NI], const int32_t (&after_next)[NI], int32_t (&behind)[NI]) __attribute__((always_inline)) {
     __syncthreads();  // every wave is done with the previous tile
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
       const int item = tid + i * 256;
       const int r = item / CPR, ch = item - r * CPR;
-      *reinterpret_cast<uint4*>(tile + r * RS + ch * 16) = KVT::expand(reg[i]);
+      uint4 v = KVT::expand(rows[i]);
+      if (s_begin + ti * TOK + r >= s_end) v = uint4{0u, 0u, 0u, 0u};      // (0 * garbage could be NaN)
+      *reinterpret_cast<uint4*>(tile + r * RS + ch * 16) = v;
     }
     __syncthreads();
-    if (ti + 1 < n_tiles) fetch(ti + 1);
-    load_idx(ti + 2);
+    load_idx(ti + 3, behind);
+    fetch(rows, after_next);
 
-    // ---- S^T = tile x Q^T (every wave, all 32 tokens x 16 heads) ----
+    // ---- S^T = tile x Q^T: a wave 16 of the tokens and half of k, the halves added by every wave ----
     f32x4 s_acc[2];
+    {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      s_acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
+      for (int ks = 0; ks < KSW; ++ks) {
         FragM a;
-        a.u = *reinterpret_cast<const uint4*>(krow + t * 16 * RS + ks * 64);
-        s_acc[t] = MfmaM<T>::mma(a, qf[ks], s_acc[t]);
+        a.u = *reinterpret_cast<const uint4*>(krow + ks * 64);
+        if (ks & 1) s1 = MfmaM<T>::mma(a, qf[ks], s1);
+        else s = MfmaM<T>::mma(a, qf[ks], s);
       }
+      part[wave][lane] = s + s1;
     }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 2; ++t) s_acc[t] = part[t][lane] + part[t + 2][lane];
     // ---- online softmax: lane = head c16, tokens t*16 + q4*4 + r ----
     const int base_tok = s_begin + ti * TOK;
     float mx = -INFINITY;
@@ -194,6 +202,12 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
           (__attribute__((address_space(3))) s16x4*)(vrow + 16 * RS + dt * 32));
       o_acc[dt] = MfmaM<T>::mma(a, pf, o_acc[dt]);
     }
+  };
+  for (int ti = 0;;) {
+    step(ti, reg[0], idx[0], idx[1]);
+    if (++ti >= n_tiles) break;
+    step(ti, reg[1], idx[1], idx[0]);
+    if (++ti >= n_tiles) break;
   }
 
   // ---- epilogue: wave w writes d in [128w, 128w+128) ----
