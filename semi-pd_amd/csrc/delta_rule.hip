@@ -9,7 +9,8 @@
 //
 //  * delta_prep_kernel: a workgroup per token, its waves taking the token's q, k and v heads in turn: convolution (inputs in
 //    front of the portion come from the state row), silu, unit norms, decay and beta -> an fp32 work row per token.
-//  * delta_conv_state_kernel: the last taps - 1 inputs of the portion (shifted in behind what the row held) -> state row.
+//  * delta_conv_state: the last taps - 1 inputs of the portion (shifted in behind what the row held) -> state row, by the first workgroups
+//    of delta_post_vec_kernel's launch or in delta_conv_state_kernel.
 //  * delta_scan_kernel: ONE WAVE per (request, head, block of columns); column j of S lives in the registers of DS adjacent
 //    lanes (D / DS rows each), so a step is two dot products over the lanes' rows, a 2-step lane reduction and one update
 //    of the column: dk = S^T k, dq = S^T q from the old S, then u = beta (v - g dk), o = g dq + u (k . q), S <- g S + k u
@@ -175,10 +176,8 @@ __global__ void __launch_bounds__(256) delta_prep_kernel(DeltaArgs a) {
 
 // ---------------------------------------------------------------------------------- the inputs the next portion looks back at
 template <typename T>
-__global__ void __launch_bounds__(256) delta_conv_state_kernel(DeltaArgs a) {
-  const int b = blockIdx.y;
+__device__ __forceinline__ void delta_conv_state(const DeltaArgs& a, int b, int c) {
   const int C = 2 * a.G * a.D + a.H * a.E;
-  const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= C) return;
   int64_t t0, n, first_pos;
   if (a.q_start == nullptr) {
@@ -202,6 +201,10 @@ __global__ void __launch_bounds__(256) delta_conv_state_kernel(DeltaArgs a) {
     else x = cs[(int64_t)(keep + l) * C + c];
     cs[(int64_t)s * C + c] = x;
   }
+}
+template <typename T>
+__global__ void __launch_bounds__(256) delta_conv_state_kernel(DeltaArgs a) {
+  delta_conv_state<T>(a, blockIdx.y, blockIdx.x * 256 + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------- the recurrence
@@ -1481,9 +1484,16 @@ __global__ void __launch_bounds__(256, W) delta_chunk_walk_small_kernel(DeltaArg
 // The same with 16-byte accesses: a head is taken by LP = E / 8 lanes (a power of two), 64 / LP heads per wave.  Bound by HBM: 7262
 // tokens of 32 heads of 128, 238 MB: 84 us -> 46.
 template <typename T, int LP>
-__global__ void __launch_bounds__(256) delta_post_vec_kernel(DeltaArgs a) {
+__global__ void __launch_bounds__(256) delta_post_vec_kernel(DeltaArgs a, int conv_blocks) {
+  // the first workgroups move the convolutions' inputs on, 256 channels of a request each: the others neither read nor write them (a
+  // launch of its own is 2.5 us)
+  if ((int)blockIdx.x < conv_blocks) {
+    const int per = (2 * a.G * a.D + a.H * a.E + 255) / 256;
+    delta_conv_state<T>(a, blockIdx.x / per, blockIdx.x % per * 256 + threadIdx.x);
+    return;
+  }
   const int lane = threadIdx.x & 63, sl = lane % LP, E = a.E;
-  const int64_t item = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / LP) + lane / LP;
+  const int64_t item = ((int64_t)(blockIdx.x - conv_blocks) * 4 + (threadIdx.x >> 6)) * (64 / LP) + lane / LP;
   const bool on = item < a.num_tokens * a.H;
   const int64_t t = on ? item / a.H : 0;
   const int h = on ? (int)(item % a.H) : 0;
@@ -1550,27 +1560,34 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   }
 }
 
-// gate and norm; 16-byte accesses where a head is a power of two of pieces and everything starts on one
+// gate and norm, and the convolutions' inputs moved on, both behind everything that reads them; in one launch unless the result may be
+// written over the inputs; 16-byte accesses where a head is a power of two of pieces and everything starts on one
 static int launch_delta_post(const DeltaArgs& a, int dtype, hipStream_t s) {
   const int lp = a.E / 8;
   const bool vec = dtype != SEMIPD_F32 && a.E % 8 == 0 && lp <= 64 && (lp & (lp - 1)) == 0 && a.gate_off % 8 == 0 && a.ld % 8 == 0 &&
                    a.out_ld % 8 == 0 && a.wld % 4 == 0 && a.o_off % 4 == 0 && aligned16(a.p) && aligned16(a.out) && aligned16(a.work) &&
                    aligned16(a.norm_w);
+  const int64_t gd = (int64_t)a.G * a.D, he = (int64_t)a.H * a.E, blocks = a.taps > 1 ? (2 * gd + he + 255) / 256 : 0;
+  auto apart = [&](int64_t off, int64_t n) { return rec_apart(a.p, off, n, a.ld, a.out, he, a.out_ld, a.num_tokens); };
+  const bool one = vec && apart(a.q_off, gd) && apart(a.k_off, gd) && apart(a.v_off, he);
+  if (blocks && !one)
+    SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)blocks, (unsigned)a.batch), dim3(256), 0, s, a));
   if (!vec) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_post_kernel<T>), dim3((unsigned)a.num_tokens), dim3(256), 0, s, a));
     return 0;
   }
   const int64_t items = a.num_tokens * a.H, per = 4 * (64 / lp);
-  const dim3 grid((unsigned)((items + per - 1) / per));
+  const int cb = (int)(one ? blocks * a.batch : 0);
+  const dim3 grid((unsigned)((items + per - 1) / per + cb));
   SEMIPD_DISPATCH_HALF(dtype, T, {
     switch (lp) {
-      case 1: hipLaunchKernelGGL((delta_post_vec_kernel<T, 1>), grid, dim3(256), 0, s, a); break;
-      case 2: hipLaunchKernelGGL((delta_post_vec_kernel<T, 2>), grid, dim3(256), 0, s, a); break;
-      case 4: hipLaunchKernelGGL((delta_post_vec_kernel<T, 4>), grid, dim3(256), 0, s, a); break;
-      case 8: hipLaunchKernelGGL((delta_post_vec_kernel<T, 8>), grid, dim3(256), 0, s, a); break;
-      case 16: hipLaunchKernelGGL((delta_post_vec_kernel<T, 16>), grid, dim3(256), 0, s, a); break;
-      case 32: hipLaunchKernelGGL((delta_post_vec_kernel<T, 32>), grid, dim3(256), 0, s, a); break;
-      default: hipLaunchKernelGGL((delta_post_vec_kernel<T, 64>), grid, dim3(256), 0, s, a); break;
+      case 1: hipLaunchKernelGGL((delta_post_vec_kernel<T, 1>), grid, dim3(256), 0, s, a, cb); break;
+      case 2: hipLaunchKernelGGL((delta_post_vec_kernel<T, 2>), grid, dim3(256), 0, s, a, cb); break;
+      case 4: hipLaunchKernelGGL((delta_post_vec_kernel<T, 4>), grid, dim3(256), 0, s, a, cb); break;
+      case 8: hipLaunchKernelGGL((delta_post_vec_kernel<T, 8>), grid, dim3(256), 0, s, a, cb); break;
+      case 16: hipLaunchKernelGGL((delta_post_vec_kernel<T, 16>), grid, dim3(256), 0, s, a, cb); break;
+      case 32: hipLaunchKernelGGL((delta_post_vec_kernel<T, 32>), grid, dim3(256), 0, s, a, cb); break;
+      default: hipLaunchKernelGGL((delta_post_vec_kernel<T, 64>), grid, dim3(256), 0, s, a, cb); break;
     }
   });
   return 0;
@@ -1666,17 +1683,10 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
   }
   if (chunks) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, if (k_dim <= 64) launch_delta_chunks<T, 64>(a, st); else launch_delta_chunks<T, 128>(a, st));
-    if (taps > 1)
-      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch),
-                                                         dim3(256), 0, st, a));
     if (launch_delta_post(a, dtype, st)) return SEMIPD_EDTYPE;
     return launch_status("delta_rule(chunks)");
   }
-  SEMIPD_DISPATCH_DTYPE(dtype, T, {
-    hipLaunchKernelGGL((delta_prep_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, st, a);
-    if (taps > 1)
-      hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch), dim3(256), 0, st, a);
-  });
+  SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_prep_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, st, a));
   // one wave per workgroup: the workgroups of a CU stage and walk their tokens independently, so the loads of one overlap
   // the arithmetic of the others
   const int threads = 64;

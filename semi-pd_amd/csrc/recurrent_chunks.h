@@ -53,6 +53,13 @@ inline unsigned rec_head_splits(int64_t items, int heads) {
   return (unsigned)(most < room ? most : room);
 }
 
+// Whether columns [off, off + n) of `rows` rows `ld` apart and the result's [rows, m] share no byte (elements of 2 bytes; the space from first
+// to last byte of each is taken as its own).
+inline bool rec_apart(const void* p, int64_t off, int64_t n, int64_t ld, const void* out, int64_t m, int64_t out_ld, int64_t rows) {
+  const uintptr_t a = (uintptr_t)p + 2 * off, b = (uintptr_t)out;
+  return a + 2 * ((rows - 1) * ld + n) <= b || b + 2 * ((rows - 1) * out_ld + m) <= a;
+}
+
 inline int64_t rec_max_chunks(int64_t num_tokens, int64_t batch) { return num_tokens / kRecChunk + batch; }
 
 // Chunk `idx` of the launch (request after request, each in chunks of 32 rows) -> request and chunk in it; a whole wave asks.

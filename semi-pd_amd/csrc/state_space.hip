@@ -11,7 +11,8 @@
 //  * ssm_prep_kernel: a workgroup per (tile of 32 tokens -- one token in small batches --, 1024 channels), four channels per
 //    thread with their taps in registers where alignment allows: convolution + bias + silu of the token's x | B | C channels (inputs in front
 //    of the portion come from the state row), dt and the decay -> an fp32 work row per token.
-//  * ssm_conv_state_kernel: the last taps - 1 inputs of the portion (shifted in behind what the row held) -> state row.
+//  * ssm_conv_state: the last taps - 1 inputs of the portion (shifted in behind what the row held) -> state row, by the first workgroups of
+//    ssm_post_vec_kernel's launch or in ssm_conv_state_kernel.
 //  * ssm_scan_kernel: ONE WAVE per (request, head, block of 64 / NS columns of S); a column of S lives in the registers of NS
 //    adjacent lanes, NPT rows each, so a step is one multiply-add per register for the update, one for the read-out, and a
 //    log2(NS)-step lane reduction.  B, C, x, dt and the decay of kStage tokens sit in LDS; the next stage's 16-byte pieces are
@@ -165,10 +166,8 @@ __global__ void __launch_bounds__(256) ssm_prep_kernel(SsmArgs a, int tile) {
 
 // ---------------------------------------------------------------------------------- the inputs the next portion looks back at
 template <typename T>
-__global__ void __launch_bounds__(256) ssm_conv_state_kernel(SsmArgs a) {
-  const int b = blockIdx.y;
+__device__ __forceinline__ void ssm_conv_state(const SsmArgs& a, int b, int c) {
   const int C = a.H * a.E + 2 * a.G * a.N;
-  const int c = blockIdx.x * 256 + threadIdx.x;
   if (c >= C) return;
   int64_t t0, n, first_pos;
   if (a.q_start == nullptr) {
@@ -190,6 +189,10 @@ __global__ void __launch_bounds__(256) ssm_conv_state_kernel(SsmArgs a) {
     else x = cs[(int64_t)(keep + l) * C + c];
     cs[(int64_t)s * C + c] = x;
   }
+}
+template <typename T>
+__global__ void __launch_bounds__(256) ssm_conv_state_kernel(SsmArgs a) {
+  ssm_conv_state<T>(a, blockIdx.y, blockIdx.x * 256 + threadIdx.x);
 }
 
 // ---------------------------------------------------------------------------------- the recurrence
@@ -824,10 +827,18 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
 // 86 = 5.5 TB/s; 32 rows 28 -> 7 us.
 constexpr int kPostPieces = 4;
 template <typename T>
-__global__ void __launch_bounds__(256) ssm_post_vec_kernel(SsmArgs a) {
+__global__ void __launch_bounds__(256) ssm_post_vec_kernel(SsmArgs a, int conv_blocks) {
   __shared__ float red[16];
+  // the first workgroups move the convolution's inputs on, 256 channels of a request each: the others neither read nor write them (a
+  // launch of its own is 2.5 us; whole call with / without it: 128 heads of 128 x 64, 8 requests of one token 23.8 / 21.1 us, 32 of them
+  // 61.0 / 59.0)
+  if ((int)blockIdx.x < conv_blocks) {
+    const int per = (a.H * a.E + 2 * a.G * a.N + 255) / 256;
+    if (blockIdx.y == 0) ssm_conv_state<T>(a, blockIdx.x / per, blockIdx.x % per * 256 + threadIdx.x);
+    return;
+  }
   const int gs = a.H * a.E / a.norm_groups;
-  const int64_t t = blockIdx.x, c0 = (int64_t)blockIdx.y * gs;
+  const int64_t t = blockIdx.x - conv_blocks, c0 = (int64_t)blockIdx.y * gs;
   const float* yr = a.work + t * a.wld + c0;
   const T* z = (const T*)a.p + t * a.ld + a.z_off + c0;
   float v[kPostPieces][8], sq = 0.f;
@@ -1086,18 +1097,23 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
   const int64_t gs = inner / norm_groups;
   const bool post8 = dtype != SEMIPD_F32 && gs % 8 == 0 && gs <= 8 * 256 * kPostPieces && z_off % 8 == 0 && ld % 8 == 0 && out_ld % 8 == 0 &&
                      work_ld % 4 == 0 && aligned16(proj) && aligned16(out) && aligned16(norm_w) && aligned16(work);
+  // ... and the convolution's inputs moved on, both behind everything that reads them; in one launch unless the result may be written over
+  // the inputs
   auto post = [&]() -> int {
-    const dim3 vgrid((unsigned)num_tokens, (unsigned)norm_groups);
-    if (post8) SEMIPD_DISPATCH_HALF(dtype, T, hipLaunchKernelGGL((ssm_post_vec_kernel<T>), vgrid, dim3(256), 0, s, a))
-    else SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a))
+    const int64_t blocks = taps > 1 ? (C + 255) / 256 : 0;
+    const bool one = post8 && rec_apart(proj, x_off, C, ld, out, inner, out_ld, num_tokens);
+    if (blocks && !one)
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), dim3((unsigned)blocks, (unsigned)batch), dim3(256), 0, s, a))
+    const int64_t moved = one ? blocks * batch : 0;
+    if (post8)
+      SEMIPD_DISPATCH_HALF(dtype, T, hipLaunchKernelGGL((ssm_post_vec_kernel<T>), dim3((unsigned)(num_tokens + moved), (unsigned)norm_groups),
+                                                        dim3(256), 0, s, a, (int)moved))
+    else
+      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_post_kernel<T>), dim3((unsigned)num_tokens), dim3(256), 0, s, a))
     return 0;
   };
   if (chunks) {
     SEMIPD_DISPATCH_DTYPE(dtype, T, if (state_size <= 64) launch_ssm_chunks<T, 64>(a, s); else launch_ssm_chunks<T, 128>(a, s));
-    if (taps > 1) {
-      const dim3 grid((unsigned)((C + 255) / 256), (unsigned)batch);
-      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), grid, dim3(256), 0, s, a));
-    }
     if (post()) return SEMIPD_EDTYPE;
     return launch_status("state_space(chunks)");
   }
@@ -1112,10 +1128,6 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
       else if (nit <= 8) hipLaunchKernelGGL((ssm_step_kernel<T, 8>), grid, dim3(256), bytes, s, a);
       else hipLaunchKernelGGL((ssm_step_kernel<T, 16>), grid, dim3(256), bytes, s, a);
     });
-    if (taps > 1) {
-      const dim3 cgrid((unsigned)((C + 255) / 256), (unsigned)batch);
-      SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), cgrid, dim3(256), 0, s, a));
-    }
     if (post()) return SEMIPD_EDTYPE;
     return launch_status("state_space(step)");
   }
@@ -1131,10 +1143,6 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     if (prep4) hipLaunchKernelGGL((ssm_prep_kernel<T, true>), pgrid, dim3(256), 0, s, a, tile);
     else hipLaunchKernelGGL((ssm_prep_kernel<T, false>), pgrid, dim3(256), 0, s, a, tile);
   });
-  if (taps > 1) {
-    const dim3 grid((unsigned)((C + 255) / 256), (unsigned)batch);
-    SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((ssm_conv_state_kernel<T>), grid, dim3(256), 0, s, a));
-  }
   // 16-byte staging reads: B, C and x of a token start on multiples of four floats
   const bool scan4 = work_ld % 4 == 0 && aligned16(work) && inner % 4 == 0 && state_size % 4 == 0 && v_dim % 4 == 0;
 #define SEMIPD_SSM_SCAN(NPT, NS)                                                                                              \

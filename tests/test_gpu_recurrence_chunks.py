@@ -471,3 +471,24 @@ def test_many_heads_of_a_group_in_chunks(kind):
     torch.testing.assert_close(got[0].view(-1, H, E)[:, others], clean[0].view(-1, H, E)[:, others], rtol=0, atol=0)
     torch.testing.assert_close(got[0][:at], clean[0][:at], rtol=1e-5, atol=1e-5)
     assert not bool(torch.isfinite(got[0].view(-1, H, E)[at:, 12]).any())
+
+
+@pytest.mark.parametrize("lens", [[40, 33, 64, 5], [1] * 6])
+@pytest.mark.parametrize("kind", ["state_space", "delta_rule"])
+def test_result_over_the_inputs(kind, lens, monkeypatch):
+    """A result written over columns that the convolution's state is taken from is the same, bit for bit, as one in a place of its own."""
+    from semi_pd_amd import ops
+    op, H, G, N, E = getattr(ops, kind), 8, 2, 32, 64
+    make, run = (_ssm_inputs, _ssm_run) if kind == "state_space" else (_delta_inputs, _delta_run)
+    w, rows, state, before = make(H, G, N, E, 4, lens, torch.bfloat16, 3)
+    first = [i % 2 * 9 for i in range(len(lens))]
+    args = (w, rows, state, before, first, H, G, N, E) + ((1,) if kind == "state_space" else ())
+    for decode in (False, True)[: 1 + (max(lens) == 1)]:
+        apart = run(*args, decode=decode)
+        col = H * E if kind == "state_space" else 2 * G * N
+        monkeypatch.setattr(ops, kind, lambda proj, *a: op(proj, *a, out=proj[:, col: col + H * E]))
+        over = run(*args, decode=decode)
+        monkeypatch.setattr(ops, kind, op)
+        for a, b in zip(apart, over):
+            for x, y in zip(a, b):
+                assert torch.equal(x, y)
