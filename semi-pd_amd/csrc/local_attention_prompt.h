@@ -18,8 +18,8 @@
 // cycles each) with five instructions around each.  Of the SIMD cycles of the batch below the vector unit is busy for 42 %, the matrix
 // pipe for 20 %, the LDS for about a third of its own; two waves a SIMD fill only part of each other's gaps (value rows of 256: 30, 19
 // and a third).  Against 16 rows a wave, steps of 32 keys (which read all of K and V from LDS for half the rows, and had four waves of
-// one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 109 us (505 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
-// 341 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.
+// one head): 7262 tokens in blocks of 1024, 32 / 8 heads of 128: 271 -> 97 us (565 TFLOP/s); 32 / 2 heads with value rows of 256: 1971 ->
+// 283 (steps of 32 keys there, eight waves: 64 would spill); 300 tokens behind 1000, 32 / 8 heads of 128: 76 -> 44; 8 x 40: 9.0 -> 8.6.
 // A fresh prompt of at most 32 tokens is one step of either, and its 32 x 64 products are four times those of the wave of 16 rows: 20
 // tokens 7.3 -> 7.4 us, 32 tokens 7.4 -> 7.9, with sigmoid weights 6.5 -> 7.1 and 6.6 -> 7.6 (behind 100 tokens 20 tokens are 12.4 -> 9.6;
 // how far a request reaches back is on the device, so the host cannot choose; leaving out a step's second 32 keys where there
@@ -99,8 +99,47 @@ __host__ __device__ inline PromptShare prompt_share(int G, uint32_t n_tiles) {
   return PromptShare{shift, (uint32_t)(G / groups), (n_tiles + (1u << shift) - 1) >> shift};
 }
 
-template <typename T, int D, int E, int NW, int KT, int W, bool SIG>
-__global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnArgs a, int hw) {
+// Place `at` of a launch's tiles by their keys, the most first -> request and tile in it (-1: past the last): tiles of 2^shift rows, up to 8
+// requests, a lane each (its tiles and the position of its first row).  Tile j of a request has u + j (mod period) tiles' rows of keys in
+// front of it, u those of the request's first row, period a block's (0: no blocks).  So the tiles of a request with at least x are counted
+// without a walk, and a lane counts them for each of up to 64 levels; within a level, request after request, neighbours next to each other.
+struct PromptTile {
+  int request, tile;
+};
+__device__ __forceinline__ PromptTile prompt_tile_by_keys(uint32_t at, int batch, int tiles, uint32_t pos, int shift, uint32_t period) {
+  const int lane = threadIdx.x & 63;
+  uint32_t u = pos >> shift, full = 0;
+  uint32_t rem = u + tiles, top = period;
+  if (period > 0) {
+    u %= period;
+    full = (u + tiles) / period;
+    rem = u + tiles - full * period;
+  } else {
+    for (int r = 0; r < batch; ++r) top = max(top, (uint32_t)__builtin_amdgcn_readlane((int)rem, r));
+  }
+  const int per = (int)((top + 63) >> 6), x = lane * per;         // (tiles' rows between levels)
+  int above = 0;                                                          // tiles with at least x in front
+  for (int r = 0; r < batch; ++r)
+    above += __builtin_amdgcn_readlane((int)full, r) * max((int)period - x, 0) + max(__builtin_amdgcn_readlane((int)rem, r) - x, 0) -
+             max(__builtin_amdgcn_readlane((int)u, r) - x, 0);
+  const int level = __builtin_popcountll(__ballot(above > (int)at)) - 1;
+  if (level < 0) return PromptTile{-1, 0};
+  int left = (int)at - (level < 63 ? __builtin_amdgcn_readlane(above, level + 1) : 0);
+  const int lo = level * per, wid = period > 0 ? min(per, (int)period - lo) : per;
+  const int skip = min(max((int)u - lo, 0), wid), mine = (int)full * wid + min(max((int)rem - lo, 0), wid) - skip;
+  int r = 0;
+  for (; r + 1 < batch; ++r) {
+    const int n = __builtin_amdgcn_readlane(mine, r);
+    if (left < n) break;
+    left -= n;
+  }
+  left += __builtin_amdgcn_readlane(skip, r);
+  const int block = left / wid;
+  return PromptTile{r, block * (int)period + lo + (left - block * wid) - __builtin_amdgcn_readlane((int)u, r)};
+}
+
+template <typename T, int D, int E, int NW, int KT, bool SIG>
+__global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnArgs a, int hw, int by_keys) {
   constexpr int NT = 64 * NW, KU = KT / 32;                     // KT: keys a step
   constexpr int KB = D * 2, VB = E * 2, CK = D / 8, CV = E / 8;  // bytes and 16-byte chunks of a row
   constexpr int NK = KT * CK / NT, NV = KT * CV / NT;          // chunks a thread stages
@@ -111,10 +150,10 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
   uint8_t* const v_lds = lds + 2 * KT * KB;                     // [2][KT][VB]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
   // Workgroup -> (kv head, tile, heads of the group), the last fastest.  An XCD (workgroup ids go round the 8) has kv heads of its own, or
-  // shares them with the fewest others, every so many tiles its own: workgroups that read the same K and V rows run next to each other
-  // on one L2, and every XCD has as many long tiles.  Tiles from the last (most keys) to the first.  A contiguous range of all items an
-  // XCD gave the one with the ends of the longest prompts up to three times the work: 32 heads over 2 of 128, values of 256, 1 prompt
-  // of 7000 tokens 1352 -> 776 us (whole call), 4 of 1900 389 -> 310.
+  // shares them with the fewest others, every so many tiles its own: workgroups that read the same K and V rows run next to each other on
+  // one L2, and every XCD has as many long tiles.  Tiles from the last (most keys) to the first, or by their keys (by_keys).  A contiguous
+  // range of all items an XCD gave the one with the ends of the longest prompts up to three times the work: 32 heads over 2 of 128, values
+  // of 256, 1 prompt of 7000 tokens 1352 -> 776 us (whole call), 4 of 1900 389 -> 310.
   // (32 bits and shifts: with 64-bit quotients here and in the search for the request 20 tokens took 8.3 us for 7.4)
   const int hw_shift = 31 - __builtin_clz(hw), shift = 31 - __builtin_clz(32 * NW) - hw_shift, rows_wg = 1 << shift;      // (hw: a power of two)
   const uint32_t rep = a.H / a.G, sets = (rep + hw - 1) >> hw_shift, n_tiles = (uint32_t)a.n_tiles;
@@ -126,7 +165,21 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
   // Its request: 64 at a time, a lane each, with all that is known of them in one round trip
   int b = -1, q0 = 0, qn = 0, base_pos = 0;
   int64_t t0 = 0, pool_row = 0;
-  {
+  if (by_keys) {
+    const int rq = min(lane, (int)a.batch - 1);
+    const int n = a.q_len[rq], len = (int)a.seq_lens[rq], start = a.q_start[rq];
+    const int64_t in_pool = a.req_pool_indices[rq];
+    const int tiles = lane < (int)a.batch ? (max(n, 0) + rows_wg - 1) >> shift : 0;
+    const PromptTile at = prompt_tile_by_keys(tile_at, (int)a.batch, tiles, tiles > 0 ? (uint32_t)(len - n) : 0u, shift, (uint32_t)a.chunk >> shift);
+    if (at.request >= 0) {
+      b = at.request;
+      q0 = at.tile << shift;
+      qn = __builtin_amdgcn_readlane(n, b);
+      base_pos = __builtin_amdgcn_readlane(len, b) - qn;
+      t0 = __builtin_amdgcn_readlane(start, b);
+      pool_row = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)in_pool, b) | (int64_t)__builtin_amdgcn_readlane((int)(in_pool >> 32), b) << 32;
+    }
+  } else {
     int left = (int)tile_id;
     for (int rq0 = 0; rq0 < (int)a.batch && b < 0; rq0 += 64) {
       const int rq = min(rq0 + lane, (int)a.batch - 1);
@@ -410,7 +463,7 @@ __global__ void __launch_bounds__(64 * NW, W) prompt_attention_kernel(LocalAttnA
 
 // true: launched.  Head sizes 64 / 64, 64 / 128, 128 / 128, 128 / 256 (sigmoid weights: 64 / 64, 128 / 128), a positive scale, 16-bit
 // types, everything aligned as local_attention_mfma_kernel wants it.
-template <typename T, int D, int E, int NW, int KT, int W, bool SIG>
+template <typename T, int D, int E, int NW, int KT, bool SIG>
 static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   const int rep = a.H / a.G;
   // heads of a group in a workgroup: the largest power of two that divides them, or the next one above them (the last set's waves are not all
@@ -426,20 +479,30 @@ static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   a.n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
   constexpr size_t tiles = 2 * KT * (size_t)(D + E) * 2, epilogue = NW * 32 * (size_t)(E * 2 + 16), bytes = tiles > epilogue ? tiles : epilogue;
   static std::atomic<uint64_t> done{0};
-  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, W, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
+  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
   const PromptShare share = prompt_share(a.G, (uint32_t)a.n_tiles);
   const int64_t blocks = 8ll * share.heads * share.tiles * ((rep + hw - 1) / hw);
-  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, W, SIG>), dim3((unsigned)blocks), dim3(64 * NW), bytes, s, a, hw);
+  // Tiles by their keys where they differ by blocks or by requests (one sequence without blocks is in that order anyway, and windows make
+  // most tiles alike) and the launch is between one (two) and eight times what the chip takes at once: below that all start together, above
+  // the end of the launch is little of it. (Blocks of a few steps: a tile's start and end are most of its time, and all are nearly alike.)
+  // Whole call, last tile first / by keys, us: 32 / 8 heads of 128, blocks of 1024, 4 prompts of 1900 tokens 107.5 / 97.7, 2 of 1500 46.4 /
+  // 38.5, 1 of 16000 217.7 / 211.1, 4 of 6000 (12 times) 337 / 338; 24 / 8 heads, blocks of 256, 4 of 1900 45.8 / 44.3, 2 of 1500 21.6 /
+  // 25.0; without blocks 2 of 3000 168 / 154, 2 of 1500 (1.5 times) 52.6 / 53.9, 16 of 500 (each workgroup asks for all 16) 83.8 / 86.8;
+  // values of 256, 2 heads, 2 of 3000 326 / 299.
+  const int64_t at_once = 256 * 8 / NW;
+  const bool by_keys = a.window == 0 && a.batch <= 8 && (a.chunk > 0 ? a.chunk >= 512 && a.chunk % rows == 0 && blocks > at_once : a.batch > 1 && blocks > 2 * at_once) &&
+                       blocks <= 8 * at_once;
+  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, SIG>), dim3((unsigned)blocks), dim3(64 * NW), bytes, s, a, hw, (int)by_keys);
   return 0;
 }
 template <typename T>
 static bool prompt_attention(const LocalAttnArgs& a, hipStream_t s, int& rc) {
   const bool sig = a.sigmoid != 0;
   if (!(a.scale > 0.f) || a.k_ld <= 0 || a.v_ld <= 0 || a.k_ld >= (1ll << 31) || a.v_ld >= (1ll << 31)) return false;
-  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, 2, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, 2, false>(a, s);
-  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, 2, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, 2, false>(a, s);
-  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, 2, false>(a, s);
-  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, 2, false>(a, s);
+  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, false>(a, s);
+  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, false>(a, s);
+  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, false>(a, s);
+  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, false>(a, s);
   else return false;
   return true;
 }

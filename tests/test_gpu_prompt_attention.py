@@ -222,3 +222,28 @@ def test_talk_mix(dtype, H, G, E):
     terms = torch.einsum("hg,tghe->the", talk.double().abs(), x.abs())
     half = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
     assert bool(((out - want).abs() <= half * want.abs() + 64 * 2.0 ** -24 * terms + 1e-7).all())
+
+
+# (launches large enough that tiles go by their keys: blocks of 18 tiles, one row past a tile's edge in front; of 70, two of which are a level;
+# requests without blocks, so many keys that three tiles are a level)
+@pytest.mark.parametrize("block,lens,olds", [(576, [700, 0, 33, 400, 1], [545, 7, 5, 0, 576]), (2240, [500, 1, 600], [2000, 64, 3]), (2240, [1100], [1999]),
+                                             (0, [900, 0, 1200, 130], [0, 9, 4001, 70]), (0, [300, 200, 260, 0, 330, 410, 290, 310], [0, 31, 32, 1, 64, 0, 5, 0])])
+def test_prompt_attention_tiles_by_their_keys(block, lens, olds):
+    """Every row is there once, whatever the order: against the dense form, into a result that holds something else."""
+    from semi_pd_amd import ops
+    H, G, D = 64, 16, 64
+    t, g = _batch(lens, olds, H, G, D, D, torch.bfloat16, sum(lens))
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+    out = torch.full((sum(lens), H * D), 7.0, dtype=torch.bfloat16, device=DEV)
+    ops.local_attention_fwd(d["q"], out, d["k"], d["v"], d["table"], torch.arange(len(lens), device=DEV), torch.tensor(t["totals"], device=DEV),
+                            start.to(DEV), n.to(DEV), max(lens), D ** -0.5, 0.0, block, None, None)
+    see = (lambda p, j: (j <= p) & (j // block == p // block)) if block else lambda p, j: j <= p          # noqa: E731
+    got, at = out.cpu().double(), 0
+    for b, (new, old) in enumerate(zip(lens, olds)):                                # (a few heads: the order is the same for all)
+        rows, p, j = t["table"][b, : new + old].long(), torch.arange(old, old + new)[:, None], torch.arange(new + old)[None]
+        for h in (0, 21, 63):
+            s = t["q"][at: at + new, h * D: (h + 1) * D].double() @ t["k"][rows, h // 4].double().t() * D ** -0.5
+            want = torch.softmax(s.masked_fill(~see(p, j), -float("inf")), -1) @ t["v"][rows, h // 4].double()
+            torch.testing.assert_close(got[at: at + new, h * D: (h + 1) * D], want, rtol=6 * 2.0 ** -8, atol=12 * 2.0 ** -8)
+        at += new
