@@ -628,21 +628,21 @@ constexpr int kDeltaHead = 6 * 256 + 4 * kRecChunk;
 // A workgroup per (chunk, key head): convolution, silu and unit norm of its q and k (a channel per thread), K K^T and Q K^T, then
 // half a wave per head of the group: gates, A, its inverse column by column (lane = column, forward substitution), weights.
 template <typename T, int NP>
-__global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) {
-  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4;
-  __shared__ __attribute__((aligned(16))) float kq_l[2 * L * CS > 8 * L * L ? 2 * L * CS : 8 * L * L];     // K [32][CS] | Q; later A, one per half wave
-  __shared__ __attribute__((aligned(16))) float kk_l[L * PS], qk_l[L * PS];
+__global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs a) {
+  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4, AL = 16 * 16 + 16 * 32, LATER = 8 * AL + 2 * L * PS;
+  // K [32][CS] | Q; later A, one per half wave (rows of 16, from row 16 on of 32: it is strictly lower triangular) | K K^T | Q K^T.  36 KB and
+  // 128 registers: four workgroups a CU (45 KB and three before: 1824 workgroups took three rounds of 20 us)
+  __shared__ __attribute__((aligned(16))) float kq_l[2 * L * CS > LATER ? 2 * L * CS : LATER];
+  float *const kk_l = kq_l + 8 * AL, *const qk_l = kk_l + L * PS;
   __shared__ double cum_l[8 * L];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4, g = blockIdx.y;
-  int b;
-  int64_t ck;
-  if (!rec_find_chunk(a.q_len, (int)a.batch, blockIdx.x, b, ck)) return;
-  const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
-  if (first_pos < 0) return;
-  const int64_t l0 = ck * L, t0 = a.q_start[b] + l0;
-  const int cnt = (int)(n - l0 < L ? n - l0 : L);
+  RecChunk at;
+  if (!rec_find_chunk(a.q_len, a.seq_lens, a.q_start, (int)a.batch, blockIdx.x, at) || at.first_pos < 0) return;
+  const int64_t l0 = at.c * L, t0 = at.q_start + l0;
+  const int cnt = (int)(at.n - l0 < L ? at.n - l0 : L);
   const int D = a.D, taps = a.taps, C = 2 * a.G * D + a.H * a.E, per = a.H / a.G;
   float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * delta_frag_elems(NP);
+  const float* kept = l0 == 0 && at.first_pos > 0 && taps > 1 ? a.conv_state + a.state_indices[at.b] * a.conv_ld : nullptr;
   bool bad = false;
   for (int ch = tid; ch < 2 * NP; ch += 256) {
     const bool is_q = ch >= NP;
@@ -652,35 +652,9 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
       const int cc = (is_q ? 0 : a.G * D) + g * D + d;                                      // channel in the state's order (q | k | v)
       const T* p = (const T*)a.p + t0 * a.ld + (is_q ? a.q_off : a.k_off) + g * D + d;
       const T* cw = (const T*)(is_q ? a.conv_q : a.conv_k) + (int64_t)(g * D + d) * taps;
-      float wt[kRecTaps], in[kRecTaps];
-#pragma unroll
-      for (int i = 0; i < kRecTaps; ++i) {
-        wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
-        in[i] = 0.f;
-        if (i > 0 && i < taps) {
-          if (l0 - i >= 0) in[i] = Elem<T>::to_f(p[-(int64_t)i * a.ld]);
-          else if (first_pos > 0) in[i] = a.conv_state[a.state_indices[b] * a.conv_ld + (int64_t)(taps - 1 + l0 - i) * C + cc];
-        }
-      }
-      float x[L];
-      if (cnt == L) {
-#pragma unroll
-        for (int i = 0; i < L; ++i) x[i] = Elem<T>::to_f(p[(int64_t)i * a.ld]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < L; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
-      }
-#pragma unroll
-      for (int t = 0; t < L; ++t) {
-        in[0] = x[t];
-        float y = 0.f;
-#pragma unroll
-        for (int i = 0; i < kRecTaps; ++i)
-          if (i < taps) y += wt[i] * in[i];
-#pragma unroll
-        for (int i = kRecTaps - 1; i > 0; --i) in[i] = in[i - 1];
-        dst[t * CS] = t < cnt ? (rec_moderate(y) ? rec_silu(y) : rec_silu_if_large(y)) : 0.f;
-      }
+      float wt[kRecTaps], in[kRecTaps], x[L];
+      rec_channel<T>(p, a.ld, cnt, cw, taps, l0 > 0, kept != nullptr ? kept + cc : nullptr, C, wt, in, x);
+      rec_conv_silu(wt, in, x, 0.f, taps, cnt, dst, CS);
     } else {
       for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
     }
@@ -751,20 +725,25 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
         qk = __builtin_amdgcn_mfma_f32_16x16x4f32(aq[s], bv[s], qk, 0, 0, 0);
       }
     }
+    __syncthreads();                                              // (K and Q have been read)
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       kk_l[(i0 + 4 * kq + r) * PS + j0 + r16] = kk[r];
       qk_l[(i0 + 4 * kq + r) * PS + j0 + r16] = qk[r];
     }
   }
-  __syncthreads();                                                // (kq_l is free from here on)
-  const int hw = tid >> 5, ln = tid & 31;
-  float* a_l = kq_l + hw * L * L;
-  double* cum = cum_l + hw * L;
-  for (int hh = blockIdx.z * 8 + hw; hh < per; hh += 8 * gridDim.z) {
-    const int h = g * per + hh;
+  __syncthreads();
+  // up to eight heads at a time, half wave `half` of wave w has w + 4 half: its decays and its inverse; the weights of a wave's heads by both
+  // halves, one head after the other (each for its own: with four heads half of the chip's waves have none, 7.3 us of a workgroup's 30)
+  const int half = lane >> 5, ln = tid & 31;
+  double* cum = cum_l + (2 * w + half) * L;
+  for (int h0 = blockIdx.z * 8; h0 < per; h0 += 8 * gridDim.z) {
+    if (h0 + w >= per) break;
+    const int heads = h0 + w + 4 < per ? 2 : 1;                  // of this wave
+    const bool mine = half < heads;
+    const int h = g * per + h0 + w + (mine ? 4 * half : 0);      // (a half wave without a head of its own goes along with the other, and lays nothing down)
     const T* pr = (const T*)a.p + (t0 + ln) * a.ld;
-    const bool on = ln < cnt;
+    const bool on = ln < cnt && mine;
     const float la = on ? -expf(a.a_log[h]) * softplus_f(Elem<T>::to_f(pr[a.a_off + h]) + a.dt_bias[h]) : 0.f;
     const float beta = on ? sigmoid_f(Elem<T>::to_f(pr[a.b_off + h])) : 0.f;
     double c = (double)la * 1.4426950408889634;
@@ -778,42 +757,55 @@ __global__ void __launch_bounds__(256) delta_chunk_operands_kernel(DeltaArgs a) 
     float* hp = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kDeltaHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c), dec = expf(la);
     const bool no = !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_moderate_decay(la);
-    hp[1536 + ln] = rec_flagged(eb, no);
-    hp[1536 + L + ln] = wt;
-    hp[1536 + 2 * L + ln] = dec;
-    hp[1536 + 3 * L + ln] = beta;
+    const float flagged = rec_flagged(eb, no);
+    if (mine) {
+      hp[1536 + ln] = flagged;
+      hp[1536 + L + ln] = wt;
+      hp[1536 + 2 * L + ln] = dec;
+      hp[1536 + 3 * L + ln] = beta;
+    }
     __builtin_amdgcn_wave_barrier();
-    // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s)
+    // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s); rows 0 .. 15 by the lower half, 16 .. 31 by the upper
     const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);
-    int lv = ln;
-    asm volatile("" : "+v"(lv));                                  // (rows of K K^T and Q K^T are read per head, not held for all of them)
+    for (int v = 0; v < heads; ++v) {
+      const double* cv = cum_l + (2 * w + v) * L;
+      const double cs = cv[ln];
+      float* av = kq_l + (2 * w + v) * AL + (half ? 256 : 0);
+      const int ald = half ? 32 : 16;
+      float* qv = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + g * per + h0 + w + 4 * v) * kDeltaHead + 768 +
+                  (half + st) * 256 + sl;
 #pragma unroll 4
-    for (int t = 0; t < L; ++t) {
-      const float bt = __shfl(beta, t, L);
-      const float e = ln <= t ? rec_exp2(cum[t] - c) : 0.f;
-      a_l[t * L + ln] = ln < t ? bt * (e * kk_l[t * PS + lv]) : 0.f;
-      if (t >= 16 || st == 0) hp[768 + ((t >> 4) + st) * 256 + sl + (t & 15) * 4] = ln <= t ? e * qk_l[t * PS + lv] : 0.f;
+      for (int u = 0; u < 16; ++u) {
+        const int t = 16 * half + u;
+        const float bt = __shfl(beta, 32 * v + t, 64);
+        const float e = ln <= t ? rec_exp2(cv[t] - cs) : 0.f;
+        if (half >= st) av[u * ald + ln] = ln < t ? bt * (e * kk_l[t * PS + ln]) : 0.f;
+        if (half >= st) qv[4 * u] = ln <= t ? e * qk_l[t * PS + ln] : 0.f;
+      }
     }
     __builtin_amdgcn_wave_barrier();
-    // column ln of (I + A)^-1, four terms of a row at a time
-    float x[L];
+    if (mine) {
+      const float* a_l = kq_l + (2 * w + half) * AL;
+      // column ln of (I + A)^-1, four terms of a row at a time
+      float x[L];
 #pragma unroll
-    for (int t = 0; t < L; ++t) {
-      float acc = t == ln ? 1.f : 0.f;
+      for (int t = 0; t < L; ++t) {
+        float acc = t == ln ? 1.f : 0.f;
 #pragma unroll
-      for (int s = 0; s < t; s += 4) {
-        const float4 av = *reinterpret_cast<const float4*>(a_l + t * L + s);
-        acc -= av.x * x[s];
-        if (s + 1 < t) acc -= av.y * x[s + 1];
-        if (s + 2 < t) acc -= av.z * x[s + 2];
-        if (s + 3 < t) acc -= av.w * x[s + 3];
+        for (int s = 0; s < t; s += 4) {
+          const float4 av = *reinterpret_cast<const float4*>(a_l + (t < 16 ? t * 16 : t * 32 - 256) + s);
+          acc -= av.x * x[s];
+          if (s + 1 < t) acc -= av.y * x[s + 1];
+          if (s + 2 < t) acc -= av.z * x[s + 2];
+          if (s + 3 < t) acc -= av.w * x[s + 3];
+        }
+        x[t] = acc;
+        asm volatile("" : "+v"(x[t]));                             // (row by row: not all rows of A first and the sums behind them)
       }
-      x[t] = acc;
-      asm volatile("" : "+v"(x[t]));                             // (row by row: not all rows of A first and the sums behind them)
-    }
 #pragma unroll
-    for (int t = 0; t < L; ++t)
-      if (t >= 16 || st == 0) hp[((t >> 4) + st) * 256 + sl + (t & 15) * 4] = x[t] * beta;
+      for (int t = 0; t < L; ++t)
+        if (t >= 16 || st == 0) hp[((t >> 4) + st) * 256 + sl + (t & 15) * 4] = x[t] * beta;
+    }
     __builtin_amdgcn_wave_barrier();
   }
   const int any_bad = __syncthreads_or(bad);

@@ -346,16 +346,14 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
   __shared__ float cb_l[L * PS];
   __shared__ double cum_l[8 * L];
   const int tid = threadIdx.x, g = blockIdx.y;
-  int b;
-  int64_t ck;
-  if (!rec_find_chunk(a.q_len, (int)a.batch, blockIdx.x, b, ck)) return;
-  const int64_t n = a.q_len[b], first_pos = a.seq_lens[b] - n;
-  if (first_pos < 0) return;
-  const int64_t l0 = ck * L, t0 = a.q_start[b] + l0;
-  const int cnt = (int)(n - l0 < L ? n - l0 : L);
+  RecChunk at;
+  if (!rec_find_chunk(a.q_len, a.seq_lens, a.q_start, (int)a.batch, blockIdx.x, at) || at.first_pos < 0) return;
+  const int64_t l0 = at.c * L, t0 = at.q_start + l0;
+  const int cnt = (int)(at.n - l0 < L ? at.n - l0 : L);
   const int N = a.N, taps = a.taps, per = a.H / a.G;
   const int C = a.H * a.E + 2 * a.G * N;
   float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * ssm_frag_elems(NP);
+  const float* kept = l0 == 0 && at.first_pos > 0 && taps > 1 ? a.conv_state + a.state_indices[at.b] * a.conv_ld : nullptr;
   bool bad = false;
   for (int ch = tid; ch < 2 * NP; ch += 256) {
     const bool is_c = ch >= NP;
@@ -365,37 +363,11 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
       const int col = a.H * a.E + (is_c ? a.G * N : 0) + g * N + r;               // among the convolution's channels
       const T* p = (const T*)a.p + t0 * a.ld + a.x_off + col;
       const T* cw = (const T*)a.conv_w + (int64_t)col * taps;
-      const float bias = a.conv_b ? Elem<T>::to_f(((const T*)a.conv_b)[col]) : 0.f;
-      float wt[kRecTaps], in[kRecTaps];                                   // weight and input i tokens back
-#pragma unroll
-      for (int i = 0; i < kRecTaps; ++i) {
-        wt[i] = i < taps ? Elem<T>::to_f(cw[taps - 1 - i]) : 0.f;
-        in[i] = 0.f;
-        if (i > 0 && i < taps) {
-          if (l0 - i >= 0) in[i] = Elem<T>::to_f(p[-(int64_t)i * a.ld]);
-          else if (first_pos > 0) in[i] = a.conv_state[a.state_indices[b] * a.conv_ld + (int64_t)(taps - 1 + l0 - i) * C + col];
-        }
-      }
-      float x[L];
-      if (cnt == L) {
-#pragma unroll
-        for (int i = 0; i < L; ++i) x[i] = Elem<T>::to_f(p[(int64_t)i * a.ld]);
-      } else {
-#pragma unroll
-        for (int i = 0; i < L; ++i) x[i] = i < cnt ? Elem<T>::to_f(p[(int64_t)i * a.ld]) : 0.f;
-      }
-#pragma unroll
-      for (int t = 0; t < L; ++t) {
-        in[0] = x[t];
-        float y = bias;
-#pragma unroll
-        for (int i = 0; i < kRecTaps; ++i)
-          if (i < taps) y += wt[i] * in[i];
-#pragma unroll
-        for (int i = kRecTaps - 1; i > 0; --i) in[i] = in[i - 1];
-        dst[t * CS] = t < cnt ? (rec_moderate(y) ? rec_silu(y) : rec_silu_if_large(y)) : 0.f;
-        bad |= t < cnt && !rec_moderate(y);
-      }
+      const T shift = *(a.conv_b ? (const T*)a.conv_b + col : cw);
+      float wt[kRecTaps], in[kRecTaps], x[L];
+      rec_channel<T>(p, a.ld, cnt, cw, taps, l0 > 0, kept != nullptr ? kept + col : nullptr, C, wt, in, x);
+      const float bias = a.conv_b ? Elem<T>::to_f(shift) : 0.f;
+      bad |= rec_conv_silu(wt, in, x, bias, taps, cnt, dst, CS);
     } else {
       for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
     }
