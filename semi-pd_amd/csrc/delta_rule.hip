@@ -1516,17 +1516,18 @@ extern "C" int64_t semipd_delta_rule_work_width(int num_heads, int num_k_heads, 
 }
 
 // The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
-// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  A chunk costs the same however few its
-// rows and heads; token by token a token's heads are prepared one behind another, so that form is ahead where there are few.
-// Token by token against chunks, whole call, 32 heads over 8 of 128 x 128: 1 request of 2 rows 51 / 43 us, 64 rows 96 / 54, 256 rows 251 / 92;
-// 4 requests of 2 rows 53 / 44; 32 requests of 8 rows 153 / 162, 16 rows 235 / 173, 256 rows 2540 / 760; 32 heads of 64 x 64: 4 requests of
-// 2 rows 53 / 36, 32 requests of 20 rows 97 / 81.  8 heads over 1 of 128 x 128: 1 request of 2 rows 27 / 43, 24 rows 44 / 47, 32 rows 49 / 46;
-// 16 over 4 of 64 x 128: 16 requests of 20 rows 49 / 57, 32 rows 60 / 65, 48 rows 74 / 67; 8 over 1 of 64 x 64: 1 request of 32 rows 34 / 39,
-// 48 rows 41 / 42, 64 rows 47 / 43.
+// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  A chunk costs the same however few its rows
+// and heads; token by token a token's heads are prepared one behind another, so that form is ahead where there are few. Token by token
+// against chunks, whole call, 32 heads over 8 of 128 x 128: 1 request of 2 rows 47 / 34 us, 48 rows 82 / 38; 16 requests of 2 rows 79 / 68;
+// 32 of 2 rows 114 / 115, 16 rows 198 / 123; 64 of 4 rows 207 / 237, 8 rows 259 / 240.  16 over 2 of 128 x 128: 1 request of 8 rows 33 / 36,
+// 12 rows 37 / 36; 16 of 12 rows 52 / 50.  8 over 1: 1 request of 16 rows 31 / 35, 24 rows 39 / 36; 32 of 12 rows 50 / 50.  Keys of up to
+// 64: 32 over 8 of 64 x 64, 4 requests of 2 rows 46 / 32, 32 of 8 rows 59 / 64, 16 rows 73 / 66; 16 over 4 of 64 x 128, 16 of 24 rows 43 /
+// 46, 32 rows 49 / 46; 8 over 1 of 64 x 64, 8 of 32 rows 30 / 35, 32 of 48 rows 49 / 42.  (Some would be ahead in chunks earlier, 8 of 12
+// rows 45 / 33, but a state of theirs is then 1.1 times as far from the 64-bit one.)
 static int64_t delta_chunk_min_rows(int64_t batch, int num_heads, int num_k_heads, int k_dim) {
   const int heads = num_heads + 2 * num_k_heads;
-  if (heads >= 32) return batch <= 4 ? 0 : 16;
-  return k_dim > 64 ? 24 : heads >= 16 ? 32 : 48;
+  if (k_dim > 64) return heads >= 32 ? (batch <= 16 ? 0 : 6) : heads >= 16 ? 12 : batch < 32 ? 22 : 14;
+  return heads >= 32 ? (batch <= 4 ? 0 : 16) : heads >= 16 ? 32 : 48;
 }
 
 extern "C" int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps) {

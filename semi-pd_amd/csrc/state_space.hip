@@ -101,6 +101,7 @@ template <typename T> __device__ __forceinline__ void load4(const T* p, float (&
 }
 
 constexpr int kPrepMaxTaps = 8;          // taps whose weights the four-channel form keeps in registers
+constexpr int kPrepTileBlocks = 512;
 constexpr int kPrepTile = 32;            // tokens a workgroup of a prompt batch walks with them
 
 template <typename T, bool VEC4>
@@ -999,15 +1000,20 @@ extern "C" int64_t semipd_state_space_work_width(int num_heads, int groups, int 
 }
 
 // The rows per request from which a prompt batch goes in chunks: on average, since the lengths are on the device.  (The time token by token
-// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call, 128 heads of 128 x 64: 1 request of 8 rows 34.0 / 36.1 us, 12 rows 37.3 / 36.4, 32 rows 56 / 40,
-// 256 rows 327 / 79; 32 requests of 8 rows 185 / 148, 32 rows 548 / 191, 256 rows 3058 / 782; 64 heads: 1 request of 12 rows 34.3 / 33.8,
-// 32 requests of 8 rows 110 / 88.  A state of 16 rows is padded to 64: 256 heads of 16 x 64, 1 request of 12 rows 54 / 59, 32 rows 65 / 62, 8
-// requests of 16 rows 90 / 107, 16 requests of 24 rows 204 / 175.
-constexpr int64_t kSsmChunkMinRows = 12;
+// is the longest request's: an uneven batch gains from chunks at a lower average than these.)  Token by token against chunks, whole call,
+// heads of 128 x 64, us: 1 request, 128 heads: 6 rows 28 / 30, 8 rows 30 / 30, 48 rows 67 / 34; 32 heads: 8 rows 25 / 26, 12 rows 29 / 26.  4 requests,
+// 128 heads: 6 rows 36 / 36; 64 heads: 8 rows 32 / 31.  8 requests, 128 heads: 4 rows 52 / 52, 6 rows 57 / 53; 64 heads: 5 rows 34 / 35, 6 rows
+// 37 / 35; 32 heads: 8 rows 30 / 29.  32 requests, 128 heads: 4 rows 155 / 146, 64 rows 893 / 241.  A state of 16 rows is padded to 64: 256 heads of
+// 16 x 64, 1 request of 16 rows 55 / 58, 24 rows 61 / 58; 8 of 24 rows 107 / 104; 16 of 24 rows 147 / 157, 32 rows 170 / 159.
+static int64_t ssm_chunk_min_rows(int64_t batch, int num_heads, int state_size) {
+  const int64_t heads = batch * num_heads;
+  if (state_size <= 16) return heads >= 4096 ? 28 : 24;
+  return heads >= 768 ? 5 : heads >= 384 ? 6 : heads >= 128 ? 8 : 12;
+}
 static int ssm_padded_state(int state_size) { return state_size <= 64 ? 64 : 128; }
 
 extern "C" int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state_size, int taps) {
-  if (batch <= 0 || groups <= 0 || num_tokens < (state_size <= 16 ? 24 : kSsmChunkMinRows) * batch || state_size > 128 || taps > kRecTaps) return 0;
+  if (batch <= 0 || groups <= 0 || num_tokens < ssm_chunk_min_rows(batch, num_heads, state_size) * batch || state_size > 128 || taps > kRecTaps) return 0;
   return rec_max_chunks(num_tokens, batch) * (groups * ssm_frag_elems(ssm_padded_state(state_size)) + (int64_t)num_heads * kSsmHead);
 }
 
@@ -1108,8 +1114,10 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
   const bool prep4 = C % 4 == 0 && x_off % 4 == 0 && ld % 4 == 0 && work_ld % 4 == 0 && (taps == 1 || conv_ld % 4 == 0) &&
                      ((uintptr_t)proj % 16) == 0 && aligned16(work) && (taps == 1 || aligned16(conv_state)) &&
                      aligned16(conv_w) && taps <= kPrepMaxTaps;
-  // a prompt batch: a workgroup walks a tile of tokens with its channels' taps in registers; one row per request: a token each
-  const int tile = (q_start != nullptr && prep4 && num_tokens >= 8 * kPrepTile) ? kPrepTile : 1;
+  // a prompt batch: a workgroup walks a tile of tokens with its channels' taps in registers, where that leaves the chip enough of them; else a
+  // token each (by tokens / by tiles, heads of 128 x 64, whole call token by token, us: 8 heads, 64 requests of 16 rows 62 / 328; 128 heads, 64 of 16
+  // rows, 328 tiles' workgroups, 606 / 831, 8 of 400 rows, 1000 of them, 1095 / 988)
+  const int tile = (q_start != nullptr && prep4 && num_tokens / kPrepTile * cblocks >= kPrepTileBlocks) ? kPrepTile : 1;
   const dim3 pgrid((unsigned)((num_tokens + tile - 1) / tile), cblocks);
   SEMIPD_DISPATCH_DTYPE(dtype, T, {
     if (prep4) hipLaunchKernelGGL((ssm_prep_kernel<T, true>), pgrid, dim3(256), 0, s, a, tile);

@@ -492,3 +492,26 @@ def test_result_over_the_inputs(kind, lens, monkeypatch):
         for a, b in zip(apart, over):
             for x, y in zip(a, b):
                 assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("lens", [[5, 1, 9, 4, 6, 3, 7, 5], [1, 3, 2, 2] * 4])
+@pytest.mark.parametrize("kind", ["state_space", "delta_rule"])
+def test_few_rows_a_request_in_chunks(kind, lens):
+    """As many heads as make chunks worth it from a few rows on; tolerances as above."""
+    from semi_pd_amd import _lib
+    H, G, N, E = (128, 1, 24, 8) if kind == "state_space" else (24, 8, 72, 16)
+    make, run, truth = (_ssm_inputs, _ssm_run, _ssm_truth) if kind == "state_space" else (_delta_inputs, _delta_run, _delta_truth)
+    extra = (1,) if kind == "state_space" else ()
+    if kind == "state_space":
+        lens = [n + 3 * (sum(lens) < 40) for n in lens]
+    elems = getattr(_lib.load(), "semipd_%s_chunk_elems" % kind)(sum(lens), len(lens), H, G, N, 4)
+    assert elems > 0
+    w, rows, state, before = make(H, G, N, E, 4, lens, torch.float32, 5)
+    first = [i % 2 * 9 for i in range(len(lens))]
+    outs, after, last = run(w, rows, state, before, first, H, G, N, E, *extra)
+    for i in range(len(lens)):
+        old = first[i] > 0
+        want, S, kept = truth(w, rows[i], state[i] * old, before[i] * old, H, G, N, E, *extra)
+        torch.testing.assert_close(outs[i].to(F64), want, rtol=2e-5, atol=2e-5)
+        torch.testing.assert_close(after[i].to(F64), S, rtol=1e-5, atol=1e-5)
+        torch.testing.assert_close(last[i].to(F64), kept, rtol=0, atol=0)
