@@ -796,6 +796,29 @@ def test_silu_and_mul_golden(ops, device):
         assert torch.all((y.float() - want).abs() <= 1.01 * ulp * want.abs() + 1e-6), ci
 
 
+# (ids over one and several workgroups of 2048, more than 64 of these, not on a 16-byte boundary, some of no expert here)
+@pytest.mark.parametrize("numel,E,block,skip", [(2048, 64, 64, 0), (4097, 200, 128, 1), (6 * 3001, 64, 128, 0), (131073, 3, 64, 3), (270001, 256, 16, 1)])
+def test_moe_align_over_several_workgroups(ops, device, numel, E, block, skip):
+    """Every id of an expert once in its rows, padding everywhere else, offsets or ends in the buffer."""
+    g = torch.Generator().manual_seed(numel)
+    ids = torch.randint(-1, E + 1, (numel + skip,), generator=g, dtype=torch.int32)
+    room = numel + E * (block - 1) + 5
+    rows, blocks = torch.full((room,), -7, dtype=torch.int32, device=device), torch.full((room // block + 1,), -7, dtype=torch.int32, device=device)
+    total, ends = torch.zeros(1, dtype=torch.int32, device=device), torch.zeros(E + 1, dtype=torch.int32, device=device)
+    ops.moe_align_block_size(ids.to(device)[skip:], E, block, rows, blocks, total, None, ends)
+    ids, rows, blocks = ids[skip:].long(), rows.cpu(), blocks.cpu()
+    counts = torch.bincount(ids[(ids >= 0) & (ids < E)], minlength=E)
+    padded = (counts + block - 1) // block * block
+    at = torch.cat([torch.zeros(1, dtype=torch.long), padded.cumsum(0)])
+    assert int(total) == int(at[-1]) and bool((rows[int(at[-1]):] == numel).all())
+    assert bool((blocks[: int(at[-1]) // block] == torch.arange(E).repeat_interleave(padded // block)).all())
+    assert ends.cpu().tolist() == (at[:-1] + (counts if numel > 4096 or room > 65536 else 0)).tolist() + [int(at[-1])]
+    for e in range(E):
+        mine = rows[int(at[e]): int(at[e + 1])]
+        assert torch.equal(mine[: int(counts[e])].sort().values.long(), torch.nonzero(ids == e).flatten())
+        assert bool((mine[int(counts[e]):] == numel).all())
+
+
 def test_moe_align_golden(ops, device):
     """Against the Triton implementation of sgl-kernel/tests/test_moe_align.py run under the interpreter
     (golden/moe_align.npz): expert_ids, num_tokens_post_pad and, per expert, the token set."""
