@@ -138,7 +138,7 @@ class HipAttnBackend(AttentionBackend):
             attn_logits = torch.empty((bs, self.num_head, splits, self.v_head_dim + 1), dtype=torch.float32,
                                       device=dev) if splits > 1 else None
             self.forward_metadata = ForwardMetadata(attn_logits, kv_indptr, kv_indices, None, 0, splits)
-            # sum_len * Hkv * (Dk + Dv) * s  +  2 * B * Hq * D * s   per layer
+            # bytes: sum_len * Hkv * (Dk + Dv) * s  +  2 * B * Hq * D * s   per layer
             es = 2
             es_kv = getattr(self.model_runner, "kv_cache_dtype", torch.bfloat16).itemsize  # 1 for fp8 rows
             self._algo = (forward_batch.seq_lens_sum * self.num_kv_head * self._kv_row_elems() * es_kv
@@ -152,7 +152,7 @@ class HipAttnBackend(AttentionBackend):
             qo_indptr[1:] = torch.cumsum(forward_batch.extend_seq_lens, dim=0)
             self.forward_metadata = ForwardMetadata(None, kv_indptr, kv_indices, qo_indptr,
                                                     max(forward_batch.extend_seq_lens_cpu), 1)
-            # 2 * Hq * (Dk + Dv) * sum_i ext_i * (pre_i + (ext_i + 1) / 2) flop
+            # work: 2 * Hq * (Dk + Dv) * sum_i ext_i * (pre_i + (ext_i + 1) / 2) flop
             pairs = sum(e * (p + (e + 1) / 2.0) for e, p in zip(forward_batch.extend_seq_lens_cpu,
                                                                  forward_batch.extend_prefix_lens_cpu))
             T = forward_batch.extend_num_tokens

@@ -7,7 +7,7 @@ torch.nn.Module over the HIP operators (semi_pd_amd.ops).  Class names follow th
                               layers/linear.py:296-460, 725-1100, 1103-1280; vocab_parallel_embedding.py:174-500
   LogitsProcessor             layers/logits_processor.py:220-445
   Sampler                     layers/sampler.py:29-171 (greedy branch)
-Dense GEMMs: hipBLASLt through F.linear (SURVEY §2.2 "TP linear") for prefill-sized calls, the persistent
+Dense GEMMs: hipBLASLt through F.linear, or the tiled GEMM where it is ahead, for prefill-sized calls, the persistent
 weight-streaming kernel (ops.stream_linear) for batches of at most 128 rows, i.e. every decode step.
 """
 from __future__ import annotations
@@ -319,7 +319,8 @@ def get_rope(head_size: int, rotary_dim: int, max_position: int, base: float, is
 
 # --------------------------------------------------------------------------- dense GEMM dispatch
 # Batches of at most 128 rows (decode steps, a short last chunk of a prefill) go through the LDS-DMA
-# weight-streaming kernel (csrc/stream_linear.hip); everything else stays on hipBLASLt (F.linear).
+# weight-streaming kernel (csrc/stream_linear.hip), up to 256 through the tiled GEMM (csrc/gemm8p.hip); larger ones through the tiled GEMM
+# where it is ahead (_prefers_tiled_gemm), else hipBLASLt (F.linear, or the solution timed on the share).
 _STREAM_LINEAR = {"enabled": False, "timing": None}
 
 
@@ -346,7 +347,7 @@ def _timed_stream(fn, x: torch.Tensor, weight: torch.Tensor, n_out: int, n_kerne
     t0 = kt.start()
     out = fn()
     es = weight.element_size()
-    # SURVEY 8d "Logits + argmax"-style weight-stream formula: the weight once, activations in, result out
+    # weight-stream formula: the weight once, activations in, result out
     kt.stop("stream_linear", t0, weight.numel() * es + x.numel() * es + x.shape[0] * n_out * es, 0.0, n_kernels)
     return out
 
@@ -354,7 +355,7 @@ def _timed_stream(fn, x: torch.Tensor, weight: torch.Tensor, n_out: int, n_kerne
 def _timed_gemm(fn, x: torch.Tensor, weight: torch.Tensor, n_out: int):
     """The four dense layers of the first decoder layer of a sampled PREFILL batch (bench.py's roofline_extra.prefill_gemm):
     whatever serves them -- a library solution timed on the share, the tiled GEMM, with or without the SiLU epilogue --
-    bracketed like the streaming GEMMs of a decode step; flops = 2 rows n k (SURVEY 8d)."""
+    bracketed like the streaming GEMMs of a decode step; flops = 2 rows n k."""
     kt = _STREAM_LINEAR["timing"]
     if kt is None or not kt.active or kt.linear_budget <= 0 or x.dim() != 2 or x.shape[0] <= GEMM_TALL_MAX_ROWS:
         return fn()
@@ -367,7 +368,7 @@ def _timed_gemm(fn, x: torch.Tensor, weight: torch.Tensor, n_out: int):
     return out
 
 
-GEMM_TALL_MAX_ROWS = 256   # above: the library GEMM (prefill-sized; its solution timed on the share where that was asked for)
+GEMM_TALL_MAX_ROWS = 256   # above (prefill-sized): the tiled GEMM where it is ahead, else the library GEMM
 
 
 def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
@@ -379,7 +380,7 @@ def dense_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
         return _timed_stream(lambda: ops.stream_linear(x, weight, out=out), x, weight, weight.shape[0], 2)
     if _STREAM_LINEAR["enabled"] and bias is None and x.dim() == 2 and _takes_tiled_gemm(x, weight):
         # the tiled ping-pong GEMM (csrc/gemm8p.hip): a tall decode batch (129 .. 256 rows) of an untuned layer, or a
-        # prefill-sized batch of a shape for which it beat the library's measured winner on this share
+        # prefill-sized batch of a shape for which it beat the library's measured winner on this share or fills the chip
         return _timed_gemm(lambda: ops.gemm_tall(x, weight, out=out), x, weight, weight.shape[0])
     if x.dim() == 2 and x.shape[0] > 0 and ops.dense_gemm_is_tuned(weight) and x.stride(1) == 1:
         # prefill-sized batch of a layer whose library solutions were timed on this process's CU share at start-up
@@ -432,7 +433,7 @@ def gate_up_silu(x: torch.Tensor, gate_up_proj: "MergedColumnParallelLinear", ac
             and isinstance(act_fn, SiluAndMul) and x.dim() == 2 and x.shape[0] > GEMM_TALL_MAX_ROWS
             and _prefers_tiled_gemm(gate_up_proj.weight, x.shape[0], fuse_silu_mul=True)
             and ops.gemm_tall_is_supported(x, gate_up_proj.weight, fuse_silu_mul=True)):
-        # prefill-sized batch: the tiled GEMM with the SiLU epilogue beat the library's winner + silu_and_mul on this share
+        # prefill-sized batch: the tiled GEMM with the SiLU epilogue beat the library's winner + silu_and_mul on this share or fills the chip
         w = gate_up_proj.weight
         return _timed_gemm(lambda: ops.gemm_tall(x, w, fuse_silu_mul=True), x, w, w.shape[0] // 2)
     return act_fn(gate_up_proj(x))

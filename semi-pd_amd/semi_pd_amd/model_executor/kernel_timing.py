@@ -3,7 +3,7 @@
 A sampled decode step runs eagerly (not through the hipGraph) and brackets every decode-attention
 launch with a pair of events recorded on the stream the kernel is launched on; prefill batches
 bracket the extend-attention launches the same way.  Alongside the elapsed time we keep the
-ALGORITHMIC bytes / flops of each launch (SURVEY §8d formulas) so that
+ALGORITHMIC bytes / flops of each launch so that
 achieved = sum(bytes) / sum(time) is independent of how many launches were sampled.
 
 Two corrections make the event pair measure the kernel rather than the launch path:

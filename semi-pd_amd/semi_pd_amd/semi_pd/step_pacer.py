@@ -2,7 +2,7 @@
 
 What it stands in for.  The reference's compute split is two static MPS percentages (semi_pd/utils.py:10-11, entrypoints/
 engine.py:588-634: prefill 80 %, decode 100 %): the decode tail under a prefill batch is whatever the non-shared percentage
-delivers.  On MI355X that is a hard trade (DESIGN.md 4.4): next to a 224-CU prefill share a decode step streams its 19 GB
+delivers.  On MI355X that is a hard trade: next to a 224-CU prefill share a decode step streams its 19 GB
 through the 32 CUs the share leaves free and takes 11-15 ms instead of 4.5 -- TTFT p50 29 ms, TBT p99 15.6 ms -- while the
 192-CU share that keeps the tail at 11.6 ms costs 11 ms of TTFT.  A deadline cuts the tail where it forms instead of paying
 for it with CUs all the time: when the decode step in flight is older than `deadline_ms`, the prefill instance stops
@@ -27,7 +27,7 @@ how many steps there were in all; every SLO_WINDOW steps it compares the share o
 weighted by their batch size, BUSY_DECODE) with 1 % and moves the deadline by SLO_STEP_MS (twice that when far off) towards the point where the 99th
 percentile sits on the objective -- the latest deadline, i.e. the fewest and shortest holds, that still keeps the tail.
 The controller is BOUNDED around the deadline it was started with (MAX_TIGHTEN_MS below, MAX_RELAX_MS above): on the frontier of
-DESIGN.md 4.5 a millisecond of TBT tail costs ~4 ms of TTFT p50, and on a slow box an unbounded controller bought 0.3 ms of
+a millisecond of TBT tail costs ~4 ms of TTFT p50, and on a slow box an unbounded controller bought 0.3 ms of
 tail with 1.25 ms of deadline and ~5 ms of TTFT (BENCH_r05: 8.5 -> 7.25 ms in 100 adjustments); bounded, what it can trade
 is at most ~2 ms of TTFT.  Every adjustment is kept (stats()["deadline_trajectory"]) so that a run shows where it went.
 

@@ -24,7 +24,7 @@ from semi_pd_amd import _lib
 # The reference's defaults (semi_pd/utils.py:10-11) are prefill 80 % of the SMs, decode 100 %: overlapping shares.  With CU masks
 # that is a NESTED pair: the prefill instance keeps to the lowest CUs, the decode instance may use every CU and has the rest to
 # itself.  Shares are whole groups of 32 CUs (one per shader engine of every XCD, csrc/ipc.hip: semipd_cu_mask_fill), so on
-# an MI355X the choice is between 192 CUs (75 .. 81 %) and 224 (82 .. 93 %); measured, Llama-3-8B at 32 req/s (DESIGN.md 4.4,
+# an MI355X the choice is between 192 CUs (75 .. 81 %) and 224 (82 .. 93 %); measured, Llama-3-8B at 32 req/s (
 # 4.5): 192 CUs TTFT p50 40.7 ms / TBT p99 11.6 ms, 224 CUs 29.4 / 15.6 -- and 224 CUs with the decode-step deadline of
 # semi_pd/step_pacer.py 33.6 / 11.9.  The default here is therefore 88 % (224 CUs) where the reference has 80; the
 # environment variables of the reference still override it.
