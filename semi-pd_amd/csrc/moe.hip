@@ -61,18 +61,19 @@ __device__ inline void wave_argmax(float& v, int& i) {
 }
 
 // mode: 0 = plain softmax top-k (fused_topk); 1 = grouped (grouped_topk / biased_grouped_topk)
-// One wave per token; lane l owns experts l, l + 64, ... (up to kMaxExperts / 64 = 8) and keeps their logits, scores and
+// One wave per token; lane l owns experts l, l + 64, ... (NE of them, up to kMaxExperts / 64 = 8) and keeps their logits, scores and
 // selection values in REGISTERS: the routing of a decode batch is a chain of dependent steps, and every LDS round trip in
 // it (the first form of this kernel kept everything in LDS: ~60 of them, 16.5 us at 256 experts in 8 groups) costs more
 // than the arithmetic.  LDS is left for the group stage only (a group's experts sit in other lanes).
-template <typename T>
+// NE: experts a lane.  With the 8 places of 512 experts what a lane does for experts that are not there holds up its chain of steps: 64 experts,
+// 6 a token, 32 / 3001 tokens 6.0 / 8.2 us, with one place 4.7 / 6.3; 256 experts, 8 a token, 8.0 / 11.0, with four 7.2 / 9.9.
+template <typename T, int NE>
 __global__ void __launch_bounds__(64)
 moe_topk_kernel(const T* __restrict__ gating, const float* __restrict__ bias,
                 float* __restrict__ topk_weights, int32_t* __restrict__ topk_ids, int E, int topk,
                 int num_group, int topk_group, int renormalize, int scoring, int grouped,
                 const float* __restrict__ planes = nullptr, int n_planes = 0, int64_t plane_elems = 0,
                 float renorm_eps = 0.f) {
-  constexpr int NE = kMaxExperts / 64;
   __shared__ float choice[kMaxExperts];  // group stage: the selection values of every expert
   __shared__ float gscore[64];
   __shared__ int gsel[64];
@@ -110,7 +111,7 @@ moe_topk_kernel(const T* __restrict__ gating, const float* __restrict__ bias,
         }
       }
 #pragma unroll
-      for (int i = 0; i < 4; ++i) logit[i0 + i] = Elem<T>::to_f(Elem<T>::from_f(acc[i]));
+      for (int i = 0; i < 4 && i0 + i < NE; ++i) logit[i0 + i] = Elem<T>::to_f(Elem<T>::from_f(acc[i]));
     }
   } else {
     const T* g = gating + t * E;
@@ -594,6 +595,15 @@ __global__ void __launch_bounds__(256) router_logits_kernel(const T* __restrict_
 
 using namespace semipd;
 
+#define SEMIPD_TOPK(...)                                                                                                                     \
+  do {                                                                                                                                       \
+    const dim3 grid((unsigned)num_tokens);                                                                                                   \
+    if (num_experts <= 64) hipLaunchKernelGGL((moe_topk_kernel<T, 1>), grid, dim3(64), 0, as_stream(stream), __VA_ARGS__);                   \
+    else if (num_experts <= 128) hipLaunchKernelGGL((moe_topk_kernel<T, 2>), grid, dim3(64), 0, as_stream(stream), __VA_ARGS__);             \
+    else if (num_experts <= 256) hipLaunchKernelGGL((moe_topk_kernel<T, 4>), grid, dim3(64), 0, as_stream(stream), __VA_ARGS__);             \
+    else hipLaunchKernelGGL((moe_topk_kernel<T, kMaxExperts / 64>), grid, dim3(64), 0, as_stream(stream), __VA_ARGS__);                      \
+  } while (0)
+
 extern "C" {
 
 int semipd_router_logits(const void* hidden, int64_t ld, const float* weight, float* out, int64_t num_tokens, int width,
@@ -618,7 +628,7 @@ int semipd_topk_softmax(const void* gating, float* topk_weights, int32_t* topk_i
                    SEMIPD_EINVAL, "topk_softmax: bad sizes (E<=%d, topk<=%d)", kMaxExperts, kMaxTopk);
   if (num_tokens == 0) return 0;
   SEMIPD_CHECK_ARG(gating && topk_weights && topk_ids, SEMIPD_EINVAL, "topk_softmax: null pointer");
-  SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((moe_topk_kernel<T>), dim3((unsigned)num_tokens), dim3(64), 0, as_stream(stream), (const T*)gating, (const float*)nullptr, topk_weights, topk_ids, num_experts, topk, 1, 1, renormalize, 0, 0));
+  SEMIPD_DISPATCH_DTYPE(dtype, T, SEMIPD_TOPK((const T*)gating, (const float*)nullptr, topk_weights, topk_ids, num_experts, topk, 1, 1, renormalize, 0, 0));
   return launch_status("topk_softmax");
 }
 
@@ -631,7 +641,7 @@ int semipd_topk_sigmoid(const void* gating, float* topk_weights, int32_t* topk_i
                    SEMIPD_EINVAL, "topk_sigmoid: bad sizes (E<=%d, topk<=%d)", kMaxExperts, kMaxTopk);
   if (num_tokens == 0) return 0;
   SEMIPD_CHECK_ARG(gating && topk_weights && topk_ids, SEMIPD_EINVAL, "topk_sigmoid: null pointer");
-  SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((moe_topk_kernel<T>), dim3((unsigned)num_tokens), dim3(64), 0, as_stream(stream), (const T*)gating, (const float*)nullptr, topk_weights, topk_ids, num_experts, topk, 1, 1, renormalize, 1, 0, (const float*)nullptr, 0, (int64_t)0, renorm_eps));
+  SEMIPD_DISPATCH_DTYPE(dtype, T, SEMIPD_TOPK((const T*)gating, (const float*)nullptr, topk_weights, topk_ids, num_experts, topk, 1, 1, renormalize, 1, 0, (const float*)nullptr, 0, (int64_t)0, renorm_eps));
   return launch_status("topk_sigmoid");
 }
 
@@ -647,7 +657,7 @@ int semipd_grouped_topk(const void* gating, const float* correction_bias, float*
   if (num_tokens == 0) return 0;
   SEMIPD_CHECK_ARG(gating && topk_weights && topk_ids, SEMIPD_EINVAL, "grouped_topk: null pointer");
   const int sc = correction_bias ? 1 : scoring;  // biased_grouped_topk always uses sigmoid
-  SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((moe_topk_kernel<T>), dim3((unsigned)num_tokens), dim3(64), 0, as_stream(stream), (const T*)gating, correction_bias, topk_weights, topk_ids, num_experts, topk, num_expert_group, topk_group, renormalize, sc, 1));
+  SEMIPD_DISPATCH_DTYPE(dtype, T, SEMIPD_TOPK((const T*)gating, correction_bias, topk_weights, topk_ids, num_experts, topk, num_expert_group, topk_group, renormalize, sc, 1));
   return launch_status("grouped_topk");
 }
 
@@ -665,7 +675,7 @@ int semipd_grouped_topk_planes(const float* planes, int n_planes, int64_t plane_
   SEMIPD_CHECK_ARG(dtype == SEMIPD_BF16 || dtype == SEMIPD_F16, SEMIPD_EDTYPE, "grouped_topk_planes: the router GEMM's "
                    "dtype (bf16 / f16) expected");
   const int sc = correction_bias ? 1 : scoring;
-  SEMIPD_DISPATCH_HALF(dtype, T, hipLaunchKernelGGL((moe_topk_kernel<T>), dim3((unsigned)num_tokens), dim3(64), 0, as_stream(stream), (const T*)nullptr, correction_bias, topk_weights, topk_ids, num_experts, topk, num_expert_group, topk_group, renormalize, sc, 1, planes, n_planes, plane_elems));
+  SEMIPD_DISPATCH_HALF(dtype, T, SEMIPD_TOPK((const T*)nullptr, correction_bias, topk_weights, topk_ids, num_experts, topk, num_expert_group, topk_group, renormalize, sc, 1, planes, n_planes, plane_elems));
   return launch_status("grouped_topk_planes");
 }
 

@@ -745,6 +745,16 @@ def test_topk_softmax_random(ops, device, T, E, k):
     _same_topk(w.cpu().numpy(), ids.cpu().numpy(), rw.numpy(), rids.numpy(), 1e-5, 1e-6)
 
 
+@pytest.mark.parametrize("E,k", [(1, 1), (63, 6), (64, 8), (65, 8), (128, 4), (129, 8), (256, 8), (257, 6), (512, 10)])
+def test_topk_softmax_experts_a_lane(ops, device, E, k):
+    """One, two, four and eight experts a lane: the edges of each."""
+    g = torch.Generator().manual_seed(E)
+    gate = torch.randn(7, E, generator=g)
+    w, ids = ops.topk_softmax(gate.to(device), k, False)
+    rw, rids = O.fused_topk_native(gate, k, False)
+    _same_topk(w.cpu().numpy(), ids.cpu().numpy(), rw.numpy(), rids.numpy(), 1e-5, 1e-6)
+
+
 @pytest.mark.parametrize("numel_tokens,topk,E,block", [(1, 6, 64, 64), (33, 6, 64, 64), (4096, 8, 256, 64), (5, 2, 8, 64)])
 def test_moe_align_block_size(ops, device, numel_tokens, topk, E, block):
     """Same comparison as sgl-kernel/tests/test_moe_align.py:151-222 (expert_ids, num_tokens_post_pad),
