@@ -9,9 +9,11 @@
 // Softmax bookkeeping is identical in the four waves, so nothing else is exchanged.
 // Bound: the flight time of the rows (40 MB of 32 requests at 1.1 k tokens are 8.4 us of a copy's time): at one or two workgroups a CU
 // a tile in flight each does not cover it, so two are, in registers.  With all of S^T made by every wave (36 products and 36 KB
-// of LDS reads a wave and tile, Q in 72 registers) the second set of rows would spill.  16 heads, bf16 rows, whole call with the merge of
-// the splits: 32 requests at 1.1 k tokens 24.1 -> 21.3 us (kernel 21.5 -> 18), on rows that no cache holds 25.8 -> 22.7; 1 at 300 19.1 -> 15.8, 160 at
-// 3 k 141 -> 131; fp8 rows 25.5 -> 20.9, 26.3 -> 22.1, 20.2 -> 15.9, 133 -> 108.
+// of LDS reads a wave and tile, Q in 72 registers) the second set of rows would spill.  Behind that the chain of a tile counts: a wave's
+// rows are addressed by scalars (no division, nine loads a tile without address arithmetic), two LDS images take turns (two barriers
+// a tile instead of three), only a request's last tile is masked, and partials leave in 16-byte stores: 1.55 -> 1.27 us a tile and
+// workgroup, 13.5 -> 13.0 us for a single tile with its merge.  16 heads, bf16 rows, whole call: 32 requests at 1.1 k tokens in 8 splits 21.5
+// -> 20.3 us (kernel 18.1 -> 16.7 under the profiler), in one split 73 -> 59, 64 at 1.1 k 30.3 -> 29.1, 128 at 2 k in 4 splits 75 -> 72.5 (fp8 rows 60 -> 54).
 //
 // Replaces _fwd_grouped_kernel_stage1 for Lk = 576 / Lv = 512
 // (layers/attention/triton_ops/decode_attention.py:234-390, BLOCK_DPE = 64 path).
@@ -56,14 +58,14 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
                   float logit_cap) {
   constexpr int DK = 576, DV = 512, KS = DK / 32, TOK = 32;
   constexpr int RS = DK * 2 + 64;  // 1216 B = 304 dwords = 48 (mod 64): conflict-free transposing reads
-  constexpr int CPR = DK / 8;      // 72 16-byte chunks per row
-  constexpr int NI = TOK * CPR / 256;  // 9 chunks per thread per tile
+  constexpr int RW = TOK / 4;          // rows of a tile that a wave fetches
   constexpr int DTW = DV / 16 / 4;     // 8 d-tiles of 16 per wave
   constexpr int KSW = KS / 2;          // k steps of S^T a wave
-  __shared__ __attribute__((aligned(16))) uint8_t tile[TOK * RS];
+  constexpr float kLog2e = 1.4426950408889634f, kLn2 = 0.6931471805599453f;
+  __shared__ __attribute__((aligned(16))) uint8_t tile[2][TOK * RS];
   __shared__ __attribute__((aligned(16))) f32x4 part[4][64];      // half sums of S^T: wave (token half, k half)
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c16 = lane & 15, q4 = lane >> 4;
   const int split = blockIdx.x % num_kv_splits;
   const int tmp = blockIdx.x / num_kv_splits;
@@ -86,58 +88,63 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
     return;
   }
 
+  const int32_t* idx_base = kv_indices + kv_start;
+  const int n_tiles = (s_end - s_begin + TOK - 1) / TOK;
+  using KVT = KVTraits<T, KV>;
+  // A wave fetches rows 8 wave .. + 7 of a tile: the first 512 elements of each in one load of all lanes, whose address is the wave's
+  // (slot of the row from a lane register) plus 8 elements a lane, and the last 64 of the eight rows in a ninth.
+  // Two tiles in flight, in two sets of registers; nothing of it is conditional (rows past the end: the last row, zeroed on its way into
+  // LDS), so that the wait for the older tile's rows leaves the younger one's in flight.
+  typename KVT::Raw reg[2][RW + 1];
+  auto load_idx = [&](int ti) __attribute__((always_inline)) { return idx_base[min(s_begin + ti * TOK + wave * RW + (lane >> 3), s_end - 1)]; };
+  auto fetch = [&](typename KVT::Raw (&to)[RW + 1], int32_t idx) __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+      to[r] = KVT::load8(kv_buf + (int64_t)__builtin_amdgcn_readlane(idx, 8 * r) * kvbuf_stride + lane * 8);
+    to[RW] = KVT::load8(kv_buf + (int64_t)idx * kvbuf_stride + DV + (lane & 7) * 8);
+  };
+
+  // (memory answers in order: the slots of a tile are asked for in front of the rows of the tile before it)
+  int32_t idx0 = load_idx(0), idx1 = load_idx(1);
+  fetch(reg[0], idx0);
+  idx0 = load_idx(2);
+  fetch(reg[1], idx1);
+
   // Q^T fragments of this wave's k half (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
   const int ks0 = (wave >> 1) * KSW;
   FragM qf[KSW];
+  {
+    const T* qrow = q + (int64_t)b * q_stride + (int64_t)(h0 + min(c16, heads - 1)) * DK + ks0 * 32 + q4 * 8;
 #pragma unroll
-  for (int ks = 0; ks < KSW; ++ks) {
-    qf[ks].u = make_uint4(0, 0, 0, 0);
-    if (head_ok)
-      qf[ks].u = *reinterpret_cast<const uint4*>(q + (int64_t)b * q_stride + (int64_t)(h0 + c16) * DK +
-                                                 (ks0 + ks) * 32 + q4 * 8);
+    for (int ks = 0; ks < KSW; ++ks) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + ks * 32);      // (heads past the last: not stored)
   }
   f32x4 o_acc[DTW];
 #pragma unroll
   for (int t = 0; t < DTW; ++t) o_acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;                 // (in units of log 2)
+  const float scale2 = sm_scale * kLog2e;
 
-  const int32_t* idx_base = kv_indices + kv_start;
-  const int n_tiles = (s_end - s_begin + TOK - 1) / TOK;
-  using KVT = KVTraits<T, KV>;
-  // Two tiles in flight, in two sets of registers; nothing of it is conditional (rows past the end: the last row, zeroed on its way into
-  // LDS), so that the wait for the older tile's rows leaves the younger one's in flight.
-  int32_t idx[2][NI];
-  typename KVT::Raw reg[2][NI];
-  auto load_idx = [&](int ti, int32_t (&idx)[NI]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) idx[i] = idx_base[min(s_begin + ti * TOK + (tid + i * 256) / CPR, s_end - 1)];
-  };
-  auto fetch = [&](typename KVT::Raw (&to)[NI], const int32_t (&idx)[NI]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < NI; ++i) to[i] = KVT::load8(kv_buf + (int64_t)idx[i] * kvbuf_stride + (tid + i * 256) % CPR * 8);
-  };
+  uint8_t* const wrow = &tile[0][0] + wave * RW * RS + lane * 16;                                   // + r * RS
+  uint8_t* const wtail = &tile[0][0] + (wave * RW + (lane >> 3)) * RS + DV * 2 + (lane & 7) * 16;
+  const uint8_t* const krow = &tile[0][0] + ((wave & 1) * 16 + c16) * RS + ks0 * 64 + q4 * 16;       // + ks*64
+  const uint8_t* const vrow = &tile[0][0] + (q4 * 4 + (c16 >> 2)) * RS + (c16 & 3) * 8 + wave * 256;  // + dt*32 (+16*RS)
 
-  const uint8_t* krow = tile + ((wave & 1) * 16 + c16) * RS + ks0 * 64 + q4 * 16;       // + ks*64
-  const uint8_t* vrow = tile + (q4 * 4 + (c16 >> 2)) * RS + (c16 & 3) * 8 + wave * 256;  // + dt*32 (+16*RS)
-
-  // (memory answers in order: the slots of a tile are asked for in front of the rows of the tile before it)
-  load_idx(0, idx[0]);
-  load_idx(1, idx[1]);
-  fetch(reg[0], idx[0]);
-  load_idx(2, idx[0]);
-  fetch(reg[1], idx[1]);
-  auto step = [&](int ti, typename KVT::Raw (&rows)[NI], const int32_t (&after_next)[NI], int32_t (&behind)[NI]) __attribute__((always_inline)) {
-    __syncthreads();  // every wave is done with the previous tile
+  // Tiles alternate between two LDS images: rows of the next one are written while slower waves still multiply this one's, and what
+  // every wave has read is behind the two barriers in between.
+  auto step = [&](int ti, auto buf_c, typename KVT::Raw (&rows)[RW + 1], int32_t after_next, int32_t& behind) __attribute__((always_inline)) {
+    constexpr int buf = decltype(buf_c)::value * TOK * RS;
+    const int n_rows = s_end - (s_begin + ti * TOK);          // rows of this tile and behind it
+    if (n_rows < TOK) {                                       // (0 * garbage could be NaN)
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int item = tid + i * 256;
-      const int r = item / CPR, ch = item - r * CPR;
-      uint4 v = KVT::expand(rows[i]);
-      if (s_begin + ti * TOK + r >= s_end) v = uint4{0u, 0u, 0u, 0u};      // (0 * garbage could be NaN)
-      *reinterpret_cast<uint4*>(tile + r * RS + ch * 16) = v;
+      for (int r = 0; r < RW; ++r)
+        if (wave * RW + r >= n_rows) rows[r] = KVT::zero();
+      if (wave * RW + (lane >> 3) >= n_rows) rows[RW] = KVT::zero();
     }
+#pragma unroll
+    for (int r = 0; r < RW; ++r) *reinterpret_cast<uint4*>(wrow + buf + r * RS) = KVT::expand(rows[r]);
+    *reinterpret_cast<uint4*>(wtail + buf) = KVT::expand(rows[RW]);
     __syncthreads();
-    load_idx(ti + 3, behind);
+    behind = load_idx(ti + 3);
     fetch(rows, after_next);
 
     // ---- S^T = tile x Q^T: a wave 16 of the tokens and half of k, the halves added by every wave ----
@@ -147,7 +154,7 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
 #pragma unroll
       for (int ks = 0; ks < KSW; ++ks) {
         FragM a;
-        a.u = *reinterpret_cast<const uint4*>(krow + ks * 64);
+        a.u = *reinterpret_cast<const uint4*>(krow + buf + ks * 64);
         if (ks & 1) s1 = MfmaM<T>::mma(a, qf[ks], s1);
         else s = MfmaM<T>::mma(a, qf[ks], s);
       }
@@ -157,24 +164,31 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
 #pragma unroll
     for (int t = 0; t < 2; ++t) s_acc[t] = part[t][lane] + part[t + 2][lane];
     // ---- online softmax: lane = head c16, tokens t*16 + q4*4 + r ----
-    const int base_tok = s_begin + ti * TOK;
-    float mx = -INFINITY;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        float s = s_acc[t][rr] * sm_scale;
-        if (logit_cap > 0.f) s = logit_cap * tanhf(s / logit_cap);
-        s = (base_tok + t * 16 + q4 * 4 + rr < s_end) ? s : -INFINITY;
-        s_acc[t][rr] = s;
-        mx = fmaxf(mx, s);
-      }
+      for (int rr = 0; rr < 4; ++rr)
+        s_acc[t][rr] = logit_cap > 0.f ? logit_cap * kLog2e * tanhf(s_acc[t][rr] * sm_scale / logit_cap) : s_acc[t][rr] * scale2;
+    if (n_rows < TOK) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr)
+          if (t * 16 + q4 * 4 + rr >= n_rows) s_acc[t][rr] = -INFINITY;
     }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    float mx = fmaxf(fmaxf(fmaxf(s_acc[0][0], s_acc[0][1]), fmaxf(s_acc[0][2], s_acc[0][3])),
+                     fmaxf(fmaxf(s_acc[1][0], s_acc[1][1]), fmaxf(s_acc[1][2], s_acc[1][3])));
+    {
+      const auto sw = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
+    {
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
     const float m_new = fmaxf(m_run, mx);
     if (__any(m_new > m_run)) {
-      const float alpha = (m_run == -INFINITY) ? 0.f : __expf(m_run - m_new);
+      const float alpha = (m_run == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
 #pragma unroll
       for (int t = 0; t < DTW; ++t) o_acc[t] *= alpha;
@@ -187,7 +201,7 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        const float p = __expf(s_acc[t][rr] - m_use);
+        const float p = __builtin_amdgcn_exp2f(s_acc[t][rr] - m_use);
         psum += p;
         pf.e[t * 4 + rr] = Elem<T>::from_f(p).v;
       }
@@ -197,16 +211,16 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
 #pragma unroll
     for (int dt = 0; dt < DTW; ++dt) {
       FragM a;
-      a.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + dt * 32));
+      a.s[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(vrow + buf + dt * 32));
       a.s[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) s16x4*)(vrow + 16 * RS + dt * 32));
+          (__attribute__((address_space(3))) s16x4*)(vrow + buf + 16 * RS + dt * 32));
       o_acc[dt] = MfmaM<T>::mma(a, pf, o_acc[dt]);
     }
   };
   for (int ti = 0;;) {
-    step(ti, reg[0], idx[0], idx[1]);
+    step(ti, std::integral_constant<int, 0>{}, reg[0], idx0, idx1);
     if (++ti >= n_tiles) break;
-    step(ti, reg[1], idx[1], idx[0]);
+    step(ti, std::integral_constant<int, 1>{}, reg[1], idx1, idx0);
     if (++ti >= n_tiles) break;
   }
 
@@ -226,13 +240,12 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
       *reinterpret_cast<uint2*>(orow + dt * 16 + q4 * 4) = w;
     }
   } else {
+    // (rows of 513 floats: 16 bytes a lane at the alignment of one float, which global memory takes)
+    typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
     float* dst = attn_logits + (((int64_t)b * num_q_heads + hq) * num_kv_splits + split) * (DV + 1);
 #pragma unroll
-    for (int dt = 0; dt < DTW; ++dt) {
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) dst[wave * 128 + dt * 16 + q4 * 4 + rr] = o_acc[dt][rr] * inv;
-    }
-    if (wave == 0 && q4 == 0) dst[DV] = m_run + __logf(l_tot);
+    for (int dt = 0; dt < DTW; ++dt) *reinterpret_cast<f32x4_any*>(dst + wave * 128 + dt * 16 + q4 * 4) = o_acc[dt] * inv;
+    if (wave == 0 && q4 == 0) dst[DV] = m_run * kLn2 + __logf(l_tot);
   }
 }
 

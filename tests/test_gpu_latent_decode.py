@@ -59,3 +59,31 @@ def test_infinity_in_the_last_row_of_a_request(splits):
     assert bool(torch.isfinite(out[torch.arange(len(LENS)) != 3]).all())
     keep = torch.arange(512) != column
     assert bool(torch.isfinite(out[3][:, keep]).all()) and not bool(torch.isfinite(out[3][:, column]).any())
+
+
+@pytest.mark.parametrize("cap", [0.0, 3.0])
+@pytest.mark.parametrize("rows", ["same", "e4m3", "e5m2"])
+@pytest.mark.parametrize("heads", [5, 16])
+def test_rows_of_every_type_and_capped_scores(heads, rows, cap):
+    """Lengths that end in every place of a wave's eight rows, the last row of a tile among them; weights and result are rounded to bf16
+    (see above), values are at most 6.  An fp8 row is exact in bf16."""
+    from semi_pd_amd import ops
+    lens = [8, 15, 23, 40, 57, 64, 95, 161]
+    g = torch.Generator(device=DEV).manual_seed(heads)
+    total = sum(lens)
+    kind = {"same": torch.bfloat16, "e4m3": torch.float8_e4m3fn, "e5m2": torch.float8_e5m2}[rows]
+    kv = torch.randn(total + 1, 1, 576, generator=g, device=DEV).to(kind)
+    slots = torch.randperm(total, generator=g, device=DEV).int() + 1
+    q = torch.randn(len(lens), heads, 576, generator=g, device=DEV).bfloat16()
+    indptr = torch.tensor([0] + lens, device=DEV).cumsum(0).int()
+    out = torch.empty(len(lens), heads, 512, device=DEV, dtype=torch.bfloat16)
+    ops.decode_attention_fwd(q, kv, kv[..., :512], out, indptr, slots, None, 1, 192 ** -0.5, cap)
+    parts = torch.empty(len(lens), heads, 3, 513, device=DEV)
+    split = torch.empty_like(out)
+    ops.decode_attention_fwd(q, kv, kv[..., :512], split, indptr, slots, parts, 3, 192 ** -0.5, cap)
+    for b, n in enumerate(lens):
+        r = kv[slots[indptr[b]: indptr[b + 1]].long(), 0].double().cpu()
+        s = q[b].double().cpu() @ r.t() * 192 ** -0.5
+        want = torch.softmax(cap * torch.tanh(s / cap) if cap else s, -1) @ r[:, :512]
+        for got in (out, split):
+            torch.testing.assert_close(got[b].double().cpu(), want, rtol=2.0 ** -8, atol=6 * 2.0 ** -8)
