@@ -653,6 +653,10 @@ gemm4w_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
   }
 }
 
+}  // namespace semipd
+#include "moe_gemm_rows.h"
+namespace semipd {
+
 // out[m, n] = T(sum_z planes[z][m][n]) in slice order (SiLU * mul variant: gate / up columns n, n + N / 2)
 template <typename T, int EPI>
 __global__ void __launch_bounds__(256)
@@ -788,6 +792,16 @@ static int g8_launch(T* out, float* planes, size_t planes_bytes, const T* x, con
   return g8_launch_geo<T, EPI, 128>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks);
 }
 
+template <typename T, int EPI>
+static int g8_launch_rows(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, hipStream_t st) {
+  const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N, cols_per_tile = EPI == G8_SILU_MUL ? RowsTile::kCols / 2 : RowsTile::kCols;
+  const int64_t tiles = max_sorted / RowsTile::kRows * ((n_cols + cols_per_tile - 1) / cols_per_tile);
+  static std::atomic<uint64_t> lds_ok{0};
+  if (ensure_dynamic_lds((const void*)moe_gemm_rows_kernel<T, EPI>, RowsTile::kLds, lds_ok, "moe_gemm_rows")) return 1;
+  hipLaunchKernelGGL((moe_gemm_rows_kernel<T, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), RowsTile::kLds, st, c, a, w, N, K, grp);
+  return launch_status("moe_gemm_rows");
+}
+
 template <typename T, int EPI, int XH>
 static int g8_launch_grouped(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, int64_t lda,
                              int64_t ldc, hipStream_t st) {
@@ -899,15 +913,21 @@ int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* top
                    "moe_gemm_tall: null pointer");
   SEMIPD_CHECK_ARG(!mul_routed_weight || topk_weights, SEMIPD_EINVAL, "moe_gemm_tall: topk_weights required");
   const int64_t n_out = fuse_silu_mul ? n / 2 : n;
-  SEMIPD_CHECK_ARG((block_m == 256 || block_m == 128) && max_sorted % block_m == 0 && k % 64 == 0 && n_out % 16 == 0 && (!fuse_silu_mul || n % 2 == 0) && aligned16(a) &&
+  SEMIPD_CHECK_ARG(block_m != RowsTile::kRows || (k % 128 == 0 && n * k < (1 << 30) && ((num_valid - 1) / top_k_div + 1) * k < (1 << 30)), SEMIPD_ESHAPE,
+                   "moe_gemm_tall: blocks of 320 rows need k %% 128 and operands below 2 GiB");
+  SEMIPD_CHECK_ARG((block_m == 320 || block_m == 256 || block_m == 128) && max_sorted % block_m == 0 && k % 64 == 0 && n_out % 16 == 0 && (!fuse_silu_mul || n % 2 == 0) && aligned16(a) &&
                        aligned16(w) && (reinterpret_cast<uintptr_t>(c) & 7u) == 0 && num_valid < (1 << 30) && n < (1 << 30) &&
                        k < (1 << 30),
-                   SEMIPD_ESHAPE, "moe_gemm_tall: block size 256 or 128, k %% 64, output width %% 16 required");
+                   SEMIPD_ESHAPE, "moe_gemm_tall: block size 320, 256 or 128, k %% 64, output width %% 16 required");
   G8Group grp{sorted_token_ids, expert_ids, num_tokens_post_pad, topk_weights, (int)num_valid, top_k_div, mul_routed_weight};
   int rc = 0;
 #define G8G(EPIV, XHV) \
   SEMIPD_DISPATCH_HALF(dtype, T, rc = (g8_launch_grouped<T, EPIV, XHV>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k, k, n_out, as_stream(stream))))
-  if (block_m == 256) {
+  if (block_m == RowsTile::kRows) {
+#define G8R(EPIV) SEMIPD_DISPATCH_HALF(dtype, T, rc = (g8_launch_rows<T, EPIV>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k, as_stream(stream))))
+    if (fuse_silu_mul) { G8R(G8_SILU_MUL); } else { G8R(G8_PLAIN); }
+#undef G8R
+  } else if (block_m == 256) {
     if (fuse_silu_mul) { G8G(G8_SILU_MUL, 128); } else { G8G(G8_PLAIN, 128); }
   } else {
     if (fuse_silu_mul) { G8G(G8_SILU_MUL, 64); } else { G8G(G8_PLAIN, 64); }

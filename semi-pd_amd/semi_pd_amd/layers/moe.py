@@ -79,6 +79,19 @@ MOE_STREAM_DECODE = os.environ.get("SEMIPD_MOE_STREAM_DECODE", "1") != "0"   # A
 MOE_STREAM_MAX_TOKENS = int(os.environ.get("SEMIPD_MOE_STREAM_MAX_TOKENS", "320"))
 
 
+def _tall_block(block_m: int, tokens: int, topk: int, E: int, K: int, F: int) -> int:
+    """Rows per block of a call that the tiled kernels take in blocks of `block_m`: 320, where the kernel whose tiles are as tall as
+    their expert needs takes both products (K and F in pairs of 64, 32-bit offsets into the operands) and is ahead.  Whole layer, both
+    products, blocks of 128 or 256 / of 320, us: 64 experts of 2048 x 1408, top 6, 400 tokens 255 / 248, 1000 273 / 255, 2000 322 / 310,
+    3001 474 / 361, 6000 739 / 640, 8192 903 / 870; 8 of 4096 x 14336, top 2, 512 tokens 795 / 611, 4096 2550 / 2450; 16 of 2048 x 1408, top 2, 1024
+    tokens 86 / 84, 4096 203 / 183.  Behind with few K steps, whose loads ahead are not covered (256 experts of 7168 x 256, 1024 tokens
+    554 / 630: its second product has four), and where its tiles are too few for the chip."""
+    numel = tokens * topk
+    wide = (ops.MOE_TALL_BLOCK_M == 256 and K % 128 == 0 and F % 128 == 0 and min(K, F) >= 512 and 2 * F * K < 1 << 30
+            and tokens * K < 1 << 30 and numel * F < 1 << 30 and max(E, numel // ops.MOE_ROWS_BLOCK_M) * (F // 128) >= 128)
+    return ops.MOE_ROWS_BLOCK_M if wide else block_m
+
+
 def _local_ids(topk_ids: torch.Tensor, expert_offset: int) -> torch.Tensor:
     """Expert-parallel ranks hold experts [offset, offset + E_local): ids are shifted so that the local ones land
     in [0, E_local); the others fall outside and moe_align_block_size drops them (their rows of the output stay
@@ -133,7 +146,7 @@ def fused_experts(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.Tenso
         tall, tall_block = True, 128
     else:
         tall_block = ops.MOE_TALL_BLOCK_M
-    block_m = tall_block if tall else (min(64, 16 * -(-T // 16)) if small else
+    block_m = _tall_block(tall_block, T, topk, E, K, N2 // 2) if tall else (min(64, 16 * -(-T // 16)) if small else
                                        (MOE_BLOCK_M if numel <= 2048 else 2 * MOE_BLOCK_M))
     max_sorted = -(-(numel + E * (block_m - 1)) // block_m) * block_m
     sorted_ids = torch.empty(max_sorted, dtype=torch.int32, device=dev)
@@ -392,7 +405,7 @@ def fused_experts_ungated(hidden_states: torch.Tensor, w_up: torch.Tensor, w_dow
     if not tall and not small and (numel >= MOE_MID_MIN_ROWS_PER_EXPERT * E and ops.moe_gemm_tall_is_supported(hidden_states, w_up, False)
                                    and F % 64 == 0 and K % 16 == 0):
         tall, tall_block = True, 128
-    block_m = tall_block if tall else (min(64, 16 * -(-T // 16)) if small else MOE_BLOCK_M)
+    block_m = _tall_block(tall_block, T, topk, E, K, F) if tall else (min(64, 16 * -(-T // 16)) if small else MOE_BLOCK_M)
     max_sorted = -(-(numel + E * (block_m - 1)) // block_m) * block_m
     sorted_ids = torch.empty(max_sorted, dtype=torch.int32, device=dev)
     expert_ids = torch.empty((max_sorted + block_m - 1) // block_m, dtype=torch.int32, device=dev)
@@ -496,7 +509,7 @@ def fused_experts_clamped(hidden_states: torch.Tensor, w13: torch.Tensor, w2: to
     if not tall and not small and (numel >= MOE_MID_MIN_ROWS_PER_EXPERT * E and ops.moe_gemm_tall_is_supported(hidden_states, w13, False)
                                    and F % 64 == 0 and K % 16 == 0):
         tall, tall_block = True, 128
-    block_m = tall_block if tall else (min(64, 16 * -(-T // 16)) if small else MOE_BLOCK_M)
+    block_m = _tall_block(tall_block, T, topk, E, K, F) if tall else (min(64, 16 * -(-T // 16)) if small else MOE_BLOCK_M)
     max_sorted = -(-(numel + E * (block_m - 1)) // block_m) * block_m
     sorted_ids = torch.empty(max_sorted, dtype=torch.int32, device=dev)
     expert_ids = torch.empty((max_sorted + block_m - 1) // block_m, dtype=torch.int32, device=dev)

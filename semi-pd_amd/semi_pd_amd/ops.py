@@ -1102,6 +1102,9 @@ import os as _os
 MOE_TALL_BLOCK_M = int(_os.environ.get("SEMIPD_MOE_TALL_BLOCK_M", "256"))   # 256: 256 x 256 tiles; 128: 128 x 512 tiles
 
 
+MOE_ROWS_BLOCK_M = 320                                                       # up to 320 rows x 256 columns (csrc/moe_gemm_rows.h)
+
+
 def moe_gemm_tall_is_supported(a: torch.Tensor, w: torch.Tensor, fuse_silu_mul: bool) -> bool:
     E, N, K = w.shape
     n_out = N // 2 if fuse_silu_mul else N
@@ -1114,14 +1117,15 @@ def moe_gemm_tall(a: torch.Tensor, w: torch.Tensor, c: torch.Tensor, topk_weight
                   num_valid: int, top_k_div: int, mul_routed_weight: bool, fuse_silu_mul: bool = False,
                   block_m: Optional[int] = None) -> None:
     """invoke_fused_moe_kernel (fused_moe.py:501-612) for prefill-sized calls with the ping-pong tile kernel
-    (csrc/gemm8p.hip, grouped form; 256 x 256 tiles for block_m = 256, 128 rows x 512 columns for block_m = 128):
+    (csrc/gemm8p.hip, grouped form; 256 x 256 tiles for block_m = 256, 128 rows x 512 columns for block_m = 128) or, block_m =
+    320, the one whose tiles are as tall as their expert needs up to 320 rows (csrc/moe_gemm_rows.h: K % 128 == 0):
     sorted_token_ids / expert_ids must come from moe_align_block_size with block size block_m (default
     MOE_TALL_BLOCK_M).  c[id] = a[id // top_k_div] @ w[expert].T (SiLU(gate) * up of it with fuse_silu_mul)."""
     E, N, K = w.shape
     n_out = N // 2 if fuse_silu_mul else N
     block_m = MOE_TALL_BLOCK_M if block_m is None else int(block_m)
     if not moe_gemm_tall_is_supported(a, w, fuse_silu_mul) or c.shape[-1] != n_out or not c.is_contiguous() \
-            or block_m not in (128, 256) or sorted_token_ids.numel() % block_m:
+            or block_m not in (128, 256, MOE_ROWS_BLOCK_M) or sorted_token_ids.numel() % block_m:
         raise RuntimeError("moe_gemm_tall: shape / contiguity / block-size mismatch")
     if sorted_token_ids.dtype != torch.int32 or expert_ids.dtype != torch.int32 or num_tokens_post_pad.dtype != torch.int32:
         raise RuntimeError("moe_gemm_tall: int32 routing tensors expected")
