@@ -339,8 +339,8 @@ int semipd_moe_stream_gemm(void* c, const void* a, const void* w, const float* t
 
 /* The grouped form of the tiled ping-pong GEMM for the fused-MoE expert GEMMs of prefill-sized calls
  * (invoke_fused_moe_kernel, python/sglang/srt/layers/moe/fused_moe_triton/fused_moe.py:501-612; kernel :54-273):
- * sorted_token_ids / expert_ids from semipd_moe_align_block_size with block size block_m = 256 (256 x 256 tiles) or 128
- * (128 x 512 tiles): one expert per tile; max_sorted = entries of sorted_token_ids, a multiple of block_m.  c[id, :] = a[id / top_k_div, :] @ w[expert]^T for every
+ * sorted_token_ids / expert_ids from semipd_moe_align_block_size with block size block_m = 256 (256 x 256 tiles), 128
+ * (128 x 512 tiles) or 320 (up to 320 x 256; k % 128 == 0, operands below 2 GiB): one expert per tile; max_sorted = entries of sorted_token_ids, a multiple of block_m.  c[id, :] = a[id / top_k_div, :] @ w[expert]^T for every
  * routed entry id < num_valid, times topk_weights[id] when mul_routed_weight; fuse_silu_mul: w[e] = merged [gate; up]
  * ([n, k], output width n / 2) and c = SiLU(gate) * up of the products rounded to dtype (the bits of the unfused pair). */
 int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* topk_weights, const int32_t* sorted_token_ids,
@@ -529,7 +529,7 @@ int semipd_moe_align_block_size(const int32_t* topk_ids, int64_t numel, int num_
  * token(r) = sorted_token_ids[r] / top_k_div (top_k_div=topk for GEMM1 where A is
  * [T,K]; 1 for GEMM2 where A is [T*k,K]); rows with id >= num_valid are skipped.
  * mul_routed_weight multiplies each output row by topk_weights[sorted id].
- * C is [T*k, N] indexed by the sorted id.  block_m (64 or 128) must equal the block_size used in
+ * C is [T*k, N] indexed by the sorted id.  block_m (64 or 128; 16 or 32 with k % 128 == 0, k <= 8192, n % 16 == 0) must equal the block_size used in
  * semipd_moe_align_block_size: 64 for decode batches, 128 for prefill chunks (one pass over an
  * expert's weights per block_m rows routed to it).
  * replaces fused_moe_kernel / invoke_fused_moe_kernel

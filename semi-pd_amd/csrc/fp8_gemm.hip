@@ -485,6 +485,11 @@ static int check_fp8_gemm_args(const char* what, int64_t N, int64_t K, int block
   return 0;
 }
 
+// fp8_stream.hip
+int launch_fp8_stream_grouped(void* c, const void* a, const float* a_s, const void* w, const float* w_s, const float* topk_weights,
+                              const int32_t* sorted_ids, const int32_t* expert_ids, const int32_t* num_post_pad, int num_valid, int N, int K,
+                              int blocks, int block_m, int block_n, int top_k_div, int mul_routed_weight, int out_dtype, hipStream_t st);
+
 }  // namespace semipd
 
 using namespace semipd;
@@ -582,11 +587,18 @@ int semipd_moe_grouped_gemm_fp8(void* c, const void* a_q, const float* a_s, cons
   SEMIPD_CHECK_ARG(c && a_q && a_s && w_q && w_s && sorted_token_ids && expert_ids && num_tokens_post_pad, SEMIPD_EINVAL,
                    "moe_grouped_gemm_fp8: null pointer");
   SEMIPD_CHECK_ARG(!mul_routed_weight || topk_weights, SEMIPD_EINVAL, "moe_grouped_gemm_fp8: routed weights missing");
-  SEMIPD_CHECK_ARG(block_m == 64 || block_m == 128, SEMIPD_ESHAPE, "moe_grouped_gemm_fp8: block_m must be 64 or 128");
+  // blocks of up to 64 rows: the LDS-DMA stream where its shapes allow (whole scale blocks of at most 8192 bytes of K, groups of 16 columns)
+  const bool stream_ok = k % 128 == 0 && k <= 8192 && n % 16 == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && num_valid < (1 << 30) && n < (1 << 30);
+  SEMIPD_CHECK_ARG(block_m == 64 || block_m == 128 || ((block_m == 16 || block_m == 32) && stream_ok), SEMIPD_ESHAPE,
+                   "moe_grouped_gemm_fp8: block_m must be 64 or 128 (16 or 32: K %% 128, K <= 8192, N %% 16)");
   SEMIPD_CHECK_ARG(top_k_div >= 1 && max_sorted >= 0, SEMIPD_ESHAPE, "moe_grouped_gemm_fp8: top_k_div %d, max_sorted %lld",
                    top_k_div, (long long)max_sorted);
   if (int rc = check_fp8_gemm_args("moe_grouped_gemm_fp8", n, k, block_n, block_k, a_q, w_q)) return rc;
   if (num_valid == 0 || max_sorted == 0) return 0;
+  if (block_m <= 64 && stream_ok)
+    return launch_fp8_stream_grouped(c, a_q, a_s, w_q, w_s, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, (int)num_valid, (int)n,
+                                     (int)k, (int)((max_sorted + block_m - 1) / block_m), block_m, block_n, top_k_div, mul_routed_weight, out_dtype,
+                                     static_cast<hipStream_t>(stream));
   return dispatch_fp8_gemm<true>(c, a_q, a_s, w_q, w_s, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad,
                                  num_valid, 0, n, k, n, (max_sorted + block_m - 1) / block_m, block_m, block_n, top_k_div,
                                  mul_routed_weight,
