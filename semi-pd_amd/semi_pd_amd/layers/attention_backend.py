@@ -428,6 +428,12 @@ class HipAttnBackend(AttentionBackend):
             return 4
         if 2 * wgs >= cus or knob == "2":
             return 8
+        # contexts of up to eight splits are the eight waves of one workgroup: one launch instead of three, on however few CUs.  Four layers
+        # + head, 333 tokens, us, three launches / one: 8 kv heads of 128, 1 request 475 / 455, 2 requests 478 / 457; of 64 261 / 237 and 269 / 243; 2 kv
+        # heads of 128, hidden 8192, 1 request 532 / 525, 3 requests 551 / 536.  A single kv head is one CU a request: 60 tokens 370 / 372, 2
+        # requests 372 / 383, 500 tokens 403 / 408.
+        if knob != "4" and 1 <= num_kv_splits <= 8 and self.num_kv_head >= 2:
+            return 8
         # several workgroups per pair: worth it from about one workgroup per eight CUs (Llama-3-8B from one request: step
         # alone 3.32 -> 3.25 ms, at 8 requests 3.65 -> 3.44; the 70B TP = 8 rank's single kv head at 1 .. 8 requests: 16 .. 32
         # workgroups, 0.5-1 % slower than the separate launches, profiles/r06_decode_step_small_batches.txt)

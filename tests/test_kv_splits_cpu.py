@@ -74,3 +74,24 @@ def test_fused_decode_launch_rule(monkeypatch):
     assert b.fused_decode_waves(1, 128) == 8 and b.fused_decode_zsplits(1, 32) == 1 and b.fused_decode_waves(256, 128) == 4
     monkeypatch.setenv("SEMIPD_FUSED_DECODE_ATTN", "4")                  # only where one workgroup per pair fills the chip
     assert [b.fused_decode_waves(n, 128) for n in (1, 15, 16, 64)] == [0, 0, 8, 4]
+
+
+def test_short_contexts_of_few_requests_take_one_launch(monkeypatch):
+    """Up to eight splits are the waves of one workgroup per (request, kv head): the fused launch with nothing behind it, whatever the
+    number of workgroups; more splits and a single kv head keep the rule by workgroups."""
+    import types
+    import torch
+    from semi_pd_amd.layers.attention_backend import HipAttnBackend
+    monkeypatch.delenv("SEMIPD_FUSED_DECODE_ATTN", raising=False)
+
+    def backend(heads, kv_heads):
+        return HipAttnBackend(types.SimpleNamespace(
+            device="cpu", num_attention_heads_local=heads, num_kv_heads_local=kv_heads, v_head_dim=128, max_context_len=8192, num_kv_splits=None,
+            req_to_token_pool=types.SimpleNamespace(req_to_token=None), kv_geometry={"kind": "mha"}, num_cus_owned=256, dtype=torch.bfloat16,
+            kv_cache_dtype=torch.bfloat16))
+
+    b = backend(32, 8)
+    assert [b.fused_decode_waves(1, 128, s) for s in (1, 5, 8, 9, 32)] == [8, 8, 8, 0, 8]
+    assert [b.fused_decode_zsplits(1, s) for s in (1, 5, 8)] == [1, 1, 1]
+    assert [backend(16, 2).fused_decode_waves(1, 128, s) for s in (8, 9)] == [8, 0]
+    assert backend(8, 1).fused_decode_waves(1, 128, 5) == 0
