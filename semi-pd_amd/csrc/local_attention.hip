@@ -520,6 +520,92 @@ __global__ void __launch_bounds__(256) talk_mix_mfma_kernel(const T* __restrict_
   for (int i = tid; i < H * E / 8; i += 256) *reinterpret_cast<uint4*>(out + t * out_ld + i * 8) = *reinterpret_cast<const uint4*>(o_l + i * 8);
 }
 
+// The same where a value row is a multiple of 64 elements: a lane reads four neighbouring elements of a head's row at a time, row r16 of
+// four tiles (elements 4 r16 + j of 64), so a wave takes 64 elements by up to 16 heads with a quarter of the LDS reads, and the 16 sums of a
+// lane are 16 neighbouring elements of one head: they leave in two 16-byte stores without LDS.  The mix lies in LDS once for all tokens of
+// a workgroup, which fetches its next token while it multiplies one (8-byte reads of the four lane groups start 32 banks apart: 32 bytes
+// behind every head).  Bound by HBM: 7262 tokens, 32 heads over 2 of 128 (178 MB) 39 us for the 64 of the form above,
+// of 64 24 for 58, 48 heads over 2 of 64 44 for 125, 32 tokens 3.9 for 5.7; the same bits.
+template <typename T, int KT>           // heads up to 16 KT
+__global__ void __launch_bounds__(256) talk_mix_rows_kernel(const T* __restrict__ parts, int64_t p_ld, const float* __restrict__ talk,
+                                                            T* __restrict__ out, int64_t out_ld, int64_t tokens, int H, int G, int E) {
+  constexpr int TS = 16 * KT + 4, AHEAD = 4;                    // floats between the mix's rows; 16-byte pieces a thread fetches ahead
+  extern __shared__ __attribute__((aligned(16))) uint8_t mix_b[];     // mix [H][TS] | H rows of G * E elements + 32 bytes
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r16 = lane & 15, kq = lane >> 4;
+  const int row = G * E, rs = row * 2 + 32, per = H / G, pieces = row / 8, n = H * pieces;
+  float* const mix = reinterpret_cast<float*>(mix_b);
+  uint8_t* const rows = mix_b + (size_t)H * TS * 4;
+  for (int i = tid; i < H * 16 * KT; i += 256) {
+    const int h = i / (16 * KT), g = i % (16 * KT);
+    mix[h * TS + g] = g < H ? talk[(int64_t)h * H + g] : 0.f;
+  }
+  int at[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) {
+    const int i = tid + u * 256;
+    at[u] = i / pieces * rs + i % pieces * 16;
+  }
+  u32x4 next[AHEAD];
+  auto fetch = [&](int64_t t) __attribute__((always_inline)) {
+    const T* p = parts + t * p_ld;
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) next[u] = *reinterpret_cast<const u32x4*>(p + (int64_t)min(tid + u * 256, n - 1) * 8);
+  };
+  const int ht = (per + 15) / 16, eg = E / 64, units = G * ht * eg;
+  int64_t t = blockIdx.x;
+  fetch(t);                                                     // (as many workgroups as tokens at most)
+  for (; t < tokens; t += gridDim.x) {
+    __syncthreads();                                            // everyone is done with the token before
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (tid + u * 256 < n) *reinterpret_cast<u32x4*>(rows + at[u]) = next[u];
+    for (int i = tid + AHEAD * 256; i < n; i += 256)
+      *reinterpret_cast<uint4*>(rows + i / pieces * rs + i % pieces * 16) = *reinterpret_cast<const uint4*>(parts + t * p_ld + (int64_t)i * 8);
+    __syncthreads();
+    if (t + gridDim.x < tokens) fetch(t + gridDim.x);
+    for (int unit = wave; unit < units; unit += 4) {
+      const int ch = unit / eg, e0 = (unit - ch * eg) * 64, c = ch / ht, h0 = c * per + (ch - c * ht) * 16;
+      const bool h_ok = h0 + r16 < (c + 1) * per;
+      const float* bp = mix + (h_ok ? h0 + r16 : h0) * TS + 4 * kq;
+      const uint8_t* ap = rows + (c * E + e0) * 2 + r16 * 8;
+      f32x4 acc[4] = {}, bv[KT];                                // talk[head][16 k + 4 kq + s]
+      uint2 av[KT][4];
+#pragma unroll
+      for (int k = 0; k < KT; ++k) {
+        bv[k] = *reinterpret_cast<const f32x4*>(bp + 16 * k);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) av[k][s] = *reinterpret_cast<const uint2*>(ap + min(16 * k + 4 * kq + s, H - 1) * rs);
+      }
+      if (H < 16 * KT)
+#pragma unroll
+        for (int k = 0; k < KT; ++k)
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+            if (16 * k + 4 * kq + s >= H) av[k][s] = uint2{0u, 0u};
+#pragma unroll
+      for (int k = 0; k < KT; ++k)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const T* x = reinterpret_cast<const T*>(&av[k][s]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(Elem<T>::to_f(x[j]), bv[k][s], acc[j], 0, 0, 0);
+        }
+      if (h_ok) {
+        uint4 w[2];
+        uint32_t* wp = reinterpret_cast<uint32_t*>(w);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          wp[2 * i] = pack2<T>(acc[0][i], acc[1][i]);
+          wp[2 * i + 1] = pack2<T>(acc[2][i], acc[3][i]);
+        }
+        uint4* o = reinterpret_cast<uint4*>(out + t * out_ld + (int64_t)(h0 + r16) * E + e0 + 16 * kq);
+        o[0] = w[0];
+        o[1] = w[1];
+      }
+    }
+  }
+}
+
 struct LocalAttnArgs {
   const void* q; int64_t q_ld;
   const void* gate; int64_t gate_ld;
@@ -1878,8 +1964,29 @@ extern "C" int semipd_talk_mix(const void* parts, int64_t parts_ld, const float*
   // of 128 5.8 / 5.1, 16 / 2 of 64 4.6 / 4.3, 16 / 4 of 128 6.7 / 7.2, 8 / 2 of 128 4.1 / 5.0, 16 / 8 of 64 5.2 / 8.3, 8 / 1 of 32 3.2 / 3.6, 32 / 4
   // of 32 5.8 / 5.9; not staged: 32 / 4 of 128 44 / 8.2, 48 / 8 of 64 57 / 14)
   const bool tiles = (num_q_heads >= 6 * num_kv_heads && v_dim >= 64) || staged > 65536;
-  if (tiles && (dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
-      aligned16(out) && held <= 65536 && num_q_heads <= 64) {
+  const bool matrix = (dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
+                      aligned16(out) && num_q_heads <= 64;
+  // Value rows of whole 64 elements and at least 8 heads: 16-byte stores, several tokens a workgroup where they are more than the chip takes at
+  // once.  Against the vector form, 32 / 7262 tokens, us: 8 heads over 2 of 128 3.4 / 24 and 3.1 / 21, 16 over 8 of 64 4.6 / 51 and 3.7 / 36, 8 over 1
+  // of 64 2.9 / 12.9 both; 6 over 3 of 64 2.9 / 12.5 and 3.0 / 19, 4 over 4 of 128 2.8 / 14 and 3.6 / 33.
+  const int kt = (num_q_heads + 15) / 16;
+  const size_t rows = (size_t)num_q_heads * ((size_t)num_kv_heads * v_dim * 2 + 32) + (size_t)num_q_heads * (16 * kt + 4) * 4;
+  if (matrix && v_dim % 64 == 0 && num_q_heads >= 8 && rows <= 65536) {
+    const int64_t at_once = 256 * (int64_t)(rows <= 20480 ? 8 : 163840 / rows), turns = (num_tokens + at_once - 1) / at_once;
+    const dim3 grid((unsigned)((num_tokens + turns - 1) / turns));
+#define TALK_ROWS(KT)                                                                                                                              \
+  hipLaunchKernelGGL((talk_mix_rows_kernel<T, KT>), grid, dim3(256), rows, as_stream(stream), (const T*)parts, parts_ld, talk, (T*)out, out_ld, num_tokens, \
+                     num_q_heads, num_kv_heads, v_dim)
+    SEMIPD_DISPATCH_HALF(dtype, T, {
+      if (kt == 1) TALK_ROWS(1);
+      else if (kt == 2) TALK_ROWS(2);
+      else if (kt == 3) TALK_ROWS(3);
+      else TALK_ROWS(4);
+    });
+#undef TALK_ROWS
+    return launch_status("talk_mix");
+  }
+  if (tiles && matrix && held <= 65536) {
     SEMIPD_DISPATCH_HALF(dtype, T, {
       if (num_q_heads <= 32)
         hipLaunchKernelGGL((talk_mix_mfma_kernel<T, 2>), dim3((unsigned)num_tokens), dim3(256), held, as_stream(stream), (const T*)parts,

@@ -224,6 +224,24 @@ def test_talk_mix(dtype, H, G, E):
     assert bool(((out - want).abs() <= half * want.abs() + 64 * 2.0 ** -24 * terms + 1e-7).all())
 
 
+# more tokens than the chip takes at once (a workgroup has several), by itself and among others, more 16-byte pieces a token than are fetched ahead
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,E,tokens", [(12, 2, 64, 4097), (24, 2, 128, 3001), (40, 4, 64, 2049), (64, 1, 256, 1300)])
+def test_talk_mix_of_many_tokens(dtype, H, G, E, tokens):
+    """Every token's row is what it is in a call of its own, and what is not finite in one stays in it."""
+    from semi_pd_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(H)
+    parts, talk = torch.randn(tokens, H * G * E, generator=g, device=DEV).to(dtype), torch.randn(H, H, generator=g, device=DEV)
+    parts[tokens - 7, 3], parts[5, 70] = float("inf"), float("nan")
+    out = ops.talk_mix(parts, talk, G)
+    finite = torch.isfinite(out.float()).all(1)
+    assert bool((finite == (torch.arange(tokens, device=DEV) != tokens - 7) & (torch.arange(tokens, device=DEV) != 5)).all())
+    for t0 in (0, tokens // 2, tokens - 11):
+        few = ops.talk_mix(parts[t0: t0 + 11].contiguous(), talk, G)
+        same = out[t0: t0 + 11]
+        assert bool(((few == same) | (torch.isnan(few) & torch.isnan(same))).all())
+
+
 # (launches large enough that tiles go by their keys: blocks of 18 tiles, one row past a tile's edge in front; of 70, two of which are a level;
 # requests without blocks, so many keys that three tiles are a level)
 @pytest.mark.parametrize("block,lens,olds", [(576, [700, 0, 33, 400, 1], [545, 7, 5, 0, 576]), (2240, [500, 1, 600], [2000, 64, 3]), (2240, [1100], [1999]),
