@@ -796,9 +796,10 @@ template <typename T, int EPI>
 static int g8_launch_rows(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, hipStream_t st) {
   const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N, cols_per_tile = EPI == G8_SILU_MUL ? RowsTile::kCols / 2 : RowsTile::kCols;
   const int64_t tiles = max_sorted / RowsTile::kRows * ((n_cols + cols_per_tile - 1) / cols_per_tile);
+  // (an XCD's share of the tiles and its share of those that come last are rounded up apart)
   static std::atomic<uint64_t> lds_ok{0};
   if (ensure_dynamic_lds((const void*)moe_gemm_rows_kernel<T, EPI>, RowsTile::kLds, lds_ok, "moe_gemm_rows")) return 1;
-  hipLaunchKernelGGL((moe_gemm_rows_kernel<T, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), RowsTile::kLds, st, c, a, w, N, K, grp);
+  hipLaunchKernelGGL((moe_gemm_rows_kernel<T, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8 + 8)), dim3(256), RowsTile::kLds, st, c, a, w, N, K, grp);
   return launch_status("moe_gemm_rows");
 }
 
@@ -913,8 +914,8 @@ int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* top
                    "moe_gemm_tall: null pointer");
   SEMIPD_CHECK_ARG(!mul_routed_weight || topk_weights, SEMIPD_EINVAL, "moe_gemm_tall: topk_weights required");
   const int64_t n_out = fuse_silu_mul ? n / 2 : n;
-  SEMIPD_CHECK_ARG(block_m != RowsTile::kRows || (k % 128 == 0 && n * k < (1 << 30) && ((num_valid - 1) / top_k_div + 1) * k < (1 << 30)), SEMIPD_ESHAPE,
-                   "moe_gemm_tall: blocks of 320 rows need k %% 128 and operands below 2 GiB");
+  SEMIPD_CHECK_ARG(block_m != RowsTile::kRows || (k % 128 == 0 && aligned16(c) && n * k < (1 << 30) && ((num_valid - 1) / top_k_div + 1) * k < (1 << 30)), SEMIPD_ESHAPE,
+                   "moe_gemm_tall: blocks of 320 rows need k %% 128, a 16-byte aligned output and operands below 2 GiB");
   SEMIPD_CHECK_ARG((block_m == 320 || block_m == 256 || block_m == 128) && max_sorted % block_m == 0 && k % 64 == 0 && n_out % 16 == 0 && (!fuse_silu_mul || n % 2 == 0) && aligned16(a) &&
                        aligned16(w) && (reinterpret_cast<uintptr_t>(c) & 7u) == 0 && num_valid < (1 << 30) && n < (1 << 30) &&
                        k < (1 << 30),

@@ -14,7 +14,8 @@
 // rows an expert's weights come from HBM once (738 MB of 64 experts of 2816 x 2048: 147 us of a read's time).  Why 320 rows: a second,
 // nearly empty tile of 256 took 0.4 of a full one; 320 accumulator registers and 144 KB of LDS are what a CU holds.  Why bodies: a wave's
 // products follow its rows in steps of 64.  64 experts, top 6, bf16, both products, tiles of 256 rows / this: 1000 tokens (94 rows an expert) 183 +
-// 95 / 167 + 89 us, 3001 (281) 296 + 182 / 227 + 134, 6000 (562) 477 + 265 / 401 + 239, 8192 572 + 332 / 535 + 333; whole layer of 3001 tokens 497 -> 403.
+// 95 / 167 + 81 us, 3001 (281) 296 + 182 / 220 + 115, 6000 (562) 477 + 265 / 391 + 208, 8192 572 + 332 / 523 + 294.  Results by way of LDS, in 256 bytes
+// of an entry instead of 32: second product of 3001 tokens 134 -> 115 us (74 MB of results).
 #pragma once
 
 namespace semipd {
@@ -180,34 +181,60 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     rows_retire<(I < 8)>(acc[I][4], acc[I][5], acc[I][6], acc[I][7]);
   });
 
-  // ---- epilogue: lane holds, of entry m0 + 32 NX h + 16 NX wr + 16 i + c16, columns 16 j + 4 q4 .. + 3 of its wave's ----
+  // ---- epilogue: lane holds, of entry m0 + 32 NX h + 16 NX wr + 16 i + c16, columns 16 j + 4 q4 .. + 3 of its wave's.  A half's rows go
+  //      through the wave's own quarter of the LDS and leave whole: 256 bytes of an entry (128 of SiLU * up) instead of 32 a store ----
+  constexpr int WCOLS = EPI == G8_SILU_MUL ? 64 : 128, LPR = WCOLS / 8, RPS = 64 / LPR;      // lanes a row, rows a store
+  constexpr int OS = WCOLS * 2 + 16;                                                            // bytes between rows in LDS
+  static_assert(16 * NX * OS <= R::kLds / 4, "a half's rows fit the wave's quarter");
+  char* const mine = smem + wave * (R::kLds / 4);
+  g8_barrier();                       // everybody has read its last fragments and has no DMA in flight
 #pragma unroll
-  for (int i = 0; i < 2 * NX; ++i) {
-    const int id = grp.sorted_ids[m0 + 32 * NX * (i / NX) + 16 * NX * wr + 16 * (i % NX) + c16];
-    const bool ok = id < grp.num_valid;
-    const float scale = EPI == G8_PLAIN && ok && grp.mul_routed_weight ? grp.topk_weights[id] : 1.f;
+  for (int h = 0; h < 2; ++h) {
+    const int32_t* ids = grp.sorted_ids + m0 + 32 * NX * h + 16 * NX * wr;
+    int to[16 * NX / RPS];
 #pragma unroll
-    for (int j = 0; j < (EPI == G8_SILU_MUL ? 4 : 8); ++j) {
-      const int n = n0 + (EPI == G8_SILU_MUL ? 64 : 128) * wc + 16 * j + 4 * q4;
-      float r[4];
+    for (int u = 0; u < 16 * NX / RPS; ++u) to[u] = ids[RPS * u + lane / LPR];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
+    for (int i = 0; i < NX; ++i) {
+      float scale = 1.f;
+      if (EPI == G8_PLAIN && grp.mul_routed_weight) {
+        const int id = ids[16 * i + c16];
+        scale = id < grp.num_valid ? grp.topk_weights[id] : 1.f;
+      }
+#pragma unroll
+      for (int j = 0; j < WCOLS / 16; ++j) {
+        float r[4];
         if (EPI == G8_SILU_MUL) {
           // the unfused pair rounds the GEMM output to T before the activation reads it
-          const float gq = Elem<T>::to_f(Elem<T>::from_f(acc[i][j][e])), uq = Elem<T>::to_f(Elem<T>::from_f(acc[i][(EPI == G8_SILU_MUL ? 4 : 0) + j][e]));
-          r[e] = gq / (1.f + __expf(-gq)) * uq;
-          asm volatile("" : "+v"(r[e]));   // (see gemm8p_kernel's epilogue: two roundings, not one fused one)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float gq = Elem<T>::to_f(Elem<T>::from_f(acc[NX * h + i][j][e]));
+            const float uq = Elem<T>::to_f(Elem<T>::from_f(acc[NX * h + i][(EPI == G8_SILU_MUL ? 4 : 0) + j][e]));
+            r[e] = gq / (1.f + __expf(-gq)) * uq;
+            asm volatile("" : "+v"(r[e]));   // (see gemm8p_kernel's epilogue: two roundings, not one fused one)
+          }
         } else {
-          r[e] = acc[i][j][e] * scale;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[e] = acc[NX * h + i][j][e] * scale;
         }
-      }
-      if (ok && n < n_cols) {
         uint2 p;
         p.x = (uint32_t)Elem<T>::from_f(r[0]).v | ((uint32_t)Elem<T>::from_f(r[1]).v << 16);
         p.y = (uint32_t)Elem<T>::from_f(r[2]).v | ((uint32_t)Elem<T>::from_f(r[3]).v << 16);
-        *reinterpret_cast<uint2*>(out + (int64_t)id * n_cols + n) = p;
+        *reinterpret_cast<uint2*>(mine + (16 * i + c16) * OS + j * 32 + q4 * 8) = p;
       }
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const int n = n0 + WCOLS * wc + lane % LPR * 8;
+#pragma unroll
+    for (int u = 0; u < 16 * NX / RPS; ++u) {
+      const uint4 v = *reinterpret_cast<const uint4*>(mine + (RPS * u + lane / LPR) * OS + lane % LPR * 16);
+      if (to[u] < grp.num_valid && n < n_cols) *reinterpret_cast<uint4*>(out + (int64_t)to[u] * n_cols + n) = v;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 }
 
@@ -222,17 +249,67 @@ moe_gemm_rows_kernel(T* __restrict__ out, const T* __restrict__ x, const T* __re
   // rows are fetched into one L2, and a second row tile's are near enough to find the weight tiles there.  Where they are more than half
   // the CUs of an XCD, up to eight row tiles of the expert take turns within them (8 experts of 4096 x 28672, 4096 tokens, top 2: 1800 ->
   // 1640 us; with 11 column tiles, second tiles of 64 rows: 328 -> 382, their short tiles no longer come last).
-  const int tiles_m = grp.num_post_pad[0] / RowsTile::kRows, total = tiles_m * tiles_n, per = (total + 7) >> 3;
-  const int at = blockIdx.x >> 3, logical = (blockIdx.x & 7) * per + at;
-  if (at >= per || logical >= total) return;
-  const int near = logical / tiles_n, expert = grp.expert_ids[near], slot = (near & ~7) + (threadIdx.x & 7);
-  const uint32_t same = (uint32_t)__ballot(grp.expert_ids[min(slot, tiles_m - 1)] == expert && slot < tiles_m) & 255u;
-  const int first = (near & ~7) + __builtin_ctz(same), n_rows = __builtin_popcount(same);
-  int tile_m = near, tile_n = logical - near * tiles_n;
-  if (tiles_n > 16) {
-    const int in_group = logical - first * tiles_n;
-    tile_n = in_group / n_rows;
-    tile_m = first + in_group - tile_n * n_rows;
+  const int tiles_m = grp.num_post_pad[0] / RowsTile::kRows, lane = threadIdx.x & 63, at = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+  int tile_m, tile_n, expert;
+  bool alone;                                                            // no other row tile reads this one's weight rows
+  if (tiles_n > 16 || tiles_m > 256) {
+    const int total = tiles_m * tiles_n, per = (total + 7) >> 3, logical = xcd * per + at;
+    if (at >= per || logical >= total) return;
+    const int near = logical / tiles_n, slot = (near & ~7) + (lane & 7);
+    expert = grp.expert_ids[near];
+    const uint32_t same = (uint32_t)__ballot(grp.expert_ids[min(slot, tiles_m - 1)] == expert && slot < tiles_m) & 255u;
+    const int first = (near & ~7) + __builtin_ctz(same), n_rows = __builtin_popcount(same);
+    tile_m = near;
+    tile_n = logical - near * tiles_n;
+    alone = n_rows == 1;
+    if (tiles_n > 16) {
+      const int in_group = logical - first * tiles_n;
+      tile_n = in_group / n_rows;
+      tile_m = first + in_group - tile_n * n_rows;
+    }
+  } else {
+    // The last row tiles of experts that have several come behind all others where they are few: a launch that ends in them ends in short
+    // tiles (64 experts, 300 rows each on average, 72 row tiles: 262 -> 230 and 151 -> 132 us).  A bit a row tile: its expert is the one
+    // before's, and it is such a last one.
+    int ids[4];
+    uint64_t again[5] = {}, tails[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int t = 64 * c + lane;
+      ids[c] = grp.expert_ids[min(t, tiles_m - 1)];
+      again[c] = __ballot(t > 0 && t < tiles_m && grp.expert_ids[max(min(t, tiles_m) - 1, 0)] == ids[c]);
+    }
+    int n_tails = 0;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      tails[c] = again[c] & ~(again[c] >> 1 | again[c + 1] << 63);
+      n_tails += __builtin_popcountll(tails[c]);
+    }
+    if (n_tails * 8 > tiles_m) n_tails = 0;
+    const int heads = (tiles_m - n_tails) * tiles_n, ends = n_tails * tiles_n, per = (heads + 7) >> 3, per_end = (ends + 7) >> 3;
+    const bool end = at >= per;
+    const int logical = end ? (at - per) + xcd * per_end : at + xcd * per;
+    if (end ? at - per >= per_end || logical >= ends : logical >= heads) return;
+    tile_m = logical / tiles_n;
+    tile_n = logical - tile_m * tiles_n;
+    if (n_tails > 0) {                                                   // the tile_m-th of its kind
+      int left = tile_m;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint64_t there = tiles_m >= 64 * (c + 1) ? ~0ull : tiles_m > 64 * c ? (1ull << (tiles_m - 64 * c)) - 1 : 0ull, kind = end ? tails[c] : there & ~tails[c];
+        const int n = __builtin_popcountll(kind);
+        if (left >= 0 && left < n) tile_m = 64 * c + __builtin_ctzll(__ballot((kind >> lane & 1) && __builtin_popcountll(kind & ((1ull << lane) - 1)) == left));
+        left -= n;
+      }
+    }
+    expert = 0;
+    alone = true;
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (tile_m >> 6 == c) {
+        expert = __builtin_amdgcn_readlane(ids[c], tile_m & 63);
+        alone = !((again[c] | (again[c] >> 1 | again[c + 1] << 63)) >> (tile_m & 63) & 1);
+      }
   }
   const int m0 = tile_m * RowsTile::kRows, n0 = tile_n * cols_per_tile;
   w += (int64_t)expert * N * K;
@@ -244,7 +321,7 @@ moe_gemm_rows_kernel(T* __restrict__ out, const T* __restrict__ x, const T* __re
   }
   // weight rows that no other workgroup reads leave the L2 to the entries' rows (64 experts of 2048 x 1408 behind 94 rows: 97 -> 89 us, 281
   // rows 143 -> 134; of 1408 x 2816 within the noise)
-  if (n_rows == 1) {
+  if (alone) {
     if (rows <= 128) moe_rows_body<T, EPI, 2, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
     else if (rows <= 192) moe_rows_body<T, EPI, 3, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
     else if (rows <= 256) moe_rows_body<T, EPI, 4, true>(g8_smem, out, x, w, N, K, m0, n0, grp);

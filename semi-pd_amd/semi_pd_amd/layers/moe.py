@@ -82,8 +82,8 @@ MOE_STREAM_MAX_TOKENS = int(os.environ.get("SEMIPD_MOE_STREAM_MAX_TOKENS", "320"
 def _tall_block(block_m: int, tokens: int, topk: int, E: int, K: int, F: int) -> int:
     """Rows per block of a call that the tiled kernels take in blocks of `block_m`: 320, where the kernel whose tiles are as tall as
     their expert needs takes both products (K and F in pairs of 64, 32-bit offsets into the operands) and is ahead.  Whole layer, both
-    products, blocks of 128 or 256 / of 320, us: 64 experts of 2048 x 1408, top 6, 400 tokens 255 / 248, 1000 273 / 255, 2000 322 / 310,
-    3001 474 / 361, 6000 739 / 640, 8192 903 / 870; 8 of 4096 x 14336, top 2, 512 tokens 795 / 611, 4096 2550 / 2450; 16 of 2048 x 1408, top 2, 1024
+    products, blocks of 128 or 256 / of 320, us: 64 experts of 2048 x 1408, top 6, 400 tokens 255 / 232, 1000 273 / 248, 2000 322 / 285,
+    3001 474 / 335, 6000 739 / 599, 8192 903 / 817; 8 of 4096 x 14336, top 2, 512 tokens 795 / 611, 4096 2550 / 2450; 16 of 2048 x 1408, top 2, 1024
     tokens 86 / 84, 4096 203 / 183.  Behind with few K steps, whose loads ahead are not covered (256 experts of 7168 x 256, 1024 tokens
     554 / 630: its second product has four), and where its tiles are too few for the chip."""
     numel = tokens * topk

@@ -10,10 +10,13 @@ DEV = "cuda"
 BM = 320
 
 
-# (rows around every body's most, a whole tile and one more; two steps of K and an uneven count of pairs; columns that end inside a tile)
+# (rows around every body's most, a whole tile and one more; two steps of K and an uneven count of pairs; columns that end inside a tile; few last
+# row tiles among many, behind the others, on both sides of 64 of them; more than 256 row tiles; row tiles in turns within many column tiles)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("counts,K,n_out,div", [([1, 16, 17, 127, 128, 129, 0, 160, 192, 193, 255, 256, 257, 319, 320, 321, 640], 128, 48, 1),
-                                                ([300, 500, 20, 290, 1000], 384, 1200, 5), ([96, 200], 640, 2320, 2)])
+                                                ([300, 500, 20, 290, 1000], 384, 1200, 5), ([96, 200], 640, 2320, 2),
+                                                ([5] * 30 + [330] + [3] * 31 + [340, 0, 350, 9] + [2] * 8, 128, 304, 1), ([1] * 250 + [400, 2, 3, 0, 2000], 128, 32, 1),
+                                                ([700, 30, 2900], 128, 2320, 1)])
 def test_rows_of_every_body(counts, K, n_out, div, dtype):
     g = torch.Generator().manual_seed(K)
     total, E = sum(counts), len(counts)
