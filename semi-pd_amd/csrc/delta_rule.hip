@@ -812,27 +812,39 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
   if (lays && tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
-// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S), two waves per 16 columns.  A wave has half the rows
-// of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the right-hand operand of a product
-// over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving its registers.  The
-// halves of K S go to the other wave through LDS and both make U; of Q S, v and the results a wave finishes 16 of the tokens.
-template <typename T, int NP>
+// The chunks of a request in turn, a workgroup of eight waves per (request, head, 16 CB columns of S), two or four waves per 16 columns.  A wave
+// has its part of the rows of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the
+// right-hand operand of a product over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving
+// its registers.  The parts of K S go to the other waves of the columns through LDS and all make U; of Q S, v and the results a wave finishes
+// 16 of the tokens.
+// Four waves per 16 columns halve what a wave does for a chunk and leave U to be made twice as often: for launches that leave CUs without
+// work at 64 columns a workgroup.  Their chunk was 4.2 us of 10 k cycles, now 7.8 k, about 500 vector instructions and 56 products of either
+// wave of a SIMD; half the work a wave left the waits for the operands, so everything is fetched a whole chunk ahead there (3.5 -> 3.2 us; the form
+// of two waves is 5 % slower so).  32 heads of 128 x 128 over 8, whole call: 1 request of 5083 rows 741 -> 583 us, of 1000 168 -> 139.
+template <typename T, int NP, int CB>
 __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
-  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / 2, HALO = kRecHalo;      // HT: 16-row tiles of S a wave
+  constexpr int PARTS = 8 / CB;                                 // waves that share 16 columns
+  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / PARTS, HALO = kRecHalo;  // HT: 16-row tiles of S a wave
+  constexpr int EX = PARTS == 2 ? 3 : 2;
+  constexpr bool AHEAD = PARTS > 2;                             // everything is fetched a whole chunk ahead, not half of one
+  static_assert(HT % 2 == 0, "two tiles are an operand");
   constexpr int PB = L * NP * 2, ALL = 3 * PB / 16, PIECES = (ALL + 511) / 512;  // bytes of a plane; 16-byte pieces of three, a thread's
   using Tile = RowTile<T, 16>;
-  static_assert(Tile::kElems * sizeof(T) <= 3072 && 16 * kOutStride * 4 <= 3072, "a wave's part of ex_l");
+  static_assert(Tile::kElems * sizeof(T) <= EX * 1024 && 16 * kOutStride * 4 <= EX * 1024, "a wave's part of ex_l");
   __shared__ __attribute__((aligned(16))) uint8_t k_l[3 * PB], q_l[3 * PB], kt_l[3 * PB];    // K, Q and K^T of the chunk, as laid down
   __shared__ __attribute__((aligned(16))) float head_l[kDeltaHead];             // the head's weights
   // by turns half sums for a wave from the other one of its columns, its raw inputs, its results on their way out (token by token: v)
-  __shared__ __attribute__((aligned(16))) uint8_t ex_l[8][3][1024];
-  __shared__ __attribute__((aligned(16))) uint8_t v_l[4][2][1024];              // v of the chunk: [columns][token tile][lane][16]
+  __shared__ __attribute__((aligned(16))) uint8_t ex_l[8][EX][1024];
+  __shared__ __attribute__((aligned(16))) uint8_t sum_l[PARTS == 2 ? 1 : 8][4][PARTS == 2 ? 16 : 1024];     // four waves: their parts of K S and Q S
+  __shared__ __attribute__((aligned(16))) uint8_t v_l[CB][2][1024];             // v of the chunk: [columns][token tile][lane][16]
   __shared__ int serial_l[2];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, kq = lane >> 4;
-  const int cw = w & 3, half = w >> 2;
+  // of four waves the first two make v, the others finish the results, either of 16 tokens; of two each does both
+  const int cw = w % CB, part = w / CB, half = part & 1;
+  const bool makes_v = PARTS == 2 || part < 2, ends = PARTS == 2 || part >= 2;
   // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
-  const int eblocks = (E + 63) / 64, members = per * eblocks;
+  const int eblocks = (E + 16 * CB - 1) / (16 * CB), members = per * eblocks;
   const RecPlace at = rec_place((int)a.batch * G, members);
   if (at.unit < 0) return;
   const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, (int)a.batch);      // (113 KB of LDS: one a CU)
@@ -842,13 +854,13 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
   const int64_t chunk0 = __builtin_amdgcn_readfirstlane((int)rec_chunks_before(a.q_len, b));
   if (chunk0 + (n + L - 1) / L > max_chunks) return;            // (requests that share rows: more rows than the launch has)
   const int h = g * per + member / eblocks;
-  const int e0 = member % eblocks * 64 + 16 * cw, e = e0 + r16;
+  const int e0 = member % eblocks * (16 * CB) + 16 * cw, e = e0 + r16;
   const bool on = e0 < E;                                        // (waves without columns take their part of the staging)
   const bool e_ok = e < E, wide = e0 + 16 <= E;
   const int C = 2 * G * D + H * E;
   const int64_t slot = a.state_indices[b];
   float* st = a.state + slot * a.state_ld + (int64_t)h * D * E + e;
-  const int row0 = half * (NP / 2) + 4 * kq;                     // this lane's rows of S: row0 + 16 t + r
+  const int row0 = part * (NP / PARTS) + 4 * kq;                 // this lane's rows of S: row0 + 16 t + r
   f32x4 S[HT];
 #pragma unroll
   for (int t = 0; t < HT; ++t)
@@ -871,7 +883,7 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
   auto fetch_v = [&](int l0) {
     int ln = lane;
     asm volatile("" : "+v"(ln));                                 // (addresses made where they are used, not held over the loop)
-    if (vec) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
+    if (vec && makes_v) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
   };
   // v of this lane's tokens 16 half + 4 kq + s, zero behind the portion; taps that the layer does not have see zeros
   auto convolve = [&](const float (&raw)[HALO + 4], int cnt, f32x4& v, bool& bad) {
@@ -893,6 +905,7 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
   // ... of the chunk at l0 into this lane's place, by way of the wave's LDS
   float in[HALO + 4];
   auto place_v = [&](int l0) {
+    if (!makes_v) return;
     T* raw = reinterpret_cast<T*>(ex_l[w][0]);
     int ln = lane;
     asm volatile("" : "+v"(ln));
@@ -908,25 +921,37 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
     for (int i = 0; i < HALO + 4; ++i) in[i] = Elem<T>::to_f(raw[(4 * (ln >> 4) + i) * Tile::kStride + (ln & 15)]);
   };
-  u32x4 stage[2 * PIECES], head;
+  u32x4 stage[2 * PIECES], stage_kt[AHEAD ? PIECES : 1], head;
   auto fetch_head = [&](const float* src) {
     if (tid < kDeltaHead / 4) head = reinterpret_cast<const u32x4*>(src)[tid];
   };
-  auto fetch = [&](const float* src, int at) {
+  auto fetch = [&](const float* src, u32x4* to) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < PIECES; ++u)
-      if (ALL % 512 == 0 || u * 512 + tid < ALL) stage[at + u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) to[u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
   };
-  auto place = [&](uint8_t* dst, int at) {
+  auto place = [&](uint8_t* dst, const u32x4* from) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < PIECES; ++u)
-      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = stage[at + u];
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = from[u];
+  };
+  // a wave's part of a sum and the others' (in pairs, so that all of them have the same)
+  auto summed = [&](const f32x4& mine, int i) __attribute__((always_inline)) {
+    if constexpr (PARTS == 2) return mine + *reinterpret_cast<const f32x4*>(&ex_l[w][i][16 * lane]);
+    else return (mine + *reinterpret_cast<const f32x4*>(&sum_l[w ^ CB][i][16 * lane])) +
+                (*reinterpret_cast<const f32x4*>(&sum_l[w ^ (2 * CB)][i][16 * lane]) + *reinterpret_cast<const f32x4*>(&sum_l[w ^ (3 * CB)][i][16 * lane]));
   };
   bool bad = false;
-  fetch(f, 0);
-  fetch(f + 3 * L * NP / 2, PIECES);
+  fetch(f, stage);
+  fetch(f + 3 * L * NP / 2, stage + PIECES);
+  float flag_next = 0.f, keep_next = 0.f;
+  if constexpr (AHEAD) {
+    fetch_head(fh);
+    fetch(f + 3 * L * NP, stage_kt);
+    flag_next = f[9 * L * NP / 2], keep_next = fh[1536 + L - 1];
+  }
   if (L < n) fetch_v(L);
-  {
+  if (makes_v) {
 #pragma unroll
     for (int i = 0; i < HALO + 4; ++i) {
       const int l = 16 * half + 4 * kq + i - HALO;
@@ -940,8 +965,8 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
     convolve(in, n, v, bad);
     *reinterpret_cast<f32x4*>(&v_l[cw][half][16 * lane]) = v;
   }
-  place(k_l, 0);
-  place(q_l, PIECES);
+  place(k_l, stage);
+  place(q_l, stage + PIECES);
   if (tid < 2) serial_l[tid] = 0;
   if (L < n) place_v(L);
   __syncthreads();
@@ -954,9 +979,15 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
     const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
     const float* fhn = fh + (more ? head_ld : 0);
     float* yr = yo + (int64_t)(l0 + 16 * half) * a.wld;
-    fetch_head(fh);
-    fetch(f + 3 * L * NP, 0);
-    const float flag = f[9 * L * NP / 2], keep = fh[1536 + L - 1];
+    const float flag = AHEAD ? flag_next : f[9 * L * NP / 2], keep = AHEAD ? keep_next : fh[1536 + L - 1];
+    if constexpr (AHEAD) {
+      fetch(fn, stage);
+      fetch(fn + 3 * L * NP / 2, stage + PIECES);
+      flag_next = fn[9 * L * NP / 2], keep_next = fhn[1536 + L - 1];
+    } else {
+      fetch_head(fh);
+      fetch(f + 3 * L * NP, stage);
+    }
     f32x4 O = {}, P[2] = {}, v[2] = {}, vn;
     bool serial = false, bad_next = false;
     if (on) {
@@ -970,25 +1001,33 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(k_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(k_l + q * PB + (i * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
           rec_mma<2>(c, s, P, Ps);
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(q_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(q_l + q * PB + (i * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
           rec_mma<2>(c, s, Q, Qs);
         }
-        convolve(in, n - l0 - L, vn, bad_next);                  // (the next chunk's, between the products; there is none: zeros)
+        if (makes_v) convolve(in, n - l0 - L, vn, bad_next);     // (the next chunk's, between the products; there is none: zeros)
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           P[i] += Ps[i];
           Q[i] += Qs[i];
         }
       }
-      // the other wave of these columns gets all of K S and the tokens of Q S that it finishes
-      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][0][16 * lane]) = P[0];
-      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][1][16 * lane]) = P[1];
-      *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][2][16 * lane]) = half ? Q[0] : Q[1];
+      // the others of these columns get all of K S and the tokens of Q S that they finish
+      if constexpr (PARTS == 2) {
+        *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][0][16 * lane]) = P[0];
+        *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][1][16 * lane]) = P[1];
+        *reinterpret_cast<f32x4*>(&ex_l[w ^ 4][2][16 * lane]) = half ? Q[0] : Q[1];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          *reinterpret_cast<f32x4*>(&sum_l[w][i][16 * lane]) = P[i];
+          *reinterpret_cast<f32x4*>(&sum_l[w][2 + i][16 * lane]) = Q[i];
+        }
+      }
       O = half ? Q[1] : Q[0];
       float z = 0.f, top = 0.f;
 #pragma unroll
@@ -1020,12 +1059,17 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
       for (int i = 0; i < 2; ++i) v[i] = *reinterpret_cast<const f32x4*>(&v_l[cw][i][16 * lane]);
     }
-    place(kt_l, 0);
+    place(kt_l, AHEAD ? stage_kt : stage);
     if (tid < kDeltaHead / 4) reinterpret_cast<u32x4*>(head_l)[tid] = head;
     if (l0 + 2 * L < n) fetch_v(l0 + 2 * L);
     __syncthreads();
-    fetch(fn, 0);
-    fetch(fn + 3 * L * NP / 2, PIECES);
+    if constexpr (AHEAD) {
+      fetch_head(fhn);
+      fetch(fn + 3 * L * NP, stage_kt);
+    } else {
+      fetch(fn, stage);
+      fetch(fn + 3 * L * NP / 2, stage + PIECES);
+    }
     serial = __builtin_amdgcn_readfirstlane(serial_l[turn]) != 0;
     if (tid == 0) serial_l[turn ^ 1] = 0;
     if (!serial) {
@@ -1033,10 +1077,10 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
           const f32x4 eb = *reinterpret_cast<const f32x4*>(head_l + 1536 + 16 * i + 4 * kq);
-          P[i] += *reinterpret_cast<const f32x4*>(&ex_l[w][i][16 * lane]);
+          P[i] = summed(P[i], i);
           v[i] -= eb * P[i];
         }
-        O = (O + *reinterpret_cast<const f32x4*>(&ex_l[w][2][16 * lane])) * *reinterpret_cast<const f32x4*>(head_l + 1536 + 16 * half + 4 * kq);
+        if (ends) O = summed(O, PARTS == 2 ? 2 : 2 + half) * *reinterpret_cast<const f32x4*>(head_l + 1536 + 16 * half + 4 * kq);
         f32x4 Ti[3], M[2], wv[2];
 #pragma unroll
         for (int i = 0; i < 3; ++i) Ti[i] = *reinterpret_cast<const f32x4*>(head_l + 256 * i + 4 * lane);
@@ -1055,19 +1099,21 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
         U[1] += U1;
         const Split3 us = rec_split8(U[0] * wv[0], U[1] * wv[1]);
         f32x4 O1 = {};
+        if (ends) {
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], U[0][s], O, 0, 0, 0);
-          if (half) O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], U[1][s], O1, 0, 0, 0);
+          for (int s = 0; s < 4; ++s) {
+            O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], U[0][s], O, 0, 0, 0);
+            if (half) O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], U[1][s], O1, 0, 0, 0);
+          }
+          O += O1;
         }
-        O += O1;
 #pragma unroll
         for (int t = 0; t < HT; t += 2) {
           Frag16 kt[2][3];
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) kt[i][q].u = *reinterpret_cast<const uint4*>(kt_l + q * PB + (half * HT + t + i) * 1024 + lane * 16);
+            for (int q = 0; q < 3; ++q) kt[i][q].u = *reinterpret_cast<const uint4*>(kt_l + q * PB + (part * HT + t + i) * 1024 + lane * 16);
           f32x4 A[2] = {}, As[2] = {};
           rec_mma<2>(kt, us, A, As);
 #pragma unroll
@@ -1081,12 +1127,13 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
     } else {
       int rows = D, step = E, ln = lane;
       asm volatile("" : "+s"(rows), "+s"(step), "+v"(ln));       // (no addresses held over the loop)
-      const int r16 = ln & 15, kq = ln >> 4, row0 = half * (NP / 2) + 4 * kq, e = e0 + r16;
+      const int r16 = ln & 15, kq = ln >> 4, row0 = part * (NP / PARTS) + 4 * kq, e = e0 + r16;
       const bool e_ok = e < E;
       float* st = a.state + slot * a.state_ld + (int64_t)h * D * E + e;
-      float* vs = reinterpret_cast<float*>(ex_l[0][0]) + 16 * cw + r16;          // v [32][64]
+      float* vs = reinterpret_cast<float*>(ex_l[0][0]) + 16 * cw + r16;          // v [32][16 CB]
+      if (makes_v)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) vs[(16 * half + 4 * kq + s) * 64] = rec_silu_if_large(half ? v[1][s] : v[0][s]);
+        for (int s = 0; s < 4; ++s) vs[(16 * half + 4 * kq + s) * (16 * CB)] = rec_silu_if_large(half ? v[1][s] : v[0][s]);
       if (e_ok)
 #pragma unroll
         for (int t = 0; t < HT; ++t)
@@ -1094,7 +1141,7 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
           for (int r = 0; r < 4; ++r)
             if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
       __syncthreads();
-      if (half == 0 && on) {
+      if (part == 0 && on) {
 #pragma unroll 1
         for (int t = 0; t < cnt; ++t) {
           // row t of K: this lane group's four of every 16
@@ -1117,7 +1164,7 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
           kd += __shfl_xor(kd, 16, 64);
           kd += __shfl_xor(kd, 32, 64);
           const float gt = fh[1536 + 2 * L + t], bt = fh[1536 + 3 * L + t];
-          const float u1 = bt * (vs[t * 64] - gt * dk);
+          const float u1 = bt * (vs[t * (16 * CB)] - gt * dk);
 #pragma unroll 1
           for (int u = 0; u < 4 * NT; ++u) {
             const int row = 16 * (u >> 2) + 4 * kq + (u & 3);
@@ -1134,12 +1181,12 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
       __builtin_amdgcn_s_waitcnt(0x0f70);                        // (vmcnt(0) here, or the other path waits for what it has in flight where they join)
       __builtin_amdgcn_sched_barrier(0);
     }
-    if (more && on) *reinterpret_cast<f32x4*>(&v_l[cw][half][16 * lane]) = vn;
+    if (more && on && makes_v) *reinterpret_cast<f32x4*>(&v_l[cw][half][16 * lane]) = vn;
     bad = bad_next;
-    place(k_l, 0);
-    place(q_l, PIECES);
+    place(k_l, stage);
+    place(q_l, stage + PIECES);
     // behind the wait for the pieces (memory answers in order), so that it is the next one's
-    if (!serial) {
+    if (!serial && ends) {
       __builtin_amdgcn_wave_barrier();
       float* ol = reinterpret_cast<float*>(ex_l[w][0]);
       int ln = lane;
@@ -1551,7 +1598,10 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
   const dim3 grid(rec_walk_blocks(a.batch * a.G, members));
   if constexpr (NP > kDeltaSmall) {
-    hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP>), grid, dim3(512), 0, s, a, chunks);
+    // 32 columns a workgroup as long as every one of them has a CU (rec_walk_blocks: of the XCD with the most)
+    const unsigned narrow = rec_walk_blocks(a.batch * a.G, (int64_t)(a.H / a.G) * ((a.E + 31) / 32));
+    if (narrow <= 256) hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 2>), dim3(narrow), dim3(512), 0, s, a, chunks);
+    else hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 4>), grid, dim3(512), 0, s, a, chunks);
   } else if (a.batch * a.G * members > 256) {
     // more workgroups than CUs: two a CU, at the price of 40 spilled registers (32 heads of 64 x 64, one / two a CU, whole call: 64 requests
     // of 64 rows 226 / 202 us; 4 requests of 96 rows, 128 workgroups: 52 / 58)

@@ -464,27 +464,36 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
   if (lays && tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
-// The chunks of a request in turn, a workgroup per (request, head, 64 columns of S), two waves per 16 columns.  A wave has half the rows
-// of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the right-hand operand of a product
-// over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving its registers.  The
-// halves of C S are added across the two waves in LDS, each finishing 16 of the tokens; it also convolves these tokens' x from raw inputs
-// in LDS of its own and hands x and the pieces of U = e^(b_last - b_t) dt_t x over: x is not written to memory.
-template <typename T, int NP>
-__global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
-  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / 2, HALO = kRecHalo;      // HT: 16-row tiles of S a wave
+// The chunks of a request in turn, a workgroup of eight waves per (request, head, 16 CB columns of S), two or four waves per 16 columns.  A wave
+// has its part of the rows of S in accumulators: lane (r16, kq) holds rows 16 t + 4 kq + r of column r16, two tiles of which are the
+// right-hand operand of a product over 32 rows (split on the way), so S goes from one chunk's sum into the next one's product without leaving
+// its registers.  The parts of C S are added across these waves in LDS, two of which finish 16 of the tokens each; two also convolve these
+// tokens' x from raw inputs in LDS of their own and hand x and the pieces of U = e^(b_last - b_t) dt_t x over: x is not written to memory.
+// Four waves per 16 columns halve what a wave does for a chunk: for launches that leave CUs without work at 64 columns a workgroup (a CU
+// holds one of theirs, not two: everything is fetched a whole chunk ahead, 2.9 -> 2.6 us a chunk, 3.3 at 64 columns).  128 heads of 128 x 64
+// over 8, whole call: 1 request of 5083 rows 611 -> 456 us, of 1000 137 -> 106.
+template <typename T, int NP, int CB>
+__global__ void __launch_bounds__(512, CB == 4 ? 4 : 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
+  constexpr int PARTS = 8 / CB;                                 // waves that share 16 columns
+  constexpr bool AHEAD = PARTS > 2;                             // everything is fetched a whole chunk ahead (half of one: two workgroups a CU cover each other's waits)
+  constexpr int L = kRecChunk, NT = NP / 16, HT = NT / PARTS, HALO = kRecHalo;  // HT: 16-row tiles of S a wave
+  static_assert(HT % 2 == 0, "two tiles are an operand");
   constexpr int PB = L * NP * 2, ALL = 3 * PB / 16, PIECES = (ALL + 511) / 512;  // bytes of a plane; 16-byte pieces of three, a thread's
   using Tile = RowTile<T, 16>;
   constexpr int OWN = Tile::kElems * (int)sizeof(T) > 16 * kOutStride * 4 ? Tile::kElems * (int)sizeof(T) : 16 * kOutStride * 4;
   __shared__ __attribute__((aligned(16))) uint8_t c_l[3 * PB], b_l[3 * PB];     // C and B^T of the chunk, as laid down
-  __shared__ __attribute__((aligned(16))) uint8_t u_l[4][3][1024];              // U of the chunk: [columns][piece][lane][16]; token by token x
-  __shared__ __attribute__((aligned(16))) uint8_t x_l[4][1024];                 // x of its tokens 0 .. 15, for the waves of 16 .. 31
+  __shared__ __attribute__((aligned(16))) uint8_t u_l[CB][3][1024];             // U of the chunk: [columns][piece][lane][16]; token by token x
+  __shared__ __attribute__((aligned(16))) uint8_t x_l[CB][PARTS / 2][1024];             // x of its tokens 0 .. 15, for the waves of 16 .. 31 (four waves: of all tokens)
   __shared__ __attribute__((aligned(16))) uint8_t own_l[8][OWN];                // by turns a wave's half sum of C S, raw inputs, results on their way out
+  __shared__ __attribute__((aligned(16))) uint8_t sum_l[PARTS == 2 ? 1 : 8][2][PARTS == 2 ? 16 : 1024];     // four waves: their parts of C S
   __shared__ int serial_l[2];
   const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), r16 = lane & 15, kq = lane >> 4;
-  const int cw = w & 3, half = w >> 2;
+  // of four waves the first two make x and U, the others finish the results, either of 16 tokens; of two each does both
+  const int cw = w % CB, part = w / CB, half = part & 1;
+  const bool makes_x = PARTS == 2 || part < 2, ends = PARTS == 2 || part >= 2;
   // workgroups of one (request, group) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, N = a.N, E = a.E, taps = a.taps, per = H / G;
-  const int eblocks = (E + 63) / 64, members = per * eblocks;
+  const int eblocks = (E + 16 * CB - 1) / (16 * CB), members = per * eblocks;
   const RecPlace at = rec_place((int)a.batch * G, members);
   if (at.unit < 0) return;
   const int member = at.member, g = at.unit % G, b = rec_by_length(a.q_len, (int)a.batch, at.unit / G, rec_first_requests((int)a.batch, G * members));
@@ -494,13 +503,13 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
   const int64_t chunk0 = __builtin_amdgcn_readfirstlane((int)rec_chunks_before(a.q_len, b));
   if (chunk0 + (n + L - 1) / L > max_chunks) return;          // (requests that share rows: more rows than the launch has)
   const int h = g * per + member / eblocks;
-  const int e0 = member % eblocks * 64 + 16 * cw, e = e0 + r16;
+  const int e0 = member % eblocks * (16 * CB) + 16 * cw, e = e0 + r16;
   const bool on = e0 < E;                                        // (waves without columns take their part of the staging)
   const bool e_ok = e < E, wide = e0 + 16 <= E;
   const int C = H * E + 2 * G * N;
   const int64_t slot = a.state_indices[b];
   float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
-  const int row0 = half * (NP / 2) + 4 * kq;                     // this lane's rows of S: row0 + 16 t + r
+  const int row0 = part * (NP / PARTS) + 4 * kq;                 // this lane's rows of S: row0 + 16 t + r
   f32x4 S[HT];
 #pragma unroll
   for (int t = 0; t < HT; ++t)
@@ -525,7 +534,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
   auto fetch_x = [&](int l0) {
     int ln = lane;
     asm volatile("" : "+v"(ln));                                 // (addresses made where they are used, not held over the loop)
-    if (vec) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
+    if (vec && makes_x) tile.fetch_clamped(p, a.ld, l0 + 16 * half, n, ln);
   };
   // x of this lane's tokens 16 half + 4 kq + s, zero behind the portion; taps that the layer does not have see zeros
   auto convolve = [&](const float (&raw)[HALO + 4], int cnt, f32x4& x, bool& bad) {
@@ -553,28 +562,40 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
   };
   // x and U = e^(b_last - b_t) dt_t x to where both waves of these columns find them
   auto hand_over = [&](const f32x4& x, const f32x4& wv) {
-    if (half == 0) *reinterpret_cast<f32x4*>(&x_l[cw][16 * lane]) = x;
+    if (PARTS > 2 || half == 0) *reinterpret_cast<f32x4*>(&x_l[cw][PARTS > 2 ? half : 0][16 * lane]) = x;
     uint2 u[3];
     rec_split2(x[0] * wv[0], x[1] * wv[1], u[0].x, u[1].x, u[2].x);
     rec_split2(x[2] * wv[2], x[3] * wv[3], u[0].y, u[1].y, u[2].y);
 #pragma unroll
     for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(&u_l[cw][i][16 * lane + 8 * half]) = u[i];
   };
-  u32x4 stage[PIECES];
-  auto fetch = [&](const float* src) {
+  u32x4 stage[PIECES], stage_b[AHEAD ? PIECES : 1];
+  auto fetch = [&](const float* src, u32x4* to) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < PIECES; ++u)
-      if (ALL % 512 == 0 || u * 512 + tid < ALL) stage[u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) to[u] = reinterpret_cast<const u32x4*>(src)[u * 512 + tid];
   };
-  auto place = [&](uint8_t* dst) {
+  auto place = [&](uint8_t* dst, const u32x4* from) __attribute__((always_inline)) {
 #pragma unroll
     for (int u = 0; u < PIECES; ++u)
-      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = stage[u];
+      if (ALL % 512 == 0 || u * 512 + tid < ALL) reinterpret_cast<u32x4*>(dst)[u * 512 + tid] = from[u];
   };
-  f32x4 x;
+  f32x4 x = {};
   bool bad = false;
-  fetch(f);
-  {
+  fetch(f, stage);
+  if constexpr (AHEAD) fetch(f + 3 * L * NP / 2, stage_b);
+  f32x4 head[3];
+  float flag_next = 0.f, keep_next = 0.f;
+  auto fetch_head = [&](const float* fh, f32x4* to) __attribute__((always_inline)) {      // row tile `half` of the weighted C B^T, weights of this lane's tokens
+    to[0] = *reinterpret_cast<const f32x4*>(fh + 256 * half + 4 * lane);
+    to[1] = *reinterpret_cast<const f32x4*>(fh + 512 * half + 4 * lane);
+    to[2] = *reinterpret_cast<const f32x4*>(fh + 768 + 16 * half + 4 * kq);
+  };
+  if constexpr (AHEAD) {
+    fetch_head(fh, head);
+    flag_next = f[3 * L * NP], keep_next = fh[768 + L - 1];
+  }
+  if (makes_x) {
     float in[HALO + 4];
 #pragma unroll
     for (int i = 0; i < HALO + 4; ++i) {
@@ -586,9 +607,9 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
       }
     }
     convolve(in, n, x, bad);
+    hand_over(x, *reinterpret_cast<const f32x4*>(fh + 768 + L + 16 * half + 4 * kq));
   }
-  hand_over(x, *reinterpret_cast<const f32x4*>(fh + 768 + L + 16 * half + 4 * kq));
-  place(c_l);
+  place(c_l, stage);
   if (tid < 2) serial_l[tid] = 0;
   if (L < n) fetch_x(L);
   __syncthreads();
@@ -601,15 +622,11 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
     const float* fn = f + (more ? frag_ld : 0);                 // (the last chunk fetches itself again)
     const float* fhn = fh + (more ? head_ld : 0);
     float* yr = yo + (int64_t)(l0 + 16 * half) * a.wld;
-    fetch(f + 3 * L * NP / 2);
-    const float flag = f[3 * L * NP], keep = fh[768 + L - 1];
+    fetch(AHEAD ? fn : f + 3 * L * NP / 2, stage);
+    const float flag = AHEAD ? flag_next : f[3 * L * NP], keep = AHEAD ? keep_next : fh[768 + L - 1];
+    if constexpr (AHEAD) flag_next = fn[3 * L * NP], keep_next = fhn[768 + L - 1];
     f32x4 M[2] = {}, eb = {}, wv = {};
-    auto fetch_head = [&]() {                                   // row tile `half` of the weighted C B^T, weights of this lane's tokens
-      M[0] = *reinterpret_cast<const f32x4*>(fh + 256 * half + 4 * lane);
-      M[1] = *reinterpret_cast<const f32x4*>(fh + 512 * half + 4 * lane);
-      eb = *reinterpret_cast<const f32x4*>(fh + 768 + 16 * half + 4 * kq);
-      wv = *reinterpret_cast<const f32x4*>(fhn + 768 + L + 16 * half + 4 * kq);
-    };
+    if constexpr (AHEAD) M[0] = head[0], M[1] = head[1], eb = head[2];
     f32x4 O = {};
     bool serial = false;
     if (on) {
@@ -621,10 +638,15 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
 #pragma unroll
         for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(c_l + q * PB + (i * (NT / 2) + half * (HT / 2) + u) * 1024 + lane * 16);
+          for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(c_l + q * PB + (i * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
         rec_mma<2>(c, s, P, Ps);
       }
-      fetch_head();
+      if constexpr (!AHEAD) {
+        f32x4 of[3];
+        fetch_head(fh, of);
+        M[0] = of[0], M[1] = of[1], eb = of[2];
+      }
+      wv = *reinterpret_cast<const f32x4*>(fhn + 768 + L + 16 * half + 4 * kq);
       float z = 0.f, top = 0.f;
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
@@ -636,7 +658,13 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
         }
       }
       O = half ? P[1] : P[0];
-      *reinterpret_cast<f32x4*>(&own_l[w ^ 4][16 * lane]) = half ? P[0] : P[1];
+      if constexpr (PARTS == 2) {
+        *reinterpret_cast<f32x4*>(&own_l[w ^ 4][16 * lane]) = half ? P[0] : P[1];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (!ends || half != i) *reinterpret_cast<f32x4*>(&sum_l[w][i][16 * lane]) = P[i];
+      }
       // An infinity or a NaN in the chunk, or one that sums of large values end in, would reach the tokens in front of it through a product
       // with a weight of zero, and so would a product of a large S with rows behind a step that resets it: the workgroup takes such a
       // chunk token by token, from S in the state row and x in LDS (a rare path: it must not set the kernel's registers)
@@ -656,30 +684,39 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
       }
       if (serial && lane == 0) serial_l[turn] = 1;
     }
-    place(b_l);
+    place(b_l, AHEAD ? stage_b : stage);
     Split3 U;
 #pragma unroll
     for (int i = 0; i < 3; ++i) U.p[i].u = *reinterpret_cast<const uint4*>(&u_l[cw][i][16 * lane]);
-    const f32x4 x0 = *reinterpret_cast<const f32x4*>(&x_l[cw][16 * lane]);
+    const f32x4 x0 = *reinterpret_cast<const f32x4*>(&x_l[cw][0][16 * lane]);
+    if constexpr (PARTS > 2) {
+      if (ends) x = half ? *reinterpret_cast<const f32x4*>(&x_l[cw][PARTS / 2 - 1][16 * lane]) : x0;
+    }
     __syncthreads();
-    fetch(fn);
+    if constexpr (AHEAD) fetch(fn + 3 * L * NP / 2, stage_b);
+    else fetch(fn, stage);
     serial = __builtin_amdgcn_readfirstlane(serial_l[turn]) != 0;
     if (tid == 0) serial_l[turn ^ 1] = 0;
     if (!serial) {
       if (on) {
-        O = (O + *reinterpret_cast<const f32x4*>(&own_l[w][16 * lane])) * eb;
-        // (a row tile of the weights is at most two products of four columns for each of its rows: as they are, in fp32)
-        if (half == 0) {
+        if (ends) {
+          if constexpr (PARTS == 2) O += *reinterpret_cast<const f32x4*>(&own_l[w][16 * lane]);
+          else O = (O + *reinterpret_cast<const f32x4*>(&sum_l[w ^ CB][half][16 * lane])) +
+                   (*reinterpret_cast<const f32x4*>(&sum_l[w ^ (2 * CB)][half][16 * lane]) + *reinterpret_cast<const f32x4*>(&sum_l[w ^ (3 * CB)][half][16 * lane]));
+          O *= eb;
+          // (a row tile of the weights is at most two products of four columns for each of its rows: as they are, in fp32)
+          if (half == 0) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x[s], O, 0, 0, 0);
-        } else {
-          f32x4 O1 = {};
+            for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x[s], O, 0, 0, 0);
+          } else {
+            f32x4 O1 = {};
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x0[s], O, 0, 0, 0);
-            O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], x[s], O1, 0, 0, 0);
+            for (int s = 0; s < 4; ++s) {
+              O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], x0[s], O, 0, 0, 0);
+              O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], x[s], O1, 0, 0, 0);
+            }
+            O += O1;
           }
-          O += O1;
         }
 #pragma unroll
         for (int t = 0; t < HT; t += 2) {
@@ -687,7 +724,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
 #pragma unroll
           for (int i = 0; i < 2; ++i) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) bt[i][q].u = *reinterpret_cast<const uint4*>(b_l + q * PB + (half * HT + t + i) * 1024 + lane * 16);
+            for (int q = 0; q < 3; ++q) bt[i][q].u = *reinterpret_cast<const uint4*>(b_l + q * PB + (part * HT + t + i) * 1024 + lane * 16);
           }
           f32x4 D[2] = {}, Ds[2] = {};
           rec_mma<2>(bt, U, D, Ds);
@@ -705,12 +742,13 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
       asm volatile("" : "+s"(rows), "+s"(step));                 // (no addresses of 16 rows held over the loop)
       int ln = lane;
       asm volatile("" : "+v"(ln));
-      const int r16 = ln & 15, kq = ln >> 4, row0 = half * (NP / 2) + 4 * kq, e = e0 + r16;
+      const int r16 = ln & 15, kq = ln >> 4, row0 = part * (NP / PARTS) + 4 * kq, e = e0 + r16;
       const bool e_ok = e < E;
       float* st = a.state + slot * a.state_ld + (int64_t)h * N * E + e;
-      float* xs = reinterpret_cast<float*>(u_l[0][0]) + 16 * cw + r16;           // x [32][64]
+      float* xs = reinterpret_cast<float*>(u_l[0][0]) + 16 * cw + r16;           // x [32][16 CB]
+      if (makes_x)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) xs[(16 * half + 4 * kq + s) * 64] = rec_silu_if_large(x[s]);
+        for (int s = 0; s < 4; ++s) xs[(16 * half + 4 * kq + s) * (16 * CB)] = rec_silu_if_large(x[s]);
       if (e_ok)
 #pragma unroll
         for (int t = 0; t < HT; ++t)
@@ -718,10 +756,10 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
           for (int r = 0; r < 4; ++r)
             if (row0 + 16 * t + r < rows) st[(row0 + 16 * t + r) * step] = S[t][r];
       __syncthreads();
-      if (half == 0 && on) {
+      if (part == 0 && on) {
 #pragma unroll 1
         for (int t = 0; t < cnt; ++t) {
-          const float xv = xs[t * 64], dt = fh[768 + 2 * L + t], dec = fh[768 + 3 * L + t], dx = dt * xv;
+          const float xv = xs[t * (16 * CB)], dt = fh[768 + 2 * L + t], dec = fh[768 + 3 * L + t], dx = dt * xv;
           // row t of C: this lane group's four of every 16; column t of B^T
           const uint16_t* cr = reinterpret_cast<const uint16_t*>(f) + (t >> 4) * (NT / 2) * 512 + 8 * (16 * kq + (t & 15));
           const uint16_t* br = reinterpret_cast<const uint16_t*>(f) + 3 * L * NP + 8 * (16 * ((t & 15) >> 2) + 4 * kq) + (t & 3) + 4 * (t >> 4);
@@ -751,7 +789,7 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
     // the next chunk's x
     f32x4 xn = {};
     bad = false;
-    if (more) {
+    if (more && makes_x) {
       T* raw = reinterpret_cast<T*>(own_l[w]);
       if (vec) {
         int ln = lane;
@@ -772,9 +810,10 @@ __global__ void __launch_bounds__(512, 4) ssm_chunk_walk_kernel(SsmArgs a, int64
       convolve(in, n - l0 - L, xn, bad);
       hand_over(xn, wv);
     }
-    place(c_l);
+    if constexpr (AHEAD) fetch_head(fhn, head);
+    place(c_l, stage);
     // behind the wait for the pieces (memory answers in order), so that it is the next one's: results out, raw inputs in
-    if (!serial) {
+    if (!serial && ends) {
       __builtin_amdgcn_wave_barrier();
       float* ol = reinterpret_cast<float*>(own_l[w]);
       int ln = lane;
@@ -1327,7 +1366,15 @@ static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
       return;
     }
   hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP, true>), operands, dim3(256), 0, s, a);
-  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP>), walk, dim3(512), 0, s, a, chunks);
+  if constexpr (NP > 64) {
+    // 32 columns a workgroup as long as every one of them has a CU (rec_walk_blocks: of the XCD with the most)
+    const unsigned narrow = rec_walk_blocks(a.batch * a.G, (int64_t)(a.H / a.G) * ((a.E + 31) / 32));
+    if (narrow <= 256) {
+      hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP, 2>), dim3(narrow), dim3(512), 0, s, a, chunks);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP, 4>), walk, dim3(512), 0, s, a, chunks);
 }
 
 static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,
