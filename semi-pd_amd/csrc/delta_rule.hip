@@ -626,15 +626,21 @@ __host__ __device__ constexpr int64_t delta_frag_elems(int np) { return (np <= k
 constexpr int kDeltaHead = 6 * 256 + 4 * kRecChunk;
 
 // A workgroup per (chunk, key head): convolution, silu and unit norm of its q and k (a channel per thread), K K^T and Q K^T, then
-// half a wave per head of the group: gates, A, its inverse column by column (lane = column, forward substitution), weights.
+// half a wave per head of the group: gates; weights, A and its inverse in blocks of 16 by whole waves.  Bound by what it lays down where the chip is
+// full of it (1848 workgroups, 185 MB) and by the chain of one workgroup where it is not: 42 k cycles, now 27 k (search 2.9, rows 3.5,
+// convolution 4.6, norms 2.1, pieces 4, products 2.7, gates 3.3, weights 1.3 (7.6 a column at a time, its exponentials one behind the other and
+// stores of 4 bytes), inverse 2.4 (7.5 as one chain of 32 rows)).  32 heads of 128 x 128 over 8, whole call: 1 request of 100 rows 44 -> 37.5
+// us, 5 of 155 81 -> 75, 4 of 1900 426 -> 414.
 template <typename T, int NP>
 __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs a) {
-  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4, AL = 16 * 16 + 16 * 32, LATER = 8 * AL + 2 * L * PS;
-  // K [32][CS] | Q; later A, one per half wave (rows of 16, from row 16 on of 32: it is strictly lower triangular) | K K^T | Q K^T.  36 KB and
+  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4, AL = 16 * 16 + 16 * 36, LATER = 8 * AL + 2 * L * PS;
+  // K [32][CS] | Q; later A, one per half wave (rows of 16, from row 16 on of 36: it is strictly lower triangular) | K K^T | Q K^T.  39 KB and
   // 128 registers: four workgroups a CU (45 KB and three before: 1824 workgroups took three rounds of 20 us)
   __shared__ __attribute__((aligned(16))) float kq_l[2 * L * CS > LATER ? 2 * L * CS : LATER];
   float *const kk_l = kq_l + 8 * AL, *const qk_l = kk_l + L * PS;
-  __shared__ double cum_l[8 * L];
+  __shared__ __attribute__((aligned(16))) double cum_l[8 * L];
+  __shared__ __attribute__((aligned(16))) float beta_l[8 * L];
+  __shared__ int bad_l;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, kq = lane >> 4, g = blockIdx.y;
   RecChunk at;
   if (!rec_find_chunk(a.q_len, a.seq_lens, a.q_start, (int)a.batch, blockIdx.x, at) || at.first_pos < 0) return;
@@ -644,6 +650,22 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
   float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * delta_frag_elems(NP);
   const float* kept = l0 == 0 && at.first_pos > 0 && taps > 1 ? a.conv_state + a.state_indices[at.b] * a.conv_ld : nullptr;
   bool bad = false;
+  // up to eight heads at a time, half wave `half` of wave w has w + 4 half: its decays and the diagonal blocks of its inverse; the weights
+  // and the rest of the inverse of a wave's heads by the whole wave, one head after the other (each for its own: with four heads half of the
+  // chip's waves have none, 7.3 us of a workgroup's 30).  What the first heads' gates are made of is fetched here.
+  const int half = lane >> 5, ln = tid & 31;
+  T gate_a, gate_b;
+  float gate_log, gate_bias;
+  auto fetch_gates = [&](int h0) {                               // (of rows and heads that there are; raw, so that nothing waits for them here)
+    const int h = g * per + min(h0 + w + 4 * half, per - 1);
+    const T* pr = (const T*)a.p + (t0 + min(ln, cnt - 1)) * a.ld;
+    gate_a = pr[a.a_off + h];
+    gate_b = pr[a.b_off + h];
+    gate_log = a.a_log[h];
+    gate_bias = a.dt_bias[h];
+  };
+  fetch_gates(blockIdx.z * 8);
+  if (tid == 0) bad_l = 0;
   for (int ch = tid; ch < 2 * NP; ch += 256) {
     const bool is_q = ch >= NP;
     const int d = is_q ? ch - NP : ch;
@@ -660,27 +682,31 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
     }
   }
   __syncthreads();
-  // unit norms: four lanes a row
+  // unit norms: four lanes a row, a quarter of it each (in turns that keep the sixteen lanes of an access in banks of their own)
   {
     const int row = tid >> 2, part = tid & 3;                    // rows 0 .. 31: k, 32 .. 63: q
-    float* x = kq_l + (row >= L ? L * CS : 0) + (row % L) * CS;
+    float* x = kq_l + (row >= L ? L * CS : 0) + (row % L) * CS + part * (NP / 4);
+    constexpr int Q = NP / 16;                                   // 16-byte pieces of a quarter
+    f32x4 v[Q];
     float sq = 0.f;
-    for (int d = 4 * part; d < NP; d += 16) {
-      const float4 v = *reinterpret_cast<const float4*>(x + d);
-      sq += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
-    }
+#pragma unroll
+    for (int i = 0; i < Q; ++i) v[i] = *reinterpret_cast<const f32x4*>(x + 4 * ((i + Q / 2 * (part >> 1)) % Q));
+#pragma unroll
+    for (int i = 0; i < Q; ++i) sq += (v[i][0] * v[i][0] + v[i][1] * v[i][1]) + (v[i][2] * v[i][2] + v[i][3] * v[i][3]);
     sq = quad_sum<4>(sq);
     const float inv = (row >= L ? rsqrtf((float)D) : 1.0f) / sqrtf(sq + 1e-6f);
-    for (int d = 4 * part; d < NP; d += 16) {
-      float4 v = *reinterpret_cast<const float4*>(x + d);
-      v = float4{v.x * inv, v.y * inv, v.z * inv, v.w * inv};
-      *reinterpret_cast<float4*>(x + d) = v;
-      bad |= !rec_finite(v.x) || !rec_finite(v.y) || !rec_finite(v.z) || !rec_finite(v.w);
+#pragma unroll
+    for (int i = 0; i < Q; ++i) {
+      v[i] *= inv;
+      *reinterpret_cast<f32x4*>(x + 4 * ((i + Q / 2 * (part >> 1)) % Q)) = v[i];
+      bad |= !rec_finite(v[i][0]) || !rec_finite(v[i][1]) || !rec_finite(v[i][2]) || !rec_finite(v[i][3]);
     }
+    if (__any(bad) && lane == 0) bad_l = 1;
   }
   __syncthreads();
   // the operands in the order in which they are held
   const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
+  if (lays && tid == 0) frag[delta_frag_elems(NP) - 4] = bad_l ? 1.f : 0.f;
   if constexpr (NP <= kDeltaSmall) {
     for (int i = lays ? tid : 2 * L * NP; i < 2 * L * NP / 4; i += 256) {              // K | Q: tile (row tile, column tile)
       const int half = i / (L * NP / 4), it = i % (L * NP / 4), tile = it >> 6, ln = it & 63, rt = tile / (NP / 16), ct = tile % (NP / 16);
@@ -705,7 +731,13 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
         x0 = f32x4{s[0], s[CS], s[2 * CS], s[3 * CS]};
         x1 = f32x4{s[16 * CS], s[17 * CS], s[18 * CS], s[19 * CS]};
       }
-      const Split3 s3 = rec_split8_any(x0, x1);
+      // (unit vectors: what is larger is not a number or infinite)
+      float z = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) z = fmaf(x1[q], 0.f, fmaf(x0[q], 0.f, z));
+      Split3 s3;
+      if (__any(z != 0.f)) s3 = rec_split8_any(x0, x1);
+      else s3 = rec_split8(x0, x1);
       uint4* dst = reinterpret_cast<uint4*>(frag + part * (3 * L * NP / 2)) + it;
   #pragma unroll
       for (int p = 0; p < 3; ++p) dst[p * (L * NP / 8)] = s3.p[p].u;
@@ -733,19 +765,16 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
     }
   }
   __syncthreads();
-  // up to eight heads at a time, half wave `half` of wave w has w + 4 half: its decays and its inverse; the weights of a wave's heads by both
-  // halves, one head after the other (each for its own: with four heads half of the chip's waves have none, 7.3 us of a workgroup's 30)
-  const int half = lane >> 5, ln = tid & 31;
   double* cum = cum_l + (2 * w + half) * L;
   for (int h0 = blockIdx.z * 8; h0 < per; h0 += 8 * gridDim.z) {
     if (h0 + w >= per) break;
     const int heads = h0 + w + 4 < per ? 2 : 1;                  // of this wave
     const bool mine = half < heads;
     const int h = g * per + h0 + w + (mine ? 4 * half : 0);      // (a half wave without a head of its own goes along with the other, and lays nothing down)
-    const T* pr = (const T*)a.p + (t0 + ln) * a.ld;
     const bool on = ln < cnt && mine;
-    const float la = on ? -expf(a.a_log[h]) * softplus_f(Elem<T>::to_f(pr[a.a_off + h]) + a.dt_bias[h]) : 0.f;
-    const float beta = on ? sigmoid_f(Elem<T>::to_f(pr[a.b_off + h])) : 0.f;
+    if (h0 != (int)blockIdx.z * 8) fetch_gates(h0);
+    const float la = on ? -expf(gate_log) * softplus_f(Elem<T>::to_f(gate_a) + gate_bias) : 0.f;
+    const float beta = on ? sigmoid_f(Elem<T>::to_f(gate_b)) : 0.f;
     double c = (double)la * 1.4426950408889634;
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) {
@@ -754,6 +783,7 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
     }
     const double last = __shfl(c, L - 1, L);
     cum[ln] = c;
+    beta_l[(2 * w + half) * L + ln] = beta;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kDeltaHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c), dec = expf(la);
     const bool no = !rec_finite(eb) || !rec_finite(wt) || !rec_finite(dec) || !rec_finite(beta) || !rec_moderate_decay(la);
@@ -765,51 +795,70 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
       hp[1536 + 3 * L + ln] = beta;
     }
     __builtin_amdgcn_wave_barrier();
-    // lane = s: A[t][s] and the weighted Q K^T, whose place in its tile is fixed by (t, s); rows 0 .. 15 by the lower half, 16 .. 31 by the upper
-    const int st = ln >> 4, sl = ((ln & 15) >> 2) * 64 + (ln & 3);
+    // A and the weighted Q K^T, four columns of a row a lane, tiles 00, 10, 11
     for (int v = 0; v < heads; ++v) {
       const double* cv = cum_l + (2 * w + v) * L;
-      const double cs = cv[ln];
-      float* av = kq_l + (2 * w + v) * AL + (half ? 256 : 0);
-      const int ald = half ? 32 : 16;
-      float* qv = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + g * per + h0 + w + 4 * v) * kDeltaHead + 768 +
-                  (half + st) * 256 + sl;
-#pragma unroll 4
-      for (int u = 0; u < 16; ++u) {
-        const int t = 16 * half + u;
-        const float bt = __shfl(beta, 32 * v + t, 64);
-        const float e = ln <= t ? rec_exp2(cv[t] - cs) : 0.f;
-        if (half >= st) av[u * ald + ln] = ln < t ? bt * (e * kk_l[t * PS + ln]) : 0.f;
-        if (half >= st) qv[4 * u] = ln <= t ? e * qk_l[t * PS + ln] : 0.f;
+      float* av = kq_l + (2 * w + v) * AL;
+      float* hv = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + g * per + h0 + w + 4 * v) * kDeltaHead;
+#pragma unroll
+      for (int tile = 0; tile < 3; ++tile) {
+        const int row = (tile ? 16 : 0) + r16, col = (tile == 2 ? 16 : 0) + 4 * kq;
+        const double ct = cv[row];
+        const float bt = beta_l[(2 * w + v) * L + row];
+        const f32x4 kk = *reinterpret_cast<const f32x4*>(kk_l + row * PS + col), qk = *reinterpret_cast<const f32x4*>(qk_l + row * PS + col);
+        f32x4 am, qm;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float x = rec_exp2(ct - cv[col + s]);
+          am[s] = col + s < row ? bt * (x * kk[s]) : 0.f;
+          qm[s] = col + s <= row ? x * qk[s] : 0.f;
+        }
+        *reinterpret_cast<f32x4*>(av + (tile ? 256 + r16 * 36 + col : r16 * 16 + col)) = am;
+        *reinterpret_cast<f32x4*>(hv + 768 + 256 * tile + 4 * lane) = qm;
       }
     }
     __builtin_amdgcn_wave_barrier();
+    // T = (I + A)^-1 in blocks of 16: the diagonal ones column by column, a lane each (four terms of a row at a time), into the place of A's,
+    // then T10 = -T11 A10 T00, as its transpose, so that it leaves as it stands.  (All 32 rows column by column were a chain of 496 terms.)
     if (mine) {
-      const float* a_l = kq_l + (2 * w + half) * AL;
-      // column ln of (I + A)^-1, four terms of a row at a time
-      float x[L];
+      const int st = ln >> 4, c = ln & 15, ald = st ? 36 : 16;
+      float* a_l = kq_l + (2 * w + half) * AL + (st ? 256 + 16 : 0);
+      float x[16];
 #pragma unroll
-      for (int t = 0; t < L; ++t) {
-        float acc = t == ln ? 1.f : 0.f;
+      for (int t = 0; t < 16; ++t) {
+        float acc = t == c ? 1.f : 0.f;
 #pragma unroll
         for (int s = 0; s < t; s += 4) {
-          const float4 av = *reinterpret_cast<const float4*>(a_l + (t < 16 ? t * 16 : t * 32 - 256) + s);
+          const float4 av = *reinterpret_cast<const float4*>(a_l + t * ald + s);
           acc -= av.x * x[s];
           if (s + 1 < t) acc -= av.y * x[s + 1];
           if (s + 2 < t) acc -= av.z * x[s + 2];
           if (s + 3 < t) acc -= av.w * x[s + 3];
         }
         x[t] = acc;
-        asm volatile("" : "+v"(x[t]));                             // (row by row: not all rows of A first and the sums behind them)
       }
+      __builtin_amdgcn_wave_barrier();
 #pragma unroll
-      for (int t = 0; t < L; ++t)
-        if (t >= 16 || st == 0) hp[((t >> 4) + st) * 256 + sl + (t & 15) * 4] = x[t] * beta;
+      for (int t = 0; t < 16; ++t) a_l[t * ald + c] = x[t];
+    }
+    __builtin_amdgcn_wave_barrier();
+    for (int v = 0; v < heads; ++v) {
+      const float *tl = kq_l + (2 * w + v) * AL, *bv = beta_l + (2 * w + v) * L;
+      float* hv = a.frags + (int64_t)gridDim.x * a.G * delta_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + g * per + h0 + w + 4 * v) * kDeltaHead;
+      const f32x4 t00 = *reinterpret_cast<const f32x4*>(tl + r16 * 16 + 4 * kq), a10 = *reinterpret_cast<const f32x4*>(tl + 256 + r16 * 36 + 4 * kq);
+      const f32x4 t11 = *reinterpret_cast<const f32x4*>(tl + 256 + r16 * 36 + 16 + 4 * kq);
+      const f32x4 b0 = *reinterpret_cast<const f32x4*>(bv + 4 * kq), b1 = *reinterpret_cast<const f32x4*>(bv + 16 + 4 * kq);
+      f32x4 y = {}, z = {};
+#pragma unroll
+      for (int s = 0; s < 4; ++s) y = __builtin_amdgcn_mfma_f32_16x16x4f32(a10[s], tl[(4 * kq + s) * 16 + r16], y, 0, 0, 0);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) z = __builtin_amdgcn_mfma_f32_16x16x4f32(y[s], t11[s], z, 0, 0, 0);
+      *reinterpret_cast<f32x4*>(hv + 4 * lane) = t00 * b0;
+      *reinterpret_cast<f32x4*>(hv + 256 + 4 * lane) = -z * b0;
+      *reinterpret_cast<f32x4*>(hv + 512 + 4 * lane) = t11 * b1;
     }
     __builtin_amdgcn_wave_barrier();
   }
-  const int any_bad = __syncthreads_or(bad);
-  if (lays && tid == 0) frag[delta_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
 // The chunks of a request in turn, a workgroup of eight waves per (request, head, 16 CB columns of S), two or four waves per 16 columns.  A wave

@@ -338,14 +338,17 @@ constexpr int kSsmHead = 3 * 256 + 4 * kRecChunk;
 // What the heads of a group share, a workgroup per (chunk, group): convolution + bias + silu of the group's B and C channels (a
 // channel per thread, its taps and the last inputs in registers), laid down as operands; the 32 x 32 products C B^T and, half a wave
 // per head in turn (lane = token), step sizes, running log decays and the weighted C B^T.  NP: N up to a multiple of 64, zeros behind
-// N and behind the portion.
+// N and behind the portion.  The first heads' gates are fetched in front of the convolution, and nothing waits for what is written: 128 heads of 128
+// x 64 over 8, 1 request of 100 rows, whole call, 37.3 -> 35.8 us, 6 of 28 51.2 -> 49.2; a chip full of it lays down 197 MB and is
+// bound by these (4 of 1900 within the noise).
 template <typename T, int NP, bool PIECES>
-__global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
-  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 1;
+__global__ void __launch_bounds__(256, 4) ssm_chunk_operands_kernel(SsmArgs a) {
+  constexpr int L = kRecChunk, CS = NP + 4, PS = L + 4;
   __shared__ __attribute__((aligned(16))) float c_l[L * CS];
   __shared__ __attribute__((aligned(16))) float b_l[L * CS];
-  __shared__ float cb_l[L * PS];
-  __shared__ double cum_l[8 * L];
+  float* const cb_l = c_l;                                      // (C B^T, behind the products)
+  __shared__ __attribute__((aligned(16))) double cum_l[8 * L];
+  __shared__ __attribute__((aligned(16))) float dt_l[8 * L];
   const int tid = threadIdx.x, g = blockIdx.y;
   RecChunk at;
   if (!rec_find_chunk(a.q_len, a.seq_lens, a.q_start, (int)a.batch, blockIdx.x, at) || at.first_pos < 0) return;
@@ -356,6 +359,17 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
   float* frag = a.frags + ((int64_t)blockIdx.x * a.G + g) * ssm_frag_elems(NP);
   const float* kept = l0 == 0 && at.first_pos > 0 && taps > 1 ? a.conv_state + a.state_indices[at.b] * a.conv_ld : nullptr;
   bool bad = false;
+  // what the first heads' step sizes are made of: raw, so that nothing waits for it here
+  const int hw = tid >> 5, t = tid & 31;
+  T gate_dt;
+  float gate_bias, gate_log;
+  auto fetch_gates = [&](int hh) {                               // (of rows and heads that there are)
+    const int h = g * per + min(hh, per - 1);
+    gate_dt = ((const T*)a.p)[(t0 + min(t, cnt - 1)) * a.ld + a.dt_off + h];
+    gate_bias = a.dt_bias[h];
+    gate_log = a.a_log[h];
+  };
+  fetch_gates(blockIdx.z * 8 + hw);
   for (int ch = tid; ch < 2 * NP; ch += 256) {
     const bool is_c = ch >= NP;
     const int r = is_c ? ch - NP : ch;
@@ -373,8 +387,9 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
       for (int t = 0; t < L; ++t) dst[t * CS] = 0.f;
     }
   }
-  __syncthreads();
+  const int any_bad = __syncthreads_or(bad);
   const bool lays = blockIdx.z == 0;                             // (the workgroups of a group's heads all have the operands, one lays them down)
+  if (lays && tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;      // (at the end that would wait for what is written)
   if constexpr (PIECES) {
     // pieces of three planes: C, tiles (16 tokens, 32 rows of S), and B^T, tiles (16 rows of S, the tokens)
     for (int i = lays ? tid : L * NP; i < 2 * (L * NP / 8); i += 256) {
@@ -390,7 +405,15 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
         x0 = f32x4{s[0], s[CS], s[2 * CS], s[3 * CS]};
         x1 = f32x4{s[16 * CS], s[17 * CS], s[18 * CS], s[19 * CS]};
       }
-      const Split3 s3 = rec_split8_any(x0, x1);
+      float most = 0.f, z = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        z = fmaf(x1[q], 0.f, fmaf(x0[q], 0.f, z));
+        most = fmaxf(most, fmaxf(fabsf(x0[q]), fabsf(x1[q])));
+      }
+      Split3 s3;
+      if (__any(z != 0.f || most > 0x1p126f)) s3 = rec_split8_any(x0, x1);
+      else s3 = rec_split8(x0, x1);
       uint4* dst = reinterpret_cast<uint4*>(frag + (is_c ? 0 : 3 * L * NP / 2)) + it;
 #pragma unroll
       for (int p = 0; p < 3; ++p) dst[p * (L * NP / 8)] = s3.p[p].u;
@@ -417,16 +440,17 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
 #pragma unroll
       for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
     }
+    __syncthreads();                                              // (C and B have been read)
 #pragma unroll
     for (int r = 0; r < 4; ++r) cb_l[(i0 + 4 * kq + r) * PS + j0 + r16] = acc[r];
   }
   __syncthreads();
-  const int hw = tid >> 5, t = tid & 31;
   double* cum = cum_l + hw * L;
   for (int hh = blockIdx.z * 8 + hw; hh < per; hh += 8 * gridDim.z) {
     const int h = g * per + hh;
-    const float dt = t < cnt ? ssm_softplus(Elem<T>::to_f(((const T*)a.p)[(t0 + t) * a.ld + a.dt_off + h]) + a.dt_bias[h]) : 0.f;
-    const float la = t < cnt ? -expf(a.a_log[h]) * dt : 0.f;
+    if (hh != (int)blockIdx.z * 8 + hw) fetch_gates(hh);
+    const float dt = t < cnt ? ssm_softplus(Elem<T>::to_f(gate_dt) + gate_bias) : 0.f;
+    const float la = t < cnt ? -expf(gate_log) * dt : 0.f;
     double c = (double)la * 1.4426950408889634;
 #pragma unroll
     for (int o = 1; o < L; o <<= 1) {
@@ -435,6 +459,7 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     }
     const double last = __shfl(c, L - 1, L);
     cum[t] = c;
+    dt_l[hw * L + t] = dt;
     float* hp = a.frags + (int64_t)gridDim.x * a.G * ssm_frag_elems(NP) + ((int64_t)blockIdx.x * a.H + h) * kSsmHead;
     const float eb = rec_exp2(c), wt = rec_exp2(last - c) * dt, dec = expf(la);
     // (a weight beyond 2^8 with B and x of up to 2^59: the pieces of a sum that leaves 32 bits would leave it with either sign)
@@ -443,16 +468,17 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     hp[768 + 2 * L + t] = dt;
     hp[768 + 3 * L + t] = dec;
     __builtin_amdgcn_wave_barrier();
-    // the weighted C B^T, 16 bytes a lane: piece i of 192 is lane i % 64 of tile i / 64; the step size of column s from lane s
+    // the weighted C B^T, 16 bytes a lane: piece i of 192 is lane i % 64 of tile i / 64
 #pragma unroll
     for (int u = 0; u < 6; ++u) {
       const int i = u * 32 + t, tile = i >> 6, ln = i & 63, row = (tile ? 16 : 0) + (ln & 15), col = (tile == 2 ? 16 : 0) + 4 * (ln >> 4);
       const double bt = cum[row];
+      const f32x4 cb = *reinterpret_cast<const f32x4*>(cb_l + row * PS + col), ds = *reinterpret_cast<const f32x4*>(dt_l + hw * L + col);
       f32x4 m;
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
-        const float ds = __shfl(dt, col + v, L);
-        m[v] = col + v <= row ? cb_l[row * PS + col + v] * (rec_exp2(bt - cum[col + v]) * ds) : 0.f;
+        const float x = cb[v] * (rec_exp2(bt - cum[col + v]) * ds[v]);
+        m[v] = col + v <= row ? x : 0.f;
         no |= !rec_finite(m[v]);
       }
       *reinterpret_cast<f32x4*>(hp + 4 * i) = m;
@@ -460,8 +486,6 @@ __global__ void __launch_bounds__(256) ssm_chunk_operands_kernel(SsmArgs a) {
     hp[768 + t] = rec_flagged(eb, no);
     __builtin_amdgcn_wave_barrier();
   }
-  const int any_bad = __syncthreads_or(bad);
-  if (lays && tid == 0) frag[ssm_frag_elems(NP) - 4] = any_bad ? 1.f : 0.f;
 }
 
 // The chunks of a request in turn, a workgroup of eight waves per (request, head, 16 CB columns of S), two or four waves per 16 columns.  A wave
