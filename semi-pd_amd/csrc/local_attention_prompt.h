@@ -137,17 +137,18 @@ __device__ __forceinline__ PromptTile prompt_tile_by_keys(uint32_t at, int batch
   return PromptTile{r, block * (int)period + lo + (left - block * wid) - __builtin_amdgcn_readlane((int)u, r)};
 }
 
-template <typename T, int D, int E, int NW, int KT, bool SIG>
-__global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnArgs a, int hw, int by_keys, int runs) {
-  constexpr int NT = 64 * NW, KU = KT / 32;                     // KT: keys a step
+template <typename T, int D, int E, int NW, int KT, int KS, bool SIG>
+__global__ void __launch_bounds__(64 * NW * KS, 2) prompt_attention_kernel(LocalAttnArgs a, int hw, int by_keys, int runs) {
+  constexpr int NT = 64 * NW, KU = KT / 32;                     // KT: keys a step; KS: groups of NW waves that take steps in turn
   constexpr int KB = D * 2, VB = E * 2, CK = D / 8, CV = E / 8;  // bytes and 16-byte chunks of a row
   constexpr int NK = KT * CK / NT, NV = KT * CV / NT;          // chunks a thread stages
   constexpr int KSW = CK < 16 ? CK - 1 : 15, VSW = E >= 128 ? 3 : 1;
   constexpr int ET = E / 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-  uint8_t* const k_lds = lds;                                   // [2][KT][KB]
-  uint8_t* const v_lds = lds + 2 * KT * KB;                     // [2][KT][VB]
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
+  const int group = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;
+  uint8_t* const k_lds = lds + group * (2 * KT * (KB + VB));    // [2][KT][KB]
+  uint8_t* const v_lds = k_lds + 2 * KT * KB;                   // [2][KT][VB]
+  const int tid = threadIdx.x % NT, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 31, hi = lane >> 5;
   // Workgroup -> (kv head, tile, heads of the group), the last fastest.  An XCD (workgroup ids go round the 8) has kv heads of its own, or
   // shares them with the fewest others, every so many tiles its own, or (runs) a run of them: workgroups that read the same K and V rows run
   // next to each other on one L2, and every XCD has as many long tiles.  Tiles from the last (most keys) to the first, or by their keys (by_keys).  A contiguous
@@ -283,21 +284,20 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   const uint8_t* va = v_lds + vrow * VB + g1 * 32 + (gi & 3) * 8;
   const int kx = col & KSW, vx = vrow & VSW;
 
-  load_slots(0);
+  load_slots(group);                                            // (a step behind the last: the last key)
   load_rows();
-  if (steps > 1) load_slots(1);
+  if (group + KS < steps) load_slots(group + KS);
   store_rows(0);
   __syncthreads();
-  for (int it = 0; it < steps; ++it) {
-    const int buf = it & 1;
-    if (it + 1 < steps) {
+  for (int it = group, buf = 0; it - group < steps; it += KS, buf ^= 1) {
+    if (it + KS < steps) {
       load_rows();
-      if (it + 2 < steps) load_slots(it + 2);
+      if (it + 2 * KS < steps) load_slots(it + 2 * KS);
     }
     const bool first = it < first_steps;
     const int j0 = first ? it * KT : key_lo + (it - first_steps) * KT;
     // 0: no row of the wave sees a key of the step; 2: every row sees all of them
-    const bool some = wave_on && (first || (j0 <= w_hi && (j0 + KT - 1 >= w_lo || j0 < keep)));
+    const bool some = wave_on && (KS == 1 || it < steps) && (first || (j0 <= w_hi && (j0 + KT - 1 >= w_lo || j0 < keep)));
     if (some) {
       const uint8_t* kb = ka + buf * KT * KB;
       const uint8_t* vb = va + buf * KT * VB;
@@ -403,8 +403,44 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
         }
       }
     }
-    if (it + 1 < steps) store_rows(buf ^ 1);
+    if (it + KS < steps) store_rows(buf ^ 1);
     __syncthreads();                                            // the next step's rows are in place, everyone is done with this step's
+  }
+  // the groups' sums, by way of LDS (the walk ended on a barrier)
+  constexpr int MERGE = ET * 4096 + 512;                        // bytes of a wave
+  if constexpr (KS > 1) {
+    if (steps > 1) {
+      if (group > 0) {
+        float* const ml = reinterpret_cast<float*>(lds + ((group - 1) * NW + wave) * MERGE);
+#pragma unroll
+        for (int t = 0; t < ET; ++t)
+#pragma unroll
+          for (int r = 0; r < 16; r += 4) *reinterpret_cast<f32x4*>(ml + (4 * t + r / 4) * 256 + 4 * lane) = f32x4{o[t][r], o[t][r + 1], o[t][r + 2], o[t][r + 3]};
+        ml[ET * 1024 + lane] = m;
+        ml[ET * 1024 + 64 + lane] = l;
+      }
+      __syncthreads();
+    }
+    if (group > 0) return;
+    for (int other = 1; other < KS && other < steps; ++other) {
+      const float* const ml = reinterpret_cast<const float*>(lds + ((other - 1) * NW + wave) * MERGE);
+      float f0 = 1.f, f1 = 1.f;
+      if constexpr (!SIG) {
+        const float m1 = ml[ET * 1024 + lane], m0 = m;
+        m = fmaxf(m0, m1);
+        f0 = m0 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m0 - m);
+        f1 = m1 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m1 - m);
+        l = fmaf(l, f0, ml[ET * 1024 + 64 + lane] * f1);
+      }
+#pragma unroll
+      for (int t = 0; t < ET; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(ml + (4 * t + r / 4) * 256 + 4 * lane);
+#pragma unroll
+          for (int u = 0; u < 4; ++u) o[t][r + u] = SIG ? o[t][r + u] + v[u] : fmaf(o[t][r + u], f0, v[u] * f1);
+        }
+    }
   }
   if constexpr (!SIG) {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(l), __float_as_uint(l), false, false);
@@ -432,7 +468,8 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
   // out through the wave's part of the tiles (the walk ended on a barrier): a lane holds four neighbouring elements of one row at a
   // time, rows leave in 16-byte pieces of consecutive lanes
   constexpr int OS = E * 2 + 16;
-  uint8_t* ol = lds + wave * 32 * OS;
+  static_assert(32 * OS <= MERGE, "a wave leaves by way of what it has merged");
+  uint8_t* ol = lds + wave * (KS == 1 ? 32 * OS : MERGE);
 #pragma unroll
   for (int t = 0; t < ET; ++t)
 #pragma unroll
@@ -463,8 +500,12 @@ __global__ void __launch_bounds__(64 * NW, 2) prompt_attention_kernel(LocalAttnA
 
 // true: launched.  Head sizes 64 / 64, 64 / 128, 128 / 128, 128 / 256 (sigmoid weights: 64 / 64, 128 / 128), a positive scale, 16-bit
 // types, everything aligned as local_attention_mfma_kernel wants it.
-template <typename T, int D, int E, int NW, int KT, bool SIG>
-static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
+struct PromptPlan {
+  int hw;
+  int64_t avg, n_tiles, blocks;
+  PromptShare share;
+};
+static PromptPlan prompt_plan(const LocalAttnArgs& a, int NW) {
   const int rep = a.H / a.G;
   // heads of a group in a workgroup: the largest power of two that divides them, or the next one above them (the last set's waves are not all
   // busy) where that makes fewer workgroups of requests of the average length.  24 / 8 heads, 32 requests of 20 tokens: one head and room
@@ -476,12 +517,19 @@ static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   const auto count = [&](int w) { return (avg + 32 * (NW / w) - 1) / (32 * (NW / w)) * ((rep + w - 1) / w); };
   if (count(wide) < count(hw)) hw = wide;
   const int rows = 32 * (NW / hw);
-  a.n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
-  constexpr size_t tiles = 2 * KT * (size_t)(D + E) * 2, epilogue = NW * 32 * (size_t)(E * 2 + 16), bytes = tiles > epilogue ? tiles : epilogue;
+  const int64_t n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
+  const PromptShare share = prompt_share(a.G, (uint32_t)n_tiles);
+  return PromptPlan{hw, avg, n_tiles, 8ll * share.heads * share.tiles * ((rep + hw - 1) / hw), share};
+}
+template <typename T, int D, int E, int NW, int KT, int KS, bool SIG>
+static int launch_prompt_attention(LocalAttnArgs a, const PromptPlan& plan, hipStream_t s) {
+  const int rep = a.H / a.G, hw = plan.hw, rows = 32 * (NW / hw);
+  const int64_t avg = plan.avg, blocks = plan.blocks;
+  const PromptShare share = plan.share;
+  a.n_tiles = plan.n_tiles;
+  constexpr size_t tiles = KS * 2 * KT * (size_t)(D + E) * 2, epilogue = NW * (KS > 1 ? (KS - 1) * (size_t)(E * 128 + 512) : 32 * (size_t)(E * 2 + 16)), bytes = tiles > epilogue ? tiles : epilogue;
   static std::atomic<uint64_t> done{0};
-  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
-  const PromptShare share = prompt_share(a.G, (uint32_t)a.n_tiles);
-  const int64_t blocks = 8ll * share.heads * share.tiles * ((rep + hw - 1) / hw);
+  if (ensure_dynamic_lds((const void*)prompt_attention_kernel<T, D, E, NW, KT, KS, SIG>, bytes, done, "local_attention")) return SEMIPD_EINVAL;
   // Tiles by their keys where they differ by blocks or by requests (one sequence without blocks is in that order anyway, and windows make
   // most tiles alike) and the launch is between one (two) and eight times what the chip takes at once: below that all start together, above
   // the end of the launch is little of it. (Blocks of a few steps: a tile's start and end are most of its time, and all are nearly alike.)
@@ -489,7 +537,7 @@ static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   // 38.5, 1 of 16000 217.7 / 211.1, 4 of 6000 (12 times) 337 / 338; 24 / 8 heads, blocks of 256, 4 of 1900 45.8 / 44.3, 2 of 1500 21.6 /
   // 25.0; without blocks 2 of 3000 168 / 154, 2 of 1500 (1.5 times) 52.6 / 53.9, 16 of 500 (each workgroup asks for all 16) 83.8 / 86.8;
   // values of 256, 2 heads, 2 of 3000 326 / 299.
-  const int64_t at_once = 256 * 8 / NW;
+  const int64_t at_once = 256 * 8 / (NW * KS);
   const bool by_keys = a.window == 0 && a.batch <= 8 && (a.chunk > 0 ? a.chunk >= 512 && a.chunk % rows == 0 && blocks > at_once : a.batch > 1 && blocks > 2 * at_once) &&
                        blocks <= 8 * at_once;
   // A run of tiles an XCD where tiles next to each other read the same few keys and are nearly alike: blocks of up to 256 of a few requests, and
@@ -502,17 +550,38 @@ static int launch_prompt_attention(LocalAttnArgs a, hipStream_t s) {
   const int64_t bound = a.window > 0 ? a.window : a.chunk;
   const bool runs = !by_keys && avg >= 256 && !(over > 0 && over <= few) &&
                     (a.batch <= 8 ? a.chunk > 0 && a.chunk <= 256 : share.shift == 3 && (bound == 0 || bound > 256));
-  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, SIG>), dim3((unsigned)blocks), dim3(64 * NW), bytes, s, a, hw, (int)by_keys, (int)runs);
+  hipLaunchKernelGGL((prompt_attention_kernel<T, D, E, NW, KT, KS, SIG>), dim3((unsigned)blocks), dim3(64 * NW * KS), bytes, s, a, hw, (int)by_keys, (int)runs);
   return 0;
+}
+// Launches of at most a workgroup a CU are as long as their longest tile, a chain of steps at 1.7 us with a wave on every SIMD and 2.7 with
+// two: tiles of 64 rows and heads whose steps four groups of two waves take in turn, then of 128 and two groups of four, as long as every
+// tile has a CU of its own; not where all walks are short, which gain nothing from it.  (Behind that a CU has the second wave from another
+// tile.)  One / two / four groups, whole call, us: 32 / 8 heads of 128, 1 prompt of 300 tokens 15.4 / 15.5 / 14.2, of 600 23.6 / 21.4 / 21.9
+// (320 tiles), of 933 33.0 / 30.0 / 32.3 (480), 30 tokens behind 900 30.6 / 27.0 / 21.9, 2 of 339 behind 104 21.3 / 19.4 / 23.5 (384); 24 / 8 heads, 1 of
+// 600 24.5 / 21.3 / 18.3; 32 / 8 of 64, 30 behind 900 22.2 / 19.6 / 15.6; blocks of 128, 1 of 933 13.0 / 13.9 / 22.4, of 256, 1 of 600 14.9 / 14.8 / 19.3.  Values
+// of 256 (the second form of 512 against eight waves in one group): 1 of 600 51.8 / 45.2, 1 of 933 72 / 62, 7 of 101 24.9 / 24.5.
+template <typename T, int D, int E, bool SIG>
+static int split_prompt_attention(const LocalAttnArgs& a, hipStream_t s) {
+  constexpr int NW = E > 128 ? 8 : 4, KT = E > 128 ? 32 : 64;
+  const int64_t bound = a.window > 0 ? a.window : a.chunk;
+  if (bound == 0 || bound >= 512) {
+    if constexpr (E <= 128) {
+      const PromptPlan few = prompt_plan(a, 2);
+      if (few.blocks <= 256) return launch_prompt_attention<T, D, E, 2, (D + E > 128 ? 32 : 64), 4, SIG>(a, few, s);
+    }
+    const PromptPlan few = prompt_plan(a, 4);
+    if (few.blocks <= 256) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
+  }
+  return launch_prompt_attention<T, D, E, NW, KT, 1, SIG>(a, prompt_plan(a, NW), s);
 }
 template <typename T>
 static bool prompt_attention(const LocalAttnArgs& a, hipStream_t s, int& rc) {
   const bool sig = a.sigmoid != 0;
   if (!(a.scale > 0.f) || a.k_ld <= 0 || a.v_ld <= 0 || a.k_ld >= (1ll << 31) || a.v_ld >= (1ll << 31)) return false;
-  if (a.D == 128 && a.E == 128) rc = sig ? launch_prompt_attention<T, 128, 128, 4, 64, true>(a, s) : launch_prompt_attention<T, 128, 128, 4, 64, false>(a, s);
-  else if (a.D == 64 && a.E == 64) rc = sig ? launch_prompt_attention<T, 64, 64, 4, 64, true>(a, s) : launch_prompt_attention<T, 64, 64, 4, 64, false>(a, s);
-  else if (a.D == 64 && a.E == 128 && !sig) rc = launch_prompt_attention<T, 64, 128, 4, 64, false>(a, s);
-  else if (a.D == 128 && a.E == 256 && !sig) rc = launch_prompt_attention<T, 128, 256, 8, 32, false>(a, s);
+  if (a.D == 128 && a.E == 128) rc = sig ? split_prompt_attention<T, 128, 128, true>(a, s) : split_prompt_attention<T, 128, 128, false>(a, s);
+  else if (a.D == 64 && a.E == 64) rc = sig ? split_prompt_attention<T, 64, 64, true>(a, s) : split_prompt_attention<T, 64, 64, false>(a, s);
+  else if (a.D == 64 && a.E == 128 && !sig) rc = split_prompt_attention<T, 64, 128, false>(a, s);
+  else if (a.D == 128 && a.E == 256 && !sig) rc = split_prompt_attention<T, 128, 256, false>(a, s);
   else return false;
   return true;
 }

@@ -278,3 +278,48 @@ def _rows_once(H, G, block, lens, olds):
             want = torch.softmax(s.masked_fill(~see(p, j), -float("inf")), -1) @ t["v"][rows, h // (H // G)].double()
             torch.testing.assert_close(got[at: at + new, h * D: (h + 1) * D], want, rtol=6 * 2.0 ** -8, atol=12 * 2.0 ** -8)
         at += new
+
+
+# (tiles of a launch: up to 256 of 64 rows and heads, of 128, more; a few steps for four groups of waves, and one or two fewer than the groups)
+@pytest.mark.parametrize("lens,olds", [([150, 33, 64], [0, 30, 700]), ([500, 200], [0, 561]), ([900, 260], [60, 0])])
+@pytest.mark.parametrize("H,G,D,E", [(32, 8, 128, 128), (24, 8, 64, 64), (16, 2, 128, 256), (32, 8, 64, 128)])
+@pytest.mark.parametrize("form", ["causal", "cap", "window", "keep", "sigmoid"])
+def test_steps_in_turns(lens, olds, H, G, D, E, form):
+    """Groups of waves that take a tile's steps in turn, and their sums together: tolerances as above."""
+    from semi_pd_amd import ops
+    dtype = torch.bfloat16
+    if E != D:
+        if form != "causal":
+            pytest.skip("shared value rows have no further options")
+        t, g = _batch(lens, olds, H, G, D, E // G, dtype, H + D, shared=True)
+    else:
+        t, g = _batch(lens, olds, H, G, D, E, dtype, H + D)
+    per_head = torch.randn(H, generator=g)
+    n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+    out = torch.empty(sum(lens), H * E, dtype=dtype, device=DEV)
+    batch = (d["q"], out, d["k"], d["v"], d["table"], torch.arange(len(lens), device=DEV), torch.tensor(t["totals"], device=DEV), start.to(DEV),
+             n.to(DEV), max(lens), D ** -0.5)
+    head, causal = per_head.to(DEV), lambda p, j: j <= p
+    if E != D:
+        ops.shared_value_attention_fwd(*batch)
+        want = _dense(t, lens, olds, H, G, D, E, causal, _softmax(), shared=True)
+    elif form in ("causal", "cap"):
+        cap = 2.0 if form == "cap" else 0.0
+        ops.local_attention_fwd(*batch, cap, 0, head if form == "causal" else None, None)
+        want = _dense(t, lens, olds, H, G, D, E, causal, _softmax(per_head if form == "causal" else None, cap=cap))
+    else:
+        keep = 0 if form == "window" else 70 if form == "keep" else 3
+        see = lambda p, j: (j <= p) & ((p - j < 520) | (j < keep))          # noqa: E731
+        if form == "sigmoid":
+            ops.window_attention_fwd(*batch, 520, keep, head, True, None, 1.2)
+            want = _dense(t, lens, olds, H, G, D, E, see, lambda s, ok, h: 1.2 * torch.sigmoid(s + per_head[h].double()).masked_fill(~ok, 0.0))
+        else:
+            ops.window_attention_fwd(*batch, 520, keep, None, False, head, 1.0)
+            want = _dense(t, lens, olds, H, G, D, E, see, _softmax(per_head))
+    ulp = 2.0 ** -8
+    err = (out.cpu().double() - want).norm() / want.norm()
+    assert float(err) < 1.5 * ulp, float(err)
+    # (sigmoid weights are not divided by their sum: rounding of up to 520 of them where above there are 40, errors of the root of that)
+    wide = (520 / 40) ** 0.5 if form == "sigmoid" else 1.0
+    torch.testing.assert_close(out.cpu().double(), want, rtol=6 * ulp, atol=12 * ulp * wide)
