@@ -3,7 +3,8 @@
 //
 //  * A workgroup: NW waves = HW query heads of ONE key/value head x NW / HW blocks of 32 rows, so the rows of K and V that it
 //    stages serve up to NW heads.  Heads share the visible range, and every wave of a workgroup has the same number of steps.
-//  * A step: KT keys (64; 32 for value rows of 256).  Their K and V rows go through two pairs of LDS tiles (step i + 1 lands in
+//  * Launches of few tiles: KS groups of NW waves in a workgroup, which take its steps in turn (split_prompt_attention has the rule).
+//  * A step: KT keys (64; 32 for value rows of 256 and groups of two waves).  Their K and V rows go through two pairs of LDS tiles (step i + 1 lands in
 //    registers while step i is multiplied; one barrier a step).  S^T = K Q^T and O^T += V^T P^T on v_mfma_f32_32x32x16: a lane holds one query's column
 //    throughout, P^T goes from the accumulators into the second product in place (its key order is matched by the rows that the
 //    transposing reads of V take).
@@ -560,6 +561,10 @@ static int launch_prompt_attention(LocalAttnArgs a, const PromptPlan& plan, hipS
 // (320 tiles), of 933 33.0 / 30.0 / 32.3 (480), 30 tokens behind 900 30.6 / 27.0 / 21.9, 2 of 339 behind 104 21.3 / 19.4 / 23.5 (384); 24 / 8 heads, 1 of
 // 600 24.5 / 21.3 / 18.3; 32 / 8 of 64, 30 behind 900 22.2 / 19.6 / 15.6; blocks of 128, 1 of 933 13.0 / 13.9 / 22.4, of 256, 1 of 600 14.9 / 14.8 / 19.3.  Values
 // of 256 (the second form of 512 against eight waves in one group): 1 of 600 51.8 / 45.2, 1 of 933 72 / 62, 7 of 101 24.9 / 24.5.
+// Up to two tiles a CU where they differ most, in one or two requests whose rows see all in front of them: two tiles at once take as long as
+// the longer one, one behind the other (the longest first) as their mean.  One / two groups: 32 / 8 heads of 128, 1 prompt of 1500 tokens 50.1 / 42.6, 2 of
+// 1000 38.4 / 36.4 (24 / 8 heads 48.5 / 39.9, 37.1 / 31.7; of 64 34.1 / 28.0, 26.6 / 24.5), values of 256, 1 of 1500 107 / 91; but windows of 1000, 1 of 2000 49.8
+// / 60.6, 4 of 300 19.6 / 23.8, values of 128 and keys of 64, 2 of 1086 46.8 / 48.6; beyond, 1 of 3000 103 / 111.
 template <typename T, int D, int E, bool SIG>
 static int split_prompt_attention(const LocalAttnArgs& a, hipStream_t s) {
   constexpr int NW = E > 128 ? 8 : 4, KT = E > 128 ? 32 : 64;
@@ -570,7 +575,8 @@ static int split_prompt_attention(const LocalAttnArgs& a, hipStream_t s) {
       if (few.blocks <= 256) return launch_prompt_attention<T, D, E, 2, (D + E > 128 ? 32 : 64), 4, SIG>(a, few, s);
     }
     const PromptPlan few = prompt_plan(a, 4);
-    if (few.blocks <= 256) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
+    const bool uneven = (a.batch == 1 || (a.batch == 2 && E == D)) && (a.window == 0 || a.window >= few.avg);
+    if (few.blocks <= (uneven ? 512 : 256)) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
   }
   return launch_prompt_attention<T, D, E, NW, KT, 1, SIG>(a, prompt_plan(a, NW), s);
 }

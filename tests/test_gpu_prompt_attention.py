@@ -281,19 +281,14 @@ def _rows_once(H, G, block, lens, olds):
 
 
 # (tiles of a launch: up to 256 of 64 rows and heads, of 128, more; a few steps for four groups of waves, and one or two fewer than the groups)
-@pytest.mark.parametrize("lens,olds", [([150, 33, 64], [0, 30, 700]), ([500, 200], [0, 561]), ([900, 260], [60, 0])])
-@pytest.mark.parametrize("H,G,D,E", [(32, 8, 128, 128), (24, 8, 64, 64), (16, 2, 128, 256), (32, 8, 64, 128)])
-@pytest.mark.parametrize("form", ["causal", "cap", "window", "keep", "sigmoid"])
+@pytest.mark.parametrize("lens,olds", [([150, 33, 64], [0, 30, 700]), ([500, 200], [0, 561]), ([900, 260], [60, 0]), ([1290], [3])])
+@pytest.mark.parametrize("H,G,D,E,form", [(H, 8, D, D, form) for H, D in ((32, 128), (24, 64)) for form in ("causal", "cap", "window", "keep", "sigmoid")] +
+                         [(16, 2, 128, 256, "causal"), (32, 8, 64, 128, "causal")])
 def test_steps_in_turns(lens, olds, H, G, D, E, form):
     """Groups of waves that take a tile's steps in turn, and their sums together: tolerances as above."""
     from semi_pd_amd import ops
     dtype = torch.bfloat16
-    if E != D:
-        if form != "causal":
-            pytest.skip("shared value rows have no further options")
-        t, g = _batch(lens, olds, H, G, D, E // G, dtype, H + D, shared=True)
-    else:
-        t, g = _batch(lens, olds, H, G, D, E, dtype, H + D)
+    t, g = _batch(lens, olds, H, G, D, E // G if E != D else E, dtype, H + D)
     per_head = torch.randn(H, generator=g)
     n, start = torch.tensor(lens, dtype=torch.int32), torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()
     d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
