@@ -22,12 +22,14 @@ decode_mfma_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __res
   const int c16 = lane & 15, q4 = lane >> 4;
   const int64_t item = (int64_t)blockIdx.x * 4 + wave;
   if (item >= total_items) return;  // no workgroup barrier below: waves are independent
-  const int split = (int)(item % num_kv_splits);
-  int64_t tmp = item / num_kv_splits;
-  const int tile = (int)(tmp % tiles_per_kv);
-  tmp /= tiles_per_kv;
+  // the kv heads of one range next to each other: a workgroup reads the rows of a token in whole KB, not 256 B of each four times as far
+  // apart (32 requests of 1100, 8 kv heads of 128, whole call: 39.3 -> 35.8 us; 19 of 146 14.0 -> 12.3; 150 of 2500 as before)
+  const int tile = (int)(item % tiles_per_kv);
+  int64_t tmp = item / tiles_per_kv;
   const int hk = (int)(tmp % num_kv_heads);
-  const int b = (int)(tmp / num_kv_heads);
+  tmp /= num_kv_heads;
+  const int split = (int)(tmp % num_kv_splits);
+  const int b = (int)(tmp / num_kv_splits);
   const int h0 = tile * 16;
   const int heads = min(16, group - h0);
   const int hq0 = hk * group + h0;

@@ -12,8 +12,12 @@
 // in-lane max of 8 values plus two lane exchanges, P^T is already in B-operand order, and the O
 // rescale is one scalar per lane.  Per 32 tokens a wave issues 16 MFMAs and ~60 VALU ops instead of
 // the ~1100 VALU ops of the shuffle kernel, so the kernel stays on the HBM roofline for G = 4..16.
-// Tile i+1 (K fragments, V rows, indices) is in flight in registers while tile i is computed.
+// Tile i+1 is in flight in registers while tile i is computed: its V rows from where those of tile i are in LDS, its K fragments from behind the
+// products of tile i's (two sets of these took 40 registers more and gained nothing).  8 kv heads of 128, whole call: 6 requests of 122 12.5 -> 9.7
+// us (fp8 rows 14.8 -> 11.6), 25 of 1340 in fp8 28.8 -> 25.8, 150 of 2500 in fp8 291 -> 256, in 16 bits as before (394: bound by HBM and its
+// access in rows of 2 KB).
 #pragma once
+#include <type_traits>
 #include "common.h"
 
 namespace semipd {
@@ -64,8 +68,8 @@ template <int D> struct DecodeWalkLds {
 // Walks tokens [s_begin, s_end) of the sequence whose pool rows are idx_base[0 .. ).  An empty range is allowed (nothing
 // is accumulated, l_tot = 0).
 //   load_q(qf): fills the Q^T fragments (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
-//   mid():      called once before the Q fragments are fetched, after the loads of the first `early_tiles` (0, 1 or 2:
-//               K and V rows of tile 0, K rows of tile 1) were issued -- the fused kernel rotates q / k there and stores
+//   mid():      called once before the Q fragments are fetched, after the loads of the first `early_tiles` (0 or more: K and V
+//               rows of tile 0) were issued -- the fused kernel rotates q / k there and stores
 //               the new token's rows; a tile that holds the new token must not be asked for before that
 // Results: o_acc (unnormalised O^T, lane = head c16, d = dt*16 + q4*4 + r), the running maximum m_run (per lane = head)
 // and l_tot, the sum of the weights over the whole range (reduced over the four 16-lane groups).
@@ -91,9 +95,11 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
   const int64_t k_head_off = (int64_t)hk * D + q4 * 8;
   const int64_t v_head_off = (int64_t)hk * D;
 
+  // Loads of the loop are unconditional, of the last token's row behind the range: with one behind a branch the compiler's count of what is in
+  // flight is that of the path that has the least, and the wait for the V rows drained the K rows just asked for (and each V row
+  // its own exchange): a memory latency a tile.
   auto load_idx = [&](int ti) -> int32_t {  // lane l (< 32) owns the index of token l of tile ti
-    const int tok = s_begin + ti * 32 + (lane & 31);
-    return (ti < n_tiles && tok < s_end) ? idx_base[tok] : 0;
+    return idx_base[min(s_begin + ti * 32 + (lane & 31), s_end - 1)];
   };
   auto issue_k = [&](KRegs<D, Raw>& r, int32_t idx_reg) {
 #pragma unroll
@@ -105,32 +111,42 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
     }
   };
   Raw vreg[NV];  // V rows of the NEXT tile, in flight while the current tile is computed
-  auto issue_v = [&](int32_t idx_reg, int ti) {
-    const int base_tok = s_begin + ti * 32;
+  auto issue_v = [&](int32_t idx_reg) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int it = j * 64 + lane;
       const int tok = it / CPR, ch = it - tok * CPR;
       const int64_t row = (int64_t)__shfl(idx_reg, tok, 64) * vbuf_stride + v_head_off;
-      vreg[j] = KVT::zero();
-      if (base_tok + tok < s_end)  // rows past the end must be zero: 0 * garbage could be NaN
-        vreg[j] = KVT::load8(v_buf + row + ch * 8);
+      vreg[j] = KVT::load8(v_buf + row + ch * 8);
     }
   };
 
   FragD qf[KS];
 
-  // compute tile ti from K registers `r` and the V registers; as soon as the V registers are in
-  // LDS they are re-used for the loads of tile ti+1 (idx_v = its indices)
-  auto compute = [&](KRegs<D, Raw>& r, int ti, int32_t idx_v) {
+  // compute tile ti from the K registers `r` and the V registers; as soon as the V registers are in LDS they are
+  // re-used for the loads of tile ti+1 (idx = its indices), the K registers behind their products
+  auto compute = [&](KRegs<D, Raw>& r, int ti, int32_t idx) __attribute__((always_inline)) {
+    const int base_tok = s_begin + ti * 32;
     // ---- V rows -> LDS (row-major, this wave's private tile) ----
+    if (base_tok + 32 > s_end) {  // rows past the end must be zero: 0 * garbage could be NaN
+#pragma unroll
+      for (int j = 0; j < NV; ++j) {
+        uint32_t keep = base_tok + (j * 64 + lane) / CPR < s_end ? ~0u : 0u;
+        uint32_t* const w = reinterpret_cast<uint32_t*>(&vreg[j]);
+#pragma unroll
+        for (int u = 0; u < (int)(sizeof(Raw) / 4); ++u) w[u] &= keep;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       const int it = j * 64 + lane;
       const int tok = it / CPR, ch = it - tok * CPR;
       *reinterpret_cast<uint4*>(v_lds + tok * RS + ch * 16) = KVT::expand(vreg[j]);
     }
-    if (ti + 1 < n_tiles) issue_v(idx_v, ti + 1);
+    // (the stages in this order: mixed by the scheduler, old and new rows are held at once, 81 registers of them in scratch)
+    __builtin_amdgcn_sched_barrier(0);
+    issue_v(idx);
+    __builtin_amdgcn_sched_barrier(0);
     // ---- S^T = K Q^T ----
     f32x4 s_acc[2];
 #pragma unroll
@@ -143,15 +159,24 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
         s_acc[t] = Mfma16<T>::mma(kf, qf[ks], s_acc[t]);
       }
     }
+    __builtin_amdgcn_sched_barrier(0);
+    issue_k(r, idx);
+    __builtin_amdgcn_sched_barrier(0);
     // ---- online softmax: lane = head c16, tokens t*16 + q4*4 + r ----
-    const int base_tok = s_begin + ti * 32;
     float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) s_acc[t] *= sm_scale;
+    if (logit_cap > 0.f) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) s_acc[t][rr] = logit_cap * tanhf(s_acc[t][rr] / logit_cap);
+    }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
 #pragma unroll
       for (int rr = 0; rr < 4; ++rr) {
-        float s = s_acc[t][rr] * sm_scale;
-        if (logit_cap > 0.f) s = logit_cap * tanhf(s / logit_cap);
+        float s = s_acc[t][rr];
         s = (base_tok + t * 16 + q4 * 4 + rr < s_end) ? s : -INFINITY;
         s_acc[t][rr] = s;
         mx = fmaxf(mx, s);
@@ -195,32 +220,26 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
     }
   };
 
-  KRegs<D, Raw> ra, rb;
-  int32_t idx_cur = load_idx(0);
-  int32_t idx_next = load_idx(1);
-  const bool k1_early = early_tiles >= 2 && n_tiles > 1;
+  KRegs<D, Raw> kreg;
+  int32_t idx_cur = 0, idx_next = 0;
+  if (n_tiles > 0) {
+    idx_cur = load_idx(0);
+    idx_next = load_idx(1);
+  }
   if (early_tiles >= 1) {
-    issue_k(ra, idx_cur);
-    issue_v(idx_cur, 0);
-    if (k1_early) issue_k(rb, idx_next);
+    issue_v(idx_cur);
+    issue_k(kreg, idx_cur);
   }
   mid();
   load_q(qf);
   if (early_tiles < 1) {
-    issue_k(ra, idx_cur);
-    issue_v(idx_cur, 0);
+    issue_v(idx_cur);
+    issue_k(kreg, idx_cur);
   }
-  for (int ti = 0; ti < n_tiles; ti += 2) {
-    if (ti + 1 < n_tiles && !(ti == 0 && k1_early)) issue_k(rb, idx_next);
-    idx_cur = idx_next;            // indices of tile ti+1 (its V rows are issued inside compute)
+  for (int ti = 0; ti < n_tiles; ++ti) {
+    idx_cur = idx_next;
     idx_next = load_idx(ti + 2);
-    compute(ra, ti, idx_cur);
-    if (ti + 1 < n_tiles) {
-      if (ti + 2 < n_tiles) issue_k(ra, idx_next);
-      idx_cur = idx_next;
-      idx_next = load_idx(ti + 3);
-      compute(rb, ti + 1, idx_cur);
-    }
+    compute(kreg, ti, idx_cur);
   }
 
   l_tot = l_run + __shfl_xor(l_run, 16, 64);

@@ -1,0 +1,44 @@
+"""Paged decode attention of grouped heads on the matrix cores (csrc/decode_mfma_walk.h) against a softmax in 64 bits, at the edges of its tiles
+of 32 tokens and of its splits."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("rows", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("H,G,D", [(8, 2, 128), (12, 4, 64), (16, 1, 128), (32, 1, 64), (10, 5, 96)])
+@pytest.mark.parametrize("splits", [1, 3, 8])
+@pytest.mark.parametrize("cap", [0.0, 2.0])
+def test_decode_at_the_edges_of_tiles(rows, H, G, D, splits, cap):
+    """Requests of one token, around whole tiles, shorter than their splits, and none; rows that belong to no request hold no numbers, and
+    neither a tile's unused rows nor the row behind the last reach the result.  Weights are rounded to 16 bits once and so is the result:
+    1.5 units of half a unit in the last place, as for prompts."""
+    from semi_pd_amd import ops
+    lens = [1, 2, 31, 32, 33, 0, 64, 65, 97, 200, 7]
+    g = torch.Generator().manual_seed(H * D + splits)
+    total = sum(lens)
+    k, v = (torch.full((2 * total + 2, G, D), float("nan")) for _ in range(2))
+    slots = torch.randperm(2 * total + 1, generator=g)[:total] + 1
+    k[slots], v[slots] = torch.randn(total, G, D, generator=g), torch.randn(total, G, D, generator=g)
+    k, v, q = k.to(rows), v.to(rows), torch.randn(len(lens), H, D, generator=g).bfloat16()
+    starts = [0]
+    for n in lens:
+        starts.append(starts[-1] + n)
+    out = torch.full((len(lens), H, D), 7.0, dtype=torch.bfloat16, device=DEV)
+    parts = torch.empty(len(lens), H, splits, D + 1, device=DEV) if splits > 1 else None
+    scale = D ** -0.5
+    ops.decode_attention_fwd(q.to(DEV), k.to(DEV), v.to(DEV), out, torch.tensor(starts, dtype=torch.int32, device=DEV), slots.int().to(DEV), parts, splits,
+                             scale, cap)
+    got, want = out.cpu().double(), torch.zeros(len(lens), H, D, dtype=torch.float64)
+    for b, n in enumerate(lens):
+        at = slots[starts[b]: starts[b + 1]]
+        for h in range(H):
+            if n:
+                s = k[at, h // (H // G)].double() @ q[b, h].double() * scale
+                want[b, h] = torch.softmax(cap * torch.tanh(s / cap) if cap else s, 0) @ v[at, h // (H // G)].double()
+    some = [b for b, n in enumerate(lens) if n]
+    ulp = 2.0 ** -8
+    assert float((got[some] - want[some]).norm() / want[some].norm()) < 1.5 * ulp
+    torch.testing.assert_close(got[some], want[some], rtol=6 * ulp, atol=12 * ulp)
