@@ -609,6 +609,12 @@ static int launch_rope_strided(T* q, T* k, const float* cache, const int64_t* po
   return launch_status("rope_strided");
 }
 
+// rope_pairs.hip
+template <typename T, bool STORE, typename KV>
+void launch_rope_pairs(int threads, T* q, T* k, const T* v, KV* k_buf, KV* v_buf, const int64_t* loc, const float* cache, const int64_t* positions,
+                       int64_t num_tokens, int Hq, int Hk, int head, int vhead, int64_t q_stride, int64_t k_stride, int64_t v_stride,
+                       int64_t kbuf_stride, int64_t vbuf_stride, hipStream_t st);
+
 template <typename T, bool STORE, typename KV = T>
 static int launch_rope(T* q, T* k, const T* v, KV* k_buf, KV* v_buf, const int64_t* loc,
                        const float* cache, const int64_t* positions, int64_t num_tokens, int Hq,
@@ -628,6 +634,14 @@ static int launch_rope(T* q, T* k, const T* v, KV* k_buf, KV* v_buf, const int64
     // one lane per work item of a token, whole waves, at most 1024 (rope_vec_kernel walks what is left over)
     const int per_head = interleave ? rot_dim / V : (rot_dim / 2) / V;
     const int items = (Hq + Hk) * per_head + (STORE ? Hk * ((head - rot_dim) / V) + Hk * vhead / V : 0);
+    // batches of four tokens a CU and more (up to there a lane an item runs them all at once): two items a lane, where a workgroup is whole
+    // heads and has all items (rope_pairs.hip has both sides' times)
+    const int pair_threads = (items + 127) / 128 * 64;
+    if (!interleave && rot_dim == head && num_tokens >= 1024 && pair_threads <= 512 && pair_threads % per_head == 0) {
+      launch_rope_pairs<T, STORE, KV>(pair_threads, q, k, v, k_buf, v_buf, loc, cache, positions, num_tokens, Hq, Hk, head, vhead, q_stride, k_stride, v_stride,
+                                      kbuf_stride, vbuf_stride, st);
+      return launch_status("rope");
+    }
     block = dim3((unsigned)std::min(1024, std::max(64, (items + 63) / 64 * 64)));
     if (interleave)
       hipLaunchKernelGGL((rope_vec_kernel<T, true, STORE, KV>), grid, block, 0, st, q, k, v, k_buf, v_buf,
