@@ -615,7 +615,7 @@ __global__ void __launch_bounds__(256) delta_post_kernel(DeltaArgs a) {
 // 128 x 128: 1861 us + 317 of preparation).  In chunks with all products in fp32, a wave all rows of 16 columns: a chain of 216 products of
 // 32 cycles a chunk, one wave a SIMD at 4 requests: 385 us.  In pieces, two waves a column block with half the rows each: 345, two waves a
 // SIMD, each with 72 products of 16 cycles, 16 or 20 of 32, 450 vector instructions and 50 LDS reads of 1 KB a chunk, which cover each other
-// in part (10 k cycles a chunk against 7 k one behind the other).  Operands 69.
+// in part (10 k cycles a chunk against 7 k one behind the other).  Operands 60.
 // Elements of the operands of one (chunk, key head), counted in fp32: keys of more than 64: K, Q and K^T in three planes of bf16 each,
 // left-hand operands of 16 x 16 x 32 products in the order in which they are held, [tile][lane][8] (see rec_split8; tiles of K and Q: 16
 // tokens x 32 rows of S, of K^T: 16 rows x the tokens); else in fp32, of 16 x 16 x 16 products, [tile][lane][4], lane (r16, kq) element s =
