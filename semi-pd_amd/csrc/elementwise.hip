@@ -317,7 +317,7 @@ __global__ void rope_vec_kernel(T* __restrict__ q, T* __restrict__ k, const T* _
   if (STORE) dst = loc[t];
   // ONE pass over every kind of work item of the token -- q rotations, k rotations (+ pool), k pass-through (+ pool), v rows
   // (+ pool) -- with a block as wide as the item count (launch_rope): every lane issues its loads at once and the token
-  // costs one memory latency.  (Until round 5: three loops one after the other on 256 threads, i.e. up to five dependent
+  // costs one memory latency.  (Before: three loops one after the other on 256 threads, i.e. up to five dependent
   // load -> store rounds per token; 20 us alone / 34 us next to a decode instance for a 1.3 k-token Llama-3-8B batch.)
   const int n_rot = q_items + k_items;
   const int pass_vec = STORE ? (head - rot_dim) / V : 0;

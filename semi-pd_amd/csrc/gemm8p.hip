@@ -391,7 +391,7 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
 }
 
 // ---------------------------------------------------------------------------------------------------------------------
-// The same 256 x 256 x 64 tile on FOUR waves (round 6): one wave per SIMD, each with a 128 x 128 quarter of the tile --
+// The same 256 x 256 x 64 tile on FOUR waves: one wave per SIMD, each with a 128 x 128 quarter of the tile --
 // 8 x 8 accumulator tiles = 256 registers, which the compiler keeps in the accumulation half of the unified register file.
 // Why: the 8-wave form reads (128 + 64) rows x 128 B of fragments per wave and K step, 192 KB per CU, and its LDS-DMA writes
 // another 64 KB: 2048 cycles of the LDS's 128 B / cycle -- exactly the 2048 cycles the K step's MFMAs take.  The kernel is
