@@ -217,6 +217,14 @@ int semipd_decode_rope_attention_planes(void* out, float* attn_logits, const flo
                                         int64_t batch, int num_q_heads, int num_kv_heads, int head_size, int64_t o_stride,
                                         int64_t kbuf_stride, int64_t vbuf_stride, int waves, int zsplits, float sm_scale,
                                         float logit_cap, int dtype, int kv_dtype, void* stream);
+/* The same with fewer kv splits than waves (zsplits = 1): splits 1 .. waves, the ranges and with them the bits of the separate
+ * calls at num_kv_splits = splits (layers/attention/triton_ops/decode_attention.py:625-670); 0: a split per wave, as above. */
+int semipd_decode_rope_attention_planes_splits(void* out, float* attn_logits, const float* planes, int n_planes, int64_t plane_elems,
+                                               void* k_buf, void* v_buf, const int64_t* loc, const float* cos_sin_cache,
+                                               const int64_t* positions, const int32_t* kv_indptr, const int32_t* kv_indices,
+                                               int64_t batch, int num_q_heads, int num_kv_heads, int head_size, int64_t o_stride,
+                                               int64_t kbuf_stride, int64_t vbuf_stride, int waves, int zsplits, int splits,
+                                               float sm_scale, float logit_cap, int dtype, int kv_dtype, void* stream);
 
 
 /* ------------------------------------------------------------------ */

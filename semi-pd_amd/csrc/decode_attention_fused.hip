@@ -8,8 +8,9 @@
 // they compute, and the split partials (8.7 MB per layer at 32 requests x 8 splits) made a round trip through HBM.
 //
 // A WORKGROUP owns one (request, kv head); its NW waves are the kv splits (same ranges as decode_mfma_kernel at
-// num_kv_splits = NW, walked by the same code: decode_mfma_walk.h).  (Small batches: Z workgroups per pair, each merging
-// its NW splits into ONE stage-1 partial; decode_stage2_kernel then merges Z partials per head instead of NW * Z.)
+// num_kv_splits = `splits`, NW of them or fewer -- the last waves have none then --, walked by the same code:
+// decode_mfma_walk.h).  (Small batches: Z workgroups per pair, each merging its NW splits into ONE stage-1 partial;
+// decode_stage2_kernel then merges Z partials per head instead of NW * Z.)
 //   1. the lanes that rotate ask for their planes and cos / sin values, then every wave asks for its first tile of K / V
 //      rows and the K rows of the second (unless they hold the new token);
 //   2. the wave whose range ends with the new token sums the planes of k and v, rotates k and stores both pool rows
@@ -32,7 +33,7 @@ decode_rope_attn_kernel(T* __restrict__ out, float* __restrict__ attn_logits, co
                         const float* __restrict__ cache, const int64_t* __restrict__ positions,
                         const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices, int num_q_heads,
                         int num_kv_heads, int group, int64_t o_stride, int64_t kbuf_stride, int64_t vbuf_stride,
-                        float sm_scale, float logit_cap) {
+                        int splits, float sm_scale, float logit_cap) {
   constexpr int KS = D / 32, DT = D / 16, V = 8;
   constexpr int PART_STRIDE = D + 4;                       // floats per head of a wave's partial (16-byte aligned rows)
   constexpr int WAVE_LDS = DecodeWalkLds<D>::BYTES >= 16 * PART_STRIDE * 4 ? DecodeWalkLds<D>::BYTES : 16 * PART_STRIDE * 4;
@@ -47,21 +48,22 @@ decode_rope_attn_kernel(T* __restrict__ out, float* __restrict__ attn_logits, co
   const int hq0 = hk * group;
   const bool head_ok = c16 < group;
 
-  // gridDim.y = Z workgroups per (request, kv head): NW * Z kv splits in all, workgroup z owns splits z * NW .. + NW - 1.
+  // gridDim.y = Z workgroups per (request, kv head): `splits` kv splits in all (NW * Z; up to NW with Z = 1), workgroup z owns
+  // splits z * NW .. + NW - 1.
   // Z = 1: the merged result is the output.  Z > 1 (batches too small to fill the chip with one workgroup per pair): the
   // workgroup's merge is ONE partial of attn_logits[b, hq, z, :] for decode_stage2_kernel -- Z partials per head instead of
   // NW * Z, and still no separate RoPE launch.
   const int Z = gridDim.y, z = blockIdx.y;
   const int kv_start = kv_indptr[b];
   const int seq_len = kv_indptr[b + 1] - kv_start;
-  const int per_split = (seq_len + NW * Z - 1) / (NW * Z);
+  const int per_split = (seq_len + splits - 1) / splits;
   const int s_begin = per_split * (z * NW + wave);
   const int s_end = min(s_begin + per_split, seq_len);
   // The new token is the last one of the sequence.  The wave whose range ends with it rotates k, copies v and stores both
   // rows itself (its later loads of that row are ordered behind its own stores by a vmcnt(0)); the other waves rotate q
   // into LDS.  Nobody else reads the new rows, so the workgroup meets on the LDS writes only (a raw barrier: no wave
   // waits for its K / V rows in flight).  Tiles that cannot reach the new token are asked for before all that.
-  const int owner_g = seq_len > 0 ? (seq_len - 1) / per_split : NW * Z - 1;
+  const int owner_g = seq_len > 0 ? (seq_len - 1) / per_split : splits - 1;
   const int owner = owner_g / NW == z ? owner_g - z * NW : -1;     // -1: the new token belongs to another workgroup
   constexpr int half = D / 2, IPH = half / V;                 // items of 8 pairs per head
   // a wave that rotates asks for its planes first and for its tiles after the barrier: loads return in order, and behind
@@ -228,7 +230,7 @@ template <typename T, typename KV>
 static int launch_decode_rope_attn(void* out, float* attn_logits, int zsplits, const float* planes, int n_planes, int64_t plane_elems, void* k_buf, void* v_buf,
                                    const int64_t* loc, const float* cache, const int64_t* positions, const int32_t* kv_indptr,
                                    const int32_t* kv_indices, int64_t batch, int Hq, int Hkv, int D, int64_t o_stride,
-                                   int64_t kbuf_stride, int64_t vbuf_stride, int waves, float sm_scale, float logit_cap,
+                                   int64_t kbuf_stride, int64_t vbuf_stride, int waves, int splits, float sm_scale, float logit_cap,
                                    hipStream_t st) {
   const int group = Hq / Hkv;
   const int64_t row_elems = (int64_t)(Hq + 2 * Hkv) * D;
@@ -236,7 +238,7 @@ static int launch_decode_rope_attn(void* out, float* attn_logits, int zsplits, c
 #define DF(DD, NW)                                                                                                     \
   hipLaunchKernelGGL((decode_rope_attn_kernel<T, DD, KV, NW>), grid, block, 0, st, (T*)out, attn_logits, planes, n_planes, plane_elems, \
                      row_elems, (KV*)k_buf, (KV*)v_buf, loc, cache, positions, kv_indptr, kv_indices, Hq, Hkv, group,      \
-                     o_stride, kbuf_stride, vbuf_stride, sm_scale, logit_cap)
+                     o_stride, kbuf_stride, vbuf_stride, splits, sm_scale, logit_cap)
   if (D == 128 && waves == 8) DF(128, 8);
   else if (D == 128 && waves == 4) DF(128, 4);
   else if (D == 64 && waves == 8) DF(64, 8);
@@ -269,6 +271,17 @@ int semipd_decode_rope_attention_planes(void* out, float* attn_logits, const flo
                                         int64_t batch, int num_q_heads, int num_kv_heads, int head_size, int64_t o_stride,
                                         int64_t kbuf_stride, int64_t vbuf_stride, int waves, int zsplits, float sm_scale,
                                         float logit_cap, int dtype, int kv_dtype, void* stream) {
+  return semipd_decode_rope_attention_planes_splits(out, attn_logits, planes, n_planes, plane_elems, k_buf, v_buf, loc, cos_sin_cache, positions,
+                                                    kv_indptr, kv_indices, batch, num_q_heads, num_kv_heads, head_size, o_stride, kbuf_stride,
+                                                    vbuf_stride, waves, zsplits, 0, sm_scale, logit_cap, dtype, kv_dtype, stream);
+}
+
+int semipd_decode_rope_attention_planes_splits(void* out, float* attn_logits, const float* planes, int n_planes, int64_t plane_elems,
+                                               void* k_buf, void* v_buf, const int64_t* loc, const float* cos_sin_cache,
+                                               const int64_t* positions, const int32_t* kv_indptr, const int32_t* kv_indices,
+                                               int64_t batch, int num_q_heads, int num_kv_heads, int head_size, int64_t o_stride,
+                                               int64_t kbuf_stride, int64_t vbuf_stride, int waves, int zsplits, int splits,
+                                               float sm_scale, float logit_cap, int dtype, int kv_dtype, void* stream) {
   SEMIPD_CHECK_ARG(batch >= 0 && n_planes >= 1 && head_size > 0 && num_q_heads > 0 && num_kv_heads > 0, SEMIPD_EINVAL,
                    "decode_rope_attention_planes: bad sizes");
   if (batch == 0) return 0;
@@ -282,6 +295,9 @@ int semipd_decode_rope_attention_planes(void* out, float* attn_logits, const flo
   SEMIPD_CHECK_ARG(waves == 4 || waves == 8, SEMIPD_EINVAL, "decode_rope_attention_planes: waves (kv splits per workgroup) must be 4 or 8");
   SEMIPD_CHECK_ARG(zsplits >= 1 && zsplits <= 64 && (zsplits == 1 || attn_logits), SEMIPD_EINVAL,
                    "decode_rope_attention_planes: 1 .. 64 workgroups per (request, kv head); attn_logits scratch required above 1");
+  SEMIPD_CHECK_ARG(splits == 0 || (zsplits == 1 && splits >= 1 && splits <= waves), SEMIPD_EINVAL,
+                   "decode_rope_attention_planes: 1 .. waves kv splits of one workgroup per (request, kv head), 0: a split per wave");
+  if (splits == 0) splits = waves * zsplits;
   SEMIPD_CHECK_ARG(batch * num_kv_heads < (1ll << 31), SEMIPD_EINVAL, "decode_rope_attention_planes: grid too large");
   const int64_t row_elems = (int64_t)(num_q_heads + 2 * num_kv_heads) * head_size;
   SEMIPD_CHECK_ARG(o_stride % 8 == 0 && kbuf_stride % 16 == 0 && vbuf_stride % 16 == 0 && plane_elems % 4 == 0 &&
@@ -293,7 +309,7 @@ int semipd_decode_rope_attention_planes(void* out, float* attn_logits, const flo
 #define GO(TT, KVT)                                                                                                       \
   rc = launch_decode_rope_attn<TT, KVT>(out, attn_logits, zsplits, planes, n_planes, plane_elems, k_buf, v_buf, loc, cos_sin_cache, positions, \
                                           kv_indptr, kv_indices, batch, num_q_heads, num_kv_heads, head_size, o_stride,    \
-                                          kbuf_stride, vbuf_stride, waves, sm_scale, logit_cap, st)
+                                          kbuf_stride, vbuf_stride, waves, splits, sm_scale, logit_cap, st)
   SEMIPD_DISPATCH_HALF(dtype, T, {
     if (kv_dtype == dtype) GO(T, T);
     else if (kv_dtype == SEMIPD_F8E5M2) GO(T, f8e5m2_t);

@@ -428,11 +428,11 @@ class HipAttnBackend(AttentionBackend):
             return 4
         if 2 * wgs >= cus or knob == "2":
             return 8
-        # contexts of up to eight splits are the eight waves of one workgroup: one launch instead of three, on however few CUs.  Four layers
+        # up to eight splits are waves of one workgroup (fused_decode_splits): one launch instead of three, on however few CUs.  Four layers
         # + head, 333 tokens, us, three launches / one: 8 kv heads of 128, 1 request 475 / 455, 2 requests 478 / 457; of 64 261 / 237 and 269 / 243; 2 kv
         # heads of 128, hidden 8192, 1 request 532 / 525, 3 requests 551 / 536.  A single kv head is one CU a request: 60 tokens 370 / 372, 2
-        # requests 372 / 383, 500 tokens 403 / 408.
-        if knob != "4" and 1 <= num_kv_splits <= 8 and self.num_kv_head >= 2:
+        # requests 372 / 383, 500 tokens 403 / 408.  (The count of a captured graph is that of the context it is captured for.)
+        if self._splits_are_waves(bs, num_kv_splits) and knob != "4":
             return 8
         # several workgroups per pair: worth it from about one workgroup per eight CUs (Llama-3-8B from one request: step
         # alone 3.32 -> 3.25 ms, at 8 requests 3.65 -> 3.44; the 70B TP = 8 rank's single kv head at 1 .. 8 requests: 16 .. 32
@@ -449,6 +449,17 @@ class HipAttnBackend(AttentionBackend):
             return 1
         return max(1, min(64, (int(num_kv_splits) + 7) // 8))
 
+    def _splits_are_waves(self, bs: int, num_kv_splits: int) -> bool:
+        return 1 <= num_kv_splits <= 8 and self.num_kv_head >= 2 and 8 * bs * self.num_kv_head < max(1, self.num_cus)
+
+    def fused_decode_splits(self, bs: int, num_kv_splits: int) -> int:
+        """kv splits of the fused launch, 0 = one per wave.  Where it stands for the separate launches of a batch below one workgroup
+        per eight CUs it has their count, and with it their bits, however many waves that leaves without a range (8 kv heads of 128, 1
+        request of 333 tokens, four layers + head: three launches 462 us, this in five ranges 444, in eight 442)."""
+        if os.environ.get("SEMIPD_FUSED_DECODE_ATTN", "1") != "2" and self._splits_are_waves(bs, num_kv_splits):
+            return int(num_kv_splits)
+        return 0
+
     def forward_decode_rope_planes(self, positions, qkv_planes, rotary_emb, layer, forward_batch: ForwardBatch, waves: int):
         md = self.forward_metadata
         pool = forward_batch.token_to_kv_pool
@@ -461,7 +472,8 @@ class HipAttnBackend(AttentionBackend):
             positions, qkv_planes, layer.tp_q_head_num, layer.tp_k_head_num, layer.head_dim, rotary_emb.cos_sin_cache,
             pool.get_key_buffer(layer.layer_id), pool.get_value_buffer(layer.layer_id), forward_batch.out_cache_loc,
             md.kv_indptr, md.kv_indices, waves, layer.scaling, layer.logit_cap, zsplits=zsplits,
-            attn_logits=md.attn_logits if zsplits > 1 else None)
+            attn_logits=md.attn_logits if zsplits > 1 else None,
+            num_kv_splits=self.fused_decode_splits(qkv_planes.rows, md.num_kv_splits) if waves == 8 else 0)
         if kt:
             kt.stop("decode_attention", t0, *self._algo, n_kernels=2 if zsplits > 1 else 1)
         return o

@@ -728,11 +728,11 @@ def decode_rope_attention_planes(positions: torch.Tensor, qkv: SplitKPlanes, num
                                  head_size: int, cos_sin_cache: torch.Tensor, k_buffer: torch.Tensor, v_buffer: torch.Tensor,
                                  loc: torch.Tensor, kv_indptr: torch.Tensor, kv_indices: torch.Tensor, waves: int,
                                  sm_scale: float, logit_cap: float = 0.0, zsplits: int = 1,
-                                 attn_logits: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """rope_and_store_kv_planes + decode_attention_fwd (`waves` kv splits, both stages) in ONE launch: the qkv row is
+                                 attn_logits: Optional[torch.Tensor] = None, num_kv_splits: int = 0) -> torch.Tensor:
+    """rope_and_store_kv_planes + decode_attention_fwd (`waves` kv splits, or num_kv_splits of them, both stages) in ONE launch: the qkv row is
     still the K-slice planes of the decode GEMM; rotated k and v go to the pool rows `loc` (the last row of each request
     in kv_indices); returns the attention output [tokens, Hq * head] (semipd_decode_rope_attention_planes).  Same bits
-    as the separate calls.  zsplits > 1 (small batches): that many workgroups per (request, kv head), each writing one
+    as the separate calls (num_kv_splits: 0 = a split per wave, else 1 .. waves of them with zsplits = 1).  zsplits > 1 (small batches): that many workgroups per (request, kv head), each writing one
     merged partial to attn_logits fp32 [tokens, Hq, zsplits, head + 1]; stage 2 follows as a second launch."""
     if cos_sin_cache.dtype != torch.float32 or cos_sin_cache.shape[1] != head_size or not cos_sin_cache.is_contiguous():
         raise RuntimeError("decode_rope_attention_planes: contiguous fp32 cos / sin cache over the whole head expected")
@@ -759,11 +759,11 @@ def decode_rope_attention_planes(positions: torch.Tensor, qkv: SplitKPlanes, num
                                "[tokens, Hq, zsplits, head + 1] required when zsplits > 1")
     qkv.check_live("decode_rope_attention_planes")
     o = torch.empty((qkv.rows, num_q_heads * head_size), dtype=qkv.dtype, device=qkv.planes.device)
-    check(_lib.load().semipd_decode_rope_attention_planes(
+    check(_lib.load().semipd_decode_rope_attention_planes_splits(
         ptr(o), ptr(attn_logits) if zsplits > 1 else None, ptr(qkv.planes), qkv.ksplit, qkv.rows * qkv.n, ptr(k_buffer),
         ptr(v_buffer), ptr(loc), ptr(cos_sin_cache), ptr(positions), ptr(kv_indptr), ptr(kv_indices), qkv.rows,
         num_q_heads, num_kv_heads, head_size, o.stride(0), k_buffer.stride(0), v_buffer.stride(0), waves, int(zsplits),
-        sm_scale, logit_cap, dtype_code(qkv.dtype),
+        int(num_kv_splits), sm_scale, logit_cap, dtype_code(qkv.dtype),
         _lib.kv_dtype_code(k_buffer.dtype), current_stream(o.device)), "decode_rope_attention_planes")
     return o
 

@@ -42,3 +42,32 @@ def test_decode_at_the_edges_of_tiles(rows, H, G, D, splits, cap):
     ulp = 2.0 ** -8
     assert float((got[some] - want[some]).norm() / want[some].norm()) < 1.5 * ulp
     torch.testing.assert_close(got[some], want[some], rtol=6 * ulp, atol=12 * ulp)
+
+
+@pytest.mark.parametrize("H,G,D,K", [(32, 8, 128, 4096), (32, 8, 64, 2048), (12, 6, 64, 768)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 5, 7, 8])
+@pytest.mark.parametrize("rows", [torch.bfloat16, torch.float8_e4m3fn])
+def test_one_launch_with_fewer_splits_than_waves_has_the_bits_of_three(H, G, D, K, splits, rows):
+    """The one-launch form at the kv splits of the launches that it stands for: the same ranges of every request, so the same bits and the
+    same pool rows, also of requests with fewer tokens than ranges and on the edges of ranges and tiles."""
+    from semi_pd_amd import ops
+    lens = [1, 2, splits, 8 * splits + 1, 32 * splits, 333, 32 * splits + 1]
+    B, total = len(lens), sum(lens)
+    g = torch.Generator().manual_seed(H + D + splits)
+    ends = torch.cumsum(torch.tensor(lens), 0)
+    starts = torch.cat([torch.zeros(1, dtype=torch.int64), ends]).int().to(DEV)
+    slots = (torch.randperm(total + 9, generator=g)[:total] + 1).int()
+    k, v = (torch.randn(total + 10, G, D, generator=g).bfloat16().to(rows).to(DEV) for _ in range(2))
+    loc, slots = slots[ends - 1].long().to(DEV), slots.to(DEV)
+    x, w = torch.randn(B, K, generator=g).bfloat16().to(DEV), (torch.randn((H + 2 * G) * D, K, generator=g) * 0.03).bfloat16().to(DEV)
+    angles = torch.arange(1024.0)[:, None] * 10000.0 ** (-torch.arange(0, D, 2) / D)
+    table, pos = torch.cat([angles.cos(), angles.sin()], 1).to(DEV), (torch.tensor(lens) - 1).to(DEV)
+    k1, v1, k2, v2 = k.clone(), v.clone(), k.clone(), v.clone()
+    q = ops.rope_and_store_kv_planes(pos, ops.stream_linear_planes(x, w), H, G, D, table, k1, v1, loc)
+    want = torch.empty(B, H, D, dtype=torch.bfloat16, device=DEV)
+    parts = torch.empty(B, H, splits, D + 1, device=DEV) if splits > 1 else None
+    ops.decode_attention_fwd(q.view(B, H, D), k1, v1, want, starts, slots, parts, splits, D ** -0.5)
+    got = ops.decode_rope_attention_planes(pos, ops.stream_linear_planes(x, w), H, G, D, table, k2, v2, loc, starts, slots, 8, D ** -0.5,
+                                           num_kv_splits=splits)
+    assert torch.equal(k1.view(torch.uint8), k2.view(torch.uint8)) and torch.equal(v1.view(torch.uint8), v2.view(torch.uint8))
+    assert torch.equal(got.view(torch.int16), want.view(B, H * D).view(torch.int16))

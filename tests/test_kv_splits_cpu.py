@@ -95,3 +95,9 @@ def test_short_contexts_of_few_requests_take_one_launch(monkeypatch):
     assert [b.fused_decode_zsplits(1, s) for s in (1, 5, 8)] == [1, 1, 1]
     assert [backend(16, 2).fused_decode_waves(1, 128, s) for s in (8, 9)] == [8, 0]
     assert backend(8, 1).fused_decode_waves(1, 128, 5) == 0
+    # ... and has the ranges of the launches it stands for; from one workgroup per eight CUs up, where it always was the route, a range a wave
+    assert [b.fused_decode_splits(1, s) for s in (1, 5, 8, 9, 32)] == [1, 5, 8, 0, 0]
+    assert [b.fused_decode_splits(n, 5) for n in (3, 4, 16, 64)] == [5, 0, 0, 0]
+    assert backend(8, 1).fused_decode_splits(1, 5) == 0
+    monkeypatch.setenv("SEMIPD_FUSED_DECODE_ATTN", "2")
+    assert b.fused_decode_splits(1, 5) == 0
