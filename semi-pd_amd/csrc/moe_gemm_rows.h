@@ -250,6 +250,7 @@ moe_gemm_rows_kernel(T* __restrict__ out, const T* __restrict__ x, const T* __re
   // the CUs of an XCD, up to eight row tiles of the expert take turns within them (8 experts of 4096 x 28672, 4096 tokens, top 2: 1800 ->
   // 1640 us; with 11 column tiles, second tiles of 64 rows: 328 -> 382, their short tiles no longer come last).
   const int tiles_m = grp.num_post_pad[0] / RowsTile::kRows, lane = threadIdx.x & 63, at = blockIdx.x >> 3, xcd = blockIdx.x & 7;
+  if (tiles_m == 0) return;                                              // (no entry is one of these experts': none of expert_ids is written)
   int tile_m, tile_n, expert;
   bool alone;                                                            // no other row tile reads this one's weight rows
   if (tiles_n > 16 || tiles_m > 256) {

@@ -53,3 +53,29 @@ def test_rows_of_every_body(counts, K, n_out, div, dtype):
     out = torch.full((total, n_out), 77.0, dtype=dtype, device=DEV)
     ops.moe_gemm_tall(d(a), d(w), out, None, d(ids), d(experts), npp, total, div, False, True, block_m=BM)
     assert torch.equal(out, ops.silu_and_mul(plain))
+
+
+@pytest.mark.parametrize("n_out", [304, 2320])                                                          # few and many column tiles
+def test_no_entry_is_one_of_the_experts(n_out):
+    """A rank whose experts no token takes: nothing is written, and in front of the blocks there are nothing is read either (expert_ids is the
+    start of its allocation)."""
+    E, K, total = 4, 128, 700
+    ids = torch.full((2 * BM,), total, dtype=torch.int32, device=DEV)
+    experts, none = torch.full((2,), 1 << 30, dtype=torch.int32, device=DEV), torch.zeros(1, dtype=torch.int32, device=DEV)
+    a, w = torch.ones(total, K, dtype=torch.bfloat16, device=DEV), torch.ones(E, 2 * n_out, K, dtype=torch.bfloat16, device=DEV)
+    for fused in (False, True):
+        out = torch.full((total, n_out if fused else 2 * n_out), 77.0, dtype=torch.bfloat16, device=DEV)
+        ops.moe_gemm_tall(a, w, out, None, ids, experts, none, total, 1, False, fused, block_m=BM)
+        assert bool((out == 77).all())
+
+
+def test_layer_of_a_rank_that_no_token_routes_to():
+    """The layer of such a rank is zero, in the blocks of up to 320 rows as in the others."""
+    from semi_pd_amd.layers import moe
+    E, K, F, T, top = 16, 512, 1024, 900, 6
+    assert moe._tall_block(256, T, top, E, K, F) == BM
+    x = torch.randn(T, K, device=DEV).bfloat16()
+    w1, w2 = torch.randn(E, 2 * F, K, device=DEV).bfloat16(), torch.randn(E, K, F, device=DEV).bfloat16()
+    ids = torch.arange(T * top, device=DEV, dtype=torch.int32).view(T, top) % 16                          # of the first rank's experts
+    out = moe.fused_experts(x, w1, w2, torch.rand(T, top, device=DEV), ids, expert_offset=48, partial_experts=True)
+    assert bool((out == 0).all())
