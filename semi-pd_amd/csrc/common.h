@@ -33,9 +33,6 @@ void set_error(const char* fmt, ...);
     }                                                                           \
   } while (0)
 
-// Opt a kernel in to more than 64 KB of dynamic LDS, once per DEVICE and call site (`done` = one bit per device: the
-// attribute is per device, a second GPU in the process would otherwise fail at launch).  Returns non-zero and sets
-// the error text when the runtime refuses.
 // Compute units this process may use (its HSA_CU_MASK share), as told through semipd_stream_linear_set_cus /
 // semipd_gemm_tall_set_cus by the model runner; 0 = never told (whole device assumed by the kernels that ask).
 inline std::atomic<int>& owned_cus() {
@@ -43,6 +40,15 @@ inline std::atomic<int>& owned_cus() {
   return v;
 }
 
+// ... as a launch counts on them that wants a CU for every one of its workgroups
+inline int64_t launch_cus() {
+  const int own = owned_cus().load(std::memory_order_relaxed);
+  return own > 0 ? own : 256;
+}
+
+// Opt a kernel in to more than 64 KB of dynamic LDS, once per DEVICE and call site (`done` = one bit per device: the
+// attribute is per device, a second GPU in the process would otherwise fail at launch).  Returns non-zero and sets
+// the error text when the runtime refuses.
 inline int ensure_dynamic_lds(const void* kernel, size_t bytes, std::atomic<uint64_t>& done, const char* what) {
   int dev = 0;
   (void)hipGetDevice(&dev);

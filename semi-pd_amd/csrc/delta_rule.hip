@@ -1647,9 +1647,9 @@ static void launch_delta_chunks(const DeltaArgs& a, hipStream_t s) {
   const int64_t members = (int64_t)(a.H / a.G) * ((a.E + 63) / 64);
   const dim3 grid(rec_walk_blocks(a.batch * a.G, members));
   if constexpr (NP > kDeltaSmall) {
-    // 32 columns a workgroup as long as every one of them has a CU (rec_walk_blocks: of the XCD with the most)
+    // 32 columns a workgroup as long as every one of them has a CU of the launch's share (rec_walk_blocks: of the XCD with the most)
     const unsigned narrow = rec_walk_blocks(a.batch * a.G, (int64_t)(a.H / a.G) * ((a.E + 31) / 32));
-    if (narrow <= 256) hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 2>), dim3(narrow), dim3(512), 0, s, a, chunks);
+    if (narrow <= launch_cus()) hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 2>), dim3(narrow), dim3(512), 0, s, a, chunks);
     else hipLaunchKernelGGL((delta_chunk_walk_kernel<T, NP, 4>), grid, dim3(512), 0, s, a, chunks);
   } else if (a.batch * a.G * members > 256) {
     // more workgroups than CUs: two a CU, at the price of 40 spilled registers (32 heads of 64 x 64, one / two a CU, whole call: 64 requests

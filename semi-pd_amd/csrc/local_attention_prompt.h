@@ -542,7 +542,7 @@ __global__ void __launch_bounds__(64 * NW * KS, 2) prompt_attention_kernel(Local
 // types, everything aligned as local_attention_mfma_kernel wants it.
 struct PromptPlan {
   int hw;
-  int64_t avg, n_tiles, blocks;
+  int64_t avg, n_tiles, blocks, expected;          // expected: workgroups that find a tile where half of the requests end in one of few rows
   PromptShare share;
 };
 static PromptPlan prompt_plan(const LocalAttnArgs& a, int NW) {
@@ -558,8 +558,9 @@ static PromptPlan prompt_plan(const LocalAttnArgs& a, int NW) {
   if (count(wide) < count(hw)) hw = wide;
   const int rows = 32 * (NW / hw);
   const int64_t n_tiles = (a.num_tokens + rows - 1) / rows + a.batch;
-  const PromptShare share = prompt_share(a.G, (uint32_t)n_tiles);
-  return PromptPlan{hw, avg, n_tiles, 8ll * share.heads * share.tiles * ((rep + hw - 1) / hw), share};
+  const PromptShare share = prompt_share(a.G, (uint32_t)n_tiles), likely = prompt_share(a.G, (uint32_t)(n_tiles - a.batch + (a.batch - 1) / 2));
+  const int64_t sets = 8ll * share.heads * ((rep + hw - 1) / hw);
+  return PromptPlan{hw, avg, n_tiles, share.tiles * sets, likely.tiles * sets, share};
 }
 template <typename T, int D, int E, int NW, int KT, int KS, bool SIG>
 static int launch_prompt_attention(LocalAttnArgs a, const PromptPlan& plan, hipStream_t s) {
@@ -604,18 +605,23 @@ static int launch_prompt_attention(LocalAttnArgs a, const PromptPlan& plan, hipS
 // the longer one, one behind the other (the longest first) as their mean.  One / two groups: 32 / 8 heads of 128, 1 prompt of 1500 tokens 50.1 / 42.6, 2 of
 // 1000 38.4 / 36.4 (24 / 8 heads 48.5 / 39.9, 37.1 / 31.7; of 64 34.1 / 28.0, 26.6 / 24.5), values of 256, 1 of 1500 107 / 91; but windows of 1000, 1 of 2000 49.8
 // / 60.6, 4 of 300 19.6 / 23.8, values of 128 and keys of 64, 2 of 1086 46.8 / 48.6; beyond, 1 of 3000 103 / 111.
+// On a share of the CUs the same by the share's, and by the tiles that are likely there.  One group / the former rule, which counted on 256 / this, on 224
+// CUs: 32 / 8 heads of 128, 2 prompts of 1000 36.3 / 39.2 / 36.2, 4 of 100 behind 800 35.3 / 23.4 / 23.5; on 192, 2 of 1000 36.3 / 43.8 / 36.2, 24 / 8 heads 35.4 / 39.6 /
+// 35.4; on 128, 1 of 300 14.6 / 18.7 / 14.7, 1 of 1500 57.3 / 71.7 / 57.3.  Two tiles a CU, one / two groups, of one request: on 192 CUs 1 of 1500 47.9 / 46.7, on 128
+// 1 of 933 32.9 / 35.6; of two: on 224 2 of 1000 (24 / 8 heads) 36.4 / 35.0, on 160 2 of 600 26.1 / 28.9.
 template <typename T, int D, int E, bool SIG>
 static int split_prompt_attention(const LocalAttnArgs& a, hipStream_t s) {
   constexpr int NW = E > 128 ? 8 : 4, KT = E > 128 ? 32 : 64;
-  const int64_t bound = a.window > 0 ? a.window : a.chunk;
+  const int64_t bound = a.window > 0 ? a.window : a.chunk, cus = std::min<int64_t>(launch_cus(), 256);
+  const auto fits = [&](const PromptPlan& p) { return p.blocks <= 256 && p.expected <= cus; };
   if (bound == 0 || bound >= 512) {
     if constexpr (E <= 128) {
       const PromptPlan few = prompt_plan(a, 2);
-      if (few.blocks <= 256) return launch_prompt_attention<T, D, E, 2, (D + E > 128 ? 32 : 64), 4, SIG>(a, few, s);
+      if (fits(few)) return launch_prompt_attention<T, D, E, 2, (D + E > 128 ? 32 : 64), 4, SIG>(a, few, s);
     }
     const PromptPlan few = prompt_plan(a, 4);
-    const bool uneven = (a.batch == 1 || (a.batch == 2 && E == D)) && (a.window == 0 || a.window >= few.avg);
-    if (few.blocks <= (uneven ? 512 : 256)) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
+    const bool uneven = (a.batch == 1 ? cus >= 160 : a.batch == 2 && E == D && cus >= 224) && (a.window == 0 || a.window >= few.avg);
+    if (fits(few) || (uneven && few.blocks <= 2 * cus)) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
   }
   return launch_prompt_attention<T, D, E, NW, KT, 1, SIG>(a, prompt_plan(a, NW), s);
 }

@@ -1391,9 +1391,10 @@ static void launch_ssm_chunks(const SsmArgs& a, hipStream_t s) {
     }
   hipLaunchKernelGGL((ssm_chunk_operands_kernel<T, NP, true>), operands, dim3(256), 0, s, a);
   if constexpr (NP > 64) {
-    // 32 columns a workgroup as long as every one of them has a CU (rec_walk_blocks: of the XCD with the most)
+    // 32 columns a workgroup as long as every one of them has a CU of the launch's share (rec_walk_blocks: of the XCD with the most)
+    // (128 heads of 128 x 64 over 8, 1 request of 1000 rows, 256 workgroups of 32: 105 us on 256 CUs; on 224 178, with 64 columns 138)
     const unsigned narrow = rec_walk_blocks(a.batch * a.G, (int64_t)(a.H / a.G) * ((a.E + 31) / 32));
-    if (narrow <= 256) {
+    if (narrow <= launch_cus()) {
       hipLaunchKernelGGL((ssm_chunk_walk_kernel<T, NP, 2>), dim3(narrow), dim3(512), 0, s, a, chunks);
       return;
     }
