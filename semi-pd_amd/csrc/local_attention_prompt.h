@@ -604,7 +604,8 @@ static int launch_prompt_attention(LocalAttnArgs a, const PromptPlan& plan, hipS
 // Up to two tiles a CU where they differ most, in one or two requests whose rows see all in front of them: two tiles at once take as long as
 // the longer one, one behind the other (the longest first) as their mean.  One / two groups: 32 / 8 heads of 128, 1 prompt of 1500 tokens 50.1 / 42.6, 2 of
 // 1000 38.4 / 36.4 (24 / 8 heads 48.5 / 39.9, 37.1 / 31.7; of 64 34.1 / 28.0, 26.6 / 24.5), values of 256, 1 of 1500 107 / 91; but windows of 1000, 1 of 2000 49.8
-// / 60.6, 4 of 300 19.6 / 23.8, values of 128 and keys of 64, 2 of 1086 46.8 / 48.6; beyond, 1 of 3000 103 / 111.
+// / 60.6, 4 of 300 19.6 / 23.8, values of 128 and keys of 64, 2 of 1086 46.8 / 48.6; beyond, 1 of 3000 103 / 111.  Short tiles have more start and end than
+// that gives back where they are many: 40 / 8 heads of 128, 2 of 600 (440 tiles) 26.3 / 27.9, 32 / 8, 2 of 600 (288) 24.3 / 21.2.
 // On a share of the CUs the same by the share's, and by the tiles that are likely there.  One group / the former rule, which counted on 256 / this, on 224
 // CUs: 32 / 8 heads of 128, 2 prompts of 1000 36.3 / 39.2 / 36.2, 4 of 100 behind 800 35.3 / 23.4 / 23.5; on 192, 2 of 1000 36.3 / 43.8 / 36.2, 24 / 8 heads 35.4 / 39.6 /
 // 35.4; on 128, 1 of 300 14.6 / 18.7 / 14.7, 1 of 1500 57.3 / 71.7 / 57.3.  Two tiles a CU, one / two groups, of one request: on 192 CUs 1 of 1500 47.9 / 46.7, on 128
@@ -621,7 +622,7 @@ static int split_prompt_attention(const LocalAttnArgs& a, hipStream_t s) {
     }
     const PromptPlan few = prompt_plan(a, 4);
     const bool uneven = (a.batch == 1 ? cus >= 160 : a.batch == 2 && E == D && cus >= 224) && (a.window == 0 || a.window >= few.avg);
-    if (fits(few) || (uneven && few.blocks <= 2 * cus)) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
+    if (fits(few) || (uneven && few.blocks <= 2 * cus && (few.blocks <= 384 || few.avg >= 800))) return launch_prompt_attention<T, D, E, 4, KT, 2, SIG>(a, few, s);
   }
   return launch_prompt_attention<T, D, E, NW, KT, 1, SIG>(a, prompt_plan(a, NW), s);
 }

@@ -58,3 +58,20 @@ def test_groups_of_waves_follow_the_share(D, tokens, share):
     with _share(share):
         assert torch.equal(run(1), many)
     assert not torch.equal(run(1), many)
+
+
+def test_many_short_tiles_have_one_group_each():
+    """Two prompts of 600 tokens, 40 / 8 heads: 440 tiles, whose rows have the bits that they have in a batch whose tiles are one group's."""
+    from semi_pd_amd import ops
+    H, G, D, lens = 40, 8, 128, [600, 600, 600, 700]
+    t, _ = _batch(lens, [0] * 4, H, G, D, D, torch.bfloat16, D)
+    d = {k: v.to(DEV) for k, v in t.items() if k != "totals"}
+
+    def run(n):
+        start = torch.tensor([0] + lens[:-1], dtype=torch.int32).cumsum(0).int()[:n]
+        out = torch.empty(sum(lens[:n]), H * D, dtype=torch.bfloat16, device=DEV)
+        ops.local_attention_fwd(d["q"][: sum(lens[:n])], out, d["k"], d["v"], d["table"], torch.arange(n, device=DEV),
+                                torch.tensor(t["totals"][:n], device=DEV), start.to(DEV), torch.tensor(lens[:n], dtype=torch.int32, device=DEV),
+                                max(lens[:n]), D ** -0.5, 0.0, 0, None, None)
+        return out[: 2 * 600]
+    assert torch.equal(run(2), run(4))
