@@ -1966,12 +1966,17 @@ extern "C" int semipd_talk_mix(const void* parts, int64_t parts_ld, const float*
   const bool tiles = (num_q_heads >= 6 * num_kv_heads && v_dim >= 64) || staged > 65536;
   const bool matrix = (dtype == SEMIPD_BF16 || dtype == SEMIPD_F16) && v_dim % 16 == 0 && parts_ld % 8 == 0 && out_ld % 8 == 0 && aligned16(parts) &&
                       aligned16(out) && num_q_heads <= 64;
-  // Value rows of whole 64 elements and at least 8 heads: 16-byte stores, several tokens a workgroup where they are more than the chip takes at
+  // Value rows of whole 64 elements: 16-byte stores, several tokens a workgroup where they are more than the chip takes at
   // once.  Against the vector form, 32 / 7262 tokens, us: 8 heads over 2 of 128 3.4 / 24 and 3.1 / 21, 16 over 8 of 64 4.6 / 51 and 3.7 / 36, 8 over 1
-  // of 64 2.9 / 12.9 both; 6 over 3 of 64 2.9 / 12.5 and 3.0 / 19, 4 over 4 of 128 2.8 / 14 and 3.6 / 33.
+  // of 64 2.9 / 12.9 both; 6 over 3 of 64 2.9 / 12.5 and 3.0 / 19, 4 over 4 of 128 2.8 / 14 and 3.6 / 33.  A product has a column a head of one key/value
+  // head, of 16, and the vector form work by the square of the heads: few heads over many stay with that one where it stages its operands (vector /
+  // this, 7000 tokens, whole call: 8 over 8 of 64 18.6 / 29.0, of 192 58 / 87, 8 over 4 of 128 24.5 / 29.5, 10 over 10 of 128 65 / 76, 8 over 2 of 64 13.2 / 14.5, 10 over
+  // 5 of 64 20.8 / 22.1; but of 192 60 / 54, 10 over 2 of 64 17.5 / 15.0, 12 over 6 of 64 26.5 / 25.2, 14 over 14 of 64 66 / 60).
+  const int per_product = num_q_heads * num_q_heads / num_kv_heads;
+  const bool columns = num_q_heads >= 14 || staged > 65536 || per_product >= (v_dim == 64 && num_q_heads < 12 ? 40 : 20);
   const int kt = (num_q_heads + 15) / 16;
   const size_t rows = (size_t)num_q_heads * ((size_t)num_kv_heads * v_dim * 2 + 32) + (size_t)num_q_heads * (16 * kt + 4) * 4;
-  if (matrix && v_dim % 64 == 0 && num_q_heads >= 8 && rows <= 65536) {
+  if (matrix && columns && v_dim % 64 == 0 && num_q_heads >= 8 && rows <= 65536) {
     const int64_t at_once = 256 * (int64_t)(rows <= 20480 ? 8 : 163840 / rows), turns = (num_tokens + at_once - 1) / at_once;
     const dim3 grid((unsigned)((num_tokens + turns - 1) / turns));
 #define TALK_ROWS(KT)                                                                                                                              \

@@ -242,6 +242,21 @@ def test_talk_mix_of_many_tokens(dtype, H, G, E, tokens):
         assert bool(((few == same) | (torch.isnan(few) & torch.isnan(same))).all())
 
 
+# few heads over many key/value heads, which do not fill a product's columns, on both sides of that line and of what the vector form stages
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,G,E", [(8, 8, 64), (8, 4, 128), (8, 2, 64), (8, 2, 128), (10, 10, 128), (10, 10, 192), (12, 12, 64), (14, 14, 64)])
+def test_talk_mix_of_few_heads_over_many(dtype, H, G, E):
+    from semi_pd_amd import ops
+    g = torch.Generator().manual_seed(H + G)
+    parts, talk = torch.randn(300, H, G, E, generator=g).to(dtype), torch.randn(H, H, generator=g)
+    out = ops.talk_mix(parts.view(300, -1).to(DEV), talk.to(DEV), G).cpu().double()
+    mine = parts.double()[:, :, torch.arange(H) // (H // G)]                                              # [token, weights of head, head, E]
+    want = torch.einsum("hg,tghe->the", talk.double(), mine).reshape(300, -1)
+    terms = torch.einsum("hg,tghe->the", talk.double().abs(), mine.abs()).reshape(300, -1)
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    assert bool(((out - want).abs() <= half * want.abs() + 64 * 2.0 ** -24 * terms + 1e-7).all())
+
+
 # (launches large enough that tiles go by their keys: blocks of 18 tiles, one row past a tile's edge in front; of 70, two of which are a level;
 # requests without blocks, so many keys that three tiles are a level)
 @pytest.mark.parametrize("block,lens,olds", [(576, [700, 0, 33, 400, 1], [545, 7, 5, 0, 576]), (2240, [500, 1, 600], [2000, 64, 3]), (2240, [1100], [1999]),
