@@ -161,7 +161,7 @@ decode_rope_attn_kernel(T* __restrict__ out, float* __restrict__ attn_logits, co
   f32x4 o_acc[DT];
   float m_run, l_tot;
   rotation_loads();
-  decode_mfma_walk<T, D, KV>(
+  decode_mfma_walk<T, D, KV, false>(
       wave_lds[wave], k_buf, v_buf, kv_indices + kv_start, s_begin, s_end, hk, kbuf_stride, vbuf_stride, sm_scale,
       logit_cap, early_tiles,
       [&](FragD (&qf)[KS]) {

@@ -7,7 +7,7 @@
 
 namespace semipd {
 
-template <typename T, int D, typename KV>
+template <typename T, int D, typename KV, bool PAUSE>
 __global__ void __launch_bounds__(256, D <= 128 ? 2 : 1)   // D = 256 needs > 256 registers: one workgroup per SIMD set instead of 672 B of scratch
 decode_mfma_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __restrict__ k_buf,
                    const KV* __restrict__ v_buf, const int32_t* __restrict__ kv_indptr,
@@ -50,7 +50,7 @@ decode_mfma_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __res
 
   f32x4 o_acc[DT];
   float m_run, l_tot;
-  decode_mfma_walk<T, D, KV>(
+  decode_mfma_walk<T, D, KV, PAUSE>(
       v_lds_all[wave], k_buf, v_buf, kv_indices + kv_start, s_begin, s_end, hk, kbuf_stride, vbuf_stride, sm_scale,
       logit_cap, 2,
       [&](FragD (&qf)[KS]) {
@@ -97,15 +97,27 @@ int launch_decode_mfma(T* out, const T* q, const KV* k_buf, const KV* v_buf, con
   const int tiles = (group + 15) / 16;
   const int64_t total = batch * Hkv * tiles * splits;
   dim3 grid((unsigned)((total + 3) / 4)), block(256);
-#define DM(DD)                                                                                      \
-  hipLaunchKernelGGL((decode_mfma_kernel<T, DD, KV>), grid, block, 0, st, out, q, k_buf, v_buf, kv_indptr, \
+  // Between one and 1.75 workgroups a CU, heads of up to 96 in 16 bits: the walk that pauses.  8 kv heads of 64, rows of 2500 tokens, us, on / pausing (and
+  // before the walk went on): 128 requests (256 workgroups) 112.8 / 112.7 (118.8), 129 137 / 168 (176), 140 196 / 186 (188), 150 202 / 192 (194), 200 218 / 214 (216), 250 247 / 245
+  // (247), 300 325 / 328 (335), 400 374 / 422 (422); of 96, 150 324 / 309 (319).  Heads of 128 differ by less than their runs; rows of 8 bits are faster by a quarter without.
+  const int64_t cus = launch_cus();
+  const bool pause = grid.x >= cus + cus / 64 && 4ll * grid.x <= 7 * cus;
+#define DM(DD, PAUSE)                                                                               \
+  hipLaunchKernelGGL((decode_mfma_kernel<T, DD, KV, PAUSE>), grid, block, 0, st, out, q, k_buf, v_buf, kv_indptr, \
                      kv_indices, attn_logits, Hq, Hkv, group, tiles, q_stride, o_stride, kbuf_stride,  \
                      vbuf_stride, splits, total, sm_scale, logit_cap)
+  if constexpr (sizeof(KV) == 2) {
+    if (pause && (D == 64 || D == 96)) {
+      if (D == 64) DM(64, true);
+      else DM(96, true);
+      return launch_status("decode_mfma");
+    }
+  }
   switch (D) {
-    case 64: DM(64); break;
-    case 96: DM(96); break;
-    case 128: DM(128); break;
-    case 256: DM(256); break;
+    case 64: DM(64, false); break;
+    case 96: DM(96, false); break;
+    case 128: DM(128, false); break;
+    case 256: DM(256, false); break;
     default: set_error("decode_mfma: head dim %d not instantiated", D); return SEMIPD_ESHAPE;
   }
 #undef DM

@@ -71,9 +71,12 @@ template <int D> struct DecodeWalkLds {
 //   mid():      called once before the Q fragments are fetched, after the loads of the first `early_tiles` (0 or more: K and V
 //               rows of tile 0) were issued -- the fused kernel rotates q / k there and stores
 //               the new token's rows; a tile that holds the new token must not be asked for before that
+//   PAUSE:      the loads of the next tile behind a branch on there being one: with that each of their waits drains what was asked for in
+//               front of it, which is slower by itself and faster where the launch leaves some CUs with twice the waves of the others
+//               (see launch_decode_mfma's rule)
 // Results: o_acc (unnormalised O^T, lane = head c16, d = dt*16 + q4*4 + r), the running maximum m_run (per lane = head)
 // and l_tot, the sum of the weights over the whole range (reduced over the four 16-lane groups).
-template <typename T, int D, typename KV, typename QLoad, typename Mid>
+template <typename T, int D, typename KV, bool PAUSE, typename QLoad, typename Mid>
 __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __restrict__ k_buf, const KV* __restrict__ v_buf,
                                                  const int32_t* __restrict__ idx_base, int s_begin, int s_end, int hk,
                                                  int64_t kbuf_stride, int64_t vbuf_stride, float sm_scale, float logit_cap,
@@ -145,7 +148,7 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
     }
     // (the stages in this order: mixed by the scheduler, old and new rows are held at once, 81 registers of them in scratch)
     __builtin_amdgcn_sched_barrier(0);
-    issue_v(idx);
+    if (!PAUSE || ti + 1 < n_tiles) issue_v(idx);
     __builtin_amdgcn_sched_barrier(0);
     // ---- S^T = K Q^T ----
     f32x4 s_acc[2];
@@ -160,7 +163,7 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
       }
     }
     __builtin_amdgcn_sched_barrier(0);
-    issue_k(r, idx);
+    if (!PAUSE || ti + 1 < n_tiles) issue_k(r, idx);
     __builtin_amdgcn_sched_barrier(0);
     // ---- online softmax: lane = head c16, tokens t*16 + q4*4 + r ----
     float mx = -INFINITY;

@@ -71,3 +71,23 @@ def test_one_launch_with_fewer_splits_than_waves_has_the_bits_of_three(H, G, D, 
                                            num_kv_splits=splits)
     assert torch.equal(k1.view(torch.uint8), k2.view(torch.uint8)) and torch.equal(v1.view(torch.uint8), v2.view(torch.uint8))
     assert torch.equal(got.view(torch.int16), want.view(B, H * D).view(torch.int16))
+
+
+@pytest.mark.parametrize("H,G,D,B", [(32, 8, 64, 150), (48, 8, 96, 131), (16, 4, 64, 280)])
+def test_walk_that_pauses_has_the_bits_of_the_one_that_goes_on(H, G, D, B):
+    """Between one and two workgroups a CU heads of up to 96 take the other walk: the same bits as in two calls of half the requests."""
+    from semi_pd_amd import ops
+    lens = [1 + (i * 37) % 131 for i in range(B)]
+    g = torch.Generator().manual_seed(D + B)
+    ends = torch.cumsum(torch.tensor(lens), 0)
+    starts = torch.cat([torch.zeros(1, dtype=torch.int64), ends]).int()
+    total = int(ends[-1])
+    slots = (torch.randperm(total + 9, generator=g)[:total] + 1).int().to(DEV)
+    k, v = (torch.randn(total + 10, G, D, generator=g).bfloat16().to(DEV) for _ in range(2))
+    q = torch.randn(B, H, D, generator=g).bfloat16().to(DEV)
+
+    def run(lo, hi):
+        out = torch.empty(hi - lo, H, D, dtype=torch.bfloat16, device=DEV)
+        ops.decode_attention_fwd(q[lo:hi], k, v, out, starts[lo: hi + 1].to(DEV), slots, None, 1, D ** -0.5)
+        return out
+    assert torch.equal(run(0, B).view(torch.int16), torch.cat([run(0, B // 2), run(B // 2, B)]).view(torch.int16))
