@@ -7,6 +7,8 @@ weights w13 [E, 2N, K] and w2 [E, K, N], TP all-reduce :637-638).
 """
 from __future__ import annotations
 
+import functools
+import math
 import os
 
 from typing import Optional
@@ -81,15 +83,46 @@ MOE_STREAM_MAX_TOKENS = int(os.environ.get("SEMIPD_MOE_STREAM_MAX_TOKENS", "320"
 
 def _tall_block(block_m: int, tokens: int, topk: int, E: int, K: int, F: int) -> int:
     """Rows per block of a call that the tiled kernels take in blocks of `block_m`: 320, where the kernel whose tiles are as tall as
-    their expert needs takes both products (K and F in pairs of 64, 32-bit offsets into the operands) and is ahead.  Whole layer, both
+    their expert needs takes both products (K and F in pairs of 64, 32-bit offsets into the operands) and is ahead.  Both
     products, blocks of 128 or 256 / of 320, us: 64 experts of 2048 x 1408, top 6, 400 tokens 255 / 232, 1000 273 / 248, 2000 322 / 285,
     3001 474 / 335, 6000 739 / 599, 8192 903 / 817; 8 of 4096 x 14336, top 2, 512 tokens 795 / 611, 4096 2550 / 2450; 16 of 2048 x 1408, top 2, 1024
     tokens 86 / 84, 4096 203 / 183.  Behind with few K steps, whose loads ahead are not covered (256 experts of 7168 x 256, 1024 tokens
-    554 / 630: its second product has four), and where its tiles are too few for the chip."""
+    554 / 630: its second product has four), and where its tiles are too few for the chip.  The rows of an expert are counted as if all
+    `tokens` went to these experts, which those of an expert-parallel rank do not: blocks may be taller than it needs there."""
     numel = tokens * topk
     wide = (ops.MOE_TALL_BLOCK_M == 256 and K % 128 == 0 and F % 128 == 0 and min(K, F) >= 512 and 2 * F * K < 1 << 30
             and tokens * K < 1 << 30 and numel * F < 1 << 30 and max(E, numel // ops.MOE_ROWS_BLOCK_M) * (F // 128) >= 128)
-    return ops.MOE_ROWS_BLOCK_M if wide else block_m
+    return ops.MOE_ROWS_BLOCK_M if wide and _rows_blocks_ahead(block_m, numel, E, K, F) else block_m
+
+
+@functools.lru_cache(maxsize=1024)
+def _rows_blocks_ahead(block_m: int, numel: int, E: int, K: int, F: int) -> bool:
+    """Whether blocks of 320 rows are ahead of `block_m`.  Two rounds of tiles and more in the second product: always (60 to 256 experts of 512 to 1536 over 2048
+    or 5120, 500 to 8192 tokens, even routing and not: 0.95 to 1.35 times as fast).  With fewer a launch is as long as its rounds of the
+    CUs, in each of which a tile of 320 rows takes longer than one of 256, and only saves what it saves of them: the rounds of both products
+    for experts with rows around the average (a tenth about it, and the root of it), a tile of 128 x 512 counted 1.75, of up to 128 rows in a
+    block of 256 0.88, and a margin.  Whole layer, blocks of 256 / of 320, us: 8 experts of 4096 x 1792, top 2, 2048 tokens 262 / 188, 2600 284 / 336; 8 of 2048 x
+    1024, 4096 tokens 151 / 121, 5000 182 / 211; 16 of 4096 x 1024, top 4, 2048 298 / 220, 2600 317 / 364; 32 of 1024 x 512, top 4, 1024 56 / 57, 4096 128 / 86."""
+    if E * -(-K // 256) >= 480:
+        return True
+    mean = numel / E
+
+    def rounds(block: int, of_gate: int, of_down: int) -> float:
+        full = short = 0.0                                                # tiles of an expert, and those of up to 128 rows
+        for z in (-1.3, -0.5, 0.0, 0.5, 1.3):
+            n, rest = divmod(max(1.0, mean * (1 + 0.1 * z) + z * mean ** 0.5), block)
+            low = block == 256 and 0 < rest <= 128
+            full += E / 5 * (n + (rest > 0 and not low))
+            short += E / 5 * low
+        t, cost = 0.0, 1.75 if block == 128 else 1.0
+        for steps, columns in ((K // 64, -(-F // of_gate)), (F // 64, -(-K // of_down))):
+            tall = full * columns / 256
+            all_ = tall + short * columns / 256
+            t += (steps + 4) * max(math.ceil(tall - 1e-6) * cost, math.ceil(all_ - 1e-6) * 0.88 if short else 0.0, tall * cost + (all_ - tall) * 0.88)
+        return t
+
+    wide = block_m == 128
+    return rounds(block_m, 256 if wide else 128, 512 if wide else 256) >= 1.08 * rounds(ops.MOE_ROWS_BLOCK_M, 128, 256)
 
 
 def _local_ids(topk_ids: torch.Tensor, expert_offset: int) -> torch.Tensor:
@@ -199,7 +232,7 @@ def fused_experts_fp8(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
     if block_m is None:
         block_m = MOE_BLOCK_M if numel <= 2048 else 2 * MOE_BLOCK_M
         if K % 128 == 0 and N2 % 256 == 0 and K <= 8192 and N2 <= 2 * 8192 and numel <= 48 * E:
-            # blocks of the LDS-DMA stream (csrc/fp8_stream.h): by the rows an expert has on average, so that few have a second block,
+            # blocks of the LDS-DMA stream (csrc/fp8_stream.hip): by the rows an expert has on average, so that few have a second block,
             # whose weights are read again.  64 experts of 2048 x 1408, top 6, whole layer in blocks of 16 / 32 / 64 / 128 rows, us: 32 tokens (3 rows)
             # 108 / 114 / 133 / 148, 96 (9) 121 / 123 / 138 / 153, 128 (12) 130 / 126 / 140 / 155, 256 (24) 203 / 146 / 150 / 165, 512 (48) 314 / 244 /
             # 174 / 191.  A token routes to an expert at most once: T tokens need no block above T.
