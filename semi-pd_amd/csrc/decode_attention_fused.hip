@@ -11,8 +11,8 @@
 // num_kv_splits = `splits`, NW of them or fewer -- the last waves have none then --, walked by the same code:
 // decode_mfma_walk.h).  (Small batches: Z workgroups per pair, each merging its NW splits into ONE stage-1 partial;
 // decode_stage2_kernel then merges Z partials per head instead of NW * Z.)
-//   1. the lanes that rotate ask for their planes and cos / sin values, then every wave asks for its first tile of K / V
-//      rows and the K rows of the second (unless they hold the new token);
+//   1. the lanes that rotate ask for their planes and cos / sin values, then every other wave asks for its first tile of
+//      K / V rows (unless it holds the new token);
 //   2. the wave whose range ends with the new token sums the planes of k and v, rotates k and stores both pool rows
 //      (and waits for its stores: it is the only reader of those rows in this launch); the other waves rotate q into LDS;
 //   3. a raw barrier on the LDS writes only: no wave waits there for the K / V rows it has in flight;
@@ -67,10 +67,11 @@ decode_rope_attn_kernel(T* __restrict__ out, float* __restrict__ attn_logits, co
   const int owner = owner_g / NW == z ? owner_g - z * NW : -1;     // -1: the new token belongs to another workgroup
   constexpr int half = D / 2, IPH = half / V;                 // items of 8 pairs per head
   // a wave that rotates asks for its planes first and for its tiles after the barrier: loads return in order, and behind
-  // the K / V rows of two tiles the planes would arrive a memory latency later -- with every wave of every CU of the
-  // launch waiting at the same barrier.  The other waves have two tiles in flight by then.
+  // the K / V rows of a tile the planes would arrive a memory latency later -- with every wave of every CU of the
+  // launch waiting at the same barrier.  The other waves have a tile in flight by then, of two the K rows of the second as well were no faster (8
+  // kv heads of 64, four layers + head, 3 requests of 1500 tokens 261 us, 128 of 1500 735; with them 262, 748).
   const bool rotates = wave == owner || ((owner < 0 || wave < owner) ? wave : wave - 1) * 64 < group * IPH;
-  const int early_tiles = rotates ? 0 : ((s_begin >= seq_len || s_begin + 64 < seq_len) ? 2 : (s_begin + 32 < seq_len ? 1 : 0));
+  const bool early = !rotates && (s_begin >= seq_len || s_begin + 32 < seq_len);
 
   // ---- the rotation ----
   constexpr int ROLE_NONE = 0, ROLE_Q = 1, ROLE_K = 2, ROLE_V = 3, PRE = 4;   // PRE planes travel before the tiles
@@ -163,7 +164,7 @@ decode_rope_attn_kernel(T* __restrict__ out, float* __restrict__ attn_logits, co
   rotation_loads();
   decode_mfma_walk<T, D, KV, false>(
       wave_lds[wave], k_buf, v_buf, kv_indices + kv_start, s_begin, s_end, hk, kbuf_stride, vbuf_stride, sm_scale,
-      logit_cap, early_tiles,
+      logit_cap, early,
       [&](FragD (&qf)[KS]) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {

@@ -52,7 +52,7 @@ decode_mfma_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __res
   float m_run, l_tot;
   decode_mfma_walk<T, D, KV, PAUSE>(
       v_lds_all[wave], k_buf, v_buf, kv_indices + kv_start, s_begin, s_end, hk, kbuf_stride, vbuf_stride, sm_scale,
-      logit_cap, 2,
+      logit_cap, true,
       [&](FragD (&qf)[KS]) {
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {

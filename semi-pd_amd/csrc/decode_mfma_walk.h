@@ -68,9 +68,9 @@ template <int D> struct DecodeWalkLds {
 // Walks tokens [s_begin, s_end) of the sequence whose pool rows are idx_base[0 .. ).  An empty range is allowed (nothing
 // is accumulated, l_tot = 0).
 //   load_q(qf): fills the Q^T fragments (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
-//   mid():      called once before the Q fragments are fetched, after the loads of the first `early_tiles` (0 or more: K and V
-//               rows of tile 0) were issued -- the fused kernel rotates q / k there and stores
-//               the new token's rows; a tile that holds the new token must not be asked for before that
+//   mid():      called once before the Q fragments are fetched, with `early` after the loads of the first tile's K and V rows were
+//               issued -- the fused kernel rotates q / k there and stores the new token's rows; a tile that holds the new token must not be
+//               asked for before that
 //   PAUSE:      the loads of the next tile behind a branch on there being one: with that each of their waits drains what was asked for in
 //               front of it, which is slower by itself and faster where the launch leaves some CUs with twice the waves of the others
 //               (see launch_decode_mfma's rule)
@@ -80,7 +80,7 @@ template <typename T, int D, typename KV, bool PAUSE, typename QLoad, typename M
 __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __restrict__ k_buf, const KV* __restrict__ v_buf,
                                                  const int32_t* __restrict__ idx_base, int s_begin, int s_end, int hk,
                                                  int64_t kbuf_stride, int64_t vbuf_stride, float sm_scale, float logit_cap,
-                                                 int early_tiles, QLoad&& load_q, Mid&& mid, f32x4 (&o_acc)[D / 16],
+                                                 bool early, QLoad&& load_q, Mid&& mid, f32x4 (&o_acc)[D / 16],
                                                  float& m_run, float& l_tot) {
   constexpr int KS = D / 32, DT = D / 16, CPR = D / 8, NV = CPR / 2;
   using KVT = KVTraits<T, KV>;
@@ -229,13 +229,13 @@ __device__ __forceinline__ void decode_mfma_walk(uint8_t* v_lds, const KV* __res
     idx_cur = load_idx(0);
     idx_next = load_idx(1);
   }
-  if (early_tiles >= 1) {
+  if (early) {
     issue_v(idx_cur);
     issue_k(kreg, idx_cur);
   }
   mid();
   load_q(qf);
-  if (early_tiles < 1) {
+  if (!early) {
     issue_v(idx_cur);
     issue_k(kreg, idx_cur);
   }

@@ -900,8 +900,8 @@ int semipd_gemm_tall_planes(void* out, float* planes, size_t planes_bytes, const
 }
 
 /* invoke_fused_moe_kernel (fused_moe.py:501-612) for prefill-sized calls with the tiled ping-pong GEMM: sorted_token_ids /
- * expert_ids from moe_align_block_size with block size block_m = 256 (256 x 256 tiles) or 128 (128 x 512 tiles): one
- * expert per tile; sorted_token_ids must hold max_sorted entries, a multiple of block_m.  c[id, :] = a[id / top_k_div, :] @ w[expert]^T for every routed entry id <
+ * expert_ids from moe_align_block_size with block size block_m = 256 (256 x 256 tiles), 128 (128 x 512
+ * tiles) or 320 (up to 320 x 256, moe_gemm_rows.h: k % 128, c 16-byte aligned, operands below 2 GiB): one expert per tile; sorted_token_ids must hold max_sorted entries, a multiple of block_m.  c[id, :] = a[id / top_k_div, :] @ w[expert]^T for every routed entry id <
  * num_valid, times topk_weights[id] when mul_routed_weight; fuse_silu_mul: w[e] = merged [gate; up] ([n, k], n = 2 x
  * output width) and c = SiLU(gate) * up of the products rounded to dtype. */
 int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* topk_weights, const int32_t* sorted_token_ids,

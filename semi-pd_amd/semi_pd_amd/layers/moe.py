@@ -235,7 +235,8 @@ def fused_experts_fp8(hidden_states: torch.Tensor, w1: torch.Tensor, w2: torch.T
             # blocks of the LDS-DMA stream (csrc/fp8_stream.hip): by the rows an expert has on average, so that few have a second block,
             # whose weights are read again.  64 experts of 2048 x 1408, top 6, whole layer in blocks of 16 / 32 / 64 / 128 rows, us: 32 tokens (3 rows)
             # 108 / 114 / 133 / 148, 96 (9) 121 / 123 / 138 / 153, 128 (12) 130 / 126 / 140 / 155, 256 (24) 203 / 146 / 150 / 165, 512 (48) 314 / 244 /
-            # 174 / 191.  A token routes to an expert at most once: T tokens need no block above T.
+            # 174 / 191.  A token routes to an expert at most once: T tokens need no block above T.  (An
+            # expert-parallel rank counts the rows of all experts: blocks of at most the 64 rows that it had before.)
             block_m = 16 if T <= 16 or numel <= 9 * E else 32 if T <= 32 or numel <= 24 * E else 64
     max_sorted = numel + E * (block_m - 1)
     sorted_ids = torch.empty(max_sorted, dtype=torch.int32, device=dev)

@@ -39,6 +39,7 @@ def test_decode_at_the_edges_of_tiles(rows, H, G, D, splits, cap):
                 s = k[at, h // (H // G)].double() @ q[b, h].double() * scale
                 want[b, h] = torch.softmax(cap * torch.tanh(s / cap) if cap else s, 0) @ v[at, h // (H // G)].double()
     some = [b for b, n in enumerate(lens) if n]
+    assert bool((got[lens.index(0)] == 0).all())
     ulp = 2.0 ** -8
     assert float((got[some] - want[some]).norm() / want[some].norm()) < 1.5 * ulp
     torch.testing.assert_close(got[some], want[some], rtol=6 * ulp, atol=12 * ulp)

@@ -1,4 +1,4 @@
-"""Block-scaled fp8 expert GEMMs through LDS-DMA (csrc/fp8_stream.h): blocks of 16, 32 and 64 rows."""
+"""Block-scaled fp8 expert GEMMs through LDS-DMA (csrc/fp8_stream.hip): blocks of 16, 32 and 64 rows."""
 import pytest
 import torch
 
