@@ -92,18 +92,18 @@ def _tall_block(block_m: int, tokens: int, topk: int, E: int, K: int, F: int) ->
     numel = tokens * topk
     wide = (ops.MOE_TALL_BLOCK_M == 256 and K % 128 == 0 and F % 128 == 0 and min(K, F) >= 512 and 2 * F * K < 1 << 30
             and tokens * K < 1 << 30 and numel * F < 1 << 30 and max(E, numel // ops.MOE_ROWS_BLOCK_M) * (F // 128) >= 128)
-    return ops.MOE_ROWS_BLOCK_M if wide and _rows_blocks_ahead(block_m, numel, E, K, F) else block_m
+    return ops.MOE_ROWS_BLOCK_M if wide and _rows_blocks_ahead(block_m, numel, E, K, F, ops.declared_cus()) else block_m
 
 
 @functools.lru_cache(maxsize=1024)
-def _rows_blocks_ahead(block_m: int, numel: int, E: int, K: int, F: int) -> bool:
-    """Whether blocks of 320 rows are ahead of `block_m`.  Two rounds of tiles and more in the second product: always (60 to 256 experts of 512 to 1536 over 2048
+def _rows_blocks_ahead(block_m: int, numel: int, E: int, K: int, F: int, cus: int) -> bool:
+    """Whether blocks of 320 rows are ahead of `block_m` on `cus` CUs.  Two rounds of tiles and more in the second product: always (60 to 256 experts of 512 to 1536 over 2048
     or 5120, 500 to 8192 tokens, even routing and not: 0.95 to 1.35 times as fast).  With fewer a launch is as long as its rounds of the
     CUs, in each of which a tile of 320 rows takes longer than one of 256, and only saves what it saves of them: the rounds of both products
     for experts with rows around the average (a tenth about it, and the root of it), a tile of 128 x 512 counted 1.75, of up to 128 rows in a
     block of 256 0.88, and a margin.  Whole layer, blocks of 256 / of 320, us: 8 experts of 4096 x 1792, top 2, 2048 tokens 262 / 188, 2600 284 / 336; 8 of 2048 x
     1024, 4096 tokens 151 / 121, 5000 182 / 211; 16 of 4096 x 1024, top 4, 2048 298 / 220, 2600 317 / 364; 32 of 1024 x 512, top 4, 1024 56 / 57, 4096 128 / 86."""
-    if E * -(-K // 256) >= 480:
+    if E * -(-K // 256) * 8 >= 15 * cus:
         return True
     mean = numel / E
 
@@ -116,8 +116,8 @@ def _rows_blocks_ahead(block_m: int, numel: int, E: int, K: int, F: int) -> bool
             short += E / 5 * low
         t, cost = 0.0, 1.75 if block == 128 else 1.0
         for steps, columns in ((K // 64, -(-F // of_gate)), (F // 64, -(-K // of_down))):
-            tall = full * columns / 256
-            all_ = tall + short * columns / 256
+            tall = full * columns / cus
+            all_ = tall + short * columns / cus
             t += (steps + 4) * max(math.ceil(tall - 1e-6) * cost, math.ceil(all_ - 1e-6) * 0.88 if short else 0.0, tall * cost + (all_ - tall) * 0.88)
         return t
 

@@ -474,6 +474,11 @@ def set_declared_cus(cus: int) -> None:
     _DENSE_GEMM["cus"] = int(cus)
 
 
+def declared_cus() -> int:
+    """That count, 256 where none was declared."""
+    return _DENSE_GEMM["cus"] or 256
+
+
 def dense_gemm_library_version() -> int:
     import ctypes as _C
     v = _C.c_int(0)
