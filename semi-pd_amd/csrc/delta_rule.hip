@@ -193,14 +193,21 @@ __device__ __forceinline__ void delta_conv_state(const DeltaArgs& a, int b, int 
   const int keep = a.taps - 1;
   // entry s of the new state is the input at index n - keep + s of the portion; a negative index reaches into the old
   // state (entry s + n > s, read before entry s is written) or, at the start of a sequence, in front of it
-  for (int s = 0; s < keep; ++s) {
+  auto input = [&](int s) {
     const int64_t l = n - keep + s;
-    float x;
-    if (l >= 0) x = Elem<T>::to_f(p[(t0 + l) * a.ld + col]);
-    else if (first_pos == 0) x = 0.f;
-    else x = cs[(int64_t)(keep + l) * C + c];
-    cs[(int64_t)s * C + c] = x;
+    if (l >= 0) return Elem<T>::to_f(p[(t0 + l) * a.ld + col]);
+    return first_pos == 0 ? 0.f : cs[(int64_t)(keep + l) * C + c];
+  };
+  if (keep <= kRecHalo) {                                        // (read at once, then written: not a round trip each)
+    float x[kRecHalo];
+#pragma unroll
+    for (int s = 0; s < kRecHalo; ++s) x[s] = s < keep ? input(s) : 0.f;
+#pragma unroll
+    for (int s = 0; s < kRecHalo; ++s)
+      if (s < keep) cs[(int64_t)s * C + c] = x[s];
+    return;
   }
+  for (int s = 0; s < keep; ++s) cs[(int64_t)s * C + c] = input(s);
 }
 template <typename T>
 __global__ void __launch_bounds__(256) delta_conv_state_kernel(DeltaArgs a) {
@@ -459,7 +466,8 @@ __global__ void __launch_bounds__(1024) delta_decode_kernel(DeltaArgs a) {
 // one workgroup, which moves their inputs on itself: ONE launch.  (gridDim.z > 1: the heads of a key head over several.)  A thread of a team has four columns and every 1024 / E-th row
 // of S, all of its pieces in flight from the start; the two dot products are summed over lanes and the team's waves.  Bound by HBM, the
 // state read and written once: 32 requests, 32 heads of 128 x 128 (134 MB): a column of S by four lanes of four bytes each 57.7 -> 32.3
-// us; 3 requests, 32 heads of 64 x 64: 10.6 (two launches) -> 9.8.
+// us; 3 requests, 32 heads of 64 x 64: 10.6 (two launches) -> 9.8.  With the loads of the convolutions and of the gates in front of the state's (they came one
+// behind the other when the state had arrived): 32 heads of 128 x 128, 32 requests, whole call 31.6 -> 28.5, 64 requests 77.7 -> 68.9.
 template <typename T, int NIT>
 __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];       // q [D] | k [D] | v, later o [per E] | sums of every team [4][2][E] | scalars
@@ -480,27 +488,88 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
   auto piece = [&](int hh, int n) {
     return !fresh && hh < per && n < D ? *reinterpret_cast<const float4*>(a.state + slot * a.state_ld + ((int64_t)(g * per + hh) * D + n) * E + e) : float4{0.f, 0.f, 0.f, 0.f};
   };
+  // Memory answers in order: what the convolutions are made of is asked for in front of the state, and with it what the team's first head needs
+  // behind the sums; their arithmetic goes on while the state is on its way, and nothing is a round trip of its own.  Up to four taps,
+  // the workgroup's first two channels a thread; others one by one.
+  const int channels = 2 * D + per * E;
+  struct Channel {
+    const T *p, *cw;
+    int ch;                                                       // its place in the kept inputs
+  };
+  auto channel = [&](int i) {
+    const bool is_v = i >= 2 * D;
+    const int d = is_v ? g * per * E + i - 2 * D : g * D + (i < D ? i : i - D);                              // channel within q, k or v
+    return Channel{p + (is_v ? a.v_off : (i < D ? a.q_off : a.k_off)) + d, (const T*)(is_v ? a.conv_v : (i < D ? a.conv_q : a.conv_k)) + (int64_t)d * taps,
+                   is_v ? 2 * G * D + d : (i < D ? d : G * D + d)};
+  };
+  auto mine = [&](int i) { return i < channels && (i < 2 * D || gridDim.z == 1 || ((i - 2 * D) / E / teams) % gridDim.z == blockIdx.z); };      // (or a head of another workgroup)
+  float* cs = a.conv_state + slot * a.conv_ld;
+  struct Inputs {
+    T cur, w[kRecTaps];
+    float x[kRecTaps];                                            // (of k tokens back)
+  } in[2];
+  const bool early = taps <= kRecTaps;
+  if (early)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const Channel c = channel(min(tid + (int)blockDim.x * u, channels - 1));
+      in[u].cur = *c.p;
+#pragma unroll
+      for (int k = 0; k < kRecTaps; ++k) {
+        in[u].w[k] = c.cw[max(taps - 1 - k, 0)];
+        in[u].x[k] = k > 0 && k < taps && !fresh ? cs[(int64_t)(taps - 1 - k) * C + c.ch] : 0.f;
+      }
+    }
+  float gate_log, gate_bias, weight[4];
+  T gate_a, gate_b, gate[4];
+  auto fetch_gates = [&](int hh) {
+    const int h = g * per + (hh < per ? hh : per - 1);
+    gate_log = a.a_log[h], gate_bias = a.dt_bias[h];
+    gate_a = p[a.a_off + h], gate_b = p[a.b_off + h];
+    if (n0 == 0)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) gate[c] = p[a.gate_off + h * E + e + c];
+  };
+  fetch_gates((int)blockIdx.z * teams + team);
+  if (n0 == 0)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) weight[c] = Elem<T>::to_f(((const T*)a.norm_w)[e + c]);
 #pragma unroll
   for (int i = 0; i < NIT; ++i) S[i] = piece((int)blockIdx.z * teams + team, n0 + i * rows);
-  float* cs = a.conv_state + slot * a.conv_ld;
-  for (int i = tid; i < 2 * D + per * E; i += blockDim.x) {
-    const bool is_v = i >= 2 * D;
-    if (is_v && gridDim.z > 1 && ((i - 2 * D) / E / teams) % gridDim.z != blockIdx.z) continue;                                  // (a head of another workgroup)
-    const int d = is_v ? g * per * E + i - 2 * D : g * D + (i < D ? i : i - D);                              // channel within q, k or v
-    const int ch = is_v ? 2 * G * D + d : (i < D ? d : G * D + d);                                           // its place in the state
-    const T* cw = (const T*)(is_v ? a.conv_v : (i < D ? a.conv_q : a.conv_k)) + (int64_t)d * taps;
-    const float cur = Elem<T>::to_f(p[(is_v ? a.v_off : (i < D ? a.q_off : a.k_off)) + d]);
-    float y = Elem<T>::to_f(cw[taps - 1]) * cur;
-    // state entry s is the input s - (taps - 1) tokens back; every entry moves one place down and the token comes in last
+  // state entry s is the input s - (taps - 1) tokens back; every entry moves one place down and the token comes in last (where several
+  // workgroups read the old inputs of q and k, in a launch of its own)
+  if (early)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = tid + (int)blockDim.x * u;
+      if (!mine(i)) continue;
+      const float cur = Elem<T>::to_f(in[u].cur);
+      float y = Elem<T>::to_f(in[u].w[0]) * cur;
+#pragma unroll
+      for (int k = 1; k < kRecTaps; ++k)
+        if (k < taps && !fresh) y += Elem<T>::to_f(in[u].w[k]) * in[u].x[k];
+      lds[i] = silu_f(y);
+      if (gridDim.z > 1) continue;
+      const int ch = channel(i).ch;
+#pragma unroll
+      for (int k = 1; k < kRecTaps - 1; ++k)
+        if (k < taps - 1) cs[(int64_t)(taps - 2 - k) * C + ch] = in[u].x[k];
+      if (taps > 1) cs[(int64_t)(taps - 2) * C + ch] = cur;
+    }
+  for (int i = early ? tid + 2 * (int)blockDim.x : tid; i < channels; i += blockDim.x) {
+    if (!mine(i)) continue;
+    const Channel c = channel(i);
+    const float cur = Elem<T>::to_f(*c.p);
+    float y = Elem<T>::to_f(c.cw[taps - 1]) * cur;
     for (int k = 1; k < taps; ++k) {
       const int s = taps - 1 - k;
-      const float x = fresh ? 0.f : cs[(int64_t)s * C + ch];
-      if (!fresh) y += Elem<T>::to_f(cw[s]) * x;
+      const float x = fresh ? 0.f : cs[(int64_t)s * C + c.ch];
+      if (!fresh) y += Elem<T>::to_f(c.cw[s]) * x;
     }
     lds[i] = silu_f(y);
-    if (gridDim.z > 1) continue;                                  // (several read the old inputs of q and k: they move on in a launch of their own)
-    for (int s = 1; s < taps - 1; ++s) cs[(int64_t)(s - 1) * C + ch] = fresh ? 0.f : cs[(int64_t)s * C + ch];
-    if (taps > 1) cs[(int64_t)(taps - 2) * C + ch] = cur;
+    if (gridDim.z > 1) continue;
+    for (int s = 1; s < taps - 1; ++s) cs[(int64_t)(s - 1) * C + c.ch] = fresh ? 0.f : cs[(int64_t)s * C + c.ch];
+    if (taps > 1) cs[(int64_t)(taps - 2) * C + c.ch] = cur;
   }
   __syncthreads();
   if (tid < 64) {
@@ -545,7 +614,7 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
       *reinterpret_cast<float4*>(sums + (tt >> 6) * 2 * E + E + e) = dq;
     }
     __syncthreads();
-    const float gt = expf(-expf(a.a_log[h]) * softplus_f(Elem<T>::to_f(p[a.a_off + h]) + a.dt_bias[h])), beta = sigmoid_f(Elem<T>::to_f(p[a.b_off + h]));
+    const float gt = expf(-expf(gate_log) * softplus_f(Elem<T>::to_f(gate_a) + gate_bias)), beta = sigmoid_f(Elem<T>::to_f(gate_b));
     float u[4], o4[4], sq_o = 0.f;
     const float* vh = v_l + (on ? hh : 0) * E + e;
 #pragma unroll
@@ -573,9 +642,9 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
       const float inv = 1.0f / sqrtf(sq_o / (float)E + a.eps);
       T* out = (T*)a.out + (int64_t)b * a.out_ld + h * E + e;
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        out[c] = Elem<T>::from_f(o4[c] * inv * Elem<T>::to_f(((const T*)a.norm_w)[e + c]) * silu_f(Elem<T>::to_f(p[a.gate_off + h * E + e + c])));
+      for (int c = 0; c < 4; ++c) out[c] = Elem<T>::from_f(o4[c] * inv * weight[c] * silu_f(Elem<T>::to_f(gate[c])));
     }
+    if (h0 + teams * (int)gridDim.z < per) fetch_gates(hh + teams * (int)gridDim.z);
     __syncthreads();
   }
 }
