@@ -393,6 +393,11 @@ decode_stage2_wave_kernel(T* __restrict__ out, const float* __restrict__ attn_lo
   stage2_merge<T>(out + (int64_t)b * o_stride + (int64_t)hq * Dv, base, n_valid, Dv, lane, 64);
 }
 
+// defined in decode_merge.hip; false: not a shape of its
+template <typename T>
+bool launch_stage2_at_once(T* out, const float* attn_logits, const int32_t* kv_indptr, int64_t batch, int num_q_heads, int head_dim_v, int64_t o_stride,
+                           int num_kv_splits, int threads, hipStream_t st);
+
 template <typename T>
 static int launch_decode_stage2_t(T* out, const float* attn_logits, const int32_t* kv_indptr, int64_t batch, int num_q_heads,
                                   int head_dim_v, int64_t o_stride, int num_kv_splits, hipStream_t st) {
@@ -403,6 +408,7 @@ static int launch_decode_stage2_t(T* out, const float* attn_logits, const int32_
   } else {
     dim3 grid((unsigned)batch, (unsigned)num_q_heads);
     const int threads = head_dim_v <= 64 ? 64 : head_dim_v <= 128 ? 128 : 256;
+    if (launch_stage2_at_once<T>(out, attn_logits, kv_indptr, batch, num_q_heads, head_dim_v, o_stride, num_kv_splits, threads, st)) return launch_status("decode_stage2");
     hipLaunchKernelGGL((decode_stage2_kernel<T>), grid, dim3(threads), 0, st, out, attn_logits, kv_indptr, num_q_heads,
                        head_dim_v, o_stride, num_kv_splits);
   }
