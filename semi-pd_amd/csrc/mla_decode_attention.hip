@@ -14,6 +14,7 @@
 // a tile instead of three), only a request's last tile is masked, and partials leave in 16-byte stores: 1.55 -> 1.27 us a tile and
 // workgroup, 13.5 -> 13.0 us for a single tile with its merge.  16 heads, bf16 rows, whole call: 32 requests at 1.1 k tokens in 8 splits 21.5
 // -> 20.3 us (kernel 18.1 -> 16.7 under the profiler), in one split 73 -> 59, 64 at 1.1 k 30.3 -> 29.1, 128 at 2 k in 4 splits 75 -> 72.5 (fp8 rows 60 -> 54).
+// Q asked for in front of the rows: 18.9 -> 18.0 (128 at 500 29.0 -> 27.8).
 //
 // Replaces _fwd_grouped_kernel_stage1 for Lk = 576 / Lv = 512
 // (layers/attention/triton_ops/decode_attention.py:234-390, BLOCK_DPE = 64 path).
@@ -75,6 +76,15 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
   const int heads = min(16, num_q_heads - h0);
   const bool head_ok = c16 < heads;
 
+  // Q^T fragments of this wave's k half (B operand): lane = head c16, d = ks*32 + q4*8 .. +8.  In front of everything: memory answers in
+  // order, and behind the rows of two tiles the first one would wait for both
+  const int ks0 = (wave >> 1) * KSW;
+  FragM qf[KSW];
+  {
+    const T* qrow = q + (int64_t)b * q_stride + (int64_t)(h0 + min(c16, heads - 1)) * DK + ks0 * 32 + q4 * 8;
+#pragma unroll
+    for (int ks = 0; ks < KSW; ++ks) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + ks * 32);      // (heads past the last: not stored)
+  }
   const int kv_start = kv_indptr[b];
   const int seq_len = kv_indptr[b + 1] - kv_start;
   const int per_split = (seq_len + num_kv_splits - 1) / num_kv_splits;
@@ -110,14 +120,6 @@ mla_decode_kernel(T* __restrict__ out, const T* __restrict__ q, const KV* __rest
   idx0 = load_idx(2);
   fetch(reg[1], idx1);
 
-  // Q^T fragments of this wave's k half (B operand): lane = head c16, d = ks*32 + q4*8 .. +8
-  const int ks0 = (wave >> 1) * KSW;
-  FragM qf[KSW];
-  {
-    const T* qrow = q + (int64_t)b * q_stride + (int64_t)(h0 + min(c16, heads - 1)) * DK + ks0 * 32 + q4 * 8;
-#pragma unroll
-    for (int ks = 0; ks < KSW; ++ks) qf[ks].u = *reinterpret_cast<const uint4*>(qrow + ks * 32);      // (heads past the last: not stored)
-  }
   f32x4 o_acc[DTW];
 #pragma unroll
   for (int t = 0; t < DTW; ++t) o_acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
