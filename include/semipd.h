@@ -170,6 +170,14 @@ int semipd_build_kv_indices(const int32_t* req_to_token, int64_t req_to_token_st
                             const int32_t* start, int32_t* kv_indptr, int32_t* kv_indices,
                             int64_t batch, void* stream);
 
+/* What a captured decode step reads of its batch, in one launch: rows 0 .. batch - 1 of token ids, pool rows, lengths, slots of the new
+ * tokens and (state_rows may be NULL) state rows from src_* to the graph's own; rows batch .. rows - 1 are padding: pool row, slot and
+ * state row 0, length pad_len, ids as they are.  src_state NULL: no state rows but the padding's.
+ * replaces the copies in CudaGraphRunner.replay (model_executor/cuda_graph_runner.py:455-531). */
+int semipd_decode_inputs(int64_t* ids, int64_t* pool_rows, int64_t* lens, int64_t* slots, int64_t* state_rows, const int64_t* src_ids,
+                         const int64_t* src_pool_rows, const int64_t* src_lens, const int64_t* src_slots, const int64_t* src_state,
+                         int64_t batch, int64_t rows, int64_t pad_len, void* stream);
+
 /* positions / extend_start_loc for an extend batch:
  * positions[start_loc[b]+j] = prefix_lens[b]+j  (j < extend_lens[b]),
  * start_loc = exclusive cumsum(extend_lens).

@@ -46,6 +46,7 @@ _SIGNATURES = {
     "semipd_kv_store_cvt": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i32, _i32, _vp],
     "semipd_build_kv_indices": [_vp, _i64, _vp, _vp, _i32, _vp, _vp, _vp, _i64, _vp],
     "semipd_compute_positions": [_vp, _vp, _vp, _vp, _i64, _vp],
+    "semipd_decode_inputs": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp],
     "semipd_decode_attention": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i32, _i32, _i32, _i32, _i64,
                                 _i64, _i64, _i64, _i32, _f32, _f32, _i32, _i32, _vp],
     "semipd_decode_rope_attention_planes_supported": [_i32, _i32, _i32, _i32, _i32],

@@ -13,6 +13,7 @@ from typing import Dict, List, Tuple
 
 import torch
 
+from semi_pd_amd import ops
 from semi_pd_amd.model_executor.forward_batch_info import ForwardBatch, ForwardMode
 
 
@@ -190,17 +191,21 @@ class HipGraphRunner:
         from semi_pd_amd.layers.basic import LogitsProcessorOutput
         raw_bs = forward_batch.batch_size
         bs = self.capture_bs[bisect.bisect_left(self.capture_bs, raw_bs)]
-        if bs != raw_bs:
-            self.seq_lens.fill_(self.seq_len_fill_value)
-            self.out_cache_loc.zero_()
-            self.req_pool_indices.zero_()
-            self.state_indices.zero_()
-        if forward_batch.state_indices is not None:
-            self.state_indices[:raw_bs].copy_(forward_batch.state_indices)
-        self.input_ids[:raw_bs].copy_(forward_batch.input_ids)
-        self.req_pool_indices[:raw_bs].copy_(forward_batch.req_pool_indices)
-        self.seq_lens[:raw_bs].copy_(forward_batch.seq_lens)
-        self.out_cache_loc[:raw_bs].copy_(forward_batch.out_cache_loc)
+        own = (self.input_ids, self.req_pool_indices, self.seq_lens, self.out_cache_loc, self.state_indices)
+        batch = (forward_batch.input_ids, forward_batch.req_pool_indices, forward_batch.seq_lens, forward_batch.out_cache_loc,
+                 forward_batch.state_indices)
+        if any(t is not None and t.shape != (raw_bs,) for t in batch) or not ops.decode_inputs(own, batch, bs, self.seq_len_fill_value):
+            if bs != raw_bs:
+                self.seq_lens.fill_(self.seq_len_fill_value)
+                self.out_cache_loc.zero_()
+                self.req_pool_indices.zero_()
+                self.state_indices.zero_()
+            if forward_batch.state_indices is not None:
+                self.state_indices[:raw_bs].copy_(forward_batch.state_indices)
+            self.input_ids[:raw_bs].copy_(forward_batch.input_ids)
+            self.req_pool_indices[:raw_bs].copy_(forward_batch.req_pool_indices)
+            self.seq_lens[:raw_bs].copy_(forward_batch.seq_lens)
+            self.out_cache_loc[:raw_bs].copy_(forward_batch.out_cache_loc)
         # the variant of the stream the instance is on (its OWN CU count: an experiment that declares another count to the
         # kernels, SEMIPD_DECLARED_CUS_*, must not change which graph is found)
         share = getattr(self.mr, "cu_share", None)

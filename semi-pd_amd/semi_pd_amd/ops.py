@@ -228,6 +228,19 @@ def compute_position(extend_prefix_lens: torch.Tensor, extend_seq_lens: torch.Te
     return positions, start_loc
 
 
+def decode_inputs(own, batch, rows: int, pad_len: int) -> bool:
+    """own = (token ids, pool rows, lengths, slots, state rows) of a captured decode step, batch = the same of a decode batch (state rows may be
+    None): one launch for the copies, with rows len(batch) .. rows - 1 padded.  False, and nothing done, where one of the batch's is not a
+    contiguous int64 tensor on the graph's device."""
+    dev = own[0].device
+    for t in batch:
+        if t is not None and (t.dtype != torch.int64 or t.device != dev or t.dim() != 1 or not t.is_contiguous()):
+            return False
+    check(_lib.load().semipd_decode_inputs(*[ptr(t) for t in own], *[ptr(t) for t in batch], batch[0].shape[0], rows, pad_len,
+                                           current_stream(dev)), "decode_inputs")
+    return True
+
+
 # --------------------------------------------------------------------------- attention
 def decode_attention_fwd(q: torch.Tensor, k_buffer: torch.Tensor, v_buffer: torch.Tensor,
                          o: torch.Tensor, kv_indptr: torch.Tensor, kv_indices: torch.Tensor,
