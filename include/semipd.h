@@ -932,7 +932,8 @@ int semipd_latent_attention(const void* q, int64_t q_ld, void* out, int64_t out_
  * S <- S + k u^T, o = S^T q; out = o / rms(o) * norm_weight * silu(gate).  S (fp32 [heads, k_dim, v_dim]) and the last
  * taps - 1 inputs (fp32 [taps - 1, channels], channels q | k | v) live in state / conv_state[state_indices[b]]: read
  * unless request b's rows start its sequence, written after its last row.  work: fp32 [num_tokens, work_ld], work_ld >=
- * semipd_delta_rule_work_width.  Batch description as in semipd_local_attention.  No reference counterpart. */
+ * semipd_delta_rule_work_width (may be NULL for batches without q_start whose v_dim is at most 256, 1024 with k_dim below 32).  Batch
+ * description as in semipd_local_attention.  No reference counterpart. */
 int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,
                       int64_t a_off, int64_t b_off, const void* conv_q, const void* conv_k, const void* conv_v,
                       const float* a_log, const float* dt_bias, const void* norm_weight, float eps, float* work,
@@ -940,6 +941,8 @@ int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
                       const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
                       const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int num_k_heads,
                       int k_dim, int v_dim, int taps, void* out, int64_t out_ld, int dtype, void* stream);
+/* The same with its 36 arguments as 64-bit words in their order, eps as a double: one argument to hand over instead of 36. */
+int semipd_delta_rule_record(const void* record);
 /* fp32 elements that semipd_delta_rule_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
 int64_t semipd_delta_rule_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int num_k_heads, int k_dim, int taps);
 /* semipd_delta_rule of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a
@@ -1020,6 +1023,8 @@ int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
                        int64_t conv_ld, const int64_t* state_indices, const int64_t* seq_lens, const int32_t* q_start,
                        const int32_t* q_len, int64_t batch, int64_t num_tokens, int num_heads, int groups, int state_size, int v_dim,
                        int taps, void* out, int64_t out_ld, int fused_decode, int dtype, void* stream);
+/* The same with its 35 arguments as 64-bit words in their order, eps as a double: one argument to hand over instead of 35. */
+int semipd_state_space_record(const void* record);
 /* fp32 elements that semipd_state_space_prompt wants as `chunk_work` to take a batch in chunks of 32 tokens (0: it would not). */
 int64_t semipd_state_space_chunk_elems(int64_t num_tokens, int64_t batch, int num_heads, int groups, int state, int taps);
 /* semipd_state_space of a prompt batch (q_start given) with room for the operands of its chunks, 16-byte aligned: 32 tokens at a

@@ -23,6 +23,8 @@
 //  * delta_post_kernel / delta_post_vec_kernel: o / rms(o) * weight * silu(gate) -> the output projection's input, a workgroup per token.
 //  * delta_step_kernel / delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, key
 //    head) where the state lies on 16-byte boundaries, else per (request, head).
+#include <cstring>
+
 #include "common.h"
 #include "recurrent_chunks.h"
 
@@ -1776,7 +1778,8 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
                    "delta_rule: %d heads over %d q / k heads", num_heads, num_k_heads);
   SEMIPD_CHECK_ARG(k_dim > 0 && k_dim <= 256 && v_dim > 0 && taps >= 1 && taps <= 64, SEMIPD_ESHAPE,
                    "delta_rule: key size %d (at most 256), value size %d, %d taps (1 .. 64)", k_dim, v_dim, taps);
-  SEMIPD_CHECK_ARG(proj && conv_q && conv_k && conv_v && a_log && dt_bias && norm_weight && work && state && state_indices &&
+  const bool in_one = q_start == nullptr && (k_dim >= 32 ? 4 : 1) * (int64_t)v_dim <= 1024;       // (decode batches that need no work rows)
+  SEMIPD_CHECK_ARG(proj && conv_q && conv_k && conv_v && a_log && dt_bias && norm_weight && (work || in_one) && state && state_indices &&
                        seq_lens && out && (conv_state || taps == 1),
                    SEMIPD_EINVAL, "delta_rule: null pointer");
   SEMIPD_CHECK_ARG((q_start == nullptr) == (q_len == nullptr), SEMIPD_EINVAL, "delta_rule: q_start and q_len come together");
@@ -1784,7 +1787,7 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
   const int64_t C = 2 * (int64_t)num_k_heads * k_dim + (int64_t)num_heads * v_dim;
   const int64_t want = q_start ? semipd_delta_rule_chunk_elems(num_tokens, batch, num_heads, num_k_heads, k_dim, taps) : 0;
   const bool chunks = want > 0 && chunk_work && chunk_elems >= want && aligned16(chunk_work);
-  SEMIPD_CHECK_ARG(work_ld >= (chunks ? (int64_t)num_heads * v_dim : C + 2 * num_heads) && state_ld >= (int64_t)num_heads * k_dim * v_dim &&
+  SEMIPD_CHECK_ARG((in_one || work_ld >= (chunks ? (int64_t)num_heads * v_dim : C + 2 * num_heads)) && state_ld >= (int64_t)num_heads * k_dim * v_dim &&
                        (taps == 1 || conv_ld >= (taps - 1) * C) && out_ld >= (int64_t)num_heads * v_dim,
                    SEMIPD_EINVAL, "delta_rule: a row of the work buffer, the state or the output is too short");
   DeltaArgs a{proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight,
@@ -1893,6 +1896,19 @@ extern "C" int semipd_delta_rule(const void* proj, int64_t ld, int64_t q_off, in
   return delta_rule(proj, ld, q_off, k_off, v_off, gate_off, a_off, b_off, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, eps, work, work_ld,
                     state, state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, num_k_heads, k_dim,
                     v_dim, taps, out, out_ld, nullptr, 0, dtype, stream);
+}
+
+extern "C" int semipd_delta_rule_record(const void* record) {
+  SEMIPD_CHECK_ARG(record != nullptr, SEMIPD_EINVAL, "delta_rule: null record");
+  int64_t r[36];
+  double eps;
+  memcpy(r, record, sizeof(r));
+  memcpy(&eps, &r[14], sizeof(eps));
+  auto at = [&](int i) { return reinterpret_cast<void*>(r[i]); };
+  return semipd_delta_rule(at(0), r[1], r[2], r[3], r[4], r[5], r[6], r[7], at(8), at(9), at(10), (const float*)at(11), (const float*)at(12), at(13), (float)eps,
+                           (float*)at(15), r[16], (float*)at(17), r[18], (float*)at(19), r[20], (const int64_t*)at(21), (const int64_t*)at(22),
+                           (const int32_t*)at(23), (const int32_t*)at(24), r[25], r[26], (int)r[27], (int)r[28], (int)r[29], (int)r[30], (int)r[31], at(32), r[33],
+                           (int)r[34], at(35));
 }
 
 extern "C" int semipd_delta_rule_prompt(const void* proj, int64_t ld, int64_t q_off, int64_t k_off, int64_t v_off, int64_t gate_off,

@@ -24,6 +24,8 @@
 //  * ssm_post_kernel / ssm_post_vec_kernel: gate, grouped norm, weight -> the output projection's input, a workgroup per token.
 //  * ssm_step_kernel: batches of one token per request in place of preparation and recurrence, a workgroup per (head, request).
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
+#include <cstring>
+
 #include "common.h"
 #include "recurrent_chunks.h"
 
@@ -1573,6 +1575,19 @@ extern "C" int semipd_state_space(const void* proj, int64_t ld, int64_t z_off, i
   return state_space(proj, ld, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_w, norm_groups, eps, work, work_ld, state,
                      state_ld, conv_state, conv_ld, state_indices, seq_lens, q_start, q_len, batch, num_tokens, num_heads, groups,
                      state_size, v_dim, taps, out, out_ld, fused_decode, nullptr, 0, dtype, stream);
+}
+
+extern "C" int semipd_state_space_record(const void* record) {
+  SEMIPD_CHECK_ARG(record != nullptr, SEMIPD_EINVAL, "state_space: null record");
+  int64_t r[35];
+  double eps;
+  memcpy(r, record, sizeof(r));
+  memcpy(&eps, &r[12], sizeof(eps));
+  auto at = [&](int i) { return reinterpret_cast<void*>(r[i]); };
+  return semipd_state_space(at(0), r[1], r[2], r[3], r[4], at(5), at(6), (const float*)at(7), (const float*)at(8), (const float*)at(9), at(10), (int)r[11],
+                            (float)eps, (float*)at(13), r[14], (float*)at(15), r[16], (float*)at(17), r[18], (const int64_t*)at(19), (const int64_t*)at(20),
+                            (const int32_t*)at(21), (const int32_t*)at(22), r[23], r[24], (int)r[25], (int)r[26], (int)r[27], (int)r[28], (int)r[29], at(30), r[31],
+                            (int)r[32], (int)r[33], at(34));
 }
 
 extern "C" int semipd_state_space_prompt(const void* proj, int64_t ld, int64_t z_off, int64_t x_off, int64_t dt_off, const void* conv_w,

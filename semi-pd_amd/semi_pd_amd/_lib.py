@@ -174,6 +174,7 @@ _SIGNATURES = {
                                 _i32, _f32, _vp, _i32, _vp, _i32, _i32, _vp],
     "semipd_delta_rule": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _i64,
                           _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _vp],
+    "semipd_delta_rule_record": [C.c_char_p],
     "semipd_delta_rule_chunk_elems": [_i64, _i64, _i32, _i32, _i32, _i32],
     "semipd_delta_rule_prompt": [_vp, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _f32, _vp, _i64, _vp, _i64,
                           _vp, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64, _i32, _vp],
@@ -193,6 +194,7 @@ _SIGNATURES = {
     "semipd_state_space_work_width": [_i32, _i32, _i32, _i32],
     "semipd_state_space": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _i64, _vp, _i64, _vp, _i64,
                            _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _i32, _i32, _vp],
+    "semipd_state_space_record": [C.c_char_p],
     "semipd_state_space_chunk_elems": [_i64, _i64, _i32, _i32, _i32, _i32],
     "semipd_state_space_prompt": [_vp, _i64, _i64, _i64, _i64, _vp, _vp, _vp, _vp, _vp, _vp, _i32, _f32, _vp, _i64, _vp, _i64, _vp, _i64,
                                   _vp, _vp, _vp, _vp, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _vp, _i64, _vp, _i64, _i32, _vp],

@@ -13,6 +13,7 @@ launches on torch's *current* stream and never synchronises.
 from __future__ import annotations
 
 import os
+import struct
 from typing import Optional, Tuple
 
 import torch
@@ -1793,6 +1794,56 @@ def _chunk_room(tokens: int, width: int, elems: int, device):
         return None, None
 
 
+# The arguments of a recurrence's call as one record of 64-bit words.
+_DELTA_RECORD, _SSM_RECORD = struct.Struct("14qd21q"), struct.Struct("12qd22q")
+
+
+def _delta_rule_step(proj, offsets, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, eps, state, conv_state, state_indices, seq_lens,
+                     num_heads, num_k_heads, k_dim, v_dim, out):
+    """A decode batch of delta_rule whose arguments are in order, without work rows and with one argument to hand over; None where they are
+    not, or where work rows are needed: the general path then says what is wrong.  Python's share of a
+    call 12.3 -> 6.9 us, 3 requests, 32 heads of 64 x 64, whole call 16.9 -> 10.9 (device 9.6)."""
+    dt = proj.dtype
+    code = _lib._DTYPE_CODE.get(dt)
+    if proj.dim() != 2 or code is None or conv_state is None or conv_q.dim() != 2 or len(offsets) != 6:
+        return None
+    (T, width), (ld, step), taps = proj.shape, proj.stride(), conv_q.shape[1]
+    gd, hv = num_k_heads * k_dim, num_heads * v_dim
+    if step != 1 or taps < 2 or v_dim > (256 if k_dim >= 32 else 1024):
+        return None
+    if conv_q.shape != (gd, taps) or conv_k.shape != (gd, taps) or conv_v.shape != (hv, taps) or a_log.shape != (num_heads,) \
+            or dt_bias.shape != (num_heads,) or norm_weight.shape != (v_dim,) or state_indices.shape != (T,) or seq_lens.shape != (T,) \
+            or state.dim() != 2 or state.shape[1] != hv * k_dim or conv_state.dim() != 2 or conv_state.shape[1] != (taps - 1) * (2 * gd + hv):
+        return None
+    if not (conv_q.dtype == conv_k.dtype == conv_v.dtype == norm_weight.dtype == dt
+            and a_log.dtype == dt_bias.dtype == state.dtype == conv_state.dtype == torch.float32
+            and state_indices.dtype == seq_lens.dtype == torch.int64):
+        return None
+    if not (conv_q.is_contiguous() and conv_k.is_contiguous() and conv_v.is_contiguous() and a_log.is_contiguous()
+            and dt_bias.is_contiguous() and norm_weight.is_contiguous()):
+        return None
+    (state_ld, step), (conv_ld, conv_step) = state.stride(), conv_state.stride()
+    q, k, v, gate, a, b = offsets
+    if step != 1 or conv_step != 1 or min(offsets) < 0 or max(q + gd, k + gd, v + hv, gate + hv, a + num_heads, b + num_heads) > width:
+        return None
+    if out is None:
+        out = proj.new_empty((T, hv))
+    elif out.shape != (T, hv) or out.dtype != dt or out.stride(1) != 1:
+        return None
+    p = [t.data_ptr() for t in (proj, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, state, conv_state, state_indices, seq_lens, out)
+         if t.is_cuda]
+    if len(p) != 12:
+        return None
+    try:
+        record = _DELTA_RECORD.pack(p[0], ld, q, k, v, gate, a, b, p[1], p[2], p[3], p[4], p[5], p[6], eps, 0, 0, p[7], state_ld, p[8], conv_ld,
+                                    p[9], p[10], 0, 0, T, T, num_heads, num_k_heads, k_dim, v_dim, taps, p[11], out.stride(0), code,
+                                    current_stream(proj.device))
+    except struct.error:                                            # (numbers of another kind)
+        return None
+    check(_lib.load().semipd_delta_rule_record(record), "delta_rule")
+    return out
+
+
 def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.Tensor, conv_v: torch.Tensor, a_log: torch.Tensor,
                dt_bias: torch.Tensor, norm_weight: torch.Tensor, eps: float, state: torch.Tensor, conv_state: Optional[torch.Tensor],
                state_indices: torch.Tensor, seq_lens: torch.Tensor, q_start: Optional[torch.Tensor], q_len: Optional[torch.Tensor],
@@ -1800,6 +1851,11 @@ def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.
     """The gated delta rule behind its projection GEMM (csrc/delta_rule.hip).  offsets = columns of q, k, v, gate, a, b in the
     rows of `proj`; conv_* [channels, taps]; a_log / dt_bias fp32 [H]; state fp32 [slots, H * k_dim * v_dim] and conv_state
     fp32 [slots, (taps - 1) * channels] are column ranges of the requests' state rows.  Returns [T, H * v_dim]."""
+    if q_start is None and q_len is None:
+        done = _delta_rule_step(proj, offsets, conv_q, conv_k, conv_v, a_log, dt_bias, norm_weight, eps, state, conv_state, state_indices,
+                                seq_lens, num_heads, num_k_heads, k_dim, v_dim, out)
+        if done is not None:
+            return done
     T, B = proj.shape[0], state_indices.shape[0]
     taps = conv_q.shape[1]
     gd, hv = num_k_heads * k_dim, num_heads * v_dim
@@ -2059,6 +2115,56 @@ def talk_mix(parts: torch.Tensor, talk: torch.Tensor, num_kv_heads: int, out: Op
 STATE_SPACE_FUSED_DECODE_BYTES = 128 << 10     # a request's state per layer up to which a decode batch takes the one-launch form
 
 
+def _state_space_step(proj, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_weight, norm_groups, eps, state, conv_state,
+                      state_indices, seq_lens, num_heads, groups, state_size, v_dim, out):
+    """A decode batch of state_space whose arguments are in order, with one argument to hand over; None where they are not: the general path
+    then says what is wrong.  Python's share of a call 11.7 -> 8.0 us, 2 requests, 64 heads of 128 x 64, whole call 19.2 -> 15.8."""
+    dt = proj.dtype
+    code = _lib._DTYPE_CODE.get(dt)
+    if proj.dim() != 2 or code is None or conv_state is None or conv_b is None or d_skip is None or conv_w.dim() != 2:
+        return None
+    (T, width), (ld, step), taps = proj.shape, proj.stride(), conv_w.shape[1]
+    inner = num_heads * v_dim
+    channels = inner + 2 * groups * state_size
+    if step != 1 or taps < 2 or conv_w.shape != (channels, taps) or conv_b.shape != (channels,) or dt_bias.shape != (num_heads,) \
+            or a_log.shape != (num_heads,) or d_skip.shape != (num_heads,) or norm_weight.shape != (inner,) or state_indices.shape != (T,) \
+            or seq_lens.shape != (T,) or state.dim() != 2 or state.shape[1] != inner * state_size or conv_state.dim() != 2 \
+            or conv_state.shape[1] != (taps - 1) * channels:
+        return None
+    if not (conv_w.dtype == conv_b.dtype == norm_weight.dtype == dt
+            and dt_bias.dtype == a_log.dtype == d_skip.dtype == state.dtype == conv_state.dtype == torch.float32
+            and state_indices.dtype == seq_lens.dtype == torch.int64):
+        return None
+    if not (conv_w.is_contiguous() and conv_b.is_contiguous() and dt_bias.is_contiguous() and a_log.is_contiguous()
+            and d_skip.is_contiguous() and norm_weight.is_contiguous()):
+        return None
+    (state_ld, step), (conv_ld, conv_step) = state.stride(), conv_state.stride()
+    if step != 1 or conv_step != 1 or min(z_off, x_off, dt_off) < 0 or max(z_off + inner, x_off + channels, dt_off + num_heads) > width:
+        return None
+    if out is None:
+        out = proj.new_empty((T, inner))
+    elif out.shape != (T, inner) or out.dtype != dt or out.stride(1) != 1:
+        return None
+    p = [t.data_ptr() for t in (proj, conv_w, conv_b, dt_bias, a_log, d_skip, norm_weight, state, conv_state, state_indices, seq_lens, out)
+         if t.is_cuda]
+    if len(p) != 12:
+        return None
+    fused = inner * state_size * 4 <= STATE_SPACE_FUSED_DECODE_BYTES
+    work, work_ld = 0, 0
+    if not fused:
+        work_ld = -(-(channels + 2 * num_heads) // 4) * 4
+        rows = proj.new_empty((T, work_ld), dtype=torch.float32)
+        work = rows.data_ptr()
+    try:
+        record = _SSM_RECORD.pack(p[0], ld, z_off, x_off, dt_off, p[1], p[2], p[3], p[4], p[5], p[6], norm_groups, eps, work, work_ld, p[7], state_ld,
+                                  p[8], conv_ld, p[9], p[10], 0, 0, T, T, num_heads, groups, state_size, v_dim, taps, p[11], out.stride(0),
+                                  1 if fused else 0, code, current_stream(proj.device))
+    except struct.error:                                            # (numbers of another kind)
+        return None
+    check(_lib.load().semipd_state_space_record(record), "state_space")
+    return out
+
+
 def state_space(proj: torch.Tensor, z_off: int, x_off: int, dt_off: int, conv_w: torch.Tensor, conv_b: Optional[torch.Tensor],
                 dt_bias: torch.Tensor, a_log: torch.Tensor, d_skip: Optional[torch.Tensor], norm_weight: torch.Tensor,
                 norm_groups: int, eps: float, state: torch.Tensor, conv_state: Optional[torch.Tensor], state_indices: torch.Tensor,
@@ -2068,6 +2174,11 @@ def state_space(proj: torch.Tensor, z_off: int, x_off: int, dt_off: int, conv_w:
     convolution's channels x [H * E] | B [G * N] | C [G * N] at x_off, dt [H] at dt_off; conv_w [channels, taps], conv_b
     [channels]; dt_bias / a_log / d_skip fp32 [H]; norm_weight [H * E]; state fp32 [slots, H * N * E] and conv_state fp32
     [slots, (taps - 1) * channels] are column ranges of the requests' state rows.  Returns [T, H * E]."""
+    if q_start is None and q_len is None:
+        done = _state_space_step(proj, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log, d_skip, norm_weight, norm_groups, eps, state,
+                                 conv_state, state_indices, seq_lens, num_heads, groups, state_size, v_dim, out)
+        if done is not None:
+            return done
     T, B = proj.shape[0], state_indices.shape[0]
     inner = num_heads * v_dim
     C = inner + 2 * groups * state_size
