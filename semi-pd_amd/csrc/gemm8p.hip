@@ -30,6 +30,7 @@
 // replaces UnquantizedLinearMethod.apply -> F.linear (+ SiluAndMul) (layers/linear.py:165-172, models/llama.py:88-92,
 // layers/activation.py:41-53) for 65 .. 256-row decode batches, and _get_logits (layers/logits_processor.py:394-445).
 #include "common.h"
+#include "mfma_frag.h"
 
 #include <type_traits>
 
@@ -102,6 +103,7 @@ struct G8Group {
   const int32_t* num_post_pad;
   const float* topk_weights;
   int num_valid, top_k_div, mul_routed_weight;
+  uint32_t inverse;                            // (2^32 - 1) / top_k_div
 };
 
 template <typename T, int EPI, bool NT, int XH, bool GR = false, int ORDER = 0>
@@ -920,7 +922,7 @@ int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* top
                        aligned16(w) && (reinterpret_cast<uintptr_t>(c) & 7u) == 0 && num_valid < (1 << 30) && n < (1 << 30) &&
                        k < (1 << 30),
                    SEMIPD_ESHAPE, "moe_gemm_tall: block size 320, 256 or 128, k %% 64, output width %% 16 required");
-  G8Group grp{sorted_token_ids, expert_ids, num_tokens_post_pad, topk_weights, (int)num_valid, top_k_div, mul_routed_weight};
+  G8Group grp{sorted_token_ids, expert_ids, num_tokens_post_pad, topk_weights, (int)num_valid, top_k_div, mul_routed_weight, 0xffffffffu / (uint32_t)top_k_div};
   int rc = 0;
 #define G8G(EPIV, XHV) \
   SEMIPD_DISPATCH_HALF(dtype, T, rc = (g8_launch_grouped<T, EPIV, XHV>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k, k, n_out, as_stream(stream))))

@@ -16,6 +16,9 @@
 // products follow its rows in steps of 64.  64 experts, top 6, bf16, both products, tiles of 256 rows / this: 1000 tokens (94 rows an expert) 183 +
 // 95 / 167 + 81 us, 3001 (281) 296 + 182 / 220 + 115, 6000 (562) 477 + 265 / 391 + 208, 8192 572 + 332 / 523 + 294.  Results by way of LDS, in 256 bytes
 // of an entry instead of 32: second product of 3001 tokens 134 -> 115 us (74 MB of results).
+// Around the K loop nothing overlaps, one workgroup a CU: of 71 us of a tile 4 pass before the first products and 9 (SiLU) or 5 behind
+// the last.  So a lane has no division and one wait for its places and weights, conversions are in pairs, and what is staged past the end
+// or for padding is no access.  The layer, before / after, us: 1000 tokens 277 / 266, 2000 324 / 312, 3001 375 / 362, 6000 655 / 631, 8192 889 / 850.
 #pragma once
 
 namespace semipd {
@@ -44,6 +47,12 @@ template <bool ACC> __device__ __forceinline__ void rows_retire(g8_f32x4& a, g8_
   else asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 7" : "+v"(a), "+v"(b), "+v"(c), "+v"(d));
 }
 
+// the low or the high half of a pair, as a float
+template <typename T> __device__ __forceinline__ float half_of(uint32_t w, int high) {
+  if constexpr (std::is_same<T, bf16_t>::value) return __uint_as_float(high ? w & 0xffff0000u : w << 16);
+  else return Elem<T>::to_f(T{(uint16_t)(high ? w >> 16 : w)});
+}
+
 struct RowsTile {
   static constexpr int kRows = 320, kCols = 256;
   static constexpr int kXHalf = 160 * 128, kWHalf = 128 * 128;         // bytes of a half-tile
@@ -59,11 +68,17 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   const int wr = wave >> 1, wc = wave & 1;
   const int c16 = lane & 15, q4 = lane >> 4;
   const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N;
-  const int nkt = K >> 6, last_kt = nkt - 1;
+  const int nkt = K >> 6;
+
+  // an entry's row: id / top_k_div, by 2^32 / top_k_div and what is left (35 instructions fewer than the division, of which a lane has 2 NX)
+  const uint32_t div = grp.top_k_div, inverse = grp.inverse;
+  auto row_of = [&](uint32_t id) __attribute__((always_inline)) {
+    const uint32_t q = __umulhi(id, inverse);
+    return (int)(q + (id - q * div >= div));
+  };
 
   // ---- DMA sources: piece p of a half-tile is its LDS rows 8 p .. + 7, 128 bytes each; chunk c of row r at c ^ ((r >> 1) & 7) ----
-  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, (int)((int64_t)((grp.num_valid - 1) / grp.top_k_div + 1) * K * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc((void*)w, 0, (int)((int64_t)N * K * 2), 0x00020000);
+  const int x_bytes = (int)((int64_t)(row_of((uint32_t)grp.num_valid - 1) + 1) * K * 2), w_bytes = (int)((int64_t)N * K * 2);
   int off_x[2][NX], off_w[2][4];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
@@ -71,7 +86,8 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     for (int e = 0; e < NX; ++e) {
       const int rp = 8 * (wave * NX + e) + (lane >> 3);
       const int id = grp.sorted_ids[m0 + 32 * NX * h + rp];
-      off_x[h][e] = ((id < grp.num_valid ? id / grp.top_k_div : 0) * K + (((lane & 7) ^ ((rp >> 1) & 7)) << 3)) * 2;     // (padding reads row 0)
+      // (padding lies behind the operand's end: zeros that nobody fetches, and products that take little power)
+      off_x[h][e] = id < grp.num_valid ? (row_of((uint32_t)id) * K + (((lane & 7) ^ ((rp >> 1) & 7)) << 3)) * 2 : (int)0x80000000;
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -81,16 +97,18 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     }
   }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)smem;
-  // piece e of this wave's share of half-tile HALF (0: x0, 1: x1, 2: W0, 3: W1) of K step kt (past the end: the last step again)
+  // piece e of this wave's share of half-tile HALF (0: x0, 1: x1, 2: W0, 3: W1) of K step kt.  Past the end, where the waits still count
+  // its loads, the operand has no bytes: nothing is fetched for them.
   auto stage1 = [&](auto half_c, auto e_c, int kt) __attribute__((always_inline)) {
     constexpr int HALF = decltype(half_c)::value, E = decltype(e_c)::value;
-    const int k = min(kt, last_kt) * 128;
+    const int k = kt < nkt ? kt * 128 : 0;
+    const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc((void*)(HALF < 2 ? x : w), 0, kt < nkt ? (HALF < 2 ? x_bytes : w_bytes) : 0, 0x00020000);
     const uint32_t at = lds0 + (kt & 1) * R::kParity;
     if constexpr (HALF < 2)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (__attribute__((address_space(3))) void*)(uintptr_t)(at + HALF * R::kXHalf + (wave * NX + E) * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(uintptr_t)(at + HALF * R::kXHalf + (wave * NX + E) * 1024), 16,
                                                off_x[HALF][E], k, 0, 0);
     else
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (__attribute__((address_space(3))) void*)(uintptr_t)(at + 2 * R::kXHalf + (HALF - 2) * R::kWHalf + (wave * 4 + E) * 1024),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(uintptr_t)(at + 2 * R::kXHalf + (HALF - 2) * R::kWHalf + (wave * 4 + E) * 1024),
                                                16, off_w[HALF - 2][E], k, 0, NT ? 2 : 0);
   };
   auto stage = [&](auto half_c, int kt) __attribute__((always_inline)) {
@@ -147,20 +165,20 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   using IX = std::integral_constant<int, NX>;
   using J4 = std::integral_constant<int, 4>;
 
-  stage(H0{}, 0), stage(H2{}, 0), stage(H3{}, 0), stage(H1{}, 0), stage(H0{}, 1), stage(H3{}, 1), stage(H2{}, 1), stage(H1{}, 1);
-  g8_wait_vm<kAll - NX>();
+  // (the first weights do not wait for the entries' rows)
+  stage(H2{}, 0), stage(H3{}, 0), stage(H0{}, 0), stage(H1{}, 0), stage(H0{}, 1), stage(H3{}, 1), stage(H2{}, 1), stage(H1{}, 1);
+  g8_wait_vm<kAll - NX - 8>();
   g8_barrier();
   rows_for<0, NX>([&](auto f) __attribute__((always_inline)) {
     fx0[decltype(f)::value][0].u = g8_lds_read16(xa + off_s[0], decltype(f)::value * 2048);
     fx0[decltype(f)::value][1].u = g8_lds_read16(xa + off_s[1], decltype(f)::value * 2048);
   });
-  g8_wait_vm<XW::value>();
-  g8_wait_lgkm0();
-  g8_barrier();
   rows_for<0, 4>([&](auto f) __attribute__((always_inline)) {
     fw0[decltype(f)::value][0].u = g8_lds_read16(wa + off_s[0], decltype(f)::value * 2048);
     fw0[decltype(f)::value][1].u = g8_lds_read16(wa + off_s[1], decltype(f)::value * 2048);
   });
+  g8_wait_lgkm0();
+  g8_barrier();
   stage(H0{}, 2);
 
   for (int kt = 0; kt < nkt; kt += 2) {                                // (an even count of K steps: the caller sees to it)
@@ -174,53 +192,60 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     phase(XX{}, fx0, xa + pa, H1{}, kt + 3, fx1, fw0, IX{}, H0{});                  // reads x0(kt + 2); x1(kt + 1) -> x1(kt + 3)
     phase(XW{}, fw0, wa + pa, H0{}, kt + 4, fx1, fw1, IX{}, J4{});                  // reads W0(kt + 2); x0(kt + 2) -> x0(kt + 4)
   }
-  g8_wait_vm<0>();                    // no DMA may land in LDS that the next workgroup owns
-  g8_wait_lgkm0();
-  rows_for<0, NX>([&](auto i_c) __attribute__((always_inline)) {
-    constexpr int I = NX + decltype(i_c)::value;
-    rows_retire<(I < 8)>(acc[I][4], acc[I][5], acc[I][6], acc[I][7]);
-  });
-
   // ---- epilogue: lane holds, of entry m0 + 32 NX h + 16 NX wr + 16 i + c16, columns 16 j + 4 q4 .. + 3 of its wave's.  A half's rows go
-  //      through the wave's own quarter of the LDS and leave whole: 256 bytes of an entry (128 of SiLU * up) instead of 32 a store ----
+  //      through the wave's own quarter of the LDS and leave whole: 256 bytes of an entry (128 of SiLU * up) instead of 32 a store.  All
+  //      entries' places, and their weights, are asked for together ----
   constexpr int WCOLS = EPI == G8_SILU_MUL ? 64 : 128, LPR = WCOLS / 8, RPS = 64 / LPR;      // lanes a row, rows a store
   constexpr int OS = WCOLS * 2 + 16;                                                            // bytes between rows in LDS
   static_assert(16 * NX * OS <= R::kLds / 4, "a half's rows fit the wave's quarter");
   char* const mine = smem + wave * (R::kLds / 4);
-  g8_barrier();                       // everybody has read its last fragments and has no DMA in flight
+  int to[2][16 * NX / RPS], entry[2][NX];
+  float weight[2][NX];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int32_t* ids = grp.sorted_ids + m0 + 32 * NX * h + 16 * NX * wr;
-    int to[16 * NX / RPS];
 #pragma unroll
-    for (int u = 0; u < 16 * NX / RPS; ++u) to[u] = ids[RPS * u + lane / LPR];
+    for (int i = 0; i < NX; ++i) entry[h][i] = EPI == G8_PLAIN ? ids[16 * i + c16] : 0;
+#pragma unroll
+    for (int u = 0; u < 16 * NX / RPS; ++u) to[h][u] = ids[RPS * u + lane / LPR];
+  }
+  g8_wait_vm<0>();                    // no DMA may land in LDS that the next workgroup owns
+  g8_wait_lgkm0();
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int i = 0; i < NX; ++i) weight[h][i] = EPI == G8_PLAIN && grp.mul_routed_weight ? grp.topk_weights[min(entry[h][i], grp.num_valid - 1)] : 1.f;   // (padding has none and is not stored)
+  rows_for<0, NX>([&](auto i_c) __attribute__((always_inline)) {
+    constexpr int I = NX + decltype(i_c)::value;
+    rows_retire<(I < 8)>(acc[I][4], acc[I][5], acc[I][6], acc[I][7]);
+  });
+  g8_barrier();                       // everybody has read its last fragments and has no DMA in flight
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
-      float scale = 1.f;
-      if (EPI == G8_PLAIN && grp.mul_routed_weight) {
-        const int id = ids[16 * i + c16];
-        scale = id < grp.num_valid ? grp.topk_weights[id] : 1.f;
-      }
+      const float scale = weight[h][i];
 #pragma unroll
       for (int j = 0; j < WCOLS / 16; ++j) {
         float r[4];
         if (EPI == G8_SILU_MUL) {
           // the unfused pair rounds the GEMM output to T before the activation reads it
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float gq = Elem<T>::to_f(Elem<T>::from_f(acc[NX * h + i][j][e]));
-            const float uq = Elem<T>::to_f(Elem<T>::from_f(acc[NX * h + i][(EPI == G8_SILU_MUL ? 4 : 0) + j][e]));
-            r[e] = gq / (1.f + __expf(-gq)) * uq;
-            asm volatile("" : "+v"(r[e]));   // (see gemm8p_kernel's epilogue: two roundings, not one fused one)
+          for (int e = 0; e < 4; e += 2) {
+            const g8_f32x4 &gate = acc[NX * h + i][j], &up = acc[NX * h + i][(EPI == G8_SILU_MUL ? 4 : 0) + j];
+            const uint32_t g2 = pack2<T>(gate[e], gate[e + 1]), u2 = pack2<T>(up[e], up[e + 1]);
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+              const float gq = half_of<T>(g2, b), uq = half_of<T>(u2, b);
+              r[e + b] = gq / (1.f + __expf(-gq)) * uq;
+              asm volatile("" : "+v"(r[e + b]));   // (see gemm8p_kernel's epilogue: two roundings, not one fused one)
+            }
           }
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e) r[e] = acc[NX * h + i][j][e] * scale;
         }
-        uint2 p;
-        p.x = (uint32_t)Elem<T>::from_f(r[0]).v | ((uint32_t)Elem<T>::from_f(r[1]).v << 16);
-        p.y = (uint32_t)Elem<T>::from_f(r[2]).v | ((uint32_t)Elem<T>::from_f(r[3]).v << 16);
-        *reinterpret_cast<uint2*>(mine + (16 * i + c16) * OS + j * 32 + q4 * 8) = p;
+        *reinterpret_cast<uint2*>(mine + (16 * i + c16) * OS + j * 32 + q4 * 8) = uint2{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3])};
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -230,7 +255,7 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
 #pragma unroll
     for (int u = 0; u < 16 * NX / RPS; ++u) {
       const uint4 v = *reinterpret_cast<const uint4*>(mine + (RPS * u + lane / LPR) * OS + lane % LPR * 16);
-      if (to[u] < grp.num_valid && n < n_cols) *reinterpret_cast<uint4*>(out + (int64_t)to[u] * n_cols + n) = v;
+      if (to[h][u] < grp.num_valid && n < n_cols) *reinterpret_cast<uint4*>(out + (int64_t)to[h][u] * n_cols + n) = v;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
