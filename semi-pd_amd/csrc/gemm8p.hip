@@ -29,54 +29,9 @@
 // the same columns), fp32 K-slice planes for split-K.
 // replaces UnquantizedLinearMethod.apply -> F.linear (+ SiluAndMul) (layers/linear.py:165-172, models/llama.py:88-92,
 // layers/activation.py:41-53) for 65 .. 256-row decode batches, and _get_logits (layers/logits_processor.py:394-445).
-#include "common.h"
-#include "mfma_frag.h"
-
-#include <type_traits>
+#include "gemm8p_parts.h"
 
 namespace semipd {
-
-typedef float g8_f32x4 __attribute__((ext_vector_type(4)));
-typedef __bf16 g8_bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 g8_f16x8 __attribute__((ext_vector_type(8)));
-
-union G8Frag {
-  uint4 u;
-  g8_bf16x8 b;
-  g8_f16x8 f;
-};
-template <typename T> struct G8Mfma;
-template <> struct G8Mfma<bf16_t> {
-  __device__ static inline g8_f32x4 mma(const G8Frag& a, const G8Frag& b, g8_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, b.b, c, 0, 0, 0);
-  }
-};
-template <> struct G8Mfma<f16_t> {
-  __device__ static inline g8_f32x4 mma(const G8Frag& a, const G8Frag& b, g8_f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a.f, b.f, c, 0, 0, 0);
-  }
-};
-
-enum { G8_PLAIN = 0, G8_SILU_MUL = 1 };
-
-#define G8_GLDS(gp, lp, aux) \
-  __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gp), \
-                                   (__attribute__((address_space(3))) void*)(lp), 16, 0, aux)
-
-__device__ inline uint4 g8_lds_read16(uint32_t addr, int imm) {
-  uint4 v;
-  asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(imm));
-  return v;
-}
-template <int N> __device__ inline void g8_wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-__device__ inline void g8_wait_lgkm0() {
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-__device__ inline void g8_barrier() {
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // Geometry of a tile: XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
 // tile for 65 .. 128 rows -- the same 32 accumulator tiles and 16 MFMAs per phase per wave, twice the weight rows per
@@ -93,19 +48,6 @@ template <int XH> struct G8Geo {
 };
 
 // NT: the weight tile is used by this workgroup only (one row of tiles): stream it non-temporally past L2 / MALL
-// Grouped form (GR; fused-MoE expert GEMMs, fused_moe.py:54-273): the x tile is 2 XH consecutive entries of
-// sorted_token_ids (moe_align_block_size with block size 2 XH: one expert per tile, expert_ids[tile]); entry id reads
-// activation row id / top_k_div and writes output row id (entries >= num_valid are padding), optionally scaled by
-// topk_weights[id]; W = w[expert].
-struct G8Group {
-  const int32_t* sorted_ids;
-  const int32_t* expert_ids;
-  const int32_t* num_post_pad;
-  const float* topk_weights;
-  int num_valid, top_k_div, mul_routed_weight;
-  uint32_t inverse;                            // (2^32 - 1) / top_k_div
-};
-
 template <typename T, int EPI, bool NT, int XH, bool GR = false, int ORDER = 0>
 __global__ void __launch_bounds__(512)
 gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restrict__ x, const T* __restrict__ w, int M, int N,
@@ -412,23 +354,6 @@ gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
 //     7 phases (~2 us of matrix work) of flight, six younger half-tiles behind every wait: s_waitcnt vmcnt(24);
 //   * phase = { vmcnt(24): my share of the half to read now; lgkmcnt(0): last phase's reads; s_barrier; 8 ds_read_b128;
 //     4 DMA; 32 MFMAs }.
-// The MFMAs of the 4-wave kernel as inline asm with the accumulator tile tied to an ACCUMULATION register ("+a"): 256 of the
-// wave's 512 registers are accumulators, and left to itself the register allocator moves fragments into the accumulation half
-// too, spills accumulators and copies them around (1.2 KB of scratch per lane, ~370 v_accvgpr moves inside the K loop in the
-// first build).  With the classes fixed -- accumulators in a[0:255], fragments and addresses in v[0:255] -- nothing spills.
-// asm volatile also keeps the issue order of a phase: the fragment reads and the DMA first, then the 32 MFMAs.
-template <typename T> struct G4Mfma;
-template <> struct G4Mfma<bf16_t> {
-  __device__ static inline void mma(g8_f32x4& c, const G8Frag& a, const G8Frag& b) {
-    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a.b), "v"(b.b));
-  }
-};
-template <> struct G4Mfma<f16_t> {
-  __device__ static inline void mma(g8_f32x4& c, const G8Frag& a, const G8Frag& b) {
-    asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a.f), "v"(b.f));
-  }
-};
-
 template <typename T, int EPI, bool NT, bool GR = false, int ORDER = 0>
 __global__ void __launch_bounds__(256)
 gemm4w_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restrict__ x, const T* __restrict__ w, int M, int N,
@@ -655,10 +580,6 @@ gemm4w_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restri
   }
 }
 
-}  // namespace semipd
-#include "moe_gemm_rows.h"
-namespace semipd {
-
 // out[m, n] = T(sum_z planes[z][m][n]) in slice order (SiLU * mul variant: gate / up columns n, n + N / 2)
 template <typename T, int EPI>
 __global__ void __launch_bounds__(256)
@@ -794,17 +715,6 @@ static int g8_launch(T* out, float* planes, size_t planes_bytes, const T* x, con
   return g8_launch_geo<T, EPI, 128>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks);
 }
 
-template <typename T, int EPI>
-static int g8_launch_rows(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, hipStream_t st) {
-  const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N, cols_per_tile = EPI == G8_SILU_MUL ? RowsTile::kCols / 2 : RowsTile::kCols;
-  const int64_t tiles = max_sorted / RowsTile::kRows * ((n_cols + cols_per_tile - 1) / cols_per_tile);
-  // (an XCD's share of the tiles and its share of those that come last are rounded up apart)
-  static std::atomic<uint64_t> lds_ok{0};
-  if (ensure_dynamic_lds((const void*)moe_gemm_rows_kernel<T, EPI>, RowsTile::kLds, lds_ok, "moe_gemm_rows")) return 1;
-  hipLaunchKernelGGL((moe_gemm_rows_kernel<T, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8 + 8)), dim3(256), RowsTile::kLds, st, c, a, w, N, K, grp);
-  return launch_status("moe_gemm_rows");
-}
-
 template <typename T, int EPI, int XH>
 static int g8_launch_grouped(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, int64_t lda,
                              int64_t ldc, hipStream_t st) {
@@ -916,7 +826,7 @@ int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* top
                    "moe_gemm_tall: null pointer");
   SEMIPD_CHECK_ARG(!mul_routed_weight || topk_weights, SEMIPD_EINVAL, "moe_gemm_tall: topk_weights required");
   const int64_t n_out = fuse_silu_mul ? n / 2 : n;
-  SEMIPD_CHECK_ARG(block_m != RowsTile::kRows || (k % 128 == 0 && aligned16(c) && n * k < (1 << 30) && ((num_valid - 1) / top_k_div + 1) * k < (1 << 30)), SEMIPD_ESHAPE,
+  SEMIPD_CHECK_ARG(block_m != kMoeRowsTile || (k % 128 == 0 && aligned16(c) && n * k < (1 << 30) && ((num_valid - 1) / top_k_div + 1) * k < (1 << 30)), SEMIPD_ESHAPE,
                    "moe_gemm_tall: blocks of 320 rows need k %% 128, a 16-byte aligned output and operands below 2 GiB");
   SEMIPD_CHECK_ARG((block_m == 320 || block_m == 256 || block_m == 128) && max_sorted % block_m == 0 && k % 64 == 0 && n_out % 16 == 0 && (!fuse_silu_mul || n % 2 == 0) && aligned16(a) &&
                        aligned16(w) && (reinterpret_cast<uintptr_t>(c) & 7u) == 0 && num_valid < (1 << 30) && n < (1 << 30) &&
@@ -926,10 +836,9 @@ int semipd_moe_gemm_tall(void* c, const void* a, const void* w, const float* top
   int rc = 0;
 #define G8G(EPIV, XHV) \
   SEMIPD_DISPATCH_HALF(dtype, T, rc = (g8_launch_grouped<T, EPIV, XHV>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k, k, n_out, as_stream(stream))))
-  if (block_m == RowsTile::kRows) {
-#define G8R(EPIV) SEMIPD_DISPATCH_HALF(dtype, T, rc = (g8_launch_rows<T, EPIV>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k, as_stream(stream))))
-    if (fuse_silu_mul) { G8R(G8_SILU_MUL); } else { G8R(G8_PLAIN); }
-#undef G8R
+  if (block_m == kMoeRowsTile) {
+    SEMIPD_DISPATCH_HALF(dtype, T, rc = (launch_moe_gemm_rows<T>((T*)c, (const T*)a, (const T*)w, grp, max_sorted, (int)n, (int)k,
+                                                                 fuse_silu_mul ? G8_SILU_MUL : G8_PLAIN, as_stream(stream))))
   } else if (block_m == 256) {
     if (fuse_silu_mul) { G8G(G8_SILU_MUL, 128); } else { G8G(G8_PLAIN, 128); }
   } else {

@@ -1,25 +1,28 @@
 // Grouped GEMM of the experts, up to 320 routed rows x 256 weight rows a workgroup (gfx950): gemm4w_kernel's tile with as many row
-// fragments as the tile's expert has rows for.  Included by gemm8p.hip behind what it needs (G8Frag, G4Mfma, G8Group, the waits).
+// fragments as the tile's expert has rows for.  Compiled in moe_gemm_rows_bf16.hip and _f16.hip.
 //
 //   c[id] = a[id / top_k_div] @ w[expert]^T  for the entries id of sorted_ids, 320 of one expert at a time (moe_align_block_size)
 //
-//  * Four waves, 2 x 2, one a SIMD; a wave owns 32 NX entries x 128 weight rows, NX = 2 .. 5 row fragments of 16 a half: 128, 192, 256
-//    or 320 entries a tile, whichever the expert fills (chosen by the workgroup from its entries; a body each).
+//  * Four waves, 2 x 2, one a SIMD; a wave owns 16 (NX0 + NX1) entries x 128 weight rows, NX0 and NX1 = 2 .. 5 row fragments of 16 in the
+//    first half and the second, as many or one less: 128, 160, ... 320 entries a tile, whichever the expert fills (chosen by the workgroup
+//    from its entries; a body each).
 //  * K in steps of 64.  The operands of a step are four half-tiles in LDS (x0, x1 of 32 NX entries, W0, W1 of 128 weight rows; SiLU * up:
 //    W0 gate rows, W1 up rows of the same columns), two steps' worth of them: 144 KB.  Phases, order of the half-tiles, swizzle and
-//    waits are those of gemm4w_kernel; loads in flight behind a wait are counted with NX a wave for an x half and 4 for a W half.
-//  * Accumulators: 16 NX tiles of 4 registers; 64 of them fill the accumulation half of the register file, the 16 of NX = 5 behind
+//    waits are those of gemm4w_kernel; loads in flight behind a wait are counted with NX0 or NX1 a wave for an x half and 4 for a W half.
+//  * Accumulators: 8 (NX0 + NX1) tiles of 4 registers; 64 of them fill the accumulation half of the register file, those behind
 //    that are ordinary registers.
-// Bound: the flight of its loads: 64 KB + of a step in LDS twice is all there is room for, 108 KB of it in flight, and behind 94 to 281
-// rows an expert's weights come from HBM once (738 MB of 64 experts of 2816 x 2048: 147 us of a read's time).  Why 320 rows: a second,
-// nearly empty tile of 256 took 0.4 of a full one; 320 accumulator registers and 144 KB of LDS are what a CU holds.  Why bodies: a wave's
-// products follow its rows in steps of 64.  64 experts, top 6, bf16, both products, tiles of 256 rows / this: 1000 tokens (94 rows an expert) 183 +
-// 95 / 167 + 81 us, 3001 (281) 296 + 182 / 220 + 115, 6000 (562) 477 + 265 / 391 + 208, 8192 572 + 332 / 523 + 294.  Results by way of LDS, in 256 bytes
-// of an entry instead of 32: second product of 3001 tokens 134 -> 115 us (74 MB of results).
+// Bound: the flight of its loads: 64 KB + of a step in LDS twice is all there is room for, 108 KB of it in flight, and behind 94 to 281 rows
+// an expert's weights come from HBM once (738 MB of 64 experts of 2816 x 2048: 147 us of a read's time).  Why 320 rows: a second, nearly
+// empty tile of 256 took 0.4 of a full one; 320 accumulator registers and 144 KB of LDS are what a CU holds.  Why bodies: a wave's products
+// follow its rows in steps of 32 (of 64 before: the layer of 2000 tokens 312 -> 307 us, 3001 362 -> 357, 6000 631 -> 617).  64 experts, top
+// 6, bf16, both products, tiles of 256 rows / this: 1000 tokens (94 rows an expert) 183 + 95 / 167 + 81 us, 3001 (281) 296 + 182 / 220 +
+// 115, 6000 (562) 477 + 265 / 391 + 208, 8192 572 + 332 / 523 + 294.  Results by way of LDS, in 256 bytes of an entry instead of 32: second
+// product of 3001 tokens 134 -> 115 us (74 MB of results).
 // Around the K loop nothing overlaps, one workgroup a CU: of 71 us of a tile 4 pass before the first products and 9 (SiLU) or 5 behind
 // the last.  So a lane has no division and one wait for its places and weights, conversions are in pairs, and what is staged past the end
 // or for padding is no access.  The layer, before / after, us: 1000 tokens 277 / 266, 2000 324 / 312, 3001 375 / 362, 6000 655 / 631, 8192 889 / 850.
 #pragma once
+#include "gemm8p_parts.h"
 
 namespace semipd {
 
@@ -54,12 +57,12 @@ template <typename T> __device__ __forceinline__ float half_of(uint32_t w, int h
 }
 
 struct RowsTile {
-  static constexpr int kRows = 320, kCols = 256;
+  static constexpr int kRows = kMoeRowsTile, kCols = 256;
   static constexpr int kXHalf = 160 * 128, kWHalf = 128 * 128;         // bytes of a half-tile
   static constexpr int kParity = 2 * (kXHalf + kWHalf), kLds = 2 * kParity;
 };
 
-template <typename T, int EPI, int NX, bool NT>
+template <typename T, int EPI, int NX0, int NX1, bool NT>
 __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, const T* __restrict__ x, const T* __restrict__ w, int N, int K,
                                               int m0, int n0, const G8Group& grp) {
   using R = RowsTile;
@@ -69,6 +72,7 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   const int c16 = lane & 15, q4 = lane >> 4;
   const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N;
   const int nkt = K >> 6;
+  static_assert(NX0 >= NX1 && NX0 <= 5, "the first half is the longer one");
 
   // an entry's row: id / top_k_div, by 2^32 / top_k_div and what is left (35 instructions fewer than the division, of which a lane has 2 NX)
   const uint32_t div = grp.top_k_div, inverse = grp.inverse;
@@ -79,13 +83,13 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
 
   // ---- DMA sources: piece p of a half-tile is its LDS rows 8 p .. + 7, 128 bytes each; chunk c of row r at c ^ ((r >> 1) & 7) ----
   const int x_bytes = (int)((int64_t)(row_of((uint32_t)grp.num_valid - 1) + 1) * K * 2), w_bytes = (int)((int64_t)N * K * 2);
-  int off_x[2][NX], off_w[2][4];
+  int off_x[2][NX0], off_w[2][4];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
 #pragma unroll
-    for (int e = 0; e < NX; ++e) {
-      const int rp = 8 * (wave * NX + e) + (lane >> 3);
-      const int id = grp.sorted_ids[m0 + 32 * NX * h + rp];
+    for (int e = 0; e < (h ? NX1 : NX0); ++e) {
+      const int rp = 8 * (wave * (h ? NX1 : NX0) + e) + (lane >> 3);
+      const int id = grp.sorted_ids[m0 + 32 * NX0 * h + rp];
       // (padding lies behind the operand's end: zeros that nobody fetches, and products that take little power)
       off_x[h][e] = id < grp.num_valid ? (row_of((uint32_t)id) * K + (((lane & 7) ^ ((rp >> 1) & 7)) << 3)) * 2 : (int)0x80000000;
     }
@@ -105,14 +109,14 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     const __amdgpu_buffer_rsrc_t from = __builtin_amdgcn_make_buffer_rsrc((void*)(HALF < 2 ? x : w), 0, kt < nkt ? (HALF < 2 ? x_bytes : w_bytes) : 0, 0x00020000);
     const uint32_t at = lds0 + (kt & 1) * R::kParity;
     if constexpr (HALF < 2)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(uintptr_t)(at + HALF * R::kXHalf + (wave * NX + E) * 1024), 16,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(uintptr_t)(at + HALF * R::kXHalf + (wave * (HALF ? NX1 : NX0) + E) * 1024), 16,
                                                off_x[HALF][E], k, 0, 0);
     else
       __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)(uintptr_t)(at + 2 * R::kXHalf + (HALF - 2) * R::kWHalf + (wave * 4 + E) * 1024),
                                                16, off_w[HALF - 2][E], k, 0, NT ? 2 : 0);
   };
   auto stage = [&](auto half_c, int kt) __attribute__((always_inline)) {
-    rows_for<0, (decltype(half_c)::value < 2 ? NX : 4)>([&](auto e) __attribute__((always_inline)) { stage1(half_c, e, kt); });
+    rows_for<0, (decltype(half_c)::value == 0 ? NX0 : decltype(half_c)::value == 1 ? NX1 : 4)>([&](auto e) __attribute__((always_inline)) { stage1(half_c, e, kt); });
   };
   using H0 = std::integral_constant<int, 0>;
   using H1 = std::integral_constant<int, 1>;
@@ -123,21 +127,21 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   uint32_t off_s[2];
 #pragma unroll
   for (int s = 0; s < 2; ++s) off_s[s] = c16 * 128 + (((4 * s + q4) ^ swz) << 4);
-  const uint32_t xa = lds0 + wr * (16 * NX * 128);                      // this wave's 16 NX rows of an x half
+  const uint32_t xa = lds0 + wr * (16 * NX0 * 128), xb = lds0 + R::kXHalf + wr * (16 * NX1 * 128);     // this wave's 16 NX rows of an x half
   const uint32_t wa = lds0 + 2 * R::kXHalf + wc * (64 * 128);           // ... and 64 of a W half
 
-  g8_f32x4 acc[2 * NX][8];
+  g8_f32x4 acc[NX0 + NX1][8];
 #pragma unroll
-  for (int i = 0; i < 2 * NX; ++i)
+  for (int i = 0; i < NX0 + NX1; ++i)
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[i][j] = g8_f32x4{0.f, 0.f, 0.f, 0.f};
-  G8Frag fx0[NX][2], fx1[NX][2], fw0[4][2], fw1[4][2];
+  G8Frag fx0[NX0][2], fx1[NX1][2], fw0[4][2], fw1[4][2];
 
   // One phase: wait for this wave's share of the half to be read (VM loads behind it may be in flight) and for the last phase's reads,
   // barrier; then 8 NX products of one quadrant with the CNT x 2 reads of RF and the DMA of one half-tile between them.
   auto phase = [&](auto vm_c, auto& rf, uint32_t rbase, auto half_c, int kt, auto& xf, auto& wf, auto i0_c, auto j0_c) __attribute__((always_inline)) {
-    constexpr int CNT = sizeof(rf) / sizeof(rf[0]), I0 = decltype(i0_c)::value, J0 = decltype(j0_c)::value;
-    constexpr int DMA = decltype(half_c)::value < 2 ? NX : 4;
+    constexpr int CNT = sizeof(rf) / sizeof(rf[0]), NX = sizeof(xf) / sizeof(xf[0]), I0 = decltype(i0_c)::value, J0 = decltype(j0_c)::value;
+    constexpr int DMA = decltype(half_c)::value == 0 ? NX0 : decltype(half_c)::value == 1 ? NX1 : 4;
     g8_wait_vm<decltype(vm_c)::value>();
     g8_wait_lgkm0();
     g8_barrier();
@@ -158,18 +162,19 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
     });
   };
   // loads of the six half-tiles behind one that is waited for: of eight in a row, four x and four W, all but itself and the one before
-  constexpr int kAll = 4 * NX + 16;
-  using XX = std::integral_constant<int, kAll - 2 * NX>;
-  using XW = std::integral_constant<int, kAll - NX - 4>;
+  constexpr int kAll = 2 * (NX0 + NX1) + 16;
+  using XX = std::integral_constant<int, kAll - NX0 - NX1>;
+  using X0W = std::integral_constant<int, kAll - NX0 - 4>;
+  using X1W = std::integral_constant<int, kAll - NX1 - 4>;
   using WW = std::integral_constant<int, kAll - 8>;
-  using IX = std::integral_constant<int, NX>;
+  using IX = std::integral_constant<int, NX0>;
   using J4 = std::integral_constant<int, 4>;
 
   // (the first weights do not wait for the entries' rows)
   stage(H2{}, 0), stage(H3{}, 0), stage(H0{}, 0), stage(H1{}, 0), stage(H0{}, 1), stage(H3{}, 1), stage(H2{}, 1), stage(H1{}, 1);
-  g8_wait_vm<kAll - NX - 8>();
+  g8_wait_vm<kAll - NX0 - 8>();
   g8_barrier();
-  rows_for<0, NX>([&](auto f) __attribute__((always_inline)) {
+  rows_for<0, NX0>([&](auto f) __attribute__((always_inline)) {
     fx0[decltype(f)::value][0].u = g8_lds_read16(xa + off_s[0], decltype(f)::value * 2048);
     fx0[decltype(f)::value][1].u = g8_lds_read16(xa + off_s[1], decltype(f)::value * 2048);
   });
@@ -184,26 +189,27 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   for (int kt = 0; kt < nkt; kt += 2) {                                // (an even count of K steps: the caller sees to it)
     constexpr uint32_t pa = 0, pb = R::kParity;
     phase(WW{}, fw1, wa + pa + R::kWHalf, H2{}, kt + 2, fx0, fw0, H0{}, H0{});      // reads W1(kt);     W0(kt) -> W0(kt + 2)
-    phase(XW{}, fx1, xa + pa + R::kXHalf, H3{}, kt + 2, fx0, fw1, H0{}, J4{});      // reads x1(kt);     W1(kt) -> W1(kt + 2)
+    phase(X1W{}, fx1, xb + pa, H3{}, kt + 2, fx0, fw1, H0{}, J4{});      // reads x1(kt);     W1(kt) -> W1(kt + 2)
     phase(XX{}, fx0, xa + pb, H1{}, kt + 2, fx1, fw1, IX{}, J4{});                  // reads x0(kt + 1); x1(kt) -> x1(kt + 2)
-    phase(XW{}, fw1, wa + pb + R::kWHalf, H0{}, kt + 3, fx1, fw0, IX{}, H0{});      // reads W1(kt + 1); x0(kt + 1) -> x0(kt + 3)
+    phase(X0W{}, fw1, wa + pb + R::kWHalf, H0{}, kt + 3, fx1, fw0, IX{}, H0{});      // reads W1(kt + 1); x0(kt + 1) -> x0(kt + 3)
     phase(WW{}, fw0, wa + pb, H3{}, kt + 3, fx0, fw1, H0{}, J4{});                  // reads W0(kt + 1); W1(kt + 1) -> W1(kt + 3)
-    phase(XW{}, fx1, xa + pb + R::kXHalf, H2{}, kt + 3, fx0, fw0, H0{}, H0{});      // reads x1(kt + 1); W0(kt + 1) -> W0(kt + 3)
+    phase(X1W{}, fx1, xb + pb, H2{}, kt + 3, fx0, fw0, H0{}, H0{});      // reads x1(kt + 1); W0(kt + 1) -> W0(kt + 3)
     phase(XX{}, fx0, xa + pa, H1{}, kt + 3, fx1, fw0, IX{}, H0{});                  // reads x0(kt + 2); x1(kt + 1) -> x1(kt + 3)
-    phase(XW{}, fw0, wa + pa, H0{}, kt + 4, fx1, fw1, IX{}, J4{});                  // reads W0(kt + 2); x0(kt + 2) -> x0(kt + 4)
+    phase(X0W{}, fw0, wa + pa, H0{}, kt + 4, fx1, fw1, IX{}, J4{});                  // reads W0(kt + 2); x0(kt + 2) -> x0(kt + 4)
   }
-  // ---- epilogue: lane holds, of entry m0 + 32 NX h + 16 NX wr + 16 i + c16, columns 16 j + 4 q4 .. + 3 of its wave's.  A half's rows go
+  // ---- epilogue: lane holds, of entry m0 + 32 NX0 h + 16 NX wr + 16 i + c16, columns 16 j + 4 q4 .. + 3 of its wave's.  A half's rows go
   //      through the wave's own quarter of the LDS and leave whole: 256 bytes of an entry (128 of SiLU * up) instead of 32 a store.  All
   //      entries' places, and their weights, are asked for together ----
   constexpr int WCOLS = EPI == G8_SILU_MUL ? 64 : 128, LPR = WCOLS / 8, RPS = 64 / LPR;      // lanes a row, rows a store
   constexpr int OS = WCOLS * 2 + 16;                                                            // bytes between rows in LDS
-  static_assert(16 * NX * OS <= R::kLds / 4, "a half's rows fit the wave's quarter");
+  static_assert(16 * NX0 * OS <= R::kLds / 4, "a half's rows fit the wave's quarter");
   char* const mine = smem + wave * (R::kLds / 4);
-  int to[2][16 * NX / RPS], entry[2][NX];
-  float weight[2][NX];
+  int to[2][16 * NX0 / RPS], entry[2][NX0];
+  float weight[2][NX0];
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int32_t* ids = grp.sorted_ids + m0 + 32 * NX * h + 16 * NX * wr;
+    const int NX = h ? NX1 : NX0;
+    const int32_t* ids = grp.sorted_ids + m0 + 32 * NX0 * h + 16 * NX * wr;
 #pragma unroll
     for (int i = 0; i < NX; ++i) entry[h][i] = EPI == G8_PLAIN ? ids[16 * i + c16] : 0;
 #pragma unroll
@@ -214,14 +220,15 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
 #pragma unroll
   for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int i = 0; i < NX; ++i) weight[h][i] = EPI == G8_PLAIN && grp.mul_routed_weight ? grp.topk_weights[min(entry[h][i], grp.num_valid - 1)] : 1.f;   // (padding has none and is not stored)
-  rows_for<0, NX>([&](auto i_c) __attribute__((always_inline)) {
-    constexpr int I = NX + decltype(i_c)::value;
+    for (int i = 0; i < (h ? NX1 : NX0); ++i) weight[h][i] = EPI == G8_PLAIN && grp.mul_routed_weight ? grp.topk_weights[min(entry[h][i], grp.num_valid - 1)] : 1.f;   // (padding has none and is not stored)
+  rows_for<0, NX1>([&](auto i_c) __attribute__((always_inline)) {
+    constexpr int I = NX0 + decltype(i_c)::value;
     rows_retire<(I < 8)>(acc[I][4], acc[I][5], acc[I][6], acc[I][7]);
   });
   g8_barrier();                       // everybody has read its last fragments and has no DMA in flight
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
+    const int NX = h ? NX1 : NX0;
 #pragma unroll
     for (int i = 0; i < NX; ++i) {
       const float scale = weight[h][i];
@@ -232,7 +239,7 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
           // the unfused pair rounds the GEMM output to T before the activation reads it
 #pragma unroll
           for (int e = 0; e < 4; e += 2) {
-            const g8_f32x4 &gate = acc[NX * h + i][j], &up = acc[NX * h + i][(EPI == G8_SILU_MUL ? 4 : 0) + j];
+            const g8_f32x4 &gate = acc[NX0 * h + i][j], &up = acc[NX0 * h + i][(EPI == G8_SILU_MUL ? 4 : 0) + j];
             const uint32_t g2 = pack2<T>(gate[e], gate[e + 1]), u2 = pack2<T>(up[e], up[e + 1]);
 #pragma unroll
             for (int b = 0; b < 2; ++b) {
@@ -243,7 +250,7 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
           }
         } else {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) r[e] = acc[NX * h + i][j][e] * scale;
+          for (int e = 0; e < 4; ++e) r[e] = acc[NX0 * h + i][j][e] * scale;
         }
         *reinterpret_cast<uint2*>(mine + (16 * i + c16) * OS + j * 32 + q4 * 8) = uint2{pack2<T>(r[0], r[1]), pack2<T>(r[2], r[3])};
       }
@@ -347,17 +354,34 @@ moe_gemm_rows_kernel(T* __restrict__ out, const T* __restrict__ x, const T* __re
   }
   // weight rows that no other workgroup reads leave the L2 to the entries' rows (64 experts of 2048 x 1408 behind 94 rows: 97 -> 89 us, 281
   // rows 143 -> 134; of 1408 x 2816 within the noise)
-  if (alone) {
-    if (rows <= 128) moe_rows_body<T, EPI, 2, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else if (rows <= 192) moe_rows_body<T, EPI, 3, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else if (rows <= 256) moe_rows_body<T, EPI, 4, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else moe_rows_body<T, EPI, 5, true>(g8_smem, out, x, w, N, K, m0, n0, grp);
-  } else {
-    if (rows <= 128) moe_rows_body<T, EPI, 2, false>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else if (rows <= 192) moe_rows_body<T, EPI, 3, false>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else if (rows <= 256) moe_rows_body<T, EPI, 4, false>(g8_smem, out, x, w, N, K, m0, n0, grp);
-    else moe_rows_body<T, EPI, 5, false>(g8_smem, out, x, w, N, K, m0, n0, grp);
+  const int pairs = max(4, (rows + 31) >> 5);                            // of row fragments, the first half's and the second's
+#define ROWS_BODY(ALONE)                                                                                         \
+  switch (pairs) {                                                                                               \
+    case 4: return moe_rows_body<T, EPI, 2, 2, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    case 5: return moe_rows_body<T, EPI, 3, 2, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    case 6: return moe_rows_body<T, EPI, 3, 3, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    case 7: return moe_rows_body<T, EPI, 4, 3, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    case 8: return moe_rows_body<T, EPI, 4, 4, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    case 9: return moe_rows_body<T, EPI, 5, 4, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                    \
+    default: return moe_rows_body<T, EPI, 5, 5, ALONE>(g8_smem, out, x, w, N, K, m0, n0, grp);                   \
   }
+  if (alone) { ROWS_BODY(true) } else { ROWS_BODY(false) }
+#undef ROWS_BODY
 }
 
+template <typename T, int EPI>
+static int launch_rows(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, hipStream_t st) {
+  const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N, cols_per_tile = EPI == G8_SILU_MUL ? RowsTile::kCols / 2 : RowsTile::kCols;
+  const int64_t tiles = max_sorted / RowsTile::kRows * ((n_cols + cols_per_tile - 1) / cols_per_tile);
+  // (an XCD's share of the tiles and its share of those that come last are rounded up apart)
+  static std::atomic<uint64_t> lds_ok{0};
+  if (ensure_dynamic_lds((const void*)moe_gemm_rows_kernel<T, EPI>, RowsTile::kLds, lds_ok, "moe_gemm_rows")) return 1;
+  hipLaunchKernelGGL((moe_gemm_rows_kernel<T, EPI>), dim3((unsigned)((tiles + 7) / 8 * 8 + 8)), dim3(256), RowsTile::kLds, st, c, a, w, N, K, grp);
+  return launch_status("moe_gemm_rows");
+}
+
+template <typename T>
+int launch_moe_gemm_rows(T* c, const T* a, const T* w, const G8Group& grp, int64_t max_sorted, int N, int K, int epi, hipStream_t st) {
+  return epi == G8_SILU_MUL ? launch_rows<T, G8_SILU_MUL>(c, a, w, grp, max_sorted, N, K, st) : launch_rows<T, G8_PLAIN>(c, a, w, grp, max_sorted, N, K, st);
+}
 }  // namespace semipd

@@ -231,8 +231,8 @@ EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 # The whole library is ~3 CPU-minutes of hipcc.  A process that serves ONE model in a checkout where nothing is built yet
 # (bin/trace_run) compiles the sources that model's path calls into and links them as a library of its own name; the
 # whole library, once built (`make -C semi-pd_amd/csrc`, __graft_entry__.build()), always takes precedence.
-CORE_SOURCES = ("elementwise.hip", "rope_pairs.hip", "skinny_gemm.hip", "stream_linear.hip", "gemm8p.hip", "dense_gemm.hip", "moe.hip",
-                "moe_tiled_gemm.hip", "sampling.hip", "ipc.hip")          # pools, GEMMs, logits, sampler, streams
+CORE_SOURCES = ("elementwise.hip", "rope_pairs.hip", "skinny_gemm.hip", "stream_linear.hip", "gemm8p.hip", "moe_gemm_rows_bf16.hip",
+                "moe_gemm_rows_f16.hip", "dense_gemm.hip", "moe.hip", "moe_tiled_gemm.hip", "sampling.hip", "ipc.hip")          # pools, GEMMs, logits, sampler, streams
 MODEL_SOURCES = {
     "Kudirax": ("local_attention.hip", "layernorm.hip"),
     "Tigotar": ("local_attention.hip", "layernorm.hip", "recurrent.hip"),
