@@ -33,11 +33,11 @@
 
 namespace semipd {
 
-// Geometry of a tile: XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
+// Geometry of a tile: W2 = rows of a W half-tile (64: the 256 x 128 tile of 129 .. 256 rows, see g8_plan_one_row_tile), XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
 // tile for 65 .. 128 rows -- the same 32 accumulator tiles and 16 MFMAs per phase per wave, twice the weight rows per
 // MFMA, so the short batches are not bound by matrix work spent on padding rows).
-template <int XH> struct G8Geo {
-  static constexpr int WH = 16384 / XH;                 // rows of a W half-tile: 128 | 256
+template <int XH, int W2 = 16384 / XH> struct G8Geo {
+  static constexpr int WH = W2;                         // rows of a W half-tile: 128 | 256, half of that in the narrow forms
   static constexpr int kXHalf = XH * 128, kWHalf = WH * 128;
   static constexpr int kParity = 2 * (kXHalf + kWHalf); // x0, x1, W0, W1 of one K-step parity: 64 KB | 80 KB
   static constexpr int kLds = 2 * kParity;              // 128 KB | 160 KB
@@ -48,11 +48,11 @@ template <int XH> struct G8Geo {
 };
 
 // NT: the weight tile is used by this workgroup only (one row of tiles): stream it non-temporally past L2 / MALL
-template <typename T, int EPI, bool NT, int XH, bool GR = false, int ORDER = 0>
+template <typename T, int EPI, bool NT, int XH, bool GR = false, int ORDER = 0, int WHALF = 16384 / XH>
 __global__ void __launch_bounds__(512)
 gemm8p_kernel(T* __restrict__ out, float* __restrict__ planes, const T* __restrict__ x, const T* __restrict__ w, int M, int N,
               int K, int64_t ldx, int64_t ldo, int kt_per_slice, G8Group grp = G8Group()) {
-  using G = G8Geo<XH>;
+  using G = G8Geo<XH, WHALF>;
   constexpr int WH = G::WH, LX = G::LX, LW = G::LW, MT2 = G::MT2, NT2 = G::NT2;
   extern __shared__ __attribute__((aligned(16))) char g8_smem[];
   const int lane = threadIdx.x & 63;
@@ -646,24 +646,53 @@ static int g8_pick_ksplit(int tiles, int nkt, int M, int N, size_t planes_bytes)
   return best;
 }
 
-template <typename T, int EPI, int XH>
+// 129 .. 256 rows (one row tile): 256 x 256 tiles or 256 x 128, and how many K slices.  What bounds these calls is the weight's stream, at what a
+// workgroup a CU draws of it, and the planes' way to memory and back: 256 x 256 tiles of 4096 columns in 8 slices are 128 workgroups.  us of the
+// kernel (fit to 12 layer shapes at 140, 206 and 256 rows, weights from memory): a K step 1.4 in tiles of 256 columns, 0.87 in tiles of 128, which
+// grows with the workgroups from 0.8 of the CUs on; a plane at the copy's rate.  Whole call, 206 rows, us, before / now: 4096 x 4096
+// 29.7 / 24.8, 6144 x 4096 33.4 / 29.1, 4096 x 14336 52.8 / 46.0, 28672 x 4096 with SiLU 73.2 / 67.0; 3072 x 3072 30.3 / 22.8, 3072 x 8192 36.4 / 28.0;
+// 2048 x 2048 24.0 / 18.9, 2048 x 8192 33.9 / 24.2.  Weights of many rows stay with the wide tiles: a half has more than half the cost.
+struct G8Plan {
+  int cols, ks;                          // columns of a tile, K slices
+};
+static G8Plan g8_plan_one_row_tile(int M, int N, int nkt, size_t planes_bytes) {
+  const int cus = max(8, g_g8_cus.load(std::memory_order_relaxed));
+  G8Plan best{256, 1};
+  float best_cost = 1e30f;
+  for (int cols = 256; cols >= 128; cols -= 128) {
+    const int tiles = (N + cols - 1) / cols;
+    for (int ks = 1; ks <= 16; ++ks) {
+      const int per = (nkt + ks - 1) / ks;
+      if (ks > 1 && (per < 4 || (size_t)ks * M * N * 4 > planes_bytes)) break;
+      if ((nkt + per - 1) / per != ks) continue;
+      const int rounds = (tiles * ks + cus - 1) / cus, at_once = min(tiles * ks, cus);
+      const float step = cols == 256 ? 1.4f : 0.87f * max(1.f, at_once / (0.8f * cus));
+      float cost = rounds * (per * step + 3.f);
+      if (ks > 1) cost += ks * (8.f * M * N / 4.83e6f) + 3.f;
+      if (cost < best_cost - 1e-3f) best_cost = cost, best = G8Plan{cols, ks};
+    }
+  }
+  return best;
+}
+
+template <typename T, int EPI, int XH, int WHALF = 16384 / XH>
 static int g8_launch_geo(T* out, float* planes, size_t planes_bytes, const T* x, const T* w, int M, int N, int K, int64_t ldx,
-                         int64_t ldo, int force_ks, hipStream_t st, int* planes_only_ks = nullptr) {
-  using G = G8Geo<XH>;
+                         int64_t ldo, int force_ks, hipStream_t st, int* planes_only_ks = nullptr, int plan_ks = 0) {
+  using G = G8Geo<XH, WHALF>;
   const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N;
   const int cols_per_tile = EPI == G8_SILU_MUL ? G::WH : G::BN;
   const int tiles_n = (n_cols + cols_per_tile - 1) / cols_per_tile, tiles_m = (M + G::BM - 1) / G::BM;
   const int tiles = tiles_n * tiles_m;
   const int nkt = K / 64;
   int ksp = 1;
-  if (planes) ksp = force_ks > 0 ? min(force_ks, nkt) : g8_pick_ksplit(tiles, nkt, M, N, planes_bytes);
+  if (planes) ksp = force_ks > 0 ? min(force_ks, nkt) : plan_ks > 0 ? plan_ks : g8_pick_ksplit(tiles, nkt, M, N, planes_bytes);
   while (ksp > 1 && (size_t)ksp * M * N * 4 > planes_bytes) --ksp;
   const int per = (nkt + ksp - 1) / ksp;
   ksp = (nkt + per - 1) / per;
   // 256 x 256 tiles: the 8-wave ping-pong kernel or the 4-wave one (one 128 x 128 quarter per wave; see gemm4w_kernel), which
   // walks K two steps at a time: only where every slice is an even count of K steps.  The K partition itself never depends on
   // the form (the SiLU epilogue on eight waves and the plain one on four must sum the same slices: fused == unfused pair)
-  const bool four = XH == 128 && g8_four_waves(EPI) && nkt % 2 == 0 && per % 2 == 0;
+  const bool four = XH == 128 && WHALF == 128 && g8_four_waves(EPI) && nkt % 2 == 0 && per % 2 == 0;
   static std::atomic<uint64_t> lds_ok_nt{0}, lds_ok{0};
 #define G8_GO(K8, K4, OK)                                                                                              \
   do {                                                                                                                 \
@@ -679,7 +708,7 @@ static int g8_launch_geo(T* out, float* planes, size_t planes_bytes, const T* x,
     }                                                                                                                  \
   } while (0)
   if (tiles_m == 1) {
-    G8_GO((gemm8p_kernel<T, EPI, true, XH>), (gemm4w_kernel<T, EPI, true>), lds_ok_nt);
+    G8_GO((gemm8p_kernel<T, EPI, true, XH, false, 0, WHALF>), (gemm4w_kernel<T, EPI, true>), lds_ok_nt);
   } else {
     // XCD-contiguous order pays where the weight does not fit the caches between row tiles (vocabulary-sized heads:
     // 128 256 x 4096 at 1024 rows 1073 -> 834 us) and is neutral to slightly negative for layer-sized weights
@@ -688,9 +717,9 @@ static int g8_launch_geo(T* out, float* planes, size_t planes_bytes, const T* x,
     const bool xcd_order = xcd_knob >= 0 ? xcd_knob != 0 : n_cols >= 32768;
     static std::atomic<uint64_t> lds_ok_x{0};
     if (xcd_order) {
-      G8_GO((gemm8p_kernel<T, EPI, false, XH, false, 1>), (gemm4w_kernel<T, EPI, false, false, 1>), lds_ok_x);
+      G8_GO((gemm8p_kernel<T, EPI, false, XH, false, 1, WHALF>), (gemm4w_kernel<T, EPI, false, false, 1>), lds_ok_x);
     } else {
-      G8_GO((gemm8p_kernel<T, EPI, false, XH>), (gemm4w_kernel<T, EPI, false>), lds_ok);
+      G8_GO((gemm8p_kernel<T, EPI, false, XH, false, 0, WHALF>), (gemm4w_kernel<T, EPI, false>), lds_ok);
     }
   }
 #undef G8_GO
@@ -712,6 +741,12 @@ static int g8_launch(T* out, float* planes, size_t planes_bytes, const T* x, con
   // up to 128 rows: the 128 x 512 tile (no matrix work on padding rows, twice the weight rows per MFMA)
   const bool narrow = force_geo ? force_geo == 64 : M <= 128;
   if (narrow) return g8_launch_geo<T, EPI, 64>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks);
+  if (force_geo == 256 || (force_geo == 0 && M <= 256)) {
+    const G8Plan plan = g8_plan_one_row_tile(M, N, K / 64, planes ? planes_bytes : 0);
+    if (force_geo == 256 || plan.cols == 128)
+      return g8_launch_geo<T, EPI, 128, 64>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks, plan.cols == 128 ? plan.ks : 0);
+    return g8_launch_geo<T, EPI, 128>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks, plan.ks);
+  }
   return g8_launch_geo<T, EPI, 128>(out, planes, planes_bytes, x, w, M, N, K, ldx, ldo, force_ks, st, planes_only_ks);
 }
 
@@ -771,7 +806,7 @@ int semipd_gemm_tall(void* out, const void* x, const void* weight, void* workspa
   hipStream_t st = as_stream(stream);
   const char* e = getenv("SEMIPD_G8_KS");
   const int force_ks = e ? atoi(e) : 0;
-  const char* eg = getenv("SEMIPD_G8_XH");     // kbench / tests: force the 256 x 256 (128) or the 128 x 512 (64) tile
+  const char* eg = getenv("SEMIPD_G8_XH");     // kbench / tests: force the 256 x 256 (128), the 256 x 128 (256) or the 128 x 512 (64) tile
   const int force_geo = eg ? atoi(eg) : 0;
   int rc = 0;
   if (fuse_silu_mul) {

@@ -1,0 +1,42 @@
+"""ops.gemm_tall for 129 .. 256 rows (UnquantizedLinearMethod.apply, layers/linear.py:165-172): tiles of 256 rows x 128 columns and its choice of K slices."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def ops():
+    from semi_pd_amd import ops
+    return ops
+
+
+def _inputs(M, N, K, dtype):
+    g = torch.Generator(device="cpu").manual_seed(M * 7 + N + K)
+    return torch.randn(M, K, generator=g).to(dtype).cuda(), (torch.randn(N, K, generator=g) * K ** -0.5).to(dtype).cuda()
+
+
+# (ragged rows and columns, one K step and several, slices that are not as long as the others; columns of one tile, of a tile and a rest)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,N,K", [(129, 16, 64), (256, 128, 128), (200, 144, 192), (255, 272, 1088), (192, 1536, 2048), (206, 4096, 4096), (1, 112, 64), (300, 400, 576)])
+def test_narrow_tiles_match_fp32(ops, monkeypatch, dtype, M, N, K):
+    x, w = _inputs(M, N, K, dtype)
+    want = x.float() @ w.float().t()
+    rtol = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)             # one rounding of the result is half of it
+    for geo in ("256", "0"):
+        monkeypatch.setenv("SEMIPD_G8_XH", geo)
+        for ks in ("0", "1", "2", "5", "16"):
+            monkeypatch.setenv("SEMIPD_G8_KS", ks)
+            # (sums of K products of size K^-1/2 in another order: K^1/2 2^-24 times a few)
+            torch.testing.assert_close(ops.gemm_tall(x, w).float(), want, rtol=rtol, atol=1e-4)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,I,K", [(129, 64, 64), (256, 80, 192), (200, 1408, 2048), (140, 8192, 1024)])
+def test_narrow_tiles_with_silu_equal_the_unfused_pair(ops, monkeypatch, dtype, M, I, K):
+    x, w = _inputs(M, 2 * I, K, dtype)
+    for geo in ("256", "0"):
+        monkeypatch.setenv("SEMIPD_G8_XH", geo)
+        for ks in ("0", "1", "3"):
+            monkeypatch.setenv("SEMIPD_G8_KS", ks)
+            assert torch.equal(ops.gemm_tall(x, w, fuse_silu_mul=True), ops.silu_and_mul(ops.gemm_tall(x, w)))
