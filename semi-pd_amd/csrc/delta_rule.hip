@@ -941,6 +941,10 @@ __global__ void __launch_bounds__(256, 4) delta_chunk_operands_kernel(DeltaArgs 
 // work at 64 columns a workgroup.  Their chunk was 4.2 us of 10 k cycles, now 7.8 k, about 500 vector instructions and 56 products of either
 // wave of a SIMD; half the work a wave left the waits for the operands, so everything is fetched a whole chunk ahead there (3.5 -> 3.2 us; the form
 // of two waves is 5 % slower so).  32 heads of 128 x 128 over 8, whole call: 1 request of 5083 rows 741 -> 583 us, of 1000 168 -> 139.
+// Of a chunk's 10.3 k cycles (4 requests of 1900 rows) the products with S take 4.6 k and what is behind them 5.7 k; a SIMD's two waves take turns
+// rather than overlap.  K S and Q S as four sums side by side, the state's update in front of the results' products, one sum for all pieces, the
+// silus of a lane's tokens side by side, and one of the two waves through its convolution while the other multiplies: whole call 417 -> 406 us,
+// 1 request of 5000 rows 566 -> 548.  No gain: the higher priority for the waves with more products (424), everything a chunk ahead (422).
 template <typename T, int NP, int CB>
 __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, int64_t max_chunks) {
   constexpr int PARTS = 8 / CB;                                 // waves that share 16 columns
@@ -962,6 +966,7 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
   // of four waves the first two make v, the others finish the results, either of 16 tokens; of two each does both
   const int cw = w % CB, part = w / CB, half = part & 1;
   const bool makes_v = PARTS == 2 || part < 2, ends = PARTS == 2 || part >= 2;
+  const bool conv_first = PARTS == 2 && part == 1;              // (the other wave of the SIMD goes through its products meanwhile)
   // workgroups of one (request, key head) read the same operands: they go to one XCD (workgroup ids go round the 8 XCDs)
   const int H = a.H, G = a.G, D = a.D, E = a.E, taps = a.taps, per = H / G;
   const int eblocks = (E + 16 * CB - 1) / (16 * CB), members = per * eblocks;
@@ -1010,16 +1015,26 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
     f32x4 y;
 #pragma unroll
     for (int s = 0; s < 4; ++s) y[s] = wt[0] * raw[s + HALO];
+    if (taps == kRecTaps) {
 #pragma unroll
-    for (int i = 1; i < kRecTaps; ++i)
+      for (int i = 1; i < kRecTaps; ++i)
 #pragma unroll
-      for (int s = 0; s < 4; ++s) y[s] += wt[i] * __int_as_float(__float_as_int(raw[s + HALO - i]) & (i < taps ? -1 : 0));
+        for (int s = 0; s < 4; ++s) y[s] += wt[i] * raw[s + HALO - i];
+    } else {
+#pragma unroll
+      for (int i = 1; i < kRecTaps - 1; ++i)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) y[s] += wt[i] * __int_as_float(__float_as_int(raw[s + HALO - i]) & (i < taps ? -1 : 0));
+    }
+    float z[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) z[s] = rec_silu(y[s]);
+    asm volatile("" : "+v"(z[0]), "+v"(z[1]), "+v"(z[2]), "+v"(z[3]));         // (all four, side by side, also of rows that there are not: see rec_conv_silu)
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const float z = rec_silu(y[s]);
-      const bool in = 16 * half + 4 * kq + s < cnt;
-      v[s] = in ? (rec_moderate(y[s]) ? z : y[s]) : 0.f;         // (one that is not: see `serial`)
-      bad |= in && !rec_moderate(y[s]);
+      const bool in = 16 * half + 4 * kq + s < cnt, large = !rec_moderate(y[s]);
+      v[s] = in ? (large ? y[s] : z[s]) : 0.f;                    // (one that is not moderate: see `serial`)
+      bad |= in & large;
     }
   };
   // ... of the chunk at l0 into this lane's place, by way of the wave's LDS
@@ -1111,30 +1126,27 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
     f32x4 O = {}, P[2] = {}, v[2] = {}, vn;
     bool serial = false, bad_next = false;
     if (on) {
-      f32x4 Q[2] = {};
+      f32x4 Q[2];
       {
-        f32x4 Ps[2] = {}, Qs[2] = {};
+        if (conv_first) convolve(in, n - l0 - L, vn, bad_next);  // (the next chunk's; there is none: zeros)
+        f32x4 PQ[4] = {};
+        Split3 s[HT / 2];
+        Frag16 c[HT / 2][4][3];
 #pragma unroll
         for (int u = 0; u < HT / 2; ++u) {
-          const Split3 s = rec_split8(S[2 * u], S[2 * u + 1]);
-          Frag16 c[2][3];
+          s[u] = rec_split8(S[2 * u], S[2 * u + 1]);
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(k_l + q * PB + (i * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
-          rec_mma<2>(c, s, P, Ps);
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) c[i][q].u = *reinterpret_cast<const uint4*>(q_l + q * PB + (i * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
-          rec_mma<2>(c, s, Q, Qs);
+            for (int q = 0; q < 3; ++q)
+              c[u][i][q].u = *reinterpret_cast<const uint4*>((i < 2 ? k_l : q_l) + q * PB + ((i & 1) * (NT / 2) + part * (HT / 2) + u) * 1024 + lane * 16);
+          rec_mma_small<4>(c[u], s[u], PQ);
         }
-        if (makes_v) convolve(in, n - l0 - L, vn, bad_next);     // (the next chunk's, between the products; there is none: zeros)
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          P[i] += Ps[i];
-          Q[i] += Qs[i];
-        }
+        for (int u = 0; u < HT / 2; ++u) rec_mma_big<4>(c[u], s[u], PQ);
+        if (makes_v && !conv_first) convolve(in, n - l0 - L, vn, bad_next);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) P[i] = PQ[i], Q[i] = PQ[2 + i];
       }
       // the others of these columns get all of K S and the tokens of Q S that they finish
       if constexpr (PARTS == 2) {
@@ -1218,30 +1230,29 @@ __global__ void __launch_bounds__(512, 2) delta_chunk_walk_kernel(DeltaArgs a, i
         }
         U[1] += U1;
         const Split3 us = rec_split8(U[0] * wv[0], U[1] * wv[1]);
+        {
+          Frag16 kt[HT][3];
+#pragma unroll
+          for (int t = 0; t < HT; ++t)
+#pragma unroll
+            for (int q = 0; q < 3; ++q) kt[t][q].u = *reinterpret_cast<const uint4*>(kt_l + q * PB + (part * HT + t) * 1024 + lane * 16);
+          f32x4 A[HT] = {};
+          rec_mma_small<HT>(kt, us, A);
+          rec_mma_big<HT>(kt, us, A);
+#pragma unroll
+          for (int t = 0; t < HT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[t][r] = fmaf(S[t][r], keep, A[t][r]);
+        }
         f32x4 O1 = {};
         if (ends) {
 #pragma unroll
-          for (int s = 0; s < 4; ++s) {
-            O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], U[0][s], O, 0, 0, 0);
-            if (half) O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], U[1][s], O1, 0, 0, 0);
+          for (int s = 0; s < 4; ++s) O = __builtin_amdgcn_mfma_f32_16x16x4f32(M[0][s], U[0][s], O, 0, 0, 0);
+          if (half) {
+#pragma unroll
+            for (int s = 0; s < 4; ++s) O1 = __builtin_amdgcn_mfma_f32_16x16x4f32(M[1][s], U[1][s], O1, 0, 0, 0);
           }
           O += O1;
-        }
-#pragma unroll
-        for (int t = 0; t < HT; t += 2) {
-          Frag16 kt[2][3];
-#pragma unroll
-          for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int q = 0; q < 3; ++q) kt[i][q].u = *reinterpret_cast<const uint4*>(kt_l + q * PB + (part * HT + t + i) * 1024 + lane * 16);
-          f32x4 A[2] = {}, As[2] = {};
-          rec_mma<2>(kt, us, A, As);
-#pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            A[i] += As[i];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) S[t + i][r] = fmaf(S[t + i][r], keep, A[i][r]);
-          }
         }
       }
     } else {

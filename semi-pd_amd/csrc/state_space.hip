@@ -504,7 +504,8 @@ __global__ void __launch_bounds__(256, 4) ssm_chunk_operands_kernel(SsmArgs a) {
 // tokens' x from raw inputs in LDS of their own and hand x and the pieces of U = e^(b_last - b_t) dt_t x over: x is not written to memory.
 // Four waves per 16 columns halve what a wave does for a chunk: for launches that leave CUs without work at 64 columns a workgroup (a CU
 // holds one of theirs, not two: everything is fetched a whole chunk ahead, 2.9 -> 2.6 us a chunk, 3.3 at 64 columns).  128 heads of 128 x 64
-// over 8, whole call: 1 request of 5083 rows 611 -> 456 us, of 1000 137 -> 106.
+// over 8, whole call: 1 request of 5083 rows 611 -> 456 us, of 1000 137 -> 106; with the silus of a lane's four tokens side by side and D in one sum 434
+// (4 of 1900 rows, 64 columns a workgroup, 453 -> 450).
 template <typename T, int NP, int CB>
 __global__ void __launch_bounds__(512, CB == 4 ? 4 : 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
   constexpr int PARTS = 8 / CB;                                 // waves that share 16 columns
@@ -585,12 +586,27 @@ __global__ void __launch_bounds__(512, CB == 4 ? 4 : 2) ssm_chunk_walk_kernel(Ss
 #pragma unroll
         for (int s = 0; s < 4; ++s) y[s] += wt[i] * __int_as_float(__float_as_int(raw[s + HALO - i]) & (i < taps ? -1 : 0));
     }
+    if constexpr (PARTS > 2) {
+      // side by side, also of rows that there are not: behind a branch each, as they are left alone, every token waits for its own exponential
+      // and quotient (two workgroups a CU have each other for that, and no registers for it: the walk of 4 of 1900 rows 345 -> 385 us)
+      float z[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const float z = rec_silu(y[s]);
-      const bool in = 16 * half + 4 * kq + s < cnt;
-      x[s] = in ? (rec_moderate(y[s]) ? z : y[s]) : 0.f;         // (one that is not: see `serial`)
-      bad |= in && !rec_moderate(y[s]);
+      for (int s = 0; s < 4; ++s) z[s] = rec_silu(y[s]);
+      asm volatile("" : "+v"(z[0]), "+v"(z[1]), "+v"(z[2]), "+v"(z[3]));
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const bool in = 16 * half + 4 * kq + s < cnt, large = !rec_moderate(y[s]);
+        x[s] = in ? (large ? y[s] : z[s]) : 0.f;                 // (one that is not moderate: see `serial`)
+        bad |= in & large;
+      }
+    } else {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        const float z = rec_silu(y[s]);
+        const bool in = 16 * half + 4 * kq + s < cnt;
+        x[s] = in ? (rec_moderate(y[s]) ? z : y[s]) : 0.f;
+        bad |= in && !rec_moderate(y[s]);
+      }
     }
   };
   // x and U = e^(b_last - b_t) dt_t x to where both waves of these columns find them
@@ -759,14 +775,13 @@ __global__ void __launch_bounds__(512, CB == 4 ? 4 : 2) ssm_chunk_walk_kernel(Ss
 #pragma unroll
             for (int q = 0; q < 3; ++q) bt[i][q].u = *reinterpret_cast<const uint4*>(b_l + q * PB + (part * HT + t + i) * 1024 + lane * 16);
           }
-          f32x4 D[2] = {}, Ds[2] = {};
-          rec_mma<2>(bt, U, D, Ds);
+          f32x4 D[2] = {};
+          rec_mma_small<2>(bt, U, D);
+          rec_mma_big<2>(bt, U, D);
 #pragma unroll
-          for (int i = 0; i < 2; ++i) {
-            D[i] += Ds[i];
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int r = 0; r < 4; ++r) S[t + i][r] = fmaf(S[t + i][r], keep, D[i][r]);
-          }
         }
         O += dskip * x;
       }
