@@ -1,0 +1,51 @@
+"""Block-scaled fp8 expert GEMMs in blocks of 128 rows (csrc/fp8_rows.hip; fused_moe_triton/fused_moe.py:174-243)."""
+import pytest
+import torch
+
+from semi_pd_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+# (one to five scale blocks of K around the three in turn, and many; columns of one group, of a workgroup and a rest; experts whose rows fill one half of
+# a block, a row more, a block, a row more; an expert with none)
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("K,N,block_n", [(128, 16, 128), (256, 256, 128), (384, 272, 16), (512, 48, 48), (640, 400, 128), (1408, 528, 128)])
+def test_blocks_of_128_rows_against_their_products(K, N, block_n, out_dtype):
+    g = torch.Generator().manual_seed(K + N)
+    div, counts = 3, [1, 64, 65, 0, 128, 129]
+    total, E, KB, NB = sum(counts), len(counts), K // 128, -(-N // block_n)
+    tokens = -(-total // div)
+    q = lambda *s: (torch.randn(*s, generator=g) * 100).clamp(-448, 448).to(torch.float8_e4m3fn)               # noqa: E731
+    a, w = q(tokens, K), q(E, N, K)
+    a_s, w_s = torch.rand(tokens, KB, generator=g) + 0.5, torch.rand(E, NB, KB, generator=g) + 0.5
+    weights = torch.rand(total, generator=g)
+    perm, expert_of, ids, experts, at = torch.randperm(total, generator=g), torch.empty(total, dtype=torch.long), [], [], 0
+    for e, n in enumerate(counts):
+        mine = torch.full((-(-n // 128) * 128,), total, dtype=torch.int32)
+        mine[:n] = perm[at: at + n]
+        expert_of[perm[at: at + n]] = e
+        at += n
+        ids.append(mine)
+        experts += [e] * (-(-n // 128))
+    npp = torch.tensor([sum(i.numel() for i in ids)], dtype=torch.int32, device=DEV)
+    ids = torch.cat(ids + [torch.full((100,), total, dtype=torch.int32)])                                     # (room that nobody needs, no whole block)
+    row = torch.arange(total) // div
+    x, y = a.double().view(tokens, KB, 128)[row], w.double().view(E, N, KB, 128)[expert_of]
+    scale = a_s.double()[row][:, None] * w_s.double()[expert_of].repeat_interleave(block_n, 1)[:, :N]
+    want = (torch.einsum("tkc,tnkc->tnk", x, y) * scale).sum(-1)
+    size = (torch.einsum("tkc,tnkc->tnk", x.abs(), y.abs()) * scale).sum(-1)
+    half = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -24}[out_dtype]
+    down = 2.0 ** -12 if out_dtype == torch.float16 else 1.0                                                # (fp16 holds up to 65504)
+    d = lambda t: t.to(DEV)                                                                              # noqa: E731
+    for scaled in (False, True):
+        s = weights.double()[:, None] if scaled else 1.0
+        out = torch.full((total + 1, N), 77.0, dtype=out_dtype, device=DEV)
+        ops.moe_grouped_gemm_fp8(d(a), d(a_s * down), d(w), d(w_s), out[:total], d(weights), d(ids), d(torch.tensor(experts, dtype=torch.int32)), npp, total,
+                                 div, scaled, [block_n, 128], 128)
+        assert bool((out[total] == 77).all())
+        # one rounding of the result, and what the matrix unit keeps of the sum of a scale block (the largest product's place and 13 bits behind
+        # it: 2^-12 of the sum at most)
+        bound = (half * (want * s).abs() + 2.0 ** -11 * size * s) * down + 2.0 ** -24
+        assert bool(((out[:total].cpu().double() - want * s * down).abs() <= bound).all())
