@@ -414,7 +414,8 @@ def _prefers_tiled_gemm(weight: torch.Tensor, rows: int, fuse_silu_mul: bool = F
     """Prefill-sized batch: what was timed at start-up where it was, else by how full the chip is."""
     if ops.dense_gemm_is_tuned(weight):
         return ops.tall_preferred(weight, rows, fuse_silu_mul=fuse_silu_mul)
-    return ops.tiled_gemm_fills_chip(weight.shape[0], weight.shape[1], rows, fuse_silu_mul)
+    n, k = weight.shape
+    return ops.tiled_gemm_fills_chip(n, k, rows, fuse_silu_mul) or (fuse_silu_mul and ops.tiled_gemm_short_tail(n, k, rows))
 
 
 def gate_up_silu(x: torch.Tensor, gate_up_proj: "MergedColumnParallelLinear", act_fn) -> torch.Tensor:

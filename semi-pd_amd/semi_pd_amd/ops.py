@@ -594,6 +594,22 @@ def tiled_gemm_fills_chip(n: int, k: int, rows: int, fuse_silu_mul: bool = False
     return filled >= 0.75 if slices > 2 else slices == 2 and filled > 0.75
 
 
+def tiled_gemm_short_tail(n: int, k: int, rows: int) -> bool:
+    """The same for gate and up with SiLU in the epilogue, where the last of several row tiles has at most 64 rows: its workgroups multiply a quarter of
+    a tile's and take 0.4 of its time, and they come last, two to a CU that the others leave free.  Ahead from 0.775 of the time that the tiles
+    take then, from 0.8 of it behind three rounds.  us of the pair of launches, library / tiled: 28672 x 4096, 1056 rows 241 / 208, 1595 338 / 304; 800
+    (0.68) 187 / 184, 1300 (0.74) 278 / 279, 1833 (0.78, four rounds) 364 / 369; 16384 x 3072, 800 rows 83 / 76, 1595 156 / 145, 2100 224 / 186, 1300
+    (0.64) 130 / 138; 16384 x 2048, 800 rows 65 / 54, 1595 112 / 103, 2100 142 / 131, 1300 94 / 97."""
+    tail, cols = rows % 256, -(-(n // 2) // 128)
+    if _DENSE_GEMM["cus"] not in (0, 256) or rows < 256 or not 0 < tail <= 64 or not 2048 <= k <= 5120 or not 0 < n <= 37888:
+        return False
+    rounds = -(-(rows // 256 * cols) // 256)
+    behind = cols - 2 * (rounds * 256 - rows // 256 * cols)          # (short ones that find no free CU)
+    if behind > 0:
+        rounds += 0.4 * -(-behind // 256)
+    return rows * (n // 2) >= (0.775 if rounds <= 3 else 0.8) * rounds * 256 * 256 * 128
+
+
 def dense_gemm_report() -> str:
     import ctypes as _C
     lib = _lib.load()

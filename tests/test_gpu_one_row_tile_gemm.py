@@ -40,3 +40,22 @@ def test_narrow_tiles_with_silu_equal_the_unfused_pair(ops, monkeypatch, dtype, 
         for ks in ("0", "1", "3"):
             monkeypatch.setenv("SEMIPD_G8_KS", ks)
             assert torch.equal(ops.gemm_tall(x, w, fuse_silu_mul=True), ops.silu_and_mul(ops.gemm_tall(x, w)))
+
+
+# (a last row tile of which one quarter of the rows is there, one row more, three quarters, one row more, all but one)
+@pytest.mark.parametrize("silu", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [257, 320, 321, 384, 385, 448, 449, 767])
+def test_last_row_tiles_of_the_eight_wave_form(ops, monkeypatch, dtype, M, silu):
+    x, w = _inputs(M, 2 * 144, 640, dtype)
+    monkeypatch.setenv("SEMIPD_G8_XH", "128")
+    ops.gemm_tall_set_form(8)
+    try:
+        plain = ops.gemm_tall(x, w)
+        got = ops.gemm_tall(x, w, fuse_silu_mul=True) if silu else plain
+    finally:
+        ops.gemm_tall_set_form(0)
+    if silu:
+        assert torch.equal(got, ops.silu_and_mul(plain))
+    else:
+        torch.testing.assert_close(got.float(), x.float() @ w.float().t(), rtol=2.0 ** (-8 if dtype == torch.bfloat16 else -11), atol=1e-4)

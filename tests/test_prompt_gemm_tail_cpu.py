@@ -1,0 +1,16 @@
+"""Gate and up of prompt batches whose last row tile is short: which of them go to the tiled GEMM, by sizes alone."""
+import pytest
+
+
+# (tails of one row, of 64 and of 65; whole tiles alone; rounds that the short tiles lengthen; narrower and wider layers than were measured)
+@pytest.mark.parametrize("n,k,rows,takes", [
+    (28672, 4096, 1595, True), (28672, 4096, 1600, True), (28672, 4096, 1601, False), (28672, 4096, 1536, False), (28672, 4096, 1537, True),
+    (28672, 4096, 1056, True), (28672, 4096, 800, False), (28672, 4096, 1300, False), (28672, 4096, 1833, False), (28672, 4096, 300, False),
+    (16384, 3072, 800, True), (16384, 3072, 1595, True), (16384, 2048, 2100, True), (16384, 2048, 1300, False), (16384, 1984, 800, False),
+    (28672, 5184, 1595, False), (37904, 2048, 800, False), (28672, 4096, 59, False), (0, 4096, 800, False), (28672, 4096, 0, False)])
+def test_short_tails(monkeypatch, n, k, rows, takes):
+    from semi_pd_amd import ops
+    monkeypatch.setitem(ops._DENSE_GEMM, "cus", 0)
+    assert ops.tiled_gemm_short_tail(n, k, rows) == takes
+    monkeypatch.setitem(ops._DENSE_GEMM, "cus", 128)
+    assert not ops.tiled_gemm_short_tail(n, k, rows)
