@@ -33,14 +33,15 @@
 
 namespace semipd {
 
-// Geometry of a tile: W2 = rows of a W half-tile (64: the 256 x 128 tile of 129 .. 256 rows, see g8_plan_one_row_tile), XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
+// Geometry of a tile: XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
 // tile for 65 .. 128 rows -- the same 32 accumulator tiles and 16 MFMAs per phase per wave, twice the weight rows per
-// MFMA, so the short batches are not bound by matrix work spent on padding rows).
+// MFMA, so the short batches are not bound by matrix work spent on padding rows), W2 = rows of a W half-tile (64 with XH = 128: a
+// 256 x 128 tile for 129 .. 256 rows, see g8_plan_one_row_tile).
 template <int XH, int W2 = 16384 / XH> struct G8Geo {
   static constexpr int WH = W2;                         // rows of a W half-tile: 128 | 256, half of that in the narrow forms
   static constexpr int kXHalf = XH * 128, kWHalf = WH * 128;
-  static constexpr int kParity = 2 * (kXHalf + kWHalf); // x0, x1, W0, W1 of one K-step parity: 64 KB | 80 KB
-  static constexpr int kLds = 2 * kParity;              // 128 KB | 160 KB
+  static constexpr int kParity = 2 * (kXHalf + kWHalf); // x0, x1, W0, W1 of one K-step parity: 64 KB | 80 KB | 48 KB
+  static constexpr int kLds = 2 * kParity;              // 128 KB | 160 KB | 96 KB
   static constexpr int LX = XH / 64, LW = WH / 64;      // DMA instructions per wave per half-tile
   static constexpr int MT2 = XH / 32, NT2 = WH / 64;    // 16-row fragments per wave and half: x | W
   static constexpr int BM = 2 * XH, BN = 2 * WH;
@@ -647,10 +648,10 @@ static int g8_pick_ksplit(int tiles, int nkt, int M, int N, size_t planes_bytes)
 
 // 129 .. 256 rows (one row tile): 256 x 256 tiles or 256 x 128, and how many K slices.  What bounds these calls is the weight's stream, at what a
 // workgroup a CU draws of it, and the planes' way to memory and back: 256 x 256 tiles of 4096 columns in 8 slices are 128 workgroups.  us of the
-// kernel (fit to 12 layer shapes at 140, 206 and 256 rows, weights from memory): a K step 1.4 in tiles of 256 columns, 0.87 in tiles of 128, which
-// grows with the workgroups from 0.8 of the CUs on; a plane at the copy's rate.  Whole call, 206 rows, us, before / now: 4096 x 4096
-// 29.7 / 24.8, 6144 x 4096 33.4 / 29.1, 4096 x 14336 52.8 / 46.0, 28672 x 4096 with SiLU 73.2 / 67.0; 3072 x 3072 30.3 / 22.8, 3072 x 8192 36.4 / 28.0;
-// 2048 x 2048 24.0 / 18.9, 2048 x 8192 33.9 / 24.2.  Weights of many rows stay with the wide tiles: a half has more than half the cost.
+// kernel (fit to 12 layer shapes at 140, 206 and 256 rows on all 256 CUs, weights from memory): a K step 1.4 in tiles of 256 columns, 0.87 in tiles of
+// 128, a plane at the copy's rate.  Whole call, 206 rows, us, tiles of 256 columns in up to 8 slices / this: 4096 x 4096 29.7 / 25.5, 6144 x 4096 33.4 / 28.1,
+// 4096 x 14336 52.8 / 42.6, 28672 x 4096 with SiLU 73.2 / 65.8; 3072 x 3072 30.3 / 23.1, 3072 x 8192 36.4 / 28.2; 2048 x 2048 24.0 / 19.1, 2048 x 8192 33.9 / 24.2.
+// Weights of many rows stay with the wide tiles: a half has more than half the cost.
 struct G8Plan {
   int cols, ks;                          // columns of a tile, K slices
 };
@@ -664,8 +665,8 @@ static G8Plan g8_plan_one_row_tile(int M, int N, int nkt, size_t planes_bytes) {
       const int per = (nkt + ks - 1) / ks;
       if (ks > 1 && (per < 4 || (size_t)ks * M * N * 4 > planes_bytes)) break;
       if ((nkt + per - 1) / per != ks) continue;
-      const int rounds = (tiles * ks + cus - 1) / cus, at_once = min(tiles * ks, cus);
-      const float step = cols == 256 ? 1.4f : 0.87f * max(1.f, at_once / (0.8f * cus));
+      const int rounds = (tiles * ks + cus - 1) / cus;
+      const float step = cols == 256 ? 1.4f : 0.87f;
       float cost = rounds * (per * step + 3.f);
       if (ks > 1) cost += ks * (8.f * M * N / 4.83e6f) + 3.f;
       if (cost < best_cost - 1e-3f) best_cost = cost, best = G8Plan{cols, ks};
