@@ -31,6 +31,8 @@
 // layers/activation.py:41-53) for 65 .. 256-row decode batches, and _get_logits (layers/logits_processor.py:394-445).
 #include "gemm8p_parts.h"
 
+#include <algorithm>
+
 namespace semipd {
 
 // Geometry of a tile: XH = rows of an x half-tile (128: a 256 x 256 tile for batches above 128 rows; 64: a 128 x 512
@@ -651,26 +653,35 @@ static int g8_pick_ksplit(int tiles, int nkt, int M, int N, size_t planes_bytes)
 // kernel (fit to 12 layer shapes at 140, 206 and 256 rows on all 256 CUs, weights from memory): a K step 1.4 in tiles of 256 columns, 0.87 in tiles of
 // 128, a plane at the copy's rate.  Whole call, 206 rows, us, tiles of 256 columns in up to 8 slices / this: 4096 x 4096 29.7 / 25.5, 6144 x 4096 33.4 / 28.1,
 // 4096 x 14336 52.8 / 42.6, 28672 x 4096 with SiLU 73.2 / 65.8; 3072 x 3072 30.3 / 23.1, 3072 x 8192 36.4 / 28.2; 2048 x 2048 24.0 / 19.1, 2048 x 8192 33.9 / 24.2.
-// Weights of many rows stay with the wide tiles: a half has more than half the cost.
+// Weights of many rows stay with the wide tiles: a half has more than half the cost.  On streams over 64, 128, 192 and 224 CUs, 36 of those calls and
+// 145 of 29 other shapes at 129 to 240 rows each: 1.07, 1.13, 1.17 and 1.19 times as fast as the tiles of 256 columns (1.22 on all); by the whole
+// chip's figures alone up to 9 % behind them (6144 x 4096, 129 rows on 64 CUs 48.3 -> 51.8 us, 32000 x 4096 on 224 81.2 -> 88.8).
 struct G8Plan {
   int cols, ks;                          // columns of a tile, K slices
 };
 static G8Plan g8_plan_one_row_tile(int M, int N, int nkt, size_t planes_bytes) {
   const int cus = max(8, g_g8_cus.load(std::memory_order_relaxed));
+  const float rate = std::min(4.83e6f, cus * 30e3f);       // bytes a us of the planes' way
+  auto cost = [&](int cols, int ks) {
+    const int per = (nkt + ks - 1) / ks, rounds = ((N + cols - 1) / cols * ks + cus - 1) / cus;
+    return rounds * (per * (cols == 256 ? 1.4f : 0.87f) + 3.f) + (ks > 1 ? ks * (8.f * M * N / rate) + 3.f : 0.f);
+  };
   G8Plan best{256, 1};
   float best_cost = 1e30f;
   for (int cols = 256; cols >= 128; cols -= 128) {
-    const int tiles = (N + cols - 1) / cols;
     for (int ks = 1; ks <= 16; ++ks) {
       const int per = (nkt + ks - 1) / ks;
       if (ks > 1 && (per < 4 || (size_t)ks * M * N * 4 > planes_bytes)) break;
       if ((nkt + per - 1) / per != ks) continue;
-      const int rounds = (tiles * ks + cus - 1) / cus;
-      const float step = cols == 256 ? 1.4f : 0.87f;
-      float cost = rounds * (per * step + 3.f);
-      if (ks > 1) cost += ks * (8.f * M * N / 4.83e6f) + 3.f;
-      if (cost < best_cost - 1e-3f) best_cost = cost, best = G8Plan{cols, ks};
+      const float c = cost(cols, ks);
+      if (c < best_cost - 1e-3f) best_cost = c, best = G8Plan{cols, ks};
     }
+  }
+  // On a share of the CUs the stream is not what bounds a wide tile's step (1.1 to 1.3 us on 64 and 192 CUs): there the choice of tiles of 256 columns
+  // alone stands unless another is 5 % ahead of it.
+  if (cus < 256) {
+    const int wide = g8_pick_ksplit((N + 255) / 256, nkt, M, N, planes_bytes);
+    if (!(best_cost < 0.95f * cost(256, wide))) return G8Plan{256, wide};
   }
   return best;
 }

@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from test_gpu_share_of_cus import _share
+
 pytestmark = pytest.mark.gpu
 
 
@@ -59,3 +61,27 @@ def test_last_row_tiles_of_the_eight_wave_form(ops, monkeypatch, dtype, M, silu)
         assert torch.equal(got, ops.silu_and_mul(plain))
     else:
         torch.testing.assert_close(got.float(), x.float() @ w.float().t(), rtol=2.0 ** (-8 if dtype == torch.bfloat16 else -11), atol=1e-4)
+
+
+def _slices(ops, rows, n, k):
+    """How many slices of K a plain product is cut into, and the product."""
+    x, w = _inputs(rows, n, k, torch.bfloat16)
+    got = ops.gemm_tall_planes(x, w)
+    if isinstance(got, torch.Tensor):
+        return 1, got, x, w
+    # (planes are fp32: their sum is the product before its rounding)
+    return got.ksplit, got.planes.view(torch.float32)[: got.ksplit * rows * n].view(got.ksplit, rows, n).sum(0), x, w
+
+
+# (the choice of 256-column tiles alone stands where the planes' way is the share's: the slices that it takes)
+@pytest.mark.parametrize("cus,rows,n,k,slices", [(64, 140, 6144, 4096, 2), (64, 206, 4096, 4096, 4), (48, 206, 28672, 4096, 1), (128, 206, 4096, 4096, 4),
+                                                 (192, 140, 28672, 4096, 1), (208, 129, 28672, 4096, 1), (224, 129, 32000, 4096, 1)])
+def test_slices_on_a_share_of_the_cus(ops, cus, rows, n, k, slices):
+    with _share(cus):
+        took, got, x, w = _slices(ops, rows, n, k)
+        out = ops.gemm_tall(x, w)
+    assert took == slices
+    want = x.float() @ w.float().t()
+    # (a rounding of the result to bf16 and sums of K products of size K^-1/2 in another order, as above)
+    torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-4)
+    torch.testing.assert_close(out.float(), want, rtol=2.0 ** -8, atol=1e-4)
