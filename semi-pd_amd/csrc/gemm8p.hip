@@ -654,8 +654,10 @@ static int g8_pick_ksplit(int tiles, int nkt, int M, int N, size_t planes_bytes)
 // 128, a plane at the copy's rate.  Whole call, 206 rows, us, tiles of 256 columns in up to 8 slices / this: 4096 x 4096 29.7 / 25.5, 6144 x 4096 33.4 / 28.1,
 // 4096 x 14336 52.8 / 42.6, 28672 x 4096 with SiLU 73.2 / 65.8; 3072 x 3072 30.3 / 23.1, 3072 x 8192 36.4 / 28.2; 2048 x 2048 24.0 / 19.1, 2048 x 8192 33.9 / 24.2.
 // Weights of many rows stay with the wide tiles: a half has more than half the cost.  On streams over 64, 128, 192 and 224 CUs, 36 of those calls and
-// 145 of 29 other shapes at 129 to 240 rows each: 1.07, 1.13, 1.17 and 1.19 times as fast as the tiles of 256 columns (1.22 on all); by the whole
-// chip's figures alone up to 9 % behind them (6144 x 4096, 129 rows on 64 CUs 48.3 -> 51.8 us, 32000 x 4096 on 224 81.2 -> 88.8).
+// 145 of 29 other shapes at 129 to 240 rows each: 1.07, 1.13, 1.17 and 1.19 times as fast as the tiles of 256 columns (1.22 on all), none more than 2 %
+// behind; by the whole chip's figures alone up to 9 % (6144 x 4096, 129 rows on 64 CUs 48.3 -> 51.8 us, 32000 x 4096 on 224 81.2 -> 88.8).  Long K, 206 rows
+// with SiLU, wide tiles in two slices / narrow ones in one (which this doesn't take: long_k): 32768 x 6144 98.4 / 107.7, 28672 x 8192 122.1 / 131.0, 30720 x
+// 5120 83.3 / 86.0; with 192 rows 94.5 / 99.3, - , 84.7 / 77.8 (taken), and of 24576 x 5120, 192 workgroups, 206 rows 79.4 / 77.8 (taken).
 struct G8Plan {
   int cols, ks;                          // columns of a tile, K slices
 };
@@ -666,13 +668,16 @@ static G8Plan g8_plan_one_row_tile(int M, int N, int nkt, size_t planes_bytes) {
     const int per = (nkt + ks - 1) / ks, rounds = ((N + cols - 1) / cols * ks + cus - 1) / cus;
     return rounds * (per * (cols == 256 ? 1.4f : 0.87f) + 3.f) + (ks > 1 ? ks * (8.f * M * N / rate) + 3.f : 0.f);
   };
+  // One slice of narrow tiles on most of the CUs over a long K takes 0.95 to 1.1 us a step: every workgroup reads all of x, 2.4 MB and more there,
+  // beside the weight's stream.
+  const bool long_k = (N + 127) / 128 > 0.8f * cus && nkt >= 80 && (M > 192 || nkt >= 96);
   G8Plan best{256, 1};
   float best_cost = 1e30f;
   for (int cols = 256; cols >= 128; cols -= 128) {
     for (int ks = 1; ks <= 16; ++ks) {
       const int per = (nkt + ks - 1) / ks;
       if (ks > 1 && (per < 4 || (size_t)ks * M * N * 4 > planes_bytes)) break;
-      if ((nkt + per - 1) / per != ks) continue;
+      if ((nkt + per - 1) / per != ks || (cols == 128 && ks == 1 && long_k)) continue;
       const float c = cost(cols, ks);
       if (c < best_cost - 1e-3f) best_cost = c, best = G8Plan{cols, ks};
     }

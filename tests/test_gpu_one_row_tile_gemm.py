@@ -85,3 +85,12 @@ def test_slices_on_a_share_of_the_cus(ops, cus, rows, n, k, slices):
     # (a rounding of the result to bf16 and sums of K products of size K^-1/2 in another order, as above)
     torch.testing.assert_close(got.float(), want, rtol=2.0 ** -8, atol=1e-4)
     torch.testing.assert_close(out.float(), want, rtol=2.0 ** -8, atol=1e-4)
+
+
+# (one slice of narrow tiles on most of the CUs over a long K is left to the wide ones in two: x does not stay in an L2 beside the weight's stream)
+@pytest.mark.parametrize("rows,n,k,slices", [(160, 32768, 6144, 2), (206, 32768, 6144, 2), (240, 30720, 5120, 2), (192, 30720, 5120, 1), (256, 24576, 5120, 1),
+                                             (206, 28672, 8192, 2), (206, 28672, 4096, 1)])
+def test_slices_of_a_long_k(ops, rows, n, k, slices):
+    took, got, x, w = _slices(ops, rows, n, k)
+    assert took == slices
+    torch.testing.assert_close(got.float(), x.float() @ w.float().t(), rtol=2.0 ** -8, atol=1e-4)
