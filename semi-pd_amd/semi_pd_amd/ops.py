@@ -1564,8 +1564,7 @@ def min_gru(proj: torch.Tensor, z_off: int, x_off: int, g_off: int, width: int, 
         raise RuntimeError("min_gru: proj / out are 2-D rows of one type, out [T, width]")
     if state.dtype != torch.float32 or state.dim() != 2 or state.shape[1] != width or state.stride(1) != 1:
         raise RuntimeError("min_gru: state is fp32 [slots, width]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("min_gru: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("min_gru", state_indices, seq_lens, B)
     for b_ in (bias_z, bias_x):
         if b_ is not None and (b_.shape != (width,) or b_.dtype != proj.dtype):
             raise RuntimeError("min_gru: biases are [width] of the activation type")
@@ -1698,6 +1697,13 @@ def rms_stream(y: Optional[torch.Tensor], stream: torch.Tensor, weight: Optional
     return out
 
 
+def _batch_ids(name: str, state_indices: torch.Tensor, seq_lens: torch.Tensor, B: int):
+    """The batch's state rows and lengths as the kernels read them, one behind the other (a column of a table is copied)."""
+    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
+        raise RuntimeError(f"{name}: state_indices / seq_lens are int64 [B]")
+    return state_indices.contiguous(), seq_lens.contiguous()
+
+
 def _batch_rows(name: str, T: int, B: int, q_start, q_len) -> None:
     if (q_start is None) != (q_len is None) or (q_start is None and T != B):
         raise RuntimeError(f"{name}: q_start and q_len come together; without them one row per request")
@@ -1719,8 +1725,7 @@ def embed_bigram(input_ids: torch.Tensor, embed: torch.Tensor, bigram: torch.Ten
         raise RuntimeError("embed_bigram: int64 ids, embed [V, W] and bigram [buckets + 1, W] contiguous and of one type")
     if prev_token.dtype != torch.int32 or prev_token.dim() != 2 or prev_token.shape[1] < 1:
         raise RuntimeError("embed_bigram: prev_token is int32 [slots, >= 1]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("embed_bigram: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("embed_bigram", state_indices, seq_lens, B)
     _batch_rows("embed_bigram", T, B, q_start, q_len)
     out = torch.empty((T, width), dtype=torch.float32, device=embed.device)
     check(_lib.load().semipd_embed_bigram(ptr(input_ids), ptr(embed), ptr(bigram), float(scale), int(mul_prev), int(mul_cur),
@@ -1836,7 +1841,7 @@ def _delta_rule_step(proj, offsets, conv_q, conv_k, conv_v, a_log, dt_bias, norm
             and state_indices.dtype == seq_lens.dtype == torch.int64):
         return None
     if not (conv_q.is_contiguous() and conv_k.is_contiguous() and conv_v.is_contiguous() and a_log.is_contiguous()
-            and dt_bias.is_contiguous() and norm_weight.is_contiguous()):
+            and dt_bias.is_contiguous() and norm_weight.is_contiguous() and state_indices.is_contiguous() and seq_lens.is_contiguous()):
         return None
     (state_ld, step), (conv_ld, conv_step) = state.stride(), conv_state.stride()
     q, k, v, gate, a, b = offsets
@@ -1890,8 +1895,7 @@ def delta_rule(proj: torch.Tensor, offsets, conv_q: torch.Tensor, conv_k: torch.
     if taps > 1 and (conv_state is None or conv_state.dtype != torch.float32 or conv_state.dim() != 2
                      or conv_state.shape[1] != (taps - 1) * (2 * gd + hv) or conv_state.stride(1) != 1):
         raise RuntimeError("delta_rule: conv_state is fp32 [slots, (taps - 1) * channels]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("delta_rule: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("delta_rule", state_indices, seq_lens, B)
     _batch_rows("delta_rule", T, B, q_start, q_len)
     ends = [offsets[0] + gd, offsets[1] + gd, offsets[2] + hv, offsets[3] + hv, offsets[4] + num_heads, offsets[5] + num_heads]
     if min(offsets) < 0 or max(ends) > proj.shape[1]:
@@ -2012,6 +2016,7 @@ def postnorm_stream(y: Optional[torch.Tensor], layer_scale: Optional[torch.Tenso
         if state_indices is None or seq_lens is None or state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 \
                 or state_indices.shape[0] != rows or seq_lens.shape[0] != rows:
             raise RuntimeError("postnorm_stream: the shifted form takes one row per request: state_indices / seq_lens int64 [rows]")
+        state_indices, seq_lens = state_indices.contiguous(), seq_lens.contiguous()
     out = torch.empty((rows, width), dtype=dt, device=stream.device) if want_out else None
     check(_lib.load().semipd_postnorm_stream(ptr(y), y.stride(0) if y is not None else 0, ptr(layer_scale), ptr(stream),
                                              stream.stride(0), float(alpha), ptr(weight), float(eps), ptr(out),
@@ -2034,8 +2039,7 @@ def token_shift(stream: torch.Tensor, mu: torch.Tensor, prev: torch.Tensor, stat
         raise RuntimeError("token_shift: mu is contiguous [width]")
     if prev.dtype != torch.float32 or prev.dim() != 2 or prev.shape[1] != width or prev.stride(1) != 1:
         raise RuntimeError("token_shift: prev is fp32 [slots, width]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("token_shift: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("token_shift", state_indices, seq_lens, B)
     _batch_rows("token_shift", T, B, q_start, q_len)
     out = torch.empty((T, width), dtype=mu.dtype, device=stream.device)
     check(_lib.load().semipd_token_shift(ptr(stream), stream.stride(0), ptr(mu), ptr(prev), prev.stride(0), ptr(state_indices),
@@ -2152,7 +2156,7 @@ def _state_space_step(proj, z_off, x_off, dt_off, conv_w, conv_b, dt_bias, a_log
             and state_indices.dtype == seq_lens.dtype == torch.int64):
         return None
     if not (conv_w.is_contiguous() and conv_b.is_contiguous() and dt_bias.is_contiguous() and a_log.is_contiguous()
-            and d_skip.is_contiguous() and norm_weight.is_contiguous()):
+            and d_skip.is_contiguous() and norm_weight.is_contiguous() and state_indices.is_contiguous() and seq_lens.is_contiguous()):
         return None
     (state_ld, step), (conv_ld, conv_step) = state.stride(), conv_state.stride()
     if step != 1 or conv_step != 1 or min(z_off, x_off, dt_off) < 0 or max(z_off + inner, x_off + channels, dt_off + num_heads) > width:
@@ -2215,8 +2219,7 @@ def state_space(proj: torch.Tensor, z_off: int, x_off: int, dt_off: int, conv_w:
     if taps > 1 and (conv_state is None or conv_state.dtype != torch.float32 or conv_state.dim() != 2
                      or conv_state.shape[1] != (taps - 1) * C or conv_state.stride(1) != 1):
         raise RuntimeError("state_space: conv_state is fp32 [slots, (taps - 1) * channels]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("state_space: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("state_space", state_indices, seq_lens, B)
     _batch_rows("state_space", T, B, q_start, q_len)
     if min(z_off, x_off, dt_off) < 0 or max(z_off + inner, x_off + C, dt_off + num_heads) > proj.shape[1]:
         raise RuntimeError("state_space: a column range leaves the row")
@@ -2422,8 +2425,7 @@ def matrix_memory(proj: torch.Tensor, offsets, num_heads: int, qk_dim: int, v_di
     if state.dtype != torch.float32 or state.dim() != 2 or state.shape[1] != matrix_memory_state_width(num_heads, qk_dim, v_dim) \
             or state.stride(1) != 1:
         raise RuntimeError("matrix_memory: state is fp32 [slots, H * D * E + H * D + H]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError("matrix_memory: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids("matrix_memory", state_indices, seq_lens, B)
     _batch_rows("matrix_memory", T, B, q_start, q_len)
     lib = _lib.load()
     work = torch.empty(int(lib.semipd_matrix_memory_workspace(T, num_heads, v_dim)), dtype=torch.float32, device=proj.device)
@@ -2539,8 +2541,7 @@ def linear_attention(proj: torch.Tensor, offsets, num_heads: int, qk_dim: int, v
         raise RuntimeError(f"{name}: norm_weight is contiguous [{'H * E' if norm_together else 'E'}] of the activation type")
     if state.dtype != torch.float32 or state.dim() != 2 or state.shape[1] != qk * v_dim or state.stride(1) != 1:
         raise RuntimeError(f"{name}: state is fp32 [slots, H * D * E]")
-    if state_indices.dtype != torch.int64 or seq_lens.dtype != torch.int64 or seq_lens.shape[0] != B:
-        raise RuntimeError(f"{name}: state_indices / seq_lens are int64 [B]")
+    state_indices, seq_lens = _batch_ids(name, state_indices, seq_lens, B)
     _batch_rows(name, T, B, q_start, q_len)
     if out is None:
         out = torch.empty((T, inner), dtype=proj.dtype, device=proj.device)

@@ -87,3 +87,22 @@ def test_step_refuses_what_the_general_call_refuses(kind):
     # numbers of another kind go the general way
     eps = torch.tensor(1e-5)
     assert torch.equal(call(**_clone({**args, "eps": eps})), call(**_clone({**args, "eps": float(eps)})))
+
+
+# (columns of a table, a length that all requests share: rows and lengths are the view's, not those of the memory behind its first element)
+@pytest.mark.parametrize("kind", ["delta_rule", "state_space"])
+@pytest.mark.parametrize("prompt", [False, True])
+def test_rows_and_lengths_that_are_views(kind, prompt):
+    T = 3
+    call, args = _step_call(kind, T, torch.Generator().manual_seed(7))
+    if prompt:
+        args.update(q_start=torch.arange(T, dtype=torch.int32).cuda(), q_len=torch.ones(T, dtype=torch.int32).cuda())
+    args["state_indices"] = torch.tensor([2, 3, 1]).cuda()
+    table = torch.stack([torch.tensor([1, 1, 2]).cuda(), args["state_indices"], torch.tensor([3, 1, 1]).cuda()], 1)           # (all of it rows that there are)
+    for lens, seen in ((torch.tensor([5, 1, 9]).cuda(), None), (torch.full((T,), 4).cuda(), torch.tensor([4]).cuda().expand(T))):
+        dense, view = _clone({**args, "seq_lens": lens}), _clone(args)
+        view["state_indices"] = table[:, 1]
+        view["seq_lens"] = torch.stack([lens, lens.flip(0)], 1)[:, 0] if seen is None else seen
+        assert not view["state_indices"].is_contiguous() and not view["seq_lens"].is_contiguous()
+        assert torch.equal(call(**view), call(**dense))
+        assert torch.equal(view["state"], dense["state"]) and torch.equal(view["conv_state"], dense["conv_state"])
