@@ -172,7 +172,7 @@ int semipd_build_kv_indices(const int32_t* req_to_token, int64_t req_to_token_st
 
 /* What a captured decode step reads of its batch, in one launch: rows 0 .. batch - 1 of token ids, pool rows, lengths, slots of the new
  * tokens and (state_rows may be NULL) state rows from src_* to the graph's own; rows batch .. rows - 1 are padding: pool row, slot and
- * state row 0, length pad_len, ids as they are.  src_state NULL: no state rows but the padding's.
+ * state row 0, length pad_len, ids as they are.  src_state NULL: the padding's state row, 0, in all rows.
  * replaces the copies in CudaGraphRunner.replay (model_executor/cuda_graph_runner.py:455-531). */
 int semipd_decode_inputs(int64_t* ids, int64_t* pool_rows, int64_t* lens, int64_t* slots, int64_t* state_rows, const int64_t* src_ids,
                          const int64_t* src_pool_rows, const int64_t* src_lens, const int64_t* src_slots, const int64_t* src_state,

@@ -750,10 +750,7 @@ __global__ void decode_inputs_kernel(int64_t* __restrict__ ids, int64_t* __restr
   pool_rows[i] = i < batch ? src_pool_rows[i] : 0;
   lens[i] = i < batch ? src_lens[i] : pad_len;
   slots[i] = i < batch ? src_slots[i] : 0;
-  if (state_rows != nullptr) {
-    if (i >= batch) state_rows[i] = 0;
-    else if (src_state != nullptr) state_rows[i] = src_state[i];
-  }
+  if (state_rows != nullptr) state_rows[i] = i < batch && src_state != nullptr ? src_state[i] : 0;
 }
 
 __global__ void compute_positions_kernel(const int32_t* __restrict__ prefix_lens,

@@ -199,6 +199,7 @@ class HipGraphRunner:
                 self.seq_lens.fill_(self.seq_len_fill_value)
                 self.out_cache_loc.zero_()
                 self.req_pool_indices.zero_()
+            if bs != raw_bs or forward_batch.state_indices is None:
                 self.state_indices.zero_()
             if forward_batch.state_indices is not None:
                 self.state_indices[:raw_bs].copy_(forward_batch.state_indices)

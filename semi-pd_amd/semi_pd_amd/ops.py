@@ -231,8 +231,8 @@ def compute_position(extend_prefix_lens: torch.Tensor, extend_seq_lens: torch.Te
 
 def decode_inputs(own, batch, rows: int, pad_len: int) -> bool:
     """own = (token ids, pool rows, lengths, slots, state rows) of a captured decode step, batch = the same of a decode batch (state rows may be
-    None): one launch for the copies, with rows len(batch) .. rows - 1 padded.  False, and nothing done, where one of the batch's is not a
-    contiguous int64 tensor on the graph's device."""
+    None: row 0, the padding's, in all of them): one launch for the copies, with rows len(batch) .. rows - 1 padded.  False, and nothing done,
+    where one of the batch's is not a contiguous int64 tensor on the graph's device."""
     dev = own[0].device
     for t in batch:
         if t is not None and (t.dtype != torch.int64 or t.device != dev or t.dim() != 1 or not t.is_contiguous()):

@@ -18,8 +18,8 @@ def test_inputs_of_a_captured_step(batch, rows, state):
         got = got.cpu()
         if want is not None:
             assert torch.equal(got[:batch], want.cpu())
-        else:
-            assert bool((got[:batch] == 7 + i).all())
+        else:                                                       # (no state rows of an earlier step)
+            assert bool((got[:batch] == 0).all())
         assert bool((got[batch: rows] == (7 + i if pad is None else pad)).all()) and bool((got[rows:] == 7 + i).all())
 
 
