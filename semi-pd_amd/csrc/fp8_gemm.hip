@@ -492,7 +492,7 @@ int launch_fp8_stream_grouped(void* c, const void* a, const float* a_s, const vo
 
 // fp8_rows.hip
 int launch_fp8_rows_grouped(void* c, const void* a, const float* a_s, const void* w, const float* w_s, const float* topk_weights, const int32_t* sorted_ids,
-                            const int32_t* expert_ids, const int32_t* num_post_pad, int num_valid, int N, int K, int blocks, int block_n, int top_k_div,
+                            const int32_t* expert_ids, const int32_t* num_post_pad, int num_valid, int N, int K, int64_t max_sorted, int block_n, int top_k_div,
                             int mul_routed_weight, int out_dtype, hipStream_t st);
 
 }  // namespace semipd
@@ -607,7 +607,7 @@ int semipd_moe_grouped_gemm_fp8(void* c, const void* a_q, const float* a_s, cons
   // blocks of 128 rows over whole scale blocks and groups of 16 columns: fp8_rows.hip (the figures are there); the others below
   if (block_m == 128 && k % 128 == 0 && n % 16 == 0 && (reinterpret_cast<uintptr_t>(c) & 15u) == 0 && num_valid < (1 << 30) && n < (1 << 30) && k < (1 << 30))
     return launch_fp8_rows_grouped(c, a_q, a_s, w_q, w_s, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad, (int)num_valid, (int)n, (int)k,
-                                   (int)((max_sorted + 127) / 128), block_n, top_k_div, mul_routed_weight, out_dtype, static_cast<hipStream_t>(stream));
+                                   max_sorted, block_n, top_k_div, mul_routed_weight, out_dtype, static_cast<hipStream_t>(stream));
   return dispatch_fp8_gemm<true>(c, a_q, a_s, w_q, w_s, topk_weights, sorted_token_ids, expert_ids, num_tokens_post_pad,
                                  num_valid, 0, n, k, n, (max_sorted + block_m - 1) / block_m, block_m, block_n, top_k_div,
                                  mul_routed_weight,

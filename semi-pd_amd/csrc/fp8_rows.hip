@@ -33,6 +33,7 @@ struct F8RowsArgs {
   const float *a_s, *w_s, *topk_weights;
   const int32_t *sorted_ids, *expert_ids, *num_post_pad;
   int num_valid, N, K, block_n, top_k_div, mul_routed_weight;
+  int64_t max_sorted;
 };
 
 template <typename OutT>
@@ -41,7 +42,8 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
   __shared__ __attribute__((aligned(16))) uint8_t rows_l[2][kF8Block];
   __shared__ __attribute__((aligned(16))) float scale_l[2][kF8Rows];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c16 = lane & 15, q4 = lane >> 4;
-  const int tiles_n = (p.N + kF8Cols - 1) / kF8Cols, tiles_m = p.num_post_pad[0] / kF8Rows, total = tiles_m * tiles_n;
+  const int64_t entries = p.num_post_pad[0] < p.max_sorted ? p.num_post_pad[0] : p.max_sorted;
+  const int tiles_n = (p.N + kF8Cols - 1) / kF8Cols, tiles_m = (int)((entries + kF8Rows - 1) / kF8Rows), total = tiles_m * tiles_n;
   const int per = (total + 7) >> 3, at = blockIdx.x >> 3, logical = (int)(blockIdx.x & 7) * per + at;
   if (at >= per || logical >= total) return;
   const int tile_m = logical / tiles_n, tile_n = logical - tile_m * tiles_n, m0 = tile_m * kF8Rows, n0 = tile_n * kF8Cols + 32 * wave;
@@ -49,7 +51,8 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
   const int64_t expert = p.expert_ids[tile_m];
   const int32_t* ids = p.sorted_ids + m0;
   const uint32_t valid = (uint32_t)p.num_valid;
-  const uint64_t low = __ballot((uint32_t)ids[lane] < valid), high = __ballot((uint32_t)ids[64 + lane] < valid);
+  auto entry = [&](int r) { return m0 + r < p.max_sorted ? (uint32_t)ids[r] : valid; };                 // (a last block that is not whole)
+  const uint64_t low = __ballot(entry(lane) < valid), high = __ballot(entry(64 + lane) < valid);
   if ((low | high) == 0) return;
   const bool upper = high != 0;                                   // (entries behind the padding there are none: up to 64 rows are the lower half's)
 
@@ -60,10 +63,10 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
 #pragma unroll
   for (int e = 0; e < NX; ++e) {
     const int r = 8 * kF8Waves * e + (tid >> 3);
-    src[e] = p.a + (int64_t)row_of(ids[r]) * p.K + ((tid & 7) << 4);
+    src[e] = p.a + (int64_t)row_of(entry(r)) * p.K + ((tid & 7) << 4);
     to[e] = r * 128 + (((tid & 7) ^ ((r >> 1) & 7)) << 4);
   }
-  const float* src_s = p.a_s + (int64_t)row_of(ids[tid & 127]) * KB;
+  const float* src_s = p.a_s + (int64_t)row_of(entry(tid & 127)) * KB;
   const uint8_t* wp[NG];
   const float* wsp[NG];
 #pragma unroll
@@ -175,7 +178,7 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
   // lane holds c[entry 16 t + c16][n0 + 16 g + 4 q4 .. + 3]
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const uint32_t id = (uint32_t)ids[16 * t + c16];
+    const uint32_t id = entry(16 * t + c16);
     if (id >= valid) continue;
     const float scale = p.mul_routed_weight ? p.topk_weights[id] : 1.f;
     OutT* dst = (OutT*)p.c + (int64_t)id * p.N + n0 + 4 * q4;
@@ -197,10 +200,10 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
 
 // K % 128 == 0, N % 16 == 0, c aligned to 16 bytes, blocks of 128 entries: the caller sees to it
 int launch_fp8_rows_grouped(void* c, const void* a, const float* a_s, const void* w, const float* w_s, const float* topk_weights, const int32_t* sorted_ids,
-                            const int32_t* expert_ids, const int32_t* num_post_pad, int num_valid, int N, int K, int blocks, int block_n, int top_k_div,
+                            const int32_t* expert_ids, const int32_t* num_post_pad, int num_valid, int N, int K, int64_t max_sorted, int block_n, int top_k_div,
                             int mul_routed_weight, int out_dtype, hipStream_t st) {
-  const F8RowsArgs p{c, (const uint8_t*)a, (const uint8_t*)w, a_s, w_s, topk_weights, sorted_ids, expert_ids, num_post_pad, num_valid, N, K, block_n, top_k_div, mul_routed_weight};
-  const int64_t tiles = (int64_t)blocks * ((N + kF8Cols - 1) / kF8Cols);
+  const F8RowsArgs p{c, (const uint8_t*)a, (const uint8_t*)w, a_s, w_s, topk_weights, sorted_ids, expert_ids, num_post_pad, num_valid, N, K, block_n, top_k_div, mul_routed_weight, max_sorted};
+  const int64_t tiles = (max_sorted + kF8Rows - 1) / kF8Rows * ((N + kF8Cols - 1) / kF8Cols);
   const dim3 grid((unsigned)((tiles + 7) / 8 * 8));
   switch (out_dtype) {
     case SEMIPD_BF16: hipLaunchKernelGGL((fp8_rows_kernel<bf16_t>), grid, dim3(64 * kF8Waves), 0, st, p); break;

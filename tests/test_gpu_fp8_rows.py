@@ -49,3 +49,23 @@ def test_blocks_of_128_rows_against_their_products(K, N, block_n, out_dtype):
         # it: 2^-12 of the sum at most)
         bound = (half * (want * s).abs() + 2.0 ** -11 * size * s) * down + 2.0 ** -24
         assert bool(((out[:total].cpu().double() - want * s * down).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("last", [1, 40, 64, 65, 127])
+def test_a_last_block_that_is_not_whole(last):
+    """Entries and their count end within a block: its rows are multiplied, and nothing behind them is read."""
+    g = torch.Generator().manual_seed(last)
+    E, K, N, total = 2, 256, 272, 128 + last
+    a, w = (torch.randn(*s, generator=g).to(torch.float8_e4m3fn).to(DEV) for s in ((total, K), (E, N, K)))
+    a_s, w_s = (torch.rand(*s, generator=g).to(DEV) for s in ((total, K // 128), (E, -(-N // 128), K // 128)))
+    experts = torch.tensor([1, 0], dtype=torch.int32, device=DEV)
+    ids = torch.randperm(total, generator=g).int()
+    outs = []
+    for entries in (ids, torch.cat([ids, torch.full((256 - total,), total, dtype=torch.int32)])):
+        memory = torch.zeros(256 + 128, dtype=torch.int32, device=DEV)                        # (behind the entries: row 0 of the result)
+        memory[: entries.numel()] = entries.to(DEV)
+        out = torch.full((total, N), 77.0, dtype=torch.bfloat16, device=DEV)
+        ops.moe_grouped_gemm_fp8(a, a_s, w, w_s, out, None, memory[: entries.numel()], experts,
+                                 torch.tensor([entries.numel()], dtype=torch.int32, device=DEV), total, 1, False, [128, 128], 128)
+        outs.append(out)
+    assert torch.equal(*outs)
