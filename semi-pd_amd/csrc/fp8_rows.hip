@@ -9,7 +9,11 @@
 //    are read by it alone and stay in its registers, three blocks in turn, asked for two blocks ahead.  One barrier a block.  (Rows by LDS-DMA:
 //    the compiler drains all loads in front of the weights' use then.)  Chunk c (16 bytes) of row r lies at c ^ ((r >> 1) & 7), as in gemm8p.hip.
 //  * An XCD (workgroup id % 8) takes a contiguous eighth of the tiles there are, the column tiles of a block next to each other: its
-//    rows are fetched into one L2, and the weight rows that several blocks of an expert read are found there.
+//    rows are fetched into one L2, and the weight rows that several blocks of an expert read are found there.  Experts of more than 24 MB
+//    are not: of theirs up to 8 column tiles of every block come first, then the next ones, so that the blocks that are at work share weight
+//    rows.  8 experts, 520 rows each, product alone, us, column tiles next to each other / in groups (/ the kernel of all block sizes): 28672 x 4096 1184 / 929
+//    (1110), 8192 x 8192 680 / 549 (635), 4096 x 14336 539 / 523 (588), 8192 x 5120 428 / 363 (422); 64 of 4096 x 7168 1928 / 1844 (2104); below the
+//    line 64 of 7168 x 2048 1042 / 1113 (1202), 16 of 5120 x 1536 with 64 rows 41.5 / 43.2.
 // Bound: of a block's 1.0 k cycles of products a SIMD the folds take as many again (80 vector instructions a wave), the rows' way through LDS 1.0 k of
 // the CU's and its loads 0.8 k (48 KB; with 128 weight rows a workgroup, two of them a CU, 64 KB and 1.0 k: 2566 tokens 409 us); behind one block an
 // expert the weights' stream.  64 experts of 2048 x 1408, top 6, whole layer, us, the kernel of all block sizes (fp8_gemm.hip: weights one block
@@ -26,6 +30,7 @@ typedef int f8r_i32x8 __attribute__((ext_vector_type(8)));
 typedef int f8r_i32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kF8Rows = 128, kF8Waves = 8, kF8Cols = 32 * kF8Waves, kF8Block = kF8Rows * 128;      // rows, columns of a tile; bytes of a block's rows
+constexpr int64_t kF8LargeExpert = 24 << 20;       // bytes of an expert's weight
 
 struct F8RowsArgs {
   void* c;
@@ -46,13 +51,25 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
   const int tiles_n = (p.N + kF8Cols - 1) / kF8Cols, tiles_m = (int)((entries + kF8Rows - 1) / kF8Rows), total = tiles_m * tiles_n;
   const int per = (total + 7) >> 3, at = blockIdx.x >> 3, logical = (int)(blockIdx.x & 7) * per + at;
   if (at >= per || logical >= total) return;
-  const int tile_m = logical / tiles_n, tile_n = logical - tile_m * tiles_n, m0 = tile_m * kF8Rows, n0 = tile_n * kF8Cols + 32 * wave;
+  int tile_m = logical / tiles_n, tile_n = logical - tile_m * tiles_n;
+  if ((int64_t)p.N * p.K > kF8LargeExpert) {
+    const int groups = (tiles_n + 7) >> 3, width = (tiles_n + groups - 1) / groups, group = logical / (tiles_m * width);
+    const int within = logical - group * tiles_m * width, cols = min(width, tiles_n - group * width);
+    tile_m = within / cols, tile_n = group * width + within - tile_m * cols;
+  }
+  const int m0 = tile_m * kF8Rows, n0 = tile_n * kF8Cols + 32 * wave;
   const int KB = p.K >> 7, NB = (p.N + p.block_n - 1) / p.block_n;
   const int64_t expert = p.expert_ids[tile_m];
   const int32_t* ids = p.sorted_ids + m0;
   const uint32_t valid = (uint32_t)p.num_valid;
-  auto entry = [&](int r) { return m0 + r < p.max_sorted ? (uint32_t)ids[r] : valid; };                 // (a last block that is not whole)
-  const uint64_t low = __ballot(entry(lane) < valid), high = __ballot(entry(64 + lane) < valid);
+  const int last = (int)(entries - m0 < kF8Rows ? entries - m0 : kF8Rows) - 1;
+  // the block's entries, a lane the one of its place in either half (a last block may not be whole); both reads at once, everything in front of
+  // the loop takes them from here
+  uint32_t id[2] = {(uint32_t)ids[min(lane, last)], (uint32_t)ids[min(64 + lane, last)]};
+  asm volatile("" : "+v"(id[0]), "+v"(id[1]));
+  if (lane > last) id[0] = valid;
+  if (64 + lane > last) id[1] = valid;
+  const uint64_t low = __ballot(id[0] < valid), high = __ballot(id[1] < valid);
   if ((low | high) == 0) return;
   const bool upper = high != 0;                                   // (entries behind the padding there are none: up to 64 rows are the lower half's)
 
@@ -63,10 +80,10 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
 #pragma unroll
   for (int e = 0; e < NX; ++e) {
     const int r = 8 * kF8Waves * e + (tid >> 3);
-    src[e] = p.a + (int64_t)row_of(entry(r)) * p.K + ((tid & 7) << 4);
+    src[e] = p.a + (int64_t)row_of(__shfl(id[e], r & 63, 64)) * p.K + ((tid & 7) << 4);
     to[e] = r * 128 + (((tid & 7) ^ ((r >> 1) & 7)) << 4);
   }
-  const float* src_s = p.a_s + (int64_t)row_of(entry(tid & 127)) * KB;
+  const float* src_s = p.a_s + (int64_t)row_of(wave & 1 ? id[1] : id[0]) * KB;
   const uint8_t* wp[NG];
   const float* wsp[NG];
 #pragma unroll
@@ -178,8 +195,8 @@ __global__ void __launch_bounds__(64 * kF8Waves, 2) fp8_rows_kernel(F8RowsArgs p
   // lane holds c[entry 16 t + c16][n0 + 16 g + 4 q4 .. + 3]
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
-    const uint32_t id = entry(16 * t + c16);
-    if (id >= valid) continue;
+    if (!((t < MT / 2 ? low : high) >> (16 * (t % (MT / 2)) + c16) & 1)) continue;
+    const uint32_t id = (uint32_t)ids[16 * t + c16];
     const float scale = p.mul_routed_weight ? p.topk_weights[id] : 1.f;
     OutT* dst = (OutT*)p.c + (int64_t)id * p.N + n0 + 4 * q4;
 #pragma unroll

@@ -69,3 +69,24 @@ def test_a_last_block_that_is_not_whole(last):
                                  torch.tensor([entries.numel()], dtype=torch.int32, device=DEV), total, 1, False, [128, 128], 128)
         outs.append(out)
     assert torch.equal(*outs)
+
+
+def test_column_tiles_of_large_experts():
+    """Experts of more than 24 MB take their column tiles in groups, 49 of them here and the last of one tile: the bits of the two halves of
+    their columns, which are below that."""
+    g = torch.Generator(device=DEV).manual_seed(3)
+    E, K, N, at, counts = 2, 256, 98432, 49152, [129, 40]
+    total = sum(counts)
+    q = lambda *s: torch.randn(*s, generator=g, device=DEV).to(torch.float8_e4m3fn)                           # noqa: E731
+    a, w = q(total, K), q(E, N, K)
+    a_s, w_s = (torch.rand(*s, generator=g, device=DEV) for s in ((total, K // 128), (E, N // 128, K // 128)))
+    ids = torch.full((384,), total, dtype=torch.int32, device=DEV)
+    ids[:129], ids[256: 296] = torch.arange(129, device=DEV).int(), torch.arange(129, total, device=DEV).int()
+    experts, npp = torch.tensor([1, 1, 0], dtype=torch.int32, device=DEV), torch.tensor([384], dtype=torch.int32, device=DEV)
+
+    def run(lo, hi):
+        out = torch.full((total, hi - lo), 77.0, dtype=torch.bfloat16, device=DEV)
+        ops.moe_grouped_gemm_fp8(a, a_s, w[:, lo:hi].contiguous(), w_s[:, lo // 128: hi // 128].contiguous(), out, None, ids, experts, npp, total, 1, False,
+                                 [128, 128], 128)
+        return out
+    assert torch.equal(run(0, N), torch.cat([run(0, at), run(at, N)], 1))
