@@ -31,3 +31,18 @@ def test_greedy_token(dtype, vocab):
     wide = torch.zeros(6, vocab + 1, dtype=dtype)
     wide[:, 1:] = x
     assert ops.greedy_argmax(wide.to(DEV)[:, 1:]).cpu().tolist() == want
+
+
+# (a row each CU and more: narrower workgroups; values with many equals, the first of which is wanted, and a few rows without any value)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rows,vocab", [(255, 24576), (256, 24576), (256, 24581), (300, 65528), (256, 65536)])
+def test_greedy_tokens_of_many_rows(dtype, rows, vocab):
+    from semi_pd_amd import ops
+    g = torch.Generator().manual_seed(rows + vocab)
+    x = torch.randint(-40, 41, (rows, vocab), generator=g).to(dtype)
+    x[3] = float("-inf")
+    x[5] = float("nan")
+    x[7, : vocab - 1] = float("nan")
+    want = x.float().nan_to_num(nan=float("-inf")).numpy().argmax(1).tolist()
+    want[5] = 0
+    assert ops.greedy_argmax(x.to(DEV)).cpu().tolist() == want
