@@ -330,16 +330,9 @@ moe_align_kernel(const int32_t* __restrict__ topk_ids, int64_t numel, int E, int
     if (e >= 0 && e < E) atomicAdd(i < c0 ? &before[e] : &rest[e], 1);
   };
   const int64_t quads = ((uintptr_t)topk_ids & 15) == 0 ? numel / 4 : 0;
-  // (four pieces a thread under way: one at a time, 18006 ids were five round trips)
-  for (int64_t i = tid; i < quads; i += 4096) {
-    int4 e[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) e[u] = reinterpret_cast<const int4*>(topk_ids)[i + 1024 * u < quads ? i + 1024 * u : quads - 1];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t at = i + 1024 * u;
-      if (at < quads) count(e[u].x, 4 * at), count(e[u].y, 4 * at), count(e[u].z, 4 * at), count(e[u].w, 4 * at);
-    }
+  for (int64_t i = tid; i < quads; i += 1024) {
+    const int4 e = reinterpret_cast<const int4*>(topk_ids)[i];
+    count(e.x, 4 * i), count(e.y, 4 * i), count(e.z, 4 * i), count(e.w, 4 * i);
   }
   for (int64_t i = 4 * quads + tid; i < numel; i += 1024) count(topk_ids[i], i);
   __syncthreads();
