@@ -25,6 +25,7 @@
 //  * ssm_step_kernel: batches of one token per request in place of preparation and recurrence, a workgroup per (head, request).
 //  * ssm_decode_kernel: all of the above for batches of one token per request whose state is small, a workgroup per request.
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 #include "recurrent_chunks.h"
@@ -1248,7 +1249,7 @@ __global__ void __launch_bounds__(256) ssm_post_kernel(SsmArgs a) {
 // the recurrence's kernel for prompts, which waited for one row per lane and step of its chain, 110 us + 10 of preparation -> 50.
 // With the convolution's loads in front of the state's: whole call 73.8 -> 62.0 us (64 requests 133.7 -> 115.9, 32 of 64 heads 33.9 -> 29.4;
 // 5 requests 20.0 -> 19.8); behind them, tap by tap, it began when the state had arrived, a round trip a tap.
-template <typename T, int NIT>
+template <typename T, int NIT, bool EARLY>
 __global__ void __launch_bounds__(256) ssm_step_kernel(SsmArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];       // x [E] | B [N] | C [N] | sums [4][E]
   const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
@@ -1263,15 +1264,14 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(SsmArgs a) {
   const T* p = (const T*)a.p + (int64_t)b * a.ld;
   const float* cs = a.conv_state + slot * a.conv_ld;
   // Memory answers in order: what the convolution and the step size are made of is asked for in front of the state, all of it at once, and
-  // their arithmetic goes on while the state is on its way.  Up to four taps, the workgroup's first 512 channels; others one by one.
+  // their arithmetic goes on while the state is on its way.  Up to four taps (EARLY), the workgroup's first 512 channels; others one by one.
   const int channels = E + 2 * N;
   auto channel = [&](int i) { return i < E ? h * E + i : inner + (i < E + N ? g * N + (i - E) : G * N + g * N + (i - E - N)); };
   struct Inputs {
     T cur, shift, w[kRecTaps];
     float x[kRecTaps];                                            // (of k tokens back)
   } in[2];
-  const bool early = taps <= kRecTaps;
-  if (early)
+  if constexpr (EARLY)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int c = channel(min(tid + 256 * u, channels - 1));
@@ -1292,7 +1292,7 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(SsmArgs a) {
     const int n = n0 + i * rows;
     S[i] = (!fresh && n < N) ? *reinterpret_cast<const float4*>(st + n * E + e) : float4{0.f, 0.f, 0.f, 0.f};
   }
-  if (early)
+  if constexpr (EARLY)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int i = tid + 256 * u;
@@ -1302,7 +1302,7 @@ __global__ void __launch_bounds__(256) ssm_step_kernel(SsmArgs a) {
         if (k < taps && !fresh) y += Elem<T>::to_f(in[u].w[k]) * in[u].x[k];
       if (i < channels) lds[i] = ssm_silu(y);
     }
-  for (int i = early ? tid + 512 : tid; i < channels; i += 256) {
+  for (int i = EARLY ? tid + 512 : tid; i < channels; i += 256) {
     const int c = channel(i);
     const T* cw = (const T*)a.conv_w + (int64_t)c * taps;
     float y = (a.conv_b ? Elem<T>::to_f(((const T*)a.conv_b)[c]) : 0.f) + Elem<T>::to_f(cw[taps - 1]) * Elem<T>::to_f(p[a.x_off + c]);
@@ -1539,9 +1539,14 @@ static int state_space(const void* proj, int64_t ld, int64_t z_off, int64_t x_of
     const size_t bytes = (size_t)(v_dim + 2 * state_size + 4 * v_dim) * sizeof(float);
     const dim3 grid((unsigned)num_heads, (unsigned)batch);
     SEMIPD_DISPATCH_DTYPE(dtype, T, {
-      if (nit <= 4) hipLaunchKernelGGL((ssm_step_kernel<T, 4>), grid, dim3(256), bytes, s, a);
-      else if (nit <= 8) hipLaunchKernelGGL((ssm_step_kernel<T, 8>), grid, dim3(256), bytes, s, a);
-      else hipLaunchKernelGGL((ssm_step_kernel<T, 16>), grid, dim3(256), bytes, s, a);
+      const auto go = [&](auto early) {
+        constexpr bool EARLY = decltype(early)::value;
+        if (nit <= 4) hipLaunchKernelGGL((ssm_step_kernel<T, 4, EARLY>), grid, dim3(256), bytes, s, a);
+        else if (nit <= 8) hipLaunchKernelGGL((ssm_step_kernel<T, 8, EARLY>), grid, dim3(256), bytes, s, a);
+        else hipLaunchKernelGGL((ssm_step_kernel<T, 16, EARLY>), grid, dim3(256), bytes, s, a);
+      };
+      if (taps <= kRecTaps) go(std::true_type{});
+      else go(std::false_type{});
     });
     if (post()) return SEMIPD_EDTYPE;
     return launch_status("state_space(step)");
