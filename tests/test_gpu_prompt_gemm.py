@@ -36,6 +36,33 @@ def test_layers_that_were_not_timed(dtype, rows, n, k, silu, tiled):
     torch.testing.assert_close(got.float(), want, rtol=half, atol=half * 0.05 + 2.0 ** -17)
 
 
+# (short last tiles: a free CU for each of them, two in turn to a free CU, a round of their own; of one row and of 64; and what goes to the library)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n,k,tiled", [(800, 16384, 2048, True), (1088, 12288, 2048, True), (1089, 12288, 2048, False), (1345, 22016, 2048, False),
+                                            (1344, 22016, 2048, True), (1281, 22016, 2048, False), (2049, 16384, 2048, True), (576, 32768, 4096, False)])
+def test_gate_and_up_with_a_short_last_tile(dtype, rows, n, k, tiled, monkeypatch):
+    """gate_up_silu takes the tiled GEMM by the rule and gives the pair's result."""
+    from semi_pd_amd import ops
+    from semi_pd_amd.layers import basic
+    assert ops.tiled_gemm_short_tail(n, k, rows) == tiled and not ops.tiled_gemm_fills_chip(n, k, rows, True)
+    g = torch.Generator(device=DEV).manual_seed(rows + n)
+    x = torch.randn(rows, k, generator=g, device=DEV).to(dtype)
+    layer = basic.MergedColumnParallelLinear(k, [n // 2, n // 2], params_dtype=dtype).to(DEV)
+    layer.weight.data.copy_(k ** -0.5 * torch.randn(n, k, generator=g, device=DEV))
+    called, gemm_tall = [], ops.gemm_tall
+    monkeypatch.setattr(ops, "gemm_tall", lambda *a, **kw: called.append(1) or gemm_tall(*a, **kw))
+    was = basic.stream_linear_enabled()
+    basic.set_stream_linear(True)
+    try:
+        got = basic.gate_up_silu(x, layer, basic.SiluAndMul())
+    finally:
+        basic.set_stream_linear(was)
+    assert bool(called) == tiled
+    gate, up = (x.float() @ layer.weight.float().t()).to(dtype).float().chunk(2, -1)
+    half = 4 * {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]           # gate and up are rounded, then the product
+    torch.testing.assert_close(got.float(), torch.nn.functional.silu(gate) * up, rtol=half, atol=half * 0.05 + 2.0 ** -17)
+
+
 def test_rule_is_for_the_whole_chip(monkeypatch):
     from semi_pd_amd import ops
     for cus, takes in ((0, True), (256, True), (128, False)):

@@ -14,3 +14,12 @@ def test_short_tails(monkeypatch, n, k, rows, takes):
     assert ops.tiled_gemm_short_tail(n, k, rows) == takes
     monkeypatch.setitem(ops._DENSE_GEMM, "cus", 128)
     assert not ops.tiled_gemm_short_tail(n, k, rows)
+
+
+# (held-out sizes on both sides of each line: weights of many rows, a round more behind the tiles, two short tiles in turn on a CU, four rounds)
+@pytest.mark.parametrize("n,k,rows,takes", [
+    (32768, 4096, 808, False), (32768, 4096, 1064, False), (35840, 5120, 1320, False), (9728, 2560, 1576, False), (9728, 2560, 1344, True),
+    (22016, 4096, 1344, True), (22016, 4096, 1281, False), (24576, 3072, 1344, True), (24576, 3072, 1320, False), (27648, 5120, 1088, False), (30720, 5120, 1088, False),
+    (18944, 3584, 2065, False), (18944, 3584, 2577, True),    (30720, 2048, 1537, True), (18432, 2304, 1344, False), (14336, 3584, 1832, True), (14336, 3584, 1600, False)])
+def test_short_tails_of_other_layers(monkeypatch, n, k, rows, takes):
+    test_short_tails(monkeypatch, n, k, rows, takes)
