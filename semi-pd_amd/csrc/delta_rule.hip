@@ -24,6 +24,7 @@
 //  * delta_step_kernel / delta_decode_kernel: all of the above for batches of one token per request, a workgroup per (request, key
 //    head) where the state lies on 16-byte boundaries, else per (request, head).
 #include <cstring>
+#include <type_traits>
 
 #include "common.h"
 #include "recurrent_chunks.h"
@@ -470,7 +471,7 @@ __global__ void __launch_bounds__(1024) delta_decode_kernel(DeltaArgs a) {
 // state read and written once: 32 requests, 32 heads of 128 x 128 (134 MB): a column of S by four lanes of four bytes each 57.7 -> 32.3
 // us; 3 requests, 32 heads of 64 x 64: 10.6 (two launches) -> 9.8.  With the loads of the convolutions and of the gates in front of the state's (they came one
 // behind the other when the state had arrived): 32 heads of 128 x 128, 32 requests, whole call 31.6 -> 28.5, 64 requests 77.7 -> 68.9.
-template <typename T, int NIT>
+template <typename T, int NIT, int EARLY>
 __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaArgs a) {
   extern __shared__ __attribute__((aligned(16))) float lds[];       // q [D] | k [D] | v, later o [per E] | sums of every team [4][2][E] | scalars
   const int g = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, team = tid >> 8, tt = tid & 255, teams = blockDim.x >> 8;
@@ -491,8 +492,8 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
     return !fresh && hh < per && n < D ? *reinterpret_cast<const float4*>(a.state + slot * a.state_ld + ((int64_t)(g * per + hh) * D + n) * E + e) : float4{0.f, 0.f, 0.f, 0.f};
   };
   // Memory answers in order: what the convolutions are made of is asked for in front of the state, and with it what the team's first head needs
-  // behind the sums; their arithmetic goes on while the state is on its way, and nothing is a round trip of its own.  Up to four taps,
-  // the workgroup's first two channels a thread; others one by one.
+  // behind the sums; their arithmetic goes on while the state is on its way, and nothing is a round trip of its own.  Up to EARLY
+  // taps, the workgroup's first two channels a thread; others (EARLY 0: more than four taps) one by one.
   const int channels = 2 * D + per * E;
   struct Channel {
     const T *p, *cw;
@@ -507,17 +508,16 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
   auto mine = [&](int i) { return i < channels && (i < 2 * D || gridDim.z == 1 || ((i - 2 * D) / E / teams) % gridDim.z == blockIdx.z); };      // (or a head of another workgroup)
   float* cs = a.conv_state + slot * a.conv_ld;
   struct Inputs {
-    T cur, w[kRecTaps];
-    float x[kRecTaps];                                            // (of k tokens back)
+    T cur, w[EARLY + 1];
+    float x[EARLY + 1];                                           // (of k tokens back)
   } in[2];
-  const bool early = taps <= kRecTaps;
-  if (early)
+  if constexpr (EARLY > 0)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const Channel c = channel(min(tid + (int)blockDim.x * u, channels - 1));
       in[u].cur = *c.p;
 #pragma unroll
-      for (int k = 0; k < kRecTaps; ++k) {
+      for (int k = 0; k < EARLY; ++k) {
         in[u].w[k] = c.cw[max(taps - 1 - k, 0)];
         in[u].x[k] = k > 0 && k < taps && !fresh ? cs[(int64_t)(taps - 1 - k) * C + c.ch] : 0.f;
       }
@@ -540,7 +540,7 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
   for (int i = 0; i < NIT; ++i) S[i] = piece((int)blockIdx.z * teams + team, n0 + i * rows);
   // state entry s is the input s - (taps - 1) tokens back; every entry moves one place down and the token comes in last (where several
   // workgroups read the old inputs of q and k, in a launch of its own)
-  if (early)
+  if constexpr (EARLY > 0)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const int i = tid + (int)blockDim.x * u;
@@ -548,17 +548,17 @@ __global__ void __launch_bounds__(NIT > 4 ? 512 : 1024) delta_step_kernel(DeltaA
       const float cur = Elem<T>::to_f(in[u].cur);
       float y = Elem<T>::to_f(in[u].w[0]) * cur;
 #pragma unroll
-      for (int k = 1; k < kRecTaps; ++k)
+      for (int k = 1; k < EARLY; ++k)
         if (k < taps && !fresh) y += Elem<T>::to_f(in[u].w[k]) * in[u].x[k];
       lds[i] = silu_f(y);
       if (gridDim.z > 1) continue;
       const int ch = channel(i).ch;
 #pragma unroll
-      for (int k = 1; k < kRecTaps - 1; ++k)
+      for (int k = 1; k < EARLY - 1; ++k)
         if (k < taps - 1) cs[(int64_t)(taps - 2 - k) * C + ch] = in[u].x[k];
       if (taps > 1) cs[(int64_t)(taps - 2) * C + ch] = cur;
     }
-  for (int i = early ? tid + 2 * (int)blockDim.x : tid; i < channels; i += blockDim.x) {
+  for (int i = EARLY > 0 ? tid + 2 * (int)blockDim.x : tid; i < channels; i += blockDim.x) {
     if (!mine(i)) continue;
     const Channel c = channel(i);
     const float cur = Elem<T>::to_f(*c.p);
@@ -1827,9 +1827,17 @@ static int delta_rule(const void* proj, int64_t ld, int64_t q_off, int64_t k_off
     const int64_t room = 256 / (batch * num_k_heads), splits = rounds < room ? rounds : (room < 1 ? 1 : room);
     const dim3 sgrid((unsigned)num_k_heads, (unsigned)batch, (unsigned)splits);
     SEMIPD_DISPATCH_DTYPE(dtype, T, {
-      if (nit <= 4) hipLaunchKernelGGL((delta_step_kernel<T, 4>), sgrid, dim3(256 * teams), step_lds, st, a);
-      else if (nit <= 8) hipLaunchKernelGGL((delta_step_kernel<T, 8>), sgrid, dim3(256 * teams), step_lds, st, a);
-      else hipLaunchKernelGGL((delta_step_kernel<T, 16>), sgrid, dim3(256 * teams), step_lds, st, a);
+      const auto go = [&](auto early) {
+        constexpr int EARLY = decltype(early)::value;
+        if (nit <= 4) hipLaunchKernelGGL((delta_step_kernel<T, 4, EARLY>), sgrid, dim3(256 * teams), step_lds, st, a);
+        else if (nit <= 8) hipLaunchKernelGGL((delta_step_kernel<T, 8, EARLY>), sgrid, dim3(256 * teams), step_lds, st, a);
+        else hipLaunchKernelGGL((delta_step_kernel<T, 16, EARLY>), sgrid, dim3(256 * teams), step_lds, st, a);
+      };
+      // (instances of their own: what is asked for early holds its registers where it is not used, five taps and more 1 to 5 % faster without;
+      // two taps with the loads of four 3 % slower in batches of a few requests)
+      if (taps <= 2) go(std::integral_constant<int, 2>{});
+      else if (taps <= kRecTaps) go(std::integral_constant<int, kRecTaps>{});
+      else go(std::integral_constant<int, 0>{});
     });
     if (splits > 1 && taps > 1)
       SEMIPD_DISPATCH_DTYPE(dtype, T, hipLaunchKernelGGL((delta_conv_state_kernel<T>), dim3((unsigned)((C + 255) / 256), (unsigned)batch),

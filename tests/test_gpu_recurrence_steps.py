@@ -22,6 +22,13 @@ def test_delta_rule_step_channels(dtype, H, G, D, E, taps):
     steps.test_delta_rule_decode_step(dtype, H, G, D, E, taps)
 
 
+# (the form of two taps: a channel left over for a third thread, fewer than threads, a head each of several workgroups)
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,G,D,E", [(774, 86, 16, 256), (4, 1, 64, 64), (24, 1, 128, 64), (4, 2, 128, 128)])
+def test_delta_rule_step_of_two_taps(dtype, H, G, D, E):
+    steps.test_delta_rule_decode_step(dtype, H, G, D, E, 2)
+
+
 def _step_call(kind, T, g, dtype=torch.bfloat16):
     """ops.<kind> and the arguments of a decode batch of T requests, by name."""
     from semi_pd_amd import ops
