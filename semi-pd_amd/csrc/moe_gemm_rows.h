@@ -72,7 +72,7 @@ __device__ __forceinline__ void moe_rows_body(char* smem, T* __restrict__ out, c
   const int c16 = lane & 15, q4 = lane >> 4;
   const int n_cols = EPI == G8_SILU_MUL ? N / 2 : N;
   const int nkt = K >> 6;
-  static_assert(NX0 >= NX1 && NX0 <= 5, "the first half is the longer one");
+  static_assert(NX0 - NX1 >= 0 && NX0 - NX1 <= 1 && NX0 <= 5, "the first half is as long as the second, or one fragment longer: the waits count on it");
 
   // an entry's row: id / top_k_div, by 2^32 / top_k_div and what is left (35 instructions fewer than the division, of which a lane has 2 NX)
   const uint32_t div = grp.top_k_div, inverse = grp.inverse;
