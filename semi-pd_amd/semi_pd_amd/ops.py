@@ -596,23 +596,28 @@ def tiled_gemm_fills_chip(n: int, k: int, rows: int, fuse_silu_mul: bool = False
 
 def tiled_gemm_short_tail(n: int, k: int, rows: int) -> bool:
     """The same for gate and up with SiLU in the epilogue, where the last of several row tiles has at most 64 rows: its workgroups come last and take 0.5
-    to 0.65 of a tile's time.  With a free CU for each of them they cost nothing, two in turn to a free CU cost 0.2 to 0.3 of a round, a round of
-    their own 0.5 to 0.65.  Where they lengthen the rounds the tiled GEMM is ahead from 0.72 of the time they take then (9728 x 2560 from later on: 0.71 +8 %), taken
-    from 0.75; else it is level at 0.7 to 0.78 (28672 x 4096, 1320 rows 0 %; 18432 x 2304, 1344 +2; 18944 x 3584, 2065, three rounds +4; 28672 x 4096, 1832, four
-    rounds, +1), taken from 0.775, from three rounds on 0.8.  Weights of 32768 rows and more, or that the memory-side cache of 256 MB does not hold, go
-    to the library, which is up to 13 % ahead (32768 x 4096, 576 rows 152 / 172 us, 1064 254 / 274; 35840 x 5120, 1320 430 / 466; 30720 x 5120, 1088 309 /
-    324; 37888 x 3584, 1576 437 / 387 and 27648 x 5120, 1064 293 / 276 go with them).  Of 32 shapes all that
-    is taken is ahead or level.  us of the pair of launches, library / tiled: 28672 x 4096, 1064 rows 239 / 210, 1576 339 / 303; 22016 x 4096, 1344
-    309 / 218; 16384 x 3072, 808 86 / 78, 2088 225 / 185; 16384 x 2048, 808 62 / 54; 24576 x 3072, 1344 195 / 185; 14336 x 3584, 1832 169 / 167."""
+    to 0.65 of a tile's time.  What they add to the rounds of the whole tiles, and from what share of all that time on they are taken (0.8 from four rounds):
+      a free CU for each: nothing; level at 0.7 to 0.78 (28672 x 4096, 1320 rows 0 %; 18944 x 3584, 2065, three rounds, +4; 28672 x 4096, 1832, four rounds,
+        +1), taken from 0.775.
+      two in turn to a free CU, 32 CUs and more (four an XCD) free: 0.2 to 0.3 of a round and the library's own last round with it; 3 to 36 % ahead from
+        0.6 of the whole rounds on, taken from 0.775.
+      two in turn to fewer free CUs: 0.6 of a round; 6 to 9 % behind (9728 x 2560 and narrower): not taken.
+      a round of their own: 0.6 of one; ahead from 0.72 (29568 x 4096, 1088 rows, 0.74, +2), taken from there.
+    Weights of 32768 rows and more, or that the memory-side cache of 256 MB does not hold, are taken in the second form alone (27648 x 5120 -5 %, 35840
+    x 5120 -15 to -22, 37888 x 3584 -11); in the others the library is up to 13 % ahead (32768 x 4096, 576 rows 152 / 172 us, 1064 254 / 274; 35840 x 5120, 1320 430 /
+    466; 30720 x 5120, 1088 309 / 324; 37888 x 3584, 832 280 / 228 goes with them).  us of the pair of launches, library / tiled: 28672 x 4096, 1064 rows 239 / 210, 1576 339 / 303; 22016 x 4096, 1281 307 / 216;
+    16384 x 3072, 808 86 / 78, 2088 225 / 185; 16384 x 2048, 808 62 / 54; 24576 x 3072, 1344 195 / 185; 14336 x 3584, 1064 117 / 99, 1832 169 / 167."""
     tail, cols = rows % 256, -(-(n // 2) // 128)
-    if _DENSE_GEMM["cus"] not in (0, 256) or rows < 256 or not 0 < tail <= 64 or not 2048 <= k <= 5120 or not 0 < n < 32768 or 2 * n * k >= 1 << 28:
+    if _DENSE_GEMM["cus"] not in (0, 256) or rows < 256 or not 0 < tail <= 64 or not 2048 <= k <= 5120 or not 0 < n <= 37888:
         return False
     whole = rows // 256 * cols
     rounds = -(-whole // 256)
     free = rounds * 256 - whole
-    longer = 0.0 if cols <= free else 0.3 if cols <= 2 * free else 0.6
-    need = 0.75 if longer and rounds < 4 else 0.8 if rounds >= 3 else 0.775
-    return rows * (n // 2) >= need * (rounds + longer) * 256 * 256 * 128
+    two_in_turn, own_round = free < cols <= 2 * free, cols > 2 * free
+    if (two_in_turn and free < 32) or (not two_in_turn and (n >= 32768 or 2 * n * k >= 1 << 28)):
+        return False
+    need = 0.8 if rounds >= 4 else 0.72 if own_round else 0.775
+    return rows * (n // 2) >= need * (rounds + 0.6 * own_round) * 256 * 256 * 128
 
 
 def dense_gemm_report() -> str:

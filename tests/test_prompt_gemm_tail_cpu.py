@@ -16,10 +16,13 @@ def test_short_tails(monkeypatch, n, k, rows, takes):
     assert not ops.tiled_gemm_short_tail(n, k, rows)
 
 
-# (held-out sizes on both sides of each line: weights of many rows, a round more behind the tiles, two short tiles in turn on a CU, four rounds)
+# (sizes that the rule was not made from, on both sides of each line: a free CU for each short tile, two in turn on few and on many free CUs, a
+# round of their own, four rounds; weights of many rows and of more than 256 MB)
 @pytest.mark.parametrize("n,k,rows,takes", [
-    (32768, 4096, 808, False), (32768, 4096, 1064, False), (35840, 5120, 1320, False), (9728, 2560, 1576, False), (9728, 2560, 1344, True),
-    (22016, 4096, 1344, True), (22016, 4096, 1281, False), (24576, 3072, 1344, True), (24576, 3072, 1320, False), (27648, 5120, 1088, False), (30720, 5120, 1088, False),
-    (18944, 3584, 2065, False), (18944, 3584, 2577, True),    (30720, 2048, 1537, True), (18432, 2304, 1344, False), (14336, 3584, 1832, True), (14336, 3584, 1600, False)])
+    (12288, 2048, 1088, True), (9728, 2560, 1344, True), (18432, 2304, 1344, False), (14336, 3584, 1832, True), (14336, 3584, 1600, False),
+    (9728, 2560, 1576, False), (8704, 3072, 1856, False), (5632, 2048, 2880, False), (14336, 3584, 1064, True), (22016, 4096, 1281, True),
+    (24576, 3072, 1320, True), (29568, 4096, 1041, False), (24576, 3072, 1025, False), (28672, 4096, 1856, False), (24576, 3072, 2049, True),
+    (32768, 4096, 808, False), (32768, 4096, 1064, False), (35840, 5120, 1320, False), (30720, 5120, 1088, False), (27648, 5120, 1064, True),
+    (37888, 3584, 1576, True), (37888, 3584, 832, False), (37889, 2048, 1576, False)])
 def test_short_tails_of_other_layers(monkeypatch, n, k, rows, takes):
     test_short_tails(monkeypatch, n, k, rows, takes)
