@@ -506,7 +506,7 @@ __global__ void __launch_bounds__(256, 4) ssm_chunk_operands_kernel(SsmArgs a) {
 // Four waves per 16 columns halve what a wave does for a chunk: for launches that leave CUs without work at 64 columns a workgroup (a CU
 // holds one of theirs, not two: everything is fetched a whole chunk ahead, 2.9 -> 2.6 us a chunk, 3.3 at 64 columns).  128 heads of 128 x 64
 // over 8, whole call: 1 request of 5083 rows 611 -> 456 us, of 1000 137 -> 106; with the silus of a lane's four tokens side by side and D in one sum 434
-// (4 of 1900 rows, 64 columns a workgroup, 456 -> 451).
+// (4 of 1900 rows, 64 columns a workgroup: within 1 %).
 template <typename T, int NP, int CB>
 __global__ void __launch_bounds__(512, CB == 4 ? 4 : 2) ssm_chunk_walk_kernel(SsmArgs a, int64_t max_chunks) {
   constexpr int PARTS = 8 / CB;                                 // waves that share 16 columns
